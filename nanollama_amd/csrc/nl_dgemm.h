@@ -7,7 +7,7 @@
 // just to read its B operand; qgemm_kernel therefore split K over workgroups (<= 6 chunks each), wrote partial slabs and left
 // the sum, the norm, the rotation and SiLU to four more launches per layer: 8 launches of 5-9 us.
 // Here the TOKEN TILE is what a workgroup keeps: 16 tokens x all of K (98 KB for K = 1536) against T 16-row weight tiles, so a
-// result element is finished inside one workgroup and the qgemm2 epilogues (RoPE + KV store, SiLU(gate) * up as the next
+// result element is finished inside one workgroup and the prompt epilogues (RoPE + KV store, SiLU(gate) * up as the next
 // GEMM's fragments, residual + the folded RMSNorm of the next GEMM) apply as they are.  The four workgroups that share a row
 // group (one per token tile) sit on the same XCD (block b runs on XCD b % 8, observed -- for speed only), so a weight byte
 // crosses the fabric once and is an L2 hit for the other three.
@@ -26,8 +26,8 @@
 //     MFMA runs as D[token][row] = x . W^T, so a lane needs ONE scale per (block, tile): 1 ds_read_b32, 4 v_fma_mix.
 //     Per (block, tile): 9 VALU (nibbles -> fp16), 2 MFMA (x = hi + lo), 4 FMA ("* d"), 2 + 2/T LDS reads.
 //   * The NWV partial accumulators of a tile meet in LDS (one barrier per launch) in wavefront order and are read back
-//     transposed, as D[row][token] = the layout qgemm2_kernel's epilogues are written for.
-// Arithmetic per output = qgemm_kernel / qgemm2_kernel (exact integer quants in fp16, f32 block sums, * d in f32); the
+//     transposed, as D[row][token] = the layout its epilogues are written for.
+// Arithmetic per output = qgemm_kernel / pgemm_kernel (exact integer quants in fp16, f32 block sums, * d in f32); the
 // summation order over blocks is block-interleaved (NWV partial sums), inside the stated tolerances; deterministic.
 // hipcc waits vmcnt(0) for a register load once LDS-DMA pieces are in flight behind it (it treats the two as unordered): the
 // fragment loads are inline asm with hand-placed waits, and the epilogue operands (compiler-tracked, requested first) are first
@@ -35,7 +35,7 @@
 // Reference: go/quant.go:45-94 (MatMulQ4_0), go/model.go:513-613 (the layer), per stream.
 #pragma once
 #include <algorithm>
-#include "nl_qgemm2.h"
+#include "nl_pgemm.h"
 
 namespace nl {
 
@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) dgemm_kernel(QGemmParams P)
         return;
     }
     if constexpr (EPI == QG_EPI_ROPE) {
-        // RoPE (go/model.go:449-477) + attention biases (:525-527) + KV store (:552-554), as qgemm2_kernel's epilogue: the
+        // RoPE (go/model.go:449-477) + attention biases (:525-527) + KV store (:552-554), as pgemm_kernel's epilogue: the
         // rotation partner of rows 4*lq + j is rows 4*(lq ^ 2) + j of the same tile and token: lane ^ 32
         const QGemmParams::Rope &R = P.rope;
         const int hd = R.head_dim, half = hd >> 1, tsh = hd == 64 ? 2 : 1, nq = R.n_q_heads * hd;
@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) dgemm_kernel(QGemmParams P)
     }
     if constexpr (EPI == QG_EPI_PLAIN) {
         // out = resid + bias + y; then (QGemmParams::NormOut) the rows as the NEXT GEMM's fragments, times its norm weights and
-        // the token's power-of-two pre-scale, plus the float64 sum of squares of this group's 32 rows (qgemm2_kernel's
+        // the token's power-of-two pre-scale, plus the float64 sum of squares of this group's 32 rows (pgemm_kernel's
         // producer epilogue with one partial per 32-row block)
         const int row0 = etile0 * TR;
         if (etile0 + EG > P.ntiles) return;        // (row counts are multiples of 32 on this path: never taken)

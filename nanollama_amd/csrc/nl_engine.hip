@@ -11,7 +11,7 @@
 #include <mutex>
 #include "nl_kernels.h"
 #include "nl_qgemm.h"
-#include "nl_qgemm2.h"
+#include "nl_pgemm.h"
 #include "nl_dgemm.h"
 #include "nl_batch.h"
 #include "nl_sample.h"
@@ -1642,31 +1642,24 @@ hipError_t launch_xsplit(int wtype, const float *x, int ldx, int cols, int n_tok
     return hipGetLastError();
 }
 
-// Long token runs over Q4_0 weights take the weights-through-LDS kernel (nl_qgemm2.h: 1.2-1.5x qgemm_kernel from 128
-// tokens up, tools/qgemm2_bench.hip; Q8_0's 32-byte rows cost more to expand and stay on qgemm_kernel).  Workgroups of
-// 64 rows: x 256 tokens (two token tiles per wavefront) when that still gives every compute unit two of them, else x 64.
-bool qgemm2_ok(int wtype, int n_tokens) {
+// Which multi-token steps run on pgemm_kernel (nl_pgemm.h).  K-quant matrices: all of them.  The other formats: matrices of at least four
+// 128-column chunks (narrower ones never fill its pipeline) and steps of at least 128 (Q4_0: shorter ones have nl_dgemm.h where that is
+// eligible) or PG_MIN tokens; below, the split-K launches of qgemm_kernel.
+constexpr int PG_MIN = 65;
+bool pgemm_ok(int wtype, int cols, int n_tokens) {
+    if (wtype == WT_Q4_K || wtype == WT_Q6_K) return true;
     const char *knob = getenv("NL_QG2_MIN_TOKENS");   // knob (tests, tools; read per launch so a test can flip it): a huge value disables
-    const int min_n = knob ? atoi(knob) : 128;
-    return wtype == WT_Q4_0 && n_tokens >= min_n;
+    const int min_n = knob ? atoi(knob) : wtype == WT_Q4_0 ? 128 : PG_MIN;
+    return (wtype == WT_Q4_0 || wtype == WT_Q8_0 || wtype == WT_F16) && n_tokens >= min_n && cols >= 512;
 }
-// the plain GEMM of a long Q4_0 token run whose unsplit 64-row x 64-token grid fills the chip: qgemm2_kernel, no split-K
-bool qgemm2_plain_unsplit(int wtype, int ntiles, int n_tokens) {
-    return qgemm2_ok(wtype, n_tokens) && ((ntiles + 3) / 4) * ((n_tokens + QG_TOK - 1) / QG_TOK) >= 128;
-}
-template <int EPI>
-hipError_t launch_qgemm2(const QGemmParams &P, int row_blocks, hipStream_t st) {
-    if ((long long)row_blocks * ((P.n_tokens + 255) / 256) >= 512)
-        hipLaunchKernelGGL((qgemm2_kernel<WT_Q4_0, 4, 2, 8, EPI>), dim3(row_blocks, (P.n_tokens + 255) / 256, 1), dim3(512), 0, st, P);
-    else
-        hipLaunchKernelGGL((qgemm2_kernel<WT_Q4_0, 4, 1, 4, EPI>), dim3(row_blocks, (P.n_tokens + 63) / 64, 1), dim3(256), 0, st, P);
-    return hipGetLastError();
-}
+bool pgemm_ok(const PackedMat &m, int n_tokens) { return pgemm_ok(m.wtype, m.cols, n_tokens); }
 
 // gate || up with the SwiGLU epilogue (nl_qgemm.h): 4 wavefronts x (gate tile, up tile) per workgroup, no split-K.
 // Worth it only when the unsplit grid fills the chip; the caller falls back to the plain launch + bswiglu otherwise.
 constexpr int QG_FUSED_WAVES = 4;
-bool qgemm_swiglu_fits(int ntiles, int n_tokens) {
+bool qgemm_swiglu_fits(const PackedMat &m, int n_tokens) {
+    if (pgemm_ok(m, n_tokens)) return true;
+    const int ntiles = m.ntiles;
     static const int min_wg = getenv("NL_FUSED_SWIGLU_MIN_WG") ? atoi(getenv("NL_FUSED_SWIGLU_MIN_WG")) : 128;   // knob: tests force 1, tools disable with a huge value
     // (a step of <= 32 tokens runs the plain kernel on one / two 16-token tiles instead: big x 8 streams 7.76 -> 7.55 ms)
     return (n_tokens > 32 || min_wg <= 1) && ((ntiles + QG_FUSED_WAVES - 1) / QG_FUSED_WAVES) * ((n_tokens + QG_TOK - 1) / QG_TOK) >= min_wg;
@@ -1674,7 +1667,7 @@ bool qgemm_swiglu_fits(int ntiles, int n_tokens) {
 hipError_t launch_qgemm_swiglu(int wtype, QGemmParams P, hipStream_t st) {
     P.nt16 = ((P.n_tokens + 63) / 64) * 4;
     P.ksplit = 1;
-    if (qgemm2_ok(wtype, P.n_tokens)) return launch_qgemm2<QG_EPI_SWIGLU>(P, (P.ntiles + 1) / 2, st);
+    if (pgemm_ok(wtype, P.cols, P.n_tokens)) return pg_launch<QG_EPI_SWIGLU>(wtype, P, st);
     const dim3 grid((P.ntiles + QG_FUSED_WAVES - 1) / QG_FUSED_WAVES, (P.n_tokens + QG_TOK - 1) / QG_TOK, 1);
     switch (wtype) {
     case WT_Q4_0: hipLaunchKernelGGL((qgemm_kernel<WT_Q4_0, QG_FUSED_WAVES, 2, QG_EPI_SWIGLU>), grid, dim3(QG_FUSED_WAVES * 64), 0, st, P); break;
@@ -1687,14 +1680,16 @@ hipError_t launch_qgemm_swiglu(int wtype, QGemmParams P, hipStream_t st) {
 
 // Q|K|V GEMM with the RoPE + KV-store epilogue (nl_qgemm.h): 128-row workgroups, no split-K -- for steps whose
 // unsplit grid fills the chip (prompts); decode batches keep the split-K GEMM + brope_kv.
-bool qgemm_rope_fits(int ntiles, int n_tokens) {
+bool qgemm_rope_fits(const PackedMat &m, int n_tokens) {
+    if (pgemm_ok(m, n_tokens)) return true;
+    const int ntiles = m.ntiles;
     static const int min_wg = getenv("NL_FUSED_ROPE_MIN_WG") ? atoi(getenv("NL_FUSED_ROPE_MIN_WG")) : 128;   // knob: tests force 1
     return ((ntiles + QG_WAVES - 1) / QG_WAVES) * ((n_tokens + QG_TOK - 1) / QG_TOK) >= min_wg;
 }
 hipError_t launch_qgemm_rope(int wtype, QGemmParams P, hipStream_t st) {
     P.nt16 = ((P.n_tokens + 63) / 64) * 4;
     P.ksplit = 1;
-    if (qgemm2_ok(wtype, P.n_tokens)) return launch_qgemm2<QG_EPI_ROPE>(P, (P.ntiles + 3) / 4, st);
+    if (pgemm_ok(wtype, P.cols, P.n_tokens)) return pg_launch<QG_EPI_ROPE>(wtype, P, st);
     P.row_groups = (P.ntiles + QG_WAVES - 1) / QG_WAVES;
     const dim3 grid(P.row_groups, (P.n_tokens + QG_TOK - 1) / QG_TOK, 1);
     switch (wtype) {
@@ -1731,13 +1726,13 @@ hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_bu
     const int tok_tiles = (P.n_tokens + QG_TOK - 1) / QG_TOK;
     const int nchunks = (P.cols / 32 + QG_KC - 1) / QG_KC;
     const int mats = P.q1 ? 2 : 1;
-    if (qgemm2_plain_unsplit(wtype, P.ntiles, P.n_tokens) && mats == 1) {   // unsplit grid fills the chip
+    if (pgemm_ok(wtype, P.cols, P.n_tokens) && mats == 1) {
         P.ksplit = 1;
         P.part = nullptr;
         if (ks_out) *ks_out = 1;
-        return launch_qgemm2<QG_EPI_PLAIN>(P, (P.ntiles + 3) / 4, st);
+        return pg_launch<QG_EPI_PLAIN>(wtype, P, st);
     }
-    if (P.nrm_out.w) return hipErrorInvalidValue;   // (the folded norm's producer epilogue exists in qgemm2_kernel only: host logic error)
+    if (P.nrm_out.w) return hipErrorInvalidValue;   // (the folded norm's producer epilogue exists in pgemm_kernel only: host logic error)
     // Workgroup height: 128 rows (8 wavefronts) when that alone fills the chip, else 64 rows (4 wavefronts) --
     // twice the workgroups and half the split-K for the small-N decode batches (goldie shapes at 16-128 tokens:
     // -4...-18 % per launch, tools/qgemm_variants.sh); then split K until ~128 workgroups exist.
@@ -1813,7 +1808,7 @@ const int NL_BATCH_MIN = getenv("NL_BATCH_MIN") ? atoi(getenv("NL_BATCH_MIN")) :
 
 bool batch_supported(const nl_engine *e) {
     if (e->G != 1 || e->force_tp_plan) return false;
-    auto ok = [](const PackedMat &m) { return m.wtype == WT_Q4_0 || m.wtype == WT_Q8_0 || m.wtype == WT_F16; };
+    auto ok = [](const PackedMat &m) { return m.wtype == WT_Q4_0 || m.wtype == WT_Q8_0 || m.wtype == WT_F16 || m.wtype == WT_Q4_K || m.wtype == WT_Q6_K; };
     for (const auto &L : e->layers)
         if (!ok(L.qkv) || !ok(L.wo) || !ok(L.gate) || !ok(L.up) || !ok(L.down)) return false;
     return ok(e->lm_head) && !getenv("NL_NO_BATCH_PATH");
@@ -1850,7 +1845,7 @@ int batch_alloc(nl_engine *e, nl_engine::Batch &b, int cap_limit = 2048) {
         HIPCK(e, dalloc(&raw, nx2 * 4, &e->bytes_state));
         b.xfrag2 = reinterpret_cast<uint4 *>(raw);
     }
-    HIPCK(e, dalloc(&b.ssq, n * (size_t)((c.dim + 31) / 32), &e->bytes_state));   // (one partial per 64 rows on qgemm2_kernel, per 32 on dgemm_kernel)
+    HIPCK(e, dalloc(&b.ssq, n * (size_t)((c.dim + 31) / 32), &e->bytes_state));   // (one partial per 64 rows on pgemm_kernel, per 32 on dgemm_kernel)
     HIPCK(e, dalloc(&b.nscale, 2 * n, &e->bytes_state));
     b.kpart_cap = (size_t)16 * QG_TOK * std::max<size_t>(std::max<size_t>(R, c.dim), e->Is);
     HIPCK(e, dalloc(&b.kpart, b.kpart_cap, &e->bytes_state));
@@ -1927,7 +1922,7 @@ bool dgemm_step_ok(const nl_engine *e, int n) {
     const char *mk = getenv("NL_DGEMM_MAX_TOKENS");
     if (mk) return n <= atoi(mk);
     // Decode batches and prompts while the largest launch (gate || up: ceil(n / 16) token tiles x I / 64 row groups) stays within
-    // about four rounds of workgroups: measured ahead of the long-run GEMM of nl_qgemm2.h up to 256 tokens on goldie (768 / 1024
+    // about four rounds of workgroups: measured ahead of the long-run GEMM up to 256 tokens on goldie (768 / 1024
     // workgroups: 2.77 against 2.88 ms, 3.23 against 3.21) and 512 on mini (1.60 against 1.74 ms; 768 tokens 2.21 against 2.19) --
     // tools/bench_short_prompt.py
     return (long long)((n + 15) / 16) * (e->cfg.interm / 64) <= 1024;
@@ -1937,11 +1932,11 @@ bool dgemm_step_ok(const nl_engine *e, int n) {
 // (with resid / bias applied) when it ran unsplit, else split-K slabs in `part` for the consumer to add.
 hipError_t qg(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, const float *resid, hipStream_t st,
               GemmOut *res, float *part, const float *bias = nullptr, const uint4 *xf = nullptr,
-              const QGemmParams::NormOut *nout = nullptr, int x1 = 0) {
+              const QGemmParams::NormOut *nout = nullptr, int x1 = 0, int out_q4 = 1) {
     QGemmParams P{};
     P.bias = bias;
     P.x1 = x1;
-    if (nout) P.nrm_out = *nout;
+    if (nout) { P.nrm_out = *nout; P.out_q4 = out_q4; }
     P.q = m.q; P.s = m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
     P.xf = xf ? xf : bt.xfrag; P.n_tokens = n; P.out = out; P.ldo = ldo; P.resid = resid;
     int ks = 1;
@@ -2028,8 +2023,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const char *rk = getenv("NL_ROPE_IN_ATTN");    // knob (tests, tools; read per step): 0 keeps the brope_kv launch
     const bool rope_attn_knob = !(rk && atoi(rk) == 0);
     GemmOut pend{nullptr, nullptr, 1, 0, nullptr};   // GEMM output not yet folded into the residual stream
-    // RMSNorm folded around the GEMMs (QGemmParams::NormOut / NormIn): when WO and down run unsplit on qgemm2_kernel and
-    // their consumers are the fused-epilogue GEMMs of the same kernel -- a Q4_0 prompt -- the producing GEMM writes the
+    // RMSNorm folded around the GEMMs (QGemmParams::NormOut / NormIn): when WO and down run on pgemm_kernel and
+    // their consumers are the fused-epilogue GEMMs of the same kernel, the producing GEMM writes the
     // next GEMM's fragments and per-block sums of squares itself and the two bnorm launches per layer disappear (mini,
     // 2047 tokens: 2 x 8.7 us of 187 us per layer).  Fragment stores then alternate: the consumer of a producing GEMM
     // reads xfrag2, everything else xfrag.
@@ -2042,14 +2037,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     bool fold = fold_knob && !c.qk_norm && D % 64 == 0 && c.n_layers > 0;
     for (int l = 0; l < c.n_layers && fold; l++) {
         const nl_engine::Layer &L = e->layers[l];
-        fold = qgemm2_plain_unsplit(L.wo.wtype, L.wo.ntiles, n) && qgemm2_plain_unsplit(L.down.wtype, L.down.ntiles, n) &&
-               L.wo.ntiles % 4 == 0 && L.down.ntiles % 4 == 0 &&
-               qgemm2_ok(L.qkv.wtype, n) && qgemm_rope_fits(L.qkv.ntiles, n) &&
-               L.up.wtype == L.gate.wtype && qgemm2_ok(L.gate.wtype, n) && qgemm_swiglu_fits(L.gate.ntiles, n);
+        fold = pgemm_ok(L.wo, n) && pgemm_ok(L.down, n) && L.wo.ntiles % 4 == 0 && L.down.ntiles % 4 == 0 && pgemm_ok(L.qkv, n) && L.up.wtype == L.gate.wtype && pgemm_ok(L.gate, n);
     }
     if (dg) fold = true;
     const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
-    // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs (qgemm2_kernel) and the
+    // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs of Q4_0 files (pgemm_kernel) and the
     // prompt attention multiply only the fp16 hi half of every activation / probability -- half / a third of the matrix work,
     // activations rounded to 11 bits.  The default x = hi + lo keeps float32-grade results (logit tolerance 1e-4).
     const char *pk = getenv("NL_PREFILL_PRECISION");
@@ -2078,7 +2070,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         bool rope_in_attn = false;
         const bool folded_in = fold && l > 0;      // the previous layer's down GEMM wrote this layer's Q|K|V input
         if (!folded_in) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
-        if (dg || (!c.qk_norm && qgemm_rope_fits(L.qkv.ntiles, n))) {
+        if (dg || (!c.qk_norm && qgemm_rope_fits(L.qkv, n))) {
             // Q|K|V, RoPE, biases and the KV store in ONE launch (QK-norm needs whole heads: unfused path)
             QGemmParams P{};
             const PackedMat &m = L.qkv;
@@ -2170,7 +2162,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(dg_plain(L.wo, b.xfrag, L.bo, &nout));
         } else if (fold) {
             const QGemmParams::NormOut nout{L.ffn_norm, b.xfrag2, b.ssq, sB};
-            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm));
+            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm, L.gate.wtype == WT_Q4_0 ? 1 : 0));
         } else {
             LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, nullptr, x1_gemm));
             LCK(norm(L.ffn_norm, L.gate, 0, n));
@@ -2178,7 +2170,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         if (L.up.wtype != L.gate.wtype)   // (a mixed-type file: the fragment k-slot order differs per type)
             return e->fail(NL_ERR_UNSUPPORTED, "gate and up projections of different quantisation types");
         const uint4 *down_in = b.xfrag;
-        if (dg || qgemm_swiglu_fits(L.gate.ntiles, n)) {
+        if (dg || qgemm_swiglu_fits(L.gate, n)) {
             // gate, up and SiLU(gate) * up in ONE launch; h leaves as fragments in the second fragment store
             // (the first is still being read by other workgroups of this launch)
             QGemmParams P{};
@@ -2216,7 +2208,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         } else if (fold && l + 1 < c.n_layers) {
             const nl_engine::Layer &Ln = e->layers[l + 1];
             const QGemmParams::NormOut nout{Ln.attn_norm, b.xfrag2, b.ssq, sA};
-            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm));
+            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm, Ln.qkv.wtype == WT_Q4_0 ? 1 : 0));
         } else {
             LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, nullptr, x1_gemm));
         }

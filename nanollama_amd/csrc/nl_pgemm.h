@@ -1,0 +1,566 @@
+// nl_pgemm.h -- the multi-token GEMM of long token runs and of K-quant files: Y[n][row] = sum_k W[row][k] X[n][k], every weight format.
+//
+// Tile: a workgroup of four wavefronts owns RT 16-row weight tiles x 4 NTW 16-token tiles.  Its threads expand the weights of a
+// 128-column chunk ONCE into fp16 MFMA fragments in LDS (two buffers); every wavefront multiplies them against its own NTW token
+// tiles, whose hi / lo activation fragments go straight from the fragment store into its registers.
+//
+// What bounds a launch of these sizes is not a pipe but latency: an activation fragment is an L2 or fabric round trip (500-2000
+// cycles) away, a block of a 64 x 64 tile is 128 cycles of matrix work, and a prompt's narrow matrices give a compute unit one or two
+// workgroups.  So the fragments of a WHOLE chunk are in flight -- block b's registers are requested again for the next chunk right
+// behind block b's last MFMA --, raw weights are requested two chunks ahead, and the barrier between chunks orders LDS only
+// (__syncthreads() also waits for every global load in flight, i.e. for exactly that prefetch).
+//
+// The activation fragment is the MFMA's A operand: D[token][row], a lane holds four tokens of ONE row, so a block's scale is one
+// register (a chunk's four scales one ds_read_b128 per row tile) instead of four.  The accumulators go through LDS once at the end and
+// the epilogues read whole rows of a token: coalesced stores, and fragments in either k-slot order.
+//
+// Arithmetic: weights as exact integers in fp16, x = hi + lo in fp16 (2^-22), float32 accumulation, then
+//   Q4_0 / Q8_0 (/ Q5_0)  acc += d_block * z                      per 32-column block (go/quant.go:74-94, :149-165)
+//   Q4_K                  z over 4 blocks of (scale * q): scale * q <= 63 * 15 is an exact fp16 integer; acc += d * z per chunk, and
+//                         acc -= (dmin * min) * sum(x) per block, sum(x) by an MFMA against ones (go/quant.go:296-323)
+//   Q6_K                  scale * (q - 32) reaches 4096, two fp16 parts (the low one at most 1): three MFMAs; acc += d * z per chunk
+//   F16                   its own operand, accumulated in the MFMA
+//
+// Measured (us a launch, weights and fragments in L2; beside it the kernels that these launches ran on before, inside a model): Q4_0, 2047
+// tokens, 768 columns: Q|K|V 15.5 (21.8), gate and up 31.8 (40.5), WO / down (2048 columns) 10.5 / 17.7 (mean 23.5); F16, 993 tokens, 1536
+// columns: 26.7 (35.6), 52.3 (85.0), 17.9 / 36.3 (mean 43.2).  A 64 x 64 tile's block costs a wavefront about 310 cycles: 128 on the matrix
+// pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses), which a SIMD does not overlap with MFMAs
+// (matrix and vector cycles add up); larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
+// be 333 single-token steps: 152 ms, now 1.55 ms.
+#pragma once
+#include "nl_qgemm.h"
+#include <type_traits>
+
+namespace nl {
+
+// LDS-only workgroup barrier
+__device__ __forceinline__ void pg_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+enum { PG_NONE = 0, PG_BLOCK = 1, PG_CHUNK = 2 };   // when a sum is multiplied by its scale
+
+// (1024 + b) for the bytes b of u as packed fp16: the two halves of four bytes
+__device__ __forceinline__ h2_t pg_bytes_lo(uint32_t u) { return bits_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)); }
+__device__ __forceinline__ h2_t pg_bytes_hi(uint32_t u) { return bits_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)); }
+__device__ __forceinline__ h2_t pg_h2(float v) { return h2_t{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ half8_t pg_join(h2_t a, h2_t b, h2_t c, h2_t d) {
+    const uint4 u = make_uint4(h2_bits(a), h2_bits(b), h2_bits(c), h2_bits(d));
+    return __builtin_bit_cast(half8_t, u);
+}
+
+// one (row, 32-column block) of the tile layout: NC 16-byte chunks and SW scale words; part w of its fragment; its scales
+template <int WT> struct PgFmt;
+template <> struct PgFmt<WT_Q4_0> {
+    static constexpr int CPP = 2, NC = 1, SW = 1, SC = PG_BLOCK, FR = 1;
+    static __device__ __forceinline__ int chunk(int h, int) { return h; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[1], const uint32_t (&)[1], int, int w, half8_t (&f)[1]) {
+        f[0] = WFrag<WT_Q4_0>::expand(w == 0 ? c[0].x : w == 1 ? c[0].y : w == 2 ? c[0].z : c[0].w);
+    }
+    static __device__ __forceinline__ float scale(const uint32_t (&s)[1], int h) { return h2f_bits((s[0] >> (16 * h)) & 0xffff); }
+    static __device__ __forceinline__ float least(const uint32_t (&)[1], int) { return 0.f; }
+};
+template <> struct PgFmt<WT_Q8_0> {
+    static constexpr int CPP = 4, NC = 2, SW = 1, SC = PG_BLOCK, FR = 1;
+    static __device__ __forceinline__ int chunk(int h, int i) { return 2 * h + i; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&)[1], int, int w, half8_t (&f)[1]) {
+        const uint4 &v = c[w >> 1];
+        const uint32_t a = ((w & 1) ? v.z : v.x) ^ 0x80808080u, b = ((w & 1) ? v.w : v.y) ^ 0x80808080u;   // 1024 + 128 + q, exact
+        const h2_t off = pg_h2(1152.f);
+        f[0] = pg_join(pg_bytes_lo(a) - off, pg_bytes_hi(a) - off, pg_bytes_lo(b) - off, pg_bytes_hi(b) - off);
+    }
+    static __device__ __forceinline__ float scale(const uint32_t (&s)[1], int h) { return h2f_bits((s[0] >> (16 * h)) & 0xffff); }
+    static __device__ __forceinline__ float least(const uint32_t (&)[1], int) { return 0.f; }
+};
+template <> struct PgFmt<WT_F16> {
+    static constexpr int CPP = 8, NC = 4, SW = 0, SC = PG_NONE, FR = 1;
+    static __device__ __forceinline__ int chunk(int h, int i) { return 4 * h + i; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[4], const uint32_t (&)[1], int, int w, half8_t (&f)[1]) { f[0] = __builtin_bit_cast(half8_t, c[w]); }
+    static __device__ __forceinline__ float scale(const uint32_t (&)[1], int) { return 1.f; }
+    static __device__ __forceinline__ float least(const uint32_t (&)[1], int) { return 0.f; }
+};
+template <> struct PgFmt<WT_Q4_K> {
+    // pair p's 32 bytes: low nibbles = block 2p, high nibbles = block 2p + 1; words d | dmin and scale0 | min0 | scale1 | min1
+    static constexpr int CPP = 2, NC = 2, SW = 2, SC = PG_CHUNK, FR = 1;
+    static __device__ __forceinline__ int chunk(int, int i) { return i; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&s)[2], int h, int w, half8_t (&f)[1]) {
+        const uint4 &v = c[w >> 1];
+        const uint32_t a = (((w & 1) ? v.z : v.x) >> (4 * h)) & 0x0f0f0f0fu, b = (((w & 1) ? v.w : v.y) >> (4 * h)) & 0x0f0f0f0fu;
+        const float sc = (float)((s[1] >> (16 * h)) & 0xff);
+        const h2_t m = pg_h2(sc), o = pg_h2(-1024.f * sc);          // (1024 + q) sc - 1024 sc, one rounding of an exact value
+        f[0] = pg_join(__builtin_elementwise_fma(pg_bytes_lo(a), m, o), __builtin_elementwise_fma(pg_bytes_hi(a), m, o),
+                       __builtin_elementwise_fma(pg_bytes_lo(b), m, o), __builtin_elementwise_fma(pg_bytes_hi(b), m, o));
+    }
+    static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int) { return h2f_bits(s[0] & 0xffff); }
+    static __device__ __forceinline__ float least(const uint32_t (&s)[2], int h) { return h2f_bits(s[0] >> 16) * (float)((s[1] >> (16 * h + 8)) & 0xff); }
+};
+template <> struct PgFmt<WT_Q6_K> {
+    // int8 (q - 32); words d and four int8 scales of 16 columns each
+    static constexpr int CPP = 4, NC = 2, SW = 2, SC = PG_CHUNK, FR = 2;
+    static __device__ __forceinline__ int chunk(int h, int i) { return 2 * h + i; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&s)[2], int h, int w, half8_t (&f)[2]) {
+        const uint4 &v = c[w >> 1];
+        const float sc = (float)(int8_t)(s[1] >> (8 * (2 * h + (w >> 1))));
+        const uint32_t u[2] = {((w & 1) ? v.z : v.x) ^ 0x80808080u, ((w & 1) ? v.w : v.y) ^ 0x80808080u};
+        const h2_t m = pg_h2(sc), off = pg_h2(1152.f);
+        h2_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const h2_t q = ((i & 1) ? pg_bytes_hi(u[i >> 1]) : pg_bytes_lo(u[i >> 1])) - off;
+            hi[i] = q * m;                                            // rounded to 11 bits
+            lo[i] = __builtin_elementwise_fma(q, m, -hi[i]);          // what the rounding took: exact, at most 1
+        }
+        f[0] = pg_join(hi[0], hi[1], hi[2], hi[3]);
+        f[1] = pg_join(lo[0], lo[1], lo[2], lo[3]);
+    }
+    static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int) { return h2f_bits(s[0] & 0xffff); }
+    static __device__ __forceinline__ float least(const uint32_t (&)[2], int) { return 0.f; }
+};
+
+// EPI: QG_EPI_PLAIN (out / resid / bias, or split-K slabs; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
+// (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  X1: the single-product precision mode of Q4_0 prompts
+// (block scales multiplied into the fp16 weights, only the hi half of every activation).
+template <int WT, int RT, int NTW, int KW, int EPI, bool X1 = false>
+__global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmParams P) {
+    using F = PgFmt<WT>;
+    static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");
+    constexpr int KB = 4;                                   // blocks per chunk
+    constexpr int ROWS = RT * TR, TOK = 64 * NTW, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
+    constexpr int SC = X1 ? PG_NONE : F::SC;
+    constexpr bool MINS = WT == WT_Q4_K;
+    // a block's plane of fragments is padded by 64 bytes: the two pairs' expansions of a wavefront land on different banks
+    constexpr int PLANE = F::FR * RT * 1024 + 64, BUF = KB * PLANE, SCP = ROWS + 16, SCB = SCP * KB * 4, WBYTES = 2 * (BUF + (SC ? SCB : 0) + (MINS ? SCB : 0));
+    constexpr int SBYTES = TOK * LD * 4, SET = WBYTES > SBYTES ? WBYTES : SBYTES, NTHR = 256 * KW;
+    __shared__ __attribute__((aligned(16))) char smem_all[KW * SET];
+    __shared__ float s_tok[TOK];                            // consumer of a folded norm: 1 / rms per token; producer: the fragments' pre-scale
+    __shared__ __attribute__((aligned(16))) float s_gain[EPI == QG_EPI_PLAIN ? ROWS : 4];
+    // KW sets of four wavefronts take every KW-th chunk each, with weight buffers of their own; the epilogue adds their sums in set order
+    const int kset = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    char *const smem = smem_all + kset * SET;
+    const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, lq = lane >> 4;
+    const int nblocks = P.cols / 32, nchunks = (nblocks + KB - 1) / KB;
+    constexpr bool FUSED = EPI == QG_EPI_SWIGLU;
+    constexpr int TPW = FUSED ? RT / 2 : RT;                // row tiles of a matrix per workgroup
+    const int nrb = (P.ntiles + TPW - 1) / TPW, ntb = (P.n_tokens + TOK - 1) / TOK, total = nrb * ntb, per = (total + 7) / 8;
+    // blocks b, b + 8, ... run on one XCD, which takes a contiguous range of the tiles: of the operand that runs along the range each XCD
+    // reads an eighth, the other one it streams whole -- the smaller one (fragments are 4 bytes a value, weights 16 CPP bytes a pair and row)
+    const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (((int)blockIdx.x >> 3) >= per || id >= total) return;
+    const bool by_rows = (long long)P.ntiles * TR * (FUSED ? 2 : 1) * F::CPP > (long long)P.n_tokens * 16;
+    const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
+
+    // staging items: pair kk of the chunk's two, row r, half h of the pair, row tile -- a wavefront's loads are runs of 32 bytes
+    const int i_kk = tid & 1, i_r = (tid >> 1) & 15, i_h = (tid >> 5) & 1, i_t = tid >> 6;
+    struct Raw { uint4 c[F::NC]; uint32_t s[SWN]; };
+    auto stage_load = [&](int chunk, Raw (&r)[IPT]) {
+#pragma unroll
+        for (int i = 0; i < IPT; i++) {
+            const int rt = i_t + 4 * i, tile = min(tile0 + (FUSED ? rt % TPW : rt), P.ntiles - 1);
+            const uint8_t *const Wq = FUSED && rt >= TPW ? P.q1 : P.q;
+            const int pair = min(chunk * 2 + i_kk, P.npairs - 1), g = pair >> 2, k = pair & 3, gsz = min(KL, P.npairs - g * KL);
+            const unsigned gp = (unsigned)(tile * P.npairs + g * KL);
+#pragma unroll
+            for (int j = 0; j < F::NC; j++)
+                r[i].c[j] = *reinterpret_cast<const uint4 *>(Wq + ((size_t)gp * (F::CPP * TR) + (unsigned)((F::chunk(i_h, j) * TR + i_r) * gsz + k)) * 16);
+            if constexpr (F::SW > 0) {
+                const uint32_t *const Ws = (FUSED && rt >= TPW ? P.s1 : P.s) + ((size_t)gp * TR + (unsigned)(i_r * gsz + k)) * F::SW;
+                if constexpr (F::SW == 2) {
+                    const uint2 v = *reinterpret_cast<const uint2 *>(Ws);
+                    r[i].s[0] = v.x;
+                    r[i].s[SWN - 1] = v.y;
+                } else r[i].s[0] = Ws[0];
+            } else r[i].s[0] = 0;
+        }
+    };
+    char *const s_sc = smem + 2 * BUF, *const s_mn = s_sc + 2 * SCB;
+    auto stage_part = [&](int chunk, int buf, int w, const Raw (&r)[IPT]) {
+#pragma unroll
+        for (int i = 0; i < IPT; i++) {
+            const int rt = i_t + 4 * i, b = 2 * i_kk + i_h;
+            const bool live = chunk * KB + b < nblocks;     // a block past the end of K contributes nothing
+            half8_t f[F::FR];
+            F::part(r[i].c, r[i].s, i_h, w, f);
+            if constexpr (X1) {
+                const _Float16 d = (_Float16)(live ? F::scale(r[i].s, i_h) : 0.f);      // (an fp16 value: exact)
+#pragma unroll
+                for (int e = 0; e < 8; e++) f[0][e] = f[0][e] * d;
+            }
+            if constexpr (SC == PG_NONE && !X1) if (!live) f[0] = half8_t{};
+#pragma unroll
+            for (int p = 0; p < F::FR; p++)
+                *reinterpret_cast<uint4 *>(smem + buf * BUF + b * PLANE + ((p * RT + rt) * 64 + w * 16 + i_r) * 16) = __builtin_bit_cast(uint4, f[p]);
+            if constexpr (SC != PG_NONE)
+                if (w == 0) *reinterpret_cast<float *>(s_sc + buf * SCB + (b * SCP + rt * 16 + i_r) * 4) = live ? F::scale(r[i].s, i_h) : 0.f;
+            if constexpr (MINS)
+                if (w == 0) *reinterpret_cast<float *>(s_mn + buf * SCB + (b * SCP + rt * 16 + i_r) * 4) = live ? F::least(r[i].s, i_h) : 0.f;
+        }
+    };
+    // activation fragments [block][token tile][hi / lo][lane] x 16 bytes: kernel argument + 32-bit offset, the block part wave-uniform
+    const char *const xsrc = reinterpret_cast<const char *>(P.xf);
+    unsigned xlane[NTW];
+#pragma unroll
+    for (int t = 0; t < NTW; t++) xlane[t] = ((unsigned)min(ttile0 + t, P.nt16 - 1) * 2u * QG_FRAG + (unsigned)lane) * 16u;
+    const unsigned xblock = (unsigned)P.nt16 * 2u * QG_FRAG * 16u;
+    uint4 xh[KB][NTW], xl[KB][NTW];
+    auto xload = [&](int chunk, int b) {
+        const unsigned uo = (unsigned)min(chunk * KB + b, nblocks - 1) * xblock;
+#pragma unroll
+        for (int t = 0; t < NTW; t++) {
+            xh[b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]));
+            if constexpr (!X1) xl[b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]) + QG_FRAG * 16);
+        }
+    };
+    f32x4_t acc[RT][NTW];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int t = 0; t < NTW; t++) acc[rt][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int step = P.ksplit * KW, niter = (nchunks - (int)blockIdx.z * KW + step - 1) / step;     // (every set runs as many chunks; past the end of K: zeros)
+    int chunk = blockIdx.z * KW + kset;
+    Raw rb[2][IPT];                                         // raw weights of the next chunk and of the one after it
+    if (niter > 0) {
+        stage_load(chunk, rb[1]);
+#pragma unroll
+        for (int b = 0; b < KB; b++) xload(chunk, b);
+        stage_load(chunk + step, rb[0]);
+    }
+    // folded RMSNorm, consumer side: 1 / rms of this workgroup's tokens from the producer's partial sums of squares, 256 / TOK threads a token
+    if constexpr (EPI != QG_EPI_PLAIN)
+        if (P.nrm_in.ssq) {
+            constexpr int TPT = 256 / TOK;
+            const int t = tid / TPT, n = min(tok0 + t, P.n_tokens - 1), p0 = tid % TPT;
+            const double *sp = P.nrm_in.ssq + (size_t)n * P.nrm_in.nrb;
+            double tot = 0.0;
+            for (int r0 = p0; r0 < P.nrm_in.nrb; r0 += 8 * TPT) {
+                double v[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = sp[min(r0 + j * TPT, P.nrm_in.nrb - 1)];
+#pragma unroll
+                for (int j = 0; j < 8; j++) tot += r0 + j * TPT < P.nrm_in.nrb ? v[j] : 0.0;
+            }
+#pragma unroll
+            for (int m = 1; m < TPT; m *= 2) tot += __shfl_xor(tot, m);
+            float inv = (float)(1.0 / sqrt(tot / (double)P.nrm_in.dim + (double)P.nrm_in.eps));
+            if (P.nrm_in.scale) {        // the producer's power-of-two pre-scale (norm_prescale, nl_qgemm.h), undone exactly
+                if (rbk == 0 && p0 == 0) P.nrm_in.scale_next[n] = norm_prescale(inv);
+                inv *= 1.0f / P.nrm_in.scale[n];
+            }
+            if (p0 == 0) s_tok[t] = inv;
+        }
+    // producer: what its epilogue needs is requested here, ahead of the K loop -- behind it, every dependent fetch is a round trip of its own
+    constexpr int RQ = ROWS / 4, NIT = TOK * RQ / NTHR, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 ? NIT : 1;
+    [[maybe_unused]] f32x4_t res[NRES];
+    [[maybe_unused]] const bool split = P.ksplit > 1, vec = (P.ldo & 3) == 0;
+    [[maybe_unused]] const float *const resid = split ? nullptr : P.resid;
+    [[maybe_unused]] auto load_res = [&](int i) {
+        const int it = i * NTHR + (int)threadIdx.x, a = it % RQ, n = min(tok0 + it / RQ, P.n_tokens - 1), row = row0 + 4 * a;
+        return resid && vec && row + 3 < P.rows ? *reinterpret_cast<const f32x4_t *>(resid + (size_t)n * P.ldo + row) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    if constexpr (EPI == QG_EPI_PLAIN) {
+        if (NRES == NIT)
+#pragma unroll
+            for (int i = 0; i < NRES; i++) res[i] = load_res(i);
+        if (P.nrm_out.w && !split) {
+            for (int i = threadIdx.x; i < ROWS; i += NTHR) s_gain[i] = P.nrm_out.w[min(row0 + i, P.rows - 1)];
+            for (int i = threadIdx.x; i < TOK; i += NTHR) s_tok[i] = P.nrm_out.scale ? P.nrm_out.scale[min(tok0 + i, P.n_tokens - 1)] : 1.0f;
+        }
+    }
+    if (niter > 0) {
+#pragma unroll
+        for (int w = 0; w < 4; w++) stage_part(chunk, 0, w, rb[1]);
+        stage_load(chunk + 2 * step, rb[1]);
+    }
+    // The K loop is a pipeline of groups (RG row tiles x NTW token tiles: four independent MFMA chains): while group i is on the matrix
+    // cores, group i + 1's weight fragments leave LDS and group i - 1's sums are scaled.  One barrier per chunk, in front of its last
+    // group: the next chunk's fragments are then complete (all parts were stored by block 2) and the last group's are already in
+    // registers, so the buffer that the next chunk's stores will overwrite has no reader left.
+    constexpr int RG = NTW == 1 ? 4 : 2, NG = RT / RG, STEPS = KB * NG;
+    static_assert(STEPS % 2 == 0, "ping-pong");
+    half8_t wf[2][F::FR][RG];
+    f32x4_t z[2][RG][NTW], zc[SC == PG_CHUNK ? RT : 1][NTW], xs[2][NTW];
+    float dv[4][RG], mv[4][RG];         // of groups idx - 1 .. idx + 1
+    auto read_w = [&](int bf, int idx) {
+        const int b = idx / NG, r0 = (idx % NG) * RG;
+#pragma unroll
+        for (int p = 0; p < F::FR; p++)
+#pragma unroll
+            for (int q = 0; q < RG; q++)
+                wf[idx & 1][p][q] = *reinterpret_cast<const half8_t *>(smem + bf * BUF + b * PLANE + (p * RT + r0 + q) * 1024 + lane * 16);
+#pragma unroll
+        for (int q = 0; q < RG; q++) {
+            if constexpr (SC != PG_NONE) dv[idx & 3][q] = *reinterpret_cast<const float *>(s_sc + bf * SCB + (b * SCP + (r0 + q) * 16 + li) * 4);
+            if constexpr (MINS) mv[idx & 3][q] = *reinterpret_cast<const float *>(s_mn + bf * SCB + (b * SCP + (r0 + q) * 16 + li) * 4);
+        }
+    };
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    // the sums of group idx into the accumulators
+    auto scale_sums = [&](int idx) {
+        const int b = idx / NG, g = idx % NG;
+#pragma unroll
+        for (int q = 0; q < RG; q++)
+#pragma unroll
+            for (int t = 0; t < NTW; t++) {
+                const int rt = g * RG + q;
+                if constexpr (SC == PG_BLOCK) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(z[idx & 1][q][t][j], dv[idx & 3][q], acc[rt][t][j]);
+                }
+                if constexpr (MINS) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(-mv[idx & 3][q], xs[b & 1][t][j], acc[rt][t][j]);
+                }
+                if constexpr (SC == PG_CHUNK)
+                    if (b == KB - 1) {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(zc[rt][t][j], dv[idx & 3][q], acc[rt][t][j]);
+                    }
+                asm volatile("" : "+v"(acc[rt][t]));     // (hipcc otherwise sinks the scalings of a chunk below its MFMAs: 4 x the live registers)
+            }
+    };
+    if (niter > 0) {
+        pg_barrier();
+        read_w(0, 0);
+    }
+    // one chunk; PAR: its parity (which buffer and which raw registers)
+    auto do_chunk = [&](auto par_tag) {
+        constexpr int PAR = decltype(par_tag)::value;
+        const int nxt = chunk + step;
+#pragma unroll
+        for (int idx = 0; idx < STEPS; idx++) {
+            const int b = idx / NG, g = idx % NG;
+            if (idx == STEPS - 1) pg_barrier();
+            if (idx + 1 < STEPS) read_w(PAR, idx + 1);
+            else read_w(PAR ^ 1, 0);
+            if constexpr (MINS)
+                if (g == 0) {
+                    const _Float16 one = (_Float16)1.f;
+                    const half8_t ones = {one, one, one, one, one, one, one, one};
+#pragma unroll
+                    for (int t = 0; t < NTW; t++) xs[b & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xl[b][t]), ones, zero, 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < NTW; t++) xs[b & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xh[b][t]), ones, xs[b & 1][t], 0, 0, 0);
+                }
+            auto mul = [&](int p, bool lo, bool start) {
+#pragma unroll
+                for (int q = 0; q < RG; q++)
+#pragma unroll
+                    for (int t = 0; t < NTW; t++) {
+                        const int rt = g * RG + q;
+                        const half8_t x = __builtin_bit_cast(half8_t, lo ? xl[b][t] : xh[b][t]);
+                        if constexpr (SC == PG_BLOCK) z[idx & 1][q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], start ? zero : z[idx & 1][q][t], 0, 0, 0);
+                        else if constexpr (SC == PG_CHUNK) zc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], start && b == 0 ? zero : zc[rt][t], 0, 0, 0);
+                        else acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], acc[rt][t], 0, 0, 0);
+                    }
+            };
+            if constexpr (!X1) mul(0, true, true);
+            if constexpr (F::FR == 2) mul(1, false, false);
+            mul(0, false, X1);
+            if (idx) scale_sums(idx - 1);
+            if (g == NG - 1) {
+                xload(nxt, b);
+                if (b < KB - 1) stage_part(nxt, PAR ^ 1, b, rb[PAR]);
+                if (b == KB - 2) {
+                    stage_part(nxt, PAR ^ 1, KB - 1, rb[PAR]);
+                    stage_load(nxt + 2 * step, rb[PAR]);
+                }
+            }
+        }
+        scale_sums(STEPS - 1);
+        chunk = nxt;
+    };
+    for (int i = 0; i < niter; i += 2) {
+        do_chunk(std::integral_constant<int, 0>{});
+        if (i + 1 < niter) do_chunk(std::integral_constant<int, 1>{});
+    }
+
+    // accumulators -> LDS [token][row], then whole rows of a token
+    __syncthreads();
+    float *const S = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int t = 0; t < NTW; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) S[((wave * NTW + t) * 16 + 4 * lq + j) * LD + rt * 16 + li] = acc[rt][t][j];
+    __syncthreads();
+    const int et = threadIdx.x;
+    const float *const S0 = reinterpret_cast<const float *>(smem_all);
+    float *const SW = reinterpret_cast<float *>(smem_all);
+    auto sum4 = [&](int off) {
+        f32x4_t v = *reinterpret_cast<const f32x4_t *>(S0 + off);
+#pragma unroll
+        for (int k = 1; k < KW; k++) v += *reinterpret_cast<const f32x4_t *>(S0 + k * (SET / 4) + off);
+        return v;
+    };
+    const bool folded_in = EPI != QG_EPI_PLAIN && P.nrm_in.ssq != nullptr;
+
+    if constexpr (EPI == QG_EPI_SWIGLU) {
+        // h = SiLU(gate) * up (go/quant.go:629-631, go/model.go:604-606), stored as the down projection's fragments
+#pragma unroll
+        for (int it0 = 0; it0 < TOK * 4 * (RT / 4); it0 += NTHR) {
+            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % (4 * NTW), hb = (it >> 6) / (4 * NTW), t = tt * 16 + li, n = tok0 + t;
+            const int hblk = tile0 / 2 + hb;
+            if (NTHR > TOK * RT && hb >= RT / 4) break;     // (two sets of wavefronts over 32 rows: the second has no item)
+            int oa, ob;
+            slot_offsets(P.out_q4, w, oa, ob);
+            const int sg = t * LD + hb * 32, su = sg + ROWS / 2;
+            f32x4_t ga = sum4(sg + oa), gb = sum4(sg + ob);
+            f32x4_t ua = sum4(su + oa), ub = sum4(su + ob);
+            if (folded_in) {
+                const float inv = s_tok[t];
+                ga *= inv; gb *= inv; ua *= inv; ub *= inv;
+            }
+            float4 a, b;
+            float *pa = &a.x, *pb = &b.x;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                pa[j] = (ga[j] / (1.0f + exp_f64_as_f32(-ga[j]))) * ua[j];
+                pb[j] = (gb[j] / (1.0f + exp_f64_as_f32(-gb[j]))) * ub[j];
+            }
+            float v[8];
+            slots_from(P.out_q4, a, b, v);
+            if (n < P.n_tokens && hblk * 32 < P.rows) store_frag(P.xf_out, P.nt16, n, hblk, w, v);
+        }
+        return;
+    }
+    if constexpr (EPI == QG_EPI_ROPE) {
+        // RoPE (go/model.go:449-477), attention biases (:525-527), KV store (:552-554): rows 0-7 of a tile hold elements i, rows 8-15
+        // elements i + hd / 2 of one head (ROWMAP_HEADPERM)
+        const QGemmParams::Rope &R = P.rope;
+        const int hd = R.head_dim, half = hd >> 1, tph = hd / 16, nq = R.n_q_heads * hd;
+#pragma unroll 2
+        for (int it0 = 0; it0 < TOK * RT * 2; it0 += NTHR) {
+            const int it = it0 + et, u = it % (RT * 2), t = it / (RT * 2), rt = u >> 1, grp = u & 1, n = tok0 + t, nn = min(n, P.n_tokens - 1);
+            const int tile = min(tile0 + rt, P.ntiles - 1), head = tile / tph, i0 = (tile % tph) * 8 + 4 * grp;
+            const bool is_q = head < R.n_q_heads, is_k = !is_q && head < R.n_q_heads + R.n_kv_heads;
+            const int kvh = head - R.n_q_heads - (is_k ? 0 : R.n_kv_heads);
+            const long long at = R.tkv[nn];       // stream and position, resolved once per token by the embedding launch
+            f32x4_t x0 = sum4(t * LD + rt * 16 + 4 * grp), x1 = sum4(t * LD + rt * 16 + 8 + 4 * grp);
+            if (folded_in) {
+                const float inv = s_tok[t];
+                x0 *= inv; x1 *= inv;
+            }
+            if (R.bias_q) {
+                const float *bp = (is_q ? R.bias_q + head * hd : is_k ? R.bias_k + kvh * hd : R.bias_v + kvh * hd) + i0;
+                x0 += *reinterpret_cast<const f32x4_t *>(bp);
+                x1 += *reinterpret_cast<const f32x4_t *>(bp + half);
+            }
+            f32x4_t o0 = x0, o1 = x1;
+            if (is_q || is_k) {
+                const f32x4_t c = *reinterpret_cast<const f32x4_t *>(R.tcos + (long long)nn * half + i0), s = *reinterpret_cast<const f32x4_t *>(R.tsin + (long long)nn * half + i0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float a0 = x0[j] * c[j], b0 = x1[j] * s[j], a1 = x0[j] * s[j], b1 = x1[j] * c[j];
+                    o0[j] = R.conj ? a0 + b0 : a0 - b0;
+                    o1[j] = R.conj ? b1 - a1 : a1 + b1;
+                }
+            }
+            if (n >= P.n_tokens || tile0 + rt >= P.ntiles) continue;
+            float *dst = is_q ? R.q + ((long long)n * nq + head * hd + i0)
+                              : (is_k ? R.kcache : R.vcache) + (at + (long long)kvh * R.seq_len * hd + i0);
+            *reinterpret_cast<f32x4_t *>(dst) = o0;
+            *reinterpret_cast<f32x4_t *>(dst + half) = o1;
+        }
+        return;
+    }
+    if constexpr (EPI == QG_EPI_PLAIN) {
+        float *const dst = split ? P.part + (long long)blockIdx.z * P.n_tokens * P.ldo : P.out;
+        const float *const bias = split ? nullptr : P.bias;
+        const bool fold = P.nrm_out.w && !split;
+        constexpr int UN = NIT < 8 ? NIT : 8;
+#pragma unroll 1
+        for (int i0 = 0; i0 < NIT; i0 += UN) {
+            f32x4_t v[UN], r[UN];
+#pragma unroll
+            for (int i = 0; i < UN; i++) r[i] = NRES == NIT ? res[i < NRES ? i : 0] : load_res(i0 + i);     // (a round's rows are requested together)
+#pragma unroll
+            for (int i = 0; i < UN; i++) {
+                const int it = (i0 + i) * NTHR + et, a = it % RQ, t = it / RQ, n = tok0 + t, row = row0 + 4 * a;
+                v[i] = sum4(t * LD + 4 * a);
+                const size_t off = (size_t)n * P.ldo + row;
+                if (vec && row + 3 < P.rows) {
+                    if (bias) v[i] += *reinterpret_cast<const f32x4_t *>(bias + row);
+                    if (resid) v[i] += r[i];
+                    if (n < P.n_tokens) *reinterpret_cast<f32x4_t *>(dst + off) = v[i];
+                } else if (n < P.n_tokens) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        if (row + j >= P.rows) continue;
+                        float y = v[i][j] + (bias ? bias[row + j] : 0.f);
+                        if (resid) y += resid[off + j];
+                        dst[off + j] = y;
+                    }
+                }
+                if (fold) {
+                    // folded RMSNorm, producer side (QGemmParams::NormOut): sum of squares of 64 rows of the new residual stream, in
+                    // float64 and a fixed order; the values stay in LDS for the fragments below
+                    *reinterpret_cast<f32x4_t *>(SW + t * LD + 4 * a) = v[i];
+                    double ss = 0.0;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) ss = fma((double)v[i][j], (double)v[i][j], ss);
+#pragma unroll
+                    for (int m = 1; m < 16; m *= 2) ss += __shfl_xor(ss, m);
+                    if ((a & 15) == 0 && n < P.n_tokens && row < P.rows) P.nrm_out.ssq[(size_t)n * (P.rows / 64) + row / 64] = ss;
+                }
+            }
+        }
+        if (!fold) return;
+        __syncthreads();
+#pragma unroll 2
+        for (int it0 = 0; it0 < TOK * 4 * (ROWS / 32); it0 += NTHR) {
+            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % (4 * NTW), kb = (it >> 6) / (4 * NTW), t = tt * 16 + li, n = tok0 + t, c0 = row0 + kb * 32;
+            if (n >= P.n_tokens || c0 >= P.rows) continue;
+            int oa, ob;
+            slot_offsets(P.out_q4, w, oa, ob);
+            const float psc = s_tok[t], *sp = S0 + t * LD + kb * 32, *gp = s_gain + kb * 32;
+            const f32x4_t ya = (*reinterpret_cast<const f32x4_t *>(sp + oa) * *reinterpret_cast<const f32x4_t *>(gp + oa)) * psc;
+            const f32x4_t yb = (*reinterpret_cast<const f32x4_t *>(sp + ob) * *reinterpret_cast<const f32x4_t *>(gp + ob)) * psc;
+            float v[8];
+            slots_from(P.out_q4, make_float4(ya[0], ya[1], ya[2], ya[3]), make_float4(yb[0], yb[1], yb[2], yb[3]), v);
+            store_frag(P.nrm_out.xf, P.nt16, n, c0 / 32, w, v);
+        }
+    }
+}
+
+template <int WT, int EPI, bool X1>
+hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
+    auto go = [&](auto rt, auto ntw, auto kw) {
+        constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT;
+        const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + 64 * NTW - 1) / (64 * NTW));
+        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, X1>), dim3((total + 7) / 8 * 8, 1, P.ksplit), dim3(256 * KW), 0, st, P);
+        return hipGetLastError();
+    };
+    using std::integral_constant;
+    const integral_constant<int, 1> one{};
+    const integral_constant<int, 2> two{};
+    const integral_constant<int, 4> four{};
+    const integral_constant<int, 8> eight{};
+    // Tiles by how many 64 x 64 ones there are.  Up to one per compute unit: eight wavefronts on each (K dealt to two sets), since the four
+    // of one set leave every SIMD waiting on its own wavefront's instructions (Q4_0 768 x 2048 x 333 tokens, 72 tiles: 14.8 us one set,
+    // 11.6 two; 64 x 128 tiles 20.3).  Up to two: 64 x 128 tiles of two sets (768 x 2048 x 2047: 17.7 us against 20.9 for 64 x 64, 22.0
+    // for it with two sets).  Beyond, one set, and tiles that grow as the grid allows it (Q4_0 4096 x 768 x 2047, gate and up: 128 x 128
+    // 31.8 us, 64 x 128 35.0, 64 x 64 37.0; Q8_0's and the K-quants' expansions leave no registers for 128 x 128: 68.9 us against 62.2).
+    const long long tiles = (long long)((P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4) * ((P.n_tokens + 63) / 64) * P.ksplit;
+    if (tiles <= 256) return go(four, one, two);
+    if (tiles <= 512) return go(four, two, two);
+    if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one);
+    if constexpr (WT == WT_Q4_0 || WT == WT_F16)
+        if (tiles >= 1792) return go(eight, two, one);
+    return go(four, two, one);
+}
+template <int EPI>
+hipError_t pg_launch(int wtype, const QGemmParams &P, hipStream_t st) {
+    switch (wtype) {
+    case WT_Q4_0: return P.x1 ? pg_launch_as<WT_Q4_0, EPI, true>(P, st) : pg_launch_as<WT_Q4_0, EPI, false>(P, st);
+    case WT_Q8_0: return pg_launch_as<WT_Q8_0, EPI, false>(P, st);
+    case WT_F16: return pg_launch_as<WT_F16, EPI, false>(P, st);
+    case WT_Q4_K: return pg_launch_as<WT_Q4_K, EPI, false>(P, st);
+    case WT_Q6_K: return pg_launch_as<WT_Q6_K, EPI, false>(P, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace nl

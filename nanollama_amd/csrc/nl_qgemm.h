@@ -45,7 +45,7 @@ struct QGemmParams {
     int rows, cols, npairs, ntiles;
     const uint4 *xf;     // activation fragments
     int nt16, n_tokens;
-    int x1;              // prompt precision mode fp16x1 (qgemm2_kernel): only the hi half of every activation is multiplied
+    int x1;              // prompt precision mode fp16x1 (pgemm_kernel, Q4_0): only the hi half of every activation is multiplied
     float *out;          // [N][ldo]
     int ldo;
     const float *resid;  // optional [N][ldo]: out = resid + y
@@ -77,7 +77,7 @@ struct QGemmParams {
         const float *tcos, *tsin;            // [N][hd/2]
         const long long *tkv;                // [N]
     } rope;
-    // RMSNorm (go/quant.go:597-607) folded around the GEMMs of a prompt (nl_qgemm2.h).  A producer -- WO or down with
+    // RMSNorm (go/quant.go:597-607) folded around the GEMMs of a prompt (nl_pgemm.h).  A producer -- WO or down with
     // the plain epilogue, unsplit, so its lanes hold finished rows of the new residual stream -- also emits those rows
     // as the NEXT GEMM's fragments, multiplied by that GEMM's norm weights but not yet by 1 / rms, plus one float64
     // sum of squares per (token, 64-row block).  The consumer (Q|K|V with the RoPE epilogue, gate || up with the
@@ -88,7 +88,7 @@ struct QGemmParams {
         uint4 *xf;           // fragment store the consumer reads
         double *ssq;         // [n_tokens][rows / 64]
         const float *scale;  // [n_tokens] exact power of two the fragments are multiplied by (norm_prescale below); nullptr = 1
-    } nrm_out;               // (the consumer is a Q4_0 GEMM of nl_qgemm2.h: Q4_0 k-slot order)
+    } nrm_out;               // (k-slot order of the consumer's weight type: out_q4)
     struct NormIn {
         const double *ssq;   // nullptr = the input fragments are already normalised
         int nrb;             // partial sums per token (dim / 64)

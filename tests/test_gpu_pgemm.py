@@ -1,0 +1,84 @@
+"""GPU: the multi-token GEMM of long token runs and of K-quant files (nl_pgemm.h) at the edges of its tiles, tilings and formats."""
+import numpy as np
+import pytest
+
+from dataclasses import replace
+
+from nanollama_amd import gguf, quant, synth
+
+pytestmark = pytest.mark.gpu
+
+LOGIT_TOL = 1e-4
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from nanollama_amd import model
+    return model
+
+
+@pytest.fixture(scope="module")
+def orc():
+    from oracle import oracle
+    return oracle
+
+
+def _decoded(raw, t, rows, cols):
+    if t == gguf.GGML_F16:
+        return raw.view(np.float16).astype(np.float64).reshape(rows, cols)
+    b = raw.reshape(-1, 34 if t == gguf.GGML_Q8_0 else 18)
+    d, q = b[:, :2].copy().view(np.float16).astype(np.float64), b[:, 2:]
+    n = q.view(np.int8).astype(np.float64) if t == gguf.GGML_Q8_0 else np.concatenate([(q & 15), (q >> 4)], 1).astype(np.float64) - 8
+    return (n * d).reshape(rows, cols)
+
+
+# tokens and rows that leave ragged tiles, K of whole and of partial 128-column chunks, and 64 x 64 tile counts on every side of the rules:
+# <= 256, <= 512, < 1024, above, >= 1792
+@pytest.mark.parametrize("rows,cols,n", [(16, 512, 65), (80, 544, 127), (272, 576, 129), (1040, 640, 1000), (2064, 512, 1000), (2320, 544, 1801), (4112, 544, 1801)])
+@pytest.mark.parametrize("kind", ["q4_0", "q8_0", "f16"])
+def test_product_against_float64(hip, kind, rows, cols, n):
+    t = synth.WTYPES[kind]
+    rng = np.random.default_rng(rows + n)
+    w, x = rng.standard_normal((rows, cols)).astype(np.float32), rng.standard_normal((n, cols)).astype(np.float32)
+    raw = quant.encode(w, t)
+    wd, xd = _decoded(raw, t, rows, cols), x.astype(np.float64)
+    got = hip.op_matmul_batch(raw, t, x, rows, cols)
+    # x = hi + lo leaves 2^-22 of an element; 32 products and a scaling per block, cols / 32 block sums, each rounded to 2^-24
+    bound = (2.0 ** -22 + (cols / 32 + 34) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T)
+    assert (np.abs(got - xd @ wd.T) <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("n", [3, 16, 64, 65, 200])
+def test_kquant_prompt_against_oracle(hip, orc, tmp_path, kind, n):
+    # every matrix's epilogue (RoPE + KV store, residual + folded norm, SwiGLU) on super-block weights, in two calls: positions > 0
+    shape = replace(synth.TIERS["tiny"], name=f"k_{kind}", dim=512, n_head=8, n_kv_head=2, interm=768, seq_len=256, n_layer=3)
+    p = tmp_path / "k.gguf"
+    synth.generate_gguf(str(p), shape, kind, 23)
+    g = gguf.load_gguf(str(p))
+    toks = synth.prompt_ids(n, shape.vocab, seed=3)
+    ref, dev = orc.OracleModel(g), hip.load_llama_model(g)
+    for pos, tok in enumerate(toks):
+        want = ref.forward(tok, pos)
+    if n > 100:
+        dev.prefill(toks[:37], want_logits=False)
+    dev.prefill(toks[37 if n > 100 else 0:], 37 if n > 100 else 0)
+    assert np.abs(dev.state.logits - want).max() <= LOGIT_TOL * max(1.0, float(want.std()))
+    dev.close()
+
+
+def test_kquant_streams_equal_the_single_token_plan(hip, tmp_path):
+    # decode streams side by side against one forward call each
+    shape = replace(synth.TIERS["tiny"], name="k_streams", dim=256, n_head=4, n_kv_head=2, interm=512, seq_len=64)
+    p = tmp_path / "s.gguf"
+    synth.generate_gguf(str(p), shape, "q4_k", 29)
+    g = gguf.load_gguf(str(p))
+    dev = hip.load_llama_model(g, max_streams=5)
+    for s in range(5):
+        for pos in range(s + 1):
+            dev.forward(7 + s + pos, pos, s)
+    _, rows = dev.forward_batch(list(range(5)), [30, 31, 32, 33, 34], [1, 2, 3, 4, 5], want_logits=True)
+    for s in range(5):
+        dev.forward(30 + s, s + 1, s)
+        assert np.abs(rows[s] - dev.state.logits).max() <= LOGIT_TOL * max(1.0, float(dev.state.logits.std()))
+    dev.close()

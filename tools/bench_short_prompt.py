@@ -1,4 +1,4 @@
-"""Developer tool: prefill time of short prompts (n tokens, one stream) on a tier -- the multi-token step below qgemm2's 128 tokens.
+"""Developer tool: prefill time of short prompts (n tokens, one stream) on a tier -- the multi-token step below pgemm's 128 tokens.
 python tools/bench_short_prompt.py mini q4_0 24 48 64 100 127"""
 import os, sys, time
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))

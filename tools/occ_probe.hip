@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdio>
 #include "nl_batch.h"
-#include "nl_qgemm2.h"
+#include "nl_pgemm.h"
 using namespace nl;
 #define CK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { printf("%s -> %s\n", #x, hipGetErrorString(e_)); return 1; } } while (0)
 
@@ -27,8 +27,6 @@ int main() {
     int n = 0;
     CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_tile16_kernel<64, 4, 32>, 512, 0)); printf("attn_tile16_kernel<64,4,32>  512 threads, 72192 B LDS: %d blocks per CU (API)\n", n);
     CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_tile16_kernel<64, 1, 128>, 512, 0)); printf("attn_tile16_kernel<64,1,128>: %d blocks per CU (API)\n", n);
-    CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, qgemm2_kernel<WT_Q4_0, 4, 2, 8, QG_EPI_SWIGLU>, 512, 0)); printf("qgemm2<4,2,8,swiglu>: %d blocks per CU (API)\n", n);
-    CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, qgemm2_kernel<WT_Q4_0, 4, 1, 4, QG_EPI_PLAIN>, 256, 0)); printf("qgemm2<4,1,4,plain>: %d blocks per CU (API)\n", n);
     int *d; CK(hipMalloc(&d, 16));
     auto run = [&](const char *what, auto kernel, int threads) {
         hipMemset(d, 0, 16);
