@@ -270,7 +270,7 @@ struct nl_engine {
     u32x4 *tp_xq = nullptr;       // 16-byte granules of the two-launch layer (nl_tp.h): q | k | v tiles of a kv group,
     u32x4 *tp_xo = nullptr;       //   the heads' attention outputs,
     u32x4 *tp_xp = nullptr;       //   the helper blocks' pass records (long contexts on one GPU),
-    bool attn_helpers = false;    //   ... when the launch's geometry has three helpers for every head (NL_ATTN_HELPERS=0: off)
+    int attn_helpers = 0;         //   ... (TpAttnParams::helpers) when the launch's geometry has three helpers for every head (NL_ATTN_HELPERS=0: off)
     u32x4 *tp_hx = nullptr;       //   g | u (or h) tiles of the feed-forward half
     int grp_tpm = 1;              // mode 2: 16-row tiles per workgroup
     bool grp_grid_fits = false;   // modes 3 / 4: the projection grid (incl. its blocks without a tile, which stay) fits the compute units
@@ -804,7 +804,7 @@ void build_plan(nl_engine *e, std::vector<Op> &plan, bool fused, bool help = fal
         Q.wo_q = L.wo.q; Q.wo_s = L.wo.s; Q.wo_npairs = L.wo.npairs; Q.wo_ntiles = L.wo.ntiles; Q.wo_gshift = e->tpg.wo_gshift;
         Q.wo_tpw = e->tpg.wo_tpw;
         Q.n_heads_local = e->Hs; Q.xq = e->tp_xq; Q.xo = e->tp_xo; Q.bias_out = L.bo; Q.x = e->x[cur];
-        Q.xp = e->tp_xp; Q.helpers = (help && e->attn_helpers) ? 1 : 0; Q.live_grid = grp_grid(e->KVs, B.members);
+        Q.xp = e->tp_xp; Q.helpers = help ? e->attn_helpers : 0; Q.live_grid = grp_grid(e->KVs, B.members);
         Q.seam = sm;
         const bool mfa = e->mf_attn;
         if (mfa) { B.qkv_q = L.qkv.q2; B.qkv_s = L.qkv.s2; }       // (WO stays on the vector pipe: nl_tp.h)
@@ -2947,9 +2947,15 @@ int nl_finalize(nl_handle e) {
             const int members = (e->gqa + 2) * 4 / e->grp_tpm, lgrid = grp_grid(e->KVs, members);
             const int grid4 = std::max(lgrid, (e->layers[0].wo.ntiles + e->tpg.wo_tpw - 1) / e->tpg.wo_tpw);
             const char *hk = getenv("NL_ATTN_HELPERS");
-            e->attn_helpers = e->fused_mode == 4 && !(hk && atoi(hk) == 0) && !c.qk_norm && members - e->gqa >= 2 * e->gqa && grid4 - lgrid >= e->Hs &&
-                              e->layers[0].qkv.wtype == WT_Q4_0;      // (the Q8_0 variant of that launch does not fit 128 registers: 278 spilled)
+            const bool helpers_ok = e->fused_mode == 4 && !(hk && atoi(hk) == 0) && !c.qk_norm && e->layers[0].qkv.wtype == WT_Q4_0;      // (Q8_0: 20 registers too many)
+            e->attn_helpers = !helpers_ok ? 0 : members - e->gqa >= 2 * e->gqa && grid4 - lgrid >= e->Hs ? 1 : c.dim >= 1280 && members - e->gqa >= 3 * e->gqa ? 2 : 0;
             if (!fm && e->attn_helpers && e->wide_ffn) e->fused_max_pos = 2 * TP_NCH_MAX * TP_PASS;
+            // helpers of the kv group, feed-forward in two launches (841M Q4_0): one pass each up to position 1024, 719 against 758 us a token
+            // on the general plan (alone: 772 at 500, 822 at 700); two passes each fall behind, 830 against 793
+            else if (!fm && e->attn_helpers == 2) e->fused_max_pos = TP_NCH_MAX * TP_PASS;
+            // Q8_0 (no helpers): one runner's passes against the general plan's split attention, 841M tier (feed-forward in two launches):
+            // 754 against 784 us a token at position 200, 822 against 787 at 300; 4096 columns: 264 against 270 at 700, 275 against 271 at 800
+            if (!fm && e->fused_mode == 4 && e->layers[0].qkv.wtype == WT_Q8_0) e->fused_max_pos = e->wide_ffn ? 3 * TP_PASS : TP_PASS;
         }
         if (e->fused_mode == 3 || e->fused_mode == 4)      // passes a head takes inside the launch
             e->fused_max_pos = std::min(e->fused_max_pos, (e->attn_helpers ? 2 : 1) * TP_NCH_MAX * TP_PASS);

@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(GRP_THREADS) qkv_attn_kernel(GroupParams P) {
         xa.x *= gv[f].x; xa.y *= gv[f].y; xa.z *= gv[f].z; xa.w *= gv[f].w;
         *reinterpret_cast<float4 *>(xw + (lane >> 4) * XS_PAIR + (lane & 15) * 4) = xa;
         __builtin_amdgcn_wave_barrier();
-        const float a1 = PairDot<WT>::run(cw[f], sw[f], xw + k * XS_PAIR, acc);
+        const float a1 = pair_dot_lean<WT>(cw[f], sw[f], xw + k * XS_PAIR, acc);
         acc = lv[f] ? a1 : acc;
         __builtin_amdgcn_wave_barrier();
     }

@@ -274,17 +274,23 @@ template <int WT> struct PairDot;
 
 template <> struct PairDot<WT_Q8_0> {
     // out = sum_b d_b * sum_j q_bj x_j  (go/quant.go:149-165)
+    // LEAN: x leaves LDS sixteen values at a time.  hipcc otherwise requests all 64 ahead of the weights' wait, and the fused launches of nl_tp.h,
+    // which hold their next weights and cache rows in 128 registers, spilled 115 to 228 of them: a token of the 841M tier took 1120 us, now
+    // 734 (general plan: 735); 4096 columns 535, now 233 (258).
+    template <bool LEAN = false>
     static __device__ __forceinline__ float run(const uint4 *c, uint2 sc2, const float *xp, float acc) {
         const uint32_t sc = sc2.x;
         const float4 *x4 = reinterpret_cast<const float4 *>(xp);
 #pragma unroll
         for (int b = 0; b < 2; b++) {
+            if (LEAN) asm volatile("" : "+v"(acc)::"memory");
             Acc4 s{0.f, 0.f, 0.f, 0.f};
             uint4 lo = c[2 * b], hi = c[2 * b + 1];
             dot4_i8(lo.x, x4[8 * b + 0], s);
             dot4_i8(lo.y, x4[8 * b + 1], s);
             dot4_i8(lo.z, x4[8 * b + 2], s);
             dot4_i8(lo.w, x4[8 * b + 3], s);
+            if (LEAN) asm volatile("" : "+v"(s.a)::"memory");
             dot4_i8(hi.x, x4[8 * b + 4], s);
             dot4_i8(hi.y, x4[8 * b + 5], s);
             dot4_i8(hi.z, x4[8 * b + 6], s);
@@ -484,6 +490,12 @@ template <> struct PairDot<WT_Q6_K> {
         return acc;
     }
 };
+
+template <int WT>
+__device__ __forceinline__ float pair_dot_lean(const uint4 *c, uint2 sc, const float *xp, float acc) {
+    if constexpr (WT == WT_Q8_0) return PairDot<WT>::template run<true>(c, sc, xp, acc);
+    else return PairDot<WT>::run(c, sc, xp, acc);
+}
 
 // ------------------------------------------------------------------ GEMV ---
 

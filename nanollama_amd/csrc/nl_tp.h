@@ -375,7 +375,8 @@ struct TpAttnParams {
     float *x;                    // residual stream, read at entry (RMSNorm input, owner rows) and rewritten by the owners
     TpSeam seam;
     u32x4 *xp;                   // [Hs][3][22] granules: a helper block's (max, sum, sum p v[64]) record of ONE attention pass, for the head's runner
-    int helpers;                 // 1: from the second 256-position pass on, the passes below the last run on three blocks that are not runners
+    int helpers;                 // from the second 256-position pass on, the passes below the last run on three blocks that are not runners:
+                                 // 2: all of the head's kv group, 1: two of it and one past the kv groups
     int live_grid;               // blocks [0, live_grid) belong to kv groups (grp_grid); the rest only multiply WO rows -- and help
     PfTiles pf;                  // round 0 of the feed-forward launch behind this one (gate, up tiles b of block b); nmat 0 = off
     PfTiles pf2;                 // the NEXT layer's projection tiles, for the memory-side Infinity Cache to keep (NL_PREFETCH bit 16; measured
@@ -492,16 +493,16 @@ __device__ __forceinline__ void tp_attn_body(const TpAttnParams &Q, char *smem, 
     const int kr = lane >> 2, kq = lane & 3, vg = lane >> 4, vc = lane & 15;
     float4 kreg[NV], vreg[NV], kregn[NV];
     // Attention passes are shared once there is more than one (go/model.go:557-587 over 256 positions per pass): the runner of a
-    // head keeps the LAST pass (the one that holds this position); pass nch - 1 - p goes to helper p = 1 .. 3 -- the two blocks of
-    // the head's own kv group that hold k / v tiles or none (mem >= G: same XCD as the runner) and one of the blocks past the kv
-    // groups.  A helper gathers the head's q itself and hands ONE record (max, sum, sum p v[64]) to the runner.
+    // head keeps the LAST pass (the one that holds this position); pass nch - 1 - p goes to helper p = 1 .. 3 -- two blocks of
+    // the head's own kv group that hold k / v tiles or none (mem >= G: same XCD as the runner) and a third one of them (helpers == 2:
+    // the group has as many) or one of the blocks past the kv groups.  A helper gathers the head's q itself and hands ONE record (max, sum, sum p v[64]) to the runner.
     const int nch = min(pos / TP_PASS + 1, (HELP && Q.helpers) ? 2 * TP_NCH_MAX : TP_NCH_MAX);
     const bool shared = HELP && Q.helpers && nch > 1;       // (HELP: the launch plan of positions from the second pass on -- the plan
                                                             //  of the first pass is compiled without any of this)
     int hhead = -1, hpart = 0;            // this block as a helper
     if (!RUNNER && shared) {
-        if (LIVE) { const int j = mem - G; hpart = 1 + j / G; hhead = hpart <= 2 ? cl * G + (j - (hpart - 1) * G) : -1; }
-        else { const int j = (int)blockIdx.x - Q.live_grid; hpart = 3; hhead = (j >= 0 && j < Q.n_heads_local) ? j : -1; }
+        if (LIVE) { const int j = mem - G; hpart = 1 + j / G; hhead = hpart <= (Q.helpers == 2 ? 3 : 2) ? cl * G + (j - (hpart - 1) * G) : -1; }
+        else if (Q.helpers == 1) { const int j = (int)blockIdx.x - Q.live_grid; hpart = 3; hhead = (j >= 0 && j < Q.n_heads_local) ? j : -1; }
     }
     // part p (0 = the runner) takes the passes [nch - (p + 1) per, nch - p per), per = ceil(nch / 4): contiguous, the last ones the runner's
     const int per = shared ? (nch + 3) >> 2 : nch;
@@ -586,7 +587,7 @@ __device__ __forceinline__ void tp_attn_body(const TpAttnParams &Q, char *smem, 
             if (!MF) {
                 *reinterpret_cast<float4 *>(xw + (lane >> 4) * XS_PAIR + (lane & 15) * 4) = xa;
                 __builtin_amdgcn_wave_barrier();
-                const float a1 = PairDot<WT>::run(cw[f], sw[f], xw + k * XS_PAIR, acc);
+                const float a1 = pair_dot_lean<WT>(cw[f], sw[f], xw + k * XS_PAIR, acc);
                 acc = lv[f] ? a1 : acc;
                 __builtin_amdgcn_wave_barrier();
             } else if (f == slot) {
@@ -802,7 +803,7 @@ __device__ __forceinline__ void tp_attn_body(const TpAttnParams &Q, char *smem, 
     __syncthreads();
     TP_STAMP(sslot, 8);
     if (wslot < tpw) {      // (on the vector pipe in every mode: the heads' outputs serve one tile, their digit image would cost what it saves)
-        const float a1 = PairDot<WT>::run(wc, wsc, ao + min(wgg * KL + k, Q.wo_npairs - 1) * XS_PAIR, 0.f);
+        const float a1 = pair_dot_lean<WT>(wc, wsc, ao + min(wgg * KL + k, Q.wo_npairs - 1) * XS_PAIR, 0.f);
         float a = wlv ? a1 : 0.f;
         a = quad_sum(a);
         if (k == 0) red2[wave * TR + r] = a;
@@ -963,7 +964,7 @@ __device__ __forceinline__ void tp_ffn_body(const TpFfnParams &P, char *smem) {
             xa.x *= gv[f].x; xa.y *= gv[f].y; xa.z *= gv[f].z; xa.w *= gv[f].w;
             *reinterpret_cast<float4 *>(xw + (lane >> 4) * XS_PAIR + (lane & 15) * 4) = xa;
             __builtin_amdgcn_wave_barrier();
-            const float a1 = PairDot<WT>::run(cw[f], sw[f], xw + k * XS_PAIR, acc);
+            const float a1 = pair_dot_lean<WT>(cw[f], sw[f], xw + k * XS_PAIR, acc);
             acc = lv[f] ? a1 : acc;
             __builtin_amdgcn_wave_barrier();
         }
@@ -1011,7 +1012,7 @@ __device__ __forceinline__ void tp_ffn_body(const TpFfnParams &P, char *smem) {
     float acc = 0.f;
 #pragma unroll
     for (int j = 0; j < NGC; j++) {
-        const float a1 = PairDot<WT>::run(dw[j], dsw[j], hs + gsel[j] * XS_PAIR, acc);
+        const float a1 = pair_dot_lean<WT>(dw[j], dsw[j], hs + gsel[j] * XS_PAIR, acc);
         acc = dlv[j] ? a1 : acc;
     }
     acc = quad_sum(acc);
@@ -1194,7 +1195,7 @@ __global__ void __launch_bounds__(TP_THREADS) wide_ffn_kernel(WideFfnParams P) {
 #pragma unroll
         for (int f = 0; f < NF; f++) {
             if (!MF) {
-                const float a1 = PairDot<WT>::run(cw[f], sw[f], xw + f * XS_WAVE + k * XS_PAIR, acc);
+                const float a1 = pair_dot_lean<WT>(cw[f], sw[f], xw + f * XS_WAVE + k * XS_PAIR, acc);
                 acc = lv[f] ? a1 : acc;
             } else {
                 const unsigned char *img = reinterpret_cast<const unsigned char *>(xw + f * XS_WAVE);
@@ -1316,7 +1317,7 @@ __global__ void __launch_bounds__(TP_THREADS) wide_ffn_kernel(WideFfnParams P) {
 #pragma unroll
     for (int j = 0; j < NGC; j++) {
         if (!MF) {
-            const float a1 = PairDot<WT>::run(dw[j], dsw[j], hs + gsel[j] * XS_PAIR, acc);
+            const float a1 = pair_dot_lean<WT>(dw[j], dsw[j], hs + gsel[j] * XS_PAIR, acc);
             acc = dlv[j] ? a1 : acc;
         } else {
             const int b0 = dgg[j] * 8 + (lane >> 4);
