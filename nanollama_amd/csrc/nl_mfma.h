@@ -423,6 +423,34 @@ struct MatParams {
     // one token: every row tile's largest result and its row, for the argmax that follows (or null)
     float *amax_val;
     int *amax_idx;
+    // few_kernel: the norm between a residual product and the next one, without a launch (48 streams, 768 columns: two launches of 4.2 us a
+    // layer; gate and up takes 0.7 us for it, the projections 0.3.  A prompt's products lose what its norms cost, 2 - 3 us each: not there).
+    // ST_RESID with fw: the new rows times the next norm's gains also go to the operand fx, and their sums of squares per row tile to
+    // fss [row tile][fss_ld tokens].  ST_F32 / ST_GATED with nss (nss_n row tiles): the results are multiplied by 1 / rms before bias and
+    // activation.
+    void *fx;
+    const float *fw;
+    float *fss;
+    int fx_nks, fss_ld;
+    const float *nss;
+    int nss_n;
+};
+
+// a folded norm's partial sums of one token: row tiles from, from + step, ...; the first NB of them are requested by first() and added by sum()
+template <int NB>
+struct PartialSums {
+    float v[NB];
+    __device__ __forceinline__ void first(const MatParams &P, int tok, int from, int step) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) v[j] = P.nss[(long long)min(from + j * step, P.nss_n - 1) * P.fss_ld + tok];
+    }
+    __device__ __forceinline__ float sum(const MatParams &P, int tok, int from, int step) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < NB; j++) ss += from + j * step < P.nss_n ? v[j] : 0.f;
+        for (int k = from + NB * step; k < P.nss_n; k += step) ss += P.nss[(long long)k * P.fss_ld + tok];
+        return ss;
+    }
 };
 
 __device__ __forceinline__ void store_rows(float *out, int ldo, int rows, int tok, int row, f32x4 v) {
@@ -441,6 +469,22 @@ __device__ __forceinline__ void add_rows(float *out, const float *add2, int ldo,
     } else
         for (int i = 0; i < 4; i++)
             if (row + i < rows) out[at + i] = out[at + i] + v[i] + (add2 ? add2[at + i] : 0.f);
+}
+// ... with the next norm folded (whole row tiles, P.ldo in vectors: the host checks it where fw is set); the four lanes of a token call together
+template <typename T>
+__device__ __forceinline__ void add_rows_folded(const MatParams &P, int tok, int rt, int g, f32x4 v) {
+    const int row = rt * 16 + 4 * g;
+    const long long at = (long long)min(tok, P.n_tokens - 1) * P.ldo + row;
+    v += *reinterpret_cast<const f32x4 *>(P.out + at);
+    if (P.add2) v += *reinterpret_cast<const f32x4 *>(P.add2 + at);
+    if (tok < P.n_tokens) {
+        *reinterpret_cast<f32x4 *>(P.out + at) = v;
+        put4(reinterpret_cast<T *>(P.fx) + op_index(tok, row, P.fx_nks), v * *reinterpret_cast<const f32x4 *>(P.fw + row));
+    }
+    float ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if (g == 0 && tok < P.n_tokens) P.fss[(long long)rt * P.fss_ld + tok] = ss;
 }
 // four consecutive feed-forward rows f16 * 16 + 4 g .. + 3 of one token
 template <typename T>
@@ -650,6 +694,13 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
             }
         }
     };
+    // a folded norm's consumer: the partial sums of its tokens, requested ahead of the weights and added behind them
+    [[maybe_unused]] float inv = 1.f;
+    constexpr bool SCALED = !NORM && (EPI == ST_F32 || EPI == ST_GATED);
+    [[maybe_unused]] PartialSums<SCALED ? 12 : 1> parts;
+    [[maybe_unused]] const int ptok = min(tt0 * 16 + tid % (NT * 16), n - 1), pfrom = tid / (NT * 16), pstep = WV * 64 / (NT * 16);
+    if constexpr (SCALED)
+        if (P.nss) parts.first(P, ptok, pfrom, pstep);
     load(w);
     T *xs = reinterpret_cast<T *>(lds);                    // NORM: [nks][4][n][8]
     if constexpr (NORM) {
@@ -718,6 +769,20 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
                 for (int r = 0; r < RB; r++) acc[r][t] = mma(a[r][u], b[u][t], acc[r][t]);
         }
     }
+    if constexpr (SCALED)
+        if (P.nss) {                                       // (every thread ends up with its epilogue token's 1 / rms)
+            float nsum = parts.sum(P, ptok, pfrom, pstep);
+            float *const s = reinterpret_cast<float *>(lds);       // [WV][NT * 16]
+#pragma unroll
+            for (int o = NT * 16; o < 64; o <<= 1) nsum += __shfl_xor(nsum, o);
+            if (lane < NT * 16) s[w * NT * 16 + lane] = nsum;
+            lds_barrier();
+            nsum = 0.f;
+#pragma unroll
+            for (int q = 0; q < WV; q++) nsum += s[q * NT * 16 + min(tid >> 6, NT - 1) * 16 + col];
+            inv = rsqrt_f32(nsum / (float)P.ndim + P.neps);
+            lds_barrier();
+        }
     // the wavefronts' partial tiles meet in LDS
     if constexpr (NORM) lds_barrier();                   // (the area held the norm)
     f32x4 *red = reinterpret_cast<f32x4 *>(lds);           // [WV][RB * NT][64]
@@ -733,6 +798,16 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
         for (int q = 0; q < WV; q++)
 #pragma unroll
             for (int r = 0; r < RB; r++) v[r] += red[(q * RB * NT + r * NT + t) * 64 + l];
+        if constexpr (SCALED) {
+            static_assert(NT <= WV, "an epilogue token per thread");
+#pragma unroll
+            for (int r = 0; r < RB; r++) v[r] *= inv;
+        }
+        if constexpr (EPI == ST_RESID)
+            if (P.fw) {
+                add_rows_folded<T>(P, tok, rt, l >> 4, v[0]);
+                continue;
+            }
         if (EPI == ST_F32 && NT == 1 && P.amax_val) {      // one token: rows of column 0, four lanes with four rows each
             float best = -INFINITY;
             int idx = 0x7fffffff;

@@ -91,6 +91,9 @@ struct nl_engine {
     // norms behind the sublayers: a second stream buffer and the last sublayer's result, which the next norm of the stream takes in
     float *x2 = nullptr, *delta = nullptr, *xcur = nullptr;
     const float *pend = nullptr; // the norm's factor, null: nothing pending
+    // no norms behind the sublayers: the last residual product left the next norm's input in h and its sums of squares here (MatParams::fw)
+    bool folded = false;
+    float *fss = nullptr;        // [row tile of the width][tokens]
     // latent attention: operand of the absorbed product, split results, expanded keys and values of kv_slots positions
     void *xq = nullptr, *ek = nullptr, *ev = nullptr;
     float *lpart = nullptr, *lml = nullptr;
@@ -356,6 +359,9 @@ hipError_t normed_product(nl_engine *e, MatParams P, const float *nw, const int 
     if (!rows && few_norm_ok(P.n_tokens, P.nks, e->c.dim, e->c.dim)) {
         P.nx = e->xcur; P.nw = nw; P.nd = e->delta; P.ndw = e->pend; P.nxo = keep; P.ndim = e->c.dim;
         s = launch_product<T, EPI>(P, e->stream, norm);
+    } else if (e->folded && !rows) {
+        P.X = e->h; P.nss = e->fss; P.nss_n = 2 * e->nksd; P.fss_ld = FEW_MAX_TOKENS; P.ndim = e->c.dim;
+        s = launch_product<T, EPI>(P, e->stream);
     } else {
         NormParams N{};
         N.x = e->xcur; N.w = nw; N.rows = rows; N.out = e->h; N.dim = e->c.dim; N.nks = e->nksd; N.n_tokens = P.n_tokens; N.eps = e->c.eps;
@@ -369,12 +375,16 @@ hipError_t normed_product(nl_engine *e, MatParams P, const float *nw, const int 
 }
 
 // a sublayer's last product: into the stream, or kept for the norm behind it
+// next: the gains of the norm that the stream meets next, where its product can take them folded (MatParams::fw)
 template <typename T>
-hipError_t residual_product(nl_engine *e, const Mat &m, const void *X, int n, const float *bias, const float *post, const float *behind) {
+hipError_t residual_product(nl_engine *e, const Mat &m, const void *X, int n, const float *bias, const float *post, const float *behind, const float *next) {
     MatParams P = product_params(e, m, X, n);
     P.ldo = e->c.dim;
     if (!post) {
         P.out = e->xcur; P.add2 = behind;
+        // (up to a few tokens the norm costs nothing: the product behind it computes it in its prologue)
+        e->folded = next && n <= FEW_MAX_TOKENS && (e->c.dim & 31) == 0 && m.nrt == 2 * e->nksd && !few_norm_ok(n, e->nksd, e->c.dim, e->c.dim);
+        if (e->folded) { P.fw = next; P.fx = e->h; P.fx_nks = e->nksd; P.fss = e->fss; P.fss_ld = FEW_MAX_TOKENS; }
         return launch_product<T, ST_RESID>(P, e->stream);
     }
     P.out = e->delta; P.bias = bias;
@@ -455,6 +465,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
     LookupParams E{};
     e->xcur = e->x;
     e->pend = nullptr;
+    e->folded = false;
     E.table = e->embed.w; E.tok = s.tok; E.nks = e->nksd; E.dim = D; E.scale = e->c.embed_scale; E.x = e->x; E.x0 = e->x0;
     hipLaunchKernelGGL(lookup_kernel<T>, dim3(s.n), dim3(256), 0, st, E);
     for (size_t r = 0; r < e->runs.size(); r++) {
@@ -463,6 +474,8 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         const nl_attn_desc &A = L.d.attn;
         const nl_linattn_desc &G = L.d.lin;
         const float *behind = R.add_embed ? e->x0 : nullptr;
+        // (the last norm has a launch: the output matrix's many row tiles would each add up the partial sums, 31 -> 35 us at 32000 x 768)
+        const float *const next = r + 1 < e->runs.size() ? e->layers[e->runs[r + 1].layer].norm1 : nullptr;
         MatParams J = product_params(e, L.proj, nullptr, s.n);
         J.out = e->proj; J.ldo = L.proj.rows;
         if ((rc = normed_product<T, ST_F32>(e, J, L.norm1))) return rc;
@@ -492,12 +505,12 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
             if (A.heads && ((rc = launch_win_prep<T>(W, s.n, st)) || (rc = launch_win_attn<T>(W, s.ntiles, st)))) return rc;
             if (G.heads && (rc = launch_gla<T>(N, s.nsubs, s.nsegs, s.nruns, st))) return rc;
         }
-        if ((rc = residual_product<T>(e, L.out, e->y, s.n, nullptr, L.norm1p, L.d.ff ? nullptr : behind))) return rc;
+        if ((rc = residual_product<T>(e, L.out, e->y, s.n, nullptr, L.norm1p, L.d.ff ? nullptr : behind, L.d.ff ? L.norm2 : next))) return rc;
         if (L.d.ff) {
             MatParams F = product_params(e, L.gateup, nullptr, s.n);
             F.act = e->act; F.act_nks = L.down.nks; F.act_silu = L.d.ff_act == NL_ACT_SILU; F.bias = L.gateb; F.bias2 = L.upb;
             if ((rc = normed_product<T, ST_GATED>(e, F, L.norm2))) return rc;
-            if ((rc = residual_product<T>(e, L.down, e->act, s.n, L.downb, L.norm2p, behind))) return rc;
+            if ((rc = residual_product<T>(e, L.down, e->act, s.n, L.downb, L.norm2p, behind, next))) return rc;
         }
         if (e->trace) {
             float *to = e->tracebuf + r * (size_t)s.n * D;
@@ -970,7 +983,7 @@ int nl_finalize(nl_handle e) {
     for (const Run &r : e->runs) loop |= r.add_embed;
     if ((rc = dev_alloc(e, e->x, (size_t)cap * D * 4, bs)) || (loop && (rc = dev_alloc(e, e->x0, (size_t)cap * D * 4, bs))) ||
         (rc = dev_alloc(e, e->proj, (size_t)cap * ldmax * 4, bs)) || (rc = dev_alloc(e, e->logits, (size_t)e->lm_cap * e->c.vocab * 4, bs)) ||
-        (rc = dev_alloc(e, e->h, std::max(tt, (size_t)up(e->lm_cap, 128) / 16) * hk * OPT * es, bs)) || (rc = dev_alloc(e, e->y, tt * yk * OPT * es, bs)) ||
+        (rc = dev_alloc(e, e->h, std::max(tt, (size_t)up(e->lm_cap, 128) / 16) * hk * OPT * es, bs)) || (rc = dev_alloc(e, e->fss, (size_t)FEW_MAX_TOKENS * 2 * e->nksd * sizeof(float), bs)) || (rc = dev_alloc(e, e->y, tt * yk * OPT * es, bs)) ||
         (ak && (rc = dev_alloc(e, e->act, tt * ak * OPT * es, bs))) || (qrow && (rc = dev_alloc(e, e->q, std::max((size_t)cap * qrow, qfew) * es, bs))) ||
         (e->c.post_norm && ((rc = dev_alloc(e, e->x2, (size_t)cap * D * 4, bs)) || (rc = dev_alloc(e, e->delta, (size_t)cap * D * 4, bs)))) ||
         (e->latent && ((rc = dev_alloc(e, e->xq, xq * es, bs)) || (rc = dev_alloc(e, e->ek, ek * es, bs)) || (rc = dev_alloc(e, e->ev, ev * es, bs)) ||
