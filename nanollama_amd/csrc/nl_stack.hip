@@ -349,6 +349,29 @@ MatParams product_params(nl_engine *e, const Mat &m, const void *X, int n) {
     return P;
 }
 
+// weights that the launches behind a decode launch read, rb row tiles to a workgroup, nearest launch first: as many lists as half of the L2s
+// (8 x 4 MB) holds.  us / step, none, 8, 16 and 24 MB: Pabalix, 1 stream, 768 columns 805, 767, 766, 767, 1536 columns 1273, 1265, 1216, 1252;
+// Ganidra, 32 streams, 1536 columns 1301, 1274, 1255, 1258.
+struct Next { const Mat *m; int rb; };
+constexpr long long AHEAD_MAX = 16 << 20;
+template <typename T>
+Ahead look_ahead(int n, std::initializer_list<Next> next) {
+    Ahead A{};
+    if (n > FEW_MAX_TOKENS) return A;
+    int i = 0;
+    long long total = 0;
+    for (const Next &x : next) {
+        if (!x.m || !x.m->w) continue;
+        if ((total += (long long)x.m->nrt * x.m->nks * OPT * sizeof(T)) > AHEAD_MAX) break;
+        A.w[i] = static_cast<const char *>(x.m->w);
+        A.units[i] = x.m->nrt / x.rb;
+        A.bytes[i] = x.rb * x.m->nks * OPT * (int)sizeof(T);
+        A.chunks += (A.units[i] + 7) / 8 * ((A.bytes[i] + 8191) / 8192);
+        i++;
+    }
+    return A;
+}
+
 // the product of norm(stream) with m, epilogue fields of P set by the caller: the norm runs inside the product's launch or leaves an operand of
 // its own; what is pending behind the last sublayer is added on the way.  rows: only these tokens, and the stream stays as it is.
 template <typename T, int EPI>
@@ -377,9 +400,11 @@ hipError_t normed_product(nl_engine *e, MatParams P, const float *nw, const int 
 // a sublayer's last product: into the stream, or kept for the norm behind it
 // next: the gains of the norm that the stream meets next, where its product can take them folded (MatParams::fw)
 template <typename T>
-hipError_t residual_product(nl_engine *e, const Mat &m, const void *X, int n, const float *bias, const float *post, const float *behind, const float *next) {
+hipError_t residual_product(nl_engine *e, const Mat &m, const void *X, int n, const float *bias, const float *post, const float *behind, const float *next,
+                            const Mat *ahead = nullptr) {
     MatParams P = product_params(e, m, X, n);
     P.ldo = e->c.dim;
+    P.ahead = look_ahead<T>(n, {{ahead, 2}});
     if (!post) {
         P.out = e->xcur; P.add2 = behind;
         // (up to a few tokens the norm costs nothing: the product behind it computes it in its prologue)
@@ -478,6 +503,9 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         const float *const next = r + 1 < e->runs.size() ? e->layers[e->runs[r + 1].layer].norm1 : nullptr;
         MatParams J = product_params(e, L.proj, nullptr, s.n);
         J.out = e->proj; J.ldo = L.proj.rows;
+        // (what reads ahead: latent attention's own launches keep up to 100 KB of LDS per workgroup, so its products do, 766 against 795 us a
+        // token; the other mixers' launch has room on every CU, 737 against 755 us a step of 48 streams)
+        if (L.d.latent.heads) J.ahead = look_ahead<T>(s.n, {{&L.uq, 1}, {&L.ukt, 1}, {&L.uv, 1}, {&L.out, 1}});
         if ((rc = normed_product<T, ST_F32>(e, J, L.norm1))) return rc;
         WinParams W{};
         W.pos = s.pos; W.stream = s.stream; W.nsplit = 1; W.y = e->y; W.y_nks = L.out.nks; W.proj = e->proj; W.ldp = L.proj.rows;
@@ -500,15 +528,19 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         if (L.d.latent.heads) {
             if ((rc = latent_mixer<T>(e, s, R, L))) return rc;
         } else if (s.decode) {
+            W.ahead = look_ahead<T>(s.n, {{&L.out, 1}, {&L.gateup, 2}, {&L.down, 1}});
             if ((rc = launch_mix_decode<T>(W, N, s.n, st))) return rc;
         } else {
             if (A.heads && ((rc = launch_win_prep<T>(W, s.n, st)) || (rc = launch_win_attn<T>(W, s.ntiles, st)))) return rc;
             if (G.heads && (rc = launch_gla<T>(N, s.nsubs, s.nsegs, s.nruns, st))) return rc;
         }
-        if ((rc = residual_product<T>(e, L.out, e->y, s.n, nullptr, L.norm1p, L.d.ff ? nullptr : behind, L.d.ff ? L.norm2 : next))) return rc;
+        if ((rc = residual_product<T>(e, L.out, e->y, s.n, nullptr, L.norm1p, L.d.ff ? nullptr : behind, L.d.ff ? L.norm2 : next,
+                                      L.d.ff && L.d.latent.heads ? &L.gateup : nullptr))) return rc;
         if (L.d.ff) {
             MatParams F = product_params(e, L.gateup, nullptr, s.n);
             F.act = e->act; F.act_nks = L.down.nks; F.act_silu = L.d.ff_act == NL_ACT_SILU; F.bias = L.gateb; F.bias2 = L.upb;
+            F.ahead = look_ahead<T>(s.n, {{L.d.latent.heads ? &L.down : nullptr, 1},
+                                          {r + 1 < e->runs.size() ? &e->layers[e->runs[r + 1].layer].proj : nullptr, 1}});
             if ((rc = normed_product<T, ST_GATED>(e, F, L.norm2))) return rc;
             if ((rc = residual_product<T>(e, L.down, e->act, s.n, L.downb, L.norm2p, behind, next))) return rc;
         }

@@ -49,6 +49,7 @@ struct WinParams {
     int nsplit;
     float *part;                // [token][heads][nsplit][dv + 2]
     unsigned *arrived;          // [token][heads], zero between launches
+    Ahead ahead;                // decode
 };
 
 template <typename T> __device__ __forceinline__ T *ring_k(const WinParams &P, int stream, int g) {
@@ -439,8 +440,12 @@ __device__ __forceinline__ void win_decode_block(const WinParams &P, int h, int 
 
 // a decode batch's mixers: grid (attention heads x splits + linear-attention heads, tokens)
 template <typename T, int M>
-__global__ void __launch_bounds__(256) mix_decode_kernel(WinParams A, GlaParams L) {
+__global__ void __launch_bounds__(256) mix_decode_kernel(WinParams A, GlaParams L, int n_tokens) {
     extern __shared__ __align__(16) char lds[];
+    if ((int)blockIdx.y >= n_tokens) {
+        A.ahead.read(blockIdx.y * gridDim.x + blockIdx.x, n_tokens * gridDim.x, 4, threadIdx.x >> 6, threadIdx.x & 63);
+        return;
+    }
     const int n = blockIdx.y, pos = A.pos[n], stream = A.stream[n], na = M ? A.heads * A.nsplit : 0;
     if constexpr (M > 0) {
         if ((int)blockIdx.x < na) {
@@ -457,7 +462,8 @@ hipError_t launch_mix_decode(const WinParams &A, const GlaParams &L, int n, hipS
     if (A.heads) lds = win_decode_lds(A.nks, A.nvt);
     if (L.heads) lds = std::max(lds, gla_decode_lds(L.dkp, L.dvp, L.rank));
     auto go = [&](auto kfn) {
-        hipLaunchKernelGGL(kfn, dim3(A.heads * A.nsplit + L.heads, n), dim3(256), lds, st, A, L);
+        const int gx = A.heads * A.nsplit + L.heads;
+        hipLaunchKernelGGL(kfn, dim3(gx, n + (A.ahead.wgs(4) + gx - 1) / gx), dim3(256), lds, st, A, L, n);
         return hipGetLastError();
     };
     if (!A.heads) return go(mix_decode_kernel<T, 0>);

@@ -1,4 +1,5 @@
-"""GPU: decode batches of layer-stack models with the norm between two products folded around them (MatParams::fw, nl_mfma.h)."""
+"""GPU: decode batches of layer-stack models with the norm between two products folded around them (MatParams::fw, nl_mfma.h), and the reading
+ahead of the next launches' weights (Ahead)."""
 import os
 import sys
 
@@ -30,4 +31,21 @@ def test_folded_norm_in_decode_batches(width, n, scale, loop, dtype):
         for i, s in enumerate(seqs):
             # (the tolerances of the unfolded products: the gains and 1 / rms are applied on the other side of the same sums)
             assert rel(rows[i], so.forward(cfg, fl, s[:len(s) + 1 - back])[-1]) < (F32_TOL if dtype == "float32" else BF16_TOL), (i, back)
+    m.close()
+
+
+# one list, all of them, and a feed-forward past what is read ahead; row tiles and workgroups that are no multiple of the XCDs
+@pytest.mark.parametrize("width,ff,n,dtype", [(64, 24, 1, "float32"), (136, 344, 1, "bfloat16"), (136, 344, 40, "float32"), (2056, 2008, 2, "float32")])
+def test_weights_read_ahead(width, ff, n, dtype):
+    cfg = config([par(heads=2, kv=1, ff=ff), gla(ff=0), gla(ff=ff)], width=width)
+    w = weights(cfg, 92)
+    seqs = [tokens(5, seed=50 + i) for i in range(n)]
+    m = load(cfg, w, dtype, max_streams=n, seq_len=16)
+    for i, s in enumerate(seqs):
+        m.prefill(s[:3], 0, i, want_logits=False)
+    for at in (3, 4):
+        _, rows = m.forward_batch(list(range(n)), [s[at] for s in seqs], [at] * n, want_logits=True)
+    fl = floats(w)
+    for i, s in enumerate(seqs):
+        assert rel(rows[i], so.forward(cfg, fl, s)[-1]) < (F32_TOL if dtype == "float32" else BF16_TOL), i
     m.close()
