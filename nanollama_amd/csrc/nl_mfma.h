@@ -655,6 +655,112 @@ __global__ void __launch_bounds__(256) many_kernel(MatParams P, TAIL tail) {
     }
 }
 
+// Prompts, where many_kernel's tiles leave the chip idle or its LDS busy (a wavefront there reads 6 tiles for 8 products): RW x TW tiles per
+// wavefront straight from L2 to registers, one step ahead, no LDS and no barrier in the loop.  WR x WT wavefronts cover WR RW x WT TW tiles, KS
+// such sets share K (k tiles dealt in turn) and meet in LDS behind the loop.  The fences keep a step's loads ahead of the products of the one
+// before it: hipcc sinks them to their use otherwise (128 x 128 tiles, 1536 x 1536 at 2047 tokens: 31 us instead of 22).
+__device__ __forceinline__ void load_tile(Frag<bf16> &f, const __amdgpu_buffer_rsrc_t rs, int lane, unsigned off) {
+    f.v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, off, 0));
+}
+__device__ __forceinline__ void load_tile(Frag<float> &f, const __amdgpu_buffer_rsrc_t rs, int lane, unsigned off) {
+    f.a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 32, off, 0));
+    f.b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 32, off + 16, 0));
+}
+// rows of tiles whose partial sums are in LDS together: all of them where 64 KB hold them, else pairs
+constexpr int direct_rows(int waves, int rw, int tw) { return waves * rw * tw <= 64 ? rw : 2; }
+template <typename T, int EPI, int WR, int WT, int KS, int RW, int TW>
+__global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P) {
+    constexpr int UNIT = OPT * sizeof(T), SET = WR * WT;
+    static_assert(RW % 2 == 0, "gate and up rows come in pairs");
+    extern __shared__ __align__(16) char lds[];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
+    const int nks = P.nks, ntt = (P.n_tokens + 15) >> 4;
+    const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = (ntt + WT * TW - 1) / (WT * TW), total = nrb * ntb;
+    const int per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);      // (as many_kernel's)
+    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+    const int rb = id / ntb, tb = id - rb * ntb, kw = w / SET, wr = w % WR, wt = w / WR % WT, r0 = (rb * WR + wr) * RW, t0 = (tb * WT + wt) * TW;
+    const __amdgpu_buffer_rsrc_t W = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.W), 0, (int)((unsigned)P.nrt * nks * UNIT), 0x00027000);
+    const __amdgpu_buffer_rsrc_t X = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.X), 0, (int)((unsigned)ntt * P.x_nks * UNIT), 0x00027000);
+    unsigned wo[RW], xo[TW];                               // (tiles past the end repeat the last one)
+#pragma unroll
+    for (int r = 0; r < RW; r++) wo[r] = (unsigned)min(r0 + r, P.nrt - 1) * nks * UNIT;
+#pragma unroll
+    for (int t = 0; t < TW; t++) xo[t] = (unsigned)min(t0 + t, ntt - 1) * P.x_nks * UNIT;
+    f32x4 acc[RW][TW] = {};
+    Frag<T> a[2][RW], b[2][TW];
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load = [&](int ks, int s) {
+        const unsigned k = (unsigned)min(ks, nks - 1) * UNIT;
+#pragma unroll
+        for (int r = 0; r < RW; r++) load_tile(a[s][r], W, lane, wo[r] + k);
+#pragma unroll
+        for (int t = 0; t < TW; t++) load_tile(b[s][t], X, lane, xo[t] + k);
+        fence();
+    };
+    auto step = [&](int s) {
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+#pragma unroll
+            for (int t = 0; t < TW; t++) acc[r][t] = mma(a[s][r], b[s][t], acc[r][t]);
+        fence();
+    };
+    load(kw, 0);
+    int ks = kw;
+    for (; ks + KS < nks; ks += 2 * KS) {
+        load(ks + KS, 1);
+        step(0);
+        load(ks + 2 * KS, 0);
+        step(1);
+    }
+    if (ks < nks) step(0);
+    auto store = [&](int r, int t, f32x4 v, f32x4 v2) {
+        const int tok = (t0 + t) * 16 + (lane & 15), rt = r0 + r, row = rt * 16 + 4 * g;
+        if (tok >= P.n_tokens || rt >= P.nrt) return;
+        if constexpr (EPI == ST_GATED) store_gated<T>(P, tok, rt >> 1, g, v, v2);
+        else {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if (rt + i >= P.nrt) break;
+                if constexpr (EPI == ST_F32) store_rows(P.out, P.ldo, P.rows, tok, row + 16 * i, with_bias(P.bias, row + 16 * i, i ? v2 : v));
+                else if constexpr (EPI == ST_HEADS) store_heads<T>(P.hd, tok, row + 16 * i, i ? v2 : v);
+                else add_rows(P.out, P.add2, P.ldo, P.rows, tok, row + 16 * i, i ? v2 : v);
+            }
+        }
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int r = 0; r < RW; r += 2)
+#pragma unroll
+            for (int t = 0; t < TW; t++) store(r, t, acc[r][t], acc[r + 1][t]);
+        return;
+    }
+    constexpr int RR = direct_rows(SET * KS, RW, TW), PAIRS = RR / 2 * TW;
+    f32x4 *red = reinterpret_cast<f32x4 *>(lds);           // [KS][SET][RR][TW][64]: RR rows of tiles at a time
+#pragma unroll
+    for (int r = 0; r < RW; r += RR) {
+        if (r) lds_barrier();
+#pragma unroll
+        for (int i = 0; i < RR; i++)
+#pragma unroll
+            for (int t = 0; t < TW; t++) red[((w * RR + i) * TW + t) * 64 + lane] = acc[r + i][t];
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < (PAIRS + KS - 1) / KS; j++) {
+            const int p = kw + j * KS, i = p / TW * 2, t = p % TW;
+            if (p >= PAIRS) break;                         // (more wavefronts than pairs)
+            f32x4 v[2] = {};
+#pragma unroll
+            for (int q = 0; q < KS; q++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) v[k] += red[(((q * SET + w % SET) * RR + i + k) * TW + t) * 64 + lane];
+            store(r + i, t, v[0], v[1]);
+        }
+    }
+}
+
 constexpr int FEW_MAX_TOKENS = 64;
 constexpr int FEW_NORM_SLOTS = 4;         // (token, 2048 columns) slots up to which few_kernel computes the norm itself
 
@@ -921,6 +1027,44 @@ hipError_t launch_many(const MatParams &P, hipStream_t st, TAIL tail = {}) {
     return go(many_kernel<T, EPI, 2, TAIL>, 4, ManyGeom<T, 2>::LDS);
 }
 
+template <typename T, int EPI, int WR, int WT, int KS, int RW, int TW>
+hipError_t launch_direct(const MatParams &P, hipStream_t st) {
+    constexpr int lds = KS == 1 ? 0 : WR * WT * KS * direct_rows(WR * WT * KS, RW, TW) * TW * 1024;
+    static_assert(lds <= 65536, "what a launch has without asking");
+    const int total = (P.nrt + WR * RW - 1) / (WR * RW) * (((P.n_tokens + 15) / 16 + WT * TW - 1) / (WT * TW));
+    hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3((total + 7) / 8 * 8), dim3(WR * WT * KS * 64), lds, st, P);
+    return hipGetLastError();
+}
+// Prompts: the largest tile with which the workgroups still cover the chip, in one round where that goes.  us, many_kernel -> direct_kernel,
+// bf16, weights from memory, rows x K at n tokens:
+//   32 x 64, K over 8 wavefronts   768 x 768 at 200 10.7 -> 4.0 (64 x 64: 5.6); 1536 x 4096 at 200 38.4 -> 10.0 (13.3); with more tiles than
+//                                  CUs behind the next: 1536 x 1536 at 700 12.4 against 11.2
+//   64 x 64, K over 4, two a CU    768 x 768 at 2047 12.4 -> 9.1; 1536 x 4096 at 400 38.7 -> 14.6; 4640 x 1536 at 400 20.9 -> 12.9
+//   96 x 128, K over 4             1536 x 1536 at 2047 24.5 -> 19.5 (64 x 64: 25.9); 1536 x 4096 at 2047 51.1 -> 31.9 (58.6); its sums are not
+//                                  worth their way through LDS below a K of 1024
+//   192 x 256 and 256 x 256        4640 x 1536 at 2047 51.6 -> 38.3; 8192 x 1536 at 2047 63.5 -> 54.3, at 1500 (192 tiles) 53.2 -> 51.1; with
+//                                  fewer CUs at work slower, at 1000 (128 tiles) 31.6 -> 46.2
+//   64 x 64 up to 3.5 a CU         4640 x 1536 at 700 23.0 -> 20.9; 8192 x 1536 at 400 21.8 -> 20.0; 2320 x 768 at 1500 14.3, both; beyond,
+//                                  8192 x 1536 at 700, 27.2 against 28.6
+// float, 1536 x 1536 at 70 and 1000: 61.7 -> 15.3, 66.4 -> 53.3 (its matrix instructions bound the large products: the small tiles only)
+template <typename T, int EPI>
+hipError_t launch_prompt(const MatParams &P, hipStream_t st) {
+    const int tt = (P.n_tokens + 15) / 16;
+    auto tiles = [&](int rt, int t) { return (long long)((P.nrt + rt - 1) / rt) * ((tt + t - 1) / t); };
+    const long long most = std::max((long long)P.nrt * P.nks, (long long)tt * P.x_nks) * OPT * (long long)sizeof(T);
+    if (most >= 1ll << 31) return launch_many<T, EPI>(P, st);        // (32-bit offsets)
+    if (tiles(2, 4) <= 256) return launch_direct<T, EPI, 1, 1, 8, 2, 4>(P, st);
+    if (tiles(4, 4) <= 512) return launch_direct<T, EPI, 1, 1, 4, 4, 4>(P, st);
+    if constexpr (sizeof(T) == 2) {
+        auto covers = [&](int rt, int t) { return tiles(rt, t) >= 192 && tiles(rt, t) <= 256; };
+        if (tiles(6, 8) <= 256 && P.nks >= 32) return launch_direct<T, EPI, 1, 1, 4, 6, 8>(P, st);
+        if (covers(12, 16)) return launch_direct<T, EPI, 2, 2, 1, 6, 8>(P, st);
+        if (covers(16, 16)) return launch_direct<T, EPI, 2, 2, 1, 8, 8>(P, st);
+    }
+    if (tiles(4, 4) <= 896) return launch_direct<T, EPI, 1, 1, 4, 4, 4>(P, st);
+    return launch_many<T, EPI>(P, st);
+}
+
 // norm: see few_kernel.  A tail rides in decode launches only (launch_few).
 template <typename T, int EPI, class TAIL = NoTail>
 hipError_t launch_product(MatParams P, hipStream_t st, int norm = 0, TAIL tail = {}) {
@@ -928,7 +1072,7 @@ hipError_t launch_product(MatParams P, hipStream_t st, int norm = 0, TAIL tail =
     if (!P.x_nks) P.x_nks = P.nks;
     if (!P.nld) P.nld = P.ndim;
     if (P.n_tokens <= FEW_MAX_TOKENS) return launch_few<T, EPI>(P, st, norm, tail);
-    return launch_many<T, EPI>(P, st);
+    return launch_prompt<T, EPI>(P, st);
 }
 
 }  // namespace nl
