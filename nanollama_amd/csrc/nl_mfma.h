@@ -11,13 +11,13 @@
 // [token][in] the B operand (rows = tokens); the accumulator of a 16 x 16 tile has D[row = 4 (lane / 16) + i][token = lane % 16],
 // so a lane ends up with four consecutive outputs of one token.
 //
-// Two kernels: many_kernel for prompts (a 128 x 128 tile per workgroup, an LDS ring filled by LDS-DMA) and few_kernel for
-// decode batches of up to 64 tokens (one row tile per workgroup, K split over its wavefronts, the weights read once straight into
-// registers; for a handful of tokens the RMS norm of the layer's input runs in its prologue, together with the norm and residual add
+// Three kernels: many_kernel for prompts (a 128 x 128 tile per workgroup, an LDS ring filled by LDS-DMA), direct_kernel for those whose
+// tiles it leaves idle or bound by LDS (fragments straight to registers, K split over wavefronts), and few_kernel for decode batches of
+// up to 64 tokens (one row tile per workgroup, K split over its wavefronts, the weights read once straight into registers; for a handful of tokens the RMS norm of the layer's input runs in its prologue, together with the norm and residual add
 // of the sublayer before where a model has norms behind its sublayers).  Epilogues: plain 32-bit store (+ bias), residual add (+ an
 // optional second addend), activation(gate) * up stored as the next product's operand, query rows by head with rotary positions, keys and
 // values in the operand order of the attention products.  A launch may carry independent work of single wavefronts behind its own
-// workgroups (TAIL).
+// workgroups (TAIL), or bring the next launches' weights into L2 (Ahead).
 #pragma once
 #include "nl_kernels.h"
 
