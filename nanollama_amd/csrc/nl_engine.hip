@@ -1966,18 +1966,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     // (kv16_build_kernel) and a workgroup takes twice the rows, one workgroup per CU (AttnTile16ShadowQT).
     int n_live = 0, max_nparts = 0;
     bool kv16_on = false;
-    // position splits any token of this step can see: the attention grids skip the rest (a decode batch at short
-    // contexts would otherwise dispatch 15 empty workgroups for every live one)
-    const bool no_tile = attn_knobs().no_tile, no_fin = attn_knobs().no_fin;
-    int nsplit = 1;
-    for (int i = 0; i < n; i++) nsplit = std::max(nsplit, b.h_meta[b.cap + i] / ATT_CH + 1);
-    nsplit = std::min(nsplit, e->nsplit_max);
-    // Prompts: attn_tile16_kernel -- unless every position lies in the first split: attn_kernel<..., FIN> then finishes each row itself and
-    // writes WO's fragments, one launch for two (prompt of 24 / 100 tokens: 89M 672 / 741 -> 583 / 683 us, 173M Q4_0 749 / 835 -> 651 / 721,
-    // 841M Q8_0 1665 / 2302 -> 1499 / 2150; from position 128 on: 33 tokens at 700, 841M 1934 against 2010)
-    const bool tile_attn = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile && (nsplit > 1 || no_fin);
     {
-        bool cons = tile_attn && !attn_knobs().f32_tile;
+        bool cons = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !attn_knobs().f32_tile && !attn_knobs().no_tile;
         for (int i = 1; i < n && cons; i++) cons = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
         const int kv16_min = getenv("NL_KV16_MIN_TOKENS") ? atoi(getenv("NL_KV16_MIN_TOKENS")) : 256;   // (read per step: a test lowers it)
         kv16_on = cons && n >= kv16_min && b.kv16 != nullptr;
@@ -2020,8 +2010,15 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         LCK(hipGetLastError());
     }
     const int nt16 = ((n + 63) / 64) * 4;
+    // position splits any token of this step can see: the attention grids skip the rest (a decode batch at short
+    // contexts would otherwise dispatch 15 empty workgroups for every live one)
+    const bool no_tile = attn_knobs().no_tile, no_fin = attn_knobs().no_fin;
+    int nsplit = 1;
+    for (int i = 0; i < n; i++) nsplit = std::max(nsplit, b.h_meta[b.cap + i] / ATT_CH + 1);
     bool consecutive = true;   // positions pos0, pos0 + 1, ...: a prompt
     for (int i = 1; i < n && consecutive; i++) consecutive = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
+    nsplit = std::min(nsplit, e->nsplit_max);
+    const bool tile_attn = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;   // prompts: attn_tile16_kernel
     const bool fin_attn = !tile_attn && nsplit == 1 && !no_fin;                                 // one split: attn_kernel<..., FIN>
     const char *rk = getenv("NL_ROPE_IN_ATTN");    // knob (tests, tools; read per step): 0 keeps the brope_kv launch
     const bool rope_attn_knob = !(rk && atoi(rk) == 0);
@@ -2107,7 +2104,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                          (float)(1.0 / std::sqrt((double)hd)), 0, b.pos, b.stream, (long long)HQ,
                          (long long)e->Hs * e->nsplit_max};
             bool merged = false;
-            if (tile_attn) {
+            if (one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile) {
                 // prefill: the step's tokens share a stream -> K/V split staged once per tile of tokens, fp16 MFMA with hi/lo-split operands (attn_tile16_kernel)
                 AttnParams T = P;
                 T.x1 = x1_attn;
@@ -2141,7 +2138,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 LCK(launch_attn(hd, e->gqa, P, dim3(e->KVs, nsplit, n), st));
             }
             if (!merged) {
-            BMergeParams M{b.part_o, b.part_ml, b.pos, tile_attn && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, L.wo.wtype == WT_Q4_0 ? 1 : 0, tile_attn ? 1 : 0};
+            const bool tile16 = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;
+            BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, L.wo.wtype == WT_Q4_0 ? 1 : 0, tile16 ? 1 : 0};
             {
                 const long long units = (long long)n * e->Hs * hd / 8;
                 if (M.nparts && max_nparts <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
