@@ -155,8 +155,8 @@ NL_API int nl_sample_decode(nl_handle h, int stream, int pos, int n_steps, const
  * round trip; last_logits_out (may be NULL) receives the logits after the last token.  Q4_0 / Q8_0 / Q5_0 / F16 / Q4_K / Q6_K
  * models take the multi-token matrix-core path (up to 2048 tokens per step): the KV
  * cache and logits agree with n nl_forward calls to the stated logit tolerance (1e-4, summation order
- * and an fp16 hi+lo activation split differ), greedy continuations are identical; F32 matrices run
- * the single-token plan n times (bitwise equal).  pos0 + n must be <= seq_len. */
+ * and an fp16 hi+lo activation split differ), greedy continuations are identical; files with Q4_K / Q6_K matrices keep float32
+ * operands and range there; F32 matrices, and F16 ones beside Q4_K / Q6_K, run the single-token plan n times (bitwise equal).  pos0 + n must be <= seq_len. */
 NL_API int nl_prefill(nl_handle h, int stream, const int *tokens, int n, int pos0, float *last_logits_out);
 /* One Forward for each of n (stream, token, pos) triples -- the concurrent decode streams of a
  * serving host.  logits_out (may be NULL) is n x vocab; next_ids (may be NULL) receives each

@@ -212,7 +212,7 @@ struct BNormParams {
     float eps;
     int dim, item0;      // token of workgroup b = item0 + b; its fragment column is b
     uint4 *xf;
-    int nt16, q4;
+    int nt16, form;
     float *scale_out;    // [N] or nullptr: norm_prescale(inv) of the token, the pre-scale of the first folded-norm producer
 };
 
@@ -221,7 +221,7 @@ struct BNormParams {
 template <int UPT>
 __global__ void __launch_bounds__(256) bnorm_kernel(BNormParams P) {
     NL_KARGS8(P.x, P.w, P.xf, P.pend.part, P.pend.bias, P.dim, P.item0, P.pend.ks);   // one batch of s_load (nl_kernels.h)
-    NL_KARGS4(P.eps, P.nt16, P.q4, P.pend.zstride);
+    NL_KARGS4(P.eps, P.nt16, P.form, P.pend.zstride);
     __shared__ double dred[4];
     const int item = P.item0 + blockIdx.x, n = P.dim, nu = n / 8;
     float *xr = P.x + (long long)item * n;
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(256) bnorm_kernel(BNormParams P) {
     for (int k = 0; k < UPT; k++) {
         const int u = min((int)threadIdx.x + k * (int)blockDim.x, nu - 1);
         int offa, offb;
-        slot_offsets(P.q4, u & 3, offa, offb);
+        slot_offsets(P.form, u & 3, offa, offb);
         ca[k] = (u >> 2) * 32 + offa; cb[k] = (u >> 2) * 32 + offb;
         xa[k] = *reinterpret_cast<const float4 *>(xr + ca[k]);
         xb[k] = *reinterpret_cast<const float4 *>(xr + cb[k]);
@@ -278,11 +278,11 @@ __global__ void __launch_bounds__(256) bnorm_kernel(BNormParams P) {
         const int u = (int)threadIdx.x + k * (int)blockDim.x;
         if (u >= nu) continue;
         float xv[8], wv[8], v[8];
-        slots_from(P.q4, xa[k], xb[k], xv);
-        slots_from(P.q4, wa[k], wb[k], wv);
+        slots_from(P.form, xa[k], xb[k], xv);
+        slots_from(P.form, wa[k], wb[k], wv);
 #pragma unroll
         for (int j = 0; j < 8; j++) v[j] = (xv[j] * inv) * wv[j];
-        store_frag(P.xf, P.nt16, blockIdx.x, u >> 2, u & 3, v);
+        store_frag(P.xf, P.nt16, blockIdx.x, u >> 2, u & 3, v, P.form);
     }
 }
 
@@ -313,10 +313,10 @@ __global__ void __launch_bounds__(256) bnorm_generic_kernel(BNormParams P) {
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const int i = blk * 32 + slot_elem(P.q4, w, j);
+            const int i = blk * 32 + slot_elem(P.form, w, j);
             v[j] = (xr[i] * inv) * P.w[i];
         }
-        store_frag(P.xf, P.nt16, blockIdx.x, blk, w, v);
+        store_frag(P.xf, P.nt16, blockIdx.x, blk, w, v, P.form);
     }
 }
 
@@ -408,13 +408,13 @@ __device__ void attn_finalize(const AttnParams &P, const float *ored, const floa
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        const int d = bl * 32 + slot_elem(P.fin_q4, w, j);
+        const int d = bl * 32 + slot_elem(P.fin_form, w, j);
         float s = 0.f;
 #pragma unroll 8
         for (int k = 0; k < NG; k++) s += ored[(k * G + g) * HD + d];
         v[j] = s * scale;
     }
-    store_frag(P.fin_xf, P.fin_nt16, item, ((kvh * G + g) * HD) / 32 + bl, w, v);
+    store_frag(P.fin_xf, P.fin_nt16, item, ((kvh * G + g) * HD) / 32 + bl, w, v, P.fin_form);
 }
 
 struct BMergeParams {
@@ -423,7 +423,7 @@ struct BMergeParams {
     const int *nparts;   // partials per item when attn_tile16_kernel folded runs of chunks (null: one per 128 positions)
     int heads, nsplit_max, head_dim;
     uint4 *xf;   // attention output [N][heads*hd] as MFMA fragments for the WO GEMM
-    int nt16, q4;
+    int nt16, form;
     int fast_exp;   // split weights on v_exp_f32 (prompts: their partials come from attn_tile16_kernel's v_exp_f32 already)
 };
 
@@ -462,7 +462,7 @@ __global__ void battn_merge_kernel(BMergeParams P, int n_items) {
         const float scale = 1.0f / L;
         const float *po = P.part_o + (pbase + (long long)h * P.nsplit_max) * hd + (blk * 32 - h * hd);
         int offa, offb;
-        slot_offsets(P.q4, w, offa, offb);
+        slot_offsets(P.form, w, offa, offb);
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) v[j] = 0.f;
@@ -473,7 +473,7 @@ __global__ void battn_merge_kernel(BMergeParams P, int n_items) {
                 // slots (w, j) of the block, as load_x_slots: only the two middle lanes of each float4 differ by type
                 const float *src = po + (long long)min(c0 + k, ns - 1) * hd;
                 const float4 a = *reinterpret_cast<const float4 *>(src + offa), b = *reinterpret_cast<const float4 *>(src + offb);
-                slots_from(P.q4, a, b, pv[k]);
+                slots_from(P.form, a, b, pv[k]);
             }
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -486,7 +486,7 @@ __global__ void battn_merge_kernel(BMergeParams P, int n_items) {
         }
 #pragma unroll
         for (int j = 0; j < 8; j++) v[j] *= scale;
-        store_frag(P.xf, P.nt16, item, blk, w, v);
+        store_frag(P.xf, P.nt16, item, blk, w, v, P.form);
     }
 }
 
@@ -496,18 +496,18 @@ struct BSwigluParams {
     GemmOut g, u;        // [N][interm]
     int interm, n_tokens;
     uint4 *xf;
-    int nt16, q4;
+    int nt16, form;
 };
 
 __global__ void bswiglu_kernel(BSwigluParams P) {
     NL_KARGS8(P.g.val, P.g.part, P.u.val, P.u.part, P.xf, P.interm, P.n_tokens, P.g.ks);   // one batch of s_load
-    NL_KARGS4(P.g.zstride, P.u.zstride, P.nt16, P.q4);
+    NL_KARGS4(P.g.zstride, P.u.zstride, P.nt16, P.form);
     const int upt = P.interm / 8;                     // units per token
     const long long total = (long long)P.n_tokens * upt;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long long)gridDim.x * blockDim.x) {
         const int n = (int)(i / upt), u = (int)(i - (long long)n * upt), blk = u >> 2, w = u & 3;
         int offa, offb;
-        slot_offsets(P.q4, w, offa, offb);
+        slot_offsets(P.form, w, offa, offb);
         const int ca = blk * 32 + offa, cb = blk * 32 + offb;
         const long long row = (long long)n * P.interm;
         float4 ga, gb, ua, ub;
@@ -521,8 +521,8 @@ __global__ void bswiglu_kernel(BSwigluParams P) {
             gemm_out_at4x2(P.u, row + ca, ca, row + cb, cb, ua, ub);
         }
         float gv[8], uv[8], v[8];
-        slots_from(P.q4, ga, gb, gv);
-        slots_from(P.q4, ua, ub, uv);
+        slots_from(P.form, ga, gb, gv);
+        slots_from(P.form, ua, ub, uv);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const float ex = exp_f64_as_f32(-gv[j]);
@@ -639,27 +639,26 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
 
     // ---- S^T = K q^T: 8 key tiles (M) x 16 rows (N); lane (j, kq) ends up holding row j's scores for keys
     //      16*mt + 4*kq + r -- exactly the A-operand layout of P in P V, so P never leaves registers ----
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
     v4f acc[8];
 #pragma unroll
-    for (int mt = 0; mt < 8; mt++) acc[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < 8; mt++) acc[mt] = zero;
 #pragma unroll
     for (int s4 = 0; s4 < DK / 4; s4++) {
         float4 kb[8];
 #pragma unroll
         for (int mt = 0; mt < 8; mt++)
             kb[mt] = *reinterpret_cast<const float4 *>(Ks + (mt * 16 + j) * KS + DK * kq + 4 * s4);
+        // (four products to a chain: one chain over a head of 64 is off by 1.4e-7, chains of four that are added by 8.3e-8, as the per-token kernel)
+        v4f part[8];
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++)
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].x, qa[4 * s4], acc[mt], 0, 0, 0);
+        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].x, qa[4 * s4], zero, 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++)
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].y, qa[4 * s4 + 1], acc[mt], 0, 0, 0);
+        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].y, qa[4 * s4 + 1], part[mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++)
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].z, qa[4 * s4 + 2], acc[mt], 0, 0, 0);
+        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].z, qa[4 * s4 + 2], part[mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++)
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].w, qa[4 * s4 + 3], acc[mt], 0, 0, 0);
+        for (int mt = 0; mt < 8; mt++) acc[mt] += __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].w, qa[4 * s4 + 3], part[mt], 0, 0, 0);
     }
 
     // ---- softmax pieces of row j: 32 keys in this lane, the rest in lanes j+16, j+32, j+48 ----
@@ -690,26 +689,21 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     // ---- O = P V: A = P[row j][key 16s+4kq+i] = acc[s][i], B = V rows from LDS ----
     v4f o[NTO];
 #pragma unroll
-    for (int nt = 0; nt < NTO; nt++) o[nt] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NTO; nt++) o[nt] = zero;
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        {
+        v4f part[NTO];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float *vr = Vs + (16 * s + 4 * kq + i) * HD + NTO * j;
-                if constexpr (NTO == 4) {
-                    const float4 vb = *reinterpret_cast<const float4 *>(vr);
-                    o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.x, o[0], 0, 0, 0);
-                    o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.y, o[1], 0, 0, 0);
-                    o[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.z, o[2], 0, 0, 0);
-                    o[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.w, o[3], 0, 0, 0);
-                } else {
-                    const float2 vb = *reinterpret_cast<const float2 *>(vr);
-                    o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.x, o[0], 0, 0, 0);
-                    o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb.y, o[1], 0, 0, 0);
-                }
-            }
+        for (int i = 0; i < 4; i++) {
+            const float *vr = Vs + (16 * s + 4 * kq + i) * HD + NTO * j;
+            float vb[NTO];
+            if constexpr (NTO == 4) *reinterpret_cast<float4 *>(vb) = *reinterpret_cast<const float4 *>(vr);
+            else *reinterpret_cast<float2 *>(vb) = *reinterpret_cast<const float2 *>(vr);
+#pragma unroll
+            for (int nt = 0; nt < NTO; nt++) part[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(acc[s][i], vb[nt], i ? part[nt] : zero, 0, 0, 0);
         }
+#pragma unroll
+        for (int nt = 0; nt < NTO; nt++) o[nt] += part[nt];
     }
 
     // O tile: this lane holds rows 4*kq+r, columns d = NTO*j .. NTO*j+NTO-1

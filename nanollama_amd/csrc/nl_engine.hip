@@ -572,9 +572,8 @@ static const AttnKnobs &attn_knobs() {
 }
 
 template <int HD, int G>
-void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st) {
+void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st, bool f32_tile) {
     constexpr int QT = AttnTileQT<G>::value;
-    const bool f32_tile = attn_knobs().f32_tile;
     if (f32_tile) hipLaunchKernelGGL((attn_tile_kernel<HD, G, QT>), dim3(kvs, nsplit, (n + QT - 1) / QT), dim3(QT * G * 4), 0, st, P, n);
     else {
         constexpr int QT16 = AttnTile16QT<G>::value;
@@ -586,13 +585,13 @@ void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, hipStre
 inline int attn_tile16_qt(int gqa) { return NL_ATT16_MUL * (gqa == 1 ? 64 : gqa == 2 ? 32 : gqa == 8 ? 8 : 16); }   // = AttnTile16QT<G>::value
 inline bool attn_tile_supported(int gqa) { return gqa == 1 || gqa == 2 || gqa == 3 || gqa == 4 || gqa == 8; }
 template <int HD>
-hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st) {
+hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st, bool f32_tile) {
     switch (gqa) {
-    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, st); break;
-    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, st); break;
-    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, st); break;
-    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, st); break;
-    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, st); break;
+    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, st, f32_tile); break;
+    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, st, f32_tile); break;
+    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, st, f32_tile); break;
+    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, st, f32_tile); break;
+    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, st, f32_tile); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1642,17 +1641,17 @@ hipError_t launch_xsplit(int wtype, const float *x, int ldx, int cols, int n_tok
     return hipGetLastError();
 }
 
-// Which multi-token steps run on pgemm_kernel (nl_pgemm.h).  K-quant matrices: all of them.  The other formats: matrices of at least four
+// Which multi-token steps run on pgemm_kernel (nl_pgemm.h).  Files with K-quant matrices: all of them (QGemmParams::exact).  The others: matrices of at least four
 // 128-column chunks (narrower ones never fill its pipeline) and steps of at least 128 (Q4_0: shorter ones have nl_dgemm.h where that is
 // eligible) or PG_MIN tokens; below, the split-K launches of qgemm_kernel.
 constexpr int PG_MIN = 65;
 bool pgemm_ok(int wtype, int cols, int n_tokens) {
-    if (wtype == WT_Q4_K || wtype == WT_Q6_K) return true;
     const char *knob = getenv("NL_QG2_MIN_TOKENS");   // knob (tests, tools; read per launch so a test can flip it): a huge value disables
     const int min_n = knob ? atoi(knob) : wtype == WT_Q4_0 ? 128 : PG_MIN;
     return (wtype == WT_Q4_0 || wtype == WT_Q8_0 || wtype == WT_F16) && n_tokens >= min_n && cols >= 512;
 }
 bool pgemm_ok(const PackedMat &m, int n_tokens) { return pgemm_ok(m.wtype, m.cols, n_tokens); }
+bool pgemm_ok(int wtype, const QGemmParams &P) { return P.exact || pgemm_ok(wtype, P.cols, P.n_tokens); }
 
 // gate || up with the SwiGLU epilogue (nl_qgemm.h): 4 wavefronts x (gate tile, up tile) per workgroup, no split-K.
 // Worth it only when the unsplit grid fills the chip; the caller falls back to the plain launch + bswiglu otherwise.
@@ -1667,7 +1666,7 @@ bool qgemm_swiglu_fits(const PackedMat &m, int n_tokens) {
 hipError_t launch_qgemm_swiglu(int wtype, QGemmParams P, hipStream_t st) {
     P.nt16 = ((P.n_tokens + 63) / 64) * 4;
     P.ksplit = 1;
-    if (pgemm_ok(wtype, P.cols, P.n_tokens)) return pg_launch<QG_EPI_SWIGLU>(wtype, P, st);
+    if (pgemm_ok(wtype, P)) return pg_launch<QG_EPI_SWIGLU>(wtype, P, st);
     const dim3 grid((P.ntiles + QG_FUSED_WAVES - 1) / QG_FUSED_WAVES, (P.n_tokens + QG_TOK - 1) / QG_TOK, 1);
     switch (wtype) {
     case WT_Q4_0: hipLaunchKernelGGL((qgemm_kernel<WT_Q4_0, QG_FUSED_WAVES, 2, QG_EPI_SWIGLU>), grid, dim3(QG_FUSED_WAVES * 64), 0, st, P); break;
@@ -1689,7 +1688,7 @@ bool qgemm_rope_fits(const PackedMat &m, int n_tokens) {
 hipError_t launch_qgemm_rope(int wtype, QGemmParams P, hipStream_t st) {
     P.nt16 = ((P.n_tokens + 63) / 64) * 4;
     P.ksplit = 1;
-    if (pgemm_ok(wtype, P.cols, P.n_tokens)) return pg_launch<QG_EPI_ROPE>(wtype, P, st);
+    if (pgemm_ok(wtype, P)) return pg_launch<QG_EPI_ROPE>(wtype, P, st);
     P.row_groups = (P.ntiles + QG_WAVES - 1) / QG_WAVES;
     const dim3 grid(P.row_groups, (P.n_tokens + QG_TOK - 1) / QG_TOK, 1);
     switch (wtype) {
@@ -1726,7 +1725,7 @@ hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_bu
     const int tok_tiles = (P.n_tokens + QG_TOK - 1) / QG_TOK;
     const int nchunks = (P.cols / 32 + QG_KC - 1) / QG_KC;
     const int mats = P.q1 ? 2 : 1;
-    if (pgemm_ok(wtype, P.cols, P.n_tokens) && mats == 1) {
+    if (pgemm_ok(wtype, P) && mats == 1) {
         P.ksplit = 1;
         P.part = nullptr;
         if (ks_out) *ks_out = 1;
@@ -1806,9 +1805,20 @@ namespace {
 // 0.82 and 1.77 vs 2.19)
 const int NL_BATCH_MIN = getenv("NL_BATCH_MIN") ? atoi(getenv("NL_BATCH_MIN")) : 3;   // env: developer knob (tools/)
 
+// Does the file hold K-quant matrices?  Its multi-token steps keep float32 throughout then, as its single-token steps do: exact activation
+// parts for every product, whatever the matrix's own format (pgemm_kernel, PG_EXACT), and the float32 tile attention.
+bool kquant_file(const nl_engine *e) {
+    auto k = [](const PackedMat &m) { return m.wtype == WT_Q4_K || m.wtype == WT_Q6_K; };
+    bool any = k(e->lm_head);
+    for (const auto &L : e->layers) any = any || k(L.qkv) || k(L.wo) || k(L.gate) || k(L.up) || k(L.down);
+    return any;
+}
 bool batch_supported(const nl_engine *e) {
     if (e->G != 1 || e->force_tp_plan) return false;
-    auto ok = [](const PackedMat &m) { return m.wtype == WT_Q4_0 || m.wtype == WT_Q8_0 || m.wtype == WT_F16 || m.wtype == WT_Q4_K || m.wtype == WT_Q6_K; };
+    const bool exact = kquant_file(e);       // (an fp16 weight is no single bf16 value: such a mixture keeps the single-token plan)
+    auto ok = [&](const PackedMat &m) {
+        return m.wtype == WT_Q4_0 || m.wtype == WT_Q8_0 || (exact ? m.wtype == WT_Q4_K || m.wtype == WT_Q6_K : m.wtype == WT_F16);
+    };
     for (const auto &L : e->layers)
         if (!ok(L.qkv) || !ok(L.wo) || !ok(L.gate) || !ok(L.up) || !ok(L.down)) return false;
     return ok(e->lm_head) && !getenv("NL_NO_BATCH_PATH");
@@ -1836,11 +1846,12 @@ int batch_alloc(nl_engine *e, nl_engine::Batch &b, int cap_limit = 2048) {
     HIPCK(e, dalloc(&b.u, n * e->Is, &e->bytes_state));
     HIPCK(e, dalloc(&b.logits, (size_t)b.lm_cap * c.vocab, &e->bytes_state));
     {
-        const size_t nx = xfrag_uint4((int)std::max<size_t>(std::max<size_t>(HQ, c.dim), e->Is), (int)n);
+        const int form = kquant_file(e) ? FRAG_EXACT : 0;
+        const size_t nx = xfrag_uint4((int)std::max<size_t>(std::max<size_t>(HQ, c.dim), e->Is), (int)n, form);
         float *raw = nullptr;
         HIPCK(e, dalloc(&raw, nx * 4, &e->bytes_state));
         b.xfrag = reinterpret_cast<uint4 *>(raw);
-        const size_t nx2 = xfrag_uint4(std::max(e->Is, c.dim), (int)n);   // SiLU(gate) * up, written by the fused gate/up GEMM (or the folded norm's fragments)
+        const size_t nx2 = xfrag_uint4(std::max(e->Is, c.dim), (int)n, form);   // SiLU(gate) * up, written by the fused gate/up GEMM (or the folded norm's fragments)
         raw = nullptr;
         HIPCK(e, dalloc(&raw, nx2 * 4, &e->bytes_state));
         b.xfrag2 = reinterpret_cast<uint4 *>(raw);
@@ -1872,7 +1883,7 @@ int batch_alloc(nl_engine *e, nl_engine::Batch &b, int cap_limit = 2048) {
 // runs its five GEMM-shaped launches per layer on dgemm_kernel (nl_dgemm.h) with the RMSNorms folded around them
 bool dgemm_model_ok(const nl_engine *e) {
     const nl_config &c = e->cfg;
-    if (c.qk_norm || c.dim % 32 || c.n_layers <= 0 || c.dim / 32 > DG_SSQ_MAX_NRB) return false;   // (nrb: the consumer's LDS area for the partial sums of squares)
+    if (c.qk_norm || c.dim % 32 || c.n_layers <= 0 || c.dim / 32 > DG_SSQ_MAX_NRB || kquant_file(e)) return false;   // (nrb: the consumer's LDS area for the partial sums of squares)
     for (const auto &L : e->layers)
         if (!dgemm_mat_ok(L.qkv, false, 3, true) || !dgemm_mat_ok(L.wo, true, 2, false) || !dgemm_mat_ok(L.gate, true, 8, true) ||
             !dgemm_mat_ok(L.up, true, 8, true) || !dgemm_mat_ok(L.down, true, 2, false) || L.gate.rows != L.up.rows || L.gate.rows % 64 ||
@@ -1932,10 +1943,11 @@ bool dgemm_step_ok(const nl_engine *e, int n) {
 // (with resid / bias applied) when it ran unsplit, else split-K slabs in `part` for the consumer to add.
 hipError_t qg(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, const float *resid, hipStream_t st,
               GemmOut *res, float *part, const float *bias = nullptr, const uint4 *xf = nullptr,
-              const QGemmParams::NormOut *nout = nullptr, int x1 = 0, int out_q4 = 1) {
+              const QGemmParams::NormOut *nout = nullptr, int x1 = 0, int out_q4 = 1, int exact = 0) {
     QGemmParams P{};
     P.bias = bias;
     P.x1 = x1;
+    P.exact = exact;
     if (nout) { P.nrm_out = *nout; P.out_q4 = out_q4; }
     P.q = m.q; P.s = m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
     P.xf = xf ? xf : bt.xfrag; P.n_tokens = n; P.out = out; P.ldo = ldo; P.resid = resid;
@@ -1945,8 +1957,9 @@ hipError_t qg(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, flo
     return s;
 }
 
-hipError_t launch_qgemm_plain(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, hipStream_t st) {
+hipError_t launch_qgemm_plain(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, hipStream_t st, int exact) {
     QGemmParams P{};
+    P.exact = exact;
     P.q = m.q; P.s = m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
     P.xf = bt.xfrag; P.n_tokens = n; P.out = out; P.ldo = ldo;
     return launch_qgemm(m.wtype, P, st, bt.kpart, bt.kpart_cap);   // split-K + its own sum launch
@@ -1966,8 +1979,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     // (kv16_build_kernel) and a workgroup takes twice the rows, one workgroup per CU (AttnTile16ShadowQT).
     int n_live = 0, max_nparts = 0;
     bool kv16_on = false;
+    const int exact = kquant_file(e) ? 1 : 0;
+    const bool f32_tile = attn_knobs().f32_tile || exact;
+    auto form = [&](const PackedMat &next) { return (next.wtype == WT_Q4_0 ? FRAG_Q4_0 : 0) | (exact ? FRAG_EXACT : 0); };
     {
-        bool cons = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !attn_knobs().f32_tile && !attn_knobs().no_tile;
+        bool cons = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !f32_tile && !attn_knobs().no_tile;
         for (int i = 1; i < n && cons; i++) cons = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
         const int kv16_min = getenv("NL_KV16_MIN_TOKENS") ? atoi(getenv("NL_KV16_MIN_TOKENS")) : 256;   // (read per step: a test lowers it)
         kv16_on = cons && n >= kv16_min && b.kv16 != nullptr;
@@ -2037,7 +2053,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     bool fold = fold_knob && !c.qk_norm && D % 64 == 0 && c.n_layers > 0;
     for (int l = 0; l < c.n_layers && fold; l++) {
         const nl_engine::Layer &L = e->layers[l];
-        fold = pgemm_ok(L.wo, n) && pgemm_ok(L.down, n) && L.wo.ntiles % 4 == 0 && L.down.ntiles % 4 == 0 && pgemm_ok(L.qkv, n) && L.up.wtype == L.gate.wtype && pgemm_ok(L.gate, n);
+        fold = L.wo.ntiles % 4 == 0 && L.down.ntiles % 4 == 0 && L.up.wtype == L.gate.wtype &&
+               (exact || (pgemm_ok(L.wo, n) && pgemm_ok(L.down, n) && pgemm_ok(L.qkv, n) && pgemm_ok(L.gate, n)));
     }
     if (dg) fold = true;
     const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
@@ -2049,11 +2066,12 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const int x1_gemm = x1 || (pk && std::string(pk) == "fp16x1-gemm"), x1_attn = x1 || (pk && std::string(pk) == "fp16x1-attn");   // (developer: one half of the mode)
     // (pre-scales: the attention norm's consumer undoes sA and leaves sB for the WO producer; the feed-forward norm's consumer
     //  undoes sB and leaves sA for the down producer; layer 0's unfolded attention norm leaves the first sB)
-    float *const sA = b.nscale, *const sB = b.nscale + b.cap;
+    //  (bf16 parts have float32's exponents: none)
+    float *const sA = exact ? nullptr : b.nscale, *const sB = exact ? nullptr : b.nscale + b.cap;
     const QGemmParams::NormIn nin_attn{b.ssq, nrb, D, c.rms_eps, sA, sB}, nin_ffn{b.ssq, nrb, D, c.rms_eps, sB, sA},
                               nin_off{nullptr, 0, 0, 0.f, nullptr, nullptr};
     auto norm = [&](const float *w, const PackedMat &next, int item0, int cnt, float *scale_out = nullptr) {
-        BNormParams P{b.x, pend, w, c.rms_eps, D, item0, b.xfrag, ((cnt + 63) / 64) * 4, next.wtype == WT_Q4_0 ? 1 : 0, scale_out};
+        BNormParams P{b.x, pend, w, c.rms_eps, D, item0, b.xfrag, ((cnt + 63) / 64) * 4, form(next), scale_out};
         const int nu = D / 8;
         if (nu <= 256) hipLaunchKernelGGL(bnorm_kernel<1>, dim3(cnt), dim3(std::min(256, (nu + 63) / 64 * 64)), 0, st, P);
         else if (nu <= 512) hipLaunchKernelGGL(bnorm_kernel<2>, dim3(cnt), dim3(256), 0, st, P);
@@ -2070,18 +2088,18 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         bool rope_in_attn = false;
         const bool folded_in = fold && l > 0;      // the previous layer's down GEMM wrote this layer's Q|K|V input
         if (!folded_in) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
-        if (dg || (!c.qk_norm && qgemm_rope_fits(L.qkv, n))) {
+        if (dg || (!c.qk_norm && (exact || qgemm_rope_fits(L.qkv, n)))) {
             // Q|K|V, RoPE, biases and the KV store in ONE launch (QK-norm needs whole heads: unfused path)
             QGemmParams P{};
             const PackedMat &m = L.qkv;
             P.q = dg ? m.q3 : m.q; P.s = dg ? m.s3 : m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
             P.xf = folded_in ? b.xfrag2 : b.xfrag; P.nrm_in = folded_in ? nin_attn : nin_off;
-            P.n_tokens = n; P.ldo = (int)R; P.x1 = x1_gemm;
+            P.n_tokens = n; P.ldo = (int)R; P.x1 = x1_gemm; P.exact = exact;
             P.rope = QGemmParams::Rope{b.pos, b.stream, e->rope_cos, e->rope_sin, b.q, kc, vc, e->kv_stream_stride,
                                        L.bq, L.bk, L.bv, hd, e->Hs, e->KVs, c.seq_len, c.rope_conjugate, b.tcos, b.tsin, b.tkv};
             LCK(dg ? launch_dgemm_rope(P, st) : launch_qgemm_rope(m.wtype, P, st));
         } else {
-            LCK(qg(e, b, L.qkv, n, b.qkv, R, nullptr, st, &qkv_out, b.kpart, nullptr, nullptr, nullptr, x1_gemm));
+            LCK(qg(e, b, L.qkv, n, b.qkv, R, nullptr, st, &qkv_out, b.kpart, nullptr, nullptr, nullptr, x1_gemm, 1, exact));
             // decode batches (every token its own stream: no token of the step attends over another's K / V row), no QK-norm:
             // the attention launch rotates and stores its own q / k / v rows (attn_rope_prologue) -- no brope_kv launch.
             // Below position 128 that is the one-split FIN kernel; with two splits per token every split rotates q and the
@@ -2122,11 +2140,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                     else hipLaunchKernelGGL(kv16_build_kernel<32>, kg, dim3(512), 0, st, KB);
                     T.kv16 = b.kv16;
                 }
-                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st)
-                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st));
+                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st, f32_tile)
+                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st, f32_tile));
             } else if (fin_attn) {
                 // every position < 128: one split per row, the attention kernel normalises and writes the fragments
-                P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_q4 = L.wo.wtype == WT_Q4_0 ? 1 : 0;
+                P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_form = form(L.wo);
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
                 LCK(hd == 64 ? launch_attn_fin_hd<64>(e->gqa, P, dim3(e->KVs, 1, n), st)
@@ -2139,7 +2157,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             }
             if (!merged) {
             const bool tile16 = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;
-            BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, L.wo.wtype == WT_Q4_0 ? 1 : 0, tile16 ? 1 : 0};
+            BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, form(L.wo), tile16 && !exact ? 1 : 0};
             {
                 const long long units = (long long)n * e->Hs * hd / 8;
                 if (M.nparts && max_nparts <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
@@ -2162,22 +2180,22 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(dg_plain(L.wo, b.xfrag, L.bo, &nout));
         } else if (fold) {
             const QGemmParams::NormOut nout{L.ffn_norm, b.xfrag2, b.ssq, sB};
-            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm, L.gate.wtype == WT_Q4_0 ? 1 : 0));
+            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm, L.gate.wtype == WT_Q4_0 ? 1 : 0, exact));
         } else {
-            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, nullptr, x1_gemm));
+            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, nullptr, x1_gemm, 1, exact));
             LCK(norm(L.ffn_norm, L.gate, 0, n));
         }
         if (L.up.wtype != L.gate.wtype)   // (a mixed-type file: the fragment k-slot order differs per type)
             return e->fail(NL_ERR_UNSUPPORTED, "gate and up projections of different quantisation types");
         const uint4 *down_in = b.xfrag;
-        if (dg || qgemm_swiglu_fits(L.gate, n)) {
+        if (dg || exact || qgemm_swiglu_fits(L.gate, n)) {
             // gate, up and SiLU(gate) * up in ONE launch; h leaves as fragments in the second fragment store
             // (the first is still being read by other workgroups of this launch)
             QGemmParams P{};
             const PackedMat &m = L.gate;
             P.q = dg ? m.q3 : m.q; P.s = dg ? m.s3 : m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
             P.xf = fold ? b.xfrag2 : b.xfrag; P.nrm_in = fold ? nin_ffn : nin_off;
-            P.n_tokens = n; P.ldo = e->Is; P.x1 = x1_gemm;
+            P.n_tokens = n; P.ldo = e->Is; P.x1 = x1_gemm; P.exact = exact;
             P.q1 = dg ? L.up.q3 : L.up.q; P.s1 = dg ? L.up.s3 : L.up.s;
             P.xf_out = fold ? b.xfrag : b.xfrag2; P.out_q4 = L.down.wtype == WT_Q4_0 ? 1 : 0;
             LCK(dg ? launch_dgemm_swiglu(P, st) : launch_qgemm_swiglu(m.wtype, P, st));
@@ -2208,9 +2226,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         } else if (fold && l + 1 < c.n_layers) {
             const nl_engine::Layer &Ln = e->layers[l + 1];
             const QGemmParams::NormOut nout{Ln.attn_norm, b.xfrag2, b.ssq, sA};
-            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm, Ln.qkv.wtype == WT_Q4_0 ? 1 : 0));
+            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm, Ln.qkv.wtype == WT_Q4_0 ? 1 : 0, exact));
         } else {
-            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, nullptr, x1_gemm));
+            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, nullptr, x1_gemm, 1, exact));
         }
     }
     if (lm_mode) {
@@ -2228,7 +2246,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             hipLaunchKernelGGL(dg_argmax_kernel, dim3(n), dim3(1024), 0, st, reinterpret_cast<const uint2 *>(b.kpart), m.ntiles, b.ids);
         } else {
             LCK(norm(e->output_norm, e->lm_head, first, cnt));
-            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, b.logits, c.vocab, st));
+            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, b.logits, c.vocab, st, exact));
             hipLaunchKernelGGL(bargmax_kernel, dim3(cnt), dim3(1024), 0, st, b.logits, c.vocab, b.ids);
         }
         LCK(hipGetLastError());

@@ -1085,7 +1085,7 @@ struct AttnParams {
     // FIN variant (multi-token step whose positions are all < 128, i.e. one split): the normalised output leaves
     // as the WO GEMM's fp16 hi/lo fragments and battn_merge_kernel is not launched
     uint4 *fin_xf;
-    int fin_nt16, fin_q4;
+    int fin_nt16, fin_form;
     int x1;   // attn_tile16_kernel: prompt precision mode fp16x1 -- one fp16 product per q.k and p.v term instead of hi*hi + lo*hi + hi*lo
     // attn_tile16_kernel: the step's positions are pos_base + item (a prompt) when pos_base_valid -- the workgroup then
     // knows its key range without reading bpos, and its K / V requests leave at entry

@@ -1,4 +1,4 @@
-// nl_pgemm.h -- the multi-token GEMM of long token runs and of K-quant files: Y[n][row] = sum_k W[row][k] X[n][k], every weight format.
+// nl_pgemm.h -- the multi-token GEMM of long token runs and of K-quant files: Y[n][row] = sum_k W[row][k] X[n][k], every block format.
 //
 // Tile: a workgroup of four wavefronts owns RT 16-row weight tiles x 4 NTW 16-token tiles.  Its threads expand the weights of a
 // 128-column chunk ONCE into fp16 MFMA fragments in LDS (two buffers); every wavefront multiplies them against its own NTW token
@@ -16,17 +16,20 @@
 //
 // Arithmetic: weights as exact integers in fp16, x = hi + lo in fp16 (2^-22), float32 accumulation, then
 //   Q4_0 / Q8_0 (/ Q5_0)  acc += d_block * z                      per 32-column block (go/quant.go:74-94, :149-165)
-//   Q4_K                  z over 4 blocks of (scale * q): scale * q <= 63 * 15 is an exact fp16 integer; acc += d * z per chunk, and
-//                         acc -= (dmin * min) * sum(x) per block, sum(x) by an MFMA against ones (go/quant.go:296-323)
-//   Q6_K                  scale * (q - 32) reaches 4096, two fp16 parts (the low one at most 1): three MFMAs; acc += d * z per chunk
 //   F16                   its own operand, accumulated in the MFMA
+// Files with K-quant matrices (PG_EXACT, every matrix of such a file): what the single-token plan computes in float32 stays that -- x as
+// three bf16 parts (all 24 bits, all exponents), every product exact, sums in float32 with their rounding carried on:
+//   Q4_0 / Q8_0           as above
+//   Q4_K                  z over q - 8; acc += d * scale * z and acc -= (dmin * min - 8 d * scale) * sum(x) per block, sum(x) by MFMAs against ones (go/quant.go:296-323)
+//   Q6_K                  scale * (q - 32) has 13 bits, two bf16 parts: six MFMAs; acc += d * z per block
 //
 // Measured (us a launch, weights and fragments in L2; beside it the kernels that these launches ran on before, inside a model): Q4_0, 2047
 // tokens, 768 columns: Q|K|V 15.5 (21.8), gate and up 31.8 (40.5), WO / down (2048 columns) 10.5 / 17.7 (mean 23.5); F16, 993 tokens, 1536
 // columns: 26.7 (35.6), 52.3 (85.0), 17.9 / 36.3 (mean 43.2).  A 64 x 64 tile's block costs a wavefront about 310 cycles: 128 on the matrix
 // pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses), which a SIMD does not overlap with MFMAs
 // (matrix and vector cycles add up); larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
-// be 333 single-token steps: 152 ms, now 1.55 ms.
+// be 333 single-token steps: 151 ms, now 1.92 ms (1.49 with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
+// steps and 1.19e-7 now, and whose range ends at 65504).
 #pragma once
 #include "nl_qgemm.h"
 #include <type_traits>
@@ -40,7 +43,7 @@ __device__ __forceinline__ void pg_barrier() {
     asm volatile("" ::: "memory");
 }
 
-enum { PG_NONE = 0, PG_BLOCK = 1, PG_CHUNK = 2 };   // when a sum is multiplied by its scale
+enum { PG_NONE = 0, PG_BLOCK = 1 };   // when a sum is multiplied by its scale
 
 // (1024 + b) for the bytes b of u as packed fp16: the two halves of four bytes
 __device__ __forceinline__ h2_t pg_bytes_lo(uint32_t u) { return bits_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)); }
@@ -81,51 +84,87 @@ template <> struct PgFmt<WT_F16> {
     static __device__ __forceinline__ float scale(const uint32_t (&)[1], int) { return 1.f; }
     static __device__ __forceinline__ float least(const uint32_t (&)[1], int) { return 0.f; }
 };
-template <> struct PgFmt<WT_Q4_K> {
-    // pair p's 32 bytes: low nibbles = block 2p, high nibbles = block 2p + 1; words d | dmin and scale0 | min0 | scale1 | min1
-    static constexpr int CPP = 2, NC = 2, SW = 2, SC = PG_CHUNK, FR = 1;
-    static __device__ __forceinline__ int chunk(int, int i) { return i; }
-    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&s)[2], int h, int w, half8_t (&f)[1]) {
-        const uint4 &v = c[w >> 1];
-        const uint32_t a = (((w & 1) ? v.z : v.x) >> (4 * h)) & 0x0f0f0f0fu, b = (((w & 1) ? v.w : v.y) >> (4 * h)) & 0x0f0f0f0fu;
-        const float sc = (float)((s[1] >> (16 * h)) & 0xff);
-        const h2_t m = pg_h2(sc), o = pg_h2(-1024.f * sc);          // (1024 + q) sc - 1024 sc, one rounding of an exact value
-        f[0] = pg_join(__builtin_elementwise_fma(pg_bytes_lo(a), m, o), __builtin_elementwise_fma(pg_bytes_hi(a), m, o),
-                       __builtin_elementwise_fma(pg_bytes_lo(b), m, o), __builtin_elementwise_fma(pg_bytes_hi(b), m, o));
+// Files with K-quant matrices (PG_EXACT): x in three bf16 parts, weights as integers that bf16 holds exactly, so every product is exact
+__device__ __forceinline__ half8_t pg_bf16(const float (&v)[8]) {       // values of at most eight bits
+    uint32_t u[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) u[i] = __float_as_uint(v[i]);
+    return __builtin_bit_cast(half8_t, pack_bf16(u));
+}
+template <int WT> struct PgExact;
+template <> struct PgExact<WT_Q4_0> : PgFmt<WT_Q4_0> {
+    static __device__ __forceinline__ void part(const uint4 (&c)[1], const uint32_t (&)[1], int, int w, half8_t (&f)[1]) {
+        const uint32_t u = w == 0 ? c[0].x : w == 1 ? c[0].y : w == 2 ? c[0].z : c[0].w;
+        float v[8];                                                   // (k-slot order: load_x_slots)
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = (float)((u >> (8 * ((j & 1) * 2 + ((j >> 1) & 1)) + 4 * (j >> 2))) & 0xf) - 8.f;
+        f[0] = pg_bf16(v);
     }
-    static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int) { return h2f_bits(s[0] & 0xffff); }
-    static __device__ __forceinline__ float least(const uint32_t (&s)[2], int h) { return h2f_bits(s[0] >> 16) * (float)((s[1] >> (16 * h + 8)) & 0xff); }
 };
-template <> struct PgFmt<WT_Q6_K> {
-    // int8 (q - 32); words d and four int8 scales of 16 columns each
-    static constexpr int CPP = 4, NC = 2, SW = 2, SC = PG_CHUNK, FR = 2;
+template <> struct PgExact<WT_Q8_0> : PgFmt<WT_Q8_0> {
+    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&)[1], int, int w, half8_t (&f)[1]) {
+        const uint4 &q = c[w >> 1];
+        const uint32_t u[2] = {(w & 1) ? q.z : q.x, (w & 1) ? q.w : q.y};
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = (float)(int)(int8_t)(u[j >> 2] >> (8 * (j & 3)));
+        f[0] = pg_bf16(v);
+    }
+};
+template <> struct PgExact<WT_Q4_K> {
+    // pair p's 32 bytes: low nibbles = block 2p, high nibbles = block 2p + 1; words d | dmin and scale0 | min0 | scale1 | min1.
+    // q - 8 and min - 8 scale: the sums of q x and of x would mostly cancel (relative error of a 512-column model 1.06e-7 instead of 7.6e-8)
+    static constexpr int CPP = 2, NC = 2, SW = 2, SC = PG_BLOCK, FR = 1;
+    static __device__ __forceinline__ int chunk(int, int i) { return i; }
+    static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&)[2], int h, int w, half8_t (&f)[1]) {
+        const uint4 &q = c[w >> 1];
+        const uint32_t u[2] = {(((w & 1) ? q.z : q.x) >> (4 * h)) & 0x0f0f0f0fu, (((w & 1) ? q.w : q.y) >> (4 * h)) & 0x0f0f0f0fu};
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = (float)((u[j >> 2] >> (8 * (j & 3))) & 0xff) - 8.f;
+        f[0] = pg_bf16(v);
+    }
+    static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int h) { return h2f_bits(s[0] & 0xffff) * (float)((s[1] >> (16 * h)) & 0xff); }     // (17 bits)
+    static __device__ __forceinline__ float least(const uint32_t (&s)[2], int h) { return h2f_bits(s[0] >> 16) * (float)((s[1] >> (16 * h + 8)) & 0xff) - 8.f * scale(s, h); }
+};
+template <> struct PgExact<WT_Q6_K> {
+    // int8 (q - 32); words d and four int8 scales of 16 columns each.  scale * (q - 32) has 13 bits: two parts
+    static constexpr int CPP = 4, NC = 2, SW = 2, SC = PG_BLOCK, FR = 2;
     static __device__ __forceinline__ int chunk(int h, int i) { return 2 * h + i; }
     static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&s)[2], int h, int w, half8_t (&f)[2]) {
-        const uint4 &v = c[w >> 1];
-        const float sc = (float)(int8_t)(s[1] >> (8 * (2 * h + (w >> 1))));
-        const uint32_t u[2] = {((w & 1) ? v.z : v.x) ^ 0x80808080u, ((w & 1) ? v.w : v.y) ^ 0x80808080u};
-        const h2_t m = pg_h2(sc), off = pg_h2(1152.f);
-        h2_t hi[4], lo[4];
+        const uint4 &q = c[w >> 1];
+        const float sc = (float)(int)(int8_t)(s[1] >> (8 * (2 * h + (w >> 1))));
+        const uint32_t u[2] = {(w & 1) ? q.z : q.x, (w & 1) ? q.w : q.y};
+        float hi[8], lo[8];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const h2_t q = ((i & 1) ? pg_bytes_hi(u[i >> 1]) : pg_bytes_lo(u[i >> 1])) - off;
-            hi[i] = q * m;                                            // rounded to 11 bits
-            lo[i] = __builtin_elementwise_fma(q, m, -hi[i]);          // what the rounding took: exact, at most 1
+        for (int j = 0; j < 8; j++) {
+            const float v = (float)(int)(int8_t)(u[j >> 2] >> (8 * (j & 3))) * sc;
+            hi[j] = __uint_as_float(__float_as_uint(v) & 0xffff0000u);
+            lo[j] = v - hi[j];
         }
-        f[0] = pg_join(hi[0], hi[1], hi[2], hi[3]);
-        f[1] = pg_join(lo[0], lo[1], lo[2], lo[3]);
+        f[0] = pg_bf16(hi);
+        f[1] = pg_bf16(lo);
     }
     static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int) { return h2f_bits(s[0] & 0xffff); }
     static __device__ __forceinline__ float least(const uint32_t (&)[2], int) { return 0.f; }
 };
+typedef __bf16 pg_bf16x8 __attribute__((ext_vector_type(8)));
+template <bool BF16>
+__device__ __forceinline__ f32x4_t pg_mma(const uint4 &x, const half8_t &w, f32x4_t c) {
+    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pg_bf16x8, x), __builtin_bit_cast(pg_bf16x8, w), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x), w, c, 0, 0, 0);
+}
+enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 
 // EPI: QG_EPI_PLAIN (out / resid / bias, or split-K slabs; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
-// (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  X1: the single-product precision mode of Q4_0 prompts
-// (block scales multiplied into the fp16 weights, only the hi half of every activation).
-template <int WT, int RT, int NTW, int KW, int EPI, bool X1 = false>
+// (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  PREC: PG_HILO; PG_HI, the single-product precision mode of
+// Q4_0 prompts (block scales multiplied into the fp16 weights, only the hi half of every activation); PG_EXACT.
+template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO>
 __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmParams P) {
-    using F = PgFmt<WT>;
+    constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
+    using F = typename std::conditional_t<EXACT, PgExact<WT>, PgFmt<WT>>;
     static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");
+    constexpr int NP = X1 ? 1 : EXACT ? 3 : 2, PS = EXACT ? 3 : 2;      // parts of an activation that are read, and that are stored
     constexpr int KB = 4;                                   // blocks per chunk
     constexpr int ROWS = RT * TR, TOK = 64 * NTW, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
     constexpr int SC = X1 ? PG_NONE : F::SC;
@@ -145,10 +184,10 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     constexpr int TPW = FUSED ? RT / 2 : RT;                // row tiles of a matrix per workgroup
     const int nrb = (P.ntiles + TPW - 1) / TPW, ntb = (P.n_tokens + TOK - 1) / TOK, total = nrb * ntb, per = (total + 7) / 8;
     // blocks b, b + 8, ... run on one XCD, which takes a contiguous range of the tiles: of the operand that runs along the range each XCD
-    // reads an eighth, the other one it streams whole -- the smaller one (fragments are 4 bytes a value, weights 16 CPP bytes a pair and row)
+    // reads an eighth, the other one it streams whole -- the smaller one (fragments are 2 PS bytes a value, weights 16 CPP bytes a pair and row)
     const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (((int)blockIdx.x >> 3) >= per || id >= total) return;
-    const bool by_rows = (long long)P.ntiles * TR * (FUSED ? 2 : 1) * F::CPP > (long long)P.n_tokens * 16;
+    const bool by_rows = (long long)P.ntiles * TR * (FUSED ? 2 : 1) * F::CPP > (long long)P.n_tokens * 8 * PS;
     const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
 
     // staging items: pair kk of the chunk's two, row r, half h of the pair, row tile -- a wavefront's loads are runs of 32 bytes
@@ -197,26 +236,28 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
                 if (w == 0) *reinterpret_cast<float *>(s_mn + buf * SCB + (b * SCP + rt * 16 + i_r) * 4) = live ? F::least(r[i].s, i_h) : 0.f;
         }
     };
-    // activation fragments [block][token tile][hi / lo][lane] x 16 bytes: kernel argument + 32-bit offset, the block part wave-uniform
+    // activation fragments [block][token tile][part][lane] x 16 bytes: kernel argument + 32-bit offset, the block part wave-uniform
     const char *const xsrc = reinterpret_cast<const char *>(P.xf);
     unsigned xlane[NTW];
 #pragma unroll
-    for (int t = 0; t < NTW; t++) xlane[t] = ((unsigned)min(ttile0 + t, P.nt16 - 1) * 2u * QG_FRAG + (unsigned)lane) * 16u;
-    const unsigned xblock = (unsigned)P.nt16 * 2u * QG_FRAG * 16u;
-    uint4 xh[KB][NTW], xl[KB][NTW];
+    for (int t = 0; t < NTW; t++) xlane[t] = ((unsigned)min(ttile0 + t, P.nt16 - 1) * (unsigned)(PS * QG_FRAG) + (unsigned)lane) * 16u;
+    const unsigned xblock = (unsigned)P.nt16 * (unsigned)(PS * QG_FRAG) * 16u;
+    uint4 xp[NP][KB][NTW];
     auto xload = [&](int chunk, int b) {
         const unsigned uo = (unsigned)min(chunk * KB + b, nblocks - 1) * xblock;
 #pragma unroll
-        for (int t = 0; t < NTW; t++) {
-            xh[b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]));
-            if constexpr (!X1) xl[b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]) + QG_FRAG * 16);
-        }
+        for (int t = 0; t < NTW; t++)
+#pragma unroll
+            for (int k = 0; k < NP; k++) xp[k][b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]) + k * QG_FRAG * 16);
     };
     f32x4_t acc[RT][NTW];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
         for (int t = 0; t < NTW; t++) acc[rt][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // PG_EXACT: the sums of two chunks are kept apart and join the accumulators with what the addition drops carried on (Kahan): a plain
+    // chain over K / 32 blocks is further off than the single-token plan's lanes and trees (relative error at K = 10752 1.8e-7 against 1.1e-7)
+    [[maybe_unused]] f32x4_t part[EXACT ? RT : 1][NTW] = {}, lost[EXACT ? RT : 1][NTW] = {};
 
     const int step = P.ksplit * KW, niter = (nchunks - (int)blockIdx.z * KW + step - 1) / step;     // (every set runs as many chunks; past the end of K: zeros)
     int chunk = blockIdx.z * KW + kset;
@@ -251,7 +292,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
             if (p0 == 0) s_tok[t] = inv;
         }
     // producer: what its epilogue needs is requested here, ahead of the K loop -- behind it, every dependent fetch is a round trip of its own
-    constexpr int RQ = ROWS / 4, NIT = TOK * RQ / NTHR, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 ? NIT : 1;
+    constexpr int RQ = ROWS / 4, NIT = TOK * RQ / NTHR, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 && !(EXACT && KW == 1) ? NIT : 1;    // (EXACT, one set: no registers for it)
     [[maybe_unused]] f32x4_t res[NRES];
     [[maybe_unused]] const bool split = P.ksplit > 1, vec = (P.ldo & 3) == 0;
     [[maybe_unused]] const float *const resid = split ? nullptr : P.resid;
@@ -277,10 +318,11 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     // cores, group i + 1's weight fragments leave LDS and group i - 1's sums are scaled.  One barrier per chunk, in front of its last
     // group: the next chunk's fragments are then complete (all parts were stored by block 2) and the last group's are already in
     // registers, so the buffer that the next chunk's stores will overwrite has no reader left.
-    constexpr int RG = NTW == 1 ? 4 : 2, NG = RT / RG, STEPS = KB * NG;
+    constexpr int RG = NTW == 1 && !EXACT ? 4 : 2, NG = RT / RG, STEPS = KB * NG;
     static_assert(STEPS % 2 == 0, "ping-pong");
     half8_t wf[2][F::FR][RG];
-    f32x4_t z[2][RG][NTW], zc[SC == PG_CHUNK ? RT : 1][NTW], xs[2][NTW];
+    f32x4_t z[2][RG][NTW], xs[2][NTW];
+    [[maybe_unused]] f32x4_t zs[2][RG][NTW];      // PG_EXACT: sums of the products with a second or third part
     float dv[4][RG], mv[4][RG];         // of groups idx - 1 .. idx + 1
     auto read_w = [&](int bf, int idx) {
         const int b = idx / NG, r0 = (idx % NG) * RG;
@@ -304,20 +346,20 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
 #pragma unroll
             for (int t = 0; t < NTW; t++) {
                 const int rt = g * RG + q;
-                if constexpr (SC == PG_BLOCK) {
+                f32x4_t &to = EXACT ? part[EXACT ? rt : 0][t] : acc[rt][t];
+                if constexpr (EXACT) {
+                    // (as many roundings as possible at the size of a block's sum instead of the running one's)
+                    const f32x4_t all = z[idx & 1][q][t] + zs[idx & 1][q][t];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(z[idx & 1][q][t][j], dv[idx & 3][q], acc[rt][t][j]);
-                }
-                if constexpr (MINS) {
-#pragma unroll
-                    for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(-mv[idx & 3][q], xs[b & 1][t][j], acc[rt][t][j]);
-                }
-                if constexpr (SC == PG_CHUNK)
-                    if (b == KB - 1) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++) acc[rt][t][j] = fmaf(zc[rt][t][j], dv[idx & 3][q], acc[rt][t][j]);
+                    for (int j = 0; j < 4; j++) {
+                        if constexpr (MINS) to[j] += fmaf(all[j], dv[idx & 3][q], -mv[idx & 3][q] * xs[b & 1][t][j]);
+                        else to[j] = fmaf(all[j], dv[idx & 3][q], to[j]);
                     }
-                asm volatile("" : "+v"(acc[rt][t]));     // (hipcc otherwise sinks the scalings of a chunk below its MFMAs: 4 x the live registers)
+                } else if constexpr (SC == PG_BLOCK) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) to[j] = fmaf(z[idx & 1][q][t][j], dv[idx & 3][q], to[j]);
+                }
+                asm volatile("" : "+v"(to));     // (hipcc otherwise sinks the scalings of a chunk below its MFMAs: 4 x the live registers)
             }
     };
     if (niter > 0) {
@@ -336,28 +378,36 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
             else read_w(PAR ^ 1, 0);
             if constexpr (MINS)
                 if (g == 0) {
-                    const _Float16 one = (_Float16)1.f;
-                    const half8_t ones = {one, one, one, one, one, one, one, one};
+                    const half8_t ones = __builtin_bit_cast(half8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 #pragma unroll
-                    for (int t = 0; t < NTW; t++) xs[b & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xl[b][t]), ones, zero, 0, 0, 0);
-#pragma unroll
-                    for (int t = 0; t < NTW; t++) xs[b & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xh[b][t]), ones, xs[b & 1][t], 0, 0, 0);
+                    for (int t = 0; t < NTW; t++) {
+                        const f32x4_t less = pg_mma<EXACT>(xp[1][b][t], ones, pg_mma<EXACT>(xp[2][b][t], ones, zero));
+                        xs[b & 1][t] = pg_mma<EXACT>(xp[0][b][t], ones, zero) + less;
+                    }
                 }
-            auto mul = [&](int p, bool lo, bool start) {
+            // part k of the activations times part p of the weights
+            auto mul = [&](int p, int k, f32x4_t (&sum)[2][RG][NTW], bool start) {
 #pragma unroll
                 for (int q = 0; q < RG; q++)
 #pragma unroll
                     for (int t = 0; t < NTW; t++) {
-                        const int rt = g * RG + q;
-                        const half8_t x = __builtin_bit_cast(half8_t, lo ? xl[b][t] : xh[b][t]);
-                        if constexpr (SC == PG_BLOCK) z[idx & 1][q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], start ? zero : z[idx & 1][q][t], 0, 0, 0);
-                        else if constexpr (SC == PG_CHUNK) zc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], start && b == 0 ? zero : zc[rt][t], 0, 0, 0);
-                        else acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, wf[idx & 1][p][q], acc[rt][t], 0, 0, 0);
+                        f32x4_t &to = SC == PG_BLOCK ? sum[idx & 1][q][t] : acc[g * RG + q][t];
+                        to = pg_mma<EXACT>(xp[k][b][t], wf[idx & 1][p][q], SC == PG_BLOCK && start ? zero : to);
                     }
             };
-            if constexpr (!X1) mul(0, true, true);
-            if constexpr (F::FR == 2) mul(1, false, false);
-            mul(0, false, X1);
+            if constexpr (EXACT) {
+                // An MFMA rounds the sum with its C operand down, not to nearest: the large products have C = 0, and their sum meets the small
+                // ones' in scale_sums (all in one chain: mean error -1.9e-8 of the result at K = 2048, and 1.3e-7 instead of 1e-7 for Q6_K)
+#pragma unroll
+                for (int k = F::FR + 1; k > 0; k--)
+#pragma unroll
+                    for (int p = F::FR - 1; p >= 0; p--)
+                        if (k - p >= 0 && k - p < 3) mul(p, k - p, zs, k == F::FR + 1);
+                mul(0, 0, z, true);
+            } else {
+                if constexpr (!X1) mul(0, 1, z, true);
+                mul(0, 0, z, X1);
+            }
             if (idx) scale_sums(idx - 1);
             if (g == NG - 1) {
                 xload(nxt, b);
@@ -374,6 +424,20 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     for (int i = 0; i < niter; i += 2) {
         do_chunk(std::integral_constant<int, 0>{});
         if (i + 1 < niter) do_chunk(std::integral_constant<int, 1>{});
+        if constexpr (EXACT) {
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int t = 0; t < NTW; t++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float y = part[rt][t][j] - lost[rt][t][j], to = acc[rt][t][j] + y;
+                        const float l = (to - acc[rt][t][j]) - y;
+                        lost[rt][t][j] = l == l ? l : 0.f;       // (an infinity stays one)
+                        acc[rt][t][j] = to;
+                        part[rt][t][j] = 0.f;
+                    }
+        }
     }
 
     // accumulators -> LDS [token][row], then whole rows of a token
@@ -422,7 +486,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
             }
             float v[8];
             slots_from(P.out_q4, a, b, v);
-            if (n < P.n_tokens && hblk * 32 < P.rows) store_frag(P.xf_out, P.nt16, n, hblk, w, v);
+            if (n < P.n_tokens && hblk * 32 < P.rows) store_frag(P.xf_out, P.nt16, n, hblk, w, v, EXACT ? FRAG_EXACT : 0);
         }
         return;
     }
@@ -520,17 +584,17 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
             const f32x4_t yb = (*reinterpret_cast<const f32x4_t *>(sp + ob) * *reinterpret_cast<const f32x4_t *>(gp + ob)) * psc;
             float v[8];
             slots_from(P.out_q4, make_float4(ya[0], ya[1], ya[2], ya[3]), make_float4(yb[0], yb[1], yb[2], yb[3]), v);
-            store_frag(P.nrm_out.xf, P.nt16, n, c0 / 32, w, v);
+            store_frag(P.nrm_out.xf, P.nt16, n, c0 / 32, w, v, EXACT ? FRAG_EXACT : 0);
         }
     }
 }
 
-template <int WT, int EPI, bool X1>
+template <int WT, int EPI, int PREC>
 hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     auto go = [&](auto rt, auto ntw, auto kw) {
         constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT;
         const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + 64 * NTW - 1) / (64 * NTW));
-        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, X1>), dim3((total + 7) / 8 * 8, 1, P.ksplit), dim3(256 * KW), 0, st, P);
+        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC>), dim3((total + 7) / 8 * 8, 1, P.ksplit), dim3(256 * KW), 0, st, P);
         return hipGetLastError();
     };
     using std::integral_constant;
@@ -542,23 +606,34 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     // of one set leave every SIMD waiting on its own wavefront's instructions (Q4_0 768 x 2048 x 333 tokens, 72 tiles: 14.8 us one set,
     // 11.6 two; 64 x 128 tiles 20.3).  Up to two: 64 x 128 tiles of two sets (768 x 2048 x 2047: 17.7 us against 20.9 for 64 x 64, 22.0
     // for it with two sets).  Beyond, one set, and tiles that grow as the grid allows it (Q4_0 4096 x 768 x 2047, gate and up: 128 x 128
-    // 31.8 us, 64 x 128 35.0, 64 x 64 37.0; Q8_0's and the K-quants' expansions leave no registers for 128 x 128: 68.9 us against 62.2).
+    // 31.8 us, 64 x 128 35.0, 64 x 64 37.0; Q8_0's expansion leaves no registers for 128 x 128: 68.9 us against 62.2).
     const long long tiles = (long long)((P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4) * ((P.n_tokens + 63) / 64) * P.ksplit;
     if (tiles <= 256) return go(four, one, two);
-    if (tiles <= 512) return go(four, two, two);
-    if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one);
-    if constexpr (WT == WT_Q4_0 || WT == WT_F16)
-        if (tiles >= 1792) return go(eight, two, one);
-    return go(four, two, one);
+    // (three parts, the sums of a chunk pair and what their additions drop leave no registers for a second token tile: 46 to 150 spilled)
+    if constexpr (PREC == PG_EXACT) return go(four, one, one);
+    else {
+        if (tiles <= 512) return go(four, two, two);
+        if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one);
+        if constexpr (WT == WT_Q4_0 || WT == WT_F16)
+            if (tiles >= 1792) return go(eight, two, one);
+        return go(four, two, one);
+    }
 }
 template <int EPI>
 hipError_t pg_launch(int wtype, const QGemmParams &P, hipStream_t st) {
+    if (P.exact) {
+        switch (wtype) {
+        case WT_Q4_0: return pg_launch_as<WT_Q4_0, EPI, PG_EXACT>(P, st);
+        case WT_Q8_0: return pg_launch_as<WT_Q8_0, EPI, PG_EXACT>(P, st);
+        case WT_Q4_K: return pg_launch_as<WT_Q4_K, EPI, PG_EXACT>(P, st);
+        case WT_Q6_K: return pg_launch_as<WT_Q6_K, EPI, PG_EXACT>(P, st);
+        default: return hipErrorInvalidValue;
+        }
+    }
     switch (wtype) {
-    case WT_Q4_0: return P.x1 ? pg_launch_as<WT_Q4_0, EPI, true>(P, st) : pg_launch_as<WT_Q4_0, EPI, false>(P, st);
-    case WT_Q8_0: return pg_launch_as<WT_Q8_0, EPI, false>(P, st);
-    case WT_F16: return pg_launch_as<WT_F16, EPI, false>(P, st);
-    case WT_Q4_K: return pg_launch_as<WT_Q4_K, EPI, false>(P, st);
-    case WT_Q6_K: return pg_launch_as<WT_Q6_K, EPI, false>(P, st);
+    case WT_Q4_0: return P.x1 ? pg_launch_as<WT_Q4_0, EPI, PG_HI>(P, st) : pg_launch_as<WT_Q4_0, EPI, PG_HILO>(P, st);
+    case WT_Q8_0: return pg_launch_as<WT_Q8_0, EPI, PG_HILO>(P, st);
+    case WT_F16: return pg_launch_as<WT_F16, EPI, PG_HILO>(P, st);
     default: return hipErrorInvalidValue;
     }
 }

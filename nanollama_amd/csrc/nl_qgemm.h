@@ -46,6 +46,7 @@ struct QGemmParams {
     const uint4 *xf;     // activation fragments
     int nt16, n_tokens;
     int x1;              // prompt precision mode fp16x1 (pgemm_kernel, Q4_0): only the hi half of every activation is multiplied
+    int exact;           // files with K-quant matrices (pgemm_kernel): fragments of three bf16 parts (FRAG_EXACT)
     float *out;          // [N][ldo]
     int ldo;
     const float *resid;  // optional [N][ldo]: out = resid + y
@@ -99,8 +100,10 @@ struct QGemmParams {
     } nrm_in;
 };
 
-inline size_t xfrag_uint4(int cols, int n_tokens) {   // uint4 elements of a fragment store
-    return (size_t)(cols / 32) * (size_t)(((n_tokens + 63) / 64) * 4) * 2 * QG_FRAG;
+// Form of a fragment store, the sum of: the consumer's k-slot order is Q4_0's; an activation is three bf16 parts instead of fp16 hi + lo.
+enum { FRAG_Q4_0 = 1, FRAG_EXACT = 2 };
+inline size_t xfrag_uint4(int cols, int n_tokens, int form = 0) {   // uint4 elements of a fragment store
+    return (size_t)(cols / 32) * (size_t)(((n_tokens + 63) / 64) * 4) * (form & FRAG_EXACT ? 3 : 2) * QG_FRAG;
 }
 
 // k-slot -> element-of-block map shared by both MFMA operands.
@@ -210,6 +213,22 @@ __device__ __forceinline__ void split_hi_lo(float v, _Float16 &hi, _Float16 &lo)
     lo = (_Float16)(v - (float)h);
 }
 
+// x = p[0] + p[1] + p[2], three bf16 values: 24 bits and float32's exponents, so every finite float32 is held exactly (but for what lies below
+// 2^-133).  Cut, not rounded, so that the largest ones do not become infinities; an infinity or NaN is the first part alone.
+__device__ __forceinline__ void split_exact(float v, uint32_t (&p)[3]) {
+    asm("" : "+v"(v));
+    const bool special = (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
+    const float a = __uint_as_float(__float_as_uint(v) & 0xffff0000u), r = v - a, b = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+    p[0] = __float_as_uint(a) | (v != v ? 0x00400000u : 0u);       // (a NaN whose low bits are cut stays one)
+    p[1] = special ? 0u : __float_as_uint(b);
+    p[2] = special ? 0u : __float_as_uint(r - b);
+}
+// the upper halves of eight words
+__device__ __forceinline__ uint4 pack_bf16(const uint32_t (&u)[8]) {
+    return make_uint4(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u),
+                      __builtin_amdgcn_perm(u[5], u[4], 0x07060302u), __builtin_amdgcn_perm(u[7], u[6], 0x07060302u));
+}
+
 // x -> fp16 hi/lo fragments.  One thread per (block, 16-token tile, slot group w, token): reads the 8 k-slot
 // elements of its token (two float4), writes the hi and the lo fragment entry (16 bytes each; the 16 tokens of a
 // tile are adjacent, so a 16-lane group writes 256 contiguous bytes).  Tokens beyond n_tokens are zero.
@@ -243,22 +262,37 @@ __global__ void xsplit_kernel(const float *x, int ldx, int nblocks, int n_tokens
 
 // the 8 k-slots (w, j) of a 32-column block from its two float4 groups a (columns offa..+3) and b (offb..+3),
 // slot_offsets() below: only the two middle lanes of each group differ between the Q4_0 and the linear order
-__device__ __forceinline__ void slots_from(int q4, const float4 &a, const float4 &b, float (&v)[8]) {
+__device__ __forceinline__ void slots_from(int form, const float4 &a, const float4 &b, float (&v)[8]) {
+    const bool q4 = form & FRAG_Q4_0;
     v[0] = a.x; v[1] = q4 ? a.z : a.y; v[2] = q4 ? a.y : a.z; v[3] = a.w;
     v[4] = b.x; v[5] = q4 ? b.z : b.y; v[6] = q4 ? b.y : b.z; v[7] = b.w;
 }
-__device__ __forceinline__ void slot_offsets(int q4, int w, int &offa, int &offb) {
+__device__ __forceinline__ void slot_offsets(int form, int w, int &offa, int &offb) {
+    const bool q4 = form & FRAG_Q4_0;
     offa = q4 ? 4 * w : 8 * w;
     offb = q4 ? 16 + 4 * w : 8 * w + 4;
 }
 
 // element (0..31) of a 32-column block that k-slot (w, j) of the MFMA operands holds (nl_qgemm.h load_x_slots)
-__device__ __forceinline__ int slot_elem(int q4, int w, int j) {
-    return q4 ? ((j >> 2) * 16 + 4 * w + ((j & 1) << 1) + ((j >> 1) & 1)) : 8 * w + j;
+__device__ __forceinline__ int slot_elem(int form, int w, int j) {
+    return form & FRAG_Q4_0 ? ((j >> 2) * 16 + 4 * w + ((j & 1) << 1) + ((j >> 1) & 1)) : 8 * w + j;
 }
 
-// the 8 k-slots (block blk, slot group w) of token n -> hi/lo entries of the fragment store
-__device__ __forceinline__ void store_frag(uint4 *xf, int nt16, int n, int blk, int w, const float (&v)[8]) {
+// the 8 k-slots (block blk, slot group w) of token n -> hi/lo entries of the fragment store, or its three parts (form)
+__device__ __forceinline__ void store_frag(uint4 *xf, int nt16, int n, int blk, int w, const float (&v)[8], int form = 0) {
+    if (form & FRAG_EXACT) {
+        uint32_t u[3][8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            uint32_t p[3];
+            split_exact(v[j], p);
+            u[0][j] = p[0]; u[1][j] = p[1]; u[2][j] = p[2];
+        }
+        const long long bt = (long long)blk * nt16 + (n >> 4);
+#pragma unroll
+        for (int k = 0; k < 3; k++) xf[(bt * 3 + k) * QG_FRAG + w * 16 + (n & 15)] = pack_bf16(u[k]);
+        return;
+    }
     half8_t hi, lo;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
