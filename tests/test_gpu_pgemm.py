@@ -48,6 +48,39 @@ def test_product_against_float64(hip, kind, rows, cols, n):
     assert (np.abs(got - xd @ wd.T) <= bound).all()
 
 
+class Scaled:
+    """A parsed file with the weights of some matrices multiplied by a power of two (their scales, or the fp16 weights themselves)."""
+
+    def __init__(self, g, part, factor):
+        self.meta, self.tensor_order, self.g, self.part, self.factor = g.meta, g.tensor_order, g, part, factor
+
+    def get_tensor(self, name):
+        raw, info = self.g.get_tensor(name)
+        if self.part in name:
+            b = np.array(raw).reshape(-1, {gguf.GGML_F16: 2, gguf.GGML_Q8_0: 34, gguf.GGML_Q4_0: 18}[info.type])
+            d = (b[:, :2].copy().view(np.float16) * np.float32(self.factor)).astype(np.float16)
+            assert np.isfinite(d).all()
+            b[:, :2], raw = d.view(np.uint8), b.reshape(-1)
+        return raw, info
+
+
+# a residual stream that grows 2^17-fold in one layer, as far as fp16 scales go: fragments that leave before the norm is known overflow
+@pytest.mark.parametrize("kind,n", [("f16", 66), ("f16", 200), ("q8_0", 66), ("q8_0", 300), ("q4_0", 200)])
+def test_stream_that_grows_within_a_layer(hip, orc, tmp_path, kind, n):
+    shape = replace(synth.TIERS["tiny"], name="grows", dim=576, n_head=9, n_kv_head=3, interm=608, seq_len=320, n_layer=3)
+    p = tmp_path / "g.gguf"
+    synth.generate_gguf(str(p), shape, kind, 29)
+    g = Scaled(gguf.load_gguf(str(p)), "blk.1.ffn_down", 2.0 ** 17)
+    toks = synth.prompt_ids(n, shape.vocab, seed=5)
+    ref, dev = orc.OracleModel(g), hip.load_llama_model(g)
+    for pos, tok in enumerate(toks):
+        want = ref.forward(tok, pos)
+    dev.prefill(toks)
+    assert np.isfinite(want).all() and np.isfinite(dev.state.logits).all()
+    assert np.abs(dev.state.logits - want).max() <= LOGIT_TOL * max(1.0, float(want.std()))
+    dev.close()
+
+
 @pytest.mark.parametrize("kind", ["q4_k", "q6_k"])
 @pytest.mark.parametrize("n", [3, 16, 64, 65, 200])
 def test_kquant_prompt_against_oracle(hip, orc, tmp_path, kind, n):
