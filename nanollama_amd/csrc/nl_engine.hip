@@ -1803,7 +1803,12 @@ namespace {
 // below this many tokens the ~10 launches per layer of the multi-token step cost more than n single-token steps
 // (measured: 2 streams nano 0.61 ms batched vs 0.55 ms as two single steps, goldie 1.77 vs 1.47; 3 streams 0.61 vs
 // 0.82 and 1.77 vs 2.19)
-const int NL_BATCH_MIN = getenv("NL_BATCH_MIN") ? atoi(getenv("NL_BATCH_MIN")) : 3;   // env: developer knob (tools/)
+const int NL_BATCH_MIN = getenv("NL_BATCH_MIN") ? atoi(getenv("NL_BATCH_MIN")) : 0;   // env: developer knob (tools/), 0 = the rule
+constexpr int BATCH_MIN = 3;
+// files with K-quant matrices, whose products are dearer: us a step, 3 / 4 streams on this path against 3 / 4 single-token steps: 173M Q4_K 1399 / 1399
+// against 1342 / 1783, Q6_K 1521 / 1517 against 1266 / 1683, 841M Q4_K 3087 / 3087 against 2347 / 3124, four layers of 4096 columns 1207 / 1215
+// against 801 / 1062; 6 streams 1397, 1521, 3090, 1209 against 2662, 2521, 4690, 1599
+constexpr int BATCH_MIN_KQUANT = 5;
 
 // Does the file hold K-quant matrices?  Its multi-token steps keep float32 throughout then, as its single-token steps do: exact activation
 // parts for every product, whatever the matrix's own format (pgemm_kernel, PG_EXACT), and the float32 tile attention.
@@ -1823,6 +1828,7 @@ bool batch_supported(const nl_engine *e) {
         if (!ok(L.qkv) || !ok(L.wo) || !ok(L.gate) || !ok(L.up) || !ok(L.down)) return false;
     return ok(e->lm_head) && !getenv("NL_NO_BATCH_PATH");
 }
+int batch_min(const nl_engine *e) { return NL_BATCH_MIN ? NL_BATCH_MIN : kquant_file(e) ? BATCH_MIN_KQUANT : BATCH_MIN; }
 
 int batch_alloc(nl_engine *e, nl_engine::Batch &b, int cap_limit = 2048) {
     if (b.ready) return NL_OK;
@@ -3520,7 +3526,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     if ((rc = note_positions(e, stream, pos0, n))) return rc;
-    if (n >= NL_BATCH_MIN && batch_supported(e)) {
+    if (n >= batch_min(e) && batch_supported(e)) {
         // multi-token path: 64-token tiles on the matrix cores; causality comes from each token's own pos
         { std::lock_guard<std::mutex> setup(g_setup_mu); if ((rc = batch_alloc(e, e->bt)) || (rc = dgemm_prepare(e))) return rc; }
         nl_engine::Batch &b = e->bt;
@@ -3583,7 +3589,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
     if (int qrc = pd_session_close(e)) return qrc;
     for (int i = 0; i < n; i++)
         if ((rc = note_positions(e, streams[i], pos[i], 1))) return rc;
-    if (n >= NL_BATCH_MIN && batch_supported(e)) {
+    if (n >= batch_min(e) && batch_supported(e)) {
         // The streams of a batch are independent: cut it into groups of >= 16 that step concurrently, each on its own HIP
         // stream with its own step buffers, so that one dependent chain's launch heads and memory round trips overlap
         // another's work (a 64-stream step of the 841M tier is ~224 launches of <= 144 workgroups on a 256-CU chip).  The

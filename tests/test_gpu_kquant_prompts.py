@@ -119,7 +119,7 @@ def test_large_grids(tmp_path, monkeypatch, types):
 # rows that fill no 64-row workgroup (heads of 32, 8 + 2 of them: 20 row tiles, a vocabulary of 520), biases, conjugate rotation, QK-norm
 @pytest.mark.parametrize("kind", ["q4_k", "q6_k"])
 @pytest.mark.parametrize("variant", ["bias_conj", "qk_norm"])
-@pytest.mark.parametrize("n", [3, 64, 133])
+@pytest.mark.parametrize("n", [5, 64, 133])
 def test_variants_against_the_oracle(tmp_path, kind, variant, n):
     from nanollama_amd import model as hip
     from oracle import oracle as orc
@@ -159,3 +159,26 @@ def test_streams_are_as_exact_as_the_single_token_plan(tmp_path, monkeypatch):
         dev.close()
     print(f"\nstreams {err[0]:.3g}, one by one {err[1]:.3g}")
     assert err[0] <= 1.25 * err[1]
+
+
+@pytest.mark.parametrize("kind", ["q4_k", "q6_k"])
+def test_few_tokens_run_the_single_token_plan(tmp_path, kind):
+    # (below five tokens a multi-token step costs more than the single-token ones: the same bits)
+    from nanollama_amd import model as hip
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), SHAPE, kind, 19)
+    dev = hip.load_llama_model(gguf.load_gguf(str(p)), max_streams=5)
+    for n in (3, 4, 5):
+        dev.prefill(list(range(7, 7 + n)))
+        got = dev.state.logits.copy()
+        dev.reset()
+        for i in range(n):
+            dev.forward(7 + i, i)
+        assert np.array_equal(got, dev.state.logits) == (n < 5), n
+        _, rows = dev.forward_batch(list(range(n)), [40 + s for s in range(n)], [0] * n, want_logits=True)
+        one = []
+        for s in range(n):
+            dev.forward(40 + s, 0, s)
+            one.append(dev.state.logits.copy())
+        assert np.array_equal(rows, one) == (n < 5), n
+    dev.close()
