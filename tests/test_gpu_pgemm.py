@@ -115,3 +115,25 @@ def test_kquant_streams_equal_the_single_token_plan(hip, tmp_path):
         dev.forward(30 + s, s + 1, s)
         assert np.abs(rows[s] - dev.state.logits).max() <= LOGIT_TOL * max(1.0, float(dev.state.logits.std()))
     dev.close()
+
+
+def test_a_changed_threshold_reaches_recorded_steps(hip, tmp_path, monkeypatch):
+    # a decode step's launches are recorded once per geometry: NL_QG2_MIN_TOKENS, read per launch, is part of what they are kept by
+    shape = replace(synth.TIERS["tiny"], name="knob", dim=512, n_head=8, n_kv_head=2, interm=768, seq_len=64)
+    p = tmp_path / "k.gguf"
+    synth.generate_gguf(str(p), shape, "q8_0", 31)
+    g = gguf.load_gguf(str(p))
+
+    def step(dev):
+        for s in range(8):
+            dev.reset(s)
+        return dev.forward_batch(list(range(8)), list(range(20, 28)), [0] * 8, want_logits=True)[1].copy()
+    dev = hip.load_llama_model(g, max_streams=8)
+    split = step(dev)
+    monkeypatch.setenv("NL_QG2_MIN_TOKENS", "8")
+    changed = step(dev)
+    dev.close()
+    dev = hip.load_llama_model(g, max_streams=8)
+    fresh = step(dev)
+    dev.close()
+    assert np.array_equal(changed, fresh) and not np.array_equal(changed, split)
