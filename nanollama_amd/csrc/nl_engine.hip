@@ -1659,7 +1659,7 @@ constexpr int QG_FUSED_WAVES = 4;
 bool qgemm_swiglu_fits(const PackedMat &m, int n_tokens) {
     if (pgemm_ok(m, n_tokens)) return true;
     const int ntiles = m.ntiles;
-    static const int min_wg = getenv("NL_FUSED_SWIGLU_MIN_WG") ? atoi(getenv("NL_FUSED_SWIGLU_MIN_WG")) : 128;   // knob: tests force 1, tools disable with a huge value
+    static const int min_wg = getenv("NL_FUSED_SWIGLU_MIN_WG") ? atoi(getenv("NL_FUSED_SWIGLU_MIN_WG")) : 128;   // knob (qgemm_kernel's launches): tests force 1, tools disable with a huge value
     // (a step of <= 32 tokens runs the plain kernel on one / two 16-token tiles instead: big x 8 streams 7.76 -> 7.55 ms)
     return (n_tokens > 32 || min_wg <= 1) && ((ntiles + QG_FUSED_WAVES - 1) / QG_FUSED_WAVES) * ((n_tokens + QG_TOK - 1) / QG_TOK) >= min_wg;
 }
@@ -1682,7 +1682,7 @@ hipError_t launch_qgemm_swiglu(int wtype, QGemmParams P, hipStream_t st) {
 bool qgemm_rope_fits(const PackedMat &m, int n_tokens) {
     if (pgemm_ok(m, n_tokens)) return true;
     const int ntiles = m.ntiles;
-    static const int min_wg = getenv("NL_FUSED_ROPE_MIN_WG") ? atoi(getenv("NL_FUSED_ROPE_MIN_WG")) : 128;   // knob: tests force 1
+    static const int min_wg = getenv("NL_FUSED_ROPE_MIN_WG") ? atoi(getenv("NL_FUSED_ROPE_MIN_WG")) : 128;   // knob (qgemm_kernel's launches): tests force 1
     return ((ntiles + QG_WAVES - 1) / QG_WAVES) * ((n_tokens + QG_TOK - 1) / QG_TOK) >= min_wg;
 }
 hipError_t launch_qgemm_rope(int wtype, QGemmParams P, hipStream_t st) {
@@ -1726,8 +1726,6 @@ hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_bu
     const int nchunks = (P.cols / 32 + QG_KC - 1) / QG_KC;
     const int mats = P.q1 ? 2 : 1;
     if (pgemm_ok(wtype, P) && mats == 1) {
-        P.ksplit = 1;
-        P.part = nullptr;
         if (ks_out) *ks_out = 1;
         return pg_launch<QG_EPI_PLAIN>(wtype, P, st);
     }

@@ -156,7 +156,7 @@ __device__ __forceinline__ f32x4_t pg_mma(const uint4 &x, const half8_t &w, f32x
 }
 enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 
-// EPI: QG_EPI_PLAIN (out / resid / bias, or split-K slabs; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
+// EPI: QG_EPI_PLAIN (out / resid / bias; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
 // (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  PREC: PG_HILO; PG_HI, the single-product precision mode of
 // Q4_0 prompts (block scales multiplied into the fp16 weights, only the hi half of every activation); PG_EXACT.
 template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO>
@@ -259,15 +259,13 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     // chain over K / 32 blocks is further off than the single-token plan's lanes and trees (relative error at K = 10752 1.8e-7 against 1.1e-7)
     [[maybe_unused]] f32x4_t part[EXACT ? RT : 1][NTW] = {}, lost[EXACT ? RT : 1][NTW] = {};
 
-    const int step = P.ksplit * KW, niter = (nchunks - (int)blockIdx.z * KW + step - 1) / step;     // (every set runs as many chunks; past the end of K: zeros)
-    int chunk = blockIdx.z * KW + kset;
+    const int niter = (nchunks + KW - 1) / KW;               // (every set runs as many chunks; past the end of K: zeros)
+    int chunk = kset;
     Raw rb[2][IPT];                                         // raw weights of the next chunk and of the one after it
-    if (niter > 0) {
-        stage_load(chunk, rb[1]);
+    stage_load(chunk, rb[1]);
 #pragma unroll
-        for (int b = 0; b < KB; b++) xload(chunk, b);
-        stage_load(chunk + step, rb[0]);
-    }
+    for (int b = 0; b < KB; b++) xload(chunk, b);
+    stage_load(chunk + KW, rb[0]);
     // folded RMSNorm, consumer side: 1 / rms of this workgroup's tokens from the producer's partial sums of squares, 256 / TOK threads a token
     if constexpr (EPI != QG_EPI_PLAIN)
         if (P.nrm_in.ssq) {
@@ -294,8 +292,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     // producer: what its epilogue needs is requested here, ahead of the K loop -- behind it, every dependent fetch is a round trip of its own
     constexpr int RQ = ROWS / 4, NIT = TOK * RQ / NTHR, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 && !(EXACT && KW == 1) ? NIT : 1;    // (EXACT, one set: no registers for it)
     [[maybe_unused]] f32x4_t res[NRES];
-    [[maybe_unused]] const bool split = P.ksplit > 1, vec = (P.ldo & 3) == 0;
-    [[maybe_unused]] const float *const resid = split ? nullptr : P.resid;
+    [[maybe_unused]] const bool vec = (P.ldo & 3) == 0;
+    [[maybe_unused]] const float *const resid = P.resid;
     [[maybe_unused]] auto load_res = [&](int i) {
         const int it = i * NTHR + (int)threadIdx.x, a = it % RQ, n = min(tok0 + it / RQ, P.n_tokens - 1), row = row0 + 4 * a;
         return resid && vec && row + 3 < P.rows ? *reinterpret_cast<const f32x4_t *>(resid + (size_t)n * P.ldo + row) : f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -304,16 +302,14 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
         if (NRES == NIT)
 #pragma unroll
             for (int i = 0; i < NRES; i++) res[i] = load_res(i);
-        if (P.nrm_out.w && !split) {
+        if (P.nrm_out.w) {
             for (int i = threadIdx.x; i < ROWS; i += NTHR) s_gain[i] = P.nrm_out.w[min(row0 + i, P.rows - 1)];
             for (int i = threadIdx.x; i < TOK; i += NTHR) s_tok[i] = P.nrm_out.scale ? P.nrm_out.scale[min(tok0 + i, P.n_tokens - 1)] : 1.0f;
         }
     }
-    if (niter > 0) {
 #pragma unroll
-        for (int w = 0; w < 4; w++) stage_part(chunk, 0, w, rb[1]);
-        stage_load(chunk + 2 * step, rb[1]);
-    }
+    for (int w = 0; w < 4; w++) stage_part(chunk, 0, w, rb[1]);
+    stage_load(chunk + 2 * KW, rb[1]);
     // The K loop is a pipeline of groups (RG row tiles x NTW token tiles: four independent MFMA chains): while group i is on the matrix
     // cores, group i + 1's weight fragments leave LDS and group i - 1's sums are scaled.  One barrier per chunk, in front of its last
     // group: the next chunk's fragments are then complete (all parts were stored by block 2) and the last group's are already in
@@ -362,14 +358,12 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
                 asm volatile("" : "+v"(to));     // (hipcc otherwise sinks the scalings of a chunk below its MFMAs: 4 x the live registers)
             }
     };
-    if (niter > 0) {
-        pg_barrier();
-        read_w(0, 0);
-    }
+    pg_barrier();
+    read_w(0, 0);
     // one chunk; PAR: its parity (which buffer and which raw registers)
     auto do_chunk = [&](auto par_tag) {
         constexpr int PAR = decltype(par_tag)::value;
-        const int nxt = chunk + step;
+        const int nxt = chunk + KW;
 #pragma unroll
         for (int idx = 0; idx < STEPS; idx++) {
             const int b = idx / NG, g = idx % NG;
@@ -414,7 +408,7 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
                 if (b < KB - 1) stage_part(nxt, PAR ^ 1, b, rb[PAR]);
                 if (b == KB - 2) {
                     stage_part(nxt, PAR ^ 1, KB - 1, rb[PAR]);
-                    stage_load(nxt + 2 * step, rb[PAR]);
+                    stage_load(nxt + 2 * KW, rb[PAR]);
                 }
             }
         }
@@ -531,9 +525,8 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
         return;
     }
     if constexpr (EPI == QG_EPI_PLAIN) {
-        float *const dst = split ? P.part + (long long)blockIdx.z * P.n_tokens * P.ldo : P.out;
-        const float *const bias = split ? nullptr : P.bias;
-        const bool fold = P.nrm_out.w && !split;
+        const float *const bias = P.bias;
+        const bool fold = P.nrm_out.w != nullptr;
         constexpr int UN = NIT < 8 ? NIT : 8;
 #pragma unroll 1
         for (int i0 = 0; i0 < NIT; i0 += UN) {
@@ -548,14 +541,14 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
                 if (vec && row + 3 < P.rows) {
                     if (bias) v[i] += *reinterpret_cast<const f32x4_t *>(bias + row);
                     if (resid) v[i] += r[i];
-                    if (n < P.n_tokens) *reinterpret_cast<f32x4_t *>(dst + off) = v[i];
+                    if (n < P.n_tokens) *reinterpret_cast<f32x4_t *>(P.out + off) = v[i];
                 } else if (n < P.n_tokens) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         if (row + j >= P.rows) continue;
                         float y = v[i][j] + (bias ? bias[row + j] : 0.f);
                         if (resid) y += resid[off + j];
-                        dst[off + j] = y;
+                        P.out[off + j] = y;
                     }
                 }
                 if (fold) {
@@ -594,7 +587,7 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     auto go = [&](auto rt, auto ntw, auto kw) {
         constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT;
         const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + 64 * NTW - 1) / (64 * NTW));
-        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC>), dim3((total + 7) / 8 * 8, 1, P.ksplit), dim3(256 * KW), 0, st, P);
+        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC>), dim3((total + 7) / 8 * 8), dim3(256 * KW), 0, st, P);
         return hipGetLastError();
     };
     using std::integral_constant;
@@ -607,7 +600,7 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     // 11.6 two; 64 x 128 tiles 20.3).  Up to two: 64 x 128 tiles of two sets (768 x 2048 x 2047: 17.7 us against 20.9 for 64 x 64, 22.0
     // for it with two sets).  Beyond, one set, and tiles that grow as the grid allows it (Q4_0 4096 x 768 x 2047, gate and up: 128 x 128
     // 31.8 us, 64 x 128 35.0, 64 x 64 37.0; Q8_0's expansion leaves no registers for 128 x 128: 68.9 us against 62.2).
-    const long long tiles = (long long)((P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4) * ((P.n_tokens + 63) / 64) * P.ksplit;
+    const long long tiles = (long long)((P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4) * ((P.n_tokens + 63) / 64);
     if (tiles <= 256) return go(four, one, two);
     // (three parts, the sums of a chunk pair and what their additions drop leave no registers for a second token tile: 46 to 150 spilled)
     if constexpr (PREC == PG_EXACT) return go(four, one, one);
