@@ -32,3 +32,28 @@ def test_fused_launch_against_the_general_plan_at_every_pass(tmp_path, monkeypat
     assert dev.decode_greedy(5, 1018, 12) == plain.decode_greedy(5, 1018, 12)      # and across the limit of the shared ones
     assert dev.last_error() == ""
     dev.close(); plain.close()
+
+
+def test_two_passes_per_helper_of_the_kv_group(tmp_path, monkeypatch):
+    # 24 kv groups of 2 heads and 192 output tiles: no blocks past the groups, the feed-forward half in one launch -- a head's passes 0 .. 6 are
+    # shared with three blocks of its own group, two each from position 1024 on
+    from nanollama_amd import model as hip
+    shape = synth.ModelShape("limits_wide", 2, 3072, 48, 24, 512, seq_len=2048, interm=3072)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), shape, "q4_0", 84, mode="qrand")
+    g = gguf.load_gguf(str(p))
+    dev = hip.load_llama_model(g)
+    info = dev.plan_info()
+    assert info["fused_mode"] == 4 and info["fused_max_pos"] == 2048, info
+    monkeypatch.setenv("NL_FUSED_ATTN", "0")
+    plain = hip.load_llama_model(g)
+    toks = synth.prompt_ids(2040, shape.vocab, seed=12)
+    for m in (dev, plain):
+        m.prefill(toks, want_logits=False)
+    for pos in (255, 256, 1023, 1024, 1279, 1280, 1535, 1536, 1792, 2046):
+        for m in (dev, plain):
+            m.forward(toks[min(pos, 2039)] % 500 + 3, pos)
+        assert np.abs(dev.state.logits - plain.state.logits).max() <= 1e-4 * max(1.0, float(plain.state.logits.std())), pos
+    assert dev.decode_greedy(5, 1018, 12) == plain.decode_greedy(5, 1018, 12)
+    assert dev.last_error() == ""
+    dev.close(); plain.close()

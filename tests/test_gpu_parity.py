@@ -759,22 +759,25 @@ def test_prefill_attention_more_workgroups_than_the_chip_holds(hip, orc, tmp_pat
     dev.close()
 
 
-@pytest.mark.parametrize("dim,heads,kv,hd,interm,n", [(160, 5, 5, 32, 224, 200), (192, 3, 1, 64, 352, 131), (256, 4, 1, 64, 96, 300)])
-def test_q4_prompt_gemm_through_lds_matches_the_per_wavefront_kernel(hip, orc, tmp_path, monkeypatch, dim, heads, kv, hd, interm, n):
-    # Q4_0 prompts of >= 128 tokens take qgemm2_kernel (weights expanded once per workgroup into LDS, nl_qgemm2.h) with
-    # its own plain / SwiGLU / RoPE epilogues.  Shapes whose K is not a multiple of the 128-column chunk, whose row count
-    # is not a multiple of the 64-row workgroup and whose token count leaves a ragged last tile: bit-identical logits,
-    # KV rows and ids to qgemm_kernel (same arithmetic per output, NL_QG2_MIN_TOKENS disables the new kernel), and
-    # within tolerance of the oracle.
-    shape = replace(synth.TIERS["tiny"], name=f"q4_{dim}_{interm}", dim=dim, n_head=heads, n_kv_head=kv, seq_len=320,
+@pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "f16"])
+@pytest.mark.parametrize("dim,heads,kv,hd,interm,n", [(544, 17, 17, 32, 1056, 200), (576, 9, 3, 64, 544, 129), (576, 18, 9, 32, 608, 300), (704, 11, 11, 64, 608, 1100)])
+def test_prompt_gemm_through_lds_matches_the_per_wavefront_kernel(hip, orc, tmp_path, monkeypatch, wtype, dim, heads, kv, hd, interm, n):
+    # Prompts of >= 128 (Q4_0) or 65 tokens over K >= 512 take pgemm_kernel (weights expanded once per workgroup into LDS, nl_pgemm.h) with
+    # its own plain / SwiGLU / RoPE epilogues.  Shapes whose K is not a multiple of the 128-column chunk, whose row count is not a multiple of
+    # the 64-row workgroup (the feed-forward's, the Q|K|V rows of heads of 32) and whose token count leaves a ragged last tile: logits and ids
+    # against qgemm_kernel (NL_QG2_MIN_TOKENS disables the other; sums in another order, so not the same bits) and against the oracle.
+    shape = replace(synth.TIERS["tiny"], name=f"pg_{dim}_{interm}", dim=dim, n_head=heads, n_kv_head=kv, seq_len=1200,
                     interm=interm, n_layer=2)
     p = tmp_path / "g.gguf"
-    synth.generate_gguf(str(p), shape, "q4_0", 17)
+    synth.generate_gguf(str(p), shape, wtype, 17)
     g = gguf.load_gguf(str(p))
     toks = synth.prompt_ids(n, shape.vocab, seed=4)
     ref = orc.OracleModel(g)
+    orc.set_threads(min(16, os.cpu_count() or 1))
     for pos, t in enumerate(toks):
         want = ref.forward(t, pos)
+    want = want.copy()
+    orc.set_threads(1)
     outs = []
     monkeypatch.setenv("NL_FOLD_NORM", "0")     # (the folded RMSNorm scales the consumer's output instead of its input: own test below)
     for knob in (None, "1000000"):
@@ -788,10 +791,10 @@ def test_q4_prompt_gemm_through_lds_matches_the_per_wavefront_kernel(hip, orc, t
         ids = dev.decode_greedy(int(np.argmax(logits)), n, 4)
         outs.append((logits, ids))
         dev.close()
-    assert np.array_equal(outs[0][0], outs[1][0])
+    assert not np.array_equal(outs[0][0], outs[1][0])        # (both kernels ran)
     assert outs[0][1] == outs[1][1]
-    err = float(np.abs(outs[0][0] - want).max())
-    assert err <= LOGIT_TOL * max(1.0, float(want.std()))
+    for logits, _ in outs:
+        assert np.abs(logits - want).max() <= LOGIT_TOL * max(1.0, float(want.std()))
 
 
 @pytest.mark.parametrize("wt_variant", ["q4_0", "q4_0_bias_conj"])
