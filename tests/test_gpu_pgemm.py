@@ -36,15 +36,16 @@ def _decoded(raw, t, rows, cols):
 # <= 256, <= 512, < 1024, above, >= 1792
 @pytest.mark.parametrize("rows,cols,n", [(16, 512, 65), (80, 544, 127), (272, 576, 129), (1040, 640, 1000), (2064, 512, 1000), (2320, 544, 1801), (4112, 544, 1801)])
 @pytest.mark.parametrize("kind", ["q4_0", "q8_0", "f16"])
-def test_product_against_float64(hip, kind, rows, cols, n):
+def test_product_against_float64(hip, monkeypatch, kind, rows, cols, n):
+    monkeypatch.setenv("NL_QG2_MIN_TOKENS", "16")            # (small matrices otherwise from the third token tile on)
     t = synth.WTYPES[kind]
     rng = np.random.default_rng(rows + n)
     w, x = rng.standard_normal((rows, cols)).astype(np.float32), rng.standard_normal((n, cols)).astype(np.float32)
     raw = quant.encode(w, t)
     wd, xd = _decoded(raw, t, rows, cols), x.astype(np.float64)
     got = hip.op_matmul_batch(raw, t, x, rows, cols)
-    # x = hi + lo leaves 2^-22 of an element; 32 products and a scaling per block, cols / 32 block sums, each rounded to 2^-24
-    bound = (2.0 ** -22 + (cols / 32 + 34) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T)
+    # x = hi + lo leaves 2^-22 of an element, of small ones 2^-25; 32 products and a scaling per block, cols / 32 block sums, each rounded to 2^-24
+    bound = (2.0 ** -22 + (cols / 32 + 34) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T) + 2.0 ** -25 * np.abs(wd).sum(1)
     assert (np.abs(got - xd @ wd.T) <= bound).all()
 
 
@@ -137,3 +138,22 @@ def test_a_changed_threshold_reaches_recorded_steps(hip, tmp_path, monkeypatch):
     fresh = step(dev)
     dev.close()
     assert np.array_equal(changed, fresh) and not np.array_equal(changed, split)
+
+
+# second token tile: matrices of 1536 rows and columns on, smaller ones keep the split-K launches (the same bits as with the other kernel disabled)
+@pytest.mark.parametrize("dim,heads,interm,n,moves", [(576, 9, 1536, 128, False), (576, 9, 1536, 129, True), (1536, 24, 1536, 64, False), (1536, 24, 1536, 65, True)])
+@pytest.mark.parametrize("kind", ["q8_0", "f16"])
+def test_which_kernel_short_prompts_take(hip, tmp_path, monkeypatch, kind, dim, heads, interm, n, moves):
+    shape = replace(synth.TIERS["tiny"], name="route", dim=dim, n_head=heads, n_kv_head=heads // 3, interm=interm, seq_len=192, n_layer=1)
+    p = tmp_path / "r.gguf"
+    synth.generate_gguf(str(p), shape, kind, 41)
+    dev = hip.load_llama_model(gguf.load_gguf(str(p)))
+    toks, rows = synth.prompt_ids(n, shape.vocab, seed=9), []
+    for knob in (None, "1000000"):
+        if knob:
+            monkeypatch.setenv("NL_QG2_MIN_TOKENS", knob)
+        dev.reset()
+        dev.prefill(toks)
+        rows.append(dev.state.logits.copy())
+    assert np.array_equal(*rows) != moves
+    dev.close()
