@@ -2975,13 +2975,19 @@ int nl_finalize(nl_handle e) {
             const int grid4 = std::max(lgrid, (e->layers[0].wo.ntiles + e->tpg.wo_tpw - 1) / e->tpg.wo_tpw);
             const char *hk = getenv("NL_ATTN_HELPERS");
             const bool helpers_ok = e->fused_mode == 4 && !(hk && atoi(hk) == 0) && !c.qk_norm && e->layers[0].qkv.wtype == WT_Q4_0;      // (Q8_0: 20 registers too many)
+            // (three of the kv group, four layers, us a token at positions 300 / 600 / 980, the general plan beside it: 1280 columns 99 / 101 / 102 against
+            //  104 / 106 / 105, 1536 101 / 102 / 103 against 107, 2048 115 / 116 / 117 against 120; at 1024 columns a token is too short for them, 91 / 93 / 95
+            //  against 91 / 93 / 94)
             e->attn_helpers = !helpers_ok ? 0 : members - e->gqa >= 2 * e->gqa && grid4 - lgrid >= e->Hs ? 1 : c.dim >= 1280 && members - e->gqa >= 3 * e->gqa ? 2 : 0;
+            // feed-forward in one launch: two passes each stay ahead to the end of the context, whichever blocks help (4096 columns 187 against 207 at
+            // position 1100, 188 against 208 at 1500; 3072 columns in 24 kv groups, all helpers from the group, 155 against 164 and 158 against 174)
             if (!fm && e->attn_helpers && e->wide_ffn) e->fused_max_pos = 2 * TP_NCH_MAX * TP_PASS;
-            // helpers of the kv group, feed-forward in two launches (841M Q4_0): one pass each up to position 1024, 719 against 758 us a token
-            // on the general plan (alone: 772 at 500, 822 at 700); two passes each fall behind, 830 against 793
+            // feed-forward in two launches, helpers of the kv group: one pass each up to position 1024; two passes each fall behind (at 1100 1280 columns
+            // 113 against 110, 1536 114 against 112, 2048 129 against 126)
             else if (!fm && e->attn_helpers == 2) e->fused_max_pos = TP_NCH_MAX * TP_PASS;
-            // Q8_0 (no helpers): one runner's passes against the general plan's split attention, 841M tier (feed-forward in two launches):
-            // 754 against 784 us a token at position 200, 822 against 787 at 300; 4096 columns: 264 against 270 at 700, 275 against 271 at 800
+            // Q8_0 (no helpers): one runner's passes against the general plan's split attention, at positions 200 and 300.  Feed-forward in two launches: 1024
+            // columns 93 / 103 against 96 / 96, 1536 104 / 114 against 108 / 109, 2048 121 / 131 against 122 / 123, 2560 148 / 158 against 157 / 158: the first
+            // pass.  In one launch: at 450 / 600 / 700 / 800, 3072 columns 180 / 191 / 193 / 204 against 184, 4096 230 / 242 / 244 / 255 against 248: three passes
             if (!fm && e->fused_mode == 4 && e->layers[0].qkv.wtype == WT_Q8_0) e->fused_max_pos = e->wide_ffn ? 3 * TP_PASS : TP_PASS;
         }
         if (e->fused_mode == 3 || e->fused_mode == 4)      // passes a head takes inside the launch

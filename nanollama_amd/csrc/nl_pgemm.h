@@ -14,7 +14,8 @@
 // register (a chunk's four scales one ds_read_b128 per row tile) instead of four.  The accumulators go through LDS once at the end and
 // the epilogues read whole rows of a token: coalesced stores, and fragments in either k-slot order.
 //
-// Arithmetic: weights as exact integers in fp16, x = hi + lo in fp16 (2^-22), float32 accumulation, then
+// Arithmetic: weights as exact integers in fp16, x = hi + lo in fp16 (2^-22 of it; 2^-25 where it is below 2^-3, and finite below 65520),
+// float32 accumulation, then
 //   Q4_0 / Q8_0 (/ Q5_0)  acc += d_block * z                      per 32-column block (go/quant.go:74-94, :149-165)
 //   F16                   its own operand, accumulated in the MFMA
 // Files with K-quant matrices (PG_EXACT, every matrix of such a file): what the single-token plan computes in float32 stays that -- x as
@@ -25,7 +26,8 @@
 //
 // Measured (us a launch, weights and fragments in L2; beside it the kernels that these launches ran on before, inside a model): Q4_0, 2047
 // tokens, 768 columns: Q|K|V 15.5 (21.8), gate and up 31.8 (40.5), WO / down (2048 columns) 10.5 / 17.7 (mean 23.5); F16, 993 tokens, 1536
-// columns: 26.7 (35.6), 52.3 (85.0), 17.9 / 36.3 (mean 43.2).  A 64 x 64 tile's block costs a wavefront about 310 cycles: 128 on the matrix
+// columns: 26.7 (35.6), 52.3 (85.0), 17.9 / 36.3 (mean 43.2); inside a model, profiled, 17.3, 36.3, mean 19.0 and 29.9, 57.0, mean 30.8; Q4_K, 333
+// tokens, 768 columns, PG_EXACT: 12.8, 22.8, mean 19.0.  A 64 x 64 tile's block costs a wavefront about 310 cycles: 128 on the matrix
 // pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses), which a SIMD does not overlap with MFMAs
 // (matrix and vector cycles add up); larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
 // be 333 single-token steps: 151 ms, now 1.92 ms (1.49 with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
