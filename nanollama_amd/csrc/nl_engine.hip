@@ -1641,17 +1641,19 @@ hipError_t launch_xsplit(int wtype, const float *x, int ldx, int cols, int n_tok
     return hipGetLastError();
 }
 
-// Which multi-token steps run on pgemm_kernel (nl_pgemm.h).  Files with K-quant matrices: all of them (QGemmParams::exact).  The others: matrices of
-// at least four 128-column chunks (narrower ones never fill its pipeline), Q4_0 from 128 tokens (shorter steps have nl_dgemm.h where that is
-// eligible), Q8_0 and F16 from the third 64-token tile on, from the second where rows and columns give it enough tiles.  us a prompt of 65 / 100 /
-// 127 / 150 tokens, this kernel against the split-K launches of qgemm_kernel: 841M (1536 columns) Q8_0 2344 / 2377 / 2397 / 2534 against 2416 /
-// 2477 / 2528 / 2840, F16 2537 / 2559 / 2581 / 2714 against 2756 / 2810 / 2867 / 3235; 173M (768) Q8_0 1162 / 1175 / 1190 / 1219 against 1141 / 1196 /
-// 1239 / 1277, F16 1304 / 1327 / 1336 / 1334 against 1231 / 1272 / 1311 / 1347; 1024 columns Q8_0 545 / 555 / 562 / 599 against 531 / 553 / 571 / 596; 4096
-// columns at 65 Q8_0 908 against 1284
+// Which multi-token steps run on pgemm_kernel (nl_pgemm.h).  Files with K-quant matrices: all of them (QGemmParams::exact).  The others: Q4_0
+// from 128 tokens (shorter steps have nl_dgemm.h where that is eligible), Q8_0 and F16 from the third 64-token tile on, from the second
+// where rows and columns give it enough tiles.  us a prompt of 65 / 100 / 127 / 150 tokens, this kernel against the split-K launches of
+// qgemm_kernel: 841M (1536 columns) Q8_0 2344 / 2377 / 2397 / 2534 against 2416 / 2477 / 2528 / 2840, F16 2537 / 2559 / 2581 / 2714 against
+// 2756 / 2810 / 2867 / 3235; 173M (768) Q8_0 1162 / 1175 / 1190 / 1219 against 1141 / 1196 / 1239 / 1277, F16 1304 / 1327 / 1336 / 1334 against 1231 /
+// 1272 / 1311 / 1347; 1024 columns Q8_0 545 / 555 / 562 / 599 against 531 / 553 / 571 / 596; 4096 columns at 65 Q8_0 908 against 1284.
+// However narrow the matrices: prompts of 129 / 300 / 1000 / 2000 tokens, 128 columns Q4_0 296 / 357 / 440 / 562 against 327 / 386 / 500 / 604, Q8_0 320 /
+// 362 / 446 / 562 against 332 / 378 / 480 / 586; 384 columns Q4_0 348 / 390 / 513 / 657 against 402 / 454 / 575 / 762, F16 360 / 406 / 522 / 698 against 406 /
+// 464 / 570 / 740
 bool pgemm_ok(int wtype, int rows, int cols, int n_tokens) {
     const char *knob = getenv("NL_QG2_MIN_TOKENS");   // knob (tests, tools; read per launch so a test can flip it): a huge value disables
     const int min_n = knob ? atoi(knob) : wtype == WT_Q4_0 ? 128 : std::min(rows, cols) >= 1536 ? 65 : 129;
-    return (wtype == WT_Q4_0 || wtype == WT_Q8_0 || wtype == WT_F16) && n_tokens >= min_n && cols >= 512;
+    return (wtype == WT_Q4_0 || wtype == WT_Q8_0 || wtype == WT_F16) && n_tokens >= min_n;
 }
 bool pgemm_ok(const PackedMat &m, int n_tokens) { return pgemm_ok(m.wtype, m.rows, m.cols, n_tokens); }
 bool pgemm_ok(int wtype, const QGemmParams &P) { return P.exact || pgemm_ok(wtype, P.rows, P.cols, P.n_tokens); }

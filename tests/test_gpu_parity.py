@@ -760,9 +760,10 @@ def test_prefill_attention_more_workgroups_than_the_chip_holds(hip, orc, tmp_pat
 
 
 @pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "f16"])
-@pytest.mark.parametrize("dim,heads,kv,hd,interm,n", [(544, 17, 17, 32, 1056, 200), (576, 9, 3, 64, 544, 129), (576, 18, 9, 32, 608, 300), (704, 11, 11, 64, 608, 1100)])
+@pytest.mark.parametrize("dim,heads,kv,hd,interm,n", [(544, 17, 17, 32, 1056, 200), (576, 9, 3, 64, 544, 129), (576, 18, 9, 32, 608, 300), (704, 11, 11, 64, 608, 1100),
+                                                     (160, 5, 5, 32, 224, 200), (192, 3, 1, 64, 352, 131), (256, 4, 1, 64, 96, 300), (64, 2, 1, 32, 32, 129)])
 def test_prompt_gemm_through_lds_matches_the_per_wavefront_kernel(hip, orc, tmp_path, monkeypatch, wtype, dim, heads, kv, hd, interm, n):
-    # Prompts of >= 128 (Q4_0) or 65 tokens over K >= 512 take pgemm_kernel (weights expanded once per workgroup into LDS, nl_pgemm.h) with
+    # Prompts of >= 128 (Q4_0) or 129 tokens take pgemm_kernel at every width (weights expanded once per workgroup into LDS, nl_pgemm.h) with
     # its own plain / SwiGLU / RoPE epilogues.  Shapes whose K is not a multiple of the 128-column chunk, whose row count is not a multiple of
     # the 64-row workgroup (the feed-forward's, the Q|K|V rows of heads of 32) and whose token count leaves a ragged last tile: logits and ids
     # against qgemm_kernel (NL_QG2_MIN_TOKENS disables the other; sums in another order, so not the same bits) and against the oracle.
@@ -791,7 +792,8 @@ def test_prompt_gemm_through_lds_matches_the_per_wavefront_kernel(hip, orc, tmp_
         ids = dev.decode_greedy(int(np.argmax(logits)), n, 4)
         outs.append((logits, ids))
         dev.close()
-    assert not np.array_equal(outs[0][0], outs[1][0])        # (both kernels ran)
+    # both kernels ran; up to three 128-column chunks both deal to two sums, with the same bits
+    assert max(dim, interm) <= 384 or not np.array_equal(outs[0][0], outs[1][0])
     assert outs[0][1] == outs[1][1]
     for logits, _ in outs:
         assert np.abs(logits - want).max() <= LOGIT_TOL * max(1.0, float(want.std()))

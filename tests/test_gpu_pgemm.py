@@ -32,9 +32,9 @@ def _decoded(raw, t, rows, cols):
     return (n * d).reshape(rows, cols)
 
 
-# tokens and rows that leave ragged tiles, K of whole and of partial 128-column chunks, and 64 x 64 tile counts on every side of the rules:
+# tokens and rows that leave ragged tiles, K of whole and of partial 128-column chunks, from a single block on, and 64 x 64 tile counts on every side of the rules:
 # <= 256, <= 512, < 1024, above, >= 1792
-@pytest.mark.parametrize("rows,cols,n", [(16, 512, 65), (80, 544, 127), (272, 576, 129), (1040, 640, 1000), (2064, 512, 1000), (2320, 544, 1801), (4112, 544, 1801)])
+@pytest.mark.parametrize("rows,cols,n", [(48, 32, 129), (80, 96, 65), (272, 160, 300), (4112, 224, 1801), (16, 512, 65), (80, 544, 127), (272, 576, 129), (1040, 640, 1000), (2064, 512, 1000), (2320, 544, 1801), (4112, 544, 1801)])
 @pytest.mark.parametrize("kind", ["q4_0", "q8_0", "f16"])
 def test_product_against_float64(hip, monkeypatch, kind, rows, cols, n):
     monkeypatch.setenv("NL_QG2_MIN_TOKENS", "16")            # (small matrices otherwise from the third token tile on)
@@ -141,7 +141,7 @@ def test_a_changed_threshold_reaches_recorded_steps(hip, tmp_path, monkeypatch):
 
 
 # second token tile: matrices of 1536 rows and columns on, smaller ones keep the split-K launches (the same bits as with the other kernel disabled)
-@pytest.mark.parametrize("dim,heads,interm,n,moves", [(576, 9, 1536, 128, False), (576, 9, 1536, 129, True), (1536, 24, 1536, 64, False), (1536, 24, 1536, 65, True)])
+@pytest.mark.parametrize("dim,heads,interm,n,moves", [(384, 6, 480, 128, False), (384, 6, 480, 129, True), (576, 9, 1536, 128, False), (576, 9, 1536, 129, True), (1536, 24, 1536, 64, False), (1536, 24, 1536, 65, True)])
 @pytest.mark.parametrize("kind", ["q8_0", "f16"])
 def test_which_kernel_short_prompts_take(hip, tmp_path, monkeypatch, kind, dim, heads, interm, n, moves):
     shape = replace(synth.TIERS["tiny"], name="route", dim=dim, n_head=heads, n_kv_head=heads // 3, interm=interm, seq_len=192, n_layer=1)
