@@ -776,12 +776,24 @@ __device__ __forceinline__ void load_act(Frag<float> &f, const __amdgpu_buffer_r
 // decode batches: one row tile (ST_GATED: a gate and an up tile) x NT token tiles per workgroup, k tiles dealt to its WV wavefronts
 // in turn; a round's loads are all in flight together
 // NORM: 0 none, 1 norm of nx, 2 norm of nx + norm(nd) ndw; NS: bound of its (token, 2048 columns) slots, four columns per thread and slot
-// (kept small: a launch this short is held up by fetching its own instructions)
-template <typename T, int EPI, int NT, int WV, int NORM, int NS, class TAIL>
+// (kept small: a launch this short is held up by fetching its own instructions); FOLD: writes (ST_RESID) or reads a folded norm's sums, an
+// instance of its own for the same reason (Ganidra, 20 layers of 768 columns, 16 and 64 streams: 600 and 769 us with
+// both in one, 582 and 754)
+template <typename T, int EPI, int NT, int WV, int NORM, int NS, class TAIL, bool FOLD>
 __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
     constexpr int RB = EPI == ST_GATED ? 2 : 1;
     constexpr int PRE = (NT == 1 ? 8 : NT == 2 ? 6 : WV == 16 ? 4 : 6) / (sizeof(T) == 4 ? 2 : 1);
     extern __shared__ __align__(16) char lds[];
+    // one batch of s_load: what is first read behind a branch costs a trip of its own, in a launch of 3 - 6 us (8 layers of 768 columns, one
+    // stream: 223 us a step without it, 208)
+    NL_KARGS8(P.W, P.X, P.nks, P.nrt, P.n_tokens, P.x_nks, P.group, P.rows);
+    if constexpr (NORM) NL_KARGS4(P.nx, P.nw, P.ndim, P.nld);
+    if constexpr (NORM == 2) NL_KARGS4(P.nd, P.ndw, P.nxo, P.neps);
+    if constexpr (EPI == ST_F32) NL_KARGS4(P.out, P.ldo, P.bias, P.amax_val);
+    if constexpr (EPI == ST_RESID) NL_KARGS4(P.out, P.ldo, P.add2, P.n_tokens);
+    if constexpr (EPI == ST_RESID && FOLD) { NL_KARGS4(P.fw, P.fx, P.fss, P.fx_nks); NL_KARGS2(P.fss_ld, P.n_tokens); }
+    if constexpr (EPI == ST_GATED) NL_KARGS4(P.act, P.act_nks, P.bias, P.bias2);
+    if constexpr (FOLD && EPI != ST_RESID) NL_KARGS4(P.nss, P.nss_n, P.fss_ld, P.ndim);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, col = lane & 15;
     const int rt = blockIdx.x * RB, tt0 = blockIdx.y * NT, nks = P.nks, n = P.n_tokens;
     if constexpr (TAIL::on)
@@ -837,11 +849,10 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
     };
     // a folded norm's consumer: the partial sums of its tokens, requested ahead of the weights and added behind them
     [[maybe_unused]] float inv = 1.f;
-    constexpr bool SCALED = !NORM && (EPI == ST_F32 || EPI == ST_GATED);
+    constexpr bool SCALED = FOLD && EPI != ST_RESID;
     [[maybe_unused]] PartialSums<SCALED ? 12 : 1> parts;
     [[maybe_unused]] const int ptok = min(tt0 * 16 + tid % (NT * 16), n - 1), pfrom = tid / (NT * 16), pstep = WV * 64 / (NT * 16);
-    if constexpr (SCALED)
-        if (P.nss) parts.first(P, ptok, pfrom, pstep);
+    if constexpr (SCALED) parts.first(P, ptok, pfrom, pstep);
     load(w);
     T *xs = reinterpret_cast<T *>(lds);                    // NORM: [nks][4][n][8]
     if constexpr (NORM) {
@@ -910,20 +921,19 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
                 for (int r = 0; r < RB; r++) acc[r][t] = mma(a[r][u], b[u][t], acc[r][t]);
         }
     }
-    if constexpr (SCALED)
-        if (P.nss) {                                       // (every thread ends up with its epilogue token's 1 / rms)
-            float nsum = parts.sum(P, ptok, pfrom, pstep);
-            float *const s = reinterpret_cast<float *>(lds);       // [WV][NT * 16]
+    if constexpr (SCALED) {                                // (every thread ends up with its epilogue token's 1 / rms)
+        float nsum = parts.sum(P, ptok, pfrom, pstep);
+        float *const s = reinterpret_cast<float *>(lds);       // [WV][NT * 16]
 #pragma unroll
-            for (int o = NT * 16; o < 64; o <<= 1) nsum += __shfl_xor(nsum, o);
-            if (lane < NT * 16) s[w * NT * 16 + lane] = nsum;
-            lds_barrier();
-            nsum = 0.f;
+        for (int o = NT * 16; o < 64; o <<= 1) nsum += __shfl_xor(nsum, o);
+        if (lane < NT * 16) s[w * NT * 16 + lane] = nsum;
+        lds_barrier();
+        nsum = 0.f;
 #pragma unroll
-            for (int q = 0; q < WV; q++) nsum += s[q * NT * 16 + min(tid >> 6, NT - 1) * 16 + col];
-            inv = rsqrt_f32(nsum / (float)P.ndim + P.neps);
-            lds_barrier();
-        }
+        for (int q = 0; q < WV; q++) nsum += s[q * NT * 16 + min(tid >> 6, NT - 1) * 16 + col];
+        inv = rsqrt_f32(nsum / (float)P.ndim + P.neps);
+        lds_barrier();
+    }
     // the wavefronts' partial tiles meet in LDS
     if constexpr (NORM) lds_barrier();                   // (the area held the norm)
     f32x4 *red = reinterpret_cast<f32x4 *>(lds);           // [WV][RB * NT][64]
@@ -944,11 +954,10 @@ __global__ void __launch_bounds__(WV * 64) few_kernel(MatParams P, TAIL tail) {
 #pragma unroll
             for (int r = 0; r < RB; r++) v[r] *= inv;
         }
-        if constexpr (EPI == ST_RESID)
-            if (P.fw) {
-                add_rows_folded<T>(P, tok, rt, l >> 4, v[0]);
-                continue;
-            }
+        if constexpr (EPI == ST_RESID && FOLD) {
+            add_rows_folded<T>(P, tok, rt, l >> 4, v[0]);
+            continue;
+        }
         if (EPI == ST_F32 && NT == 1 && P.amax_val) {      // one token: rows of column 0, four lanes with four rows each
             float best = -INFINITY;
             int idx = 0x7fffffff;
@@ -977,8 +986,13 @@ hipError_t launch_few_nt(const MatParams &P, hipStream_t st, TAIL tail) {
     const int tt = (P.n_tokens + 15) / 16;
     size_t lds = (size_t)WV * RB * NT * 64 * 16;           // at most 64 KB
     if (NORM) lds = std::max(lds, (size_t)P.nks * 32 * P.n_tokens * sizeof(T) + (size_t)P.n_tokens * WV * 4 * NORM);
-    hipLaunchKernelGGL((few_kernel<T, EPI, NT, WV, NORM, NS, TAIL>), dim3(P.nrt / RB + (TAIL::on ? (tail.units + WV - 1) / WV : P.ahead.wgs(WV)), (tt + NT - 1) / NT), dim3(WV * 64), lds, st, P, tail);
-    return hipGetLastError();
+    auto go = [&](auto kfn) {
+        hipLaunchKernelGGL(kfn, dim3(P.nrt / RB + (TAIL::on ? (tail.units + WV - 1) / WV : P.ahead.wgs(WV)), (tt + NT - 1) / NT), dim3(WV * 64), lds, st, P, tail);
+        return hipGetLastError();
+    };
+    if constexpr (!NORM && !TAIL::on && (EPI == ST_F32 || EPI == ST_GATED || EPI == ST_RESID))
+        if (P.nss || P.fw) return go(few_kernel<T, EPI, NT, WV, NORM, NS, TAIL, true>);
+    return go(few_kernel<T, EPI, NT, WV, NORM, NS, TAIL, false>);
 }
 // is the norm of the product's input (rows of dim values, ld apart) computed inside the launch?
 inline int few_norm_slots(int n, int nks) { return n * ((nks * 32 + 2047) / 2048); }

@@ -442,6 +442,10 @@ __device__ __forceinline__ void win_decode_block(const WinParams &P, int h, int 
 template <typename T, int M>
 __global__ void __launch_bounds__(256) mix_decode_kernel(WinParams A, GlaParams L, int n_tokens) {
     extern __shared__ __align__(16) char lds[];
+    NL_KARGS4(n_tokens, A.pos, A.stream, A.nsplit);      // (one batch of s_load: a trip less in front of the positions)
+    NL_KARGS8(L.proj, L.state, L.a2, L.a2b, L.norm, L.y, L.ldp, L.rank);
+    NL_KARGS8(L.off_q, L.off_k, L.off_v, L.off_g, L.off_a1, L.dk, L.dv, L.heads);
+    if constexpr (M > 0) NL_KARGS8(A.proj, A.K, A.V, A.ldp, A.heads, A.kv_heads, A.dk, A.dv);
     if ((int)blockIdx.y >= n_tokens) {
         A.ahead.read(blockIdx.y * gridDim.x + blockIdx.x, n_tokens * gridDim.x, 4, threadIdx.x >> 6, threadIdx.x & 63);
         return;
