@@ -93,6 +93,7 @@ struct nl_engine {
     const float *pend = nullptr; // the norm's factor, null: nothing pending
     // no norms behind the sublayers: the last residual product left the next norm's input in h and its sums of squares here (MatParams::fw)
     bool folded = false;
+    bool read_ahead = false;     // decode launches bring the next ones' weights into L2 (AHEAD_WEIGHTS)
     float *fss = nullptr;        // [row tile of the width][tokens]
     // latent attention: operand of the absorbed product, split results, expanded keys and values of kv_slots positions
     void *xq = nullptr, *ek = nullptr, *ev = nullptr;
@@ -352,12 +353,19 @@ MatParams product_params(nl_engine *e, const Mat &m, const void *X, int n) {
 // weights that the launches behind a decode launch read, rb row tiles to a workgroup, nearest launch first: as many lists as half of the L2s
 // (8 x 4 MB) holds.  us / step, none, 8, 16 and 24 MB: Pabalix, 1 stream, 768 columns 805, 767, 766, 767, 1536 columns 1273, 1265, 1216, 1252;
 // Ganidra, 32 streams, 1536 columns 1301, 1274, 1255, 1258.
+// Only where the weights that a step reads are more than the 256 MB memory-side cache keeps from one step to the next, and for latent layers up to
+// 32 tokens.  Gain in percent of a step at 1 / 16 / 48 streams, by MB of weights: Ganidra 127 -3.5 / -2.4 / -3.6, 154 -2.8 / -1.9 / -1.6, 181
+// -3.1 / 0 / +1.9, 226 -2.7 / 0 / -2.0, 235 +2.9 / +8.6 / +3.0, 261 +4.9 / +9.3 / +1.9, 315 +5.2 / +8.0 / +1.5, 570 +3.3 / +2.4 / +0.4; Pabalix 123 -0.4 / 0 /
+// -2.0, 211 -0.7 / +0.7 / -1.3, 237 0 / -1.1 / -2.7, 249 +2.9 / +5.1 / +1.7, 299 +4.9 / +6.8 / +1.0, 410 +1.2 / +1.9 / -1.5; its prompts of 40 tokens -3 on average.
+constexpr size_t AHEAD_WEIGHTS = (size_t)240 << 20;
+// (two token tiles in 32 bits below 1024 columns: -2.5 / -3.4 / -0.6 at 17 / 20 / 24 tokens, +10 at 16; 1024 columns +2.9 at 17)
+inline int ahead_tokens(bool latent, bool f32, int dim) { return !latent ? FEW_MAX_TOKENS : f32 && dim < 1024 ? 16 : 32; }
 struct Next { const Mat *m; int rb; };
 constexpr long long AHEAD_MAX = 16 << 20;
 template <typename T>
-Ahead look_ahead(int n, std::initializer_list<Next> next) {
+Ahead look_ahead(const nl_engine *e, int n, std::initializer_list<Next> next) {
     Ahead A{};
-    if (n > FEW_MAX_TOKENS) return A;
+    if (!e->read_ahead || n > ahead_tokens(e->latent, e->f32(), e->c.dim)) return A;
     int i = 0;
     long long total = 0;
     for (const Next &x : next) {
@@ -404,7 +412,7 @@ hipError_t residual_product(nl_engine *e, const Mat &m, const void *X, int n, co
                             const Mat *ahead = nullptr) {
     MatParams P = product_params(e, m, X, n);
     P.ldo = e->c.dim;
-    P.ahead = look_ahead<T>(n, {{ahead, 2}});
+    P.ahead = look_ahead<T>(e, n, {{ahead, 2}});
     if (!post) {
         P.out = e->xcur; P.add2 = behind;
         // (up to a few tokens the norm costs nothing: the product behind it computes it in its prologue)
@@ -505,7 +513,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         J.out = e->proj; J.ldo = L.proj.rows;
         // (what reads ahead: latent attention's own launches keep up to 100 KB of LDS per workgroup, so its products do, 766 against 795 us a
         // token; the other mixers' launch has room on every CU, 737 against 755 us a step of 48 streams)
-        if (L.d.latent.heads) J.ahead = look_ahead<T>(s.n, {{&L.uq, 1}, {&L.ukt, 1}, {&L.uv, 1}, {&L.out, 1}});
+        if (L.d.latent.heads) J.ahead = look_ahead<T>(e, s.n, {{&L.uq, 1}, {&L.ukt, 1}, {&L.uv, 1}, {&L.out, 1}});
         if ((rc = normed_product<T, ST_F32>(e, J, L.norm1))) return rc;
         WinParams W{};
         W.pos = s.pos; W.stream = s.stream; W.nsplit = 1; W.y = e->y; W.y_nks = L.out.nks; W.proj = e->proj; W.ldp = L.proj.rows;
@@ -528,7 +536,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         if (L.d.latent.heads) {
             if ((rc = latent_mixer<T>(e, s, R, L))) return rc;
         } else if (s.decode) {
-            W.ahead = look_ahead<T>(s.n, {{&L.out, 1}, {&L.gateup, 2}, {&L.down, 1}});
+            W.ahead = look_ahead<T>(e, s.n, {{&L.out, 1}, {&L.gateup, 2}, {&L.down, 1}});
             if ((rc = launch_mix_decode<T>(W, N, s.n, st))) return rc;
         } else {
             if (A.heads && ((rc = launch_win_prep<T>(W, s.n, st)) || (rc = launch_win_attn<T>(W, s.ntiles, st)))) return rc;
@@ -539,7 +547,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         if (L.d.ff) {
             MatParams F = product_params(e, L.gateup, nullptr, s.n);
             F.act = e->act; F.act_nks = L.down.nks; F.act_silu = L.d.ff_act == NL_ACT_SILU; F.bias = L.gateb; F.bias2 = L.upb;
-            F.ahead = look_ahead<T>(s.n, {{L.d.latent.heads ? &L.down : nullptr, 1},
+            F.ahead = look_ahead<T>(e, s.n, {{L.d.latent.heads ? &L.down : nullptr, 1},
                                           {r + 1 < e->runs.size() ? &e->layers[e->runs[r + 1].layer].proj : nullptr, 1}});
             if ((rc = normed_product<T, ST_GATED>(e, F, L.norm2))) return rc;
             if ((rc = residual_product<T>(e, L.down, e->act, s.n, L.downb, L.norm2p, behind, next))) return rc;
@@ -954,6 +962,13 @@ int nl_finalize(nl_handle e) {
     if (e->stage) { HIPCK(e, hipFree(e->stage)); e->stage = nullptr; e->stage_cap = 0; }
     const int D = e->c.dim, S = e->c.max_streams;
     const size_t es = e->esize();
+    {   // what a decode step reads: everything but an untied lookup table and the expanded keys' matrix, which prompts use
+        auto bytes = [&](const Mat &m) { return m.w ? (size_t)m.nrt * m.nks * OPT * es : 0; };
+        size_t read = e->bytes_weights - (e->c.untied ? bytes(e->embed) : 0);
+        for (const Layer &L : e->layers) read -= bytes(L.uk);
+        const char *knob = getenv("NL_STACK_AHEAD");     // knob (tests): 0 never, else always
+        e->read_ahead = knob ? atoi(knob) != 0 : read > AHEAD_WEIGHTS;
+    }
     e->cap = std::min(up(e->c.max_step_tokens, 64), up(std::max(e->c.seq_len, std::min(S, FEW_MAX_TOKENS)), 64));
     const int cap = e->cap, few = std::min(std::max(S, 1), FEW_MAX_TOKENS);
     e->lm_cap = std::max(FEW_MAX_TOKENS, std::min(cap, 256));

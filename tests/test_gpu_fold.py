@@ -36,7 +36,8 @@ def test_folded_norm_in_decode_batches(width, n, scale, loop, dtype):
 
 # one list, all of them, and a feed-forward past what is read ahead; row tiles and workgroups that are no multiple of the XCDs
 @pytest.mark.parametrize("width,ff,n,dtype", [(64, 24, 1, "float32"), (136, 344, 1, "bfloat16"), (136, 344, 40, "float32"), (2056, 2008, 2, "float32")])
-def test_weights_read_ahead(width, ff, n, dtype):
+def test_weights_read_ahead(monkeypatch, width, ff, n, dtype):
+    monkeypatch.setenv("NL_STACK_AHEAD", "1")            # (models of this size otherwise stay in the caches by themselves)
     cfg = config([par(heads=2, kv=1, ff=ff), gla(ff=0), gla(ff=ff)], width=width)
     w = weights(cfg, 92)
     seqs = [tokens(5, seed=50 + i) for i in range(n)]
