@@ -351,7 +351,7 @@ MatParams product_params(nl_engine *e, const Mat &m, const void *X, int n) {
 }
 
 // weights that the launches behind a decode launch read, rb row tiles to a workgroup, nearest launch first: as many lists as half of the L2s
-// (8 x 4 MB) holds.  us / step, none, 8, 16 and 24 MB: Pabalix, 1 stream, 768 columns 805, 767, 766, 767, 1536 columns 1273, 1265, 1216, 1252;
+// (8 x 4 MB) holds.  us / step, none, 8, 16 and 24 MB (each launch 0.3 - 0.7 us longer than now): Pabalix, 1 stream, 768 columns 805, 767, 766, 767, 1536 columns 1273, 1265, 1216, 1252;
 // Ganidra, 32 streams, 1536 columns 1301, 1274, 1255, 1258.
 // Only where the weights that a step reads are more than the 256 MB memory-side cache keeps from one step to the next, and for latent layers up to
 // 32 tokens.  Gain in percent of a step at 1 / 16 / 48 streams, by MB of weights: Ganidra 127 -3.5 / -2.4 / -3.6, 154 -2.8 / -1.9 / -1.6, 181
@@ -511,8 +511,8 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         const float *const next = r + 1 < e->runs.size() ? e->layers[e->runs[r + 1].layer].norm1 : nullptr;
         MatParams J = product_params(e, L.proj, nullptr, s.n);
         J.out = e->proj; J.ldo = L.proj.rows;
-        // (what reads ahead: latent attention's own launches keep up to 100 KB of LDS per workgroup, so its products do, 766 against 795 us a
-        // token; the other mixers' launch has room on every CU, 737 against 755 us a step of 48 streams)
+        // (what reads ahead: latent attention's own launches keep up to 100 KB of LDS per workgroup, so its products do, 707 against 744 us a
+        // token; the other mixers' launch has room on every CU, 582 against 631 us a step of 16 streams)
         if (L.d.latent.heads) J.ahead = look_ahead<T>(e, s.n, {{&L.uq, 1}, {&L.ukt, 1}, {&L.uv, 1}, {&L.out, 1}});
         if ((rc = normed_product<T, ST_F32>(e, J, L.norm1))) return rc;
         WinParams W{};
