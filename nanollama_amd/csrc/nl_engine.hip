@@ -13,6 +13,7 @@
 #include "nl_qgemm.h"
 #include "nl_pgemm.h"
 #include "nl_dgemm.h"
+#include "nl_sgemm.h"
 #include "nl_batch.h"
 #include "nl_sample.h"
 #include "nl_p2p.h"
@@ -1724,33 +1725,25 @@ void launch_qgemm_nt(int nt, dim3 grid, hipStream_t st, const QGemmParams &P) {
     }
 }
 
-hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_buf = nullptr, size_t part_cap = 0,
-                        int *ks_out = nullptr) {
-    P.nt16 = ((P.n_tokens + 63) / 64) * 4;
-    const int tok_tiles = (P.n_tokens + QG_TOK - 1) / QG_TOK;
-    const int nchunks = (P.cols / 32 + QG_KC - 1) / QG_KC;
-    const int mats = P.q1 ? 2 : 1;
-    if (pgemm_ok(wtype, P) && mats == 1) {
-        if (ks_out) *ks_out = 1;
-        return pg_launch<QG_EPI_PLAIN>(wtype, P, st);
-    }
-    if (P.nrm_out.w) return hipErrorInvalidValue;   // (the folded norm's producer epilogue exists in pgemm_kernel only: host logic error)
+// A split-K launch of qgemm_kernel: wavefronts of a workgroup, their row tiles, and the K splits.  (sgemm_kernel's wavefronts take the same splits)
+struct QgGeom { int waves, rt, row_groups, ks; };
+QgGeom qgemm_geometry(int ntiles, int mats, int cols, int n_tokens, bool may_split, int ldo, size_t part_cap) {
+    const int tok_tiles = (n_tokens + QG_TOK - 1) / QG_TOK, nchunks = (cols / 32 + QG_KC - 1) / QG_KC;
     // Workgroup height: 128 rows (8 wavefronts) when that alone fills the chip, else 64 rows (4 wavefronts) --
     // twice the workgroups and half the split-K for the small-N decode batches (goldie shapes at 16-128 tokens:
     // -4...-18 % per launch, tools/qgemm_variants.sh); then split K until ~128 workgroups exist.
     static const int force_waves = getenv("NL_QG_FORCE_WAVES") ? atoi(getenv("NL_QG_FORCE_WAVES")) : 0;   // developer knob
     int waves = QG_WAVES, rt = QG_RT;
-    if (((P.ntiles + QG_WAVES - 1) / QG_WAVES) * mats * tok_tiles < 128) waves = 4;
+    if (((ntiles + QG_WAVES - 1) / QG_WAVES) * mats * tok_tiles < 128) waves = 4;
     if (force_waves == 4 || force_waves == 8) waves = force_waves;
     // decode batches (one 64-token tile): a workgroup's ingest is dominated by the activation fragments (256 B per
     // column against 72 B of Q4_0 weights for a 128-row workgroup), so tall workgroups -- 8 wavefronts x 2 tiles = 256
     // rows -- with a deep K split move the least data per launch
     static const int dec_geom = getenv("NL_QG_DEC_GEOM") ? atoi(getenv("NL_QG_DEC_GEOM")) : 0;   // developer knob: 82 = 8 waves x 2 tiles
-    if (tok_tiles == 1 && part_buf && P.ldo == P.rows && dec_geom == 82 && QG_RT == 1) { waves = 8; rt = 2; }
-    const int row_groups = (P.ntiles + waves * rt - 1) / (waves * rt);
-    P.row_groups = row_groups;
+    if (tok_tiles == 1 && may_split && dec_geom == 82 && QG_RT == 1) { waves = 8; rt = 2; }
+    const int row_groups = (ntiles + waves * rt - 1) / (waves * rt);
     int ks = 1;
-    if (part_buf && P.ldo == P.rows) {
+    if (may_split) {
         static const int ks_cap = getenv("NL_KS_CAP") ? atoi(getenv("NL_KS_CAP")) : 16;   // developer knob (tools/)
         static const int min_wg = getenv("NL_QG_MIN_WG") ? atoi(getenv("NL_QG_MIN_WG")) : 128;
         static const int max_chunks = getenv("NL_QG_MAX_CHUNKS") ? atoi(getenv("NL_QG_MAX_CHUNKS")) : 6;   // goldie x 64 streams: 2.06 -> 1.94 ms per step (tools/sweep_qg_split.sh)
@@ -1761,8 +1754,24 @@ hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_bu
                (row_groups * mats * tok_tiles * ks < min_wg ||
                 (tok_tiles == 1 && (nchunks + ks - 1) / ks > max_chunks && row_groups * mats * ks * 2 <= max_wg)))
             ks *= 2;
-        while (ks > 1 && (size_t)ks * P.n_tokens * P.ldo > part_cap) ks /= 2;
+        while (ks > 1 && (size_t)ks * n_tokens * ldo > part_cap) ks /= 2;
     }
+    return QgGeom{waves, rt, row_groups, ks};
+}
+
+hipError_t launch_qgemm(int wtype, QGemmParams P, hipStream_t st, float *part_buf = nullptr, size_t part_cap = 0,
+                        int *ks_out = nullptr) {
+    P.nt16 = ((P.n_tokens + 63) / 64) * 4;
+    const int tok_tiles = (P.n_tokens + QG_TOK - 1) / QG_TOK;
+    const int mats = P.q1 ? 2 : 1;
+    if (pgemm_ok(wtype, P) && mats == 1) {
+        if (ks_out) *ks_out = 1;
+        return pg_launch<QG_EPI_PLAIN>(wtype, P, st);
+    }
+    if (P.nrm_out.w) return hipErrorInvalidValue;   // (the folded norm's producer epilogue exists in pgemm_kernel only: host logic error)
+    const QgGeom G = qgemm_geometry(P.ntiles, mats, P.cols, P.n_tokens, part_buf && P.ldo == P.rows, P.ldo, part_cap);
+    const int waves = G.waves, rt = G.rt, row_groups = G.row_groups, ks = G.ks;
+    P.row_groups = row_groups;
     P.ksplit = ks;
     P.part = part_buf;
     dim3 grid(row_groups * mats, tok_tiles, ks);
@@ -1948,6 +1957,24 @@ bool dgemm_step_ok(const nl_engine *e, int n) {
     return (long long)((n + 15) / 16) * (e->cfg.interm / 64) <= 1024;
 }
 
+// ---- short multi-token steps on sgemm_kernel (nl_sgemm.h): the splits that qgemm_kernel's launches of the same step would take ----
+int sgemm_splits(const nl_engine::Batch &b, const PackedMat &m, int mats, int n, bool whole) {
+    return whole ? 1 : qgemm_geometry(m.ntiles, mats, m.cols, n, true, m.rows, b.kpart_cap).ks;
+}
+int sgemm_splits_qkv(const nl_engine::Batch &b, const nl_engine::Layer &L, int n) { return sgemm_splits(b, L.qkv, 1, n, qgemm_rope_fits(L.qkv, n)); }
+int sgemm_splits_gate(const nl_engine::Batch &b, const nl_engine::Layer &L, int n) { return sgemm_splits(b, L.gate, 2, n, qgemm_swiglu_fits(L.gate, n)); }
+bool sgemm_step_ok(const nl_engine *e, const nl_engine::Batch &b, int n) {
+    const char *k = getenv("NL_SGEMM");                 // knob (tests, tools; read per step): 0 keeps qgemm_kernel's launches
+    const nl_config &c = e->cfg;
+    if ((k && atoi(k) == 0) || c.qk_norm || e->Is % 32) return false;      // (QK-norm needs whole heads between the product and the rotation)
+    auto ok = [&](const PackedMat &m, bool norm, int rt, int ks) { return !pgemm_ok(m, n) && m.ntiles * TR == m.rows && sg_fits(norm, rt, m.cols, ks); };
+    for (const auto &L : e->layers)
+        if (L.up.wtype != L.gate.wtype || !ok(L.qkv, true, 1, sgemm_splits_qkv(b, L, n)) || !ok(L.gate, true, 2, sgemm_splits_gate(b, L, n)) ||
+            !ok(L.wo, false, 1, sgemm_splits(b, L.wo, 1, n, false)) || !ok(L.down, false, 1, sgemm_splits(b, L.down, 1, n, false)))
+            return false;
+    return true;
+}
+
 // GEMM of the multi-token step: input = the fragment store the producing kernel just filled; output = `out`
 // (with resid / bias applied) when it ran unsplit, else split-K slabs in `part` for the consumer to add.
 hipError_t qg(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, const float *resid, hipStream_t st,
@@ -2068,6 +2095,17 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                (exact || (fills(L.wo, 4) && fills(L.down, 4) && fills(L.qkv, QG_WAVES) && fills(L.gate, QG_FUSED_WAVES)));
     }
     if (dg) fold = true;
+    const bool sg = !dg && !fold && !exact && sgemm_step_ok(e, b, n);      // ... of the other formats and widths: nl_sgemm.h
+    auto sg_params = [&](const PackedMat &m, int ks) {
+        SGemmParams P{};
+        P.q = m.q; P.s = m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles; P.n_tokens = n; P.ks = ks; P.eps = c.rms_eps;
+        return P;
+    };
+    auto sg_plain = [&](const PackedMat &m, const uint4 *in, const float *bias) {       // x += W . in (+ bias)
+        SGemmParams P = sg_params(m, sgemm_splits(b, m, 1, n, false));
+        P.xf = in; P.out = b.x; P.bias = bias;
+        return sg_launch<QG_EPI_PLAIN>(m.wtype, P, st);
+    };
     const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
     // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs of Q4_0 files (pgemm_kernel) and the
     // prompt attention multiply only the fp16 hi half of every activation / probability -- half / a third of the matrix work,
@@ -2098,8 +2136,14 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         GemmOut qkv_out{nullptr, nullptr, 1, 0, nullptr};
         bool rope_in_attn = false;
         const bool folded_in = fold && l > 0;      // the previous layer's down GEMM wrote this layer's Q|K|V input
-        if (!folded_in) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
-        if (dg || (!c.qk_norm && (exact || qgemm_rope_fits(L.qkv, n)))) {
+        if (!folded_in && !sg) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
+        if (sg) {
+            SGemmParams P = sg_params(L.qkv, sgemm_splits_qkv(b, L, n));
+            P.x = b.x; P.normw = L.attn_norm;
+            P.rope = QGemmParams::Rope{b.pos, b.stream, e->rope_cos, e->rope_sin, b.q, kc, vc, e->kv_stream_stride,
+                                       L.bq, L.bk, L.bv, hd, e->Hs, e->KVs, c.seq_len, c.rope_conjugate, b.tcos, b.tsin, b.tkv};
+            LCK(sg_launch<QG_EPI_ROPE>(L.qkv.wtype, P, st));
+        } else if (dg || (!c.qk_norm && (exact || qgemm_rope_fits(L.qkv, n)))) {
             // Q|K|V, RoPE, biases and the KV store in ONE launch (QK-norm needs whole heads: unfused path)
             QGemmParams P{};
             const PackedMat &m = L.qkv;
@@ -2186,7 +2230,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             pend = GemmOut{b.x, nullptr, 1, (long long)n * D, nullptr};
             return launch_dgemm_plain(P, st);
         };
-        if (fold && dg) {
+        if (sg) {
+            LCK(sg_plain(L.wo, b.xfrag, L.bo));
+        } else if (fold && dg) {
             const QGemmParams::NormOut nout{L.ffn_norm, b.xfrag2, b.ssq, sB};
             LCK(dg_plain(L.wo, b.xfrag, L.bo, &nout));
         } else if (fold) {
@@ -2199,6 +2245,13 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         if (L.up.wtype != L.gate.wtype)   // (a mixed-type file: the fragment k-slot order differs per type)
             return e->fail(NL_ERR_UNSUPPORTED, "gate and up projections of different quantisation types");
         const uint4 *down_in = b.xfrag;
+        if (sg) {
+            SGemmParams P = sg_params(L.gate, sgemm_splits_gate(b, L, n));
+            P.x = b.x; P.normw = L.ffn_norm; P.q1 = L.up.q; P.s1 = L.up.s; P.xf_out = b.xfrag2; P.out_form = form(L.down);
+            LCK(sg_launch<QG_EPI_SWIGLU>(L.gate.wtype, P, st));
+            LCK(sg_plain(L.down, b.xfrag2, nullptr));
+            continue;
+        }
         if (dg || exact || qgemm_swiglu_fits(L.gate, n)) {
             // gate, up and SiLU(gate) * up in ONE launch; h leaves as fragments in the second fragment store
             // (the first is still being read by other workgroups of this launch)
@@ -3609,8 +3662,9 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
         //  part of the key of a cached step graph)
         auto batch_knob_sig = [] {
             const char *rk = getenv("NL_ROPE_IN_ATTN"), *fk = getenv("NL_FOLD_NORM"), *pk = getenv("NL_PREFILL_PRECISION"), *kk = getenv("NL_KV16_MIN_TOKENS"),
-                       *dk = getenv("NL_DGEMM"), *dm = getenv("NL_DGEMM_MAX_TOKENS"), *hk = getenv("NL_DGEMM_HEAD"), *qk = getenv("NL_QG2_MIN_TOKENS");
-            return 40503 * (hk ? atoi(hk) + 1 : 0) + 7919 * (qk ? (atoi(qk) & 0xfff) + 1 : 0) + (rk ? atoi(rk) + 1 : 0) + 3 * (fk ? atoi(fk) + 1 : 0) + 9 * (pk && !strcmp(pk, "fp16x1") ? 1 : 0) +
+                       *dk = getenv("NL_DGEMM"), *dm = getenv("NL_DGEMM_MAX_TOKENS"), *hk = getenv("NL_DGEMM_HEAD"), *qk = getenv("NL_QG2_MIN_TOKENS"),
+                       *sk = getenv("NL_SGEMM");
+            return 24593 * (sk ? atoi(sk) + 1 : 0) + 40503 * (hk ? atoi(hk) + 1 : 0) + 7919 * (qk ? (atoi(qk) & 0xfff) + 1 : 0) + (rk ? atoi(rk) + 1 : 0) + 3 * (fk ? atoi(fk) + 1 : 0) + 9 * (pk && !strcmp(pk, "fp16x1") ? 1 : 0) +
                    18 * (dk ? atoi(dk) + 1 : 0) + 54 * (dm ? (atoi(dm) & 0xff) + 1 : 0) + 13878 * (kk ? (atoi(kk) & 0xfff) + 1 : 0);
         };
         if (groups > 1 && groups <= 4) {

@@ -1,0 +1,86 @@
+"""GPU tests of the short multi-token steps on sgemm_kernel (nanollama_amd/csrc/nl_sgemm.h): Q8_0, F16 and Q4_0 files, any width of whole
+32-value blocks.  The kernel takes qgemm_kernel's K splits in qgemm_kernel's order, so the same handle's split-K launches (NL_SGEMM=0) give the
+same bits: rows, logits and cache.  A sampled reply depends on that.  Reference: go/model.go:510-612 per stream, go/quant.go:45-165, :527-563."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from nanollama_amd import gguf, synth
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    # three blocks and seven: a last chunk, group and pair that are not whole; head_dim 32, grouped heads, biases
+    "d96_i224": synth.ModelShape("sg_a", 2, 96, 3, 1, 160, seq_len=160, interm=224, attn_bias=True),
+    # the smallest tier's widths (two and a quarter groups), conjugate rotation
+    "d576_i1536": synth.ModelShape("sg_b", 2, 576, 9, 3, 256, seq_len=160, interm=1536, rope_conjugate=True),
+    # few rows, long columns: sixteen splits of the down projection; a group of three pairs
+    "d160_i4000": synth.ModelShape("sg_c", 1, 160, 5, 5, 96, seq_len=96, interm=4000),
+    # two row tiles a wavefront from 33 tokens on, six chunks a split
+    "d1536_i4096": synth.ModelShape("sg_d", 1, 1536, 24, 6, 128, seq_len=96, interm=4096),
+}
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from nanollama_amd import _lib, model
+    if _lib.lib().nl_device_count() < 1:
+        pytest.fail("no HIP device visible: the GPU tests must run on the MI355X box")
+    return model
+
+
+@pytest.mark.parametrize("wtype", ["q8_0", "f16", "q4_0", "q5_0"])
+@pytest.mark.parametrize("name", list(SHAPES))
+def test_short_steps_give_the_bits_of_the_split_k_launches(hip, tmp_path, monkeypatch, name, wtype):
+    monkeypatch.setenv("NL_DGEMM", "0")                  # (widths of whole 256-column groups too)
+    shape = SHAPES[name]
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), shape, wtype, 17)
+    m = hip.load_llama_model(gguf.load_gguf(str(p)), max_streams=40)
+    rng = np.random.default_rng(3)
+    toks = [int(t) for t in rng.integers(3, shape.vocab, size=shape.seq_len)]
+    for n in (3, 9, 16, 17, 48, 64, 70):
+        got = {}
+        for knob in ("0", "1"):
+            monkeypatch.setenv("NL_SGEMM", knob)
+            m.reset()
+            m.prefill(toks[:n])
+            rows = [m.state.logits.copy()]
+            m.prefill(toks[n:n + 9], n)                  # over the rows that the first prompt left in the cache
+            got[knob] = rows + [m.state.logits.copy()]
+        for a, b in zip(got["0"], got["1"]):
+            assert np.isfinite(a).all() and np.array_equal(a, b), (n, float(np.abs(a - b).max()))
+    for ns, ctx in ((3, 5), (40, 5), (21, 80)):
+        ctx = min(ctx, shape.seq_len - 4)
+        got = {}
+        for knob in ("0", "1"):
+            monkeypatch.setenv("NL_SGEMM", "0")
+            for s in range(ns):
+                m.reset(s)
+                m.prefill(toks[s % 7:][:ctx - s % 3], 0, s, want_logits=False)
+            monkeypatch.setenv("NL_SGEMM", knob)
+            got[knob] = [m.forward_batch(list(range(ns)), toks[i:i + ns], [ctx - s % 3 + i for s in range(ns)], want_logits=True)[1].copy() for i in range(3)]
+        for a, b in zip(got["0"], got["1"]):
+            assert np.isfinite(a).all() and np.array_equal(a, b), (ns, ctx, float(np.abs(a - b).max()))
+    m.close()
+
+
+@pytest.mark.parametrize("wtype", ["q8_0", "f16"])
+def test_short_steps_match_the_oracle(hip, tmp_path, wtype):
+    from oracle import oracle
+    shape = SHAPES["d576_i1536"]
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), shape, wtype, 18)
+    g = gguf.load_gguf(str(p))
+    toks = [int(t) for t in np.random.default_rng(4).integers(3, shape.vocab, size=29)]
+    ref = oracle.OracleModel(g)
+    for pos, t in enumerate(toks):
+        want = ref.forward(t, pos)
+    m = hip.load_llama_model(g)
+    m.prefill(toks)
+    assert float(np.abs(m.state.logits - want).max()) <= 1e-4 * max(1.0, float(want.std()))
+    m.close()
