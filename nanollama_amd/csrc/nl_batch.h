@@ -790,7 +790,8 @@ template <int HD> struct Kv16Image {
 // f32 cache rows of one chunk -> the image (split_hi_lo, V transposed with the key -> position map of the kernel below).
 // Thread (key pair rp, float4 column c4) owns keys 2rp, 2rp+1 (clamped loads, zero beyond nrows so that masked
 // probabilities meet finite values); all loads are issued before the first LDS store.
-template <int HD, int NTH>
+// FEW: key tiles that lie past nrows rounded up to 64 may stay as they are -- the caller skips them.
+template <int HD, int NTH, bool FEW = false>
 __device__ __forceinline__ void kv16_stage(const float4 *K4, const float4 *V4, int nrows, int tid,
                                            _Float16 *Kh, _Float16 *Kl, _Float16 *VTh, _Float16 *VTl, bool sync_before_store) {
     typedef Kv16Image<HD> Img;
@@ -815,6 +816,7 @@ __device__ __forceinline__ void kv16_stage(const float4 *K4, const float4 *V4, i
     for (int it = 0; it < NIT; it++) {
         const int i = tid + it * NTH, rp = i / R4, c4 = i % R4;
         if (i >= ATT_CH / 2 * R4) continue;
+        if (FEW && it * NTH / R4 * 2 >= ((nrows + 63) & ~63)) break;       // (the same in all lanes)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const bool live = 2 * rp + h < nrows;
@@ -991,7 +993,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
         } else {
             const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
             const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
-            kv16_stage<HD, NTH>(K4, V4, nrows, tid, Kh, Kl, VTh, VTl, c > 0);
+            kv16_stage<HD, NTH, true>(K4, V4, nrows, tid, Kh, Kl, VTh, VTl, c > 0);
         }
         ATT_STAMP(10 * c + 3);
         __syncthreads();                               // the chunk is in LDS; every wavefront is past the previous chunk
@@ -999,6 +1001,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
             if (c + 1 < c_count) dma_chunk(c_first + c + 1, (c + 1) & 1);
         }
         ATT_STAMP(10 * c + 4);
+        if (!SHADOW && i0 + w * 16 / G >= n_items) continue;      // no query in this wavefront: the pipes are the others'
 
         // ---- S^T = K q^T: 8 key tiles x 16 rows; lane (j, kq) ends up with row j's scores for keys 16*mt + 4*kq + r
         v4f acc[8];
@@ -1011,6 +1014,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
             for (int ks = 0; ks < NKS; ks++) {
 #pragma unroll
                 for (int mh = 0; mh < 8; mh += 4) {        // four key tiles at a time: 32 operand registers live, not 64
+                    if (!SHADOW && mh * 16 >= nrows) break;      // (no keys there: a short prompt.  The same in all lanes)
                     half8_t kh[4], kl[4];
 #pragma unroll
                     for (int mt = 0; mt < 4; mt++) {
@@ -1094,6 +1098,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
             constexpr bool X1 = decltype(x1_tag)::value;
 #pragma unroll
             for (int mm = 0; mm < 4; mm++) {
+                if (!SHADOW && mm * 32 >= nrows) break;
                 // p * 2^10 = hi + lo: hi = the leading 11 bits (a mask, exact in fp16 down to its subnormals), lo = the rest
                 // (fp16x1: p rounded to fp16, no lo)
                 half8_t ph, pl;
@@ -1132,6 +1137,34 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
     // bytes per nt); rows that see no key of this run leave no partial (the merge does not count this slot for them)
     constexpr float unscale = 1.0f / 1024.0f;
     const int t_first = c_first * ATT_CH;
+    if (!SHADOW && P.fin_xf) {
+        // every row's only run (a prompt within 128 positions): o / l as the WO GEMM's fragments, battn_merge_kernel's arithmetic for one
+        // partial.  A lane's four elements are half an entry; 24 tokens, nine heads: 7.9 + 4.0 us in two launches, now 6.3 in one
+        if (npos[w * 16 + j] > 0) {
+            typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+            const int vh = w * 16 + j, item = i0 + vh / G, h = kvh * G + vh % G;
+            const float scale = 1.0f / (l * unscale);
+            const bool q4 = P.fin_form & FRAG_Q4_0;
+#pragma unroll
+            for (int nt = 0; nt < NTO; nt++) {
+                const v4f ov = o[nt] * unscale;
+                const float v[4] = {ov[0] * scale, (q4 ? ov[2] : ov[1]) * scale, (q4 ? ov[1] : ov[2]) * scale, ov[3] * scale};
+                half4_t hi, lo;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    _Float16 a, b;
+                    split_hi_lo(v[r], a, b);
+                    hi[r] = a; lo[r] = b;
+                }
+                const int e0 = (nt & 1) * 16 + 4 * kq, sw = q4 ? kq : e0 >> 3, sh = q4 ? nt & 1 : kq & 1;       // slot group, half of its entry
+                const long long bt = (long long)(h * (HD / 32) + (nt >> 1)) * P.fin_nt16 + (item >> 4);
+                const int fl = sw * 16 + (item & 15);
+                reinterpret_cast<half4_t *>(P.fin_xf + (bt * 2 + 0) * QG_FRAG + fl)[sh] = hi;
+                reinterpret_cast<half4_t *>(P.fin_xf + (bt * 2 + 1) * QG_FRAG + fl)[sh] = lo;
+            }
+        }
+        return;
+    }
     if (npos[w * 16 + j] > t_first) {
         const int vh = w * 16 + j, item = i0 + vh / G, h = kvh * G + vh % G;
         const long long slot = (long long)item * P.part_item_stride + (long long)h * P.nsplit_max + split;

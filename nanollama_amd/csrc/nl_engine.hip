@@ -564,11 +564,10 @@ hipError_t launch_attn(int hd, int gqa, AttnParams P, dim3 grid, hipStream_t st)
 // developer knobs of the prompt attention, read ONCE per process and in one place: the workgroup list of batched_step
 // and the launchers below must agree on which kernel runs (a list built for attn_tile16_kernel is not a grid of the f32
 // tile kernel)
-struct AttnKnobs { bool f32_tile, no_tile, no_fin; };
+struct AttnKnobs { bool f32_tile, no_tile; };
 static const AttnKnobs &attn_knobs() {
     static const AttnKnobs k{getenv("NL_ATTN_F32") != nullptr,       // the f32-MFMA tile kernel
-                             getenv("NL_NO_ATTN_TILE") != nullptr,   // no tile kernel at all: attn_kernel per token
-                             getenv("NL_NO_ATTN_FIN") != nullptr};
+                             getenv("NL_NO_ATTN_TILE") != nullptr};  // no tile kernel at all: attn_kernel per token
     return k;
 }
 
@@ -2064,7 +2063,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const int nt16 = ((n + 63) / 64) * 4;
     // position splits any token of this step can see: the attention grids skip the rest (a decode batch at short
     // contexts would otherwise dispatch 15 empty workgroups for every live one)
-    const bool no_tile = attn_knobs().no_tile, no_fin = attn_knobs().no_fin;
+    const bool no_tile = attn_knobs().no_tile, no_fin = getenv("NL_NO_ATTN_FIN") != nullptr;   // (no_fin: knob of tests, read per step: the merge launch always)
     int nsplit = 1;
     for (int i = 0; i < n; i++) nsplit = std::max(nsplit, b.h_meta[b.cap + i] / ATT_CH + 1);
     bool consecutive = true;   // positions pos0, pos0 + 1, ...: a prompt
@@ -2185,6 +2184,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 T.pos_base_valid = consecutive ? 1 : 0;   // (a prompt: the kernel derives its key range without reading bpos)
                 T.pos_base = b.h_meta[b.cap];
                 T.live_map = n_live > 0 ? b.tok + 3 * b.cap : nullptr;
+                // every row's keys in one run: no partials, the launch writes WO's fragments (not the float32 tile)
+                if (n_live > 0 && max_nparts == 1 && !kv16_on && !no_fin) {
+                    T.fin_xf = b.xfrag; T.fin_nt16 = nt16; T.fin_form = form(L.wo);
+                    merged = true;
+                }
                 if (n_live > 0 && kv16_on) {
                     // every chunk the prompt can see, split into fp16 halves once for all the tiles that read it
                     const long long so = T.single_stream ? 0 : (long long)b.h_meta[2 * b.cap] * e->kv_stream_stride;
@@ -3664,7 +3668,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
             const char *rk = getenv("NL_ROPE_IN_ATTN"), *fk = getenv("NL_FOLD_NORM"), *pk = getenv("NL_PREFILL_PRECISION"), *kk = getenv("NL_KV16_MIN_TOKENS"),
                        *dk = getenv("NL_DGEMM"), *dm = getenv("NL_DGEMM_MAX_TOKENS"), *hk = getenv("NL_DGEMM_HEAD"), *qk = getenv("NL_QG2_MIN_TOKENS"),
                        *sk = getenv("NL_SGEMM");
-            return 24593 * (sk ? atoi(sk) + 1 : 0) + 40503 * (hk ? atoi(hk) + 1 : 0) + 7919 * (qk ? (atoi(qk) & 0xfff) + 1 : 0) + (rk ? atoi(rk) + 1 : 0) + 3 * (fk ? atoi(fk) + 1 : 0) + 9 * (pk && !strcmp(pk, "fp16x1") ? 1 : 0) +
+            return (getenv("NL_NO_ATTN_FIN") ? 61 * 1024 : 0) + 24593 * (sk ? atoi(sk) + 1 : 0) + 40503 * (hk ? atoi(hk) + 1 : 0) + 7919 * (qk ? (atoi(qk) & 0xfff) + 1 : 0) + (rk ? atoi(rk) + 1 : 0) + 3 * (fk ? atoi(fk) + 1 : 0) + 9 * (pk && !strcmp(pk, "fp16x1") ? 1 : 0) +
                    18 * (dk ? atoi(dk) + 1 : 0) + 54 * (dm ? (atoi(dm) & 0xff) + 1 : 0) + 13878 * (kk ? (atoi(kk) & 0xfff) + 1 : 0);
         };
         if (groups > 1 && groups <= 4) {
