@@ -45,6 +45,16 @@ __device__ __forceinline__ void pg_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// raw buffer loads: a base in scalar registers, a lane's and a scalar 32-bit offset
+typedef unsigned pg_u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned pg_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pg_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, 0xffffffff, 0x00020000);       // (raw, 32-bit elements)
+}
+__device__ __forceinline__ uint4 pg_load16(__amdgpu_buffer_rsrc_t r, unsigned lane_off, unsigned off) {
+    return __builtin_bit_cast(uint4, (pg_u32x4)__builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
+}
+
 enum { PG_NONE = 0, PG_BLOCK = 1 };   // when a sum is multiplied by its scale
 
 // (1024 + b) for the bytes b of u as packed fp16: the two halves of four bytes
@@ -193,25 +203,38 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
     const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
 
     // staging items: pair kk of the chunk's two, row r, half h of the pair, row tile -- a wavefront's loads are runs of 32 bytes
-    const int i_kk = tid & 1, i_r = (tid >> 1) & 15, i_h = (tid >> 5) & 1, i_t = tid >> 6;
+    const int i_kk = tid & 1, i_r = (tid >> 1) & 15, i_h = (tid >> 5) & 1, i_t = wave;
     struct Raw { uint4 c[F::NC]; uint32_t s[SWN]; };
-    auto stage_load = [&](int chunk, Raw (&r)[IPT]) {
+    // Weights as raw buffer loads from the workgroup's first tile: the wavefront's row tile and the chunk are scalar arithmetic, the lane's part is a
+    // register that changes in the last group only.  (With a 64-bit address per load a chunk's staging was 100 of a wavefront's 224 vector
+    // instructions beside 128 MFMAs, and the two add up on a SIMD: 841M F16, 993 tokens 5456 us, now 5400; 173M Q4_K, 333 tokens 1961, now 1911)
+    constexpr unsigned QG = F::CPP * TR * 16, SG = TR * F::SW * 4;      // bytes of a pair over a tile's rows
+    const __amdgpu_buffer_rsrc_t rq0 = pg_rsrc(P.q + (size_t)tile0 * P.npairs * QG), rq1 = pg_rsrc((FUSED ? P.q1 : P.q) + (size_t)tile0 * P.npairs * QG);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs0 = pg_rsrc(reinterpret_cast<const char *>(P.s) + (size_t)tile0 * P.npairs * SG),
+                                                  rs1 = pg_rsrc(reinterpret_cast<const char *>(FUSED ? P.s1 : P.s) + (size_t)tile0 * P.npairs * SG);
+    const unsigned lane_q = (unsigned)((F::chunk(i_h, 0) * TR + i_r) * KL + i_kk) * 16u;
+    auto stage_load = [&](int chunk, Raw (&r)[IPT]) __attribute__((always_inline)) {
+        const int c = min(chunk, (P.npairs - 1) >> 1), g = c >> 1, k0 = (c & 1) * 2, gsz = min(KL, P.npairs - g * KL);      // (a chunk past the end: the last one's, never used)
+        unsigned lq_ = lane_q, step = TR * KL * 16u;          // chunk F::chunk(i_h, j) of the pair: j steps on
+        if (gsz != KL) {
+            lq_ = (unsigned)((F::chunk(i_h, 0) * TR + i_r) * gsz + min(i_kk, gsz - 1 - k0)) * 16u;
+            step = (unsigned)(TR * gsz) * 16u;
+        }
+        [[maybe_unused]] const unsigned ls_ = (lq_ - (unsigned)F::chunk(i_h, 0) * step) / 4u * F::SW;       // (row, pair) words
 #pragma unroll
         for (int i = 0; i < IPT; i++) {
-            const int rt = i_t + 4 * i, tile = min(tile0 + (FUSED ? rt % TPW : rt), P.ntiles - 1);
-            const uint8_t *const Wq = FUSED && rt >= TPW ? P.q1 : P.q;
-            const int pair = min(chunk * 2 + i_kk, P.npairs - 1), g = pair >> 2, k = pair & 3, gsz = min(KL, P.npairs - g * KL);
-            const unsigned gp = (unsigned)(tile * P.npairs + g * KL);
+            const int rt = wave + 4 * i, dt = min(FUSED ? rt % TPW : rt, P.ntiles - 1 - tile0);
+            const bool second = FUSED && rt >= TPW;
+            const unsigned gp = (unsigned)(dt * P.npairs + g * KL);
 #pragma unroll
-            for (int j = 0; j < F::NC; j++)
-                r[i].c[j] = *reinterpret_cast<const uint4 *>(Wq + ((size_t)gp * (F::CPP * TR) + (unsigned)((F::chunk(i_h, j) * TR + i_r) * gsz + k)) * 16);
+            for (int j = 0; j < F::NC; j++) r[i].c[j] = pg_load16(second ? rq1 : rq0, lq_, gp * QG + (unsigned)k0 * 16u + j * step);
             if constexpr (F::SW > 0) {
-                const uint32_t *const Ws = (FUSED && rt >= TPW ? P.s1 : P.s) + ((size_t)gp * TR + (unsigned)(i_r * gsz + k)) * F::SW;
+                const unsigned so = gp * SG + (unsigned)k0 * 4u * F::SW;
                 if constexpr (F::SW == 2) {
-                    const uint2 v = *reinterpret_cast<const uint2 *>(Ws);
-                    r[i].s[0] = v.x;
-                    r[i].s[SWN - 1] = v.y;
-                } else r[i].s[0] = Ws[0];
+                    const pg_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(second ? rs1 : rs0, ls_, so, 0);
+                    r[i].s[0] = v[0];
+                    r[i].s[SWN - 1] = v[1];
+                } else r[i].s[0] = __builtin_amdgcn_raw_buffer_load_b32(second ? rs1 : rs0, ls_, so, 0);
             } else r[i].s[0] = 0;
         }
     };
@@ -239,18 +262,18 @@ __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmP
         }
     };
     // activation fragments [block][token tile][part][lane] x 16 bytes: kernel argument + 32-bit offset, the block part wave-uniform
-    const char *const xsrc = reinterpret_cast<const char *>(P.xf);
-    unsigned xlane[NTW];
+    const __amdgpu_buffer_rsrc_t rx = pg_rsrc(P.xf);
+    unsigned xtile[NTW];
 #pragma unroll
-    for (int t = 0; t < NTW; t++) xlane[t] = ((unsigned)min(ttile0 + t, P.nt16 - 1) * (unsigned)(PS * QG_FRAG) + (unsigned)lane) * 16u;
-    const unsigned xblock = (unsigned)P.nt16 * (unsigned)(PS * QG_FRAG) * 16u;
+    for (int t = 0; t < NTW; t++) xtile[t] = (unsigned)min(ttile0 + t, P.nt16 - 1) * (unsigned)(PS * QG_FRAG * 16);
+    const unsigned xblock = (unsigned)P.nt16 * (unsigned)(PS * QG_FRAG) * 16u, xlane = (unsigned)lane * 16u;
     uint4 xp[NP][KB][NTW];
-    auto xload = [&](int chunk, int b) {
+    auto xload = [&](int chunk, int b) __attribute__((always_inline)) {
         const unsigned uo = (unsigned)min(chunk * KB + b, nblocks - 1) * xblock;
 #pragma unroll
         for (int t = 0; t < NTW; t++)
 #pragma unroll
-            for (int k = 0; k < NP; k++) xp[k][b][t] = *reinterpret_cast<const uint4 *>(xsrc + (uo + xlane[t]) + k * QG_FRAG * 16);
+            for (int k = 0; k < NP; k++) xp[k][b][t] = pg_load16(rx, xlane, uo + xtile[t] + k * QG_FRAG * 16);
     };
     f32x4_t acc[RT][NTW];
 #pragma unroll

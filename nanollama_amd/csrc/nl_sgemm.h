@@ -47,13 +47,6 @@ inline size_t sg_lds_bytes(bool norm, int cols, int waves, int tpl) {
 
 // Raw buffer loads: one SGPR base, 32-bit offsets.  (Skipping the vector L1, as nl_dgemm.h does, loses here: a token tile's rows and a row's second
 // half of a sector are hits.  gate || up of 1536 x 4096 F16, 64 tokens: 18.2 us a launch through it, 22.8 past it)
-typedef unsigned sg_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t sg_rsrc(const void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, 0xffffffff, 0x00020000);       // (raw, 32-bit elements)
-}
-__device__ __forceinline__ uint4 sg_load16(__amdgpu_buffer_rsrc_t r, unsigned lane_off, unsigned off) {
-    return __builtin_bit_cast(uint4, (sg_u32x4)__builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
-}
 
 // A chunk (two pairs of blocks) of one 16-row tile, 16 bytes a lane and load: lane (row li, group lq) takes pair lq & 1, so that a row's two pairs
 // (32 bytes) travel in one request, and the operand order -- each of the four groups an eighth of a block -- is made by swapping 16- and
@@ -134,7 +127,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
     float *const part = reinterpret_cast<float *>(sg_lds + (NORM ? (size_t)nblocks * 2048 + (size_t)P.cols * 4 + (size_t)nw * 128 : 0));    // [wavefront][token][row]
 
     // ---- requests, oldest first: the rows (NORM), then the weights ----
-    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rx = sg_rsrc(NORM ? (const void *)P.x : (const void *)P.xf);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rx = pg_rsrc(NORM ? (const void *)P.x : (const void *)P.xf);
     // (NORM: four lanes take 64 bytes of a row's 128-byte block, lane >> 2 is the row)
     const int xr = lane >> 2, xq = lane & 3;
     [[maybe_unused]] const unsigned xrow = (unsigned)min(tt * 16 + xr, P.n_tokens - 1) * (unsigned)P.cols * 4u + (unsigned)xq * 16u;
@@ -145,8 +138,8 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
 #pragma unroll
         for (int i = 0; i < XB; i++) {
             const unsigned o = (unsigned)min(wv + (i0 + i) * nw, nblocks - 1) * 128u;
-            xa[i] = sg_load16(rx, xrow, o);
-            xb[i] = sg_load16(rx, xrow, o + 64u);
+            xa[i] = pg_load16(rx, xrow, o);
+            xb[i] = pg_load16(rx, xrow, o + 64u);
         }
     };
     if constexpr (NORM) {
@@ -160,7 +153,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
     [[maybe_unused]] uint32_t wd[DEP][TPL];                           // pair lq & 1's two scales
     [[maybe_unused]] uint4 xh[DEP][QG_KC], xl[DEP][QG_KC];
     [[maybe_unused]] const unsigned xblock = (unsigned)P.nt16 * (2 * QG_FRAG * 16), xtile = (unsigned)tt * (2 * QG_FRAG * 16);
-    const __amdgpu_buffer_rsrc_t rw = sg_rsrc(FUSED && mat ? P.q1 : P.q), rs = sg_rsrc(FUSED && mat ? P.s1 : P.s);
+    const __amdgpu_buffer_rsrc_t rw = pg_rsrc(FUSED && mat ? P.q1 : P.q), rs = pg_rsrc(FUSED && mat ? P.s1 : P.s);
     auto request = [&](int d, int c) __attribute__((always_inline)) {                           // chunk c of this split into ring place d (clamped past the last one, never used there)
         const int b0 = min(z + c * P.ks, nchunks - 1) * QG_KC, g = b0 >> 3, k0 = (b0 >> 1) & 3;
         const int gsz = min(KL, P.npairs - g * KL), second = k0 + 1 < gsz ? 1 : 0;
@@ -168,8 +161,8 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
 #pragma unroll
             for (int b = 0; b < QG_KC; b++) {
                 const unsigned o = xtile + (unsigned)min(b0 + b, nblocks - 1) * xblock;
-                xl[d][b] = sg_load16(rx, lane * 16u, o + QG_FRAG * 16);
-                xh[d][b] = sg_load16(rx, lane * 16u, o);
+                xl[d][b] = pg_load16(rx, lane * 16u, o + QG_FRAG * 16);
+                xh[d][b] = pg_load16(rx, lane * 16u, o);
             }
         }
         const unsigned lw = SgW<WT>::lane(li, lq, gsz, second), ls = (unsigned)(li * gsz + (lq & second)) * 4u;
@@ -178,7 +171,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
             const unsigned gp = (unsigned)(min(tile0 + t, P.ntiles - 1) * P.npairs + g * KL);
             const unsigned gq = gp * (WFrag<WT>::CPP * TR * 16) + (unsigned)k0 * 16u;
 #pragma unroll
-            for (int i = 0; i < NL; i++) wq[d][t][i] = sg_load16(rw, lw, gq + SgW<WT>::uni(i, gsz, second));
+            for (int i = 0; i < NL; i++) wq[d][t][i] = pg_load16(rw, lw, gq + SgW<WT>::uni(i, gsz, second));
             if constexpr (WTraits<WT>::SCALED) wd[d][t] = __builtin_amdgcn_raw_buffer_load_b32(rs, ls, gp * (TR * 4) + (unsigned)k0 * 4u, 0);
         }
     };
