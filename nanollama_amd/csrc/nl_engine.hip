@@ -2001,7 +2001,7 @@ hipError_t launch_qgemm_plain(nl_engine *e, nl_engine::Batch &bt, const PackedMa
 }
 
 // One multi-token step: n <= 64 (token, pos, stream) triples through every layer on the MFMA path.
-// lm_mode: 0 = no LM head, 1 = logits + argmax for every token, 2 = logits + argmax for the LAST token only.
+// lm_mode: 0 = no LM head, 1 = logits + argmax for every token, 2 = logits + argmax for the LAST token only, in e->logits / e->result.
 // The caller has filled bt.h_meta; stream-ordered, no synchronisation inside.
 int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int lm_mode, bool one_stream = false) {
     const nl_config &c = e->cfg;
@@ -2300,7 +2300,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         }
     }
     if (lm_mode) {
-        // logits rows [0, cnt) of bt.logits / ids [0, cnt): all tokens (mode 1, n <= lm_cap) or just the last (mode 2)
+        // logits rows [0, cnt) of bt.logits / ids [0, cnt): all tokens (mode 1, n <= lm_cap); or just the last one's (mode 2)
         const int first = lm_mode == 2 ? n - 1 : 0, cnt = lm_mode == 2 ? 1 : n;
         if (cnt > b.lm_cap) return e->fail(NL_ERR_INVALID, "LM head batch %d exceeds %d", cnt, b.lm_cap);
         if (dg_head) {
@@ -2313,9 +2313,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(launch_dgemm_head(P, st, e->num_cus));
             hipLaunchKernelGGL(dg_argmax_kernel, dim3(n), dim3(1024), 0, st, reinterpret_cast<const uint2 *>(b.kpart), m.ntiles, b.ids);
         } else {
+            // (the last token's go where single-token steps leave theirs)
+            float *const rows = lm_mode == 2 ? e->logits : b.logits;
             LCK(norm(e->output_norm, e->lm_head, first, cnt));
-            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, b.logits, c.vocab, st, exact));
-            hipLaunchKernelGGL(bargmax_kernel, dim3(cnt), dim3(1024), 0, st, b.logits, c.vocab, b.ids);
+            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, rows, c.vocab, st, exact));
+            hipLaunchKernelGGL(bargmax_kernel, dim3(cnt), dim3(1024), 0, st, rows, c.vocab, lm_mode == 2 ? e->result : b.ids);
         }
         LCK(hipGetLastError());
     }
@@ -3605,12 +3607,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
                 b.h_meta[2 * b.cap + i] = stream;
             }
             const bool last = t0 + m == n;
-            if ((rc = batched_step(e, b, e->stream, m, last ? 2 : 0, true))) return rc;
-            if (last) {
-                // keep the single-token state coherent: logits / argmax of the last token
-                HIPCK(e, hipMemcpyAsync(e->logits, b.logits, (size_t)e->cfg.vocab * 4, hipMemcpyDeviceToDevice, e->stream));
-                HIPCK(e, hipMemcpyAsync(e->result, b.ids, sizeof(int), hipMemcpyDeviceToDevice, e->stream));
-            }
+            if ((rc = batched_step(e, b, e->stream, m, last ? 2 : 0, true))) return rc;      // (2: logits / argmax of the last token, in e->logits / e->result)
         }
     } else {
         for (int attempt = 0;; attempt++) {

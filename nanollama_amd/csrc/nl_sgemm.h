@@ -9,7 +9,7 @@
 // and what sums them; now): 89M Q8_0, 24 tokens, Q|K|V 3.5 + 4.7 + 4.6, now 5.8; gate || up 3.5 + 4.8 + 4.0, now 6; WO 4.6, now 3.6; a prompt of 24 / 64 tokens
 // 632 -> 457 / 722 -> 503 us, 173M Q8_0 1120 -> 770 / 1200 -> 796, 841M 1650 -> 1390 / 1970 -> 1720, F16 1840 -> 1570 / 2080 -> 1906; a step of 64 streams
 // at position 150: 89M 785 -> 604, 173M 1105 -> 823, 841M Q8_0 1923 -> 1750, F16 1968 -> 1934.  What bounds a launch now is one workgroup's chain: requests,
-// the norm (2.5 of 5.8 us), products at the vector pipe's rate (10 instructions an expansion, 4 a scaling), the meeting of the partial tiles.
+// the norm (2.2 of 5.0 us), products at the vector pipe's rate (10 instructions an expansion, 4 a scaling), the meeting of the partial tiles.
 //
 // A workgroup owns 16 tokens x TW (x 2: gate and up) 16-row weight tiles; its KS x TW wavefronts are (split z, tile).  Split z multiplies the
 // 128-column chunks z, z + KS, ... in order, exactly those that a split of qgemm_kernel takes (KS is qgemm_kernel's rule too), and the
@@ -37,6 +37,7 @@ struct SGemmParams {
     int ks, tw;                  // K splits, row tiles of a workgroup
     int out_form;                // k-slot order of xf_out
     float eps;
+    double rcols;                // 1 / cols
     QGemmParams::Rope rope;
 };
 
@@ -107,12 +108,13 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
     extern __shared__ __attribute__((aligned(16))) uint8_t sg_lds[];
     NL_KARGS8(P.q, P.s, P.x, P.normw, P.xf, P.out, P.bias, P.xf_out);
     NL_KARGS8(P.rows, P.cols, P.npairs, P.ntiles, P.nt16, P.n_tokens, P.ks, P.tw);
+    if constexpr (NORM) NL_KARGS2(P.eps, P.rcols);
     if constexpr (FUSED) NL_KARGS4(P.q1, P.s1, P.out_form, P.eps);
     if constexpr (EPI == QG_EPI_ROPE) {
         NL_KARGS8(P.rope.tcos, P.rope.tsin, P.rope.tkv, P.rope.q, P.rope.kcache, P.rope.vcache, P.rope.bias_q, P.rope.bias_k);
         NL_KARGS8(P.rope.bias_v, P.rope.head_dim, P.rope.n_q_heads, P.rope.n_kv_heads, P.rope.seq_len, P.rope.conj, P.eps, P.s);
     }
-    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nw = (int)blockDim.x >> 6;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nw = NORM ? NWV : (int)blockDim.x >> 6;      // (NORM: always that many)
     const int li = lane & 15, lq = lane >> 4;
     // wavefront: split, then (tile, matrix)
     const int ksl = 31 - __builtin_clz(P.ks), z = wv & (P.ks - 1), tw = (wv >> ksl) / MT, mat = MT == 1 ? 0 : (wv >> ksl) & 1;
@@ -216,15 +218,23 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
         if (tid * 4 < P.cols) *reinterpret_cast<uint4 *>(ws + tid * 4) = wn;
         for (int i = (tid + nw * 64) * 4; i < P.cols; i += nw * 256) *reinterpret_cast<float4 *>(ws + i) = *reinterpret_cast<const float4 *>(P.normw + i);
         for (int i0 = XB; i0 < nxb; i0 += XB) { xload(i0); xput(i0); }     // (more than 2048 columns: none fit the LDS)
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
+        ss += dpp_f64<DPP_QUAD_XOR1>(ss);
+        ss += dpp_f64<DPP_QUAD_XOR2>(ss);
         if (xq == 0) red[wv * 16 + xr] = ss;
         pg_barrier();
         int offa, offb;
         slot_offsets(FORM, lq, offa, offb);
-        double tot = 0.0;
-        for (int k = 0; k < nw; k++) tot += red[k * 16 + li];
-        const float inv = dg_inv_rms(tot, P.cols, P.eps);
+        double tot = 0.0, sq[NWV];
+#pragma unroll
+        for (int k = 0; k < NWV; k++) sq[k] = red[k * 16 + li];      // (in flight together)
+#pragma unroll
+        for (int k = 0; k < NWV; k++) tot += sq[k];
+        // dg_inv_rms with its division on the host
+        const double m = fma(tot, P.rcols, (double)P.eps);
+        double y0 = __builtin_amdgcn_rsq(m);
+        y0 = y0 * fma(-0.5 * m * y0, y0, 1.5);
+        y0 = y0 * fma(-0.5 * m * y0, y0, 1.5);
+        const float inv = (float)y0;
         for (int i = 0; i < nxb; i++) {
             const int blk = wv + i * nw;
             uint4 *const at = xs + (size_t)blk * (2 * QG_FRAG);
@@ -415,6 +425,7 @@ inline hipError_t sg_launch(int wtype, SGemmParams P, hipStream_t st) {
     constexpr bool NORM = EPI != QG_EPI_PLAIN;
     constexpr int MT = EPI == QG_EPI_SWIGLU ? 2 : 1;
     P.nt16 = ((P.n_tokens + 63) / 64) * 4;
+    P.rcols = 1.0 / (double)P.cols;
     if (!sg_fits(NORM, MT, P.cols, P.ks)) return hipErrorInvalidValue;
     P.tw = sg_tw(NORM, MT, P.ks, P.ntiles, P.n_tokens);
     const int waves = sg_waves(NORM, MT, P.ks, P.tw);
