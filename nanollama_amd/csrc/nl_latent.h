@@ -88,6 +88,123 @@ template <typename T> struct LatentStore {
     }
 };
 
+// The queries of a step of up to LQ_TOKENS tokens in one launch: norm of their latent, product with uq, rotation, and for the unrotated part
+// the product with uk's transpose behind it.  Launch latency bounds both products, not their weights (a head's 96 + 64 KB at 128 dimensions,
+// latents of 384 and 256), so a head's unrotated queries are computed by every workgroup that needs them, one per eight row tiles of the second
+// product, a row tile to a wavefront, whose weights are in flight beside the first product's.  Workgroups of a head are 8 h' apart and share an
+// L2.  Sums are few_kernel's: k tile ks of the first product in partial ks % 8, every k tile of the second in a partial of its own, partials
+// added in order; the queries pass from one product to the other in the operand's type.  One launch fewer a layer: 36.6 -> 34.5 us (768 columns).
+constexpr int LQ_TOKENS = 4, LQ_ROWS = 8, LQ_KS = 3;   // tokens; row tiles of a head; k tiles per wavefront
+struct LatentQueryParams {
+    const void *W1, *W2;        // uq; uk's transpose, w2t row tiles per head
+    const float *nx, *nw;       // queries' latent [token][nld], weights of its norm
+    int nks, n, ndim, nld, heads, dt, nrot, w2t, chunks;    // dt: row tiles of a head's unrotated rows; nrot: rotated row tiles of all heads
+    float eps;
+    HeadRows hd;                // of the first product
+};
+// workgroups of a chunk: heads, groups of as many rotated row tiles as a head has, up to a multiple of the XCDs
+__host__ __device__ inline int latent_query_units(const LatentQueryParams &P) { return (P.heads + (P.nrot + P.dt - 1) / P.dt + 7) & ~7; }
+inline bool latent_query_ok(int n, int nks, int dimp) { return n <= LQ_TOKENS && nks <= 8 * LQ_KS && dimp <= 16 * LQ_ROWS; }
+
+template <int NS, int KT>
+__global__ void __launch_bounds__(512) latent_query_kernel(LatentQueryParams P, LatentStore<bf16> tail) {
+    __shared__ __align__(16) f32x4 red[8 * LQ_ROWS * 4 * NS];               // [wavefront][row tile][g][token]
+    __shared__ __align__(16) bf16 xs[8 * KT * 32 * NS];                     // [k tile][g][token][8]
+    __shared__ __align__(16) bf16 qs[LQ_ROWS / 2 * 32 * NS];
+    __shared__ __align__(16) float nsum[NS * 8];
+    NL_KARGS8(P.W1, P.W2, P.nx, P.nw, P.nks, P.n, P.ndim, P.nld);           // one batch of s_load
+    NL_KARGS8(P.heads, P.dt, P.nrot, P.w2t, P.chunks, P.eps, P.hd.q, P.hd.ld);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, col = lane & 15, n = P.n, nks = P.nks;
+    const int hs = latent_query_units(P), c = blockIdx.x / hs, h = blockIdx.x - c * hs;    // h: a head, or a group of rotated rows behind them
+    if (c == P.chunks) {
+        if (h * 8 + w < tail.units) tail.unit(h * 8 + w, lane);
+        return;
+    }
+    const bool rot = h >= P.heads;
+    const int rt0 = h * P.dt, nrt = min(P.heads * P.dt + P.nrot - rt0, P.dt);
+    if (nrt <= 0 || (rot && c)) return;
+    f32x4 xv[NS], wv = {};
+    const bool in = tid * 4 < P.ndim;
+    if (in) wv = *reinterpret_cast<const f32x4 *>(P.nw + tid * 4);
+#pragma unroll
+    for (int s = 0; s < NS; s++) xv[s] = in && s < n ? *reinterpret_cast<const f32x4 *>(P.nx + (long long)s * P.nld + tid * 4) : f32x4{};
+    Frag<bf16> a[KT][LQ_ROWS], a2[LQ_ROWS / 2];
+#pragma unroll
+    for (int u = 0; u < KT; u++)
+#pragma unroll
+        for (int r = 0; r < LQ_ROWS; r++)
+            a[u][r] = reinterpret_cast<const Frag<bf16> *>(P.W1)[((long long)(rt0 + min(r, nrt - 1)) * nks + min(w + 8 * u, nks - 1)) * 64 + lane];
+    const int row2 = c * 8 + w, nk2 = P.dt / 2;
+    const bool second = !rot && row2 < P.w2t;
+    if (second)
+#pragma unroll
+        for (int k = 0; k < LQ_ROWS / 2; k++)
+            a2[k] = reinterpret_cast<const Frag<bf16> *>(P.W2)[((long long)(h * P.w2t + row2) * nk2 + min(k, nk2 - 1)) * 64 + lane];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const float ss = wave_sum(0.f + (xv[s][0] * xv[s][0] + xv[s][1] * xv[s][1] + xv[s][2] * xv[s][2] + xv[s][3] * xv[s][3]));
+        if (lane == 0) nsum[s * 8 + w] = ss;
+    }
+    lds_barrier();
+    if (tid * 4 < nks * 32)
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const f32x4 q = *reinterpret_cast<const f32x4 *>(nsum + s * 8) + *reinterpret_cast<const f32x4 *>(nsum + s * 8 + 4);
+            const float inv = rsqrt_f32(((q[0] + q[1]) + (q[2] + q[3])) / (float)P.ndim + P.eps);
+            put4(xs + ((tid >> 1) * NS + s) * 8 + (tid & 1) * 4, xv[s] * inv * wv);
+        }
+    lds_barrier();
+    f32x4 acc[LQ_ROWS] = {};
+#pragma unroll
+    for (int u = 0; u < KT; u++) {
+        const int ks = w + 8 * u;
+        if (ks >= nks) break;
+        Frag<bf16> x;
+        frag_zero(x);
+        if (col < n) x = *reinterpret_cast<const Frag<bf16> *>(xs + ((ks * 4 + g) * NS + col) * 8);
+#pragma unroll
+        for (int r = 0; r < LQ_ROWS; r++) acc[r] = mma(a[u][r], x, acc[r]);
+    }
+    if (col < NS)
+#pragma unroll
+        for (int r = 0; r < LQ_ROWS; r++) red[((w * LQ_ROWS + r) * 4 + g) * NS + col] = acc[r];
+    lds_barrier();
+    if (tid < LQ_ROWS * 4 * NS) {
+        const int tok = tid % NS, rg = tid / NS, r = rg >> 2;               // rows 4 rg .. 4 rg + 3
+        f32x4 v = {};
+#pragma unroll
+        for (int q = 0; q < 8; q++) v += red[q * LQ_ROWS * 4 * NS + tid];
+        if (r < nrt && tok < n) {
+            if (rot) store_heads<bf16>(P.hd, tok, rt0 * 16 + rg * 4, v);
+            else put4(qs + ((rg >> 1) * NS + tok) * 8 + (rg & 1) * 4, v);
+        }
+    }
+    if (rot) return;
+    lds_barrier();
+    if (!second) return;
+    f32x4 o = {};
+#pragma unroll
+    for (int k = 0; k < LQ_ROWS / 2; k++)
+        if (k < nk2) {
+            Frag<bf16> x;
+            frag_zero(x);
+            if (col < n) x = *reinterpret_cast<const Frag<bf16> *>(qs + ((k * 4 + g) * NS + col) * 8);
+            o += mma(a2[k], x, f32x4{});
+        }
+    if (col < n) put4(reinterpret_cast<bf16 *>(P.hd.q) + ((long long)col * P.heads + h) * P.hd.ld + row2 * 16 + 4 * g, o);
+}
+
+inline hipError_t launch_latent_query(const LatentQueryParams &P, const LatentStore<bf16> &store, hipStream_t st) {
+    const dim3 grid(P.chunks * latent_query_units(P) + (store.units + 7) / 8);   // (one workgroup for at most LQ_TOKENS units)
+    auto go = [&](auto kfn) {
+        hipLaunchKernelGGL(kfn, grid, dim3(512), 0, st, P, store);
+        return hipGetLastError();
+    };
+    const bool two = P.nks <= 16;
+    if (P.n == 1) return two ? go(latent_query_kernel<1, 2>) : go(latent_query_kernel<1, 3>);
+    return two ? go(latent_query_kernel<LQ_TOKENS, 2>) : go(latent_query_kernel<LQ_TOKENS, 3>);
+}
+
 // one wavefront per (key tile of the list, rotated tile): r behind every head's expanded key
 template <typename T> struct RotatedKeys {
     static constexpr bool on = true;

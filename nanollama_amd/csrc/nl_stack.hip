@@ -433,6 +433,14 @@ hipError_t logits_launch(nl_engine *e, const int *rows, int n, float *out) {
     return normed_product<T, ST_F32>(e, P, e->final_norm, rows, true);
 }
 
+// do a decode step's queries take one launch?  Wherever the kernel can hold them: us a step as two launches and as one, positions around 260,
+// 20 layers of 768 columns, 1 / 2 / 4 streams: 732 / 823 / 907, 691 / 783 / 861; 28 of 1536: 1230 / 1349 / 1491, 1160 / 1307 / 1446.  It
+// recomputes a head's queries per 128 latent columns, which 32-bit weights would double: those keep two launches.
+template <typename T>
+bool one_query_launch(int n, const Layer &L) {
+    return std::is_same_v<T, bf16> && few_norm_ok(n, L.uq.nks, L.d.latent.q_rank, L.proj.rows) && latent_query_ok(n, L.uq.nks, L.dimp);
+}
+
 // behind the projections: everything up to the output matrix's operand
 template <typename T>
 hipError_t latent_mixer(nl_engine *e, const StepIn &s, const Run &R, const Layer &L) {
@@ -453,6 +461,14 @@ hipError_t latent_mixer(nl_engine *e, const StepIn &s, const Run &R, const Layer
     H.ld = (s.decode ? L.nks : qt) * 32;
     H.col[1] = s.decode ? L.kvt * 32 : L.dimp;
     if (s.decode) { H.xq = e->xq; H.xq_nks = L.xq_nks(); }
+    if constexpr (std::is_same_v<T, bf16>)
+        if (s.decode && one_query_launch<T>(s.n, L)) {
+            LatentQueryParams Q{};
+            Q.W1 = L.uq.w; Q.W2 = L.ukt.w; Q.nx = e->proj + L.tdq; Q.nw = L.dqnorm; Q.nks = L.uq.nks; Q.n = s.n; Q.ndim = N.q_rank; Q.nld = L.proj.rows;
+            Q.heads = N.heads; Q.dt = L.dimp / 16; Q.nrot = L.uq.nrt - N.heads * Q.dt; Q.w2t = L.kvt * 2; Q.chunks = (Q.w2t + 7) / 8; Q.eps = e->c.eps; Q.hd = H;
+            if ((rc = launch_latent_query(Q, store, st)) || (rc = launch_latent_decode<T>(A, s.n, st))) return rc;
+            return launch_latent_out<T>(A, s.n, st);
+        }
     if (few_norm_ok(s.n, L.uq.nks, N.q_rank, L.proj.rows)) {
         P.nx = e->proj + L.tdq; P.nw = L.dqnorm; P.ndim = N.q_rank; P.nld = L.proj.rows;
         rc = store.units ? launch_product<T, ST_HEADS>(P, st, 1, store) : launch_product<T, ST_HEADS>(P, st, 1);
@@ -513,7 +529,10 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
         J.out = e->proj; J.ldo = L.proj.rows;
         // (what reads ahead: latent attention's own launches keep up to 100 KB of LDS per workgroup, so its products do, 707 against 744 us a
         // token; the other mixers' launch has room on every CU, 582 against 631 us a step of 16 streams)
-        if (L.d.latent.heads) J.ahead = look_ahead<T>(e, s.n, {{&L.uq, 1}, {&L.ukt, 1}, {&L.uv, 1}, {&L.out, 1}});
+        if (L.d.latent.heads) {
+            const bool one = s.decode && one_query_launch<T>(s.n, L);
+            J.ahead = look_ahead<T>(e, s.n, {{&L.uq, one ? L.dimp / 16 : 1}, {&L.ukt, one ? L.kvt * 2 : 1}, {&L.uv, 1}, {&L.out, 1}});
+        }
         if ((rc = normed_product<T, ST_F32>(e, J, L.norm1))) return rc;
         WinParams W{};
         W.pos = s.pos; W.stream = s.stream; W.nsplit = 1; W.y = e->y; W.y_nks = L.out.nks; W.proj = e->proj; W.ldp = L.proj.rows;
