@@ -6,8 +6,9 @@
 // down in slabs).  Here the K splits of a tile are wavefronts of ONE workgroup, so their partial tiles meet in LDS and the rotation, SiLU and
 // residual epilogues follow in the same launch; the norm is the prologue of the launch that consumes it: 6 launches a layer, 5 for decode
 // batches.  Measured (profiled, us a launch, before: a norm, a GEMM in slabs
-// and what sums them; now): 89M Q8_0, 24 tokens, Q|K|V 3.5 + 4.7 + 4.6, now 5.8; gate || up 3.5 + 4.8 + 4.0, now 6; WO 4.6, now 3.6; a prompt of 24 / 64 tokens
-// 632 -> 457 / 722 -> 503 us, 173M Q8_0 1120 -> 770 / 1200 -> 796, 841M 1650 -> 1390 / 1970 -> 1720, F16 1840 -> 1570 / 2080 -> 1906; a step of 64 streams
+// and what sums them; now): 89M Q8_0, 24 tokens, Q|K|V 3.5 + 4.7 + 4.6, now 5.0; gate || up 3.5 + 4.8 + 4.0, now 5.2; WO 4.6, now 3.6; a prompt of 24 / 64 tokens
+// (its attention in one launch a layer as well, nl_batch.h) 703 -> 409 / 774 -> 434 us, 173M Q8_0 1092 -> 641 / 1227 -> 711, 841M 1766 -> 1255 / 2026 -> 1552,
+// F16 1831 -> 1394 / 2074 -> 1742; a step of 64 streams
 // at position 150: 89M 785 -> 604, 173M 1105 -> 823, 841M Q8_0 1923 -> 1750, F16 1968 -> 1934.  What bounds a launch now is one workgroup's chain: requests,
 // the norm (2.2 of 5.0 us), products at the vector pipe's rate (10 instructions an expansion, 4 a scaling), the meeting of the partial tiles.
 //
