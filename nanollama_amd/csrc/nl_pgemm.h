@@ -171,8 +171,11 @@ enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 // EPI: QG_EPI_PLAIN (out / resid / bias; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
 // (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  PREC: PG_HILO; PG_HI, the single-product precision mode of
 // Q4_0 prompts (block scales multiplied into the fp16 weights, only the hi half of every activation); PG_EXACT.
+// Wavefronts per SIMD: a plain 64 x 64 Q4_0 tile is held to 168 registers, three workgroups a compute unit (172 without the bound, since the
+// loads are buffer loads: two.  WO and down of 2112 x 2112 and 2112 x 5632, 1000 tokens, 528 workgroups, mean of both: 63.4 us two at a time,
+// 53.9 three).  What it spills is one value of the epilogue's, around the K loop.
 template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO>
-__global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) pgemm_kernel(QGemmParams P) {
+__global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT == 4 && NTW == 1 && PREC == PG_HILO ? 3 : 2)) pgemm_kernel(QGemmParams P) {
     constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
     using F = typename std::conditional_t<EXACT, PgExact<WT>, PgFmt<WT>>;
     static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");

@@ -1,0 +1,42 @@
+"""Registers and LDS of launches whose tiling counts on so many workgroups a compute unit, read from the built library's own kernel metadata."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from nanollama_amd import _lib
+
+LLVM = "/opt/rocm/llvm/bin/"
+
+# kernel<template arguments>, wavefronts of a workgroup, workgroups on a compute unit (512 registers a SIMD lane over four SIMDs, 160 KB of LDS)
+RESIDENT = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 1, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 2, 0>", 4, 3)]
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    if not os.path.exists(LLVM + "clang-offload-bundler"):
+        pytest.skip("no LLVM tools")
+    _lib.lib()                                     # (builds it where nothing is built)
+    d = tmp_path_factory.mktemp("co")
+    run = lambda *a: subprocess.run(a, check=True, capture_output=True, text=True).stdout
+    run(LLVM + "llvm-objcopy", "--dump-section", f".hip_fatbin={d}/fat", _lib.LIB_PATH, "/dev/null")
+    run(LLVM + "clang-offload-bundler", "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={d}/fat", f"--output={d}/co")
+    out, cur = {}, {}
+    for line in run(LLVM + "llvm-readelf", "--notes", f"{d}/co").splitlines():
+        m = re.match(r" +(?:- )?\.(symbol|vgpr_count|group_segment_fixed_size|max_flat_workgroup_size): +(\S+)", line)
+        if m:
+            cur[m[1]] = m[2].strip("'")
+        if ".wavefront_size" in line:
+            out[cur.pop("symbol")] = cur
+            cur = {}
+    names = subprocess.run(["c++filt"], input="\n".join(n.removesuffix(".kd") for n in out), capture_output=True, text=True, check=True).stdout.splitlines()
+    return dict(zip(names, out.values()))
+
+
+@pytest.mark.parametrize("name,waves,groups", RESIDENT)
+def test_workgroups_a_compute_unit(kernels, name, waves, groups):
+    k, = [v for n, v in kernels.items() if name in n]
+    assert int(k["max_flat_workgroup_size"]) == waves * 64
+    registers = -(-int(k["vgpr_count"]) // 8) * 8
+    assert 4 * (512 // registers) // waves >= groups and 160 * 1024 // int(k["group_segment_fixed_size"]) >= groups, k
