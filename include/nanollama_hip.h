@@ -193,7 +193,9 @@ NL_API int nl_persist_info(nl_handle h, int *ready, int *max_pos, long long *lau
 /* Device bytes held by the handle (weights, KV, state). */
 NL_API int nl_memory_usage(nl_handle h, uint64_t *weights, uint64_t *kv_cache, uint64_t *state);
 /* Read back a device state buffer for tests ("x","q","xb2","hb","logits",
- * "k_cache","v_cache"); returns floats copied (<= max_floats). */
+ * "k_cache","v_cache"), or, as one float, which kernels the last multi-token step
+ * ran on ("step_path": 1 | 2 decode-batch / short-step GEMM, 4 | 8 attention of a
+ * prompt / of a decode batch in one launch); returns floats copied (<= max_floats). */
 NL_API int64_t nl_debug_read(nl_handle h, const char *which, int stream, float *out, int64_t max_floats);
 
 /* Shader-clock phase stamps of one GEMV launch (developer tool, tools/phase_probe.py). */

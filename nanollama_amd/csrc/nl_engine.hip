@@ -134,6 +134,9 @@ struct Op {
 
 }  // namespace
 
+// nl_engine::step_path: which kernels a layer of a multi-token step ran on (none of the first two: qgemm_kernel / pgemm_kernel, by matrix)
+enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */ };
+
 struct nl_engine {
     nl_config cfg{};
     std::string err;
@@ -225,13 +228,14 @@ struct nl_engine {
         Batch bt;
         hipStream_t st = nullptr;
         hipEvent_t done = nullptr;
-        struct G { int n, nsplit; hipGraph_t graph; hipGraphExec_t exec; };
+        struct G { int n, nsplit; hipGraph_t graph; hipGraphExec_t exec; int path; };
         std::vector<G> graphs;
     } sub[4];
     int dg_state = 0;             // dgemm_kernel's weight copies: 0 not looked at yet, 1 built, -1 the model does not qualify
     bool dg_head = false;         // ... and the LM head has one too (decode batches: dgemm_kernel with the argmax candidates in its epilogue)
     std::vector<SubBatch::G> bt_graphs;   // step graphs of the whole-batch decode step (bt), same key
     hipEvent_t sub_fork = nullptr;
+    int step_path = 0;            // launches of the last multi-token step (PATH_* bits; nl_debug_read "step_path")
     int sub_batches = 1;          // NL_SUB_BATCHES: groups a decode batch is cut into (1 = the whole batch as one step: measured fastest, profiles/r04_subbatch_groups.log)
 
     // on-device sampling (nl_sample_decode): scratch for one vocabulary, allocated on first use
@@ -1957,20 +1961,33 @@ bool dgemm_step_ok(const nl_engine *e, int n) {
 }
 
 // ---- short multi-token steps on sgemm_kernel (nl_sgemm.h): the splits that qgemm_kernel's launches of the same step would take ----
-int sgemm_splits(const nl_engine::Batch &b, const PackedMat &m, int mats, int n, bool whole) {
-    return whole ? 1 : qgemm_geometry(m.ntiles, mats, m.cols, n, true, m.rows, b.kpart_cap).ks;
+struct SgSplits { int qkv, gate, wo, down; };
+SgSplits sgemm_splits(const nl_engine::Batch &b, const nl_engine::Layer &L, int n) {
+    auto of = [&](const PackedMat &m, int mats, bool whole) { return whole ? 1 : qgemm_geometry(m.ntiles, mats, m.cols, n, true, m.rows, b.kpart_cap).ks; };
+    return SgSplits{of(L.qkv, 1, qgemm_rope_fits(L.qkv, n)), of(L.gate, 2, qgemm_swiglu_fits(L.gate, n)), of(L.wo, 1, false), of(L.down, 1, false)};
 }
-int sgemm_splits_qkv(const nl_engine::Batch &b, const nl_engine::Layer &L, int n) { return sgemm_splits(b, L.qkv, 1, n, qgemm_rope_fits(L.qkv, n)); }
-int sgemm_splits_gate(const nl_engine::Batch &b, const nl_engine::Layer &L, int n) { return sgemm_splits(b, L.gate, 2, n, qgemm_swiglu_fits(L.gate, n)); }
-bool sgemm_step_ok(const nl_engine *e, const nl_engine::Batch &b, int n) {
-    const char *k = getenv("NL_SGEMM");                 // knob (tests, tools; read per step): 0 keeps qgemm_kernel's launches
+// Which steps: those whose four launches a layer are few rounds of workgroups.  sgemm_kernel reads and expands the weights once per 16 tokens, the
+// launches it replaces once per 64, so it wins by the four to six launches it saves and loses where it is rounds long.  Its gain over them, layers of
+// 1024 to 2112 columns (a recorded step of 3 to 64 streams / an eager prompt of 3 to 128 tokens), least and median by rounds:
+//   Q8_0, F16  4 rounds 1.05 1.13 / 1.11 1.26;  5 0.99 1.04 / 1.07 1.16;  6 0.94 0.99 / 1.01 1.07;  7 0.93 0.95 / 0.98 1.02;  8 0.90 0.94 / 0.95 1.01
+//   Q4_0       4 1.14 1.19 / 1.10 1.33;  5 1.07 1.11 / 1.15 1.22;  6 1.02 1.05 / 1.04 1.16;  7 0.98 0.99 / 1.04 1.05;  8 0.99 1.00 / 1.03 1.08
+bool sgemm_rounds_ok(const nl_engine::Layer &L, const SgSplits &s, int n, bool prompt) {
+    const int rounds = sg_rounds(true, 1, s.qkv, L.qkv.ntiles, n) + sg_rounds(true, 2, s.gate, L.gate.ntiles, n) +
+                       sg_rounds(false, 1, s.wo, L.wo.ntiles, n) + sg_rounds(false, 1, s.down, L.down.ntiles, n);
+    return rounds <= (L.gate.wtype == WT_Q4_0 ? (prompt ? 8 : 6) : (prompt ? 6 : 5));
+}
+bool sgemm_step_ok(const nl_engine *e, const nl_engine::Batch &b, int n, bool prompt) {
+    const char *k = getenv("NL_SGEMM");                 // knob (tests, tools; read per step): 0 keeps qgemm_kernel's launches, 2 asks no rounds
     const nl_config &c = e->cfg;
-    if ((k && atoi(k) == 0) || c.qk_norm || e->Is % 32) return false;      // (QK-norm needs whole heads between the product and the rotation)
+    const int knob = k ? atoi(k) : 1;
+    if (knob == 0 || c.qk_norm || e->Is % 32) return false;      // (QK-norm needs whole heads between the product and the rotation)
     auto ok = [&](const PackedMat &m, bool norm, int rt, int ks) { return !pgemm_ok(m, n) && m.ntiles * TR == m.rows && sg_fits(norm, rt, m.cols, ks); };
-    for (const auto &L : e->layers)
-        if (L.up.wtype != L.gate.wtype || !ok(L.qkv, true, 1, sgemm_splits_qkv(b, L, n)) || !ok(L.gate, true, 2, sgemm_splits_gate(b, L, n)) ||
-            !ok(L.wo, false, 1, sgemm_splits(b, L.wo, 1, n, false)) || !ok(L.down, false, 1, sgemm_splits(b, L.down, 1, n, false)))
+    for (const auto &L : e->layers) {
+        const SgSplits s = sgemm_splits(b, L, n);
+        if (L.up.wtype != L.gate.wtype || !ok(L.qkv, true, 1, s.qkv) || !ok(L.gate, true, 2, s.gate) || !ok(L.wo, false, 1, s.wo) ||
+            !ok(L.down, false, 1, s.down) || (knob != 2 && !sgemm_rounds_ok(L, s, n, prompt)))
             return false;
+    }
     return true;
 }
 
@@ -2094,17 +2111,18 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                (exact || (fills(L.wo, 4) && fills(L.down, 4) && fills(L.qkv, QG_WAVES) && fills(L.gate, QG_FUSED_WAVES)));
     }
     if (dg) fold = true;
-    const bool sg = !dg && !fold && !exact && sgemm_step_ok(e, b, n);      // ... of the other formats and widths: nl_sgemm.h
+    const bool sg = !dg && !fold && !exact && sgemm_step_ok(e, b, n, one_stream);      // ... of the other formats and widths: nl_sgemm.h
     auto sg_params = [&](const PackedMat &m, int ks) {
         SGemmParams P{};
         P.q = m.q; P.s = m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles; P.n_tokens = n; P.ks = ks; P.eps = c.rms_eps;
         return P;
     };
-    auto sg_plain = [&](const PackedMat &m, const uint4 *in, const float *bias) {       // x += W . in (+ bias)
-        SGemmParams P = sg_params(m, sgemm_splits(b, m, 1, n, false));
+    auto sg_plain = [&](const PackedMat &m, int ks, const uint4 *in, const float *bias) {       // x += W . in (+ bias)
+        SGemmParams P = sg_params(m, ks);
         P.xf = in; P.out = b.x; P.bias = bias;
         return sg_launch<QG_EPI_PLAIN>(m.wtype, P, st);
     };
+    e->step_path = dg ? PATH_DGEMM : sg ? PATH_SGEMM : 0;
     const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
     // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs of Q4_0 files (pgemm_kernel) and the
     // prompt attention multiply only the fp16 hi half of every activation / probability -- half / a third of the matrix work,
@@ -2134,10 +2152,11 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         float *vc = e->vcache + (long long)l * e->kv_layer_stride;
         GemmOut qkv_out{nullptr, nullptr, 1, 0, nullptr};
         bool rope_in_attn = false;
+        const SgSplits sp = sg ? sgemm_splits(b, L, n) : SgSplits{};
         const bool folded_in = fold && l > 0;      // the previous layer's down GEMM wrote this layer's Q|K|V input
         if (!folded_in && !sg) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
         if (sg) {
-            SGemmParams P = sg_params(L.qkv, sgemm_splits_qkv(b, L, n));
+            SGemmParams P = sg_params(L.qkv, sp.qkv);
             P.x = b.x; P.normw = L.attn_norm;
             P.rope = QGemmParams::Rope{b.pos, b.stream, e->rope_cos, e->rope_sin, b.q, kc, vc, e->kv_stream_stride,
                                        L.bq, L.bk, L.bv, hd, e->Hs, e->KVs, c.seq_len, c.rope_conjugate, b.tcos, b.tsin, b.tkv};
@@ -2188,6 +2207,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 if (n_live > 0 && max_nparts == 1 && !kv16_on && !no_fin) {
                     T.fin_xf = b.xfrag; T.fin_nt16 = nt16; T.fin_form = form(L.wo);
                     merged = true;
+                    e->step_path |= PATH_TILE_FIN;
                 }
                 if (n_live > 0 && kv16_on) {
                     // every chunk the prompt can see, split into fp16 halves once for all the tiles that read it
@@ -2209,6 +2229,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 LCK(hd == 64 ? launch_attn_fin_hd<64>(e->gqa, P, dim3(e->KVs, 1, n), st)
                              : launch_attn_fin_hd<32>(e->gqa, P, dim3(e->KVs, 1, n), st));
                 merged = true;
+                e->step_path |= PATH_ATTN_FIN;
             } else {
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
@@ -2235,7 +2256,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             return launch_dgemm_plain(P, st);
         };
         if (sg) {
-            LCK(sg_plain(L.wo, b.xfrag, L.bo));
+            LCK(sg_plain(L.wo, sp.wo, b.xfrag, L.bo));
         } else if (fold && dg) {
             const QGemmParams::NormOut nout{L.ffn_norm, b.xfrag2, b.ssq, sB};
             LCK(dg_plain(L.wo, b.xfrag, L.bo, &nout));
@@ -2250,10 +2271,10 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             return e->fail(NL_ERR_UNSUPPORTED, "gate and up projections of different quantisation types");
         const uint4 *down_in = b.xfrag;
         if (sg) {
-            SGemmParams P = sg_params(L.gate, sgemm_splits_gate(b, L, n));
+            SGemmParams P = sg_params(L.gate, sp.gate);
             P.x = b.x; P.normw = L.ffn_norm; P.q1 = L.up.q; P.s1 = L.up.s; P.xf_out = b.xfrag2; P.out_form = form(L.down);
             LCK(sg_launch<QG_EPI_SWIGLU>(L.gate.wtype, P, st));
-            LCK(sg_plain(L.down, b.xfrag2, nullptr));
+            LCK(sg_plain(L.down, sp.down, b.xfrag2, nullptr));
             continue;
         }
         if (dg || exact || qgemm_swiglu_fits(L.gate, n)) {
@@ -3696,7 +3717,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
                 HIPCK(e, hipStreamWaitEvent(sb.st, e->sub_fork, 0));
                 hipGraphExec_t exec = nullptr;
                 for (auto &G : sb.graphs)
-                    if (G.n == m && G.nsplit == key_split) exec = G.exec;
+                    if (G.n == m && G.nsplit == key_split) { exec = G.exec; e->step_path = G.path; }
                 if (!exec && e->use_graph) {
                     // the step reads its tokens / positions / streams from the pinned block behind h_meta (a copy node of the
                     // graph), so one graph serves every step of m streams with as many position splits
@@ -3706,7 +3727,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
                         const int rc2 = batched_step(e, b, sb.st, m, 1);
                         const hipError_t ce = hipStreamEndCapture(sb.st, &gr);
                         if (!rc2 && ce == hipSuccess && gr && hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) == hipSuccess) {
-                            sb.graphs.push_back({m, key_split, gr, exec});
+                            sb.graphs.push_back({m, key_split, gr, exec, e->step_path});
                         } else {
                             if (gr) (void)hipGraphDestroy(gr);
                             (void)hipGetLastError();
@@ -3755,7 +3776,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
                 for (int i = 0; i < m; i++) nsplit = std::max(nsplit, pos[t0 + i] / ATT_CH + 1);
                 const int key_split = nsplit * 131072 + batch_knob_sig() % 131072;
                 for (auto &G : e->bt_graphs)
-                    if (G.n == m && G.nsplit == key_split) exec = G.exec;
+                    if (G.n == m && G.nsplit == key_split) { exec = G.exec; e->step_path = G.path; }
                 if (!exec) {
                     std::lock_guard<std::mutex> setup(g_setup_mu);      // (a capture must not overlap another thread's allocations)
                     hipGraph_t gr = nullptr;
@@ -3763,7 +3784,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
                         const int rc2 = batched_step(e, b, e->stream, m, 1);
                         const hipError_t ce = hipStreamEndCapture(e->stream, &gr);
                         if (!rc2 && ce == hipSuccess && gr && hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) == hipSuccess) {
-                            e->bt_graphs.push_back({m, key_split, gr, exec});
+                            e->bt_graphs.push_back({m, key_split, gr, exec, e->step_path});
                         } else {
                             if (gr) (void)hipGraphDestroy(gr);
                             exec = nullptr;
@@ -3914,6 +3935,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     const float *src = nullptr;
     int64_t n = 0;
     std::string w = which;
+    if (w == "step_path") { if (max_floats < 1) return 0; out[0] = (float)e->step_path; return 1; }      // (host state)
     if (w == "x") { src = e->x[0]; n = e->cfg.dim; }
     else if (w == "x1") { src = e->x[1]; n = e->cfg.dim; }
     else if (w == "q") { src = e->qbuf; n = (int64_t)e->Hs * e->hd; }

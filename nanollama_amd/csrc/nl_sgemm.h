@@ -395,6 +395,11 @@ inline int sg_tw(bool norm, int mats, int ks, int ntiles, int n_tokens) {
     while ((tw + 1) * mats * ks <= SG_WAVES && (long long)((ntiles + tw - 1) / tw) * ((n_tokens + 15) / 16) > SG_ROUND) tw++;
     return tw;
 }
+// rounds of workgroups of a launch, one a compute unit (their registers or LDS leave room for no second one where it matters)
+inline int sg_rounds(bool norm, int mats, int ks, int ntiles, int n_tokens) {
+    const int tw = sg_tw(norm, mats, ks, ntiles, n_tokens);
+    return (int)(((long long)((ntiles + tw - 1) / tw) * ((n_tokens + 15) / 16) + SG_ROUND - 1) / SG_ROUND);
+}
 inline int sg_waves(bool norm, int mats, int ks, int tw) { return !norm ? ks : ks * mats * tw <= 8 ? 8 : SG_WAVES; }
 inline bool sg_fits(bool norm, int mats, int cols, int ks) {
     if (cols % 32 || cols < 32 || ks < 1 || ks * mats > (norm ? SG_WAVES : 16) || (ks & (ks - 1)) || sg_cps(cols, ks) > 6) return false;

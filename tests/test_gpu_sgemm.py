@@ -84,3 +84,23 @@ def test_short_steps_match_the_oracle(hip, tmp_path, wtype):
     m.prefill(toks)
     assert float(np.abs(m.state.logits - want).max()) <= 1e-4 * max(1.0, float(want.std()))
     m.close()
+
+
+# steps of four to eight rounds of workgroups, either side of the limits: sgemm_kernel up to the last of them
+@pytest.mark.parametrize("dim,heads,kvs,interm,wtype,stream_steps,prompts", [
+    (1600, 25, 25, 4288, "q8_0", {17: True, 48: True, 49: False, 64: False}, {48: True, 49: False}),
+    (1600, 25, 25, 4288, "q4_0", {48: True, 49: False}, {49: True, 64: True}),
+    (2112, 33, 11, 5632, "f16", {17: True, 33: False, 64: False}, {33: True, 49: False})])
+def test_steps_of_many_rounds_keep_the_split_k_launches(hip, tmp_path, dim, heads, kvs, interm, wtype, stream_steps, prompts):
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("sg_r", 1, dim, heads, kvs, 64, seq_len=96, interm=interm), wtype, 5)
+    m = hip.load_llama_model(gguf.load_gguf(str(p)), max_streams=64)
+    path = lambda: int(m.debug_read("step_path", 1)[0]) & 2 != 0
+    for n, short in prompts.items():
+        m.prefill([5] * n, 0, 0)
+        assert path() == short, (n, "prompt")
+    m.reset()
+    for n, short in stream_steps.items():
+        m.forward_batch(list(range(n)), [7] * n, [0] * n)
+        assert path() == short, (n, "streams")
+    m.close()
