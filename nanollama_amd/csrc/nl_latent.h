@@ -395,17 +395,7 @@ __global__ void __launch_bounds__(256) latent_out_kernel(LatentParams P, int n_t
         for (int i = 0; i < NK; i++)
             if (w + 4 * i < kvt) a[i] = W[((long long)min(r0 + r, P.tph - 1) * kvt + w + 4 * i) * 64];
     };
-    // trips to memory bound the launch: the splits' values, their (max, sum), the weights and the gate are requested together (us a step, after
-    // one another and together: 28 layers of 1536 columns, 8 streams 1733, 1703; 20 of 768, 1 stream 699, 698, 24 streams 1275, 1256)
-    const int nv = nt * kvt * 8;
-    f32x4 x[8];
-    auto values = [&](int i, int s0) {
-        const int t = i / (kvt * 8), d = (i - t * kvt * 8) * 4;
-        const float *p = P.part + ((long long)(n0 + t) * P.heads + h) * ns * kvt * 32 + d;
-#pragma unroll
-        for (int s = 0; s < 8; s++) x[s] = *reinterpret_cast<const f32x4 *>(p + (long long)min(s0 + s, ns - 1) * kvt * 32);
-    };
-    const float gate = P.off_g >= 0 ? P.proj[(long long)(n0 + min(c, nt - 1)) * P.ldp + P.off_g + h] : 0.f;
+    load(0);
     float *wt = reinterpret_cast<float *>(lds);            // [16][ns]
     T *xs = reinterpret_cast<T *>(lds + ((16 * ns * 4 + 15) & ~15));        // [kvt][4][16 tokens][8]
     f32x4 *red = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(xs) + kvt * OPT * sizeof(T));    // [4][RB][64]
@@ -413,33 +403,26 @@ __global__ void __launch_bounds__(256) latent_out_kernel(LatentParams P, int n_t
         const int t = tid >> 4, j = tid & 15;
         const float sk = P.sink ? P.sink[h] * LOG2E : -INFINITY;
         const float *ml = P.ml + ((long long)(n0 + min(t, nt - 1)) * P.heads + h) * ns * 2;
-        float mm, den = 0.f;
-        float2 s0 = {-INFINITY, 0.f}, s1 = s0;
-        if (j < ns) s0 = *reinterpret_cast<const float2 *>(ml + j * 2);
-        if (j + 16 < ns) s1 = *reinterpret_cast<const float2 *>(ml + (j + 16) * 2);
-        load(0);
-        if (tid < nv) values(tid, 0);
-        mm = fmaxf(s0.x, s1.x);
-        for (int s = j + 32; s < ns; s += 16) mm = fmaxf(mm, ml[s * 2]);     // (more only beside layers of other kinds)
+        float mm = -INFINITY, den = 0.f;
+        for (int s = j; s < ns; s += 16) mm = fmaxf(mm, ml[s * 2]);
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) mm = fmaxf(mm, __shfl_xor(mm, o));
         mm = fmaxf(mm, sk);
-        if (j < ns) den += s0.y * exp2_f32(s0.x - mm);
-        if (j + 16 < ns) den += s1.y * exp2_f32(s1.x - mm);
-        for (int s = j + 32; s < ns; s += 16) den += ml[s * 2 + 1] * exp2_f32(ml[s * 2] - mm);
+        for (int s = j; s < ns; s += 16) den += ml[s * 2 + 1] * exp2_f32(ml[s * 2] - mm);
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) den += __shfl_xor(den, o);
         const float inv = 1.f / (den + exp2_f32(sk - mm));
-        if (j < ns) wt[t * ns + j] = exp2_f32(s0.x - mm) * inv;
-        if (j + 16 < ns) wt[t * ns + j + 16] = exp2_f32(s1.x - mm) * inv;
-        for (int s = j + 32; s < ns; s += 16) wt[t * ns + s] = exp2_f32(ml[s * 2] - mm) * inv;
+        for (int s = j; s < ns; s += 16) wt[t * ns + s] = exp2_f32(ml[s * 2] - mm) * inv;
     }
     lds_barrier();
-    for (int i = tid; i < nv; i += 256) {
+    for (int i = tid; i < nt * kvt * 8; i += 256) {
         const int t = i / (kvt * 8), d = (i - t * kvt * 8) * 4;
+        const float *p = P.part + ((long long)(n0 + t) * P.heads + h) * ns * kvt * 32 + d;
         f32x4 v = {};
         for (int s0 = 0; s0 < ns; s0 += 8) {
-            if (i != tid || s0) values(i, s0);
+            f32x4 x[8];
+#pragma unroll
+            for (int s = 0; s < 8; s++) x[s] = *reinterpret_cast<const f32x4 *>(p + (long long)min(s0 + s, ns - 1) * kvt * 32);
 #pragma unroll
             for (int s = 0; s < 8; s++)
                 if (s0 + s < ns) {
@@ -470,7 +453,7 @@ __global__ void __launch_bounds__(256) latent_out_kernel(LatentParams P, int n_t
         const int r = i >> 6, l = i & 63, tok = n0 + (l & 15), d = (r0 + r) * 16 + 4 * (l >> 4), k = h * P.dv + d;
         if ((l & 15) >= nt || r0 + r >= P.tph) continue;
         f32x4 v = red[r * 64 + l] + red[(RB + r) * 64 + l] + red[(2 * RB + r) * 64 + l] + red[(3 * RB + r) * 64 + l];
-        if (P.off_g >= 0) v *= sigmoid_f32(gate);          // (lane l & 15 is this thread's c)
+        if (P.off_g >= 0) v *= sigmoid_f32(P.proj[(long long)tok * P.ldp + P.off_g + h]);
         T *y = reinterpret_cast<T *>(P.y);
         if (d + 3 < P.dv && (k & 3) == 0) put4(y + op_index(tok, k, P.y_nks), v);
         else
