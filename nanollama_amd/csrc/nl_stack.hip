@@ -114,7 +114,8 @@ struct nl_engine {
     int ids_cap = 1024;
     float *h_logits = nullptr;
     std::vector<int> next_pos;   // per stream: the position its next token must have (or 0)
-    struct Graph { hipGraph_t g; hipGraphExec_t x; };
+    int one_query = 0;           // layers of the last launch sequence whose queries took one launch (nl_debug_read "one_query")
+    struct Graph { hipGraph_t g; hipGraphExec_t x; int one_query; };
     std::map<std::tuple<int, int, int>, Graph> graphs;
     SampScratch sp;
     int sp_cap = 0;
@@ -435,7 +436,9 @@ hipError_t logits_launch(nl_engine *e, const int *rows, int n, float *out) {
 
 // do a decode step's queries take one launch?  Wherever the kernel can hold them: us a step as two launches and as one, positions around 260,
 // 20 layers of 768 columns, 1 / 2 / 4 streams: 732 / 823 / 907, 691 / 783 / 861; 28 of 1536: 1230 / 1349 / 1491, 1160 / 1307 / 1446.  It
-// recomputes a head's queries per 128 latent columns, which 32-bit weights would double: those keep two launches.
+// recomputes a head's queries per 128 latent columns, and still wins where that is six times (6 layers, 1 / 4 streams: 64 heads of 128, latents of 704,
+// 302 / 355 and 279 / 326; 3 heads 190 / 224 and 180 / 212; 128 heads of 64, latents of 512, 311 / 364 and 258 / 301).  32-bit weights would double the
+// recomputation: those keep two launches.
 template <typename T>
 bool one_query_launch(int n, const Layer &L) {
     return std::is_same_v<T, bf16> && few_norm_ok(n, L.uq.nks, L.d.latent.q_rank, L.proj.rows) && latent_query_ok(n, L.uq.nks, L.dimp);
@@ -466,6 +469,7 @@ hipError_t latent_mixer(nl_engine *e, const StepIn &s, const Run &R, const Layer
             LatentQueryParams Q{};
             Q.W1 = L.uq.w; Q.W2 = L.ukt.w; Q.nx = e->proj + L.tdq; Q.nw = L.dqnorm; Q.nks = L.uq.nks; Q.n = s.n; Q.ndim = N.q_rank; Q.nld = L.proj.rows;
             Q.heads = N.heads; Q.dt = L.dimp / 16; Q.nrot = L.uq.nrt - N.heads * Q.dt; Q.w2t = L.kvt * 2; Q.chunks = (Q.w2t + 7) / 8; Q.eps = e->c.eps; Q.hd = H;
+            e->one_query++;
             if ((rc = launch_latent_query(Q, store, st)) || (rc = launch_latent_decode<T>(A, s.n, st))) return rc;
             return launch_latent_out<T>(A, s.n, st);
         }
@@ -515,6 +519,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
     e->xcur = e->x;
     e->pend = nullptr;
     e->folded = false;
+    e->one_query = 0;
     E.table = e->embed.w; E.tok = s.tok; E.nks = e->nksd; E.dim = D; E.scale = e->c.embed_scale; E.x = e->x; E.x0 = e->x0;
     hipLaunchKernelGGL(lookup_kernel<T>, dim3(s.n), dim3(256), 0, st, E);
     for (size_t r = 0; r < e->runs.size(); r++) {
@@ -639,15 +644,17 @@ int queue_decode(nl_engine *e, int kind, int n, int max_pos, int steps = 1) {
     const auto key = std::make_tuple(n, nsplit, kind * 64 + steps);
     auto it = e->graphs.find(key);
     if (it == e->graphs.end()) {
-        nl_engine::Graph G{nullptr, nullptr};
+        nl_engine::Graph G{nullptr, nullptr, 0};
         HIPCK(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         const int rc = body();
         const hipError_t ce = hipStreamEndCapture(e->stream, &G.g);
         if (rc) { if (G.g) (void)hipGraphDestroy(G.g); return rc; }
         if (ce != hipSuccess || !G.g) return e->fail(NL_ERR_HIP, "graph capture: %s", hipGetErrorString(ce));
         HIPCK(e, hipGraphInstantiate(&G.x, G.g, nullptr, nullptr, 0));
+        G.one_query = e->one_query;
         it = e->graphs.emplace(key, G).first;
     }
+    e->one_query = it->second.one_query;
     HIPCK(e, hipGraphLaunch(it->second.x, e->stream));
     return NL_OK;
 }
@@ -1396,6 +1403,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     }
     const float *src = nullptr;
     int64_t n = 0;
+    if (!strcmp(which, "one_query")) { if (max_floats < 1) return 0; out[0] = (float)e->one_query; return 1; }      // (host state)
     if (!strcmp(which, "x")) { src = e->xcur ? e->xcur : e->x; n = e->c.dim; }
     else if (!strcmp(which, "logits")) { src = e->logits; n = e->c.vocab; }
     else if (!strncmp(which, "state", 5)) {              // "state<run>": the recurrent state of a layer run

@@ -30,10 +30,10 @@ def test_one_run_gives_the_bits_of_partials_and_merge(tmp_path, monkeypatch, hea
             m.reset(0)
             m.reset(1)
             rows = []
-            m.prefill(toks[:n], 0, 1)
-            rows.append(m.state.logits.copy())
-            m.prefill(toks[n:n + 11], n, 1)              # behind a context, across position 128 too
-            rows.append(m.state.logits.copy())
+            for at, to in ((0, n), (n, n + 11)):         # the second behind a context, across position 128 too
+                m.prefill(toks[at:to], at, 1)
+                rows.append(m.state.logits.copy())
+                assert int(m.debug_read("step_path", 1)[0]) & 4 == (4 if to <= 128 and not knob else 0), (at, to, knob)
             got[knob] = rows
         for a, b in zip(got[False], got[True]):
             assert np.isfinite(a).all() and np.array_equal(a, b), (n, float(np.abs(a - b).max()))

@@ -557,10 +557,12 @@ def test_many_streams_in_one_decode_batch(n, dtype):
 
 # ---- the programs ---------------------------------------------------------------------------------------------------------------
 
-# the queries of up to four tokens in one launch: either side of its bounds (heads of 128, latents of 768), more units than XCDs, ragged chunks
-@pytest.mark.parametrize("heads,dim,rot,kv_rank,q_rank", [(1, 32, 2, 24, 4), (6, 128, 64, 256, 384), (9, 100, 64, 300, 512), (9, 20, 34, 40, 516),
-                                                          (17, 33, 8, 130, 768), (2, 128, 32, 64, 772), (2, 130, 32, 64, 40), (3, 64, 16, 136, 42)])
-def test_queries_of_few_tokens(heads, dim, rot, kv_rank, q_rank):
+# the queries of up to four tokens in one launch: either side of its bounds (heads of 128, latents of 768, whole float4s), more units than
+# XCDs, ragged chunks, six of them
+@pytest.mark.parametrize("heads,dim,rot,kv_rank,q_rank,one", [(1, 32, 2, 24, 4, True), (6, 128, 64, 256, 384, True), (9, 100, 64, 300, 512, True), (9, 20, 34, 40, 516, True),
+                                                              (17, 33, 8, 130, 768, True), (3, 96, 32, 720, 64, True), (2, 128, 32, 64, 772, False), (2, 130, 32, 64, 40, False),
+                                                              (3, 64, 16, 136, 42, False)])
+def test_queries_of_few_tokens(heads, dim, rot, kv_rank, q_rank, one):
     cfg = lconfig([lat(2, heads=heads, dim=dim, rot=rot, kv_rank=kv_rank, q_rank=q_rank, ff=40), lat(3, heads=heads, dim=dim, rot=rot, kv_rank=kv_rank, q_rank=q_rank)])
     w = weights(cfg, 8)
     fl = floats(w)
@@ -572,6 +574,7 @@ def test_queries_of_few_tokens(heads, dim, rot, kv_rank, q_rank):
     for n in range(1, 6):                      # 1, 2 .. 5 tokens beside each other; the streams from n on stay where they are
         at = [len(s) - 5 + (n - 1 - i) for i, s in enumerate(seqs[:n])]
         _, lg = m.forward_batch(list(range(n)), [s[p] for s, p in zip(seqs, at)], at, want_logits=True)
+        assert m.debug_read("one_query", 1)[0] == (2 if one and n <= 4 else 0), n
         for i in range(n):
             assert rel(lg[i], want[i][at[i]]) < bound("bfloat16", cfg, fl, seqs[i], want[i]), (n, i)
 

@@ -20,6 +20,7 @@ out = {}
 for n in (8, 40, 127):
     dev.reset()
     dev.prefill(synth.prompt_ids(n, 2048, seed=n))
+    assert int(dev.debug_read("step_path", 1)[0]) & 8 == 0
     out[f"logits{n}"] = dev.state.logits.copy()
     u = np.random.default_rng(n).random(24, dtype=np.float32)
     out[f"ids{n}"], _ = dev.sample_decode(n, 24, temperature=0.8, top_p=0.9, top_k=50, rep_penalty=1.15, rep_window=64, uniforms=u, recent=[])
@@ -31,7 +32,8 @@ dev.close()
 @pytest.mark.parametrize("wtype", ["q8_0", "q4_0"])
 def test_short_prompts_run_the_tiled_attention(tmp_path, wtype):
     # A sampled reply hangs on the last bits of its prompt (a pick that flips changes all that follow), so a prompt's attention must not depend
-    # on where it ends: the kernel that finishes one-split rows of decode batches (NL_NO_ATTN_FIN=1: off, read once per process) stays out of it.
+    # on where it ends: the kernel that finishes one-split rows of decode batches stays out of it.  NL_NO_ATTN_FIN=1 switches that one off, and makes
+    # the tiled kernel leave partials to a merge launch, which are the same bits.
     p = tmp_path / "m.gguf"
     synth.generate_gguf(str(p), synth.ModelShape("short", 4, 576, 9, 3, 2048, seq_len=256, interm=1536), wtype, 71)
     runs = []
