@@ -381,48 +381,71 @@ hipError_t launch_latent_decode(const LatentParams &P, int n, hipStream_t st) {
     return go(latent_decode_kernel<T, 12>);
 }
 
-// grid (row tiles of Uv / RB, token tiles): merges the splits of one head for 16 tokens, multiplies, gates, stores y's columns
-template <typename T, int RB>
+// grid (row tiles of Uv / RB, token tiles): merges the splits of one head for 16 tokens, multiplies, gates, stores y's columns.
+// Trips to memory bound the launch: the (max, sum) of the splits, the weights, the splits' values and the gate are requested together, every one
+// under a clamped index instead of a branch -- behind a branch the compiler no longer knows how many loads are in flight, and the weights of the
+// splits then wait for all of them.  us a step, one load after another / together behind branches / this, positions around 260: 20 layers of 768
+// columns, 1 / 8 / 48 streams 681 / 952 / 1184, 684 / 948 / 1178, 669 / 934 / 1173; 28 of 1536: 1136 / 1585 / 1963, 1133 / 1580 / 1969, 1116 / 1558 / 1944.
+// NK by the latents' size: with the most k tiles for all, the loads past the last one would be half of them or more.
+template <typename T, int RB, int NK>        // NK: k tiles of a wavefront
 __global__ void __launch_bounds__(256) latent_out_kernel(LatentParams P, int n_tokens) {
-    constexpr int NK = LT_MAX_TILES / 4;
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15, kvt = P.kvt, ns = P.nsplit;
     const int per = (P.tph + RB - 1) / RB, h = blockIdx.x / per, r0 = (blockIdx.x - h * per) * RB, n0 = blockIdx.y * 16, nt = min(16, n_tokens - n0);
     const Frag<T> *W = reinterpret_cast<const Frag<T> *>(P.W) + (long long)(h * P.tph) * kvt * 64 + lane;
     Frag<T> a[NK];
-    auto load = [&](int r) {                               // (row tiles past the head's end repeat its last one)
+    auto load = [&](int r) {                               // (row tiles past the head's end and k tiles past the last repeat it)
 #pragma unroll
-        for (int i = 0; i < NK; i++)
-            if (w + 4 * i < kvt) a[i] = W[((long long)min(r0 + r, P.tph - 1) * kvt + w + 4 * i) * 64];
+        for (int i = 0; i < NK; i++) a[i] = W[((long long)min(r0 + r, P.tph - 1) * kvt + min(w + 4 * i, kvt - 1)) * 64];
     };
-    load(0);
+    const int nv = nt * kvt * 8, row = kvt * 32;
+    f32x4 x[8];
+    auto values = [&](const float *p, int s0) {
+#pragma unroll
+        for (int s = 0; s < 8; s++) x[s] = *reinterpret_cast<const f32x4 *>(p + (long long)min(s0 + s, ns - 1) * row);
+    };
+    auto from = [&](int i, int &t, int &d) {               // value i: its token and columns
+        t = i / (kvt * 8); d = (i - t * kvt * 8) * 4;
+        return P.part + ((long long)(n0 + t) * P.heads + h) * ns * row + d;
+    };
+    const float *gp = P.proj + (P.off_g >= 0 ? (long long)(n0 + min(c, nt - 1)) * P.ldp + P.off_g + h : 0);
     float *wt = reinterpret_cast<float *>(lds);            // [16][ns]
     T *xs = reinterpret_cast<T *>(lds + ((16 * ns * 4 + 15) & ~15));        // [kvt][4][16 tokens][8]
     f32x4 *red = reinterpret_cast<f32x4 *>(reinterpret_cast<char *>(xs) + kvt * OPT * sizeof(T));    // [4][RB][64]
+    float gate;
     {
         const int t = tid >> 4, j = tid & 15;
         const float sk = P.sink ? P.sink[h] * LOG2E : -INFINITY;
         const float *ml = P.ml + ((long long)(n0 + min(t, nt - 1)) * P.heads + h) * ns * 2;
-        float mm = -INFINITY, den = 0.f;
-        for (int s = j; s < ns; s += 16) mm = fmaxf(mm, ml[s * 2]);
+        float2 s0 = *reinterpret_cast<const float2 *>(ml + min(j, ns - 1) * 2), s1 = *reinterpret_cast<const float2 *>(ml + min(j + 16, ns - 1) * 2);
+        load(0);
+        int vt, vd;
+        values(from(min(tid, nv - 1), vt, vd), 0);
+        gate = *gp;
+        if (j >= ns) s0.x = -INFINITY;
+        if (j + 16 >= ns) s1.x = -INFINITY;
+        float mm = fmaxf(s0.x, s1.x), den = 0.f;
+        for (int s = j + 32; s < ns; s += 16) mm = fmaxf(mm, ml[s * 2]);     // (more only beside layers of other kinds)
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) mm = fmaxf(mm, __shfl_xor(mm, o));
         mm = fmaxf(mm, sk);
-        for (int s = j; s < ns; s += 16) den += ml[s * 2 + 1] * exp2_f32(ml[s * 2] - mm);
+        if (j < ns) den += s0.y * exp2_f32(s0.x - mm);
+        if (j + 16 < ns) den += s1.y * exp2_f32(s1.x - mm);
+        for (int s = j + 32; s < ns; s += 16) den += ml[s * 2 + 1] * exp2_f32(ml[s * 2] - mm);
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) den += __shfl_xor(den, o);
         const float inv = 1.f / (den + exp2_f32(sk - mm));
-        for (int s = j; s < ns; s += 16) wt[t * ns + s] = exp2_f32(ml[s * 2] - mm) * inv;
+        if (j < ns) wt[t * ns + j] = exp2_f32(s0.x - mm) * inv;
+        if (j + 16 < ns) wt[t * ns + j + 16] = exp2_f32(s1.x - mm) * inv;
+        for (int s = j + 32; s < ns; s += 16) wt[t * ns + s] = exp2_f32(ml[s * 2] - mm) * inv;
     }
     lds_barrier();
-    for (int i = tid; i < nt * kvt * 8; i += 256) {
-        const int t = i / (kvt * 8), d = (i - t * kvt * 8) * 4;
-        const float *p = P.part + ((long long)(n0 + t) * P.heads + h) * ns * kvt * 32 + d;
+    for (int i = tid; i < nv; i += 256) {
+        int t, d;
+        const float *p = from(i, t, d);
         f32x4 v = {};
         for (int s0 = 0; s0 < ns; s0 += 8) {
-            f32x4 x[8];
-#pragma unroll
-            for (int s = 0; s < 8; s++) x[s] = *reinterpret_cast<const f32x4 *>(p + (long long)min(s0 + s, ns - 1) * kvt * 32);
+            if (i != tid || s0) values(p, s0);
 #pragma unroll
             for (int s = 0; s < 8; s++)
                 if (s0 + s < ns) {
@@ -453,7 +476,7 @@ __global__ void __launch_bounds__(256) latent_out_kernel(LatentParams P, int n_t
         const int r = i >> 6, l = i & 63, tok = n0 + (l & 15), d = (r0 + r) * 16 + 4 * (l >> 4), k = h * P.dv + d;
         if ((l & 15) >= nt || r0 + r >= P.tph) continue;
         f32x4 v = red[r * 64 + l] + red[(RB + r) * 64 + l] + red[(2 * RB + r) * 64 + l] + red[(3 * RB + r) * 64 + l];
-        if (P.off_g >= 0) v *= sigmoid_f32(P.proj[(long long)tok * P.ldp + P.off_g + h]);
+        if (P.off_g >= 0) v *= sigmoid_f32(gate);          // (lane l & 15 is this thread's c)
         T *y = reinterpret_cast<T *>(P.y);
         if (d + 3 < P.dv && (k & 3) == 0) put4(y + op_index(tok, k, P.y_nks), v);
         else
@@ -473,7 +496,10 @@ hipError_t launch_latent_out(const LatentParams &P, int n, hipStream_t st) {
         return hipGetLastError();
     };
     // few tokens: a row tile per workgroup; many: the merged head serves several of them
-    return P.tph >= 2 && P.heads * ((P.tph + 3) / 4) * tt >= 128 ? go(latent_out_kernel<T, 4>, 4) : go(latent_out_kernel<T, 1>, 1);
+    const bool four = P.tph >= 2 && P.heads * ((P.tph + 3) / 4) * tt >= 128;
+    if (P.kvt <= 8) return four ? go(latent_out_kernel<T, 4, 2>, 4) : go(latent_out_kernel<T, 1, 2>, 1);
+    if (P.kvt <= 16) return four ? go(latent_out_kernel<T, 4, 4>, 4) : go(latent_out_kernel<T, 1, 4>, 1);
+    return four ? go(latent_out_kernel<T, 4, 6>, 4) : go(latent_out_kernel<T, 1, 6>, 1);
 }
 
 }  // namespace nl

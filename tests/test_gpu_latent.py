@@ -555,6 +555,30 @@ def test_many_streams_in_one_decode_batch(n, dtype):
     m.close()
 
 
+# the output launch either side of its k tiles a wavefront, of 8, 16 and 24 latents' tiles; one and four row tiles a workgroup (64 heads, 17 tokens);
+# 1 to 32 splits, ragged rows and latents, a sink and a gate
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,vdim,kv_rank", [(2, 16, 32), (64, 24, 256), (3, 40, 260), (64, 32, 512), (2, 24, 516), (64, 32, 700)])
+def test_output_launch(heads, vdim, kv_rank, dtype):
+    cfg = lconfig([lat(3, heads=heads, dim=16, rot=8, vdim=vdim, kv_rank=kv_rank, q_rank=24), lat(2, heads=heads, dim=16, rot=8, vdim=vdim, kv_rank=kv_rank, q_rank=24)])
+    w = weights(cfg, 13)
+    fl = floats(w)
+    m = load(cfg, w, dtype, max_streams=17, seq_len=1024)
+    seqs = [tokens(1003 if i == 2 else 5 + 29 * i, seed=20 + i) for i in range(17)]
+    check = (0, 2, 16)
+    want = {i: so.forward(cfg, fl, seqs[i]) for i in check}
+    m.step([(i, s[:-2], 0, []) for i, s in enumerate(seqs)])
+    one = m.step([(2, seqs[2][-2:-1], 1001, [0])])
+    assert rel(one[0], want[2][-2]) < bound(dtype, cfg, fl, seqs[2], want[2])
+    for k in (2, 1):
+        at = [i for i in range(17) if k == 1 or i != 2]
+        out = dict(zip(at, m.step([(i, [seqs[i][-k]], len(seqs[i]) - k, [0]) for i in at])))
+        for i in check:
+            if i in out:
+                assert rel(out[i], want[i][-k]) < bound(dtype, cfg, fl, seqs[i], want[i]), (i, k)
+    m.close()
+
+
 # ---- the programs ---------------------------------------------------------------------------------------------------------------
 
 # the queries of up to four tokens in one launch: either side of its bounds (heads of 128, latents of 768, whole float4s), more units than
