@@ -88,11 +88,10 @@ __device__ unsigned g_dg_log_n;
 #define DG_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
 
 typedef unsigned dg_u32x4 __attribute__((ext_vector_type(4)));
-// 1 / sqrt(ss / dim + eps) as float32 (go/quant.go:597-607 computes it in float64): v_rsq_f64 + two Newton steps -- relative error
-// < 1e-30 before the rounding to float32, the same float32 as the IEEE divide and square root give except at rounding boundaries of
-// measure zero -- instead of sixty dependent float64 instructions behind the last product of the launch (nl_persist.h pd_inv_rms)
-__device__ __forceinline__ float dg_inv_rms(double ss, int dim, float eps) {
-    const double rdim = 1.0 / (double)dim;                 // (independent of ss: off the critical path)
+// 1 / sqrt(ss / dim + eps) as float32 (go/quant.go:597-607 computes it in float64): v_rsq_f64 + two Newton steps -- a few float64
+// ulps off before the rounding to float32, so the same float32 as the IEEE divide and square root give unless that lies as close to a rounding
+// boundary -- instead of sixty dependent float64 instructions behind the last product of the launch (nl_persist.h pd_inv_rms)
+__device__ __forceinline__ float dg_inv_rms(double ss, double rdim, float eps) {      // rdim: 1 / columns
     const double m = fma(ss, rdim, (double)eps);
     double y = __builtin_amdgcn_rsq(m);
     y = y * fma(-0.5 * m * y, y, 1.5);
@@ -316,7 +315,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) dgemm_kernel(QGemmParams P)
             const double lo2 = (lq & 1) ? t1 + tot : tot + t1;          // (lq 0 + lq 1) resp. (lq 2 + lq 3), same order in both lanes
             const double t2 = __shfl_xor(lo2, 32);
             tot = (lq & 2) ? t2 + lo2 : lo2 + t2;
-            inv = dg_inv_rms(tot, P.nrm_in.dim, P.nrm_in.eps);
+            inv = dg_inv_rms(tot, 1.0 / (double)P.nrm_in.dim, P.nrm_in.eps);
             if (P.nrm_in.scale) {     // the producer's power-of-two pre-scale (norm_prescale, nl_qgemm.h): undone exactly
                 if (rg == 0 && wv == 0 && lq == 0 && live) P.nrm_in.scale_next[n] = norm_prescale(inv);
                 inv *= 1.0f / nsc;
@@ -658,7 +657,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) dghead_kernel(QGemmParams P
             const double lo2 = (lq & 1) ? t1 + tot : tot + t1;
             const double t2 = __shfl_xor(lo2, 32);
             tot = (lq & 2) ? t2 + lo2 : lo2 + t2;
-            inv = dg_inv_rms(tot, P.nrm_in.dim, P.nrm_in.eps);
+            inv = dg_inv_rms(tot, 1.0 / (double)P.nrm_in.dim, P.nrm_in.eps);
             if (P.nrm_in.scale) {
                 float nsc;
                 asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(nsc) : "v"(dg_lds_addr(lds_all + DG_SSQ_BYTES / 16) + (unsigned)li * 4u) : "memory");

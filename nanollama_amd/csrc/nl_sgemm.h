@@ -4,20 +4,21 @@
 // What bounds such a step is the number of its launches: 24 tokens against 89M Q8_0 parameters move 75 MB and were 10 launches a layer of 3 - 8 us
 // (norm, Q|K|V in split-K slabs, slab sum + rotation, attention, merge, WO in slabs, slab sum + norm, gate || up in slabs, slab sum + SiLU,
 // down in slabs).  Here the K splits of a tile are wavefronts of ONE workgroup, so their partial tiles meet in LDS and the rotation, SiLU and
-// residual epilogues follow in the same launch; the norm is the prologue of the launch that consumes it: 6 launches a layer, 5 for decode
-// batches.  Measured (profiled, us a launch, before: a norm, a GEMM in slabs
-// and what sums them; now): 89M Q8_0, 24 tokens, Q|K|V 3.5 + 4.7 + 4.6, now 5.0; gate || up 3.5 + 4.8 + 4.0, now 5.2; WO 4.6, now 3.6; a prompt of 24 / 64 tokens
-// (its attention in one launch a layer as well, nl_batch.h) 703 -> 409 / 774 -> 434 us, 173M Q8_0 1092 -> 641 / 1227 -> 711, 841M 1766 -> 1255 / 2026 -> 1552,
-// F16 1831 -> 1394 / 2074 -> 1742; a step of 64 streams
-// at position 150: 89M 785 -> 604, 173M 1105 -> 823, 841M Q8_0 1923 -> 1750, F16 1968 -> 1934.  What bounds a launch now is one workgroup's chain: requests,
-// the norm (2.2 of 5.0 us), products at the vector pipe's rate (10 instructions an expansion, 4 a scaling), the meeting of the partial tiles.
+// residual epilogues follow in the same launch; the norm is the prologue of the launch that consumes it: 5 launches a layer, 6 where the
+// attention leaves partials (positions of 128 on).  Measured, profiled, us a launch -- a norm, a GEMM in slabs and what sums them; this kernel --, 89M
+// Q8_0, 24 tokens: Q|K|V 3.5 + 4.7 + 4.6, 5.5; gate || up 3.5 + 4.8 + 4.0, 5.8; WO and down (mean) 4.6, 4.4.  A prompt of 24 / 64 tokens
+// (its attention in one launch a layer as well, nl_batch.h) 703 -> 394 / 774 -> 434 us, 173M Q8_0 1092 -> 641 / 1227 -> 711, 841M 1766 -> 1255 / 2026 -> 1552,
+// F16 1831 -> 1394 / 2074 -> 1742; a step of 64 streams at position 150: 89M 785 -> 604, 173M 1105 -> 823, 841M Q8_0 1923 -> 1750, F16 1968 -> 1934.
+// What bounds a launch now is one workgroup's chain: requests, the norm (almost half of two launches), products at the vector pipe's rate
+// (10 instructions an expansion, 4 a scaling), the meeting of the partial tiles.
 //
 // A workgroup owns 16 tokens x TW (x 2: gate and up) 16-row weight tiles; its KS x TW wavefronts are (split z, tile).  Split z multiplies the
 // 128-column chunks z, z + KS, ... in order, exactly those that a split of qgemm_kernel takes (KS is qgemm_kernel's rule too), and the
-// partial tiles are added in split order as the slabs' consumers add them: the results are the same bits, so a sampled reply does not
-// depend on which of the two kernels its prompt ran on.
+// partial tiles are added in split order as the slabs' consumers add them, so the products are qgemm_kernel's bits.  The norm's factor is
+// bnorm_kernel's to a few float64 ulps (its sum in another order, a reciprocal and Newton steps instead of a division and a square root), and
+// the same float32 unless it lies that close to a rounding boundary, about one row in 10^8: none was seen.
 //   * The weights of the first chunks (all of them where registers allow) are requested in the prologue, in front of the norm's round trip.
-//   * NORM: the token tile's rows go to LDS once per workgroup as the fragments of all its wavefronts (16 x 2048 columns fit), through the
+//   * NORM: the token tile's rows go to LDS once per workgroup as the fragments of all its wavefronts (up to 2112 columns fit), through the
 //     same rounding as bnorm_kernel: 1 / rms is known before anything is rounded, so no range is lost.
 //   * otherwise the fragments are read straight into registers, a chunk ring of DEP deep.
 //   * Barriers order LDS only (pg_barrier): the weights in flight stay in flight.
@@ -47,10 +48,9 @@ inline size_t sg_lds_bytes(bool norm, int cols, int waves, int tpl) {
     return (norm ? (size_t)(cols / 32) * 2048 + (size_t)cols * 4 + (size_t)waves * 128 : 0) + (size_t)waves * tpl * 1024;
 }
 
-// Raw buffer loads: one SGPR base, 32-bit offsets.  (Skipping the vector L1, as nl_dgemm.h does, loses here: a token tile's rows and a row's second
-// half of a sector are hits.  gate || up of 1536 x 4096 F16, 64 tokens: 18.2 us a launch through it, 22.8 past it)
-
-// A chunk (two pairs of blocks) of one 16-row tile, 16 bytes a lane and load: lane (row li, group lq) takes pair lq & 1, so that a row's two pairs
+// A chunk (two pairs of blocks) of one 16-row tile, as raw buffer loads (pg_load16; skipping the vector L1, as nl_dgemm.h does, loses here: a token
+// tile's rows and a row's second half of a sector are hits.  gate || up of 1536 x 4096 F16, 64 tokens: 18.2 us a launch through it, 22.8 past it),
+// 16 bytes a lane and load: lane (row li, group lq) takes pair lq & 1, so that a row's two pairs
 // (32 bytes) travel in one request, and the operand order -- each of the four groups an eighth of a block -- is made by swapping 16- and
 // 32-lane rows between registers.  (Asked for in operand order, four or eight bytes a lane, every request moved a whole sector for a
 // quarter of it or less: gate || up of 1536 x 4096, Q8_0, 33 tokens, 22.8 us a launch against 19.8.)
@@ -218,7 +218,8 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
         xput(0);
         if (tid * 4 < P.cols) *reinterpret_cast<uint4 *>(ws + tid * 4) = wn;
         for (int i = (tid + nw * 64) * 4; i < P.cols; i += nw * 256) *reinterpret_cast<float4 *>(ws + i) = *reinterpret_cast<const float4 *>(P.normw + i);
-        for (int i0 = XB; i0 < nxb; i0 += XB) { xload(i0); xput(i0); }     // (more than 2048 columns: none fit the LDS)
+        for (int i0 = XB; i0 < nxb; i0 += XB) { xload(i0); xput(i0); }     // (blocks past XB per wavefront: beyond 1024 columns of eight, 2048 of
+                                                                             //  sixteen.  They are asked for behind the weights)
         ss += dpp_f64<DPP_QUAD_XOR1>(ss);
         ss += dpp_f64<DPP_QUAD_XOR2>(ss);
         if (xq == 0) red[wv * 16 + xr] = ss;
@@ -230,12 +231,7 @@ __global__ void __launch_bounds__(NWV * 64, NWV / 4) sgemm_kernel(SGemmParams P)
         for (int k = 0; k < NWV; k++) sq[k] = red[k * 16 + li];      // (in flight together)
 #pragma unroll
         for (int k = 0; k < NWV; k++) tot += sq[k];
-        // dg_inv_rms with its division on the host
-        const double m = fma(tot, P.rcols, (double)P.eps);
-        double y0 = __builtin_amdgcn_rsq(m);
-        y0 = y0 * fma(-0.5 * m * y0, y0, 1.5);
-        y0 = y0 * fma(-0.5 * m * y0, y0, 1.5);
-        const float inv = (float)y0;
+        const float inv = dg_inv_rms(tot, P.rcols, P.eps);       // (the division is the host's)
         for (int i = 0; i < nxb; i++) {
             const int blk = wv + i * nw;
             uint4 *const at = xs + (size_t)blk * (2 * QG_FRAG);
