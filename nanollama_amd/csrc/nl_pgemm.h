@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     constexpr int KB = 4;                                   // blocks per chunk
     constexpr int ROWS = RT * TR, TOK = 64 * NTW, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
     constexpr int SC = X1 ? PG_NONE : F::SC;
-    constexpr bool MINS = WT == WT_Q4_K;
+    constexpr bool MINS = WT == WT_Q4_K, PAIRS = EXACT || WT == WT_Q4_0;
     // a block's plane of fragments is padded by 64 bytes: the two pairs' expansions of a wavefront land on different banks
     constexpr int PLANE = F::FR * RT * 1024 + 64, BUF = KB * PLANE, SCP = ROWS + 16, SCB = SCP * KB * 4, WBYTES = 2 * (BUF + (SC ? SCB : 0) + (MINS ? SCB : 0));
     constexpr int SBYTES = TOK * LD * 4, SET = WBYTES > SBYTES ? WBYTES : SBYTES, NTHR = 256 * KW;
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const int kset = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     char *const smem = smem_all + kset * SET;
     const int tid = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, lq = lane >> 4;
-    const int nblocks = P.cols / 32, nchunks = (nblocks + KB - 1) / KB;
+    const int nblocks = P.cols / 32, nchunks = P.npairs / KL * 2 + ((P.npairs % KL) + 1) / 2;
     constexpr bool FUSED = EPI == QG_EPI_SWIGLU;
     constexpr int TPW = FUSED ? RT / 2 : RT;                // row tiles of a matrix per workgroup
     const int nrb = (P.ntiles + TPW - 1) / TPW, ntb = (P.n_tokens + TOK - 1) / TOK, total = nrb * ntb, per = (total + 7) / 8;
@@ -205,34 +205,47 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const bool by_rows = (long long)P.ntiles * TR * (FUSED ? 2 : 1) * F::CPP > (long long)P.n_tokens * 8 * PS;
     const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
 
-    // staging items: pair kk of the chunk's two, row r, half h of the pair, row tile -- a wavefront's loads are runs of 32 bytes
-    const int i_kk = tid & 1, i_r = (tid >> 1) & 15, i_h = (tid >> 5) & 1, i_t = wave;
+    // F16 and Q8_0: a group of four pairs is two chunks, the even blocks of its pairs, then the odd ones.  A wavefront's load is then one 16-byte plane of
+    // all four pairs over a tile's rows, a whole KiB; two pairs with both their blocks (PAIRS) are half of every 64-byte run, twice the sectors.  F16, 993
+    // tokens, 1536 columns: Q|K|V 30.8 us, now 25.0, gate and up 61.5 and 57.5, WO 19.4 and 17.6, down 41.1 and 35.5; Q8_0, 700 tokens: 19.9 and 19.2, 53.9
+    // and 52.5, 17.2 and 16.7, 35.7 and 35.0.  Q4_0's blocks are one plane, K-quants' two share their bytes: nothing to gain (17.3 and 17.6, 11.8 and 11.9).
+    // A last group of one or two pairs is one chunk of both their blocks.
+    // staging items: block kk of the chunk, row r, row tile
+    const int i_kk = PAIRS ? 2 * (tid & 1) + ((tid >> 5) & 1) : tid & 3, i_r = (PAIRS ? tid >> 1 : tid >> 2) & 15, i_t = wave;
     struct Raw { uint4 c[F::NC]; uint32_t s[SWN]; };
     // Weights as raw buffer loads from the workgroup's first tile: the wavefront's row tile and the chunk are scalar arithmetic, the lane's part is a
     // register that changes in the last group only.  (With a 64-bit address per load a chunk's staging was 100 of a wavefront's 224 vector
-    // instructions beside 128 MFMAs, and the two add up on a SIMD: 841M F16, 993 tokens 5456 us, now 5400; 173M Q4_K, 333 tokens 1961, now 1911)
+    // instructions beside 128 MFMAs: 841M F16, 993 tokens 5456 us against 5400; 173M Q4_K, 333 tokens 1961 against 1911)
     constexpr unsigned QG = F::CPP * TR * 16, SG = TR * F::SW * 4;      // bytes of a pair over a tile's rows
     const __amdgpu_buffer_rsrc_t rq0 = pg_rsrc(P.q + (size_t)tile0 * P.npairs * QG), rq1 = pg_rsrc((FUSED ? P.q1 : P.q) + (size_t)tile0 * P.npairs * QG);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs0 = pg_rsrc(reinterpret_cast<const char *>(P.s) + (size_t)tile0 * P.npairs * SG),
                                                   rs1 = pg_rsrc(reinterpret_cast<const char *>(FUSED ? P.s1 : P.s) + (size_t)tile0 * P.npairs * SG);
-    const unsigned lane_q = (unsigned)((F::chunk(i_h, 0) * TR + i_r) * KL + i_kk) * 16u;
+    const int last_g = (P.npairs - 1) / KL, last_sz = P.npairs - last_g * KL;
+    // a chunk's group; whether it holds both blocks of two pairs
+    auto group_of = [&](int chunk) __attribute__((always_inline)) { return min(chunk, nchunks - 1) >> 1; };
+    auto paired = [&](int g) __attribute__((always_inline)) { return PAIRS || (g == last_g && last_sz <= 2); };
+    const unsigned lane_s = (unsigned)(i_r * KL + (PAIRS ? i_kk >> 1 : i_kk)), lane_q = (lane_s + (PAIRS ? (unsigned)F::chunk(i_kk & 1, 0) * (TR * KL) : 0u)) * 16u;
     auto stage_load = [&](int chunk, Raw (&r)[IPT]) __attribute__((always_inline)) {
-        const int c = min(chunk, (P.npairs - 1) >> 1), g = c >> 1, k0 = (c & 1) * 2, gsz = min(KL, P.npairs - g * KL);      // (a chunk past the end: the last one's, never used)
-        unsigned lq_ = lane_q, step = TR * KL * 16u;          // chunk F::chunk(i_h, j) of the pair: j steps on
-        if (gsz != KL) {
-            lq_ = (unsigned)((F::chunk(i_h, 0) * TR + i_r) * gsz + min(i_kk, gsz - 1 - k0)) * 16u;
-            step = (unsigned)(TR * gsz) * 16u;
+        const int c = min(chunk, nchunks - 1), g = c >> 1;      // (a chunk past the end: the last one's, never used)
+        unsigned lq_ = lane_q, ls_ = lane_s * F::SW * 4u, step = TR * KL * 16u;          // plane F::chunk(h, j): j steps on
+        const unsigned k0 = PAIRS ? (unsigned)(c & 1) * 2u : 0u;
+        if (PAIRS ? min(KL, P.npairs - g * KL) != KL : last_sz != KL && g == last_g) {
+            const bool both = paired(g);
+            const unsigned row_pair = (unsigned)(i_r * last_sz + min(both ? i_kk >> 1 : i_kk, last_sz - 1 - (int)k0));
+            step = (unsigned)(TR * last_sz) * 16u;
+            lq_ = row_pair * 16u + (both ? (unsigned)F::chunk(i_kk & 1, 0) * step : 0u);
+            ls_ = row_pair * F::SW * 4u;
         }
-        [[maybe_unused]] const unsigned ls_ = (lq_ - (unsigned)F::chunk(i_h, 0) * step) / 4u * F::SW;       // (row, pair) words
+        const unsigned first = k0 * 16u + (paired(g) ? 0u : (unsigned)F::chunk(c & 1, 0) * step);
 #pragma unroll
         for (int i = 0; i < IPT; i++) {
             const int rt = wave + 4 * i, dt = min(FUSED ? rt % TPW : rt, P.ntiles - 1 - tile0);
             const bool second = FUSED && rt >= TPW;
             const unsigned gp = (unsigned)(dt * P.npairs + g * KL);
 #pragma unroll
-            for (int j = 0; j < F::NC; j++) r[i].c[j] = pg_load16(second ? rq1 : rq0, lq_, gp * QG + (unsigned)k0 * 16u + j * step);
+            for (int j = 0; j < F::NC; j++) r[i].c[j] = pg_load16(second ? rq1 : rq0, lq_, gp * QG + first + j * step);
             if constexpr (F::SW > 0) {
-                const unsigned so = gp * SG + (unsigned)k0 * 4u * F::SW;
+                const unsigned so = gp * SG + k0 * 4u * F::SW;
                 if constexpr (F::SW == 2) {
                     const pg_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(second ? rs1 : rs0, ls_, so, 0);
                     r[i].s[0] = v[0];
@@ -242,11 +255,18 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         }
     };
     char *const s_sc = smem + 2 * BUF, *const s_mn = s_sc + 2 * SCB;
+    // block b of a chunk
+    auto block_of = [&](int chunk, int b) __attribute__((always_inline)) {
+        if (PAIRS) return chunk * KB + b;
+        const int g = group_of(chunk);
+        return g * 2 * KL + (paired(g) ? b : 2 * b + (chunk & 1));
+    };
     auto stage_part = [&](int chunk, int buf, int w, const Raw (&r)[IPT]) {
+        const int g = group_of(chunk), i_h = paired(g) ? i_kk & 1 : chunk & 1, b = i_kk;
+        const bool live = (PAIRS || chunk < nchunks) && block_of(chunk, i_kk) < nblocks;     // a block past the end of K contributes nothing
 #pragma unroll
         for (int i = 0; i < IPT; i++) {
-            const int rt = i_t + 4 * i, b = 2 * i_kk + i_h;
-            const bool live = chunk * KB + b < nblocks;     // a block past the end of K contributes nothing
+            const int rt = i_t + 4 * i;
             half8_t f[F::FR];
             F::part(r[i].c, r[i].s, i_h, w, f);
             if constexpr (X1) {
@@ -272,7 +292,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const unsigned xblock = (unsigned)P.nt16 * (unsigned)(PS * QG_FRAG) * 16u, xlane = (unsigned)lane * 16u;
     uint4 xp[NP][KB][NTW];
     auto xload = [&](int chunk, int b) __attribute__((always_inline)) {
-        const unsigned uo = (unsigned)min(chunk * KB + b, nblocks - 1) * xblock;
+        const unsigned uo = (unsigned)min(block_of(chunk, b), nblocks - 1) * xblock;
 #pragma unroll
         for (int t = 0; t < NTW; t++)
 #pragma unroll

@@ -49,6 +49,13 @@ def test_product_against_float64(hip, monkeypatch, kind, rows, cols, n):
     assert (np.abs(got - xd @ wd.T) <= bound).all()
 
 
+# last groups of one to four pairs, with and without a last odd block, behind whole groups: a group's chunks are its even and its odd blocks, a short one's both
+@pytest.mark.parametrize("cols", [288, 320, 352, 384, 416, 448, 480])
+@pytest.mark.parametrize("kind", ["q4_0", "q8_0", "f16"])
+def test_last_groups_of_a_row(hip, monkeypatch, kind, cols):
+    test_product_against_float64(hip, monkeypatch, kind, 272, cols, 129)
+
+
 class Scaled:
     """A parsed file with the weights of some matrices multiplied by a power of two (their scales, or the fp16 weights themselves)."""
 
