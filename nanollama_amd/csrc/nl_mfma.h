@@ -20,6 +20,7 @@
 // workgroups (TAIL), or bring the next launches' weights into L2 (Ahead).
 #pragma once
 #include "nl_kernels.h"
+#include <algorithm>
 
 namespace nl {
 
@@ -77,14 +78,12 @@ __device__ __forceinline__ float exp_f32(float x) {
 }
 __device__ __forceinline__ float rcp_f32(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float rsqrt_f32(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ float sigmoid_f32(float z) {
-    const float e = exp_f32(-fminf(fabsf(z), 100.f)), r = rcp_f32(1.f + e);
-    return z >= 0.f ? r : e * r;
-}
+// (past 88.72 the exponential is no float32; v_rcp_f32 leaves 0 below 2^-126, from 87.3 on)
+__device__ __forceinline__ float sigmoid_f32(float z) { return rcp_f32(1.f + exp_f32(__builtin_amdgcn_fmed3f(-z, -88.72f, 88.72f))); }
 __device__ __forceinline__ float silu_f32(float z) { return z * sigmoid_f32(z); }
 __device__ __forceinline__ float gelu_tanh_f32(float z) {
     // 0.5 (1 + tanh u) = sigmoid(2 u)
-    return z * sigmoid_f32(1.5957691216057308f * (z + 0.044715f * z * z * z));
+    return z * sigmoid_f32(z * fmaf(0.071354816f, z * z, 1.5957691216057308f));
 }
 template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
     return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -429,6 +428,48 @@ struct KeyRows {
     int hrows, nt, slots;
 };
 
+// ------------------------------------------------- a prompt product's tiles on XCDs ---
+
+// Blocks b, b + 8, ... run on one XCD and share its L2.  Each XCD gets a rectangle of the nrb x ntb tiles, `rows` x 8 / rows of them cover the product, and
+// reads 1 / rows of the weights and rows / 8 of the activations; where no rectangle shares the tiles out evenly, a range of them, row block after row
+// block (rows 0).  (A range always, us a launch, bf16: 1920 tokens, 768 x 2048 18.8, now 15.5, 2047 tokens, 1536 x 1536 19.5 and 18.3, 1536 x 4096 33.0 and
+// 32.0; a document of 2047 tokens, 863M: 6625 and 6581.  The nearest rectangle for 4640 x 1536, 25 x 8 tiles: 39.9 and 41.9.  Quantised files' prompts, whose
+// weights are smaller: F16 5140 and 5180, nothing.)
+struct XcdTiles {
+    int rows, nrb, ntb, r, t;               // XCDs along the rows (0: a range of tiles); tiles; an XCD's rectangle
+    __host__ __device__ __forceinline__ XcdTiles(int rows_, int nrb_, int ntb_) : rows(rows_), nrb(nrb_), ntb(ntb_) {
+        r = rows ? (nrb + rows - 1) / rows : (nrb * ntb + 7) / 8;
+        t = rows ? (ntb + 8 / rows - 1) / (8 / rows) : 1;
+    }
+    __host__ __device__ __forceinline__ int blocks() const { return 8 * r * t; }
+    // block b's tile; false: it has none
+    __host__ __device__ __forceinline__ bool tile(int b, int &rb, int &tb) const {
+        const int xcd = b & 7, at = b >> 3;
+        if (rows) {
+            rb = xcd % rows * r + at / t;
+            tb = xcd / rows * t + at % t;
+        } else {
+            rb = (xcd * r + at) / ntb;
+            tb = xcd * r + at - rb * ntb;
+        }
+        return at < r * t && rb < nrb && tb < ntb;
+    }
+};
+// The fewest operand bytes among those that give no XCD more tiles than a range does; row_bytes, tok_bytes: a row block's and a token block's bytes
+// of a column, in any unit
+inline int xcd_rows(int nrb, int ntb, int row_bytes, int tok_bytes) {
+    const long long per = ((long long)nrb * ntb + 7) / 8;
+    int best = 0;
+    // (a range starts inside a row of tiles)
+    long long best_b = std::min<long long>(nrb, (per + ntb - 1) / ntb + (per % ntb ? 1 : 0)) * row_bytes + std::min<long long>(ntb, per) * tok_bytes;
+    for (int rows = 1; rows <= 8; rows *= 2) {
+        const XcdTiles x(rows, nrb, ntb);
+        const long long b = (long long)x.r * row_bytes + (long long)x.t * tok_bytes;
+        if ((long long)x.r * x.t == per && b <= best_b) best = rows, best_b = b;
+    }
+    return best;
+}
+
 struct MatParams {
     const void *W;         // [nrt][nks] operand tiles; ST_GATED: gate tile, up tile, gate tile, ...
     const void *X;         // [token tiles][nks]
@@ -440,6 +481,7 @@ struct MatParams {
     int act_nks, act_silu; // activation: silu or tanh-gelu
     const float *bias, *bias2;   // ST_F32: per row; ST_GATED: of gate and up; whole row tiles long, or null
     int x_nks;             // k tiles per token tile of X (0: nks)
+    int xcd_rows;          // many_kernel, direct_kernel: XCDs along the rows (XcdTiles)
     int group;             // few_kernel: row tiles of a group; group i multiplies X's k tiles from i * nks on (0: one group)
     const int *x_tile;     // many_kernel: which tile of X is token tile t (null: t)
     HeadRows hd;
@@ -517,18 +559,19 @@ __device__ __forceinline__ void add_rows_folded(const MatParams &P, int tok, int
     if (g == 0 && tok < P.n_tokens) P.fss[(long long)rt * P.fss_ld + tok] = ss;
 }
 // four consecutive feed-forward rows f16 * 16 + 4 g .. + 3 of one token
-template <typename T>
-__device__ __forceinline__ void store_gated(const MatParams &P, int tok, int f16, int g, f32x4 gate, f32x4 up) {
+template <bool SILU> __device__ __forceinline__ f32x4 gated(f32x4 gate, f32x4 up) {
     f32x4 v;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (P.bias) {
-            gate[i] += P.bias[f16 * 16 + 4 * g + i];
-            up[i] += P.bias2[f16 * 16 + 4 * g + i];
-        }
-        v[i] = (P.act_silu ? silu_f32(gate[i]) : gelu_tanh_f32(gate[i])) * up[i];
+    for (int i = 0; i < 4; i++) v[i] = (SILU ? silu_f32(gate[i]) : gelu_tanh_f32(gate[i])) * up[i];
+    return v;
+}
+template <typename T>
+__device__ __forceinline__ void store_gated(const MatParams &P, int tok, int f16, int g, f32x4 gate, f32x4 up) {
+    if (P.bias) {
+        gate += *reinterpret_cast<const f32x4 *>(P.bias + f16 * 16 + 4 * g);
+        up += *reinterpret_cast<const f32x4 *>(P.bias2 + f16 * 16 + 4 * g);
     }
-    put4(reinterpret_cast<T *>(P.act) + op_index(tok, f16 * 16 + 4 * g, P.act_nks), v);
+    put4(reinterpret_cast<T *>(P.act) + op_index(tok, f16 * 16 + 4 * g, P.act_nks), P.act_silu ? gated<true>(gate, up) : gated<false>(gate, up));
 }
 
 __device__ __forceinline__ f32x4 with_bias(const float *bias, int row, f32x4 v) {
@@ -567,19 +610,16 @@ __global__ void __launch_bounds__(256) many_kernel(MatParams P, TAIL tail) {
     constexpr int PW = STAGE / 4096;                       // 1 KiB pieces per stage and wavefront
     extern __shared__ __align__(16) char lds[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4;
-    const int nrb = (P.nrt + RT - 1) / RT, ntt = (P.n_tokens + 15) >> 4, ntb = (ntt + NT - 1) / NT, total = nrb * ntb;
-    // blocks b, b + 8, ... run on one XCD: give each XCD a contiguous range of (row block, token block), token blocks fastest, so
-    // that the token blocks of a row block share its weights in one L2
-    const int per = (total + 7) / 8;
+    const int nrb = (P.nrt + RT - 1) / RT, ntt = (P.n_tokens + 15) >> 4, ntb = (ntt + NT - 1) / NT;
+    const XcdTiles xt(P.xcd_rows, nrb, ntb);
     if constexpr (TAIL::on)
-        if ((int)blockIdx.x >= per * 8) {
-            const int u = (blockIdx.x - per * 8) * 4 + w;
+        if ((int)blockIdx.x >= xt.blocks()) {
+            const int u = (blockIdx.x - xt.blocks()) * 4 + w;
             if (u < tail.units) tail.unit(u, lane);
             return;
         }
-    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
-    const int rb = id / ntb, tb = id - rb * ntb;
+    int rb, tb;
+    if (!xt.tile(blockIdx.x, rb, tb)) return;
     const int wr = w & 1, wt = w >> 1, nks = P.nks;
     f32x4 acc[RTW][4] = {};
     const char *src[PW];                                   // this wavefront's pieces of k tile 0
@@ -675,10 +715,10 @@ __global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P) 
     extern __shared__ __align__(16) char lds[];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
     const int nks = P.nks, ntt = (P.n_tokens + 15) >> 4;
-    const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = (ntt + WT * TW - 1) / (WT * TW), total = nrb * ntb;
-    const int per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);      // (as many_kernel's)
-    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
-    const int rb = id / ntb, tb = id - rb * ntb, kw = w / SET, wr = w % WR, wt = w / WR % WT, r0 = (rb * WR + wr) * RW, t0 = (tb * WT + wt) * TW;
+    const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = (ntt + WT * TW - 1) / (WT * TW);
+    int rb, tb;
+    if (!XcdTiles(P.xcd_rows, nrb, ntb).tile(blockIdx.x, rb, tb)) return;
+    const int kw = w / SET, wr = w % WR, wt = w / WR % WT, r0 = (rb * WR + wr) * RW, t0 = (tb * WT + wt) * TW;
     const __amdgpu_buffer_rsrc_t W = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.W), 0, (int)((unsigned)P.nrt * nks * UNIT), 0x00027000);
     const __amdgpu_buffer_rsrc_t X = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.X), 0, (int)((unsigned)ntt * P.x_nks * UNIT), 0x00027000);
     unsigned wo[RW], xo[TW];                               // (tiles past the end repeat the last one)
@@ -707,6 +747,20 @@ __global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P) 
             for (int t = 0; t < TW; t++) acc[r][t] = mma(a[s][r], b[s][t], acc[r][t]);
         fence();
     };
+    // residual rows of this wavefront's results, requested in front of the loop: behind it every pair of tiles waits for its own
+    constexpr int RR = KS == 1 ? 2 : direct_rows(SET * KS, RW, TW), PAIRS = RR / 2 * TW, PJ = KS == 1 ? TW : (PAIRS + KS - 1) / KS, NP = RW / RR * PJ;
+    constexpr bool HELD = EPI == ST_RESID && NP <= 8;
+    [[maybe_unused]] const bool ahead = HELD && (P.ldo & 3) == 0 && (P.rows & 15) == 0;
+    [[maybe_unused]] f32x4 held[HELD ? 2 * NP : 1];
+    if constexpr (HELD)
+        if (ahead)
+#pragma unroll
+            for (int at = 0; at < NP; at++) {
+                const int p = KS == 1 ? at % PJ : min(kw + at % PJ * KS, PAIRS - 1), r = at / PJ * RR + p / TW * 2, t = p % TW;
+                const float *x = P.out + (long long)min((t0 + t) * 16 + (lane & 15), P.n_tokens - 1) * P.ldo + 4 * g;
+#pragma unroll
+                for (int i = 0; i < 2; i++) held[2 * at + i] = *reinterpret_cast<const f32x4 *>(x + min(r0 + r + i, P.nrt - 1) * 16);
+            }
     load(kw, 0);
     int ks = kw;
     for (; ks + KS < nks; ks += 2 * KS) {
@@ -716,48 +770,86 @@ __global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P) 
         step(1);
     }
     if (ks < nks) step(0);
-    auto store = [&](int r, int t, f32x4 v, f32x4 v2) {
-        const int tok = (t0 + t) * 16 + (lane & 15), rt = r0 + r, row = rt * 16 + 4 * g;
-        if (tok >= P.n_tokens || rt >= P.nrt) return;
-        if constexpr (EPI == ST_GATED) store_gated<T>(P, tok, rt >> 1, g, v, v2);
-        else {
+    // What this wavefront finishes: pairs of row tiles.  All of it as the sum of KS sets, in rounds of RR rows of tiles
+    auto finish = [&](auto each) __attribute__((always_inline)) {
+        if constexpr (KS == 1) {
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                if (rt + i >= P.nrt) break;
-                if constexpr (EPI == ST_F32) store_rows(P.out, P.ldo, P.rows, tok, row + 16 * i, with_bias(P.bias, row + 16 * i, i ? v2 : v));
-                else if constexpr (EPI == ST_HEADS) store_heads<T>(P.hd, tok, row + 16 * i, i ? v2 : v);
-                else add_rows(P.out, P.add2, P.ldo, P.rows, tok, row + 16 * i, i ? v2 : v);
+            for (int r = 0; r < RW; r += 2)
+#pragma unroll
+                for (int t = 0; t < TW; t++) each(r / 2 * TW + t, r, t, acc[r][t], acc[r + 1][t]);
+        } else {
+            f32x4 *red = reinterpret_cast<f32x4 *>(lds);   // [KS][SET][RR][TW][64]
+#pragma unroll
+            for (int r = 0; r < RW; r += RR) {
+                if (r) lds_barrier();
+#pragma unroll
+                for (int i = 0; i < RR; i++)
+#pragma unroll
+                    for (int t = 0; t < TW; t++) red[((w * RR + i) * TW + t) * 64 + lane] = acc[r + i][t];
+                lds_barrier();
+#pragma unroll
+                for (int j = 0; j < PJ; j++) {
+                    const int p = kw + j * KS, i = p / TW * 2, t = p % TW;
+                    if (p >= PAIRS) break;                 // (more wavefronts than pairs)
+                    f32x4 v[2] = {};
+#pragma unroll
+                    for (int q = 0; q < KS; q++)
+#pragma unroll
+                        for (int k = 0; k < 2; k++) v[k] += red[(((q * SET + w % SET) * RR + i + k) * TW + t) * 64 + lane];
+                    each(r / RR * PJ + j, r + i, t, v[0], v[1]);
+                }
             }
         }
     };
-    if constexpr (KS == 1) {
+    if constexpr (EPI == ST_GATED) {
+        // (chosen once: with the choice inside, every tile is basic blocks of its own, and a SIMD's only wavefront waits out each exponential)
+        [[maybe_unused]] f32x4 gb[RW / 2] = {}, ub[RW / 2] = {};
+        auto biases = [&](int r, f32x4 &b, f32x4 &b2) __attribute__((always_inline)) {
+            const int row = min((r0 + r) >> 1, (P.nrt >> 1) - 1) * 16 + 4 * g;
+            b = *reinterpret_cast<const f32x4 *>(P.bias + row);
+            b2 = *reinterpret_cast<const f32x4 *>(P.bias2 + row);
+        };
+        if constexpr (KS == 1)
+            if (P.bias)
 #pragma unroll
-        for (int r = 0; r < RW; r += 2)
+                for (int r = 0; r < RW; r += 2) biases(r, gb[r / 2], ub[r / 2]);
+        auto with = [&](auto silu) __attribute__((always_inline)) {
+            finish([&](int, int r, int t, f32x4 gate, f32x4 up) __attribute__((always_inline)) {
+                const int tok = (t0 + t) * 16 + (lane & 15), f16 = (r0 + r) >> 1;
+                if constexpr (KS == 1) {
+                    gate += gb[r / 2];
+                    up += ub[r / 2];
+                } else if (P.bias) {
+                    f32x4 b, b2;
+                    biases(r, b, b2);
+                    gate += b;
+                    up += b2;
+                }
+                f32x4 v = gated<decltype(silu)::value>(gate, up);
+                asm volatile("" : "+v"(v));
+                if (tok < P.n_tokens && r0 + r < P.nrt) put4(reinterpret_cast<T *>(P.act) + op_index(tok, f16 * 16 + 4 * g, P.act_nks), v);
+            });
+        };
+        if (P.act_silu) with(std::true_type{});
+        else with(std::false_type{});
+    } else {
+        finish([&](int at, int r, int t, f32x4 v, f32x4 v2) __attribute__((always_inline)) {
+            const int tok = (t0 + t) * 16 + (lane & 15), rt = r0 + r, row = rt * 16 + 4 * g;
+            if (tok >= P.n_tokens) return;
 #pragma unroll
-            for (int t = 0; t < TW; t++) store(r, t, acc[r][t], acc[r + 1][t]);
-        return;
-    }
-    constexpr int RR = direct_rows(SET * KS, RW, TW), PAIRS = RR / 2 * TW;
-    f32x4 *red = reinterpret_cast<f32x4 *>(lds);           // [KS][SET][RR][TW][64]: RR rows of tiles at a time
-#pragma unroll
-    for (int r = 0; r < RW; r += RR) {
-        if (r) lds_barrier();
-#pragma unroll
-        for (int i = 0; i < RR; i++)
-#pragma unroll
-            for (int t = 0; t < TW; t++) red[((w * RR + i) * TW + t) * 64 + lane] = acc[r + i][t];
-        lds_barrier();
-#pragma unroll
-        for (int j = 0; j < (PAIRS + KS - 1) / KS; j++) {
-            const int p = kw + j * KS, i = p / TW * 2, t = p % TW;
-            if (p >= PAIRS) break;                         // (more wavefronts than pairs)
-            f32x4 v[2] = {};
-#pragma unroll
-            for (int q = 0; q < KS; q++)
-#pragma unroll
-                for (int k = 0; k < 2; k++) v[k] += red[(((q * SET + w % SET) * RR + i + k) * TW + t) * 64 + lane];
-            store(r + i, t, v[0], v[1]);
-        }
+            for (int i = 0; i < 2; i++) {
+                if (rt + i >= P.nrt) break;
+                const f32x4 u = i ? v2 : v;
+                if constexpr (EPI == ST_F32) store_rows(P.out, P.ldo, P.rows, tok, row + 16 * i, with_bias(P.bias, row + 16 * i, u));
+                else if constexpr (EPI == ST_HEADS) store_heads<T>(P.hd, tok, row + 16 * i, u);
+                else if (ahead) {
+                    const long long to = (long long)tok * P.ldo + row + 16 * i;
+                    f32x4 x = u + held[HELD ? 2 * at + i : 0];
+                    if (P.add2) x += *reinterpret_cast<const f32x4 *>(P.add2 + to);
+                    *reinterpret_cast<f32x4 *>(P.out + to) = x;
+                } else add_rows(P.out, P.add2, P.ldo, P.rows, tok, row + 16 * i, u);
+            }
+        });
     }
 }
 
@@ -1033,11 +1125,15 @@ template <typename T, int EPI, class TAIL = NoTail>
 hipError_t launch_many(const MatParams &P, hipStream_t st, TAIL tail = {}) {
     const int ntb = (P.n_tokens + 127) / 128;
     auto go = [&](auto kfn, int rt, int lds) {
-        const int total = (P.nrt + rt - 1) / rt * ntb;
-        hipLaunchKernelGGL(kfn, dim3((total + 7) / 8 * 8 + (TAIL::on ? (tail.units + 3) / 4 : 0)), dim3(256), lds, st, P, tail);
+        MatParams Q = P;
+        const int nrb = (P.nrt + rt - 1) / rt;
+        Q.xcd_rows = xcd_rows(nrb, ntb, rt, 8);
+        hipLaunchKernelGGL(kfn, dim3(XcdTiles(Q.xcd_rows, nrb, ntb).blocks() + (TAIL::on ? (tail.units + 3) / 4 : 0)), dim3(256), lds, st, Q, tail);
         return hipGetLastError();
     };
-    if ((P.nrt + 7) / 8 * ntb >= 512) return go(many_kernel<T, EPI, 4, TAIL>, 8, ManyGeom<T, 4>::LDS);
+    // 64 x 128 tiles up to three of them a compute unit, 128 x 128 beyond (bf16, 2047 tokens, K 1536: 3072 rows 27.6 us against 30.5, 3456 rows 38.4 against 31.3;
+    // K 768, 1200 tokens, 4096 rows 14.8 against 16.5)
+    if (sizeof(T) == 2 ? (long long)((P.nrt + 3) / 4) * ntb > 768 : (P.nrt + 7) / 8 * ntb >= 512) return go(many_kernel<T, EPI, 4, TAIL>, 8, ManyGeom<T, 4>::LDS);
     return go(many_kernel<T, EPI, 2, TAIL>, 4, ManyGeom<T, 2>::LDS);
 }
 
@@ -1045,8 +1141,10 @@ template <typename T, int EPI, int WR, int WT, int KS, int RW, int TW>
 hipError_t launch_direct(const MatParams &P, hipStream_t st) {
     constexpr int lds = KS == 1 ? 0 : WR * WT * KS * direct_rows(WR * WT * KS, RW, TW) * TW * 1024;
     static_assert(lds <= 65536, "what a launch has without asking");
-    const int total = (P.nrt + WR * RW - 1) / (WR * RW) * (((P.n_tokens + 15) / 16 + WT * TW - 1) / (WT * TW));
-    hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3((total + 7) / 8 * 8), dim3(WR * WT * KS * 64), lds, st, P);
+    const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = ((P.n_tokens + 15) / 16 + WT * TW - 1) / (WT * TW);
+    MatParams Q = P;
+    Q.xcd_rows = xcd_rows(nrb, ntb, WR * RW, WT * TW);
+    hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3(XcdTiles(Q.xcd_rows, nrb, ntb).blocks()), dim3(WR * WT * KS * 64), lds, st, Q);
     return hipGetLastError();
 }
 // Prompts: the largest tile with which the workgroups still cover the chip, in one round where that goes.  us, many_kernel -> direct_kernel,
@@ -1056,10 +1154,12 @@ hipError_t launch_direct(const MatParams &P, hipStream_t st) {
 //   64 x 64, K over 4, two a CU    768 x 768 at 2047 12.4 -> 9.1; 1536 x 4096 at 400 38.7 -> 14.6; 4640 x 1536 at 400 20.9 -> 12.9
 //   96 x 128, K over 4             1536 x 1536 at 2047 24.5 -> 19.5 (64 x 64: 25.9); 1536 x 4096 at 2047 51.1 -> 31.9 (58.6); its sums are not
 //                                  worth their way through LDS below a K of 1024
-//   192 x 256 and 256 x 256        4640 x 1536 at 2047 51.6 -> 38.3; 8192 x 1536 at 2047 63.5 -> 54.3, at 1500 (192 tiles) 53.2 -> 51.1; with
-//                                  fewer CUs at work slower, at 1000 (128 tiles) 31.6 -> 46.2
 //   64 x 64 up to 3.5 a CU         4640 x 1536 at 700 23.0 -> 20.9; 8192 x 1536 at 400 21.8 -> 20.0; 2320 x 768 at 1500 14.3, both; beyond,
 //                                  8192 x 1536 at 700, 27.2 against 28.6
+//   192 x 256 and 256 x 256        a compute unit holds one, of many_kernel's 128 x 128 two.  A round of those takes about 1.25 and 1.45 times as long as a full
+//                                  round of many_kernel's, whose last one, with no more than one a compute unit, takes 0.6 of it: 128 x 128 / 192 x 256 / 256 x 256
+//                                  4128 x 1536 at 2047 48.0 / 36.0 / 42.5, 8192 x 1536 at 1000 31.5 / 39.8 / 45.3, at 1100 47.6 / 37.7 / 43.4, at 1408 53.3 / 64.7 / 44.7,
+//                                  22016 x 4096 at 500 117 / 107 / 120, at 2047 382 / 369 / 315, 12352 x 4096 at 993 128 / 169 / 114, 11008 x 2048 at 2047 101 / 85 / 98
 // float, 1536 x 1536 at 70 and 1000: 61.7 -> 15.3, 66.4 -> 53.3 (its matrix instructions bound the large products: the small tiles only)
 template <typename T, int EPI>
 hipError_t launch_prompt(const MatParams &P, hipStream_t st) {
@@ -1070,12 +1170,15 @@ hipError_t launch_prompt(const MatParams &P, hipStream_t st) {
     if (tiles(2, 4) <= 256) return launch_direct<T, EPI, 1, 1, 8, 2, 4>(P, st);
     if (tiles(4, 4) <= 512) return launch_direct<T, EPI, 1, 1, 4, 4, 4>(P, st);
     if constexpr (sizeof(T) == 2) {
-        auto covers = [&](int rt, int t) { return tiles(rt, t) >= 192 && tiles(rt, t) <= 256; };
         if (tiles(6, 8) <= 256 && P.nks >= 32) return launch_direct<T, EPI, 1, 1, 4, 6, 8>(P, st);
-        if (covers(12, 16)) return launch_direct<T, EPI, 2, 2, 1, 6, 8>(P, st);
-        if (covers(16, 16)) return launch_direct<T, EPI, 2, 2, 1, 8, 8>(P, st);
     }
     if (tiles(4, 4) <= 896) return launch_direct<T, EPI, 1, 1, 4, 4, 4>(P, st);
+    if constexpr (sizeof(T) == 2) {
+        auto rounds = [&](int rt, int t) { return (double)((tiles(rt, t) + 255) / 256); };
+        const long long n = tiles(8, 8), last = n % 512;
+        const double many = tiles(4, 8) <= 768 ? 0.85 : (double)(n / 512) + (last == 0 ? 0.0 : last <= 256 ? 0.6 : 1.0), by12 = 1.25 * rounds(12, 16), by16 = 1.45 * rounds(16, 16);
+        if (std::min(by12, by16) < many) return by12 <= by16 ? launch_direct<T, EPI, 2, 2, 1, 6, 8>(P, st) : launch_direct<T, EPI, 2, 2, 1, 8, 8>(P, st);
+    }
     return launch_many<T, EPI>(P, st);
 }
 

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import stack_oracle as so
-from stack_models import BF16_TOL, F32_TOL, bits, config, floats, gla, load, par, rel, tokens, weights
+from stack_models import BF16_TOL, F32_TOL, bits, config, floats, gla, lat, lconfig, load, par, rel, tokens, weights
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -225,6 +225,19 @@ def test_more_wanted_rows_than_one_logits_buffer(base):
     ids = tokens(600, seed=4)
     m = load(cfg, w, "float32", max_streams=1, seq_len=600)
     assert rel(whole(m, ids), so.forward(cfg, floats(w), ids)) < F32_TOL
+    m.close()
+
+
+# Prompts whose products take many_kernel's 128 x 128 tiles, 192 x 256 and 256 x 256 ones (one and two rounds of them), and 96 x 128 with the residual rows
+# requested early; ragged tiles either way, widths of whole and of partial row tiles, both activations, with and without biases.
+@pytest.mark.parametrize("family", ["ganidra", "pabalix"])
+@pytest.mark.parametrize("width,ff,n", [(100, 2752, 1300), (96, 2064, 2030), (96, 4104, 1400), (96, 5504, 2047), (1056, 1100, 2047)])
+def test_prompt_tiles(family, width, ff, n):
+    cfg = lconfig([lat(ff=ff)], width=width) if family == "pabalix" else config([gla(ff=ff)], width=width)
+    w = weights(cfg, 5)
+    ids = tokens(n, seed=n)
+    m = load(cfg, w, "bfloat16", max_streams=1, seq_len=2048)
+    assert rel(whole(m, ids), so.forward(cfg, floats(w), ids)) < BF16_TOL
     m.close()
 
 
