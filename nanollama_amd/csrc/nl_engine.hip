@@ -135,7 +135,8 @@ struct Op {
 }  // namespace
 
 // nl_engine::step_path: which kernels a layer of a multi-token step ran on (none of the first two: qgemm_kernel / pgemm_kernel, by matrix)
-enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */ };
+enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */,
+       PATH_IMAGES = 16 /* the projections of a prompt wrote the attention's K and V^T images */ };
 
 struct nl_engine {
     nl_config cfg{};
@@ -2080,6 +2081,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const int nt16 = ((n + 63) / 64) * 4;
     // position splits any token of this step can see: the attention grids skip the rest (a decode batch at short
     // contexts would otherwise dispatch 15 empty workgroups for every live one)
+    const bool kv16_launch = getenv("NL_KV16_LAUNCH") != nullptr;       // knob (tests, read per step): the images by a launch of their own always
     const bool no_tile = attn_knobs().no_tile, no_fin = getenv("NL_NO_ATTN_FIN") != nullptr;   // (no_fin: knob of tests, read per step: the merge launch always)
     int nsplit = 1;
     for (int i = 0; i < n; i++) nsplit = std::max(nsplit, b.h_meta[b.cap + i] / ATT_CH + 1);
@@ -2151,7 +2153,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         float *kc = e->kcache + (long long)l * e->kv_layer_stride;
         float *vc = e->vcache + (long long)l * e->kv_layer_stride;
         GemmOut qkv_out{nullptr, nullptr, 1, 0, nullptr};
-        bool rope_in_attn = false;
+        bool rope_in_attn = false, images = false;      // images: the Q|K|V launch leaves K and V^T as the attention's images, too
         const SgSplits sp = sg ? sgemm_splits(b, L, n) : SgSplits{};
         const bool folded_in = fold && l > 0;      // the previous layer's down GEMM wrote this layer's Q|K|V input
         if (!folded_in && !sg) LCK(norm(L.attn_norm, L.qkv, 0, n, fold ? sB : nullptr));
@@ -2170,6 +2172,13 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             P.n_tokens = n; P.ldo = (int)R; P.x1 = x1_gemm; P.exact = exact;
             P.rope = QGemmParams::Rope{b.pos, b.stream, e->rope_cos, e->rope_sin, b.q, kc, vc, e->kv_stream_stride,
                                        L.bq, L.bk, L.bv, hd, e->Hs, e->KVs, c.seq_len, c.rope_conjugate, b.tcos, b.tsin, b.tkv};
+            // (a prompt from position 0, whose token tiles are the images' chunks or halves of them)
+            images = kv16_on && !dg && !exact && hd == 64 && b.h_meta[b.cap] == 0 && pgemm_ok(m, n) && !kv16_launch;
+            if (images) {
+                P.rope.kv16 = b.kv16;
+                P.rope.kv16_chunks = e->nsplit_max;
+                e->step_path |= PATH_IMAGES;
+            }
             LCK(dg ? launch_dgemm_rope(P, st) : launch_qgemm_rope(m.wtype, P, st));
         } else {
             LCK(qg(e, b, L.qkv, n, b.qkv, R, nullptr, st, &qkv_out, b.kpart, nullptr, nullptr, nullptr, x1_gemm, 1, exact));
@@ -2215,8 +2224,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                     const int n_keys = b.h_meta[b.cap] + n;
                     Kv16BuildParams KB{kc + so, vc + so, b.kv16, c.seq_len, e->nsplit_max, n_keys};
                     const dim3 kg(e->KVs, (n_keys + ATT_CH - 1) / ATT_CH);
-                    if (hd == 64) hipLaunchKernelGGL(kv16_build_kernel<64>, kg, dim3(512), 0, st, KB);
-                    else hipLaunchKernelGGL(kv16_build_kernel<32>, kg, dim3(512), 0, st, KB);
+                    if (hd == 64 && !images) hipLaunchKernelGGL(kv16_build_kernel<64>, kg, dim3(512), 0, st, KB);
+                    else if (hd != 64) hipLaunchKernelGGL(kv16_build_kernel<32>, kg, dim3(512), 0, st, KB);
                     T.kv16 = b.kv16;
                 }
                 LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st, f32_tile)

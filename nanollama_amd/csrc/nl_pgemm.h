@@ -569,6 +569,62 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
                               : (is_k ? R.kcache : R.vcache) + (at + (long long)kvh * R.seq_len * hd + i0);
             *reinterpret_cast<f32x4_t *>(dst) = o0;
             *reinterpret_cast<f32x4_t *>(dst + half) = o1;
+            if (R.kv16 && is_k) {
+                // ... and as the attention's image: elements i0 .. + 3 and the same of the other half, hi and lo (position = token)
+                typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+                typedef Kv16Image<64> Img;
+                _Float16 *const K = reinterpret_cast<_Float16 *>(R.kv16 + ((long long)kvh * R.kv16_chunks + n / ATT_CH) * (Img::BYTES / 16));
+                half4_t h0, l0, h1, l1;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    _Float16 a, b;
+                    split_hi_lo(o0[j], a, b);
+                    h0[j] = a; l0[j] = b;
+                    split_hi_lo(o1[j], a, b);
+                    h1[j] = a; l1[j] = b;
+                }
+                const int k0 = Img::k_off(n % ATT_CH, i0 >> 3) + (i0 & 4), k1 = Img::k_off(n % ATT_CH, (i0 >> 3) + 4) + (i0 & 4);
+                *reinterpret_cast<half4_t *>(K + k0) = h0;
+                *reinterpret_cast<half4_t *>(K + ATT_CH * Img::KS + k0) = l0;
+                *reinterpret_cast<half4_t *>(K + k1) = h1;
+                *reinterpret_cast<half4_t *>(K + ATT_CH * Img::KS + k1) = l1;
+            }
+        }
+        if (R.kv16) {
+            // V^T: eight keys of one element per item, one 16-byte segment of hi and of lo; keys past the prompt up to the chunk's end are zeros (their
+            // probabilities are, too, and must meet finite values).  A head is four tiles.
+            typedef Kv16Image<64> Img;
+            const bool last = tok0 + TOK >= P.n_tokens;
+            const int keys = last ? (tok0 + TOK + ATT_CH - 1) / ATT_CH * ATT_CH - tok0 : TOK;      // (a last 64-token tile may be half of its chunk)
+#pragma unroll
+            for (int hh = 0; hh < RT / 4; hh++) {
+                const int kvh = (tile0 >> 2) + hh - R.n_q_heads - R.n_kv_heads;
+                if (kvh < 0 || tile0 + 4 * hh >= P.ntiles) continue;
+                for (int it = et; it < 8 * keys; it += NTHR) {
+                    const int sg = it & 7, d = (it >> 3) & 63, t0 = (it >> 9) * 64 + (sg >> 2) * 32 + (sg & 3) * 4, n0 = tok0 + t0;
+                    const int col = hh * 64 + ((d & 31) >> 3) * 16 + (d & 7) + 8 * (d >> 5);
+                    const float bias = R.bias_v ? R.bias_v[kvh * 64 + d] : 0.f;
+                    half8_t hi = {}, lo = {};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int t = t0 + (e >> 2) * 16 + (e & 3);
+                        if (tok0 + t < P.n_tokens) {
+                            float v = S0[t * LD + col];
+#pragma unroll
+                            for (int k = 1; k < KW; k++) v += S0[k * (SET / 4) + t * LD + col];
+                            if (folded_in) v *= s_tok[t];
+                            if (R.bias_v) v += bias;
+                            _Float16 a, b;
+                            split_hi_lo(v, a, b);
+                            hi[e] = a; lo[e] = b;
+                        }
+                    }
+                    _Float16 *const V = reinterpret_cast<_Float16 *>(R.kv16 + ((long long)kvh * R.kv16_chunks + n0 / ATT_CH) * (Img::BYTES / 16)) + Img::K_HALVES;
+                    const int vo = Img::v_off(d, (n0 % ATT_CH) / 32 * 4 + (sg & 3));
+                    *reinterpret_cast<half8_t *>(V + vo) = hi;
+                    *reinterpret_cast<half8_t *>(V + 64 * Img::VS + vo) = lo;
+                }
+            }
         }
         return;
     }

@@ -77,6 +77,10 @@ struct QGemmParams {
         // rows cos / sin[pos[n]][hd / 2] and stream[n] * kv_stream_stride + pos[n] * hd -- so that no launch of a layer chases pos -> table
         const float *tcos, *tsin;            // [N][hd/2]
         const long long *tkv;                // [N]
+        // pgemm_kernel, a prompt from position 0, heads of 64: the layer's K and V^T also as attn_tile16_kernel's images (Kv16Image), [kv][kv16_chunks]
+        // (null: not)
+        uint4 *kv16;
+        int kv16_chunks;
     } rope;
     // RMSNorm (go/quant.go:597-607) folded around the GEMMs of a prompt (nl_pgemm.h).  A producer -- WO or down with
     // the plain epilogue, unsplit, so its lanes hold finished rows of the new residual stream -- also emits those rows
@@ -98,6 +102,28 @@ struct QGemmParams {
         const float *scale;  // the power of two the producer multiplied this token's fragments by (undone through inv); nullptr = 1
         float *scale_next;   // written by the workgroups of row block 0: the pre-scale of the NEXT producer, from this inv
     } nrm_in;
+};
+
+// LDS image of one 128-key chunk of one kv head, in halves: Kh | Kl [key][HD], then VTh | VTl [d][128].  Rows are not
+// padded; the 16-byte segments of a row are XOR-swizzled so that the kernel's ds_read_b128 are conflict-free.  A wave64
+// ds_read_b128 is serviced in four groups of 16 lanes -- {0-3,12-15,20-27}, {4-11,16-19,28-31} and the same + 32
+// (MI355X_MICROARCH.md, LDS) -- i.e. with lane = j + 16*kq every group holds each j once, half of them with segment s and
+// half with s ^ 1; the padded layouts of round 2 (rows of HD + 8 / 128 + 8 halves) put 7 of those 16 lanes on a busy
+// bank and every read took 8 LDS cycles instead of 4 (SQ_LDS_BANK_CONFLICT = 4 per ds_read_b128, measured).
+template <int HD> struct Kv16Image {
+    static constexpr int KS = HD;                   // K row: HD halves = HD/8 segments
+    static constexpr int VS = ATT_CH;               // V^T row: 128 halves = 16 segments = one 256-byte bank row
+    static constexpr int K_HALVES = 2 * ATT_CH * KS, V_HALVES = 2 * HD * VS;
+    static constexpr int K_BYTES = K_HALVES * 2, V_BYTES = V_HALVES * 2, BYTES = K_BYTES + V_BYTES;
+    static_assert(K_BYTES % 1024 == 0 && V_BYTES % 1024 == 0, "whole 1 KB LDS-DMA instructions");
+    // offset (halves) of segment `seg` (8 halves) of K row `row`: HD = 64: two rows per bank row, rows r and r + 2 differ
+    // by one segment; HD = 32: four rows per bank row
+    static __device__ __forceinline__ int k_off(int row, int seg) {
+        const int sw = HD == 64 ? ((row >> 1) & 7) : ((0 - (row >> 2)) & 3);
+        return row * KS + ((seg ^ sw) << 3);
+    }
+    // offset (halves) of segment `seg` (8 key positions) of V^T row d
+    static __device__ __forceinline__ int v_off(int d, int seg) { return d * VS + ((seg ^ (d & 15)) << 3); }
 };
 
 // Form of a fragment store, the sum of: the consumer's k-slot order is Q4_0's; an activation is three bf16 parts instead of fp16 hi + lo.

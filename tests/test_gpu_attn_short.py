@@ -38,3 +38,36 @@ def test_one_run_gives_the_bits_of_partials_and_merge(tmp_path, monkeypatch, hea
         for a, b in zip(got[False], got[True]):
             assert np.isfinite(a).all() and np.array_equal(a, b), (n, float(np.abs(a - b).max()))
     m.close()
+
+
+# The projections' launch leaves K and V^T as the attention's images, or a launch of its own converts the cache: the same bits.  Token tiles of 64 and 128 (the
+# last half of a chunk without a tile), one and two sets of wavefronts, 128 rows of the matrix (two heads), one to eight query heads a group; behind a
+# context the images are converted.
+@pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "f16"])
+@pytest.mark.parametrize("heads,kvs,lengths", [(4, 2, (256, 257, 319, 320, 321, 383, 384, 385, 449)), (8, 1, (260, 300)), (6, 2, (300, 400)), (4, 4, (512, 520)),
+                                               (8, 8, (1000,)), (24, 24, (1601,))])
+def test_images_from_the_projections(tmp_path, monkeypatch, heads, kvs, lengths, wtype):
+    from nanollama_amd import model
+    monkeypatch.setenv("NL_DGEMM", "0")                   # (short Q4_0 prompts otherwise)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("images", 2, heads * 64, heads, kvs, 128, seq_len=max(lengths) + 300, interm=256), wtype, 31)
+    m = model.load_llama_model(gguf.load_gguf(str(p)), max_streams=2)
+    toks = [int(t) for t in np.random.default_rng(7).integers(3, 128, size=max(lengths) + 300)]
+    for n in lengths:
+        got = {}
+        for knob in (False, True):
+            if knob:
+                monkeypatch.setenv("NL_KV16_LAUNCH", "1")
+            else:
+                monkeypatch.delenv("NL_KV16_LAUNCH", raising=False)
+            m.reset(0)
+            m.reset(1)
+            rows = []
+            for at, to in ((0, n), (n, n + 290)):
+                m.prefill(toks[at:to], at, 1)
+                rows.append(m.state.logits.copy())
+                assert int(m.debug_read("step_path", 1)[0]) & 16 == (16 if at == 0 and not knob else 0), (at, to, knob)
+            got[knob] = rows
+        for a, b in zip(got[False], got[True]):
+            assert np.isfinite(a).all() and np.array_equal(a, b), (n, float(np.abs(a - b).max()))
+    m.close()
