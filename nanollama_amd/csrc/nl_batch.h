@@ -48,10 +48,10 @@ __device__ __forceinline__ void gemm_out_at2(const GemmOut &g, long long ia, int
 // (go/model.go:552-554).  What brope_kv_kernel does per token, done per (token, kv head) by the consumer: one launch less
 // per layer.  Element e of a head sits at packed row (head * hd/16 + (e % half) / 8) * 16 + (e % half) % 8 + 8 * (e / half)
 // (ROWMAP_HEADPERM), its rotation partner at that row ^ 8.
-template <int HD, int G>
+template <int HD, int G, int NT>
 __device__ void attn_rope_prologue(const AttnParams &P, int kvh, int item, int pos, long long soff, float *qs, float *krow, float *vcur, bool kv_part) {
     constexpr int half = HD / 2, tph = HD / 16;
-    constexpr int NIT = ((G + 2) * HD + ATT_THREADS - 1) / ATT_THREADS;   // elements per thread
+    constexpr int NIT = ((G + 2) * HD + NT - 1) / NT;   // elements per thread
     const AttnParams::Rope &R = P.rp;
     const long long src0 = (long long)item * R.R;
     const int count = (kv_part ? G + 2 : G) * HD;
@@ -61,8 +61,8 @@ __device__ void attn_rope_prologue(const AttnParams &P, int kvh, int item, int p
     float v[NIT], partner[NIT], rc[NIT], rs[NIT];
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-        if (it * ATT_THREADS >= count) { v[it] = partner[it] = rc[it] = rs[it] = 0.f; continue; }   // (uniform: a q-only split has fewer elements)
-        const int i = min((int)threadIdx.x + it * ATT_THREADS, count - 1);
+        if (it * NT >= count) { v[it] = partner[it] = rc[it] = rs[it] = 0.f; continue; }   // (uniform: a q-only split has fewer elements)
+        const int i = min((int)threadIdx.x + it * NT, count - 1);
         const int hs = i / HD, e = i % HD, ih = e % half, hi = e / half;
         const int head = hs < G ? kvh * G + hs : hs == G ? R.n_q_heads + kvh : R.n_q_heads + P.n_kv_heads + kvh;
         const int rho = (head * tph + ih / 8) * 16 + (ih % 8) + 8 * hi;
@@ -76,7 +76,7 @@ __device__ void attn_rope_prologue(const AttnParams &P, int kvh, int item, int p
     }
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-        const int i = (int)threadIdx.x + it * ATT_THREADS;
+        const int i = (int)threadIdx.x + it * NT;
         if (i >= count) continue;
         const int hs = i / HD, e = i % HD, hi = e / half;
         float outv = v[it];
@@ -399,21 +399,14 @@ __global__ void brope_kv_kernel(BRopeParams P) {
 // FIN epilogue of attn_kernel (nl_kernels.h): the only split of every row is complete, so x = o / l -- the ns == 1
 // arithmetic of battn_merge_kernel -- goes straight into the WO GEMM's fragments.  One thread per 8 k-slots.
 template <int HD, int G>
-__device__ void attn_finalize(const AttnParams &P, const float *ored, const float *ml, int kvh, int item) {
-    constexpr int NG = ATT_THREADS / (HD / 4);
+__device__ void attn_finalize(const AttnParams &P, const float *sums, const float *ml, int kvh, int item) {
     const int tid = threadIdx.x;
     if (tid >= G * HD / 8) return;
     const int g = tid / (HD / 8), u = tid % (HD / 8), bl = u >> 2, w = u & 3;
     const float scale = 1.0f / ml[2 * g + 1];
     float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int d = bl * 32 + slot_elem(P.fin_form, w, j);
-        float s = 0.f;
-#pragma unroll 8
-        for (int k = 0; k < NG; k++) s += ored[(k * G + g) * HD + d];
-        v[j] = s * scale;
-    }
+    for (int j = 0; j < 8; j++) v[j] = sums[g * HD + bl * 32 + slot_elem(P.fin_form, w, j)] * scale;
     store_frag(P.fin_xf, P.fin_nt16, item, ((kvh * G + g) * HD) / 32 + bl, w, v, P.fin_form);
 }
 

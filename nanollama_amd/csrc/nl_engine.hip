@@ -519,51 +519,36 @@ GemvParams base_params(const nl_engine *e, const PackedMat &m, int mats = 1) {
     return P;
 }
 
-template <int HD>
-hipError_t launch_attn_hd(int gqa, AttnParams P, dim3 grid, hipStream_t st) {
+// Eight wavefronts shorten the phases of a workgroup that waits for its own round trips; where more than two workgroups share a compute unit the others' hide
+// them and four do as well with fewer barriers.  us a step, four and eight wavefronts: one stream of 841M Q8_0 at position 700 792 and 779, of 173M Q4_0 421 and 410;
+// 64 streams of 841M Q4_0 at 60 (384 workgroups) 1308 and 1273, at 200 (768) 1505 and 1526, at 900 (3072) 2227 and 2297; 24 of 841M Q8_0 at 200 (288) 1366 and
+// 1359, of 173M Q4_0 at 900 (576) 880 and 885.  (Eight heads: att_threads.)
+template <int HD, bool FIN, bool ROPE>
+hipError_t launch_attn_as(int gqa, AttnParams P, dim3 grid, int num_cus, hipStream_t st) {
+    const bool wide = (long long)grid.x * grid.y * grid.z <= 2ll * num_cus;
+    auto go = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        if (wide) hipLaunchKernelGGL((attn_kernel<HD, G, FIN, ROPE, att_threads(G)>), grid, dim3(att_threads(G)), 0, st, P);
+        else hipLaunchKernelGGL((attn_kernel<HD, G, FIN, ROPE, 256>), grid, dim3(256), 0, st, P);
+        return hipGetLastError();
+    };
     switch (gqa) {
-    case 1: hipLaunchKernelGGL((attn_kernel<HD, 1>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 2: hipLaunchKernelGGL((attn_kernel<HD, 2>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 3: hipLaunchKernelGGL((attn_kernel<HD, 3>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 4: hipLaunchKernelGGL((attn_kernel<HD, 4>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 8: hipLaunchKernelGGL((attn_kernel<HD, 8>), grid, dim3(ATT_THREADS), 0, st, P); break;
+    case 1: return go(std::integral_constant<int, 1>{});
+    case 2: return go(std::integral_constant<int, 2>{});
+    case 3: return go(std::integral_constant<int, 3>{});
+    case 4: return go(std::integral_constant<int, 4>{});
+    case 8: return go(std::integral_constant<int, 8>{});
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
-
-template <int HD>
-hipError_t launch_attn_fin_hd(int gqa, AttnParams P, dim3 grid, hipStream_t st) {
-    switch (gqa) {
-    case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 2: hipLaunchKernelGGL((attn_kernel<HD, 2, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 3: hipLaunchKernelGGL((attn_kernel<HD, 3, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 4: hipLaunchKernelGGL((attn_kernel<HD, 4, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 8: hipLaunchKernelGGL((attn_kernel<HD, 8, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+hipError_t launch_attn_fin(int hd, int gqa, AttnParams P, dim3 grid, int num_cus, hipStream_t st) {
+    return hd == 64 ? launch_attn_as<64, true, true>(gqa, P, grid, num_cus, st) : launch_attn_as<32, true, true>(gqa, P, grid, num_cus, st);
 }
-
-// several position splits per token with the RoPE prologue (decode batches at positions >= 128, AttnParams::rp)
-template <int HD>
-hipError_t launch_attn_rope_hd(int gqa, AttnParams P, dim3 grid, hipStream_t st) {
-    switch (gqa) {
-    case 1: hipLaunchKernelGGL((attn_kernel<HD, 1, false, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 2: hipLaunchKernelGGL((attn_kernel<HD, 2, false, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 3: hipLaunchKernelGGL((attn_kernel<HD, 3, false, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 4: hipLaunchKernelGGL((attn_kernel<HD, 4, false, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    case 8: hipLaunchKernelGGL((attn_kernel<HD, 8, false, true>), grid, dim3(ATT_THREADS), 0, st, P); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_attn(int hd, int gqa, AttnParams P, dim3 grid, hipStream_t st) {
-    if (P.rp.on) return hd == 64 ? launch_attn_rope_hd<64>(gqa, P, grid, st) : hd == 32 ? launch_attn_rope_hd<32>(gqa, P, grid, st) : hipErrorInvalidValue;
-    if (hd == 64) return launch_attn_hd<64>(gqa, P, grid, st);
-    if (hd == 32) return launch_attn_hd<32>(gqa, P, grid, st);
-    return hipErrorInvalidValue;
+// (several position splits per token with the RoPE prologue: decode batches at positions >= 128, AttnParams::rp)
+hipError_t launch_attn(int hd, int gqa, AttnParams P, dim3 grid, int num_cus, hipStream_t st) {
+    if (hd != 64 && hd != 32) return hipErrorInvalidValue;
+    if (P.rp.on) return hd == 64 ? launch_attn_as<64, false, true>(gqa, P, grid, num_cus, st) : launch_attn_as<32, false, true>(gqa, P, grid, num_cus, st);
+    return hd == 64 ? launch_attn_as<64, false, false>(gqa, P, grid, num_cus, st) : launch_attn_as<32, false, false>(gqa, P, grid, num_cus, st);
 }
 
 // developer knobs of the prompt attention, read ONCE per process and in one place: the workgroup list of batched_step
@@ -1017,7 +1002,7 @@ void build_plan(nl_engine *e, std::vector<Op> &plan, bool fused, bool help = fal
             dim3 grid(e->KVs, e->nsplit_max);
             int hd = e->hd, gqa = e->gqa;
             plan.push_back({K_ATTN, 0, nullptr, 0,
-                               [hd, gqa, P, grid](hipStream_t st) { return launch_attn(hd, gqa, P, grid, st); }});
+                               [hd, gqa, P, grid, cus = e->num_cus](hipStream_t st) { return launch_attn(hd, gqa, P, grid, cus, st); }});
         }
         }   // five-launch projection / attention
         {   // WO + residual (go/model.go:590-594); the prologue merges the attention splits
@@ -2235,14 +2220,13 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_form = form(L.wo);
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
-                LCK(hd == 64 ? launch_attn_fin_hd<64>(e->gqa, P, dim3(e->KVs, 1, n), st)
-                             : launch_attn_fin_hd<32>(e->gqa, P, dim3(e->KVs, 1, n), st));
+                LCK(launch_attn_fin(hd, e->gqa, P, dim3(e->KVs, 1, n), e->num_cus, st));
                 merged = true;
                 e->step_path |= PATH_ATTN_FIN;
             } else {
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
-                LCK(launch_attn(hd, e->gqa, P, dim3(e->KVs, nsplit, n), st));
+                LCK(launch_attn(hd, e->gqa, P, dim3(e->KVs, nsplit, n), e->num_cus, st));
             }
             if (!merged) {
             const bool tile16 = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;

@@ -28,7 +28,8 @@ constexpr int TR = 16;           // rows per tile
 constexpr int KL = 4;            // k-lanes per wavefront (64 / TR)
 constexpr int PAIR = 64;         // columns per pair
 constexpr int ATT_CH = 128;      // positions per attention split
-constexpr int ATT_THREADS = 256;
+// most threads of a workgroup of the decode attention, by query heads of a kv group: at eight heads the partial rows of 32 row groups no longer fit K's LDS
+constexpr int att_threads(int g) { return g <= 4 ? 512 : 256; }
 constexpr int CTL_TOKEN = 0, CTL_POS = 1, CTL_CHAIN = 2, CTL_STEP = 3, CTL_STREAM = 4, CTL_HOSTOUT = 5, CTL_WORDS = 8;
 
 // A word written by an EARLIER launch (ctl / epoch counters) read through the scalar cache: s_load_dword, counted on
@@ -1112,8 +1113,8 @@ struct AttnParams {
 };
 
 template <int HD, int G>
-__device__ void attn_finalize(const AttnParams &P, const float *ored, const float *ml, int kvh, int item);   // nl_batch.h
-template <int HD, int G>
+__device__ void attn_finalize(const AttnParams &P, const float *sums, const float *ml, int kvh, int item);   // nl_batch.h
+template <int HD, int G, int NT>
 __device__ void attn_rope_prologue(const AttnParams &P, int kvh, int item, int pos, long long soff, float *qs, float *krow, float *vcur, bool kv_part);   // nl_batch.h
 
 // GQA decode attention for one token (go/model.go:557-587): one workgroup per
@@ -1152,16 +1153,17 @@ __device__ long long g_attn_stamps[16];   // developer build (-DNL_ATTN_STAMPS):
 #else
 #define ATTN_STAMP(i) do { } while (0)
 #endif
-template <int HD, int G, bool FIN = false, bool ROPE = FIN>   // ROPE: the instantiation carries the RoPE prologue (AttnParams::rp)
-__global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
+template <int HD, int G, bool FIN, bool ROPE, int NT>   // ROPE: the instantiation carries the RoPE prologue (AttnParams::rp)
+__global__ void __launch_bounds__(NT) attn_kernel(AttnParams P) {
+    constexpr int NQ = NT / ATT_CH;
     ATTN_STAMP(0);
     const int split = blockIdx.y, t0 = split * ATT_CH;
     const int kvh = blockIdx.x, tid = threadIdx.x;
     constexpr int KS = HD + 4;               // padded row stride, 16-byte aligned: a lane reads its key's row as float4s and
                                              // consecutive rows sit one 16-byte slot apart (conflict-free ds_read_b128)
-    static_assert(ATT_THREADS == 2 * ATT_CH, "scores: thread = (key row, half of the group's heads)");
+    static_assert(NT % ATT_CH == 0, "scores: thread = (key row, share of the group's heads)");
     constexpr int R4 = HD / 4;               // float4 per row
-    constexpr int NG = ATT_THREADS / R4;     // row groups
+    constexpr int NG = NT / R4;              // row groups
     constexpr int NV = ATT_CH / NG;          // rows per thread
     // the per-row-group partial outputs (ored, written after the last read of the staged K) reuse K's storage when they fit:
     // 52 -> 37 KB of LDS for HD = 64, G = 4, i.e. four workgroups per CU instead of three -- at long contexts this kernel
@@ -1232,7 +1234,7 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
             // round trips per launch instead of one.  What the requests above return for row `pos` is discarded below.)
             if (P.rp.on) {
                 __builtin_amdgcn_sched_barrier(0);
-                attn_rope_prologue<HD, G>(P, kvh, item, pos, soff, qs, Kt + (pos - t0) * KS, vcur, pos - t0 < ATT_CH);
+                attn_rope_prologue<HD, G, NT>(P, kvh, item, pos, soff, qs, Kt + (pos - t0) * KS, vcur, pos - t0 < ATT_CH);
             }
         }
     }
@@ -1240,7 +1242,7 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
     const bool roped = ROPE && P.rp.on;      // q comes from the RoPE prologue above ...
     const int own = roped && pos - t0 < ATT_CH ? pos - t0 : -1;   // ... and so does this staged row of K / V (the step's own position)
     if (!roped)
-        for (int i = tid; i < G * HD; i += ATT_THREADS) qs[i] = qsrc[kvh * G * HD + i];
+        for (int i = tid; i < G * HD; i += NT) qs[i] = qsrc[kvh * G * HD + i];
 #pragma unroll
     for (int k = 0; k < NV; k++) {
         int row = tg + k * NG;
@@ -1258,30 +1260,31 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
     }
 
     ATTN_STAMP(2);
-    // scores: thread (key row t, half gp of the group's heads) -> q.k over d.  The row is read once, as float4s, for all the
-    // heads of the half; q is a broadcast read.  Per (t, g): four partial sums over d = 0, 4, 8, ... / 1, 5, ... / ..., the
+    // scores: thread (key row t, share gp of the group's heads) -> q.k over d.  The row is read once, as float4s, for all the
+    // heads of the share; q is a broadcast read.  Per (t, g): four partial sums over d = 0, 4, 8, ... / 1, 5, ... / ..., the
     // order the one-float-at-a-time loop of rounds 1-2 used (256 ds_read_b32 per thread against 48 ds_read_b128 now).
     {
-        constexpr int GH = (G + 1) / 2;
-        const int t = tid & (ATT_CH - 1), gp = tid >> 7;
-        if (t < n) {
+        constexpr int GH = (G + NQ - 1) / NQ;
+        const int t = tid & (ATT_CH - 1), gp = tid / ATT_CH;
+        if (t < n && gp * GH < G) {
             float d[GH][4];
 #pragma unroll
             for (int gi = 0; gi < GH; gi++) d[gi][0] = d[gi][1] = d[gi][2] = d[gi][3] = 0.f;
-            // (sixteen dims per round of LDS reads: one-float4-at-a-time left a dependent LDS round trip per step, 3.8k of a
+            // (sixteen dims per round of LDS reads, 32 of a single head: one-float4-at-a-time left a dependent LDS round trip per step, 3.8k of a
             // decode-batch launch's 15k cycles)
+            constexpr int DR = GH == 1 ? 8 : 4;
 #pragma unroll 1
-            for (int d0 = 0; d0 < HD; d0 += 16) {      // (not unrolled: hipcc otherwise hoists every round's reads -- 230+ registers)
-                float4 kv[4], qv[GH][4];
+            for (int d0 = 0; d0 < HD; d0 += 4 * DR) {      // (not unrolled: hipcc otherwise hoists every round's reads -- 230+ registers)
+                float4 kv[DR], qv[GH][DR];
 #pragma unroll
-                for (int u = 0; u < 4; u++) kv[u] = *reinterpret_cast<const float4 *>(Kt + t * KS + d0 + 4 * u);
+                for (int u = 0; u < DR; u++) kv[u] = *reinterpret_cast<const float4 *>(Kt + t * KS + d0 + 4 * u);
 #pragma unroll
                 for (int gi = 0; gi < GH; gi++)
 #pragma unroll
-                    for (int u = 0; u < 4; u++) qv[gi][u] = *reinterpret_cast<const float4 *>(qs + min(gp * GH + gi, G - 1) * HD + d0 + 4 * u);
+                    for (int u = 0; u < DR; u++) qv[gi][u] = *reinterpret_cast<const float4 *>(qs + min(gp * GH + gi, G - 1) * HD + d0 + 4 * u);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < 4; u++)
+                for (int u = 0; u < DR; u++)
 #pragma unroll
                     for (int gi = 0; gi < GH; gi++) {
                         d[gi][0] = fmaf(qv[gi][u].x, kv[u].x, d[gi][0]);
@@ -1302,7 +1305,7 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
     ATTN_STAMP(3);
     // softmax pieces per head: wave w handles heads w, w+4, ...
     const int wave = tid >> 6, lane = tid & 63;
-    for (int g = wave; g < G; g += ATT_THREADS / 64) {
+    for (int g = wave; g < G; g += NT / 64) {
         float s0 = lane < n ? sc[g * ATT_CH + lane] : -INFINITY;
         float s1 = lane + 64 < n ? sc[g * ATT_CH + lane + 64] : -INFINITY;
         float m = wave_max_f32(fmaxf(s0, s1));
@@ -1338,22 +1341,30 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnParams P) {
     for (int g = 0; g < G; g++) *reinterpret_cast<float4 *>(ored + (tg * G + g) * HD + c4 * 4) = o[g];
     __syncthreads();
     ATTN_STAMP(5);
-    if constexpr (FIN) {
-        attn_finalize<HD, G>(P, ored, ml, kvh, item);
-        ATTN_STAMP(6);
-        return;
-    }
-    for (int i = tid; i < G * HD; i += ATT_THREADS) {
-        int g = i / HD, dd = i % HD;
+    // the row groups' sums of a value, in order: NS threads each add a run of them (neighbouring lanes)
+    constexpr int NS = G * HD * 2 <= NT ? 2 : 1;
+    for (int i = tid; i < G * HD * NS; i += NT) {
+        const int part = i % NS, g = i / NS / HD, dd = i / NS % HD;
         float s = 0.f;
 #pragma unroll 8
-        for (int k = 0; k < NG; k++) s += ored[(k * G + g) * HD + dd];
+        for (int k = 0; k < NG / NS; k++) s += ored[((part * (NG / NS) + k) * G + g) * HD + dd];
+        if constexpr (NS == 2) s += dpp_f32<DPP_QUAD_XOR1>(s);
+        if (part) continue;
+        if constexpr (FIN) {
+            qs[g * HD + dd] = s;                 // (q has no reader left)
+            continue;
+        }
         int h = kvh * G + g;
         part_o[((long long)h * P.nsplit_max + split) * HD + dd] = s;
         if (dd == 0) {
             part_ml[((long long)h * P.nsplit_max + split) * 2] = ml[2 * g];
             part_ml[((long long)h * P.nsplit_max + split) * 2 + 1] = ml[2 * g + 1];
         }
+    }
+    if constexpr (FIN) {
+        __syncthreads();
+        attn_finalize<HD, G>(P, qs, ml, kvh, item);
+        ATTN_STAMP(6);
     }
 }
 

@@ -71,3 +71,27 @@ def test_images_from_the_projections(tmp_path, monkeypatch, heads, kvs, lengths,
         for a, b in zip(got[False], got[True]):
             assert np.isfinite(a).all() and np.array_equal(a, b), (n, float(np.abs(a - b).max()))
     m.close()
+
+
+# Decode batches around two workgroups a compute unit, where the attention's workgroups go from eight wavefronts to four: one split (fragments from the launch)
+# and two, one to eight query heads a group, against each stream by itself.
+@pytest.mark.parametrize("heads,kvs,at", [(9, 9, 40), (9, 9, 130), (18, 9, 131), (36, 9, 45), (27, 9, 129), (72, 9, 140)])
+def test_decode_batches_of_many_workgroups(tmp_path, heads, kvs, at):
+    from nanollama_amd import model
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("batch", 1, heads * 32, heads, kvs, 128, seq_len=192, interm=256), "q8_0", 43)
+    m = model.load_llama_model(gguf.load_gguf(str(p)), max_streams=64)
+    toks = np.random.default_rng(9).integers(3, 128, size=(64, at + 1))
+    for s in range(64):
+        m.prefill([int(t) for t in toks[s, :at]], 0, s, want_logits=False)
+    edge = 512 // kvs // (1 if at < 128 else 2)
+    alone = []
+    for s in (0, edge - 1, edge):
+        m.forward(int(toks[s, at]), at, s)
+        alone.append(m.state.logits.copy())
+    for n in (edge, edge + 1):                             # at most two workgroups a compute unit, and more
+        _, rows = m.forward_batch(list(range(n)), [int(t) for t in toks[:n, at]], [at] * n, want_logits=True)
+        for s, want in zip((0, edge - 1, edge), alone):
+            if s < n:
+                assert np.isfinite(rows[s]).all() and np.abs(rows[s] - want).max() <= 1e-4 * max(1.0, float(want.std())), (n, s)
+    m.close()
