@@ -81,9 +81,10 @@ __device__ __forceinline__ float rsqrt_f32(float x) { return __builtin_amdgcn_rs
 // (past 88.72 the exponential is no float32; v_rcp_f32 leaves 0 below 2^-126, from 87.3 on)
 __device__ __forceinline__ float sigmoid_f32(float z) { return rcp_f32(1.f + exp_f32(__builtin_amdgcn_fmed3f(-z, -88.72f, 88.72f))); }
 __device__ __forceinline__ float silu_f32(float z) { return z * sigmoid_f32(z); }
+__device__ __forceinline__ float gelu_arg(float z) { return z * fmaf(0.071354816f, z * z, 1.5957691216057308f); }
 __device__ __forceinline__ float gelu_tanh_f32(float z) {
     // 0.5 (1 + tanh u) = sigmoid(2 u)
-    return z * sigmoid_f32(z * fmaf(0.071354816f, z * z, 1.5957691216057308f));
+    return z * sigmoid_f32(gelu_arg(z));
 }
 template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
     return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -571,7 +572,10 @@ __device__ __forceinline__ void store_gated(const MatParams &P, int tok, int f16
         gate += *reinterpret_cast<const f32x4 *>(P.bias + f16 * 16 + 4 * g);
         up += *reinterpret_cast<const f32x4 *>(P.bias2 + f16 * 16 + 4 * g);
     }
-    put4(reinterpret_cast<T *>(P.act) + op_index(tok, f16 * 16 + 4 * g, P.act_nks), P.act_silu ? gated<true>(gate, up) : gated<false>(gate, up));
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = gate[i] * sigmoid_f32(P.act_silu ? gate[i] : gelu_arg(gate[i])) * up[i];
+    put4(reinterpret_cast<T *>(P.act) + op_index(tok, f16 * 16 + 4 * g, P.act_nks), v);
 }
 
 __device__ __forceinline__ f32x4 with_bias(const float *bias, int row, f32x4 v) {
