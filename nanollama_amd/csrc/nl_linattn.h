@@ -104,59 +104,80 @@ __global__ void __launch_bounds__(256) gla_decay_kernel(GlaParams P) {
 }
 
 // grid (segments, heads), max(dvp, dkp) / 16 wavefronts; wavefront w < dvp / 16 owns value columns 16 w .. 16 w + 15, all of them load.
-// The next sub-chunk's operands are requested before the current one is multiplied.
-// NE: operand elements per thread, at least 16 dkp / threads (at most 4); WV: most wavefronts of a launch
+// NE: operand elements per thread and sub-chunk, at least 16 dkp / threads (at most 4); WV: most wavefronts of a launch.
+// What a workgroup spends is spread: matrix products (36 of 32 cycles per sub-chunk, wavefront and 64 channels, in float32), exponentials, sums over the
+// value columns, and the wavefronts meeting.  The outputs of a head of at most 64 channels therefore take a whole segment a step: A's shared out over the
+// wavefronts at once, S through all sub-chunks without a barrier, one meeting for all norms (three barriers a segment where a sub-chunk a step has
+// twelve); more channels have no registers for it, and the increments, which meet once a sub-chunk, are faster with the next sub-chunk's operands requested
+// before the current one is multiplied (12.5 us, a whole segment at once 13.9).  Addresses are minima of byte offsets and the sums over 16 lanes are
+// row operations.  The outputs of 2047 tokens, 64 channels, 128 values: twelve heads 32.5 -> 28.8 us, six 23.8 -> 18.4; that 384 workgroups are two for
+// half of the 256 compute units is the difference between the two.
+constexpr int la_subs(int dkt, int wv, bool out) { return out && wv <= 8 && dkt <= 4 ? LA_SEG / LA_SUB : 1; }   // sub-chunks a step
+__host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * subs ? 4 : nw >= 2 * subs ? 2 : 1; }   // wavefronts that share one A
+__host__ __device__ constexpr int la_ldk(int dkp) { return (dkp >> 4) & 1 ? dkp : dkp + 16; }   // rows g of k e^{l_end - l} in other banks
+__host__ __device__ inline size_t gla_seg_lds(int dkp, int nw, int subs, bool out) {
+    const int rows = subs * LA_SUB;
+    return (size_t)(rows * la_ldk(dkp) + subs * dkp + (out ? 2 * rows * (dkp + 4) + subs * la_parts(subs, nw) * 256 + nw * rows + 16 : 0)) * 4;
+}
+
 template <typename T, int DKT, int NE, int WV, bool OUT>
-__global__ void __launch_bounds__(WV * 64) gla_seg_kernel(GlaParams P) {
+__global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_kernel(GlaParams P) {
     extern __shared__ __align__(16) char lds[];
+    constexpr int SUBS = la_subs(DKT, WV, OUT), ROWS = SUBS * LA_SUB;
     const GlaSeg sg = P.segs[blockIdx.x];
     if (!OUT && (sg.nseg == 1 || sg.index + 1 == sg.nseg)) return;     // nobody starts from the state behind the last segment
     const int h = blockIdx.y, tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, w = tid >> 6, nw = nthr >> 6, g = lane >> 4, c = lane & 15;
-    const int dk = P.dk, dkp = P.dkp, nkt = dkp >> 4, ld = dkp + 4, C = P.heads * dk, dvc = w * 16 + c;
-    const int nv = P.dvp >> 4;
+    const int dk = P.dk, dkp = P.dkp, nkt = dkp >> 4, ld = dkp + 4, ldk = la_ldk(dkp), C = P.heads * dk, dvc = w * 16 + c;
+    const int nv = P.dvp >> 4, np = la_parts(SUBS, nw);
     const bool owner = w < nv, value = dvc < P.dv;
-    float *qd = reinterpret_cast<float *>(lds);          // [16][ld]  q e^l
-    float *ki = qd + 16 * ld;                            // [16][ld]  k e^-l
-    float *ke = ki + 16 * ld;                            // [16][ld]  k e^{l_end - l}
-    float *etot = ke + 16 * ld;                          // [dkp]     e^{l_end}
-    float *A = etot + dkp;                                // [16][20]
-    float *ssq = A + 16 * 20;                            // [nw][16] sums of squares
-    int *flag = reinterpret_cast<int *>(ssq + nw * 16);  // [16] wavefront saw a decay beyond the factored range
-    float *part = ssq + nw * 16 + 16;                    // [nw][256] partial A
+    float *ke = reinterpret_cast<float *>(lds);          // [ROWS][ldk] k e^{l_end - l}
+    float *etot = ke + ROWS * ldk;                       // [SUBS][dkp] e^{l_end}
+    float *qd = etot + SUBS * dkp;                       // [ROWS][ld]  q e^l
+    float *ki = qd + ROWS * ld;                          // [ROWS][ld]  k e^-l
+    float *part = ki + ROWS * ld;                        // [SUBS][np][256] partial A
+    float *ssq = part + SUBS * np * 256;                 // [nw][ROWS] sums of squares
+    int *flag = reinterpret_cast<int *>(ssq + nw * ROWS);  // [16] sub-chunks in which the wavefront saw a decay beyond the factored range
     f32x4 S[DKT];
     const long long shead = (long long)dkp * P.dvp;
     float *stream_state = P.state + sg.stream * P.state_stride + h * shead;
     float *seg_state = P.inc + ((long long)blockIdx.x * P.heads + h) * shead;
-    const int nsub = (sg.len + LA_SUB - 1) / LA_SUB;
-    float rq[NE], rk[NE], rl[NE], re[NE], rv[4], rg[4];
+    float rq[SUBS][NE], rk[SUBS][NE], rl[SUBS][NE], re[SUBS][NE], rv[SUBS][4];
     int et[NE], ed[NE];                                  // this thread's elements: token of the sub-chunk (16: none), channel
+    int lk[NE], lq[NE];
+    unsigned ep[NE], el[NE];                             // and where they lie: row t of the projections and of ldec; (t, d) of the LDS images
 #pragma unroll
     for (int e = 0; e < NE; e++) {
         const int i = tid + e * nthr;
         et[e] = min(i / dkp, LA_SUB);
         ed[e] = i - i / dkp * dkp;
+        ep[e] = (unsigned)(et[e] * P.ldp) * 4u;
+        el[e] = (unsigned)(et[e] * C) * 4u;
+        lk[e] = et[e] * ldk + ed[e];
+        lq[e] = et[e] * ld + ed[e];
     }
+    const unsigned vrow = (unsigned)(g * P.ldp) * 4u, grow = 4 * vrow, prow = P.ldp * 4u;
+    const unsigned vcol = (unsigned)(h * P.dv + min(dvc, P.dv - 1)) * 4u;
     const char *proj = reinterpret_cast<const char *>(P.proj + (long long)sg.tok0 * P.ldp), *ldec = reinterpret_cast<const char *>(P.ldec + (long long)sg.tok0 * C + h * dk);
-    auto fetch = [&](int sub) {
-        const int u0 = sub * LA_SUB, len = min(LA_SUB, sg.len - u0);
+    // (every address is clamped into the segment and the row, so that no load waits in a branch; what lies beyond is dropped below.  Row offsets are
+    //  minima of byte offsets: a product per load costs four times an addition)
+    auto fetch = [&](int u0) {
+        const int last = sg.len - 1;
+        const unsigned plast = last * prow;
 #pragma unroll
-        for (int e = 0; e < NE; e++) {
-            rq[e] = rk[e] = rl[e] = re[e] = 0.f;
-            if (et[e] < LA_SUB && ed[e] < dk) {
-                re[e] = ld_off<float>(ldec, (unsigned)((u0 + len - 1) * C + ed[e]) * 4u);
-                if (et[e] < len) {
-                    const unsigned at = (unsigned)((u0 + et[e]) * P.ldp + h * dk + ed[e]);
-                    rk[e] = ld_off<float>(proj, (at + P.off_k) * 4u);
-                    rl[e] = ld_off<float>(ldec, (unsigned)((u0 + et[e]) * C + ed[e]) * 4u);
-                    if (OUT) rq[e] = ld_off<float>(proj, (at + P.off_q) * 4u);
-                }
+        for (int s = 0; s < SUBS; s++) {
+            const int us = u0 + s * LA_SUB, end = min(us + LA_SUB - 1, last);
+            const unsigned pend = end * prow, lend = (unsigned)(end * C) * 4u, p0 = us * prow, l0 = (unsigned)(us * C) * 4u;
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const unsigned d = (unsigned)min(ed[e], dk - 1) * 4u, at = min(ep[e] + p0, pend) + h * dk * 4u + d;
+                rk[s][e] = ld_off<float>(proj + P.off_k * 4ll, at);
+                rl[s][e] = ld_off<float>(ldec, min(el[e] + l0, lend) + d);
+                re[s][e] = ld_off<float>(ldec, lend + d);
+                if (OUT) rq[s][e] = ld_off<float>(proj + P.off_q * 4ll, at);
             }
-        }
-        // value columns in B-operand order: step s holds token 4 s + g; the gates in accumulator order: token 4 g + i
+            // value columns in B-operand order: step i holds token 4 i + g
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            rv[s] = owner && value && 4 * s + g < len ? ld_off<float>(proj, (unsigned)((u0 + 4 * s + g) * P.ldp + P.off_v + h * P.dv + dvc) * 4u) : 0.f;
-            if (OUT) rg[s] = owner && value && 4 * g + s < len ? ld_off<float>(proj, (unsigned)((u0 + 4 * g + s) * P.ldp + P.off_g + h * P.dv + dvc) * 4u) : 0.f;
+            for (int i = 0; i < 4; i++) rv[s][i] = ld_off<float>(proj + P.off_v * 4ll, min(vrow + p0 + 4 * i * prow, plast) + vcol);
         }
     };
     fetch(0);
@@ -173,130 +194,157 @@ __global__ void __launch_bounds__(WV * 64) gla_seg_kernel(GlaParams P) {
     const float inv_dv = 1.f / (float)P.dv;
     const int ycol = (int)op_index(0, P.y_k0 + h * P.dv + dvc, P.y_nks);
     const float nrm = OUT && value ? P.norm[dvc] * P.oscale : 0.f;
-    for (int sub = 0; sub < nsub; sub++) {
-        const int t0 = sg.tok0 + sub * LA_SUB, len = min(LA_SUB, sg.len - sub * LA_SUB);
-        // operands of the sub-chunk; tokens beyond its length and channels beyond dk are zero
-        bool strong = false;
+    float tot = 0.f;                                     // thread d < dkp: channel d's log decay up to here
+    for (int u0 = 0; u0 < sg.len; u0 += ROWS) {
+        const int left = sg.len - u0;                    // tokens from this step's first on
+        if (ROWS < LA_SEG && u0) lds_barrier();          // the step before has been read
+        // the step's operands; tokens beyond its length and channels beyond dk are zero
+        int strong = 0;
+        float v[SUBS][4];
 #pragma unroll
-        for (int e = 0; e < NE; e++) {
-            const int t = et[e], d = ed[e];
-            if (t < LA_SUB) {
-                ke[t * ld + d] = rk[e] * exp_f32(re[e] - rl[e]);
-                if (OUT) {
-                    strong |= re[e] < -LA_FACTOR_MAX;
-                    qd[t * ld + d] = rq[e] * P.qscale * exp_f32(rl[e]);
-                    ki[t * ld + d] = rk[e] * exp_f32(fminf(-rl[e], LA_FACTOR_MAX));
+        for (int s = 0; s < SUBS; s++) {
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                const int t = et[e], d = ed[e], row = s * LA_SUB + t, ak = s * LA_SUB * ldk + lk[e], aq = s * LA_SUB * ld + lq[e];
+                const bool chan = d < dk && s * LA_SUB < left, live = d < dk && row < left;
+                const float l = live ? rl[s][e] : 0.f, end = chan ? re[s][e] : 0.f, k = live ? rk[s][e] : 0.f;
+                if (t < LA_SUB) {
+                    ke[ak] = k * exp_f32(end - l);
+                    if (OUT) {
+                        strong |= end < -LA_FACTOR_MAX ? 1 << s : 0;
+                        qd[aq] = (live ? rq[s][e] : 0.f) * P.qscale * exp_f32(l);
+                        ki[aq] = k * exp_f32(fminf(-l, LA_FACTOR_MAX));
+                    }
+                    if (t == 0) {
+                        etot[s * dkp + d] = exp_f32(end);
+                        tot += end;                      // (only e == 0 has t == 0: nthr >= 4 dkp)
+                    }
                 }
-                if (t == 0) etot[d] = exp_f32(re[e]);
             }
-        }
-        float v[4], gz[4];
 #pragma unroll
-        for (int s = 0; s < 4; s++) { v[s] = rv[s]; gz[s] = rg[s]; }
+            for (int i = 0; i < 4; i++) v[s][i] = value && s * LA_SUB + 4 * i + g < left ? rv[s][i] : 0.f;
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (OUT) {
-            const bool any = __any(strong);
+            int any = 0;
+#pragma unroll
+            for (int s = 0; s < SUBS; s++) any |= __any(strong >> s & 1) ? 1 << s : 0;
             if (lane == 0) flag[w] = any;
         }
         lds_barrier();
-        if (sub + 1 < nsub) fetch(sub + 1);
-        bool slow = false;
-        if (OUT)
-            for (int q = 0; q < nw; q++) slow |= flag[q] != 0;
-        f32x4 o = {};
+        if (ROWS < LA_SEG && u0 + ROWS < sg.len) fetch(u0 + ROWS);
         if (OUT) {
-            if (!slow) {
+            int slow = 0;
+            for (int q = 0; q < nw; q++) slow |= flag[q];
+            for (int task = w; task < SUBS * np; task += nw) {
+                const int s = task % SUBS, p = task / SUBS;
+                if (slow >> s & 1) continue;
                 f32x4 a = {};
-                for (int ks = w; ks < dkp / 4; ks += nw)
-                    a = __builtin_amdgcn_mfma_f32_16x16x4f32(qd[c * ld + 4 * ks + g], ki[c * ld + 4 * ks + g], a, 0, 0, 0);
+                for (int ks = p; ks < dkp / 4; ks += np)
+                    a = __builtin_amdgcn_mfma_f32_16x16x4f32(qd[(s * LA_SUB + c) * ld + 4 * ks + g], ki[(s * LA_SUB + c) * ld + 4 * ks + g], a, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) part[w * 256 + (4 * g + i) * 16 + c] = a[i];
+                for (int i = 0; i < 4; i++) part[(s * np + p) * 256 + (4 * g + i) * 16 + c] = a[i];
             }
-            if (owner) {
-#pragma unroll
-                for (int dt = 0; dt < DKT; dt++)
-                    if (dt < nkt) {
-                        const f32x4 qv = *reinterpret_cast<const f32x4 *>(qd + c * ld + dt * 16 + 4 * g);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i], S[dt][i], o, 0, 0, 0);
-                    }
-            }
-        }
-        if (owner) {
-#pragma unroll
-            for (int dt = 0; dt < DKT; dt++)
-                if (dt < nkt) {
-                    const f32x4 tl = *reinterpret_cast<const f32x4 *>(etot + dt * 16 + 4 * g);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) S[dt][i] *= tl[i];
-#pragma unroll
-                    for (int s = 0; s < 4; s++) S[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ke[(4 * s + g) * ld + dt * 16 + c], v[s], S[dt], 0, 0, 0);
-                }
-        }
-        lds_barrier();
-        if (OUT) {
-            for (int i = tid; i < 256; i += nthr) {
-                const int t = i >> 4, s = i & 15;
-                float a = 0.f;
-                if (s <= t && t < len) {
-                    if (!slow) {
-                        const int np = min(nw, dkp / 4);
-                        for (int q0 = 0; q0 < np; q0 += 8) {
-                            float x[8];
-#pragma unroll
-                            for (int q = 0; q < 8; q++) x[q] = part[min(q0 + q, np - 1) * 256 + i];
-#pragma unroll
-                            for (int q = 0; q < 8; q++) a += q0 + q < np ? x[q] : 0.f;
-                        }
-                    } else {
+            if (slow)
+                for (int i = tid; i < SUBS * 256; i += nthr) {
+                    const int sub = i >> 8, t = i >> 4 & 15, s = i & 15;
+                    if (!(slow >> sub & 1)) continue;
+                    float a = 0.f;
+                    if (s <= t && sub * LA_SUB + t < left) {
+                        const int t0 = sg.tok0 + u0 + sub * LA_SUB;
                         const float *qp = P.proj + (long long)(t0 + t) * P.ldp + P.off_q + h * dk, *kp = P.proj + (long long)(t0 + s) * P.ldp + P.off_k + h * dk;
                         const float *lt = P.ldec + (long long)(t0 + t) * C + h * dk, *ls = P.ldec + (long long)(t0 + s) * C + h * dk;
 #pragma unroll 1
                         for (int d = 0; d < dk; d++) a += qp[d] * P.qscale * kp[d] * exp_f32(lt[d] - ls[d]);
                     }
+                    for (int p = 0; p < np; p++) part[(sub * np + p) * 256 + (i & 255)] = p == 0 ? a : 0.f;
                 }
-                A[t * 20 + s] = a;
-            }
             lds_barrier();
+        }
+        f32x4 o[SUBS];
+        float gz[SUBS][4];                               // gates, in accumulator order: token 4 g + i
+        if (OUT)
 #pragma unroll
-            for (int s = 0; s < 4; s++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(A[c * 20 + 4 * s + g], v[s], o, 0, 0, 0);
-            // norm over the head's value columns: sums of squares over 16 lanes, then over the wavefronts
+            for (int s = 0; s < SUBS; s++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float ss = o[i] * o[i];
+                for (int i = 0; i < 4; i++) gz[s][i] = ld_off<float>(proj + P.off_g * 4ll, min(grow + (u0 + s * LA_SUB + i) * prow, (sg.len - 1) * prow) + vcol);
+        if (owner) {
 #pragma unroll
-                for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m);
-                if (c == 0) ssq[w * 16 + 4 * g + i] = ss;
+            for (int s = 0; s < SUBS; s++) {
+                __builtin_amdgcn_sched_barrier(0);       // (or the scheduler holds the next one's operands too, and half the wavefronts fit)
+                o[s] = f32x4{};
+                if (s * LA_SUB < left) {
+                    if (OUT) {
+#pragma unroll
+                        for (int dt = 0; dt < DKT; dt++)
+                            if (dt < nkt) {
+                                const f32x4 qv = *reinterpret_cast<const f32x4 *>(qd + (s * LA_SUB + c) * ld + dt * 16 + 4 * g);
+#pragma unroll
+                                for (int i = 0; i < 4; i++) o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[i], S[dt][i], o[s], 0, 0, 0);
+                            }
+                        float a[4];                      // row c, columns 4 i + g of A: nothing flows back in time
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const float *pa = part + s * np * 256 + c * 16 + 4 * i + g;
+                            float x = pa[0];
+                            for (int p = 1; p < np; p++) x += pa[p * 256];
+                            a[i] = 4 * i + g <= c ? x : 0.f;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], v[s][i], o[s], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int dt = 0; dt < DKT; dt++)
+                        if (dt < nkt) {
+                            const f32x4 tl = *reinterpret_cast<const f32x4 *>(etot + s * dkp + dt * 16 + 4 * g);
+#pragma unroll
+                            for (int i = 0; i < 4; i++) S[dt][i] *= tl[i];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) S[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ke[(s * LA_SUB + 4 * i + g) * ldk + dt * 16 + c], v[s][i], S[dt], 0, 0, 0);
+                        }
+                }
             }
+        }
+        if (OUT) {
+            // norm over the head's value columns: sums of squares over 16 lanes, then over the wavefronts
+            if (owner)
+#pragma unroll
+                for (int s = 0; s < SUBS; s++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float ss = o[s][i] * o[s][i];
+                        ss += dpp_f32<DPP_QUAD_XOR1>(ss);
+                        ss += dpp_f32<DPP_QUAD_XOR2>(ss);
+                        ss += dpp_f32<DPP_HALF_MIRROR>(ss);
+                        ss += dpp_f32<DPP_ROW_MIRROR>(ss);
+                        if (c == 0) ssq[w * ROWS + s * LA_SUB + 4 * g + i] = ss;
+                    }
             lds_barrier();
             T *y = reinterpret_cast<T *>(P.y);
-            f32x4 s2 = {};
-            for (int q0 = 0; q0 < nv; q0 += 4) {
-                f32x4 x[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const f32x4 *>(ssq + min(q0 + q, nv - 1) * 16 + 4 * g);
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (q0 + q < nv) s2 += x[q];
-            }
             if (owner && value)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int t = 4 * g + i;
-                    if (t < len) {
-                        put(y + (unsigned)(((t0 + t) >> 4) * P.y_nks * OPT + ((t0 + t) & 15) * 8 + ycol), o[i] * rsqrt_f32(s2[i] * inv_dv + P.eps) * nrm * (gz[i] * sigmoid_f32(gz[i])));
+                for (int s = 0; s < SUBS; s++) {
+                    if (s * LA_SUB >= left) continue;
+                    f32x4 s2 = {};
+                    for (int q0 = 0; q0 < nv; q0 += 4) {
+                        f32x4 x[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const f32x4 *>(ssq + min(q0 + q, nv - 1) * ROWS + s * LA_SUB + 4 * g);
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            if (q0 + q < nv) s2 += x[q];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int row = s * LA_SUB + 4 * g + i, t = sg.tok0 + u0 + row;
+                        if (row < left)
+                            put(y + (unsigned)((t >> 4) * P.y_nks * OPT + (t & 15) * 8 + ycol), o[s][i] * rsqrt_f32(s2[i] * inv_dv + P.eps) * nrm * (gz[s][i] * sigmoid_f32(gz[s][i])));
                     }
                 }
         }
+        if (ROWS >= LA_SEG) break;                       // (a segment is one step; a loop would keep its operands)
     }
-    if (!OUT) {
-        // the segment's total log decay (every channel by one thread, from the sub-chunks' ends)
-        for (int d = tid; d < dkp; d += nthr) {
-            float a = 0.f;
-            if (d < dk)
-                for (int sub = 0; sub < nsub; sub++) a += P.ldec[(long long)(sg.tok0 + min(sub * LA_SUB + LA_SUB, sg.len) - 1) * C + h * dk + d];
-            P.totlog[((long long)blockIdx.x * P.heads + h) * dkp + d] = a;
-        }
-    }
+    if (!OUT && tid < dkp) P.totlog[((long long)blockIdx.x * P.heads + h) * dkp + tid] = tot;      // (channels beyond dk: zero)
     if (owner && (!OUT || sg.index + 1 == sg.nseg)) {
         float *to = OUT ? stream_state : seg_state;
 #pragma unroll
@@ -416,8 +464,8 @@ __device__ __forceinline__ void gla_decode_block(const GlaParams &P, int h, int 
 template <typename T, bool OUT>
 hipError_t launch_gla_seg(const GlaParams &P, int nsegs, hipStream_t st) {
     const int nw = std::max(P.dvp, P.dkp) / 16;
-    const size_t lds = (size_t)(3 * 16 * (P.dkp + 4) + P.dkp + 16 * 20 + nw * 16 + 16 + nw * 256) * 4;
-    auto go = [&](auto kfn) {
+    auto go = [&](auto kfn, int subs) {
+        const size_t lds = gla_seg_lds(P.dkp, nw, subs, OUT);
         if (lds > 65536)
             if (hipError_t s = hipFuncSetAttribute(reinterpret_cast<const void *>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) return s;
         hipLaunchKernelGGL(kfn, dim3(nsegs, P.heads), dim3(nw * 64), lds, st, P);
@@ -425,11 +473,11 @@ hipError_t launch_gla_seg(const GlaParams &P, int nsegs, hipStream_t st) {
     };
     if (nw <= 8) {
         const bool two = 16 * P.dkp <= 2 * nw * 64;
-        if (P.dkp <= 64) return two ? go(gla_seg_kernel<T, 4, 2, 8, OUT>) : go(gla_seg_kernel<T, 4, 4, 8, OUT>);
-        return go(gla_seg_kernel<T, 8, 4, 8, OUT>);        // nw <= 8: dkp <= 128
+        if (P.dkp <= 64) return two ? go(gla_seg_kernel<T, 4, 2, 8, OUT>, la_subs(4, 8, OUT)) : go(gla_seg_kernel<T, 4, 4, 8, OUT>, la_subs(4, 8, OUT));
+        return go(gla_seg_kernel<T, 8, 4, 8, OUT>, la_subs(8, 8, OUT));     // nw <= 8: dkp <= 128
     }
-    if (P.dkp <= 128) return go(gla_seg_kernel<T, 8, 4, 16, OUT>);
-    return go(gla_seg_kernel<T, 16, 4, 16, OUT>);
+    if (P.dkp <= 128) return go(gla_seg_kernel<T, 8, 4, 16, OUT>, la_subs(8, 16, OUT));
+    return go(gla_seg_kernel<T, 16, 4, 16, OUT>, la_subs(16, 16, OUT));
 }
 
 // the recurrence of a ragged step: runs = streams' token runs with more than one segment (their first segments in P.runs)

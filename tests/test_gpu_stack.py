@@ -362,6 +362,25 @@ def test_decays_from_none_to_total(bias, dtype):
     m.close()
 
 
+@pytest.mark.parametrize("dim,vdim", [(16, 16), (20, 60), (64, 128), (40, 144), (128, 70), (250, 40)])
+@pytest.mark.parametrize("n", [15, 49, 64, 65, 145])
+def test_subchunks_within_and_beyond_the_factored_range(dim, vdim, n):
+    """Decays of about e^-40 a sub-chunk: of a segment's four some take the factored product and some the exponent per pair; heads of one to sixteen
+    wavefronts, whose shares of a product differ, and prompts that end inside and at the end of a sub-chunk and of a segment."""
+    cfg = config([gla(heads=2, dim=dim, vdim=vdim, tau=1.0)])
+    w = floats(weights(cfg, 5))
+    w["l0.mix.a2.b"] = w["l0.mix.a2.b"] * 0.02 - 2.5
+    w["l0.mix.a2.b"][::3] = 6.0
+    w = bits(w)
+    ids = tokens(n, seed=n)
+    want = so.forward(cfg, floats(w), ids)
+    m = load(cfg, w, "float32")
+    assert rel(whole(m, ids), want) < F32_TOL
+    m.step([(1, ids[:-1], 0, [])])                         # and the state behind it
+    assert rel(by_token(m, ids[-1:], 1, n - 1), want[-1:]) < F32_TOL
+    m.close()
+
+
 def test_state_carries_the_first_token():
     """A state that barely decays: the first token's mark is there hundreds of tokens later, whatever lies between."""
     cfg = config([gla(heads=1, dim=16, vdim=16, tau=64.0)])
