@@ -117,7 +117,7 @@ __host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * 
 __host__ __device__ constexpr int la_ldk(int dkp) { return (dkp >> 4) & 1 ? dkp : dkp + 16; }   // rows g of k e^{l_end - l} in other banks
 __host__ __device__ inline size_t gla_seg_lds(int dkp, int nw, int subs, bool out) {
     const int rows = subs * LA_SUB;
-    return (size_t)(rows * la_ldk(dkp) + subs * dkp + (out ? 2 * rows * (dkp + 4) + subs * la_parts(subs, nw) * 256 + nw * rows + 16 : 0)) * 4;
+    return (size_t)(rows * la_ldk(dkp) + subs * dkp + (out ? 2 * rows * (dkp + 4) + subs * la_parts(subs, nw) * 256 + 16 : 0)) * 4;
 }
 
 template <typename T, int DKT, int NE, int WV, bool OUT>
@@ -135,8 +135,8 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
     float *qd = etot + SUBS * dkp;                       // [ROWS][ld]  q e^l
     float *ki = qd + ROWS * ld;                          // [ROWS][ld]  k e^-l
     float *part = ki + ROWS * ld;                        // [SUBS][np][256] partial A
-    float *ssq = part + SUBS * np * 256;                 // [nw][ROWS] sums of squares
-    int *flag = reinterpret_cast<int *>(ssq + nw * ROWS);  // [16] sub-chunks in which the wavefront saw a decay beyond the factored range
+    float *ssq = ki;                                     // [nw][ROWS] sums of squares, once the A's are made
+    int *flag = reinterpret_cast<int *>(part + SUBS * np * 256);  // [16] sub-chunks in which the wavefront saw a decay beyond the factored range
     f32x4 S[DKT];
     const long long shead = (long long)dkp * P.dvp;
     float *stream_state = P.state + sg.stream * P.state_stride + h * shead;
