@@ -173,7 +173,7 @@ enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 // Q4_0 prompts (block scales multiplied into the fp16 weights, only the hi half of every activation); PG_EXACT.
 // Wavefronts per SIMD: a plain 64 x 64 Q4_0 tile is held to 168 registers, three workgroups a compute unit (172 without the bound, since the
 // loads are buffer loads: two.  WO and down of 2112 x 2112 and 2112 x 5632, 1000 tokens, 528 workgroups, mean of both: 63.4 us two at a time,
-// 53.9 three).  What it spills is one value of the epilogue's, around the K loop.
+// 53.9 three).  What it spills are values of the epilogue's, around the K loop.
 template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO>
 __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT == 4 && NTW == 1 && PREC == PG_HILO ? 3 : 2)) pgemm_kernel(QGemmParams P) {
     constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
