@@ -193,12 +193,7 @@ __global__ void bembed_kernel(BEmbedParams P) {
         }
         if (threadIdx.x == 0) P.tkv[blockIdx.x] = (long long)strm * P.kv_stream_stride + (long long)pos * P.hd;
     }
-    const int gr = P.gamma_row ? P.gamma_row[token] : -1;
-    for (int i = threadIdx.x; i < P.dim; i += blockDim.x) {
-        float v = embed_value(P.table, P.wtype, P.dim, token, i);
-        if (gr >= 0) v += P.gamma_val[(long long)gr * P.dim + i];
-        x[i] = v;
-    }
+    embed_row(P.table, P.wtype, P.dim, token, P.gamma_row, P.gamma_val, x);
 }
 
 // Which of the launch's blocks this one stands for: blocks b, b + 8, ... run on one XCD, which gets a run of them.  The sixteen tokens of a fragment

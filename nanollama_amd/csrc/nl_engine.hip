@@ -667,7 +667,7 @@ void build_plan_blocks(nl_engine *e, std::vector<Op> &plan) {
         EmbedParams P{e->embd_raw, e->embd_type, c.dim, e->ctl, e->x[0], e->gamma_row, e->gamma_val, e->tick};
         e->plan_embed = P;
         plan.push_back({K_EMBED, 0, nullptr, 0, [P](hipStream_t st) {
-                               hipLaunchKernelGGL(embed_kernel, dim3(1), dim3(256), 0, st, P);
+                               hipLaunchKernelGGL(embed_kernel, dim3(1), dim3(P.dim <= 1024 ? 256 : 1024), 0, st, P);
                                return hipGetLastError();
                            }});
     }
@@ -763,7 +763,7 @@ void build_plan(nl_engine *e, std::vector<Op> &plan, bool fused, bool help = fal
         EmbedParams P{e->embd_raw, e->embd_type, c.dim, e->ctl, e->x[0], e->gamma_row, e->gamma_val, p2p ? e->p2p.epoch : e->tick};
         e->plan_embed = P;
         plan.push_back({K_EMBED, 0, nullptr, 0, [P](hipStream_t st) {
-                               hipLaunchKernelGGL(embed_kernel, dim3(1), dim3(256), 0, st, P);
+                               hipLaunchKernelGGL(embed_kernel, dim3(1), dim3(P.dim <= 1024 ? 256 : 1024), 0, st, P);
                                return hipGetLastError();
                            }});
     }

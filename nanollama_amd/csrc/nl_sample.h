@@ -62,12 +62,7 @@ __device__ __forceinline__ void samp_embed_tail(const SampleParams &P, int token
     if (!P.embed) return;
     const EmbedParams &E = P.emb;
     if (E.epoch && threadIdx.x == 0) *E.epoch = *E.epoch + 1;            // the forward counter, as embed_kernel advances it
-    const int gr = E.gamma_row ? E.gamma_row[token] : -1;
-    for (int i = threadIdx.x; i < E.dim; i += blockDim.x) {
-        float v = embed_value(E.table, E.wtype, E.dim, token, i);
-        if (gr >= 0) v += E.gamma_val[(long long)gr * E.dim + i];
-        E.x[i] = v;
-    }
+    embed_row(E.table, E.wtype, E.dim, token, E.gamma_row, E.gamma_val, E.x);
 }
 
 // device scratch of one sampler (one vocabulary)

@@ -177,6 +177,28 @@ def _run_teacher_forced(hip, orc, path, tokens):
     return worst, scale
 
 
+@pytest.mark.parametrize("dim", [32, 992, 1056, 2080, 4128])
+@pytest.mark.parametrize("wtype", ["q8_0", "q4_0", "f16", "f32"])
+def test_embedding_rows_of_every_width(hip, orc, tmp_path, wtype, dim):
+    # a thread of the lookup takes four elements of a row a round: rows of less than one round, of a round's remainder and of two workgroup sizes,
+    # in the single step, behind the argmax of a chain and in a prompt
+    path = str(tmp_path / "m.gguf")
+    synth.generate_gguf(path, synth.ModelShape("emb", 1, dim, dim // 32, dim // 32, 64, seq_len=32, interm=64), wtype, 9)
+    g = gguf.load_gguf(path)
+    dev, ref = hip.load_llama_model(g), orc.OracleModel(g)
+    tok, want_ids = 5, []
+    for pos in range(4):
+        want = ref.forward(tok, pos)
+        dev.forward(tok, pos)
+        assert float(np.abs(dev.state.logits - want).max()) <= LOGIT_TOL * max(1.0, float(want.std())), pos
+        tok = int(np.argmax(want))
+        want_ids.append(tok)
+    assert list(dev.decode_greedy(5, 0, 4)) == want_ids
+    dev.prefill([5] + want_ids[:3])
+    assert float(np.abs(dev.state.logits - want).max()) <= LOGIT_TOL * max(1.0, float(want.std()))
+    dev.close()
+
+
 @pytest.mark.parametrize("tag", MODELS)
 def test_forward_logits_match_oracle_and_goldens(hip, orc, tag):
     path = os.path.join(GOLDEN, tag + ".gguf")
