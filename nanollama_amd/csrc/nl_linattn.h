@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256) gla_decay_kernel(GlaParams P) {
 // wavefronts at once, S through all sub-chunks without a barrier, one meeting for all norms (three barriers a segment where a sub-chunk a step has
 // twelve); more channels have no registers for it, and the increments, which meet once a sub-chunk, are faster with the next sub-chunk's operands requested
 // before the current one is multiplied (12.5 us, a whole segment at once 13.9).  Addresses are minima of byte offsets and the sums over 16 lanes are
-// row operations.  The outputs of 2047 tokens, 64 channels, 128 values: twelve heads 32.5 -> 28.8 us, six 23.8 -> 18.4; that 384 workgroups are two for
+// row operations.  The outputs of 2047 tokens, 64 channels, 128 values: twelve heads 32.5 -> 29.9 us, six 23.8 -> 19.4; that 384 workgroups are two for
 // half of the 256 compute units is the difference between the two.
 constexpr int la_subs(int dkt, int wv, bool out) { return out && wv <= 8 && dkt <= 4 ? LA_SEG / LA_SUB : 1; }   // sub-chunks a step
 __host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * subs ? 4 : nw >= 2 * subs ? 2 : 1; }   // wavefronts that share one A
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
     const long long shead = (long long)dkp * P.dvp;
     float *stream_state = P.state + sg.stream * P.state_stride + h * shead;
     float *seg_state = P.inc + ((long long)blockIdx.x * P.heads + h) * shead;
-    float rq[SUBS][NE], rk[SUBS][NE], rl[SUBS][NE], re[SUBS][NE], rv[SUBS][4];
+    float rq[SUBS][NE] = {}, rk[SUBS][NE] = {}, rl[SUBS][NE] = {}, re[SUBS][NE] = {}, rv[SUBS][4] = {};
     int et[NE], ed[NE];                                  // this thread's elements: token of the sub-chunk (16: none), channel
     int lk[NE], lq[NE];
     unsigned ep[NE], el[NE];                             // and where they lie: row t of the projections and of ldec; (t, d) of the LDS images
@@ -166,6 +166,7 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
 #pragma unroll
         for (int s = 0; s < SUBS; s++) {
             const int us = u0 + s * LA_SUB, end = min(us + LA_SUB - 1, last);
+            if (SUBS > 1 && us > last) break;                // (54 runs of ten tokens: 12.0 us as a sub-chunk a step, 14.8 with all four requested, 13.0 so)
             const unsigned pend = end * prow, lend = (unsigned)(end * C) * 4u, p0 = us * prow, l0 = (unsigned)(us * C) * 4u;
 #pragma unroll
             for (int e = 0; e < NE; e++) {
@@ -200,9 +201,10 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
         if (ROWS < LA_SEG && u0) lds_barrier();          // the step before has been read
         // the step's operands; tokens beyond its length and channels beyond dk are zero
         int strong = 0;
-        float v[SUBS][4];
+        float v[SUBS][4] = {};
 #pragma unroll
         for (int s = 0; s < SUBS; s++) {
+            if (SUBS > 1 && s * LA_SUB >= left) break;
 #pragma unroll
             for (int e = 0; e < NE; e++) {
                 const int t = et[e], d = ed[e], row = s * LA_SUB + t, ak = s * LA_SUB * ldk + lk[e], aq = s * LA_SUB * ld + lq[e];
@@ -238,7 +240,7 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
             for (int q = 0; q < nw; q++) slow |= flag[q];
             for (int task = w; task < SUBS * np; task += nw) {
                 const int s = task % SUBS, p = task / SUBS;
-                if (slow >> s & 1) continue;
+                if (slow >> s & 1 || s * LA_SUB >= left) continue;
                 f32x4 a = {};
                 for (int ks = p; ks < dkp / 4; ks += np)
                     a = __builtin_amdgcn_mfma_f32_16x16x4f32(qd[(s * LA_SUB + c) * ld + 4 * ks + g], ki[(s * LA_SUB + c) * ld + 4 * ks + g], a, 0, 0, 0);
@@ -265,9 +267,11 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
         float gz[SUBS][4];                               // gates, in accumulator order: token 4 g + i
         if (OUT)
 #pragma unroll
-            for (int s = 0; s < SUBS; s++)
+            for (int s = 0; s < SUBS; s++) {
+                if (SUBS > 1 && s * LA_SUB >= left) break;
 #pragma unroll
                 for (int i = 0; i < 4; i++) gz[s][i] = ld_off<float>(proj + P.off_g * 4ll, min(grow + (u0 + s * LA_SUB + i) * prow, (sg.len - 1) * prow) + vcol);
+            }
         if (owner) {
 #pragma unroll
             for (int s = 0; s < SUBS; s++) {
