@@ -112,8 +112,14 @@ __global__ void __launch_bounds__(256) gla_decay_kernel(GlaParams P) {
 // before the current one is multiplied (12.5 us, a whole segment at once 13.9).  Addresses are minima of byte offsets and the sums over 16 lanes are
 // row operations.  The outputs of 2047 tokens, 64 channels, 128 values: twelve heads 32.5 -> 29.9 us, six 23.8 -> 19.4; that 384 workgroups are two for
 // half of the 256 compute units is the difference between the two.
+// Past 64 channels the registers bound it (the increments: past 128), so a thread keeps of its elements only which they are and makes offsets of that each time;
+// held, those were sixteen registers through the products, and with them 104 and 228 bytes of scratch a lane at 128 and 256 channels.  The outputs of 2047
+// tokens: twelve heads of 128 channels and values 63.5 -> 50.1 us, six of 256 values with 128 channels 65.6 -> 51.4, with 256 118 -> 94, with 64 (eight
+// channel tiles, four elements a thread -> four and two) 48.3 -> 36.0.  Heads of 64 channels and fewer have them to spare (32: held 16.8, made 18.0).
 constexpr int la_subs(int dkt, int wv, bool out) { return out && wv <= 8 && dkt <= 4 ? LA_SEG / LA_SUB : 1; }   // sub-chunks a step
 __host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * subs ? 4 : nw >= 2 * subs ? 2 : 1; }   // wavefronts that share one A
+// t n, t <= 16, without a 32-bit product (four times an addition's time)
+__device__ __forceinline__ unsigned la_rows(unsigned t, unsigned n) { return __umul24(t, n & 0xffff) + (__umul24(t, n >> 16) << 16); }
 __host__ __device__ constexpr int la_ldk(int dkp) { return (dkp >> 4) & 1 ? dkp : dkp + 16; }   // rows g of k e^{l_end - l} in other banks
 __host__ __device__ inline size_t gla_seg_lds(int dkp, int nw, int subs, bool out) {
     const int rows = subs * LA_SUB;
@@ -121,7 +127,7 @@ __host__ __device__ inline size_t gla_seg_lds(int dkp, int nw, int subs, bool ou
 }
 
 template <typename T, int DKT, int NE, int WV, bool OUT>
-__global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_kernel(GlaParams P) {
+__global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 || (OUT && DKT > 4) ? 4 : 2) gla_seg_kernel(GlaParams P) {
     extern __shared__ __align__(16) char lds[];
     constexpr int SUBS = la_subs(DKT, WV, OUT), ROWS = SUBS * LA_SUB;
     const GlaSeg sg = P.segs[blockIdx.x];
@@ -142,19 +148,24 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
     float *stream_state = P.state + sg.stream * P.state_stride + h * shead;
     float *seg_state = P.inc + ((long long)blockIdx.x * P.heads + h) * shead;
     float rq[SUBS][NE] = {}, rk[SUBS][NE] = {}, rl[SUBS][NE] = {}, re[SUBS][NE] = {}, rv[SUBS][4] = {};
-    int et[NE], ed[NE];                                  // this thread's elements: token of the sub-chunk (16: none), channel
-    int lk[NE], lq[NE];
-    unsigned ep[NE], el[NE];                             // and where they lie: row t of the projections and of ldec; (t, d) of the LDS images
+    // this thread's elements: token of the sub-chunk (16: none) and channel; where they lie: row t of the projections and of ldec, (t, d) of the LDS images
+    struct Elem { int t, d, lk, lq; unsigned ep, el; };
+    constexpr bool KEEP = OUT ? DKT <= 4 : DKT <= 8;     // (see above)
+    unsigned elems[NE];
+    Elem held[NE];
 #pragma unroll
     for (int e = 0; e < NE; e++) {
-        const int i = tid + e * nthr;
-        et[e] = min(i / dkp, LA_SUB);
-        ed[e] = i - i / dkp * dkp;
-        ep[e] = (unsigned)(et[e] * P.ldp) * 4u;
-        el[e] = (unsigned)(et[e] * C) * 4u;
-        lk[e] = et[e] * ldk + ed[e];
-        lq[e] = et[e] * ld + ed[e];
+        const int i = tid + e * nthr, t = min(i / dkp, LA_SUB), d = i - i / dkp * dkp;
+        elems[e] = t << 16 | d;
+        held[e] = Elem{t, d, t * ldk + d, t * ld + d, (unsigned)(t * P.ldp) * 4u, (unsigned)(t * C) * 4u};
     }
+    auto elem = [&](int e, bool keep) __attribute__((always_inline)) {
+        if (keep) return held[e];
+        unsigned x = elems[e];
+        asm volatile("" : "+v"(x));                      // (or hipcc keeps what is made of it)
+        const int t = x >> 16, d = x & 0xffff;
+        return Elem{t, d, (int)__umul24(t, ldk) + d, (int)__umul24(t, ld) + d, la_rows(t, P.ldp) * 4u, la_rows(t, C) * 4u};
+    };
     const unsigned vrow = (unsigned)(g * P.ldp) * 4u, grow = 4 * vrow, prow = P.ldp * 4u;
     const unsigned vcol = (unsigned)(h * P.dv + min(dvc, P.dv - 1)) * 4u;
     const char *proj = reinterpret_cast<const char *>(P.proj + (long long)sg.tok0 * P.ldp), *ldec = reinterpret_cast<const char *>(P.ldec + (long long)sg.tok0 * C + h * dk);
@@ -170,9 +181,10 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
             const unsigned pend = end * prow, lend = (unsigned)(end * C) * 4u, p0 = us * prow, l0 = (unsigned)(us * C) * 4u;
 #pragma unroll
             for (int e = 0; e < NE; e++) {
-                const unsigned d = (unsigned)min(ed[e], dk - 1) * 4u, at = min(ep[e] + p0, pend) + h * dk * 4u + d;
+                const Elem E = elem(e, KEEP);
+                const unsigned d = (unsigned)min(E.d, dk - 1) * 4u, at = min(E.ep + p0, pend) + h * dk * 4u + d;
                 rk[s][e] = ld_off<float>(proj + P.off_k * 4ll, at);
-                rl[s][e] = ld_off<float>(ldec, min(el[e] + l0, lend) + d);
+                rl[s][e] = ld_off<float>(ldec, min(E.el + l0, lend) + d);
                 re[s][e] = ld_off<float>(ldec, lend + d);
                 if (OUT) rq[s][e] = ld_off<float>(proj + P.off_q * 4ll, at);
             }
@@ -207,7 +219,8 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 ? 4 : 2) gla_seg_ke
             if (SUBS > 1 && s * LA_SUB >= left) break;
 #pragma unroll
             for (int e = 0; e < NE; e++) {
-                const int t = et[e], d = ed[e], row = s * LA_SUB + t, ak = s * LA_SUB * ldk + lk[e], aq = s * LA_SUB * ld + lq[e];
+                const Elem E = elem(e, KEEP || !OUT);
+                const int t = E.t, d = E.d, row = s * LA_SUB + t, ak = s * LA_SUB * ldk + E.lk, aq = s * LA_SUB * ld + E.lq;
                 const bool chan = d < dk && s * LA_SUB < left, live = d < dk && row < left;
                 const float l = live ? rl[s][e] : 0.f, end = chan ? re[s][e] : 0.f, k = live ? rk[s][e] : 0.f;
                 if (t < LA_SUB) {
@@ -480,6 +493,7 @@ hipError_t launch_gla_seg(const GlaParams &P, int nsegs, hipStream_t st) {
         if (P.dkp <= 64) return two ? go(gla_seg_kernel<T, 4, 2, 8, OUT>, la_subs(4, 8, OUT)) : go(gla_seg_kernel<T, 4, 4, 8, OUT>, la_subs(4, 8, OUT));
         return go(gla_seg_kernel<T, 8, 4, 8, OUT>, la_subs(8, 8, OUT));     // nw <= 8: dkp <= 128
     }
+    if (P.dkp <= 64) return go(gla_seg_kernel<T, 4, 2, 16, OUT>, la_subs(4, 16, OUT));     // (more than 128 values: two elements a thread)
     if (P.dkp <= 128) return go(gla_seg_kernel<T, 8, 4, 16, OUT>, la_subs(8, 16, OUT));
     return go(gla_seg_kernel<T, 16, 4, 16, OUT>, la_subs(16, 16, OUT));
 }

@@ -1,4 +1,5 @@
-"""Registers and LDS of launches whose tiling counts on so many workgroups a compute unit, read from the built library's own kernel metadata."""
+"""Registers, LDS and scratch of launches that count on so many workgroups a compute unit or on no spilled registers, read from the built libraries' own
+kernel metadata."""
 import os
 import re
 import subprocess
@@ -13,18 +14,21 @@ LLVM = "/opt/rocm/llvm/bin/"
 RESIDENT = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 1, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 2, 0>", 4, 3)]
 
 
-@pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
+# kernel<template arguments>, bytes of scratch a lane at most
+SPILLED = [("gla_seg_kernel<float, 4, 2, 8, true>", 0), ("gla_seg_kernel<float, 4, 4, 8, true>", 0), ("gla_seg_kernel<float, 8, 4, 8, true>", 0),
+           ("gla_seg_kernel<float, 4, 2, 16, true>", 0), ("gla_seg_kernel<float, 8, 4, 16, true>", 0), ("gla_seg_kernel<float, 16, 4, 16, true>", 92),
+           ("gla_seg_kernel<float, 16, 4, 16, false>", 0)]
+
+
+def _kernels(lib, d):
     if not os.path.exists(LLVM + "clang-offload-bundler"):
         pytest.skip("no LLVM tools")
-    _lib.lib()                                     # (builds it where nothing is built)
-    d = tmp_path_factory.mktemp("co")
     run = lambda *a: subprocess.run(a, check=True, capture_output=True, text=True).stdout
-    run(LLVM + "llvm-objcopy", "--dump-section", f".hip_fatbin={d}/fat", _lib.LIB_PATH, "/dev/null")
+    run(LLVM + "llvm-objcopy", "--dump-section", f".hip_fatbin={d}/fat", lib, "/dev/null")
     run(LLVM + "clang-offload-bundler", "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={d}/fat", f"--output={d}/co")
     out, cur = {}, {}
     for line in run(LLVM + "llvm-readelf", "--notes", f"{d}/co").splitlines():
-        m = re.match(r" +(?:- )?\.(symbol|vgpr_count|group_segment_fixed_size|max_flat_workgroup_size): +(\S+)", line)
+        m = re.match(r" +(?:- )?\.(symbol|vgpr_count|private_segment_fixed_size|group_segment_fixed_size|max_flat_workgroup_size): +(\S+)", line)
         if m:
             cur[m[1]] = m[2].strip("'")
         if ".wavefront_size" in line:
@@ -34,9 +38,27 @@ def kernels(tmp_path_factory):
     return dict(zip(names, out.values()))
 
 
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    _lib.lib()                                     # (builds it where nothing is built)
+    return _kernels(_lib.LIB_PATH, tmp_path_factory.mktemp("co"))
+
+
+@pytest.fixture(scope="module")
+def stack_kernels(tmp_path_factory):
+    _lib.stack_lib()
+    return _kernels(_lib.STACK_LIB_PATH, tmp_path_factory.mktemp("co"))
+
+
 @pytest.mark.parametrize("name,waves,groups", RESIDENT)
 def test_workgroups_a_compute_unit(kernels, name, waves, groups):
     k, = [v for n, v in kernels.items() if name in n]
     assert int(k["max_flat_workgroup_size"]) == waves * 64
     registers = -(-int(k["vgpr_count"]) // 8) * 8
     assert 4 * (512 // registers) // waves >= groups and 160 * 1024 // int(k["group_segment_fixed_size"]) >= groups, k
+
+
+@pytest.mark.parametrize("name,most", SPILLED)
+def test_scratch_of_the_stack_family(stack_kernels, name, most):
+    k, = [v for n, v in stack_kernels.items() if name in n]
+    assert int(k["private_segment_fixed_size"]) <= most, k
