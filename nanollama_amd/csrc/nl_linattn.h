@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(256) gla_decay_kernel(GlaParams P) {
 // What a workgroup spends is spread: matrix products (36 of 32 cycles per sub-chunk, wavefront and 64 channels, in float32), exponentials, sums over the
 // value columns, and the wavefronts meeting.  The outputs of a head of at most 64 channels therefore take a whole segment a step: A's shared out over the
 // wavefronts at once, S through all sub-chunks without a barrier, one meeting for all norms (three barriers a segment where a sub-chunk a step has
-// twelve); more channels have no registers for it, and the increments, which meet once a sub-chunk, are faster with the next sub-chunk's operands requested
+// fifteen); more channels have no registers for it, and the increments, which meet once a sub-chunk, are faster with the next sub-chunk's operands requested
 // before the current one is multiplied (12.5 us, a whole segment at once 13.9).  Addresses are minima of byte offsets and the sums over 16 lanes are
 // row operations.  The outputs of 2047 tokens, 64 channels, 128 values: twelve heads 32.5 -> 29.9 us, six 23.8 -> 19.4; that 384 workgroups are two for
 // half of the 256 compute units is the difference between the two.
@@ -116,25 +116,26 @@ __global__ void __launch_bounds__(256) gla_decay_kernel(GlaParams P) {
 // held, those were sixteen registers through the products, and with them 104 and 228 bytes of scratch a lane at 128 and 256 channels.  The outputs of 2047
 // tokens: twelve heads of 128 channels and values 63.5 -> 50.1 us, six of 256 values with 128 channels 65.6 -> 51.4, with 256 118 -> 94, with 64 (eight
 // channel tiles, four elements a thread -> four and two) 48.3 -> 36.0.  Heads of 64 channels and fewer have them to spare (32: held 16.8, made 18.0).
-constexpr int la_subs(int dkt, int wv, bool out) { return out && wv <= 8 && dkt <= 4 ? LA_SEG / LA_SUB : 1; }   // sub-chunks a step
-__host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * subs ? 4 : nw >= 2 * subs ? 2 : 1; }   // wavefronts that share one A
+constexpr int la_subs(int dkt, int wv, bool out) { return out && wv <= 8 && dkt <= 4 ? LA_SEG / LA_SUB : 1; }   // sub-chunks a step of longer runs
+__host__ __device__ constexpr int la_parts(int subs, int nw) { return nw >= 4 * subs ? 4 : nw >= 2 * subs ? 2 : 1; }   // parts of one A
 // t n, t <= 16, without a 32-bit product (four times an addition's time)
 __device__ __forceinline__ unsigned la_rows(unsigned t, unsigned n) { return __umul24(t, n & 0xffff) + (__umul24(t, n >> 16) << 16); }
 __host__ __device__ constexpr int la_ldk(int dkp) { return (dkp >> 4) & 1 ? dkp : dkp + 16; }   // rows g of k e^{l_end - l} in other banks
-__host__ __device__ inline size_t gla_seg_lds(int dkp, int nw, int subs, bool out) {
+__host__ __device__ constexpr size_t gla_seg_lds(int dkp, int subs, int np, bool out) {
     const int rows = subs * LA_SUB;
-    return (size_t)(rows * la_ldk(dkp) + subs * dkp + (out ? 2 * rows * (dkp + 4) + subs * la_parts(subs, nw) * 256 + 16 : 0)) * 4;
+    return (size_t)(rows * la_ldk(dkp) + subs * dkp + (out ? 2 * rows * (dkp + 4) + subs * np * 256 + 16 : 0)) * 4;
 }
+static_assert(gla_seg_lds(64, LA_SEG / LA_SUB, 2, true) <= 65536 && gla_seg_lds(256, 1, 4, true) <= 65536, "what a launch has without asking");
 
-template <typename T, int DKT, int NE, int WV, bool OUT>
+template <typename T, int DKT, int NE, int WV, bool OUT, int SUBS = la_subs(DKT, WV, OUT)>
 __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 || (OUT && DKT > 4) ? 4 : 2) gla_seg_kernel(GlaParams P) {
     extern __shared__ __align__(16) char lds[];
-    constexpr int SUBS = la_subs(DKT, WV, OUT), ROWS = SUBS * LA_SUB;
+    constexpr int ROWS = SUBS * LA_SUB;
     const GlaSeg sg = P.segs[blockIdx.x];
     if (!OUT && (sg.nseg == 1 || sg.index + 1 == sg.nseg)) return;     // nobody starts from the state behind the last segment
     const int h = blockIdx.y, tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, w = tid >> 6, nw = nthr >> 6, g = lane >> 4, c = lane & 15;
     const int dk = P.dk, dkp = P.dkp, nkt = dkp >> 4, ld = dkp + 4, ldk = la_ldk(dkp), C = P.heads * dk, dvc = w * 16 + c;
-    const int nv = P.dvp >> 4, np = la_parts(SUBS, nw);
+    const int nv = P.dvp >> 4, np = la_parts(la_subs(DKT, WV, OUT), nw);    // (short runs take the same parts: the same bits)
     const bool owner = w < nv, value = dvc < P.dv;
     float *ke = reinterpret_cast<float *>(lds);          // [ROWS][ldk] k e^{l_end - l}
     float *etot = ke + ROWS * ldk;                       // [SUBS][dkp] e^{l_end}
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(WV * 64, WV > 8 || NE <= 2 || (OUT && DKT > 4)
 #pragma unroll
         for (int s = 0; s < SUBS; s++) {
             const int us = u0 + s * LA_SUB, end = min(us + LA_SUB - 1, last);
-            if (SUBS > 1 && us > last) break;                // (54 runs of ten tokens: 12.0 us as a sub-chunk a step, 14.8 with all four requested, 13.0 so)
+            if (SUBS > 1 && us > last) break;                // (requests of all four by short runs among longer ones cost as much again as the first)
             const unsigned pend = end * prow, lend = (unsigned)(end * C) * 4u, p0 = us * prow, l0 = (unsigned)(us * C) * 4u;
 #pragma unroll
             for (int e = 0; e < NE; e++) {
@@ -478,35 +479,43 @@ __device__ __forceinline__ void gla_decode_block(const GlaParams &P, int h, int 
     }
 }
 
+// longest: tokens of the longest run.  Up to one sub-chunk, the outputs are better off with a workgroup that holds one (64 channels, 128 values, 54 runs of
+// 5 to 16 tokens: six heads 13.2 -> 12.4 us, twelve 19.8 -> 18.2; runs of 24, twelve heads: a sub-chunk a step 28.6, a segment 27.9)
 template <typename T, bool OUT>
-hipError_t launch_gla_seg(const GlaParams &P, int nsegs, hipStream_t st) {
+hipError_t launch_gla_seg(const GlaParams &P, int nsegs, int longest, hipStream_t st) {
     const int nw = std::max(P.dvp, P.dkp) / 16;
-    auto go = [&](auto kfn, int subs) {
-        const size_t lds = gla_seg_lds(P.dkp, nw, subs, OUT);
-        if (lds > 65536)
-            if (hipError_t s = hipFuncSetAttribute(reinterpret_cast<const void *>(kfn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) return s;
-        hipLaunchKernelGGL(kfn, dim3(nsegs, P.heads), dim3(nw * 64), lds, st, P);
+    auto go = [&](auto dkt, auto ne, auto wv, auto subs) {
+        constexpr int DKT = decltype(dkt)::value, NE = decltype(ne)::value, WV = decltype(wv)::value, SUBS = decltype(subs)::value;
+        hipLaunchKernelGGL((gla_seg_kernel<T, DKT, NE, WV, OUT, SUBS>), dim3(nsegs, P.heads), dim3(nw * 64), gla_seg_lds(P.dkp, SUBS, la_parts(la_subs(DKT, WV, OUT), nw), OUT), st, P);
         return hipGetLastError();
     };
+    using std::integral_constant;
+    const integral_constant<int, 1> one{};
+    const integral_constant<int, 2> two{};
+    const integral_constant<int, 4> four{};
+    const integral_constant<int, 8> eight{};
+    const integral_constant<int, 16> sixteen{};
+    const bool half = 16 * P.dkp <= 2 * nw * 64;                 // two elements a thread
     if (nw <= 8) {
-        const bool two = 16 * P.dkp <= 2 * nw * 64;
-        if (P.dkp <= 64) return two ? go(gla_seg_kernel<T, 4, 2, 8, OUT>, la_subs(4, 8, OUT)) : go(gla_seg_kernel<T, 4, 4, 8, OUT>, la_subs(4, 8, OUT));
-        return go(gla_seg_kernel<T, 8, 4, 8, OUT>, la_subs(8, 8, OUT));     // nw <= 8: dkp <= 128
+        if (P.dkp > 64) return go(eight, four, eight, one);      // (dkp <= 128)
+        if constexpr (OUT)
+            if (longest > LA_SUB) return half ? go(four, two, eight, four) : go(four, four, eight, four);
+        return half ? go(four, two, eight, one) : go(four, four, eight, one);
     }
-    if (P.dkp <= 64) return go(gla_seg_kernel<T, 4, 2, 16, OUT>, la_subs(4, 16, OUT));     // (more than 128 values: two elements a thread)
-    if (P.dkp <= 128) return go(gla_seg_kernel<T, 8, 4, 16, OUT>, la_subs(8, 16, OUT));
-    return go(gla_seg_kernel<T, 16, 4, 16, OUT>, la_subs(16, 16, OUT));
+    if (P.dkp <= 64) return go(four, two, sixteen, one);         // (more than 128 values: two elements a thread)
+    if (P.dkp <= 128) return go(eight, four, sixteen, one);
+    return go(sixteen, four, sixteen, one);
 }
 
 // the recurrence of a ragged step: runs = streams' token runs with more than one segment (their first segments in P.runs)
 template <typename T>
-hipError_t launch_gla(const GlaParams &P, int nsubs, int nsegs, int nruns, hipStream_t st) {
+hipError_t launch_gla(const GlaParams &P, int nsubs, int nsegs, int nruns, int longest, hipStream_t st) {
     hipLaunchKernelGGL(gla_decay_kernel, dim3(nsubs, (P.heads * P.dk + 255) / 256), dim3(256), (size_t)LA_SUB * P.rank * 4, st, P);
     if (nruns > 0) {
-        if (hipError_t s = launch_gla_seg<T, false>(P, nsegs, st)) return s;
+        if (hipError_t s = launch_gla_seg<T, false>(P, nsegs, longest, st)) return s;
         hipLaunchKernelGGL(gla_scan_kernel, dim3((P.dkp * P.dvp / 4 + 255) / 256, P.heads, nruns), dim3(256), 0, st, P);
     }
-    return launch_gla_seg<T, true>(P, nsegs, st);
+    return launch_gla_seg<T, true>(P, nsegs, longest, st);
 }
 
 }  // namespace nl

@@ -338,7 +338,7 @@ struct StepIn {                  // one launch sequence
     const int *tok, *pos, *stream;   // device
     int nsplit = 1;              // decode
     bool decode = true;
-    int nsubs = 0, nsegs = 0, nruns = 0, ntiles = 0;
+    int nsubs = 0, nsegs = 0, nruns = 0, ntiles = 0, longest = 0;   // longest: tokens of the longest piece
     std::vector<KeyGroup> groups;
     int n_out = 0;               // rows of logits: of tokens rows[0 .. n_out) (device), or of every token when rows is null
     const int *rows = nullptr;
@@ -564,7 +564,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
             if ((rc = launch_mix_decode<T>(W, N, s.n, st))) return rc;
         } else {
             if (A.heads && ((rc = launch_win_prep<T>(W, s.n, st)) || (rc = launch_win_attn<T>(W, s.ntiles, st)))) return rc;
-            if (G.heads && (rc = launch_gla<T>(N, s.nsubs, s.nsegs, s.nruns, st))) return rc;
+            if (G.heads && (rc = launch_gla<T>(N, s.nsubs, s.nsegs, s.nruns, s.longest, st))) return rc;
         }
         if ((rc = residual_product<T>(e, L.out, e->y, s.n, nullptr, L.norm1p, L.d.ff ? nullptr : behind, L.d.ff ? L.norm2 : next,
                                       L.d.ff && L.d.latent.heads ? &L.gateup : nullptr))) return rc;
@@ -718,6 +718,7 @@ int run_pieces(nl_engine *e, const std::vector<Piece> &ps, const int *tokens, co
         }
         for (int t = 0; t < p.n; t += WA_Q) tiles[ntiles++] = WinTile{n + t, std::min(WA_Q, p.n - t), p.pos0 + t, p.stream, key0};
         for (; w < want.size() && want[w] < p.tok0 + p.n; w++) rows.push_back(n + want[w] - p.tok0);
+        s.longest = std::max(s.longest, p.n);
         n += p.n;
     }
     s.n = n; s.nsubs = nsubs; s.nsegs = nsegs; s.nruns = nruns; s.ntiles = ntiles;

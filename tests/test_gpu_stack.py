@@ -381,6 +381,23 @@ def test_subchunks_within_and_beyond_the_factored_range(dim, vdim, n):
     m.close()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim,vdim", [(16, 16), (20, 60), (64, 128), (64, 64), (64, 256), (128, 70), (112, 128)])
+def test_short_runs_alone_and_beside_longer_ones(dim, vdim, dtype):
+    """A step whose runs are all within a sub-chunk takes another workgroup than one with longer runs: the same bits, outputs and states."""
+    cfg = config([gla(heads=2, dim=dim, vdim=vdim), gla(heads=2, dim=dim, vdim=vdim)])
+    w = weights(cfg, 5)
+    a, b, c = tokens(10, seed=1), tokens(16, seed=2), tokens(30, seed=3)
+    m = load(cfg, w, dtype)
+    got = {}
+    for name, others in (("short", [(1, b, 0, []), (2, c[:14], 0, [])]), ("long", [(1, c, 0, [])])):       # forty tokens either way
+        m.reset(0)
+        rows = m.step([(0, a, 0, list(range(10)))] + others)
+        got[name] = np.concatenate([rows[0] if isinstance(rows, (list, tuple)) else rows, by_token(m, b[:3], 0, 10)])
+    assert np.isfinite(got["short"]).all() and np.array_equal(got["short"], got["long"])
+    m.close()
+
+
 def test_state_carries_the_first_token():
     """A state that barely decays: the first token's mark is there hundreds of tokens later, whatever lies between."""
     cfg = config([gla(heads=1, dim=16, vdim=16, tau=64.0)])

@@ -15,9 +15,9 @@ RESIDENT = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1,
 
 
 # kernel<template arguments>, bytes of scratch a lane at most
-SPILLED = [("gla_seg_kernel<float, 4, 2, 8, true>", 0), ("gla_seg_kernel<float, 4, 4, 8, true>", 0), ("gla_seg_kernel<float, 8, 4, 8, true>", 0),
-           ("gla_seg_kernel<float, 4, 2, 16, true>", 0), ("gla_seg_kernel<float, 8, 4, 16, true>", 0), ("gla_seg_kernel<float, 16, 4, 16, true>", 92),
-           ("gla_seg_kernel<float, 16, 4, 16, false>", 0)]
+SPILLED = [("gla_seg_kernel<float, 4, 2, 8, true, 4>", 0), ("gla_seg_kernel<float, 4, 4, 8, true, 4>", 0), ("gla_seg_kernel<float, 8, 4, 8, true, 1>", 0),
+           ("gla_seg_kernel<float, 4, 2, 16, true, 1>", 0), ("gla_seg_kernel<float, 8, 4, 16, true, 1>", 0), ("gla_seg_kernel<float, 16, 4, 16, true, 1>", 92),
+           ("gla_seg_kernel<float, 16, 4, 16, false, 1>", 0)]
 
 
 def _kernels(lib, d):
