@@ -433,40 +433,40 @@ struct KeyRows {
 
 // Blocks b, b + 8, ... run on one XCD and share its L2.  Each XCD gets a rectangle of the nrb x ntb tiles, `rows` x 8 / rows of them cover the product, and
 // reads 1 / rows of the weights and rows / 8 of the activations; where no rectangle shares the tiles out evenly, a range of them, row block after row
-// block (rows 0).  (A range always, us a launch, bf16: 1920 tokens, 768 x 2048 18.8, now 15.5, 2047 tokens, 1536 x 1536 19.5 and 18.3, 1536 x 4096 33.0 and
+// block (shift -1).  (A range always, us a launch, bf16: 1920 tokens, 768 x 2048 18.8, now 15.5, 2047 tokens, 1536 x 1536 19.5 and 18.3, 1536 x 4096 33.0 and
 // 32.0; a document of 2047 tokens, 863M: 6625 and 6581.  The nearest rectangle for 4640 x 1536, 25 x 8 tiles: 39.9 and 41.9.  Quantised files' prompts, whose
 // weights are smaller: F16 5140 and 5180, nothing.)
-struct XcdTiles {
-    int rows, nrb, ntb, r, t;               // XCDs along the rows (0: a range of tiles); tiles; an XCD's rectangle
-    __host__ __device__ __forceinline__ XcdTiles(int rows_, int nrb_, int ntb_) : rows(rows_), nrb(nrb_), ntb(ntb_) {
-        r = rows ? (nrb + rows - 1) / rows : (nrb * ntb + 7) / 8;
-        t = rows ? (ntb + 8 / rows - 1) / (8 / rows) : 1;
-    }
-    __host__ __device__ __forceinline__ int blocks() const { return 8 * r * t; }
+struct XcdTiles {                           // (made on the host: divided out in the kernel, its rectangles were four divisions in front of the first load, 0.3 us a launch)
+    int shift, nrb, ntb, r, t;              // log2 of XCDs along the rows (-1: a range of tiles); tiles; an XCD's rectangle
+    int blocks() const { return 8 * r * t; }
     // block b's tile; false: it has none
     __host__ __device__ __forceinline__ bool tile(int b, int &rb, int &tb) const {
-        const int xcd = b & 7, at = b >> 3;
-        if (rows) {
-            rb = xcd % rows * r + at / t;
-            tb = xcd / rows * t + at % t;
-        } else {
-            rb = (xcd * r + at) / ntb;
-            tb = xcd * r + at - rb * ntb;
+        const int xcd = b & 7, at = b >> 3, n = shift < 0 ? xcd * r + at : at, w = shift < 0 ? ntb : t, q = n / w;
+        rb = q;
+        tb = n - q * w;
+        if (shift >= 0) {
+            rb += (xcd & ((1 << shift) - 1)) * r;
+            tb += (xcd >> shift) * t;
         }
         return at < r * t && rb < nrb && tb < ntb;
     }
 };
+inline XcdTiles xcd_rect(int shift, int nrb, int ntb) {
+    if (shift < 0) return {shift, nrb, ntb, (nrb * ntb + 7) / 8, 1};
+    const int rows = 1 << shift, toks = 8 >> shift;
+    return {shift, nrb, ntb, (nrb + rows - 1) / rows, (ntb + toks - 1) / toks};
+}
 // The fewest operand bytes among those that give no XCD more tiles than a range does; row_bytes, tok_bytes: a row block's and a token block's bytes
 // of a column, in any unit
-inline int xcd_rows(int nrb, int ntb, int row_bytes, int tok_bytes) {
+inline XcdTiles xcd_tiles(int nrb, int ntb, int row_bytes, int tok_bytes) {
     const long long per = ((long long)nrb * ntb + 7) / 8;
-    int best = 0;
+    XcdTiles best = xcd_rect(-1, nrb, ntb);
     // (a range starts inside a row of tiles)
     long long best_b = std::min<long long>(nrb, (per + ntb - 1) / ntb + (per % ntb ? 1 : 0)) * row_bytes + std::min<long long>(ntb, per) * tok_bytes;
-    for (int rows = 1; rows <= 8; rows *= 2) {
-        const XcdTiles x(rows, nrb, ntb);
+    for (int shift = 0; shift <= 3; shift++) {
+        const XcdTiles x = xcd_rect(shift, nrb, ntb);
         const long long b = (long long)x.r * row_bytes + (long long)x.t * tok_bytes;
-        if ((long long)x.r * x.t == per && b <= best_b) best = rows, best_b = b;
+        if ((long long)x.r * x.t == per && b <= best_b) best = x, best_b = b;
     }
     return best;
 }
@@ -482,7 +482,6 @@ struct MatParams {
     int act_nks, act_silu; // activation: silu or tanh-gelu
     const float *bias, *bias2;   // ST_F32: per row; ST_GATED: of gate and up; whole row tiles long, or null
     int x_nks;             // k tiles per token tile of X (0: nks)
-    int xcd_rows;          // many_kernel, direct_kernel: XCDs along the rows (XcdTiles)
     int group;             // few_kernel: row tiles of a group; group i multiplies X's k tiles from i * nks on (0: one group)
     const int *x_tile;     // many_kernel: which tile of X is token tile t (null: t)
     HeadRows hd;
@@ -608,17 +607,16 @@ template <typename T, int RTW> struct ManyGeom {
     static constexpr int RT = 2 * RTW, NT = 8, UNIT = OPT * sizeof(T), NST = sizeof(T) == 2 ? 4 : 2, STAGE = (RT + NT) * UNIT, LDS = NST * STAGE;   // 48 or 64 KB
 };
 template <typename T, int EPI, int RTW, class TAIL>
-__global__ void __launch_bounds__(256) many_kernel(MatParams P, TAIL tail) {
+__global__ void __launch_bounds__(256) many_kernel(MatParams P, XcdTiles xt, TAIL tail) {
     using G = ManyGeom<T, RTW>;
     constexpr int RT = G::RT, NT = G::NT, UNIT = G::UNIT, NST = G::NST, STAGE = G::STAGE;
     constexpr int PW = STAGE / 4096;                       // 1 KiB pieces per stage and wavefront
     extern __shared__ __align__(16) char lds[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4;
-    const int nrb = (P.nrt + RT - 1) / RT, ntt = (P.n_tokens + 15) >> 4, ntb = (ntt + NT - 1) / NT;
-    const XcdTiles xt(P.xcd_rows, nrb, ntb);
+    const int ntt = (P.n_tokens + 15) >> 4;
     if constexpr (TAIL::on)
-        if ((int)blockIdx.x >= xt.blocks()) {
-            const int u = (blockIdx.x - xt.blocks()) * 4 + w;
+        if ((int)blockIdx.x >= 8 * xt.r * xt.t) {
+            const int u = (blockIdx.x - 8 * xt.r * xt.t) * 4 + w;
             if (u < tail.units) tail.unit(u, lane);
             return;
         }
@@ -630,9 +628,9 @@ __global__ void __launch_bounds__(256) many_kernel(MatParams P, TAIL tail) {
 #pragma unroll
     for (int i = 0; i < PW; i++) {
         const int u = i * 4 + w, t = u / (UNIT / 1024), piece = u % (UNIT / 1024);
-        const int xt = min(tb * NT + t - RT, ntt - 1);
+        const int xtile = min(tb * NT + t - RT, ntt - 1);
         src[i] = (t < RT ? reinterpret_cast<const char *>(P.W) + (long long)min(rb * RT + t, P.nrt - 1) * nks * UNIT
-                         : reinterpret_cast<const char *>(P.X) + (long long)(P.x_tile ? P.x_tile[xt] : xt) * P.x_nks * UNIT) + piece * 1024 + lane * 16;
+                         : reinterpret_cast<const char *>(P.X) + (long long)(P.x_tile ? P.x_tile[xtile] : xtile) * P.x_nks * UNIT) + piece * 1024 + lane * 16;
     }
     auto issue = [&](int ks, int st) {
 #pragma unroll
@@ -713,15 +711,14 @@ __device__ __forceinline__ void load_tile(Frag<float> &f, const __amdgpu_buffer_
 // rows of tiles whose partial sums are in LDS together: all of them where 64 KB hold them, else pairs
 constexpr int direct_rows(int waves, int rw, int tw) { return waves * rw * tw <= 64 ? rw : 2; }
 template <typename T, int EPI, int WR, int WT, int KS, int RW, int TW>
-__global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P) {
+__global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P, XcdTiles xt) {
     constexpr int UNIT = OPT * sizeof(T), SET = WR * WT;
     static_assert(RW % 2 == 0, "gate and up rows come in pairs");
     extern __shared__ __align__(16) char lds[];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
     const int nks = P.nks, ntt = (P.n_tokens + 15) >> 4;
-    const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = (ntt + WT * TW - 1) / (WT * TW);
     int rb, tb;
-    if (!XcdTiles(P.xcd_rows, nrb, ntb).tile(blockIdx.x, rb, tb)) return;
+    if (!xt.tile(blockIdx.x, rb, tb)) return;
     const int kw = w / SET, wr = w % WR, wt = w / WR % WT, r0 = (rb * WR + wr) * RW, t0 = (tb * WT + wt) * TW;
     const __amdgpu_buffer_rsrc_t W = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.W), 0, (int)((unsigned)P.nrt * nks * UNIT), 0x00027000);
     const __amdgpu_buffer_rsrc_t X = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.X), 0, (int)((unsigned)ntt * P.x_nks * UNIT), 0x00027000);
@@ -1130,10 +1127,8 @@ template <typename T, int EPI, class TAIL = NoTail>
 hipError_t launch_many(const MatParams &P, hipStream_t st, TAIL tail = {}) {
     const int ntb = (P.n_tokens + 127) / 128;
     auto go = [&](auto kfn, int rt, int lds) {
-        MatParams Q = P;
-        const int nrb = (P.nrt + rt - 1) / rt;
-        Q.xcd_rows = xcd_rows(nrb, ntb, rt, 8);
-        hipLaunchKernelGGL(kfn, dim3(XcdTiles(Q.xcd_rows, nrb, ntb).blocks() + (TAIL::on ? (tail.units + 3) / 4 : 0)), dim3(256), lds, st, Q, tail);
+        const XcdTiles xt = xcd_tiles((P.nrt + rt - 1) / rt, ntb, rt, 8);
+        hipLaunchKernelGGL(kfn, dim3(xt.blocks() + (TAIL::on ? (tail.units + 3) / 4 : 0)), dim3(256), lds, st, P, xt, tail);
         return hipGetLastError();
     };
     // 64 x 128 tiles up to three of them a compute unit, 128 x 128 beyond (bf16, 2047 tokens, K 1536: 3072 rows 27.6 us against 30.5, 3456 rows 38.4 against 31.3;
@@ -1147,9 +1142,8 @@ hipError_t launch_direct(const MatParams &P, hipStream_t st) {
     constexpr int lds = KS == 1 ? 0 : WR * WT * KS * direct_rows(WR * WT * KS, RW, TW) * TW * 1024;
     static_assert(lds <= 65536, "what a launch has without asking");
     const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = ((P.n_tokens + 15) / 16 + WT * TW - 1) / (WT * TW);
-    MatParams Q = P;
-    Q.xcd_rows = xcd_rows(nrb, ntb, WR * RW, WT * TW);
-    hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3(XcdTiles(Q.xcd_rows, nrb, ntb).blocks()), dim3(WR * WT * KS * 64), lds, st, Q);
+    const XcdTiles xt = xcd_tiles(nrb, ntb, WR * RW, WT * TW);
+    hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3(xt.blocks()), dim3(WR * WT * KS * 64), lds, st, P, xt);
     return hipGetLastError();
 }
 // Prompts: the largest tile with which the workgroups still cover the chip, in one round where that goes.  us, many_kernel -> direct_kernel,
