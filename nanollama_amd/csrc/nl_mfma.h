@@ -749,9 +749,11 @@ __global__ void __launch_bounds__(WR * WT * KS * 64) direct_kernel(MatParams P, 
         fence();
     };
     // residual rows of this wavefront's results, requested in front of the loop: behind it every pair of tiles waits for its own.
-    // (Not with eight sets, whose loops are too short to hide them: 540 tokens, 768 rows and columns, float32 17.8 against 15.8 us)
+    // (Not with eight sets, whose loops are too short to hide them: 540 tokens, 768 rows and columns, float32 17.8 against 15.8 us.  Nor in float32, whose loop
+    // waits for its matrix instructions and gains nothing: past one round of workgroups they cost 10 %, 2047 tokens, 1536 rows and columns, 133 and 147 us
+    // the mean with a K of 4096)
     constexpr int RR = KS == 1 ? 2 : direct_rows(SET * KS, RW, TW), PAIRS = RR / 2 * TW, PJ = KS == 1 ? TW : (PAIRS + KS - 1) / KS, NP = RW / RR * PJ;
-    constexpr bool HELD = EPI == ST_RESID && NP <= 8 && KS <= 4;
+    constexpr bool HELD = EPI == ST_RESID && sizeof(T) == 2 && NP <= 8 && KS <= 4;
     [[maybe_unused]] const bool ahead = HELD && (P.ldo & 3) == 0 && (P.rows & 15) == 0;
     [[maybe_unused]] f32x4 held[HELD ? 2 * NP : 1];
     if constexpr (HELD)
