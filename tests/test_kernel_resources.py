@@ -15,7 +15,8 @@ RESIDENT = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1,
 
 
 # kernel<template arguments>, bytes of scratch a lane at most
-SPILLED = [("gla_seg_kernel<float, 4, 2, 8, true, 4>", 0), ("gla_seg_kernel<float, 4, 4, 8, true, 4>", 0), ("gla_seg_kernel<float, 8, 4, 8, true, 1>", 0),
+SPILLED = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 20), ("pgemm_kernel<2, 8, 2, 1, 2, 0>", 0),
+           ("gla_seg_kernel<float, 4, 2, 8, true, 4>", 0), ("gla_seg_kernel<float, 4, 4, 8, true, 4>", 0), ("gla_seg_kernel<float, 8, 4, 8, true, 1>", 0),
            ("gla_seg_kernel<float, 4, 2, 16, true, 1>", 0), ("gla_seg_kernel<float, 8, 4, 16, true, 1>", 0), ("gla_seg_kernel<float, 16, 4, 16, true, 1>", 92),
            ("gla_seg_kernel<float, 16, 4, 16, false, 1>", 0)]
 
@@ -59,6 +60,6 @@ def test_workgroups_a_compute_unit(kernels, name, waves, groups):
 
 
 @pytest.mark.parametrize("name,most", SPILLED)
-def test_scratch_of_the_stack_family(stack_kernels, name, most):
-    k, = [v for n, v in stack_kernels.items() if name in n]
+def test_scratch(kernels, stack_kernels, name, most):
+    k, = [v for n, v in {**kernels, **stack_kernels}.items() if name in n]
     assert int(k["private_segment_fixed_size"]) <= most, k
