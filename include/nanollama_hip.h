@@ -195,8 +195,11 @@ NL_API int nl_memory_usage(nl_handle h, uint64_t *weights, uint64_t *kv_cache, u
 /* Read back a device state buffer for tests ("x","q","xb2","hb","logits",
  * "k_cache","v_cache"), or, as one float, which kernels the last multi-token step
  * ran on ("step_path": 1 | 2 decode-batch / short-step GEMM, 4 | 8 attention of a
- * prompt / of a decode batch in one launch; layer-stack models "one_query": layers
- * whose queries took one launch); returns floats copied (<= max_floats). */
+ * prompt / of a decode batch in one launch, 16 its images from the projections, 32
+ * folded norms, 64 decode attention with eight wavefronts; "num_cus": the
+ * device's compute units; layer-stack models "one_query": layers
+ * whose queries took one launch, "prompt_tiles": the tiles of a prompt's products);
+ * returns floats copied (<= max_floats). */
 NL_API int64_t nl_debug_read(nl_handle h, const char *which, int stream, float *out, int64_t max_floats);
 
 /* Shader-clock phase stamps of one GEMV launch (developer tool, tools/phase_probe.py). */

@@ -136,7 +136,8 @@ struct Op {
 
 // nl_engine::step_path: which kernels a layer of a multi-token step ran on (none of the first two: qgemm_kernel / pgemm_kernel, by matrix)
 enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */,
-       PATH_IMAGES = 16 /* the projections of a prompt wrote the attention's K and V^T images */ };
+       PATH_IMAGES = 16 /* the projections of a prompt wrote the attention's K and V^T images */, PATH_FOLD = 32 /* norms folded around the GEMMs */,
+       PATH_ATTN_WIDE = 64 /* decode attention with eight wavefronts a workgroup */ };
 
 struct nl_engine {
     nl_config cfg{};
@@ -523,9 +524,10 @@ GemvParams base_params(const nl_engine *e, const PackedMat &m, int mats = 1) {
 // them and four do as well with fewer barriers.  us a step, four and eight wavefronts: one stream of 841M Q8_0 at position 700 792 and 779, of 173M Q4_0 421 and 410;
 // 64 streams of 841M Q4_0 at 60 (384 workgroups) 1308 and 1273, at 200 (768) 1505 and 1526, at 900 (3072) 2227 and 2297; 24 of 841M Q8_0 at 200 (288) 1366 and
 // 1359, of 173M Q4_0 at 900 (576) 880 and 885.  (Eight heads: att_threads.)
+bool attn_wide(int gqa, dim3 grid, int num_cus) { return att_threads(gqa) > 256 && (long long)grid.x * grid.y * grid.z <= 2ll * num_cus; }
 template <int HD, bool FIN, bool ROPE>
 hipError_t launch_attn_as(int gqa, AttnParams P, dim3 grid, int num_cus, hipStream_t st) {
-    const bool wide = (long long)grid.x * grid.y * grid.z <= 2ll * num_cus;
+    const bool wide = attn_wide(gqa, grid, num_cus);
     auto go = [&](auto g) {
         constexpr int G = decltype(g)::value;
         if (wide) hipLaunchKernelGGL((attn_kernel<HD, G, FIN, ROPE, att_threads(G)>), grid, dim3(att_threads(G)), 0, st, P);
@@ -2109,7 +2111,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         P.xf = in; P.out = b.x; P.bias = bias;
         return sg_launch<QG_EPI_PLAIN>(m.wtype, P, st);
     };
-    e->step_path = dg ? PATH_DGEMM : sg ? PATH_SGEMM : 0;
+    e->step_path = (dg ? PATH_DGEMM : sg ? PATH_SGEMM : 0) | (fold ? PATH_FOLD : 0);
     const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
     // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs of Q4_0 files (pgemm_kernel) and the
     // prompt attention multiply only the fp16 hi half of every activation / probability -- half / a third of the matrix work,
@@ -2220,13 +2222,16 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_form = form(L.wo);
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
-                LCK(launch_attn_fin(hd, e->gqa, P, dim3(e->KVs, 1, n), e->num_cus, st));
+                const dim3 grid(e->KVs, 1, n);
+                LCK(launch_attn_fin(hd, e->gqa, P, grid, e->num_cus, st));
                 merged = true;
-                e->step_path |= PATH_ATTN_FIN;
+                e->step_path |= PATH_ATTN_FIN | (attn_wide(e->gqa, grid, e->num_cus) ? PATH_ATTN_WIDE : 0);
             } else {
                 if (rope_in_attn)
                     P.rp = AttnParams::Rope{1, qkv_out, (int)R, e->Hs, c.rope_conjugate, e->rope_cos, e->rope_sin, L.bq, L.bk, L.bv, kc, vc};
-                LCK(launch_attn(hd, e->gqa, P, dim3(e->KVs, nsplit, n), e->num_cus, st));
+                const dim3 grid(e->KVs, nsplit, n);
+                LCK(launch_attn(hd, e->gqa, P, grid, e->num_cus, st));
+                e->step_path |= attn_wide(e->gqa, grid, e->num_cus) ? PATH_ATTN_WIDE : 0;
             }
             if (!merged) {
             const bool tile16 = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;
@@ -3928,6 +3933,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     const float *src = nullptr;
     int64_t n = 0;
     std::string w = which;
+    if (w == "num_cus") { if (max_floats < 1) return 0; out[0] = (float)e->num_cus; return 1; }
     if (w == "step_path") { if (max_floats < 1) return 0; out[0] = (float)e->step_path; return 1; }      // (host state)
     if (w == "x") { src = e->x[0]; n = e->cfg.dim; }
     else if (w == "x1") { src = e->x[1]; n = e->cfg.dim; }

@@ -471,6 +471,9 @@ inline XcdTiles xcd_tiles(int nrb, int ntb, int row_bytes, int tok_bytes) {
     return best;
 }
 
+// The tiles that a launch sequence's prompt products ran on, rows x tokens (nl_debug_read "prompt_tiles")
+enum { PT_32_64 = 1, PT_64_64 = 2, PT_96_128 = 4, PT_192_256 = 8, PT_256_256 = 16, PT_MANY_64 = 32, PT_MANY_128 = 64 };
+
 struct MatParams {
     const void *W;         // [nrt][nks] operand tiles; ST_GATED: gate tile, up tile, gate tile, ...
     const void *X;         // [token tiles][nks]
@@ -506,6 +509,7 @@ struct MatParams {
     const float *nss;
     int nss_n;
     Ahead ahead;
+    int *tiles_ran;        // host memory: PT_* bits of the launches, or null
 };
 
 // a folded norm's partial sums of one token: row tiles from, from + step, ...; the first NB of them are requested by first() and added by sum()
@@ -1130,6 +1134,7 @@ hipError_t launch_many(const MatParams &P, hipStream_t st, TAIL tail = {}) {
     const int ntb = (P.n_tokens + 127) / 128;
     auto go = [&](auto kfn, int rt, int lds) {
         const XcdTiles xt = xcd_tiles((P.nrt + rt - 1) / rt, ntb, rt, 8);
+        if (P.tiles_ran) *P.tiles_ran |= rt == 8 ? PT_MANY_128 : PT_MANY_64;
         hipLaunchKernelGGL(kfn, dim3(xt.blocks() + (TAIL::on ? (tail.units + 3) / 4 : 0)), dim3(256), lds, st, P, xt, tail);
         return hipGetLastError();
     };
@@ -1145,6 +1150,7 @@ hipError_t launch_direct(const MatParams &P, hipStream_t st) {
     static_assert(lds <= 65536, "what a launch has without asking");
     const int nrb = (P.nrt + WR * RW - 1) / (WR * RW), ntb = ((P.n_tokens + 15) / 16 + WT * TW - 1) / (WT * TW);
     const XcdTiles xt = xcd_tiles(nrb, ntb, WR * RW, WT * TW);
+    if (P.tiles_ran) *P.tiles_ran |= WR * RW == 2 ? PT_32_64 : WR * RW == 4 ? PT_64_64 : WR * RW == 6 ? PT_96_128 : WR * RW == 12 ? PT_192_256 : PT_256_256;
     hipLaunchKernelGGL((direct_kernel<T, EPI, WR, WT, KS, RW, TW>), dim3(xt.blocks()), dim3(WR * WT * KS * 64), lds, st, P, xt);
     return hipGetLastError();
 }

@@ -114,6 +114,7 @@ struct nl_engine {
     int ids_cap = 1024;
     float *h_logits = nullptr;
     std::vector<int> next_pos;   // per stream: the position its next token must have (or 0)
+    int prompt_tiles = 0;        // tiles of the last launch sequence's prompt products (PT_* bits; nl_debug_read "prompt_tiles")
     int one_query = 0;           // layers of the last launch sequence whose queries took one launch (nl_debug_read "one_query")
     struct Graph { hipGraph_t g; hipGraphExec_t x; int one_query; };
     std::map<std::tuple<int, int, int>, Graph> graphs;
@@ -347,7 +348,7 @@ struct StepIn {                  // one launch sequence
 
 MatParams product_params(nl_engine *e, const Mat &m, const void *X, int n) {
     MatParams P{};
-    P.W = m.w; P.X = X; P.nks = m.nks; P.nrt = m.nrt; P.n_tokens = n; P.rows = m.rows; P.neps = e->c.eps;
+    P.W = m.w; P.X = X; P.nks = m.nks; P.nrt = m.nrt; P.n_tokens = n; P.rows = m.rows; P.neps = e->c.eps; P.tiles_ran = &e->prompt_tiles;
     return P;
 }
 
@@ -519,7 +520,7 @@ hipError_t launch_sequence(nl_engine *e, const StepIn &s) {
     e->xcur = e->x;
     e->pend = nullptr;
     e->folded = false;
-    e->one_query = 0;
+    e->one_query = e->prompt_tiles = 0;
     E.table = e->embed.w; E.tok = s.tok; E.nks = e->nksd; E.dim = D; E.scale = e->c.embed_scale; E.x = e->x; E.x0 = e->x0;
     hipLaunchKernelGGL(lookup_kernel<T>, dim3(s.n), dim3(256), 0, st, E);
     for (size_t r = 0; r < e->runs.size(); r++) {
@@ -1407,6 +1408,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     }
     const float *src = nullptr;
     int64_t n = 0;
+    if (!strcmp(which, "prompt_tiles")) { if (max_floats < 1) return 0; out[0] = (float)e->prompt_tiles; return 1; }
     if (!strcmp(which, "one_query")) { if (max_floats < 1) return 0; out[0] = (float)e->one_query; return 1; }      // (host state)
     if (!strcmp(which, "x")) { src = e->xcur ? e->xcur : e->x; n = e->c.dim; }
     else if (!strcmp(which, "logits")) { src = e->logits; n = e->c.vocab; }

@@ -231,13 +231,14 @@ def test_more_wanted_rows_than_one_logits_buffer(base):
 # Prompts whose products take many_kernel's 128 x 128 tiles, 192 x 256 and 256 x 256 ones (one and two rounds of them), and 96 x 128 with the residual rows
 # requested early; ragged tiles either way, widths of whole and of partial row tiles, both activations, with and without biases.
 @pytest.mark.parametrize("family", ["ganidra", "pabalix"])
-@pytest.mark.parametrize("width,ff,n", [(100, 2752, 1300), (96, 2064, 2030), (96, 4104, 1400), (96, 5504, 2047), (1056, 1100, 2047)])
-def test_prompt_tiles(family, width, ff, n):
+@pytest.mark.parametrize("width,ff,n,tiles", [(100, 2752, 1300, 64), (96, 2064, 2030, 8), (96, 4104, 1400, 16), (96, 5504, 2047, 8), (1056, 1100, 2047, 4)])
+def test_prompt_tiles(family, width, ff, n, tiles):
     cfg = lconfig([lat(ff=ff)], width=width) if family == "pabalix" else config([gla(ff=ff)], width=width)
     w = weights(cfg, 5)
     ids = tokens(n, seed=n)
     m = load(cfg, w, "bfloat16", max_streams=1, seq_len=2048)
     assert rel(whole(m, ids), so.forward(cfg, floats(w), ids)) < BF16_TOL
+    assert int(m.debug_read("prompt_tiles", 1)[0]) & tiles                      # (PT_*, nl_mfma.h)
     m.close()
 
 

@@ -63,3 +63,9 @@ def test_workgroups_a_compute_unit(kernels, name, waves, groups):
 def test_scratch(kernels, stack_kernels, name, most):
     k, = [v for n, v in {**kernels, **stack_kernels}.items() if name in n]
     assert int(k["private_segment_fixed_size"]) <= most, k
+
+
+def test_float32_products_hold_no_residual_rows(stack_kernels):
+    # ST_RESID takes the registers of ST_F32: rows requested in front of its loop were sixteen more
+    plain, resid = ([int(v["vgpr_count"]) for n, v in stack_kernels.items() if f"direct_kernel<float, {epi}, 1, 1, 4, 4, 4>" in n] for epi in (0, 1))
+    assert len(plain) == len(resid) == 1 and resid <= plain
