@@ -28,7 +28,9 @@ constexpr int TR = 16;           // rows per tile
 constexpr int KL = 4;            // k-lanes per wavefront (64 / TR)
 constexpr int PAIR = 64;         // columns per pair
 constexpr int ATT_CH = 128;      // positions per attention split
-// most threads of a workgroup of the decode attention, by query heads of a kv group: at eight heads the partial rows of 32 row groups no longer fit K's LDS
+// most threads of a workgroup of the decode attention, by query heads of a kv group: at eight heads of 64 the partial rows of 32 row groups no longer fit K's
+// LDS.  Heads of 32 have 64 row groups at 512 threads; with three or four heads a group those rows take an array of their own (45 and 54 KB a workgroup), which
+// the two workgroups a compute unit that such launches are made for can have.
 constexpr int att_threads(int g) { return g <= 4 ? 512 : 256; }
 constexpr int CTL_TOKEN = 0, CTL_POS = 1, CTL_CHAIN = 2, CTL_STEP = 3, CTL_STREAM = 4, CTL_HOSTOUT = 5, CTL_WORDS = 8;
 
@@ -1288,8 +1290,10 @@ __global__ void __launch_bounds__(NT) attn_kernel(AttnParams P) {
 #pragma unroll
             for (int gi = 0; gi < GH; gi++) d[gi][0] = d[gi][1] = d[gi][2] = d[gi][3] = 0.f;
             // (sixteen dims per round of LDS reads, 32 of a single head: one-float4-at-a-time left a dependent LDS round trip per step, 3.8k of a
-            // decode-batch launch's 15k cycles)
-            constexpr int DR = GH == 1 ? 8 : 4;
+            // decode-batch launch's 15k cycles.  Sixteen at four wavefronts of heads of 32, where registers and not LDS bound what a SIMD holds: 58 to 70
+            // instead of 88 to 92.  64 streams, six layers, us a step with 32 and 16: 24 kv heads at position 60 238 and 231, at 200 332 and 331, at 900 592 and 600;
+            // twelve of two query heads 213 and 209, 264 and 260, 428 both)
+            constexpr int DR = GH == 1 && !(HD == 32 && NT == 256) ? 8 : 4;
 #pragma unroll 1
             for (int d0 = 0; d0 < HD; d0 += 4 * DR) {      // (not unrolled: hipcc otherwise hoists every round's reads -- 230+ registers)
                 float4 kv[DR], qv[GH][DR];

@@ -12,7 +12,9 @@ LLVM = "/opt/rocm/llvm/bin/"
 
 # kernel<template arguments>, wavefronts of a workgroup, workgroups on a compute unit (512 registers a SIMD lane over four SIMDs, 160 KB of LDS)
 RESIDENT = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 1, 0>", 4, 3), ("pgemm_kernel<2, 4, 1, 1, 2, 0>", 4, 3)]
-
+# decode attention of heads of 32 at four wavefronts: as many workgroups as LDS holds, eight; seven where the rotation comes with it
+RESIDENT += [(f"attn_kernel<32, {g}, {fin}, {rope}, 256>", 4, 7 if rope == "true" else 8)
+             for g in (1, 2) for fin, rope in (("false", "false"), ("false", "true"), ("true", "true"))]
 
 # kernel<template arguments>, bytes of scratch a lane at most
 SPILLED = [("pgemm_kernel<2, 4, 1, 1, 0, 0>", 20), ("pgemm_kernel<2, 8, 2, 1, 2, 0>", 0),
