@@ -1042,22 +1042,31 @@ __device__ __forceinline__ float embed_value(const uint8_t *table, int wtype, in
 // row `token`, plus its gamma row, to x, by a whole workgroup.  A lone workgroup's lookup is memory round trips and nothing else, so a thread asks
 // for four elements at once (clamped index, masked store): that takes a choice of the format around the loads, not between them.
 // (4096 columns of Q4_0: 12.3 us by 256 threads with a choice per element, 5.3 by 1024 so; past 1024 columns 1024 threads have the row in a round.)
+// Where a row has fewer elements than that, one or two: asked for four times, a short row behind the argmax of a greedy chain cost it 0.1 to 0.6 us a token
+// (two layers, us a token with four always, so, and with a choice per element: Q4_0 512 columns 35.0, 34.5, 34.6, 1024 43.4, 42.7, 42.9, 2048 52.2, 51.8, 52.1; Q4_K 512
+// 44.9, 44.4, 44.9; Q6_K 1536 49.5, 48.9, 49.5).
 __device__ __forceinline__ void embed_row(const uint8_t *table, int wtype, int dim, int token, const int *gamma_row, const float *gamma_val, float *x) {
     const int gr = gamma_row ? gamma_row[token] : -1, nthr = blockDim.x;
     auto rows = [&](auto type) {
         constexpr int WT = decltype(type)::value;
-        for (int i0 = threadIdx.x; i0 < dim; i0 += 4 * nthr) {
-            float v[4];
+        auto each = [&](auto per) {
+            constexpr int N = decltype(per)::value;
+            for (int i0 = threadIdx.x; i0 < dim; i0 += N * nthr) {
+                float v[N];
 #pragma unroll
-            for (int k = 0; k < 4; k++) v[k] = embed_value(table, WT, dim, token, min(i0 + k * nthr, dim - 1));
-            if (gr >= 0) {
+                for (int k = 0; k < N; k++) v[k] = embed_value(table, WT, dim, token, min(i0 + k * nthr, dim - 1));
+                if (gr >= 0) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) v[k] += gamma_val[(long long)gr * dim + min(i0 + k * nthr, dim - 1)];
+                    for (int k = 0; k < N; k++) v[k] += gamma_val[(long long)gr * dim + min(i0 + k * nthr, dim - 1)];
+                }
+#pragma unroll
+                for (int k = 0; k < N; k++)
+                    if (i0 + k * nthr < dim) x[i0 + k * nthr] = v[k];
             }
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (i0 + k * nthr < dim) x[i0 + k * nthr] = v[k];
-        }
+        };
+        if (dim <= nthr) each(std::integral_constant<int, 1>{});
+        else if (dim <= 2 * nthr) each(std::integral_constant<int, 2>{});
+        else each(std::integral_constant<int, 4>{});
     };
     using std::integral_constant;
     switch (wtype) {

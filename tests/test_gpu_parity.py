@@ -177,10 +177,10 @@ def _run_teacher_forced(hip, orc, path, tokens):
     return worst, scale
 
 
-@pytest.mark.parametrize("dim", [32, 992, 1056, 2080, 4128])
+@pytest.mark.parametrize("dim", [32, 256, 512, 544, 992, 1024, 1056, 2048, 2080, 4128])
 @pytest.mark.parametrize("wtype", ["q8_0", "q4_0", "f16", "f32"])
 def test_embedding_rows_of_every_width(hip, orc, tmp_path, wtype, dim):
-    # a thread of the lookup takes four elements of a row a round: rows of less than one round, of a round's remainder and of two workgroup sizes,
+    # a thread of the lookup takes one element of a row, two, or four a round: rows on both sides of each, of less than one round, of a round's remainder and of two workgroup sizes,
     # in the single step, behind the argmax of a chain and in a prompt
     path = str(tmp_path / "m.gguf")
     synth.generate_gguf(path, synth.ModelShape("emb", 1, dim, dim // 32, dim // 32, 64, seq_len=32, interm=64), wtype, 9)
