@@ -62,7 +62,14 @@ __device__ __forceinline__ void samp_embed_tail(const SampleParams &P, int token
     if (!P.embed) return;
     const EmbedParams &E = P.emb;
     if (E.epoch && threadIdx.x == 0) *E.epoch = *E.epoch + 1;            // the forward counter, as embed_kernel advances it
-    embed_row(E.table, E.wtype, E.dim, token, E.gamma_row, E.gamma_val, E.x);
+    // (an element a round, the format chosen in the loop: embed_row, a larger piece of code per format, costs this launch more than it saves -- us for 48 sampled
+    //  tokens: Q8_0, 576 columns 9925, by embed_row 9951 to 9964; Q4_0, 28 layers of 1536 32690 and 32780)
+    const int gr = E.gamma_row ? E.gamma_row[token] : -1;
+    for (int i = threadIdx.x; i < E.dim; i += blockDim.x) {
+        float v = embed_value(E.table, E.wtype, E.dim, token, i);
+        if (gr >= 0) v += E.gamma_val[(long long)gr * E.dim + i];
+        E.x[i] = v;
+    }
 }
 
 // device scratch of one sampler (one vocabulary)
