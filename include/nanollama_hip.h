@@ -198,7 +198,8 @@ NL_API int nl_memory_usage(nl_handle h, uint64_t *weights, uint64_t *kv_cache, u
  * prompt / of a decode batch in one launch, 16 its images from the projections, 32
  * folded norms, 64 decode attention with eight wavefronts; "num_cus": the
  * device's compute units; layer-stack models "one_query": layers
- * whose queries took one launch, "prompt_tiles": the tiles of a prompt's products);
+ * whose queries took one launch, "prompt_tiles": the tiles of a prompt's products,
+ * "splits": key-range splits of the last decode step);
  * returns floats copied (<= max_floats). */
 NL_API int64_t nl_debug_read(nl_handle h, const char *which, int stream, float *out, int64_t max_floats);
 

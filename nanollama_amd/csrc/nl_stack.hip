@@ -115,6 +115,7 @@ struct nl_engine {
     float *h_logits = nullptr;
     std::vector<int> next_pos;   // per stream: the position its next token must have (or 0)
     int prompt_tiles = 0;        // tiles of the last launch sequence's prompt products (PT_* bits; nl_debug_read "prompt_tiles")
+    int splits = 0;              // key-range splits of the last decode step (nl_debug_read "splits")
     int one_query = 0;           // layers of the last launch sequence whose queries took one launch (nl_debug_read "one_query")
     struct Graph { hipGraph_t g; hipGraphExec_t x; int one_query; };
     std::map<std::tuple<int, int, int>, Graph> graphs;
@@ -598,7 +599,9 @@ int run_sequence(nl_engine *e, const StepIn &s) {
     return NL_OK;
 }
 
-// key-range splits of a decode step: enough workgroups for the chip, at least 128 keys each, never more keys than one split holds
+// key-range splits of a decode step, the most that a layer wants.  Softmax attention: enough workgroups for the chip, at least 128 keys each, never more keys
+// than one split holds.  Latent attention: workgroups up to the compute units, down to one block of LT_KEYS keys each, past the last block none (such a
+// split has weight 0).
 int splits_for(const nl_engine *e, int n, int max_pos) {
     int out = 1;
     for (const Layer &L : e->layers) {
@@ -606,9 +609,10 @@ int splits_for(const nl_engine *e, int n, int max_pos) {
             const int wgs = n * ((L.d.latent.heads + 15) / 16), nb = max_pos / LT_KEYS + 1, want = std::min({256 / std::max(1, wgs), nb, LT_MAX_SPLITS});
             int p = 1;
             while (p * 2 <= want) p *= 2;
-            // up to sixteen splits of one block of keys, where each still finds a compute unit: one token of 20 layers of 768 columns at 200 639 us in four splits,
-            // 599 in eight, at 310 664 in eight, 643 in sixteen (24 streams at 310, 192 workgroups 1063, 384 1117; four at 900, sixteen 812, 32 822)
-            if (p < nb && p * 2 <= 16 && p * 2 * wgs <= 256) p *= 2;
+            // up to sixteen splits of one block of keys, as long as what the launch behind merges is little beside them: eight up to 128 workgroups, sixteen up to 64.
+            // us a step of 20 layers of 768 columns: one token at 200 in four splits 639, in eight 599, at 310 in eight 664, in sixteen 643; sixteen tokens at 200 954 and
+            // 949; four at 300 771 and 756, five 907 and 912, nine 933 and 966, sixteen 974 and 1041 (four at 900, sixteen 812, 32 822)
+            if (p < nb && p * 2 <= 16 && p * 2 * wgs <= (p * 2 <= 8 ? 128 : 64)) p *= 2;
             out = std::max(out, p);
         }
         if (!L.d.attn.heads) continue;
@@ -626,7 +630,7 @@ constexpr int CHAIN_STEPS = 16;
 
 // queue one decode step (kind CH_CHAIN: `steps` of them): from the batch arrays (CH_BATCH) or the control block
 int queue_decode(nl_engine *e, int kind, int n, int max_pos, int steps = 1) {
-    const int nsplit = splits_for(e, n, max_pos);
+    const int nsplit = e->splits = splits_for(e, n, max_pos);
     StepIn s;
     s.n = n; s.nsplit = nsplit; s.n_out = n; s.logits = e->logits;
     if (kind == CH_BATCH) { s.tok = e->d_meta; s.pos = e->d_meta + e->m_pos; s.stream = e->d_meta + e->m_stream; }
@@ -1409,6 +1413,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     const float *src = nullptr;
     int64_t n = 0;
     if (!strcmp(which, "prompt_tiles")) { if (max_floats < 1) return 0; out[0] = (float)e->prompt_tiles; return 1; }
+    if (!strcmp(which, "splits")) { if (max_floats < 1) return 0; out[0] = (float)e->splits; return 1; }
     if (!strcmp(which, "one_query")) { if (max_floats < 1) return 0; out[0] = (float)e->one_query; return 1; }      // (host state)
     if (!strcmp(which, "x")) { src = e->xcur ? e->xcur : e->x; n = e->c.dim; }
     else if (!strcmp(which, "logits")) { src = e->logits; n = e->c.vocab; }

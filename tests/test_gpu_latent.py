@@ -555,6 +555,23 @@ def test_many_streams_in_one_decode_batch(n, dtype):
     m.close()
 
 
+# Splits of a decode step by its workgroups (one a token up to sixteen heads): to eight of one block up to 128, to sixteen up to 64; one token's step
+# takes the most.  Every split of a position, and beyond it, against each stream by itself.
+@pytest.mark.parametrize("n,at,splits", [(1, 200, 8), (16, 200, 8), (17, 200, 4), (1, 310, 16), (4, 310, 16), (5, 310, 8), (16, 310, 8), (2, 40, 2), (2, 70, 4)])
+def test_splits_of_a_batch(n, at, splits):
+    cfg = lconfig([lat(2, ff=24), lat(1)])
+    w = weights(cfg, 7)
+    ids = [tokens(at + 1 if s == n - 1 else 3 + 9 * s, seed=s) for s in range(n)]
+    m = load(cfg, w, "float32", max_streams=n)
+    for s, t in enumerate(ids):
+        whole(m, t[:-1], [], s)
+    _, rows = m.forward_batch(list(range(n)), [t[-1] for t in ids], [len(t) - 1 for t in ids], want_logits=True)
+    assert m.debug_read("splits", 1)[0] == splits
+    for s, t in enumerate(ids):
+        assert rel(rows[s], so.forward(cfg, floats(w), t)[-1]) < F32_TOL, s
+    m.close()
+
+
 # the output launch either side of its k tiles a wavefront, of 8, 16 and 24 latents' tiles; one and four row tiles a workgroup (64 heads, 17 tokens);
 # 1 to 32 splits, ragged rows and latents, a sink and a gate
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
