@@ -426,7 +426,7 @@ struct BMergeParams {
 // online-softmax merge of the position splits (same arithmetic and summation order as the decode GEMV's
 // PRO_ATTN prologue); one thread per 8 k-slots of the output row.  The (max, sum) pairs of all splits and the
 // partial rows of four splits at a time are fetched with clamped indices before anything consumes them
-// (a runtime-bounded "for c < ns: load" loop is ns dependent round trips, DESIGN 4.6); splits past ns get weight 0.
+// (a runtime-bounded "for c < ns: load" loop is ns dependent round trips); splits past ns get weight 0.
 template <int MAXS>   // most partials an item can have: 16 (seq_len <= 2048, go/model.go:145-148, one per 128 keys), or 4 when the
                       // prompt attention kernel folded runs of chunks (12 of the 16 (max, sum) loads and weights were masked work)
 __global__ void battn_merge_kernel(BMergeParams P, int n_items) {
@@ -734,12 +734,15 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
 //     S^T accumulators leave P in registers (lane (row, kg) holds keys 16*mt + 4kg + e of key tile mt): P is converted
 //     in place, never moved, and V^T is read with one ds_read_b128 per operand.
 //   * Both are XOR-swizzled 16-byte segments of unpadded rows (Kv16Image): conflict-free under ds_read_b128's lane groups.
-//   * A workgroup folds a RUN of chunks with the online softmax in registers: log2 domain, two elements per instruction;
+//   * A workgroup folds a RUN of chunks with the online softmax in registers, in the log2 domain;
 //     p * 2^10 = hi (a mask) + lo, the running output as O^T = V^T P^T so that a query row stays in one lane column.
-//   * From 256 tokens on (SHADOW) the images are built once per layer by kv16_build_kernel and a workgroup takes 256 rows.
+//   * From 256 tokens on (SHADOW) the images are there before the launch, once per layer: from the Q|K|V launch (pgemm_kernel's RoPE epilogue: heads
+//     of 64, a prompt from position 0) or from kv16_build_kernel, and a workgroup takes 256 rows.  Of the last chunk, keys past the prompt are zeros in
+//     V^T; K's rows there are zeros from kv16_build_kernel and ANYTHING from the epilogue.  Their scores are therefore selected away, never
+//     masked by an addition or a product, and their probabilities are zeros.
 // Partials (max, sum, sum p*v) leave in the decode kernel's layout, one per run, so battn_merge_kernel is shared.
-// Measured (mini, 2047 tokens, per layer): 52 us attention + 15 us merge at the start of round 3 (one chunk per
-// workgroup, every workgroup converting its chunk) -> 31 + 6 (images) + 7 us.  What is left: the matrix, vector and LDS
+// Measured (mini, 2047 tokens, per layer): 52 us attention + 15 us merge with one chunk per workgroup, every workgroup
+// converting its chunk -> 29.4 + 1.4 (images, in the Q|K|V launch; 5.4 in one of their own) + 7.5 us.  What is left: the matrix, vector and LDS
 // pipes of a SIMD take turns -- all the wavefronts between two chunk barriers are in the same phase -- at ~38 % MFMA
 // busy (profiles/r03_prompt_attention.txt has the stamps, the census and the SQ counters of every step).
 #ifdef NL_ATT_STAMPS
@@ -900,12 +903,12 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
     c_count = min(c_count, maxpos / ATT_CH + 1 - c_first);
     const int lane = tid & 63, w = tid >> 6, j = lane & 15, kq = lane >> 4;
     ATT_STAMP(0);
-    // SHADOW: a chunk's images, built by kv16_build_kernel, go straight into LDS (global_load_lds_dwordx4: 1 KB per
+    // SHADOW: a chunk's images, in memory since before the launch, go straight into LDS (global_load_lds_dwordx4: 1 KB per
     // instruction, 64 per chunk) one chunk ahead of the arithmetic.  What bounds this kernel is the rate at which a CU
-    // pulls those images out of the L2 -- 11-13 B/clk (MI355X_MICROARCH.md, the prologue-burst row; measured here as
+    // pulls those images out of the L2 -- 11-13 B/clk (measured here as
     // ~5k cycles per 64 KB chunk however the requests were placed) against ~3k cycles of MFMA work per 128 rows -- so a
     // workgroup takes 256 rows (16 wavefronts, one workgroup per CU) per staged chunk and double-buffers the images.
-    // The DMA is issued from inline asm (cdna_hip_programming.md 5.7): hipcc counts a builtin LDS-DMA and drains it
+    // The DMA is issued from inline asm: hipcc counts a builtin LDS-DMA and drains it
     // (vmcnt(0)) in front of the next LDS read it cannot prove disjoint, i.e. right away; these it does not see, and the
     // one wait per chunk is written out.  Source = scalar base + one VGPR of lane offsets: a per-lane 64-bit address kept
     // across the loop is spilled by hipcc and reloaded from scratch behind every barrier.
@@ -1015,8 +1018,8 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
         // ---- online softmax of row j: 32 keys of this chunk in this lane, the rest in lanes j+16, j+32, j+48.  Chunks
         //      below the tile's diagonal see all 128 keys in every row (uniform test): no per-element masks there.
         //      The vector pipe is this kernel's busiest (SQ_INSTS_VALU x 4 cycles ~ 40 % of the launch, all of it on the
-        //      critical path of the longest runs), so everything is kept in the log2 domain and two elements per
-        //      instruction (v_pk_mul_f32 / v_pk_add_f32): t = s * (scale * log2 e); p * 2^10 = exp2(t + (10 - max)) on
+        //      critical path of the longest runs), so everything is kept in the log2 domain:
+        //      t = s * (scale * log2 e); p * 2^10 = exp2(t + (10 - max)) on
         //      v_exp_f32 (~1 ulp; the two roundings of the argument add < 1.5e-6 relative for |t| < 32); max and sum
         //      leave in natural units (max * ln 2, sum * 2^-10) ----
         //      (two separate instruction streams: with the masked variant merely branched around, hipcc hoists its 32

@@ -523,7 +523,8 @@ GemvParams base_params(const nl_engine *e, const PackedMat &m, int mats = 1) {
 // Eight wavefronts shorten the phases of a workgroup that waits for its own round trips; where more than two workgroups share a compute unit the others' hide
 // them and four do as well with fewer barriers.  us a step, four and eight wavefronts: one stream of 841M Q8_0 at position 700 792 and 779, of 173M Q4_0 421 and 410;
 // 64 streams of 841M Q4_0 at 60 (384 workgroups) 1308 and 1273, at 200 (768) 1505 and 1526, at 900 (3072) 2227 and 2297; 24 of 841M Q8_0 at 200 (288) 1366 and
-// 1359, of 173M Q4_0 at 900 (576) 880 and 885.  (Eight heads: att_threads.)
+// 1359, of 173M Q4_0 at 900 (576) 880 and 885.  Counted are the workgroups of the grid, whether they find keys or leave: a recorded step's grid has the
+// context's splits at every position, a ragged batch's the longest stream's, so a short position there takes four.  (Eight heads: att_threads.)
 bool attn_wide(int gqa, dim3 grid, int num_cus) { return att_threads(gqa) > 256 && (long long)grid.x * grid.y * grid.z <= 2ll * num_cus; }
 template <int HD, bool FIN, bool ROPE>
 hipError_t launch_attn_as(int gqa, AttnParams P, dim3 grid, int num_cus, hipStream_t st) {
@@ -2016,7 +2017,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     // run of consecutive 128-key chunks under the diagonal (AttnParams::live_map), and how many partials every token gets.
     // Run length: the shortest that lets every workgroup be resident at once (2 per CU); tiles are cut into equal runs.
     // Prompts of several query tiles (n >= NL_KV16_MIN_TOKENS): the chunks are split into fp16 halves once per layer
-    // (kv16_build_kernel) and a workgroup takes twice the rows, one workgroup per CU (AttnTile16ShadowQT).
+    // (kv16_build_kernel, or the Q|K|V launch) and a workgroup takes twice the rows, one workgroup per CU (AttnTile16ShadowQT).
     int n_live = 0, max_nparts = 0;
     bool kv16_on = false;
     const int exact = kquant_file(e) ? 1 : 0;
@@ -3044,7 +3045,7 @@ int nl_finalize(nl_handle e) {
         //  stay ahead of the five-launch plan through three passes -- 1.69 against 1.85 ms at position 470, 1.81 against 1.86 at
         //  600 -- and fall behind in the fourth, 1.98 against 1.87 at 900)
         //  (mode 3 runs the same attention half: 512 = two of its passes, where 384 was three of the old 128-position ones)
-        //  (round 5, the same tool with the feed-forward launch on the matrix pipe and its first round warm: 1.76 against 1.85 ms at
+        //  (the same tool with the feed-forward launch on the matrix pipe and its first round warm: 1.76 against 1.85 ms at
         //  position 800, 1.80 against 1.86 at 980 -- the two-launch layers now stay ahead through all four passes)
         e->fused_max_pos = fm ? atoi(fm) : e->fused_mode == 4 ? (e->wide_ffn ? 1024 : 768) : (e->fused_mode == 1 || e->fused_mode == 3) ? 512 : 384;
         {

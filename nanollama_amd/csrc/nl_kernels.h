@@ -1126,7 +1126,8 @@ struct AttnParams {
     // are a long run and a short one.
     const int *live_map;
     // ... and K / V^T arrive already split into fp16 hi / lo halves and laid out as the workgroup's LDS image, one image per
-    // (kv head, 128-key chunk), built once per layer by kv16_build_kernel (null: every workgroup converts its own chunks)
+    // (kv head, 128-key chunk), once per layer, by kv16_build_kernel or the Q|K|V launch (null: every workgroup converts its own chunks).  K's rows past the
+    // prompt may hold anything
     const uint4 *kv16;
     // FIN variant with the RoPE prologue (decode batches, nl_batch.h attn_rope_prologue): q / k / v of the step's tokens are
     // still the Q|K|V GEMM's output -- packed row order, possibly split-K slabs -- and this kernel rotates and stores them
@@ -1290,7 +1291,7 @@ __global__ void __launch_bounds__(NT) attn_kernel(AttnParams P) {
     ATTN_STAMP(2);
     // scores: thread (key row t, share gp of the group's heads) -> q.k over d.  The row is read once, as float4s, for all the
     // heads of the share; q is a broadcast read.  Per (t, g): four partial sums over d = 0, 4, 8, ... / 1, 5, ... / ..., the
-    // order the one-float-at-a-time loop of rounds 1-2 used (256 ds_read_b32 per thread against 48 ds_read_b128 now).
+    // order of a loop over one float at a time (which takes 256 ds_read_b32 per thread, this one 48 ds_read_b128).
     {
         constexpr int GH = (G + NQ - 1) / NQ;
         const int t = tid & (ATT_CH - 1), gp = tid / ATT_CH;

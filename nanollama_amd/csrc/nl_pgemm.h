@@ -24,12 +24,12 @@
 //   Q4_K                  z over q - 8; acc += d * scale * z and acc -= (dmin * min - 8 d * scale) * sum(x) per block, sum(x) by MFMAs against ones (go/quant.go:296-323)
 //   Q6_K                  scale * (q - 32) has 13 bits, two bf16 parts: six MFMAs; acc += d * z per block
 //
-// Measured (us a launch, weights and fragments in L2; beside it the kernels that these launches ran on before, inside a model): Q4_0, 2047
-// tokens, 768 columns: Q|K|V 15.5 (21.8), gate and up 31.8 (40.5), WO / down (2048 columns) 10.5 / 17.7 (mean 23.5); F16, 993 tokens, 1536
-// columns: 26.7 (35.6), 52.3 (85.0), 17.9 / 36.3 (mean 43.2); inside a model, profiled, 17.3, 36.3, mean 19.0 and 29.9, 57.0, mean 30.8; Q4_K, 333
-// tokens, 768 columns, PG_EXACT: 12.8, 22.8, mean 19.0.  A 64 x 64 tile's block costs a wavefront about 310 cycles: 128 on the matrix
-// pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses), which a SIMD does not overlap with MFMAs
-// (matrix and vector cycles add up); larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
+// Measured (us a launch inside a model, profiled; Q|K|V, gate and up, mean of WO and down; in brackets the kernels that these launches ran on
+// before): Q4_0, 2047 tokens, 768 columns: 18.9 (21.8), 37.2 (40.5), 18.5 (23.5); F16, 993 tokens, 1536 columns: 27.6 (35.6), 53.5 (85.0), 28.3
+// (43.2), Q|K|V of both with the attention's images; Q4_K, 333 tokens, 768 columns, PG_EXACT: 12.6, 22.0, 18.6.  A 64 x 64 tile's block costs a
+// wavefront about 310 cycles: 128 on the matrix pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses).  Those
+// overlap with the MFMAs of the SIMD's other wavefronts (1.47 PFLOP/s beside four vector instructions an MFMA) and not with its own, and a SIMD
+// holds two or three; larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
 // be 333 single-token steps: 151 ms, now 1.92 ms (1.49 with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
 // steps and 1.19e-7 now, and whose range ends at 65504).
 #pragma once
@@ -209,9 +209,10 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
 
     // F16 and Q8_0: a group of four pairs is two chunks, the even blocks of its pairs, then the odd ones.  A wavefront's load is then one 16-byte plane of
-    // all four pairs over a tile's rows, a whole KiB; two pairs with both their blocks (PAIRS) are half of every 64-byte run, twice the sectors.  F16, 993
-    // tokens, 1536 columns: Q|K|V 30.8 us, now 25.0, gate and up 61.5 and 57.5, WO 19.4 and 17.6, down 41.1 and 35.5; Q8_0, 700 tokens: 19.9 and 19.2, 53.9
-    // and 52.5, 17.2 and 16.7, 35.7 and 35.0.  Q4_0's blocks are one plane, K-quants' two share their bytes: nothing to gain (17.3 and 17.6, 11.8 and 11.9).
+    // all four pairs over a tile's rows, a whole KiB; two pairs with both their blocks (PAIRS) are half of every 64-byte run, twice the sectors.  Profiled
+    // inside a model, Q|K|V / gate and up / mean of WO and down: F16, 993 tokens, 1536 columns 29.9 / 57.0 / 30.8 us, now 27.6 / 53.5 / 28.3; Q8_0, 700 tokens
+    // 20.9 / 53.3 / 28.5, now 20.8 / 50.4 / 26.4 (and Q|K|V writes the attention's images now).  Q4_0's blocks are one plane, K-quants' two share their bytes:
+    // nothing to gain (Q|K|V 17.3 and 17.6, 11.8 and 11.9).
     // A last group of one or two pairs is one chunk of both their blocks.
     // staging items: block kk of the chunk, row r, row tile
     const int i_kk = PAIRS ? 2 * (tid & 1) + ((tid >> 5) & 1) : tid & 3, i_r = (PAIRS ? tid >> 1 : tid >> 2) & 15, i_t = wave;
