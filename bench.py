@@ -39,7 +39,7 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-HBM_PEAK_GBS = 8000.0  # /opt/skills/guides/MI355X_MICROARCH.md: HBM3E 8.0 TB/s spec
+HBM_PEAK_GBS = 8000.0  # HBM3E, 8.0 TB/s by its specification
 PROMPT_LEN = 8
 SEGMENT = 128  # greedy 128-token decode
 REPEATS = 5
@@ -84,7 +84,7 @@ def launch_ranks(n, argv, timeout_s=None):
 # ------------------------------------------------------------------ measurement ---
 
 def kernel_bytes(shape, wtype, pos, tp=1, wo_in_block=None):
-    """Algorithmic HBM bytes per LAUNCH of each kernel kind (DESIGN.md section 4):
+    """Algorithmic HBM bytes per LAUNCH of each kernel kind:
     every weight byte once + the vectors the kernel must read/write."""
     from nanollama_amd import gguf, synth
     t = synth.WTYPES[wtype]
@@ -172,7 +172,7 @@ ID_MARGIN = 1e-3   # a greedy id may differ from the CPU engine's only where the
 
 
 def ids_check(cpu, dev_first, dev_ids):
-    """the device's greedy ids against the ids the CPU baseline generated on the same file (the same
+    """The device's greedy ids against the ids the CPU baseline generated on the same file (the same
     prompt, the same first token): equal one for one, up to a step where the CPU engine's own top-2 margin is < ID_MARGIN
     (after such a step the two runs are different texts and the comparison stops)."""
     ids, margins = cpu.pop("_ids"), cpu.pop("_margins")
@@ -219,7 +219,7 @@ def dropin_lib():
 
 
 def dropin_rates(dev, first, pos0, n, chained_ids):
-    """VERDICT r3 item 3b: tok/s of the per-token loops -- nl_forward + host argmax (what integration/go/model_hip.patch gives an
+    """tok/s of the per-token loops -- nl_forward + host argmax (what integration/go/model_hip.patch gives an
     UNMODIFIED Engine.Generate, go/main.go:173-219) and nl_forward_argmax -- next to the chained nl_decode_greedy headline."""
     import ctypes as C
     import numpy as np
@@ -372,7 +372,7 @@ def run_workload(tier, wtype, rdv, steps, warmup, profile_pos, model, tp=True, c
         step_gbs = step_bytes / (ms_per_step * 1e-3) / 1e9
         # The smallest tier's greedy chain is ONE persistent launch per segment (nl_persist.h): that launch IS the timed region's
         # dominant kernel.  Its duration is measured live with HIP events on the engine's stream around single launches of the
-        # timed segment; achieved = algorithmic bytes of the segment's tokens (SURVEY 8d: weights + f32 KV read per token, each
+        # timed segment; achieved = algorithmic bytes of the segment's tokens (weights + f32 KV read per token, each
         # byte counted once per token although the weights stay on chip for the whole launch) / that duration.
         pinfo = dev.persist_info() if world == 1 and not shard_of else {"ready": False}
         persist_roof = None
@@ -437,7 +437,7 @@ def run_workload(tier, wtype, rdv, steps, warmup, profile_pos, model, tp=True, c
 
 
 def prefill_x1(dev, toks, dt_hilo, gemm_flop):
-    """The same prompt in the single-product precision mode (NL_PREFILL_PRECISION=fp16x1, DESIGN.md): time, and its logits
+    """The same prompt in the single-product precision mode (NL_PREFILL_PRECISION=fp16x1): time, and its logits
     against the default hi + lo mode's on this device (the hi + lo mode is the one held to 1e-4 against the CPU engine)."""
     import numpy as np
     dev.reset()
@@ -621,7 +621,7 @@ def side_configs(model):
 
 
 def shard_probe(model, rdv, ns=(2, 4, 8), seam_us=2.0, steps=96, warmup=16, base=None):
-    """per-rank step time of big Q4_0 at tp_size N with NO contention -- rank 0's shard alone on
+    """Per-rank step time of big Q4_0 at tp_size N with NO contention -- rank 0's shard alone on
     this GPU with the real tensor-parallel plan (grids, granule stores into its own receive slots, polls;
     nl_p2p_loopback), only the xGMI hop missing.  predicted = per-rank time + 2 L seams x an ASSUMED wire latency
     (seam_us per seam: no xGMI figure has been measured by this repo) -- a prediction, labelled as such."""
@@ -921,7 +921,7 @@ def main():
                 if b.get("dropin"):
                     out["secondary"]["dropin_forward_loop"] = b["dropin"]
                 if not args.no_cpu_baseline:
-                    # north_star tabulates both tiers next to the CPU engine; SURVEY 8(d) allows a shortened run for big
+                    # both tiers stand next to the CPU engine; a shortened run does for big
                     out["secondary"]["cpu_baseline"] = cpu_baseline(b["path"], b["prompt"], budget_s=12.0, min_tokens=4, max_tokens=16)
                     out["secondary"]["greedy_ids_vs_cpu"] = ids_check(out["secondary"]["cpu_baseline"], b["first_id"], b["head_ids"])
                     if not out["secondary"]["greedy_ids_vs_cpu"]["ids_match_cpu"]:
@@ -964,7 +964,7 @@ def main():
     tp_res, transport, notes = None, None, []
     watchdog = None
     if not args.no_secondary:
-        # The tensor-parallel wire has never run across devices on this repository's test pool (DESIGN.md section 7): whatever it
+        # The tensor-parallel wire has never run across devices on this repository's test pool: whatever it
         # does on the real node -- every poll in it is bounded, RCCL runs in guarded children -- it must not take the measured
         # headline with it.  Past the deadline every rank leaves; rank 0 prints the line it has.
         import threading
@@ -1004,7 +1004,7 @@ def main():
                     if not d <= tol:
                         err = f"tensor-parallel logits differ from the 1-GPU logits by {d:.3g} (tolerance {tol:.3g})"
                     # ... and the first greedy ids (16-step graphs, argmax exchange, logits gather) must be the 1-GPU ids: the
-                    # cross-device wire has never been validated by a test on this repo's 1-GPU pool (DESIGN.md section 7)
+                    # cross-device wire has never been validated by a test on this repo's 1-GPU pool
                     elif list(cand.get("head_ids", []))[:8] != list(ref1.get("head_ids", []))[:8]:
                         err = f"tensor-parallel greedy ids {cand.get('head_ids', [])[:8]} differ from the 1-GPU ids {ref1.get('head_ids', [])[:8]}"
                 failed = rdv.max_over_ranks(1.0 if (cand is None or err) else 0.0, tag="vote:p2p") > 0

@@ -4,7 +4,7 @@
  *
  * The reference (ariannamethod/nanollama, go/) is single-package pure Go with
  * no FFI; the seams this ABI replaces are the three methods the Go host calls
- * on its model object (SURVEY.md section 8b):
+ * on its model object:
  *
  *   LoadLlamaModel(gguf)            go/model.go:121   -> nl_create + nl_upload_tensor* + nl_finalize
  *   (*LlamaModel).Forward(tok,pos)  go/model.go:490   -> nl_forward   (fills the caller's Logits slice)
@@ -153,7 +153,7 @@ NL_API int nl_sample_decode(nl_handle h, int stream, int pos, int n_steps, const
 /* Prompt prefill (go/main.go:160-166 feeds the prompt token-at-a-time through Forward): runs
  * tokens[0..n) at positions pos0..pos0+n-1 of `stream` back to back on the device with no host
  * round trip; last_logits_out (may be NULL) receives the logits after the last token.  Q4_0 / Q8_0 / Q5_0 / F16 / Q4_K / Q6_K
- * models take the multi-token matrix-core path (up to 2048 tokens per step, DESIGN.md 4.2-4.3): the KV
+ * models take the multi-token matrix-core path (up to 2048 tokens per step): the KV
  * cache and logits agree with n nl_forward calls to the stated logit tolerance (1e-4, summation order
  * and an fp16 hi+lo activation split differ), greedy continuations are identical; files with Q4_K / Q6_K matrices keep float32
  * operands and range there; F32 matrices, and F16 ones beside Q4_K / Q6_K, run the single-token plan n times (bitwise equal).  pos0 + n must be <= seq_len. */

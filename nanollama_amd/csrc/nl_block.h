@@ -9,7 +9,7 @@
 //     RMSNorm(x) -> each member projects one 16-row tile of q, of k and of v (the k / v rows of a GQA group are
 //     recomputed by every head of the group: the work is latency, not bytes) -> bias, RoPE -> the members exchange
 //     their 3 x 16 values through 8-byte {tag, value} granules (the only cross-workgroup step: 192 values per head,
-//     cdna_hip_programming.md G16 form R2; cluster members are the blocks b, b+8, b+16, b+24, which the dispatcher
+//     each its own flag; cluster members are the blocks b, b+8, b+16, b+24, which the dispatcher
 //     happens to place on one XCD -- observed, used for speed only, never relied on) -> QK-norm -> KV store (first
 //     head of the group) -> every member runs the head's softmax
 //     attention over the cache (the cache rows come from L2) -> each member multiplies ITS quarter of the head's

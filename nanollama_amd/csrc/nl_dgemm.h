@@ -19,7 +19,7 @@
 //   * Everything a wavefront multiplies is requested at its first instruction: its NS activation fragment pairs straight into
 //     registers (global_load_dwordx4 sc1: the fragment store is in MFMA operand order, and a load that skips the vector L1
 //     streams L2-resident data at 110 GB/s per compute unit against 37 through the L1 and 25-45 measured here through
-//     LDS-DMA: EXPERIMENTS, tools/ingest_probe.hip), its NS x T x (256 B of nibbles + 64 B of fp16 scale words) by LDS-DMA
+//     LDS-DMA: tools/ingest_probe.hip), its NS x T x (256 B of nibbles + 64 B of fp16 scale words) by LDS-DMA
 //     (the source picked per lane) into its own LDS area.  The issue order is static, so "step s has landed" is one
 //     s_waitcnt vmcnt(immediate) on the wavefront's own counter (loads return in order).
 //   * The nibbles of (block, tile) land as [row][16 B]: the B-operand read -- dword lq of row li -- is conflict-free.  The
@@ -78,8 +78,8 @@ __device__ unsigned g_dg_log_n;
 #endif
 
 // cache policy of the LDS-DMA pieces (CPol bits of global_load_lds: 1 = sc0, 2 = nt, 16 = sc1).  The vector L1's fill path gives
-// a compute unit 37 GB/s of L2-resident data whatever is in flight; loads that skip the L1 (a scope bit) reach 110 (EXPERIMENTS,
-// tools/ingest_probe.hip) -- and every byte here is used once per compute unit, so the L1 has nothing to offer.
+// a compute unit 37 GB/s of L2-resident data whatever is in flight; loads that skip the L1 (a scope bit) reach 110
+// (tools/ingest_probe.hip) -- and every byte here is used once per compute unit, so the L1 has nothing to offer.
 #ifndef DG_AUX
 #define DG_AUX 16
 #endif

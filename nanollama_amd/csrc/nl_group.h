@@ -4,7 +4,7 @@
 // kv group), so the projection keeps its chip-wide spread -- one or two 16-row tiles per workgroup, 16 wavefronts
 // splitting the columns -- and only the tiny attention step is pulled in: the workgroups that hold the tiles of one kv
 // group form a cluster (blocks with equal index mod 8: one XCD as observed -- speed only; a poll that gives up makes the host redo the step on the general plan), publish their rows as 8-byte {tag, value} granules
-// (cdna_hip_programming.md G16 form R2), and G of them -- one per query head of the group -- gather q, k, v and run the
+// (each its own flag), and G of them -- one per query head of the group -- gather q, k, v and run the
 // softmax attention, writing the same (max, sum, sum p*v) partials the stand-alone attention launch writes; the WO
 // GEMV's prologue consumes them unchanged.  This removes one of the five dependent launches per layer (~6.5 us of pure
 // latency at short contexts for the 7.9B tier) for the price of the exchange + attention inside the projection launch.
@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(GRP_THREADS) qkv_attn_kernel(GroupParams P) {
         acc = lv[f] ? a1 : acc;
         __builtin_amdgcn_wave_barrier();
     }
-    // The head's cache rows are requested only now, after the projection dots (round 4): a wavefront issues in order and a
+    // The head's cache rows are requested only now, after the projection dots: a wavefront issues in order and a
     // compute unit ingests ~11 B/clk, so requested at entry the 64 KB of rows delayed the attention blocks' projection tiles
     // -- and with them the exchange every block of the cluster waits for.  Rows beyond pos repeat row pos (the same cache
     // lines; they are masked below), the row AT pos comes from LDS.

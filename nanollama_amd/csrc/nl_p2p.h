@@ -10,7 +10,7 @@
 //
 // Transport: 8-byte granules {tag, float bits}, each written by ONE system-scope store and polled with
 // system-scope loads -- the data is its own flag, so no fence or separate flag orders anything
-// (cdna_hip_programming.md Guideline 16 form R2, here across devices).  The receive area is allocated
+// across the devices.  The receive area is allocated
 // uncached and mapped into the peers with hipIpc* (one process per GPU).  tag = (forward counter << 8) | seam,
 // the counter living on each device and advancing once per Forward, so a captured graph needs no per-launch
 // argument.  Slots are double-buffered by seam parity: a rank can only be one seam ahead of its slowest peer.

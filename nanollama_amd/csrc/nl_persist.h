@@ -1,4 +1,4 @@
-// nl_persist.h -- weight-stationary, XCD-pipelined persistent greedy decode for the smallest tier (round 5).
+// nl_persist.h -- weight-stationary, XCD-pipelined persistent greedy decode for the smallest tier.
 //
 // go/main.go:173-219 decodes token after token through go/model.go:490-620.  For nano (75 MB of Q8_0) the HBM time of a
 // token is 9 us, yet the launch plans of nl_block.h need 180: thirty dependent launches, each re-fetching its weights cold

@@ -9,7 +9,7 @@
 //   recent window append / drop-oldest                                                        :197-200
 // The uniform u comes from the host's generator (one float32 per step, uploaded up front): Go's math/rand
 // stream is not reproducible from another language anyway, the algorithm around it is what is mirrored.
-// No library sort is involved (round 5): top-k finds its k-th largest logit by a 2-bit-per-pass selection on the keys' bits,
+// No library sort is involved: top-k finds its k-th largest logit by a 2-bit-per-pass selection on the keys' bits,
 // collects the candidates above it (equal ones by ascending index, as the Go insertion list keeps them) and orders the <= 1024
 // of them with a bitonic network in LDS (samp_topk_kernel); its sums run sequentially over the <= top_k terms exactly as the Go
 // loop's.  top-p needs no order at all:

@@ -12,7 +12,7 @@
 //                    -> published as granules.  CONSUMER workgroups: request their rows of this rank's W_down column
 //                    slice at entry, gather h, multiply -> push all-reduce finished by the row's owner lane.
 //
-// Every in-launch hand-off is cdna_hip_programming.md Guideline 16 form R2 (8-byte {tag, value} granules, relaxed
+// Every in-launch hand-off is a polled 8-byte granule ({tag, value}, relaxed
 // agent-scope stores and polls, the value is its own flag); tag = (forward counter << 8) | layer, the counter advanced by
 // the embedding launch, so a replayed graph needs no per-launch argument.  Producers never wait, so the launches cannot
 // deadlock on their own; every poll is bounded and a give-up is reported like the other fused launches' (nl_block.h).
@@ -128,7 +128,7 @@ __device__ __forceinline__ void gran16_load4(const u32x4 *p0, const u32x4 *p1, c
                  : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d) : "v"(p0), "v"(p1), "v"(p2), "v"(p3) : "memory");
 }
 
-// ---- warming the NEXT launch's first weight bytes (round 5; tools/l2_prefetch_probe.hip, profiles/r05_l2_prefetch_probe.log) ----
+// ---- warming the NEXT launch's first weight bytes (tools/l2_prefetch_probe.hip, profiles/r05_l2_prefetch_probe.log) ----
 // A launch of the wide tier starts cold: its first weight round (18.9 MB of gate || up, 14.2 MB of Q | K | V) costs the 2 us of a
 // first fetch plus 3 us of transfer while nothing else can run -- and the launch before it leaves HBM idle for longer than that
 // (the attention chain; the h gather and the tail).  So wavefronts that are waiting anyway read ONE dword of every 128-byte
@@ -248,7 +248,7 @@ __device__ __forceinline__ void tp_gather16(const u32x4 *src, const u32x4 *src2,
     }
 }
 
-// ---- Q4_0 dot products on the matrix pipe (round 5; profiles/r05_fake_dot.log: with a quarter of the vector instructions of
+// ---- Q4_0 dot products on the matrix pipe (profiles/r05_fake_dot.log: with a quarter of the vector instructions of
 // the dot products the 7.9B step drops from 1.43 to 1.23 ms -- the decode GEMV of a wide layer is NOT purely memory-bound on
 // this chip: 2.1 vector operations and 4 bytes of LDS per weight leave 6.5 us of a 35 us layer exposed) ----------------------
 // The arithmetic is nl_persist.h's: a 32-element block of the input is scaled by a power of two so that its largest element
@@ -1135,8 +1135,8 @@ __global__ void __launch_bounds__(TP_THREADS) wide_ffn_kernel(WideFfnParams P) {
     const bool o_act = tid < TR && b < P.dn_ntiles && o_row < D;
     const float e_resid = P.x[min(o_row, D - 1)];
     // (One weight buffer.  A second one -- a round's dot products running while the next round's weights are in flight -- was
-    //  measured twice and lost both times: 20.9 against 19.7 us on the vector pipe (round 4), 19.1 against 17.8 us with the
-    //  matrix-pipe dot products and 98 registers (round 5): two rounds in flight are 38 MB against 32 MB of L2.)
+    //  measured twice and lost both times: 20.9 against 19.7 us on the vector pipe, 19.1 against 17.8 us with the
+    //  matrix-pipe dot products and 98 registers: two rounds in flight are 38 MB against 32 MB of L2.)
     auto load_round = [&](int rnd) {
         const int t = min(b + rnd * nb, P.gu_tiles - 1);                       // (a block without a tile in the last round repeats a request)
 #pragma unroll

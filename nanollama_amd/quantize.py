@@ -1,5 +1,5 @@
 """GGUF re-quantiser -- the job of scripts/quantize_gguf.py (F16/F32 GGUF -> Q8_0 GGUF, 1-D tensors to F32),
-vectorised, plus Q4_0 which the reference CLI cannot produce (SURVEY.md section 8f-4).
+vectorised, plus Q4_0 which the reference CLI cannot produce.
 
     python -m nanollama_amd.quantize in-f16.gguf out-q8_0.gguf [--type q8_0|q4_0]
 

@@ -1,4 +1,4 @@
-"""Deterministic random-weight GGUF generator (SURVEY.md section 8d).
+"""Deterministic random-weight GGUF generator.
 
 There is no network for checkpoints, so every parity and bench input is a
 random-weight GGUF written here in the reference exporter's exact layout
@@ -69,7 +69,7 @@ class ModelShape:
         return self.n_layer * per_layer + self.vocab * d
 
 
-# NAMED_CONFIGS nanollama/llama.py:40-51; vocab tiers README.md:49-54 (SURVEY 8).
+# NAMED_CONFIGS nanollama/llama.py:40-51; vocab tiers README.md:49-54.
 TIERS: Dict[str, ModelShape] = {
     "nano": ModelShape("nano", 13, 576, 9, 9, 32000),
     "mini": ModelShape("mini", 20, 768, 12, 3, 32000),
@@ -91,7 +91,7 @@ QRAND_ONLY = (GGML_Q5_0, GGML_Q4_K, GGML_Q6_K)
 
 
 def token_list(vocab: int) -> List[str]:
-    """V single-code-point pieces so prompts map 1:1 to ids (SURVEY 8a quirk 5)."""
+    """V single-code-point pieces so prompts map 1:1 to ids."""
     toks = ["<unk>", "<s>", "</s>"]
     for i in range(3, vocab):
         cp = 0x100 + i
@@ -215,7 +215,7 @@ def generate_gguf(path: str, shape: ModelShape, wtype: str = "q8_0", seed: Optio
     w.add_float32_array("tokenizer.ggml.scores", [0.0] * shape.vocab)
     w.add_int32_array("tokenizer.ggml.token_type", [2, 3, 3] + [1] * (shape.vocab - 3))
     w.add_uint32("tokenizer.ggml.bos_token_id", 1)
-    w.add_int32("tokenizer.ggml.eos_token_id", -1)  # random models must not stop early (SURVEY 8a quirk 6)
+    w.add_int32("tokenizer.ggml.eos_token_id", -1)  # random models must not stop early
     w.add_bool("tokenizer.ggml.add_space_prefix", False)
 
     floats: Dict[str, np.ndarray] = {}
@@ -241,14 +241,14 @@ def generate_gguf(path: str, shape: ModelShape, wtype: str = "q8_0", seed: Optio
 
 
 def prompt_ids(n: int, vocab: int, seed: int = 7) -> List[int]:
-    """Fixed prompt ids from PCG64(seed) (SURVEY 8d); BOS=1 first, as Encode(addBos) does."""
+    """Fixed prompt ids from PCG64(seed); BOS=1 first, as Encode(addBos) does."""
     rng = np.random.Generator(np.random.PCG64(seed))
     ids = rng.integers(3, vocab, size=max(n - 1, 0))
     return [1] + [int(x) for x in ids]
 
 
 def weight_bytes_per_token(shape: ModelShape, wtype: str) -> float:
-    """Algorithmic weight bytes per decoded token (SURVEY 8d): every 2-D tensor
+    """Algorithmic weight bytes per decoded token: every 2-D tensor
     in the layers + LM head once, norms, one embedding row."""
     t = WTYPES[wtype]
     bpe = ggml_block_size(t) / ggml_block_elements(t)

@@ -63,7 +63,7 @@ def test_create_group_without_gpu_fails_loudly():
 
 
 # What "using the oracle" looks like in source: an import, an include, a dlopen / CDLL of the checker's library, or a path
-# into oracle/.  (A comment that merely names the oracle as the thing a kernel is held to is not a use; the round-4 tree
+# into oracle/.  (A comment that merely names the oracle as the thing a kernel is held to is not a use; an earlier tree
 # went red on exactly such a comment.)
 _ORACLE_USE = [
     re.compile(r"^\s*(from|import)\s+oracle\b", re.M),                 # import oracle / from oracle import ...

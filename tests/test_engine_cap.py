@@ -89,7 +89,7 @@ def test_without_a_cap_all_tokens_are_emitted():
 
 
 def test_greedy_path_stops_the_device_within_a_chunk_of_the_cap():
-    # (advisor, round 3) the greedy fast path used to run all max_tokens steps and truncate afterwards: the rate was
+    # the greedy fast path used to run all max_tokens steps and truncate afterwards: the rate was
     # understated and the device state ran past where the Go loop stops
     m = FakeModel()
     eng = Engine(m, rep_penalty=1.0, eos_id=-1, rep_window=6, seed=11)

@@ -19,7 +19,7 @@ def test_quantisers_match_reference_bytes():
         assert quant.quantize_q8_0(x).tobytes() == k[f"{name}_q8"].tobytes(), name
         assert quant.quantize_q4_0(x).tobytes() == k[f"{name}_q4"].tobytes(), name
         assert quant.to_f16_bytes(x).tobytes() == k[f"{name}_f16"].tobytes(), name
-    assert bytes(k["randn_q8"][:6]).hex() == "4424bcbbf1e6"  # SURVEY 8c captured prefixes
+    assert bytes(k["randn_q8"][:6]).hex() == "4424bcbbf1e6"  # captured prefixes
     assert bytes(k["randn_q4"][:6]).hex() == "3b343424a7b6"
 
 
@@ -98,7 +98,7 @@ def test_tier_shapes_match_survey_table():
     t = synth.TIERS
     assert (t["nano"].ffn, t["mini"].ffn, t["goldie"].ffn, t["big"].ffn) == (1536, 2048, 4096, 11008)
     assert [round(t[k].matrix_params() / 1e6, 1) for k in ("nano", "mini", "goldie", "big")] == [70.2, 148.4, 767.4, 7481.6]
-    # SURVEY 8 table quotes the matrices term alone; weight_bytes_per_token adds norms + one embedding row (8d formula)
+    # the matrices term alone; weight_bytes_per_token adds norms + one embedding row
     assert round(t["nano"].matrix_params() * 34 / 32 / 1e6, 2) == 74.58
     assert round(t["big"].matrix_params() * 18 / 32 / 1e6, 2) == 4208.39
     assert 74.58e6 < synth.weight_bytes_per_token(t["nano"], "q8_0") < 74.70e6

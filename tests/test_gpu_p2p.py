@@ -139,7 +139,7 @@ def test_two_launch_layer_ranks_match_the_in_process_group(tmp_path, monkeypatch
 
 
 def test_a_fused_exchange_timeout_on_one_rank_retires_the_plan_on_every_rank(tmp_path):
-    # ADVICE r3: a cluster exchange of a fused launch gives up on ONE rank only (NL_FUSED_SPIN_LIMIT=0 there).  The give-up
+    # a cluster exchange of a fused launch gives up on ONE rank only (NL_FUSED_SPIN_LIMIT=0 there).  The give-up
     # travels with the argmax exchange of the same step, so BOTH ranks retire their fused plans and redo the call from a
     # common forward counter: the logits are the five-launch plan's, bit for bit, and nothing hangs or desynchronises.
     from nanollama_amd import model
@@ -162,7 +162,7 @@ def test_a_fused_exchange_timeout_on_one_rank_retires_the_plan_on_every_rank(tmp
 def test_push_allreduce_across_devices(tmp_path, n):
     # One rank per GPU: the only test in which a granule crosses xGMI.  Skipped on boxes with fewer devices (the
     # 1-GPU test pool) -- until it has run green on a multi-GPU node the cross-device wire counts as UNVERIFIED
-    #  and bench.py keeps its 1-GPU logit / greedy-id self-check and the RCCL fallback.
+    # and bench.py keeps its 1-GPU logit / greedy-id self-check and the RCCL fallback.
     from nanollama_amd import _lib, model
     if _lib.lib().nl_device_count() < n:
         pytest.skip(f"needs {n} devices")

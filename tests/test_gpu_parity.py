@@ -866,7 +866,7 @@ def test_prompt_with_rmsnorm_folded_into_the_gemms_matches_oracle(hip, orc, tmp_
 
 @pytest.mark.parametrize("stream_scale", [2.0 ** -6, 2.0 ** 15])
 def test_folded_rmsnorm_at_small_and_large_residual_magnitudes(hip, orc, tmp_path, monkeypatch, stream_scale):
-    # (advisor, round 3) the folded norm hands x * g to the consumer as fp16 hi / lo fragments BEFORE 1 / rms is known.  A
+    # the folded norm hands x * g to the consumer as fp16 hi / lo fragments BEFORE 1 / rms is known.  A
     # residual stream of rms ~1e-2 puts every lo half into the fp16 denormals (absolute instead of relative precision; smaller
     # still and RMSNorm's eps takes the model over), one of rms ~3e4
     # has elements beyond 65504 (inf - inf = NaN).  The producer therefore pre-scales by an exact power of two near the
@@ -901,7 +901,7 @@ def test_folded_rmsnorm_at_small_and_large_residual_magnitudes(hip, orc, tmp_pat
 
 def test_mini_full_size_long_prefill_matches_oracle(hip, orc, tmp_path, monkeypatch):
     # BASELINE.json configs[2] at its own shape (mini, 173M, Q4_0): a 1920-token prompt through the matrix-core
-    # path in ONE step vs the CPU oracle fed token by token (SURVEY 8d: 1920 prompt positions for parity), then a
+    # path in ONE step vs the CPU oracle fed token by token (1920 prompt positions for parity), then a
     # greedy continuation on the decode path from the cache the prefill wrote.
     shape = synth.TIERS["mini"]
     p = tmp_path / "mini.gguf"

@@ -1,4 +1,4 @@
-"""TEST INFRASTRUCTURE: the tensor-parallel shard plan (SURVEY.md section 8e) restated on the host, so the CPU tests can
+"""TEST INFRASTRUCTURE: the tensor-parallel shard plan restated on the host, so the CPU tests can
 check with the oracle's GEMVs that such slices reproduce the full products.  The product slices on the device
 (nl_upload_tensor -> matrix_upload call sites in nanollama_amd/csrc/nl_engine.hip); its results are checked on the GPU
 against the single-GPU engine and the oracle (tests/test_gpu_parity.py, tests/test_gpu_p2p.py).
