@@ -193,7 +193,7 @@ __global__ void bembed_kernel(BEmbedParams P) {
         }
         if (threadIdx.x == 0) P.tkv[blockIdx.x] = (long long)strm * P.kv_stream_stride + (long long)pos * P.hd;
     }
-    embed_row(P.table, P.wtype, P.dim, token, P.gamma_row, P.gamma_val, x);
+    embed_row<4>(P.table, P.wtype, P.dim, token, P.gamma_row, P.gamma_val, x);
 }
 
 // Which of the launch's blocks this one stands for: blocks b, b + 8, ... run on one XCD, which gets a run of them.  The sixteen tokens of a fragment

@@ -1085,7 +1085,7 @@ void build_plan(nl_engine *e, std::vector<Op> &plan, bool fused, bool help = fal
         P.epoch = e->p2p.epoch; P.status = e->p2p.status; P.timeout_ticks = e->p2p.timeout_ticks;
         e->plan_p2p_argmax = P;
         plan.push_back({K_ARGMAX, 0, nullptr, 0, [P](hipStream_t st) {
-                               hipLaunchKernelGGL(p2p_argmax_kernel, dim3(1), dim3(1024), 0, st, P);
+                               hipLaunchKernelGGL(p2p_argmax_kernel<1>, dim3(1), dim3(1024), 0, st, P);
                                return hipGetLastError();
                            }});
     } else {
@@ -1172,10 +1172,13 @@ int capture_graph(nl_engine *e, nl_engine::PlanSet &S) {
                 if (fuse_embed && op.kind == K_ARGMAX && e->p2p.on) {
                     P2PArgmaxParams PA = e->plan_p2p_argmax;
                     PA.E = e->plan_embed;     // the winner's embedding row opens the next step (and advances the counter)
-                    hipLaunchKernelGGL(p2p_argmax_kernel, dim3(1), dim3(1024), 0, e->stream, PA);
+                    const int each = embed_each(PA.E.dim, 1024);
+                    hipLaunchKernelGGL(each == 1 ? p2p_argmax_kernel<1> : each == 2 ? p2p_argmax_kernel<2> : p2p_argmax_kernel<4>, dim3(1), dim3(1024), 0, e->stream, PA);
                     ls = hipGetLastError();
                 } else if (fuse_embed && op.kind == K_ARGMAX) {
-                    hipLaunchKernelGGL(argmax_embed_kernel, dim3(1), dim3(1024), 0, e->stream, e->plan_argmax, e->plan_embed);
+                    const int each = embed_each(e->plan_embed.dim, 1024);
+                    hipLaunchKernelGGL(each == 1 ? argmax_embed_kernel<1> : each == 2 ? argmax_embed_kernel<2> : argmax_embed_kernel<4>, dim3(1), dim3(1024), 0, e->stream,
+                                       e->plan_argmax, e->plan_embed);
                     ls = hipGetLastError();
                 } else ls = op.fn(e->stream);
                 if (ls != hipSuccess) { rc2 = e->fail(NL_ERR_HIP, "multi-step capture: %s", hipGetErrorString(ls)); break; }

@@ -1040,33 +1040,29 @@ __device__ __forceinline__ float embed_value(const uint8_t *table, int wtype, in
 }
 
 // row `token`, plus its gamma row, to x, by a whole workgroup.  A lone workgroup's lookup is memory round trips and nothing else, so a thread asks
-// for four elements at once (clamped index, masked store): that takes a choice of the format around the loads, not between them.
+// for N elements at once (clamped index, masked store): that takes a choice of the format around the loads, not between them.
 // (4096 columns of Q4_0: 12.3 us by 256 threads with a choice per element, 5.3 by 1024 so; past 1024 columns 1024 threads have the row in a round.)
-// Where a row has fewer elements than that, one or two: asked for four times, a short row behind the argmax of a greedy chain cost it 0.1 to 0.6 us a token
-// (two layers, us a token with four always, so, and with a choice per element: Q4_0 512 columns 35.0, 34.5, 34.6, 1024 43.4, 42.7, 42.9, 2048 52.2, 51.8, 52.1; Q4_K 512
-// 44.9, 44.4, 44.9; Q6_K 1536 49.5, 48.9, 49.5).
+// N is four, and behind the argmax of a chain, whose 1024 threads have most rows in fewer, what the row has (embed_each; two layers, us a token with four always,
+// so, and with a choice per element: Q4_0 512 columns 35.0, 34.5, 34.6, 1024 43.4, 42.7, 42.9, 2048 52.2, 51.8, 52.1; Q4_K 512 44.9, 44.4, 44.9; Q6_K 1536 49.5, 48.9,
+// 49.5).  It is chosen by the host: all three in a kernel are instructions that a launch fetches, 0.5 to 1.7 us of a prompt's lookup.
+inline int embed_each(int dim, int threads) { return dim <= threads ? 1 : dim <= 2 * threads ? 2 : 4; }
+template <int N>
 __device__ __forceinline__ void embed_row(const uint8_t *table, int wtype, int dim, int token, const int *gamma_row, const float *gamma_val, float *x) {
     const int gr = gamma_row ? gamma_row[token] : -1, nthr = blockDim.x;
     auto rows = [&](auto type) {
         constexpr int WT = decltype(type)::value;
-        auto each = [&](auto per) {
-            constexpr int N = decltype(per)::value;
-            for (int i0 = threadIdx.x; i0 < dim; i0 += N * nthr) {
-                float v[N];
+        for (int i0 = threadIdx.x; i0 < dim; i0 += N * nthr) {
+            float v[N];
 #pragma unroll
-                for (int k = 0; k < N; k++) v[k] = embed_value(table, WT, dim, token, min(i0 + k * nthr, dim - 1));
-                if (gr >= 0) {
+            for (int k = 0; k < N; k++) v[k] = embed_value(table, WT, dim, token, min(i0 + k * nthr, dim - 1));
+            if (gr >= 0) {
 #pragma unroll
-                    for (int k = 0; k < N; k++) v[k] += gamma_val[(long long)gr * dim + min(i0 + k * nthr, dim - 1)];
-                }
-#pragma unroll
-                for (int k = 0; k < N; k++)
-                    if (i0 + k * nthr < dim) x[i0 + k * nthr] = v[k];
+                for (int k = 0; k < N; k++) v[k] += gamma_val[(long long)gr * dim + min(i0 + k * nthr, dim - 1)];
             }
-        };
-        if (dim <= nthr) each(std::integral_constant<int, 1>{});
-        else if (dim <= 2 * nthr) each(std::integral_constant<int, 2>{});
-        else each(std::integral_constant<int, 4>{});
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                if (i0 + k * nthr < dim) x[i0 + k * nthr] = v[k];
+        }
     };
     using std::integral_constant;
     switch (wtype) {
@@ -1082,7 +1078,7 @@ __device__ __forceinline__ void embed_row(const uint8_t *table, int wtype, int d
 
 __global__ void embed_kernel(EmbedParams P) {
     if (P.epoch && threadIdx.x == 0) *P.epoch = *P.epoch + 1;
-    embed_row(P.table, P.wtype, P.dim, sload_i32(P.ctl + CTL_TOKEN), P.gamma_row, P.gamma_val, P.x);
+    embed_row<4>(P.table, P.wtype, P.dim, sload_i32(P.ctl + CTL_TOKEN), P.gamma_row, P.gamma_val, P.x);
 }
 
 // ------------------------------------------------------------- attention ---
@@ -1517,6 +1513,7 @@ __global__ void __launch_bounds__(1024) bargmax_kernel(const float *logits, int 
 
 // argmax of step k + embedding lookup of step k+1 in one launch (chained greedy decode inside the multi-step
 // graph): the token goes from the reduction to the row fetch through LDS instead of through ctl and a kernel boundary
+template <int N>   // embed_each
 __global__ void __launch_bounds__(1024) argmax_embed_kernel(ArgmaxParams P, EmbedParams E) {
     __shared__ float bv[16];
     __shared__ int bi[16];
@@ -1563,7 +1560,7 @@ __global__ void __launch_bounds__(1024) argmax_embed_kernel(ArgmaxParams P, Embe
         if (E.epoch) *E.epoch = (unsigned)c_epoch + 1u;   // this embedding opens the next Forward
     }
     __syncthreads();
-    embed_row(E.table, E.wtype, E.dim, tok, E.gamma_row, E.gamma_val, E.x);
+    embed_row<N>(E.table, E.wtype, E.dim, tok, E.gamma_row, E.gamma_val, E.x);
 }
 
 

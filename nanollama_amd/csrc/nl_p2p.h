@@ -48,6 +48,7 @@ struct P2PArgmaxParams {
 // argmax of this rank's slice, one {value, index} pair pushed to every rank, every rank picks the same winner.
 // The sender's LM-head kernel has completed before this kernel starts and a system-scope fence precedes the
 // push, so a rank that sees the pair also sees that sender's logits slice in its gathered logits buffer.
+template <int N>   // embed_each
 __global__ void __launch_bounds__(1024) p2p_argmax_kernel(P2PArgmaxParams P) {
     __shared__ float bv[16];
     __shared__ int bi[16];
@@ -128,7 +129,7 @@ __global__ void __launch_bounds__(1024) p2p_argmax_kernel(P2PArgmaxParams P) {
     }
     if (!P.E.x) return;
     __syncthreads();
-    embed_row(P.E.table, P.E.wtype, P.E.dim, tok, P.E.gamma_row, P.E.gamma_val, P.E.x);
+    embed_row<N>(P.E.table, P.E.wtype, P.E.dim, tok, P.E.gamma_row, P.E.gamma_val, P.E.x);
 }
 
 }  // namespace nl
