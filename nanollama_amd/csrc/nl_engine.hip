@@ -11,6 +11,7 @@
 #include <mutex>
 #include "nl_kernels.h"
 #include "nl_qgemm.h"
+#include "nl_layers.h"
 #include "nl_pgemm.h"
 #include "nl_dgemm.h"
 #include "nl_sgemm.h"
@@ -256,7 +257,8 @@ struct nl_engine {
         hipGraphExec_t multi_exec = nullptr;  // (one inter-graph gap per graph_steps tokens instead of per token)
         hipGraph_t call = nullptr;           // the plan between a fetch of the step's control words from the pinned call box and a
         hipGraphExec_t call_exec = nullptr;   // store of {sequence, argmax} into its done word: one nl_forward, no copy, no synchronise
-    } ps[3];                                 // (ps[2]: ps[1] with the attention launch whose passes are shared by helper blocks: wide tier, one GPU, from the second pass on)
+    } ps[4];                                 // (ps[2]: ps[1] with the attention launch whose passes are shared by helper blocks: wide tier, one GPU, from the second pass on;
+                                             //  ps[3]: all layers in one launch, nl_layers.h)
     bool fused = false;           // ps[1] exists
     int fused_mode = 0;           // 1: whole attention half per layer (nl_block.h); 2: projection + attention (nl_group.h);
                                   // 3: a tensor-parallel rank's layer as two launches (nl_tp.h); 4: one GPU, wide tier: mode 3's
@@ -285,6 +287,12 @@ struct nl_engine {
     float *parts_ffn = nullptr;   // [I / 256][D] per-slice W_down partials
     unsigned long long *xchg_ffn = nullptr;   // [I] granules
     int fused_max_pos = 0;        // ps[1] serves steps whose position is below this
+    struct Layers {               // nl_layers.h: steps below max_pos and from min_pos on run all layers in one launch (ps[3])
+        bool on = false;
+        int min_pos = 0, max_pos = 0;
+        LayersEntry *tab = nullptr;
+        u32x4 *gran = nullptr;    // gq | gr | go | gp | gh | gx | the XCDs' copies | tickets
+    } ly;
     float *parts = nullptr;       // [Hs][D] per-head WO partials of the fused block
     unsigned long long *xchg = nullptr;   // [Hs][192] granules exchanged inside a head's cluster
     unsigned *tick = nullptr;     // {forward counter, status} device words of the fused block
@@ -298,9 +306,9 @@ struct nl_engine {
     ArgmaxParams plan_argmax{};
     P2PArgmaxParams plan_p2p_argmax{};
     // sampled chained decode: {sampler, plan} x graph_steps, captured per sampling-parameter set
-    hipGraph_t samp_graph[3] = {nullptr, nullptr, nullptr};          // per launch plan (ps[0] / ps[1] / ps[2])
-    hipGraphExec_t samp_graph_exec[3] = {nullptr, nullptr, nullptr};
-    nl_sample_params samp_graph_params[3]{};
+    hipGraph_t samp_graph[4] = {};          // per launch plan (ps[0 .. 3])
+    hipGraphExec_t samp_graph_exec[4] = {};
+    nl_sample_params samp_graph_params[4]{};
     bool samp_graph_failed = false;
     bool use_graph = true;
     void *comm = nullptr;
@@ -658,6 +666,29 @@ BlockParams attn_block_params(nl_engine *e, int l, const float *x_in) {
     return B;
 }
 
+// final RMSNorm, LM head and argmax of a plan that leaves the finished residual stream in x
+void push_head(nl_engine *e, std::vector<Op> &plan, const float *x) {
+    const nl_config &c = e->cfg;
+    int lm_blocks, lm_spb;
+    {   // final RMSNorm + LM head (go/model.go:616-619)
+        GemvParams P = base_params(e, e->lm_head);
+        P.x = x; P.normw = e->output_norm;
+        P.out = e->logits; P.amax_val = e->amax_val; P.amax_idx = e->amax_idx;
+        P.host_out = e->d_h_logits;
+        lm_blocks = (P.ntiles + P.tw - 1) / P.tw;
+        lm_spb = (P.tw * TR + 63) / 64;
+        push_gemv(plan, K_LMHEAD, 0, e->logits, (size_t)e->Vs, e->lm_head.wtype, PRO_NORM, EPI_STORE, P);
+    }
+    {
+        ArgmaxParams P{e->logits, c.vocab, e->amax_val, e->amax_idx, lm_blocks * lm_spb, e->ctl, e->ids, e->result};
+        e->plan_argmax = P;
+        plan.push_back({K_ARGMAX, 0, nullptr, 0, [P](hipStream_t st) {
+                               hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, P);
+                               return hipGetLastError();
+                           }});
+    }
+}
+
 // Small models at short contexts, both halves of a layer fused (nl_block.h): embed -> { attn_block -> ffn_block } x L ->
 // lm_head -> argmax, 2 launches per layer.  Each block adds its predecessor's partial vectors to the residual stream in
 // its prologue (one designated workgroup stores the sum): the feed-forward block reads x[0] and writes x[1], the
@@ -714,24 +745,48 @@ void build_plan_blocks(nl_engine *e, std::vector<Op> &plan) {
                                }});
         }
     }
-    int lm_blocks, lm_spb;
-    {   // final RMSNorm + LM head (go/model.go:616-619)
-        GemvParams P = base_params(e, e->lm_head);
-        P.x = e->x[1]; P.normw = e->output_norm;
-        P.out = e->logits; P.amax_val = e->amax_val; P.amax_idx = e->amax_idx;
-        P.host_out = e->d_h_logits;
-        lm_blocks = (P.ntiles + P.tw - 1) / P.tw;
-        lm_spb = (P.tw * TR + 63) / 64;
-        push_gemv(plan, K_LMHEAD, 0, e->logits, (size_t)e->Vs, e->lm_head.wtype, PRO_NORM, EPI_STORE, P);
-    }
+    push_head(e, plan, e->x[1]);
+    link_prefetch(plan);
+}
+
+// Models and positions whose steps gain by nl_layers.h.  Its start (pointers into LDS, the first weights cold) costs as much as two layers gain: 2 layers of
+// 1024 columns 56.5 -> 54.5 us a token in Q8_0 and 49.0 -> 51.8 in Q4_0, four 97.2 -> 86.4 and 87.7 -> 83.7, sixteen 338 -> 284 and 307 -> 273,
+// 28 of 1536 747 -> 576 and 633 -> 546 (position 130; 400: 775 -> 590 and 696 -> 559).  Against two launches a layer (mode 1) it loses while their
+// attention is at its first or second pass: 20 layers of 768 columns 313 -> 328 us at position 140, 323 -> 331 at 230, 349 -> 334 at 256, 384 -> 334 at 400.
+bool layers_pay(const nl_engine *e) { return e->cfg.n_layers >= 4; }
+int layers_min_pos(const nl_engine *e) { return e->fused_mode == 1 ? 2 * LY_PASS : 0; }
+
+// nl_layers.h: embed -> all layers -> lm_head -> argmax
+void build_plan_layers(nl_engine *e, std::vector<Op> &plan) {
+    plan.clear();
+    const nl_config &c = e->cfg;
     {
-        ArgmaxParams P{e->logits, c.vocab, e->amax_val, e->amax_idx, lm_blocks * lm_spb, e->ctl, e->ids, e->result};
-        e->plan_argmax = P;
-        plan.push_back({K_ARGMAX, 0, nullptr, 0, [P](hipStream_t st) {
-                               hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, P);
+        EmbedParams P{e->embd_raw, e->embd_type, c.dim, e->ctl, e->x[0], e->gamma_row, e->gamma_val, e->tick};
+        e->plan_embed = P;
+        plan.push_back({K_EMBED, 0, nullptr, 0, [P](hipStream_t st) {
+                               hipLaunchKernelGGL(embed_kernel, dim3(1), dim3(P.dim <= 1024 ? 256 : 1024), 0, st, P);
                                return hipGetLastError();
                            }});
     }
+    const nl_engine::Layer &L0 = e->layers[0];
+    LayersParams P{};
+    P.layers = e->ly.tab; P.L = c.n_layers; P.D = c.dim; P.H = e->Hs; P.KV = e->KVs; P.gqa = e->gqa; P.seq_len = c.seq_len;
+    P.rope_conj = c.rope_conjugate; P.single_stream = c.max_streams == 1 ? 1 : 0;
+    P.np_d = L0.qkv.npairs; P.np_o = L0.wo.npairs; P.np_i = L0.down.npairs; P.t_qkv = L0.qkv.ntiles; P.t_d = L0.wo.ntiles; P.t_i = L0.gate.ntiles;
+    P.eps = c.rms_eps; P.scale = (float)(1.0 / std::sqrt((double)e->hd));
+    P.x = e->x[0]; P.rope_cos = e->rope_cos; P.rope_sin = e->rope_sin;
+    P.kcache = e->kcache; P.vcache = e->vcache; P.kv_layer_stride = e->kv_layer_stride; P.kv_stream_stride = e->kv_stream_stride;
+    P.ctl = e->ctl; P.tick = e->tick; P.status = e->tick + 1; P.host_status = e->h_status; P.spin_limit = e->spin_limit;
+    P.rec_max = layers_records(c.seq_len);
+    P.loc_n = layers_loc(P.t_d, P.t_i);
+    u32x4 *g = e->ly.gran;
+    auto take = [&](int n) { u32x4 *at = g; g += n; return at; };
+    P.gq = take(P.t_qkv * GPT); P.gr = take(P.H * P.rec_max * LY_REC); P.go = take(P.H * LY_REC);
+    P.gp = take(P.t_d * 2 * LY_HG); P.gh = take(P.t_i * GPT); P.gx = take(P.t_d * 2 * LY_HG); P.loc = take(LY_XCDS * P.loc_n);
+    P.tickets = reinterpret_cast<unsigned *>(g);                         // (LY_XCDS * 4 granules)
+    const int wt = L0.qkv.wtype, grid = e->num_cus;
+    plan.push_back({K_FFNBLOCK, 0, nullptr, 0, [P, wt, grid](hipStream_t st) { return launch_layers(wt, P, grid, st); }});
+    push_head(e, plan, e->x[0]);
     link_prefetch(plan);
 }
 
@@ -1194,7 +1249,7 @@ int capture_graph(nl_engine *e, nl_engine::PlanSet &S) {
 }
 
 void destroy_samp_graphs(nl_engine *e) {
-    for (int k = 0; k < 3; k++) {
+    for (int k = 0; k < 4; k++) {
         if (e->samp_graph_exec[k]) { (void)hipGraphExecDestroy(e->samp_graph_exec[k]); e->samp_graph_exec[k] = nullptr; }
         if (e->samp_graph[k]) { (void)hipGraphDestroy(e->samp_graph[k]); e->samp_graph[k] = nullptr; }
     }
@@ -1204,6 +1259,7 @@ void destroy_samp_graphs(nl_engine *e) {
 // (ps[2]: the fused plan of the wide tier on one GPU from the second attention pass on -- its attention launch is the variant
 //  whose passes are shared by helper blocks, nl_tp.h; the first pass keeps the launch compiled without them: 0.7 us per layer)
 int plan_index(const nl_engine *e, int pos_last) {
+    if (e->ly.on && pos_last >= e->ly.min_pos && pos_last < e->ly.max_pos) return 3;
     if (!(e->fused && pos_last < e->fused_max_pos)) return 0;
     return (e->attn_helpers && pos_last >= TP_PASS) ? 2 : 1;
 }
@@ -1253,9 +1309,11 @@ int build_all(nl_engine *e) {
     build_plan(e, e->ps[0].ops, false);
     if (e->fused) build_plan(e, e->ps[1].ops, true);
     if (e->fused && e->attn_helpers) build_plan(e, e->ps[2].ops, true, true);
+    if (e->ly.on) build_plan_layers(e, e->ps[3].ops);
     const bool has_coll = (e->G > 1 || e->force_tp_plan) && !e->p2p.on;
     if (e->use_graph && !(e->cfg.flags & NL_FLAG_LOCAL_GROUP)) {
-        for (int k = 0; k < (e->fused ? (e->attn_helpers ? 3 : 2) : 1); k++) {
+        for (int k = 0; k < 4; k++) {
+            if (k == 3 ? !e->ly.on : k && !(e->fused && (k == 1 || e->attn_helpers))) continue;
             int rc = capture_graph(e, e->ps[k]);
             if (rc && has_coll) {
                 // RCCL inside a captured graph is not guaranteed on every RCCL build: fall back to eager launches
@@ -1323,7 +1381,7 @@ bool take_fused_timeout(nl_engine *e) {
     *e->h_status = 0;
     (void)hipMemsetAsync(e->tick + 1, 0, sizeof(unsigned), e->stream);
     (void)hipStreamSynchronize(e->stream);
-    e->fused = false;
+    e->fused = e->ly.on = false;
     e->fused_retired = true;
     destroy_samp_graphs(e);
     e->fail(NL_OK, "warning: a fused-launch cluster exchange timed out (status %u); the step was redone on the general plan, "
@@ -3083,6 +3141,20 @@ int nl_finalize(nl_handle e) {
                 okf = okf && L.dn_slice.ready && L.dn_slice.wtype == L.qkv.wtype && L.gate.wtype == L.qkv.wtype && L.up.wtype == L.qkv.wtype;
             e->ffn_fused = okf;
         }
+        {
+            const nl_engine::Layer &L0 = e->layers[0];
+            const char *lk = getenv("NL_LAYERS");              // knob (tests, tools): 0 never, 2 wherever the launch can run
+            const int lv = lk ? atoi(lk) : 1;
+            bool ok = lv != 0 && (lv == 2 || !fa) && e->G == 1 && !e->force_tp_plan && !e->p2p.on && !(c.flags & NL_FLAG_LOCAL_GROUP) && e->hd == 64 && !c.qk_norm &&
+                      c.n_layers <= LY_MAX_LAYERS && e->num_cus == LY_XCDS * LY_PER_XCD && e->gqa <= LY_MAX_HPU && c.dim % PAIR == 0 && e->Is % PAIR == 0 && c.dim <= LY_MAX_COLS && e->Hs * e->hd <= LY_MAX_COLS &&
+                      e->Is <= LY_MAX_FF && L0.qkv.ntiles <= e->num_cus && L0.gate.ntiles <= e->num_cus && 2 * L0.wo.ntiles <= e->num_cus && e->KVs <= e->num_cus;
+            for (const auto &L : e->layers)
+                for (const PackedMat *m : {&L.qkv, &L.wo, &L.gate, &L.up, &L.down})
+                    ok = ok && (m->wtype == WT_Q8_0 || m->wtype == WT_Q4_0) && m->wtype == L0.qkv.wtype && m->ntiles * TR == m->rows && m->npairs * PAIR == m->cols;
+            e->ly.on = ok && (lv == 2 || layers_pay(e));
+            e->ly.max_pos = std::min({c.seq_len, e->num_cus / e->KVs * LY_PASS, LY_MAX_REC * LY_PASS});
+            e->ly.min_pos = lv == 2 ? 0 : layers_min_pos(e);
+        }
         if (e->ffn_fused) {
             HIPCK(e, dalloc(&e->parts_ffn, (size_t)(e->Is / FFN_SLICE) * c.dim, &e->bytes_state));
             HIPCK(e, dalloc(&e->xchg_ffn, (size_t)e->Is, &e->bytes_state));
@@ -3093,10 +3165,24 @@ int nl_finalize(nl_handle e) {
             const size_t nx = e->fused_mode == 1 ? (size_t)e->Hs * 192 : (size_t)e->KVs * (e->gqa + 2) * 64;
             HIPCK(e, dalloc(&e->xchg, nx, &e->bytes_state));
             HIPCK(e, hipMemset(e->xchg, 0, nx * 8));
+        }
+        if (e->fused || e->ly.on) {
             HIPCK(e, dalloc(&e->tick, (size_t)2, &e->bytes_state));
             HIPCK(e, hipMemset(e->tick, 0, 8));
             HIPCK(e, hipHostMalloc((void **)&e->h_status, sizeof(unsigned), hipHostMallocMapped | hipHostMallocCoherent));
             *e->h_status = 0;
+        }
+        if (e->ly.on) {
+            const nl_engine::Layer &L0 = e->layers[0];
+            std::vector<LayersEntry> tab;
+            for (const auto &L : e->layers)
+                tab.push_back(LayersEntry{{L.qkv.q, L.wo.q, L.gate.q, L.up.q, L.down.q}, {L.qkv.s, L.wo.s, L.gate.s, L.up.s, L.down.s}, L.attn_norm, L.ffn_norm, L.bq, L.bk, L.bv, L.bo});
+            HIPCK(e, dalloc(&e->ly.tab, tab.size(), &e->bytes_state));
+            HIPCK(e, hipMemcpy(e->ly.tab, tab.data(), tab.size() * sizeof(LayersEntry), hipMemcpyHostToDevice));
+            const size_t n = (size_t)L0.qkv.ntiles * GPT + (size_t)e->Hs * (layers_records(c.seq_len) + 1) * LY_REC +
+                             (size_t)(LY_XCDS + 1) * layers_loc(L0.wo.ntiles, L0.gate.ntiles) + LY_XCDS * 4;
+            HIPCK(e, dalloc(&e->ly.gran, n, &e->bytes_state));
+            HIPCK(e, hipMemset(e->ly.gran, 0, n * sizeof(u32x4)));
         }
         if (e->fused_mode == 3 || e->fused_mode == 4) {
             const size_t nq = (size_t)e->KVs * (e->gqa + 2) * 4 * GPT, no = (size_t)e->Hs * 4 * GPT, nh = (size_t)2 * e->layers[0].gate.ntiles * GPT;
@@ -3269,7 +3355,7 @@ int nl_destroy(nl_handle e) {
         if (e->p2p.epoch) (void)hipFree(e->p2p.epoch);
     }
     void *bufs[] = {e->embd_raw, e->output_norm, e->rope_cos, e->rope_sin, e->x[0], e->x[1], e->qbuf, e->part_o,
-                    e->part_ml, e->hb, e->ar, e->parts, e->xchg, e->tp_xq, e->tp_xo, e->tp_xp, e->tp_hx, e->tick, e->parts_ffn, e->xchg_ffn, e->samp_keep, e->logits, e->kcache, e->vcache, e->ctl, e->ids, e->result, e->amax_val,
+                    e->part_ml, e->hb, e->ar, e->parts, e->xchg, e->tp_xq, e->tp_xo, e->tp_xp, e->tp_hx, e->tick, e->ly.tab, e->ly.gran, e->parts_ffn, e->xchg_ffn, e->samp_keep, e->logits, e->kcache, e->vcache, e->ctl, e->ids, e->result, e->amax_val,
                     e->amax_idx};
     for (void *b : bufs) if (b) hipFree(b);
     if (e->h_ctl) hipHostFree(e->h_ctl);
@@ -3498,7 +3584,7 @@ int nl_sample_decode(nl_handle e, int stream, int pos, int n_steps, const nl_sam
     }
     const SampScratch &s = e->sp;
     const int n_recent_in = *n_recent;
-    if (e->fused) {   // a redo after a fused-launch timeout restarts from the logits this call found (take_fused_timeout)
+    if (e->fused || e->ly.on) {   // a redo after a fused-launch timeout restarts from the logits this call found (take_fused_timeout)
         if (!e->samp_keep) { std::lock_guard<std::mutex> setup(g_setup_mu); HIPCK(e, dalloc(&e->samp_keep, (size_t)e->cfg.vocab, &e->bytes_state)); }
         HIPCK(e, hipMemcpyAsync(e->samp_keep, e->logits, (size_t)e->cfg.vocab * 4, hipMemcpyDeviceToDevice, e->stream));
     }
@@ -3938,6 +4024,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     int64_t n = 0;
     std::string w = which;
     if (w == "num_cus") { if (max_floats < 1) return 0; out[0] = (float)e->num_cus; return 1; }
+    if (w == "layers_max_pos") { if (max_floats < 1) return 0; out[0] = e->ly.on ? (float)e->ly.max_pos : 0.f; return 1; }      // (host state)
     if (w == "step_path") { if (max_floats < 1) return 0; out[0] = (float)e->step_path; return 1; }      // (host state)
     if (w == "x") { src = e->x[0]; n = e->cfg.dim; }
     else if (w == "x1") { src = e->x[1]; n = e->cfg.dim; }

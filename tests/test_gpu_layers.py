@@ -1,0 +1,102 @@
+"""GPU: all layers of a decode step in one launch (nl_layers.h) against the five-launch plan, at the edges of its passes, units and column groups."""
+import numpy as np
+import pytest
+
+from nanollama_amd import gguf, synth
+
+pytestmark = pytest.mark.gpu
+
+# layers, width, query heads, kv heads, feed-forward, options; positions
+SHAPES = {
+    "middle": ((2, 1536, 24, 6, 4096, {}), (0, 1, 15, 16, 126, 127, 128, 129, 255, 256, 640, 1030)),                    # the largest feed-forward: a tile a workgroup
+    "ragged": ((3, 576, 9, 9, 1472, {}), (0, 17, 127, 128, 300)),                                                      # last groups of one and three pairs
+    "small": ((2, 128, 2, 1, 192, {}), (0, 5, 127, 128, 140)),                                                         # half a group a row
+    "widest": ((2, 2048, 32, 8, 4096, {}), (0, 127, 128, 1023, 1024, 1100, 2046)),                                     # from 1024 on two heads a unit
+    "eight_to_one": ((2, 1024, 16, 2, 2048, {}), (3, 200, 2040)),
+    "variant": ((2, 768, 12, 3, 2048, dict(rope_conjugate=True, attn_bias=True)), (0, 60, 127, 128, 200)),
+}
+
+
+def _models(tmp_path, monkeypatch, name, wtype, vocab=512, seq_len=2048):
+    from nanollama_amd import model as hip
+    (layers, dim, heads, kv, ff, opts), _ = SHAPES[name]
+    shape = synth.ModelShape(name, layers, dim, heads, kv, vocab, seq_len=seq_len, interm=ff, **opts)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), shape, wtype, 91, mode="qrand")
+    g = gguf.load_gguf(str(p))
+    monkeypatch.setenv("NL_LAYERS", "2")
+    dev = hip.load_llama_model(g)
+    monkeypatch.setenv("NL_LAYERS", "0")
+    monkeypatch.setenv("NL_FUSED_ATTN", "0")
+    plain = hip.load_llama_model(g)
+    return shape, dev, plain
+
+
+@pytest.mark.parametrize("name,wtype", [(n, w) for n in SHAPES for w in ("q8_0", "q4_0")] + [("middle", "q5_0")])
+def test_against_the_five_launch_plan(tmp_path, monkeypatch, name, wtype):
+    shape, dev, plain = _models(tmp_path, monkeypatch, name, wtype)
+    assert dev.debug_read("layers_max_pos", 1)[0] == 2048 and plain.debug_read("layers_max_pos", 1)[0] == 0
+    positions = SHAPES[name][1]
+    toks = synth.prompt_ids(max(positions) + 1, shape.vocab, seed=11)
+    for m in (dev, plain):
+        m.prefill(toks, want_logits=False)
+    for pos in positions:
+        for m in (dev, plain):
+            m.forward(toks[pos] % 500 + 3, pos)
+        # (float32 sums in another order through two or three layers)
+        assert np.abs(dev.state.logits - plain.state.logits).max() <= 1e-4 * max(1.0, float(plain.state.logits.std())), pos
+    n = shape.n_layer * shape.n_kv_head * shape.seq_len * 64
+    for which in ("k_cache", "v_cache"):       # rows that both wrote at those positions, of values up to 10
+        a, b = dev.debug_read(which, n).reshape(-1, shape.seq_len, 64), plain.debug_read(which, n).reshape(-1, shape.seq_len, 64)
+        assert np.abs(a - b).max() <= 1e-4
+    assert dev.decode_greedy(5, 120, 40) == plain.decode_greedy(5, 120, 40)        # graphs of sixteen steps and single ones, across a pass
+    assert dev.last_error() == ""
+    dev.close(); plain.close()
+
+
+def test_streams_and_sampled_chains(tmp_path, monkeypatch):
+    from nanollama_amd import model as hip
+    (layers, dim, heads, kv, ff, opts), _ = SHAPES["middle"]
+    shape = synth.ModelShape("streams", layers, dim, heads, kv, 512, seq_len=300, interm=ff)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), shape, "q8_0", 92, mode="qrand")
+    g = gguf.load_gguf(str(p))
+    out = []
+    for knob in ("2", "0"):
+        monkeypatch.setenv("NL_LAYERS", knob)
+        m = hip.load_llama_model(g, max_streams=3)
+        assert (m.debug_read("layers_max_pos", 1)[0] > 0) == (knob == "2")
+        got = []
+        for s, n in ((2, 140), (0, 20)):
+            toks = synth.prompt_ids(n, shape.vocab, seed=s)
+            m.prefill(toks, 0, s)
+            ids, _ = m.sample_decode(n, 37, temperature=0.8, top_p=0.9, top_k=50, rep_penalty=1.15, rep_window=64,
+                                     uniforms=np.random.default_rng(s).random(37, dtype=np.float32), recent=[], stream=s)
+            got.append(ids)
+        out.append(got)
+        m.close()
+    assert out[0] == out[1]
+
+
+def test_a_wait_that_gives_up_is_redone_on_the_five_launch_plan(tmp_path, monkeypatch):
+    monkeypatch.setenv("NL_FUSED_SPIN_LIMIT", "0")
+    monkeypatch.setenv("NL_QUIET", "1")
+    shape, dev, plain = _models(tmp_path, monkeypatch, "variant", "q8_0")
+    toks = synth.prompt_ids(6, shape.vocab, seed=3)
+    for pos, t in enumerate(toks):
+        for m in (dev, plain):
+            m.forward(t, pos)
+        assert np.array_equal(dev.state.logits, plain.state.logits), pos
+    assert "timed out" in dev.last_error() and dev.debug_read("layers_max_pos", 1)[0] == 0
+    dev.close(); plain.close()
+
+
+@pytest.mark.parametrize("layers,wtype,runs", [(2, "q8_0", False), (4, "q8_0", True), (4, "q4_k", False)])
+def test_models_that_take_the_launch(tmp_path, monkeypatch, layers, wtype, runs):
+    from nanollama_amd import model as hip
+    monkeypatch.delenv("NL_LAYERS", raising=False)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("rule", layers, 1024, 16, 4, 512, seq_len=160, interm=1024), wtype, 5, mode="qrand")
+    m = hip.load_llama_model(gguf.load_gguf(str(p)))
+    assert m.debug_read("layers_max_pos", 1)[0] == (160 if runs else 0)
+    m.close()
