@@ -1,6 +1,6 @@
 // nl_pgemm.h -- the multi-token GEMM of long token runs and of K-quant files: Y[n][row] = sum_k W[row][k] X[n][k], every block format.
 //
-// Tile: a workgroup of four wavefronts owns RT 16-row weight tiles x 4 NTW 16-token tiles.  Its threads expand the weights of a
+// Tile: a workgroup of four wavefronts owns RT 16-row weight tiles x 4 NTW / WR 16-token tiles.  Its threads expand the weights of a
 // 128-column chunk ONCE into fp16 MFMA fragments in LDS (two buffers); every wavefront multiplies them against its own NTW token
 // tiles, whose hi / lo activation fragments go straight from the fragment store into its registers.
 //
@@ -168,20 +168,22 @@ __device__ __forceinline__ f32x4_t pg_mma(const uint4 &x, const half8_t &w, f32x
 }
 enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 
+// WR: the wavefronts of a set split the rows WR ways and share 64 NTW / WR tokens.
 // EPI: QG_EPI_PLAIN (out / resid / bias; optionally the folded norm's fragments and sums of squares), QG_EPI_SWIGLU
 // (RT / 2 tiles of gate, the same of up), QG_EPI_ROPE (a layer's packed Q|K|V).  PREC: PG_HILO; PG_HI, the single-product precision mode of
 // Q4_0 prompts (block scales multiplied into the fp16 weights, only the hi half of every activation); PG_EXACT.
 // Wavefronts per SIMD: a plain 64 x 64 Q4_0 tile is held to 168 registers, three workgroups a compute unit (172 without the bound, since the
 // loads are buffer loads: two.  WO and down of 2112 x 2112 and 2112 x 5632, 1000 tokens, 528 workgroups, mean of both: 63.4 us two at a time,
 // 53.9 three).  What it spills is a value of the epilogue's, around the K loop.
-template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO>
+template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO, int WR = 1>
 __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT == 4 && NTW == 1 && PREC == PG_HILO ? 3 : 2)) pgemm_kernel(QGemmParams P) {
     constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
     using F = typename std::conditional_t<EXACT, PgExact<WT>, PgFmt<WT>>;
     static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");
     constexpr int NP = X1 ? 1 : EXACT ? 3 : 2, PS = EXACT ? 3 : 2;      // parts of an activation that are read, and that are stored
     constexpr int KB = 4;                                   // blocks per chunk
-    constexpr int ROWS = RT * TR, TOK = 64 * NTW, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
+    constexpr int RTW = RT / WR, TTW = 4 * NTW / WR;        // row tiles of a wavefront, token tiles of a workgroup
+    constexpr int ROWS = RT * TR, TOK = TTW * 16, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
     constexpr int SC = X1 ? PG_NONE : F::SC;
     constexpr bool MINS = WT == WT_Q4_K, PAIRS = EXACT || WT == WT_Q4_0;
     // The bounded tile whose epilogue spills makes the scales' offset of the weights' (52 bytes of scratch otherwise: 2112 columns, 1000 tokens, all of its
@@ -206,7 +208,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (((int)blockIdx.x >> 3) >= per || id >= total) return;
     const bool by_rows = (long long)P.ntiles * TR * (FUSED ? 2 : 1) * F::CPP > (long long)P.n_tokens * 8 * PS;
-    const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, ttile0 = tb * 4 * NTW + wave * NTW;
+    const int tb = by_rows ? id % ntb : id / nrb, rbk = by_rows ? id / ntb : id % nrb, tile0 = rbk * TPW, row0 = tile0 * TR, tok0 = tb * TOK, wt0 = wave % (4 / WR) * NTW, ttile0 = tb * TTW + wt0, wr0 = wave / (4 / WR) * RTW;
 
     // F16 and Q8_0: a group of four pairs is two chunks, the even blocks of its pairs, then the odd ones.  A wavefront's load is then one 16-byte plane of
     // all four pairs over a tile's rows, a whole KiB; two pairs with both their blocks (PAIRS) are half of every 64-byte run, twice the sectors.  Profiled
@@ -303,14 +305,14 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
 #pragma unroll
             for (int k = 0; k < NP; k++) xp[k][b][t] = pg_load16(rx, xlane, uo + xtile[t] + k * QG_FRAG * 16);
     };
-    f32x4_t acc[RT][NTW];
+    f32x4_t acc[RTW][NTW];
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++)
+    for (int rt = 0; rt < RTW; rt++)
 #pragma unroll
         for (int t = 0; t < NTW; t++) acc[rt][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     // PG_EXACT: the sums of two chunks are kept apart and join the accumulators with what the addition drops carried on (Kahan): a plain
     // chain over K / 32 blocks is further off than the single-token plan's lanes and trees (relative error at K = 10752 1.8e-7 against 1.1e-7)
-    [[maybe_unused]] f32x4_t part[EXACT ? RT : 1][NTW] = {}, lost[EXACT ? RT : 1][NTW] = {};
+    [[maybe_unused]] f32x4_t part[EXACT ? RTW : 1][NTW] = {}, lost[EXACT ? RTW : 1][NTW] = {};
 
     const int niter = (nchunks + KW - 1) / KW;               // (every set runs as many chunks; past the end of K: zeros)
     int chunk = kset;
@@ -343,7 +345,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
             if (p0 == 0) s_tok[t] = inv;
         }
     // producer: what its epilogue needs is requested here, ahead of the K loop -- behind it, every dependent fetch is a round trip of its own
-    constexpr int RQ = ROWS / 4, NIT = TOK * RQ / NTHR, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 && !(EXACT && KW == 1) ? NIT : 1;    // (EXACT, one set: no registers for it)
+    constexpr int RQ = ROWS / 4, NIT = TOK * RQ > NTHR ? TOK * RQ / NTHR : 1, NRES = EPI == QG_EPI_PLAIN && NIT <= 4 && !(EXACT && KW == 1) ? NIT : 1;    // (EXACT, one set: no registers for it)
     [[maybe_unused]] f32x4_t res[NRES];
     [[maybe_unused]] const bool vec = (P.ldo & 3) == 0;
     [[maybe_unused]] const float *const resid = P.resid;
@@ -367,7 +369,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     // cores, group i + 1's weight fragments leave LDS and group i - 1's sums are scaled.  One barrier per chunk, in front of its last
     // group: the next chunk's fragments are then complete (all parts were stored by block 2) and the last group's are already in
     // registers, so the buffer that the next chunk's stores will overwrite has no reader left.
-    constexpr int RG = NTW == 1 && !EXACT ? 4 : 2, NG = RT / RG, STEPS = KB * NG;
+    constexpr int RG = RTW == 1 ? 1 : NTW == 1 && !EXACT && RTW >= 4 ? 4 : 2, NG = RTW / RG, STEPS = KB * NG;
     static_assert(STEPS % 2 == 0, "ping-pong");
     half8_t wf[2][F::FR][RG];
     f32x4_t z[2][RG][NTW], xs[2][NTW];
@@ -379,11 +381,11 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         for (int p = 0; p < F::FR; p++)
 #pragma unroll
             for (int q = 0; q < RG; q++)
-                wf[idx & 1][p][q] = *reinterpret_cast<const half8_t *>(smem + bf * BUF + b * PLANE + (p * RT + r0 + q) * 1024 + lane * 16);
+                wf[idx & 1][p][q] = *reinterpret_cast<const half8_t *>(smem + bf * BUF + b * PLANE + (p * RT + wr0 + r0 + q) * 1024 + lane * 16);
 #pragma unroll
         for (int q = 0; q < RG; q++) {
-            if constexpr (SC != PG_NONE) dv[idx & 3][q] = *reinterpret_cast<const float *>(s_sc + bf * SCB + (b * SCP + (r0 + q) * 16 + li) * 4);
-            if constexpr (MINS) mv[idx & 3][q] = *reinterpret_cast<const float *>(s_mn + bf * SCB + (b * SCP + (r0 + q) * 16 + li) * 4);
+            if constexpr (SC != PG_NONE) dv[idx & 3][q] = *reinterpret_cast<const float *>(s_sc + bf * SCB + (b * SCP + (wr0 + r0 + q) * 16 + li) * 4);
+            if constexpr (MINS) mv[idx & 3][q] = *reinterpret_cast<const float *>(s_mn + bf * SCB + (b * SCP + (wr0 + r0 + q) * 16 + li) * 4);
         }
     };
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -473,7 +475,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         if (i + 1 < niter) do_chunk(std::integral_constant<int, 1>{});
         if constexpr (EXACT) {
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++)
+            for (int rt = 0; rt < RTW; rt++)
 #pragma unroll
                 for (int t = 0; t < NTW; t++)
 #pragma unroll
@@ -491,11 +493,11 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     __syncthreads();
     float *const S = reinterpret_cast<float *>(smem);
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++)
+    for (int rt = 0; rt < RTW; rt++)
 #pragma unroll
         for (int t = 0; t < NTW; t++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) S[((wave * NTW + t) * 16 + 4 * lq + j) * LD + rt * 16 + li] = acc[rt][t][j];
+            for (int j = 0; j < 4; j++) S[((wt0 + t) * 16 + 4 * lq + j) * LD + (wr0 + rt) * 16 + li] = acc[rt][t][j];
     __syncthreads();
     const int et = threadIdx.x;
     const float *const S0 = reinterpret_cast<const float *>(smem_all);
@@ -512,9 +514,9 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         // h = SiLU(gate) * up (go/quant.go:629-631, go/model.go:604-606), stored as the down projection's fragments
 #pragma unroll
         for (int it0 = 0; it0 < TOK * 4 * (RT / 4); it0 += NTHR) {
-            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % (4 * NTW), hb = (it >> 6) / (4 * NTW), t = tt * 16 + li, n = tok0 + t;
+            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % TTW, hb = (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t;
             const int hblk = tile0 / 2 + hb;
-            if (NTHR > TOK * RT && hb >= RT / 4) break;     // (two sets of wavefronts over 32 rows: the second has no item)
+            if (NTHR > TOK * RT && hb >= RT / 4) break;     // (more threads than items of 32 rows)
             int oa, ob;
             slot_offsets(P.out_q4, w, oa, ob);
             const int sg = t * LD + hb * 32, su = sg + ROWS / 2;
@@ -545,6 +547,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
 #pragma unroll 2
         for (int it0 = 0; it0 < TOK * RT * 2; it0 += NTHR) {
             const int it = it0 + et, u = it % (RT * 2), t = it / (RT * 2), rt = u >> 1, grp = u & 1, n = tok0 + t, nn = min(n, P.n_tokens - 1);
+            if (NTHR > TOK * RT * 2 && t >= TOK) break;
             const int tile = min(tile0 + rt, P.ntiles - 1), head = tile / tph, i0 = (tile % tph) * 8 + 4 * grp;
             const bool is_q = head < R.n_q_heads, is_k = !is_q && head < R.n_q_heads + R.n_kv_heads;
             const int kvh = head - R.n_q_heads - (is_k ? 0 : R.n_kv_heads);
@@ -606,7 +609,8 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
                 const int kvh = (tile0 >> 2) + hh - R.n_q_heads - R.n_kv_heads;
                 if (kvh < 0 || tile0 + 4 * hh >= P.ntiles) continue;
                 for (int it = et; it < 8 * keys; it += NTHR) {
-                    const int sg = it & 7, d = (it >> 3) & 63, t0 = (it >> 9) * 64 + (sg >> 2) * 32 + (sg & 3) * 4, n0 = tok0 + t0;
+                    constexpr int SG = TOK % 64 ? 4 : 8;                // segments of an element: a tile's keys, or 64
+                    const int sg = it % SG, d = (it / SG) & 63, t0 = it / (SG * 64) * (SG * 8) + (sg >> 2) * 32 + (sg & 3) * 4, n0 = tok0 + t0;
                     const int col = hh * 64 + ((d & 31) >> 3) * 16 + (d & 7) + 8 * (d >> 5);
                     const float bias = R.bias_v ? R.bias_v[kvh * 64 + d] : 0.f;
                     half8_t hi = {}, lo = {};
@@ -645,6 +649,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
 #pragma unroll
             for (int i = 0; i < UN; i++) {
                 const int it = (i0 + i) * NTHR + et, a = it % RQ, t = it / RQ, n = tok0 + t, row = row0 + 4 * a;
+                if (NTHR > TOK * RQ && t >= TOK) continue;
                 v[i] = sum4(t * LD + 4 * a);
                 const size_t off = (size_t)n * P.ldo + row;
                 if (vec && row + 3 < P.rows) {
@@ -677,7 +682,8 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         __syncthreads();
 #pragma unroll 2
         for (int it0 = 0; it0 < TOK * 4 * (ROWS / 32); it0 += NTHR) {
-            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % (4 * NTW), kb = (it >> 6) / (4 * NTW), t = tt * 16 + li, n = tok0 + t, c0 = row0 + kb * 32;
+            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % TTW, kb = (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t, c0 = row0 + kb * 32;
+            if (NTHR > TOK * ROWS / 8 && kb >= ROWS / 32) break;
             if (n >= P.n_tokens || c0 >= P.rows) continue;
             int oa, ob;
             slot_offsets(P.out_q4, w, oa, ob);
@@ -693,13 +699,13 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
 
 template <int WT, int EPI, int PREC>
 hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
-    auto go = [&](auto rt, auto ntw, auto kw) {
-        constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT;
-        const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + 64 * NTW - 1) / (64 * NTW));
-        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC>), dim3((total + 7) / 8 * 8), dim3(256 * KW), 0, st, P);
+    using std::integral_constant;
+    auto go = [&](auto rt, auto ntw, auto kw, auto wr) {
+        constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, WR = decltype(wr)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT, TOK = 64 * NTW / WR;
+        const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + TOK - 1) / TOK);
+        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC, WR>), dim3((total + 7) / 8 * 8), dim3(256 * KW), 0, st, P);
         return hipGetLastError();
     };
-    using std::integral_constant;
     const integral_constant<int, 1> one{};
     const integral_constant<int, 2> two{};
     const integral_constant<int, 4> four{};
@@ -710,15 +716,25 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     // for it with two sets).  Beyond, one set, and tiles that grow as the grid allows it (Q4_0 4096 x 768 x 2047, gate and up: 128 x 128
     // 31.8 us, 64 x 128 35.0, 64 x 64 37.0; Q8_0's expansion leaves no registers for 128 x 128: 68.9 us against 62.2).
     const long long tiles = (long long)((P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4) * ((P.n_tokens + 63) / 64);
-    if (tiles <= 256) return go(four, one, two);
+    // Half or a quarter of a unit's tokens where that many workgroups still find a unit each: the wavefronts share the tokens and split the rows, a row
+    // tile's scalings and products are half or a quarter a wavefront, the expansion of the weights is done two or four times over the chip.  The order of the
+    // sums stays.  us a launch, 64 x 64 / x 32 / x 16: Q4_K 768 x 768 and x 2048, 333 tokens 11.3 / 8.9 / 8.3 and 22.0 / 16.7 / 15.1; 1152 x 768 11.6 / 9.3 / 14.3
+    // (378 workgroups); Q6_K 12.5 / 9.6 and 24.7 / 18.4; Q4_0 7.2 / 5.9 / 5.6 and 12.0 / 9.7 / 9.3, 1536 x 4096 at 150 19.8 / 15.1 / 14.3, at 500 21.8 / 26.5 (384);
+    // Q8_0 7.3 / 6.2 / 6.0 and 12.3 / 10.0 / 9.6; F16 6.6 / 6.0 / 5.9 and 10.7 / 9.6 / 9.6: no quarters.  (none either where V^T's image
+    // is written: its segments hold keys of two 16-token tiles)
+    const long long rb = (P.ntiles * (EPI == QG_EPI_SWIGLU ? 2 : 1) + 3) / 4;
+    if constexpr (WT != WT_F16)
+        if (rb * ((P.n_tokens + 15) / 16) <= 256 && !(EPI == QG_EPI_ROPE && P.rope.kv16)) return go(four, one, two, four);
+    if (rb * ((P.n_tokens + 31) / 32) <= 256) return go(four, one, two, two);
+    if (tiles <= 256) return go(four, one, two, one);
     // (three parts, the sums of a chunk pair and what their additions drop leave no registers for a second token tile: 46 to 150 spilled)
-    if constexpr (PREC == PG_EXACT) return go(four, one, one);
+    if constexpr (PREC == PG_EXACT) return go(four, one, one, one);
     else {
-        if (tiles <= 512) return go(four, two, two);
-        if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one);
+        if (tiles <= 512) return go(four, two, two, one);
+        if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one, one);
         if constexpr (WT == WT_Q4_0 || WT == WT_F16)
-            if (tiles >= 1792) return go(eight, two, one);
-        return go(four, two, one);
+            if (tiles >= 1792) return go(eight, two, one, one);
+        return go(four, two, one, one);
     }
 }
 template <int EPI>
