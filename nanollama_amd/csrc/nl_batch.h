@@ -581,8 +581,10 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     const int kvh = blockIdx.x, split = blockIdx.y, i0 = blockIdx.z * QT, tid = threadIdx.x;
     const int t0 = split * ATT_CH;
     int maxpos = -1;
-    for (int i = 0; i < QT; i++)
-        if (i0 + i < n_items) maxpos = max(maxpos, P.bpos[i0 + i]);
+    if (P.pos_base_valid) maxpos = P.pos_base + min(i0 + QT, n_items) - 1;      // a prompt: consecutive positions, nothing to read
+    else
+        for (int i = 0; i < QT; i++)
+            if (i0 + i < n_items) maxpos = max(maxpos, P.bpos[i0 + i]);
     if (t0 > maxpos) return;
     const int nrows = min(ATT_CH, maxpos + 1 - t0);
     const int lane = tid & 63, w = tid >> 6, j = lane & 15, kq = lane >> 4;
@@ -604,13 +606,17 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
             for (int s = 0; s < DK; s++) qa[s] = 0.f;
         }
     }
-    const long long soff = (long long)P.bstream[i0] * P.kv_stream_stride;
+    const long long soff = P.single_stream ? 0 : (long long)P.bstream[i0] * P.kv_stream_stride;
     const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
     const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
-    // every global load of the staging pass is issued before the first LDS store (one memory latency, not NIT);
-    // all 8 key tiles are always computed (uniform, branch-free MFMA stream); rows beyond nrows are zero-filled
-    // (masked to p = 0 by the softmax, and 0 * garbage could be NaN in P V otherwise)
+    // every global load of the staging pass is issued before the first LDS store (one memory latency, not NIT).
+    // Key tiles are computed two at a time and only where a row of the workgroup can see one (uniform tests: masked probabilities are zeros, so
+    // the sums are the same bits); rows beyond nrows of the last two are zero-filled (masked to p = 0 by the softmax, and 0 * garbage could be
+    // NaN in P V otherwise).  What bounds the launch is one wavefront's chain: 256 products of 32 cycles and 32 exponentials a lane where all eight
+    // tiles are taken, 4 us.  us a launch with the merge behind it, three kv heads of four: 17 tokens 10.0 + 4.8, now 6.9; 100 tokens 10.7 + 4.7, now 10.6; six
+    // kv heads, 33 tokens 10.2 + 5.0, now 8.4; partials and merge of 333 tokens as before
     constexpr int NIT = (ATT_CH * R4 + NTH - 1) / NTH;
+    const int nfill = (nrows + 31) & ~31;
     float4 kreg[NIT], vreg[NIT];
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
@@ -622,14 +628,14 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
         const int i = tid + it * NTH, row = i / R4, c4 = i % R4;
-        if (i < ATT_CH * R4) {
+        if (row < nfill) {
             *reinterpret_cast<float4 *>(Ks + row * KS + c4 * 4) = kreg[it];
             *reinterpret_cast<float4 *>(Vs + row * HD + c4 * 4) = vreg[it];
         }
     }
     if (tid < VH) {
         const int item = i0 + tid / G;
-        nv[tid] = item < n_items ? min(ATT_CH, max(0, P.bpos[item] + 1 - t0)) : 0;
+        nv[tid] = item < n_items ? min(ATT_CH, max(0, (P.pos_base_valid ? P.pos_base + item : P.bpos[item]) + 1 - t0)) : 0;
     }
     __syncthreads();
 
@@ -638,23 +644,26 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
     v4f acc[8];
 #pragma unroll
-    for (int mt = 0; mt < 8; mt++) acc[mt] = zero;
+    for (int mg = 0; mg < 8; mg += 2) {
+        acc[mg] = acc[mg + 1] = zero;
+        if (mg * 16 >= nfill) continue;
 #pragma unroll
-    for (int s4 = 0; s4 < DK / 4; s4++) {
-        float4 kb[8];
+        for (int s4 = 0; s4 < DK / 4; s4++) {
+            float4 kb[2];
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++)
-            kb[mt] = *reinterpret_cast<const float4 *>(Ks + (mt * 16 + j) * KS + DK * kq + 4 * s4);
-        // (four products to a chain: one chain over a head of 64 is off by 1.4e-7, chains of four that are added by 8.3e-8, as the per-token kernel)
-        v4f part[8];
+            for (int mt = 0; mt < 2; mt++)
+                kb[mt] = *reinterpret_cast<const float4 *>(Ks + ((mg + mt) * 16 + j) * KS + DK * kq + 4 * s4);
+            // (four products to a chain: one chain over a head of 64 is off by 1.4e-7, chains of four that are added by 8.3e-8, as the per-token kernel)
+            v4f part[2];
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].x, qa[4 * s4], zero, 0, 0, 0);
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].x, qa[4 * s4], zero, 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].y, qa[4 * s4 + 1], part[mt], 0, 0, 0);
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].y, qa[4 * s4 + 1], part[mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].z, qa[4 * s4 + 2], part[mt], 0, 0, 0);
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].z, qa[4 * s4 + 2], part[mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) acc[mt] += __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].w, qa[4 * s4 + 3], part[mt], 0, 0, 0);
+            for (int mt = 0; mt < 2; mt++) acc[mg + mt] += __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].w, qa[4 * s4 + 3], part[mt], 0, 0, 0);
+        }
     }
 
     // ---- softmax pieces of row j: 32 keys in this lane, the rest in lanes j+16, j+32, j+48 ----
@@ -672,13 +681,15 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     m = fmaxf(m, __shfl_xor(m, 32));
     float l = 0.f;
 #pragma unroll
-    for (int mt = 0; mt < 8; mt++)
+    for (int mt = 0; mt < 8; mt++) {
+        if (mt * 16 >= nfill) continue;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const float pv = mt * 16 + 4 * kq + r < nvj ? expf(acc[mt][r] - m) : 0.f;
             acc[mt][r] = pv;
             l += pv;
         }
+    }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
 
@@ -688,6 +699,7 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     for (int nt = 0; nt < NTO; nt++) o[nt] = zero;
 #pragma unroll
     for (int s = 0; s < 8; s++) {
+        if (s * 16 >= nfill) continue;
         v4f part[NTO];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -700,6 +712,36 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
         }
 #pragma unroll
         for (int nt = 0; nt < NTO; nt++) o[nt] += part[nt];
+    }
+
+    if (P.fin_xf) {
+        // every row's only split (positions below 128): o / l as the WO GEMM's fragments, battn_merge_kernel's arithmetic for one partial, by way
+        // of LDS, where K was
+        constexpr int OS = HD + 4;
+        static_assert(VH * OS <= ATT_CH * KS, "the rows fit");
+        __syncthreads();
+        const float il = 1.0f / l;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float sc = __shfl(il, 4 * kq + r);                         // (lane j holds row j's)
+            float *po = Ks + (w * 16 + 4 * kq + r) * OS + NTO * j;
+            if constexpr (NTO == 4) *reinterpret_cast<float4 *>(po) = make_float4(o[0][r] * sc, o[1][r] * sc, o[2][r] * sc, o[3][r] * sc);
+            else *reinterpret_cast<float2 *>(po) = make_float2(o[0][r] * sc, o[1][r] * sc);
+        }
+        __syncthreads();
+        // the tokens of an entry's fragment side by side: thread = (head, entry of a head's HD / 8, token)
+#pragma unroll
+        for (int i = tid; i < VH * HD / 8; i += NTH) {
+            const int t = i % QT, u = i / QT, e = u % (HD / 8), g = u / (HD / 8), item = i0 + t;
+            if (item >= n_items) continue;
+            const float *src = Ks + (t * G + g) * OS + (e >> 2) * 32;
+            int offa, offb;
+            slot_offsets(P.fin_form, e & 3, offa, offb);
+            float v[8];
+            slots_from(P.fin_form, *reinterpret_cast<const float4 *>(src + offa), *reinterpret_cast<const float4 *>(src + offb), v);
+            store_frag(P.fin_xf, P.fin_nt16, item, ((kvh * G + g) * HD) / 32 + (e >> 2), e & 3, v, P.fin_form);
+        }
+        return;
     }
 
     // O tile: this lane holds rows 4*kq+r, columns d = NTO*j .. NTO*j+NTO-1

@@ -2262,7 +2262,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 T.pos_base = b.h_meta[b.cap];
                 T.live_map = n_live > 0 ? b.tok + 3 * b.cap : nullptr;
                 // every row's keys in one run: no partials, the launch writes WO's fragments (not the float32 tile)
-                if (n_live > 0 && max_nparts == 1 && !kv16_on && !no_fin) {
+                if ((f32_tile ? nsplit == 1 : n_live > 0 && max_nparts == 1 && !kv16_on) && !no_fin) {
                     T.fin_xf = b.xfrag; T.fin_nt16 = nt16; T.fin_form = form(L.wo);
                     merged = true;
                     e->step_path |= PATH_TILE_FIN;
