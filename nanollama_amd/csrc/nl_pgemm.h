@@ -130,10 +130,19 @@ template <> struct PgExact<WT_Q4_K> {
     static __device__ __forceinline__ int chunk(int, int i) { return i; }
     static __device__ __forceinline__ void part(const uint4 (&c)[2], const uint32_t (&)[2], int h, int w, half8_t (&f)[1]) {
         const uint4 &q = c[w >> 1];
-        const uint32_t u[2] = {(((w & 1) ? q.z : q.x) >> (4 * h)) & 0x0f0f0f0fu, (((w & 1) ? q.w : q.y) >> (4 * h)) & 0x0f0f0f0fu};
+        const uint32_t u[2] = {(w & 1) ? q.z : q.x, (w & 1) ? q.w : q.y};
+        // the nibbles where they are, in the mantissa of fp16 numbers: 1024 + q or 1024 + 16 q, and q - 8 by one v_fma_mix_f32 each, exactly.  (A field extraction,
+        // a subtraction and a conversion a value: 223 vector instructions a chunk beside its 24 MFMAs, now 175.  us a launch: 1536 x 1536 and x 4096, 33 tokens, the
+        // mean 18.4 -> 16.7, 768 x 768 and x 2048, 100 tokens 12.0 -> 10.8, gate and up there 12.2 -> 11.6.  Q6_K's products by a scale gain nothing by it: 20.6, 20.8)
+        const uint32_t mask = h ? 0x00f000f0u : 0x000f000fu;
+        const float mul = h ? 0.0625f : 1.f, add = h ? -72.f : -1032.f;
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = (float)((u[j >> 2] >> (8 * (j & 3))) & 0xff) - 8.f;
+        for (int j = 0; j < 4; j++) {
+            const h2_t n = bits_h2(((u[j >> 1] >> (8 * (j & 1))) & mask) | 0x64006400u);      // bytes j & 1 and (j & 1) + 2
+            v[4 * (j >> 1) + (j & 1)] = fmaf((float)n[0], mul, add);
+            v[4 * (j >> 1) + (j & 1) + 2] = fmaf((float)n[1], mul, add);
+        }
         f[0] = pg_bf16(v);
     }
     static __device__ __forceinline__ float scale(const uint32_t (&s)[2], int h) { return h2f_bits(s[0] & 0xffff) * (float)((s[1] >> (16 * h)) & 0xff); }     // (17 bits)
