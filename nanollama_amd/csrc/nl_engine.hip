@@ -293,6 +293,8 @@ struct nl_engine {
         LayersEntry *tab = nullptr;
         u32x4 *gran = nullptr;    // gq | gr | go | gp | gh | gx | the XCDs' copies | tickets
     } ly;
+    hipEvent_t turn_done = nullptr;   // chip_turn: behind this handle's last launch whose workgroups wait for each other
+    bool turn_on = false;             // ... the handle is on its device's list
     float *parts = nullptr;       // [Hs][D] per-head WO partials of the fused block
     unsigned long long *xchg = nullptr;   // [Hs][192] granules exchanged inside a head's cluster
     unsigned *tick = nullptr;     // {forward counter, status} device words of the fused block
@@ -1265,26 +1267,82 @@ int plan_index(const nl_engine *e, int pos_last) {
 }
 nl_engine::PlanSet &pick_plan(nl_engine *e, int pos_last) { return e->ps[plan_index(e, pos_last)]; }
 
-int launch_step(nl_engine *e, int pos) {
-    nl_engine::PlanSet &S = pick_plan(e, pos);
-    if (S.exec) {
-        HIPCK(e, hipGraphLaunch(S.exec, e->stream));
-        return NL_OK;
+// A launch of nl_layers.h needs every compute unit of its device.  Two of them, of two handles whose threads decode at the same time, or one beside another
+// launch whose workgroups wait for each other (nl_block.h, nl_group.h, nl_tp.h, nl_persist.h), could each hold units that the other waits for until a bounded
+// poll gives up: half a second, and the handle is back on five launches a layer.  So where a device has several handles with such plans, and one of them
+// nl_layers.h's, these launches take turns, on the device: each waits for the event behind the last one of another handle.  A handle that is alone
+// records and waits for nothing.
+std::mutex g_turn_mu;
+struct ChipTurns { std::vector<nl_engine *> handles; nl_engine *last = nullptr; };
+ChipTurns g_turns[64];
+template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
+    if (!e->turn_on || !waits) return launch();
+    std::lock_guard<std::mutex> lk(g_turn_mu);
+    ChipTurns &T = g_turns[e->dev];
+    bool shared = false;
+    if (T.handles.size() > 1)
+        for (const nl_engine *h : T.handles) shared = shared || h->ly.tab;
+    if (!shared) return launch();
+    if (T.last && T.last != e) HIPCK(e, hipStreamWaitEvent(e->stream, T.last->turn_done, 0));
+    const int rc = launch();
+    HIPCK(e, hipEventRecord(e->turn_done, e->stream));
+    T.last = e;
+    return rc;
+}
+// (nl_finalize, nl_destroy)
+int chip_turn_join(nl_engine *e) {
+    if (e->dev < 0 || e->dev >= 64 || e->G != 1 || e->force_tp_plan || e->p2p.on || !(e->fused || e->ly.on || e->pd.candidate)) return NL_OK;
+    HIPCK(e, hipEventCreateWithFlags(&e->turn_done, hipEventDisableTiming));
+    std::lock_guard<std::mutex> setup(g_setup_mu), lk(g_turn_mu);        // (the other handle's stream must not be in a capture)
+    ChipTurns &T = g_turns[e->dev];
+    if (T.handles.size() == 1) {                             // what the other one launched while it was alone
+        T.last = T.handles[0];
+        HIPCK(e, hipEventRecord(T.last->turn_done, T.last->stream));
     }
-    return run_plan_eager(e, S);
+    T.handles.push_back(e);
+    e->turn_on = true;
+    return NL_OK;
+}
+void chip_turn_leave(nl_engine *e) {
+    if (e->turn_on) {
+        std::lock_guard<std::mutex> lk(g_turn_mu);
+        ChipTurns &T = g_turns[e->dev];
+        T.handles.erase(std::remove(T.handles.begin(), T.handles.end(), e), T.handles.end());
+        if (T.last == e) T.last = nullptr;
+    }
+    if (e->turn_done) (void)hipEventDestroy(e->turn_done);
+    e->turn_done = nullptr;
+    e->turn_on = false;
+}
+
+int launch_step(nl_engine *e, int pos) {
+    const int k = plan_index(e, pos);
+    nl_engine::PlanSet &S = e->ps[k];
+    return chip_turn(e, k > 0, [&]() -> int {
+        if (S.exec) {
+            HIPCK(e, hipGraphLaunch(S.exec, e->stream));
+            return NL_OK;
+        }
+        return run_plan_eager(e, S);
+    });
 }
 
 // One step through the call box: true = served (the done word carries the step's argmax in *id); false = this plan has no call
 // graph and the caller copies, launches and synchronises as before.
 bool call_step(nl_engine *e, int token, int pos, int stream, int hostout, int *id, int *rc) {
-    nl_engine::PlanSet &S = pick_plan(e, pos);
+    const int k = plan_index(e, pos);
+    nl_engine::PlanSet &S = e->ps[k];
     *rc = NL_OK;
     if (!S.call_exec) return false;
     const unsigned seq = ++e->box_seq;
     e->h_box[CTL_TOKEN] = token; e->h_box[CTL_POS] = pos; e->h_box[CTL_CHAIN] = 0; e->h_box[CTL_STEP] = 0;
     e->h_box[CTL_STREAM] = stream; e->h_box[CTL_HOSTOUT] = hostout;
     __atomic_store_n(e->h_box + 8, (int)seq, __ATOMIC_RELEASE);
-    if (hipGraphLaunch(S.call_exec, e->stream) != hipSuccess) { *rc = e->fail(NL_ERR_HIP, "hipGraphLaunch (call graph): %s", hipGetErrorString(hipGetLastError())); return true; }
+    *rc = chip_turn(e, k > 0, [&]() -> int {
+        if (hipGraphLaunch(S.call_exec, e->stream) != hipSuccess) return e->fail(NL_ERR_HIP, "hipGraphLaunch (call graph): %s", hipGetErrorString(hipGetLastError()));
+        return NL_OK;
+    });
+    if (*rc) return true;
     // spin on the done word; a step that does not answer within two seconds is looked at through the stream instead
     const auto t0 = std::chrono::steady_clock::now();
     unsigned long long d;
@@ -1527,11 +1585,15 @@ int pd_launch(nl_engine *e, int stream, int token, int pos, int n, float *host_l
     P.gx = d.gx; P.gqkv = d.gqkv; P.go = d.go; P.gxp = d.gxp; P.gh = d.gh; P.gam = d.gam; P.gpart = d.gpart;
     P.ids_out = e->ids; P.logits = e->logits; P.host_logits = host_logits;
     P.status = d.status; P.host_status = d.h_status; P.dbg = d.dbg;
-    if (c.dim == 576 && c.n_kv_heads == 9) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 9>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
-    else if (c.dim == 576) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 3>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
-    else if (c.n_kv_heads == 4) hipLaunchKernelGGL((pd_decode_kernel<8, 16, 4>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
-    else hipLaunchKernelGGL((pd_decode_kernel<8, 16, 2>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
-    HIPCK(e, hipGetLastError());
+    const int rc = chip_turn(e, true, [&]() -> int {
+        if (c.dim == 576 && c.n_kv_heads == 9) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 9>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
+        else if (c.dim == 576) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 3>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
+        else if (c.n_kv_heads == 4) hipLaunchKernelGGL((pd_decode_kernel<8, 16, 4>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
+        else hipLaunchKernelGGL((pd_decode_kernel<8, 16, 2>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
+        HIPCK(e, hipGetLastError());
+        return NL_OK;
+    });
+    if (rc) return rc;
     d.launches++; d.tokens += n;
     return NL_OK;
 }
@@ -3230,6 +3292,7 @@ int nl_finalize(nl_handle e) {
     HIPCK(e, hipStreamSynchronize(e->stream));
     if (int rc = build_all(e)) return rc;
     if (int rc = pd_build(e)) return rc;
+    if (int rc = chip_turn_join(e)) return rc;
     e->finalized = true;
     return NL_OK;
 }
@@ -3318,6 +3381,7 @@ int nl_destroy(nl_handle e) {
     (void)pd_session_close(e);
     pd_session_record(e, false);
     hipDeviceSynchronize();
+    chip_turn_leave(e);
     samp_free(e->sp);
     for (auto &S : e->ps) destroy_graphs(S);
     destroy_samp_graphs(e);
@@ -3514,9 +3578,10 @@ int nl_decode_greedy(nl_handle e, int stream, int token, int pos, int n_steps, i
             if ((rc = set_ctl(e, tok, p0, 1, stream))) return rc;
             int i = 0;
             for (; i + e->graph_steps <= m && e->graph_steps > 1; i += e->graph_steps) {
-                nl_engine::PlanSet &S = pick_plan(e, p0 + i + e->graph_steps - 1);   // highest position of these steps
+                const int k = plan_index(e, p0 + i + e->graph_steps - 1);   // highest position of these steps
+                nl_engine::PlanSet &S = e->ps[k];
                 if (!S.multi_exec) break;
-                HIPCK(e, hipGraphLaunch(S.multi_exec, e->stream));
+                if ((rc = chip_turn(e, k > 0, [&]() -> int { HIPCK(e, hipGraphLaunch(S.multi_exec, e->stream)); return NL_OK; }))) return rc;
             }
             for (; i < m; i++)
                 if ((rc = launch_step(e, p0 + i))) return rc;
@@ -3635,7 +3700,7 @@ int nl_sample_decode(nl_handle e, int stream, int pos, int n_steps, const nl_sam
                     break;
                 }
             }
-            HIPCK(e, hipGraphLaunch(e->samp_graph_exec[k], e->stream));
+            if ((rc = chip_turn(e, k > 0, [&]() -> int { HIPCK(e, hipGraphLaunch(e->samp_graph_exec[k], e->stream)); return NL_OK; }))) return rc;
             i += e->graph_steps;
         }
         for (; i < n; i++) {
