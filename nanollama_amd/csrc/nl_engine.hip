@@ -1275,14 +1275,16 @@ nl_engine::PlanSet &pick_plan(nl_engine *e, int pos_last) { return e->ps[plan_in
 std::mutex g_turn_mu;
 struct ChipTurns { std::vector<nl_engine *> handles; nl_engine *last = nullptr; };
 ChipTurns g_turns[64];
+// (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
 template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
     if (!e->turn_on || !waits) return launch();
-    std::lock_guard<std::mutex> lk(g_turn_mu);
     ChipTurns &T = g_turns[e->dev];
-    bool shared = false;
-    if (T.handles.size() > 1)
-        for (const nl_engine *h : T.handles) shared = shared || h->ly.tab;
-    if (!shared) return launch();
+    auto shared = [&] { return T.handles.size() > 1 && std::any_of(T.handles.begin(), T.handles.end(), [](const nl_engine *h) { return h->ly.tab != nullptr; }); };
+    {
+        std::lock_guard<std::mutex> lk(g_turn_mu);
+        if (!shared()) return launch();
+    }
+    std::scoped_lock lk(g_setup_mu, g_turn_mu);
     if (T.last && T.last != e) HIPCK(e, hipStreamWaitEvent(e->stream, T.last->turn_done, 0));
     const int rc = launch();
     HIPCK(e, hipEventRecord(e->turn_done, e->stream));
@@ -1293,7 +1295,7 @@ template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
 int chip_turn_join(nl_engine *e) {
     if (e->dev < 0 || e->dev >= 64 || e->G != 1 || e->force_tp_plan || e->p2p.on || !(e->fused || e->ly.on || e->pd.candidate)) return NL_OK;
     HIPCK(e, hipEventCreateWithFlags(&e->turn_done, hipEventDisableTiming));
-    std::lock_guard<std::mutex> setup(g_setup_mu), lk(g_turn_mu);        // (the other handle's stream must not be in a capture)
+    std::scoped_lock lk(g_setup_mu, g_turn_mu);              // (the other handle's stream must not be in a capture)
     ChipTurns &T = g_turns[e->dev];
     if (T.handles.size() == 1) {                             // what the other one launched while it was alone
         T.last = T.handles[0];
