@@ -1276,6 +1276,7 @@ std::mutex g_turn_mu;
 struct ChipTurns { std::vector<nl_engine *> handles; nl_engine *last = nullptr; };
 ChipTurns g_turns[64];
 // (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
+// (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
 template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
     if (!e->turn_on || !waits) return launch();
     ChipTurns &T = g_turns[e->dev];
@@ -3214,7 +3215,7 @@ int nl_finalize(nl_handle e) {
                       e->Is <= LY_MAX_FF && L0.qkv.ntiles <= e->num_cus && L0.gate.ntiles <= e->num_cus && 2 * L0.wo.ntiles <= e->num_cus && e->KVs <= e->num_cus;
             for (const auto &L : e->layers)
                 for (const PackedMat *m : {&L.qkv, &L.wo, &L.gate, &L.up, &L.down})
-                    ok = ok && (m->wtype == WT_Q8_0 || m->wtype == WT_Q4_0) && m->wtype == L0.qkv.wtype && m->ntiles * TR == m->rows && m->npairs * PAIR == m->cols;
+                    ok = ok && (m->wtype == WT_Q8_0 || m->wtype == WT_Q4_0 || m->wtype == WT_Q4_K || m->wtype == WT_Q6_K) && m->wtype == L0.qkv.wtype && m->ntiles * TR == m->rows && m->npairs * PAIR == m->cols;
             e->ly.on = ok && (lv == 2 || layers_pay(e));
             e->ly.max_pos = std::min({c.seq_len, e->num_cus / e->KVs * LY_PASS, LY_MAX_REC * LY_PASS});
             e->ly.min_pos = lv == 2 ? 0 : layers_min_pos(e);

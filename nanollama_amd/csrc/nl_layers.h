@@ -644,6 +644,8 @@ inline hipError_t launch_layers(int wtype, const LayersParams &P, int grid, hipS
     switch (wtype) {
     case WT_Q8_0: hipLaunchKernelGGL(layers_kernel<WT_Q8_0>, dim3(grid), dim3(LY_THREADS), 0, st, P); break;
     case WT_Q4_0: hipLaunchKernelGGL(layers_kernel<WT_Q4_0>, dim3(grid), dim3(LY_THREADS), 0, st, P); break;
+    case WT_Q4_K: hipLaunchKernelGGL(layers_kernel<WT_Q4_K>, dim3(grid), dim3(LY_THREADS), 0, st, P); break;
+    case WT_Q6_K: hipLaunchKernelGGL(layers_kernel<WT_Q6_K>, dim3(grid), dim3(LY_THREADS), 0, st, P); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

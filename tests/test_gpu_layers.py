@@ -12,6 +12,7 @@ SHAPES = {
     "ragged": ((3, 576, 9, 9, 1472, {}), (0, 17, 127, 128, 300)),                                                      # last groups of one and three pairs
     "small": ((2, 128, 2, 1, 192, {}), (0, 5, 127, 128, 140)),                                                         # half a group a row
     "widest": ((2, 2048, 32, 8, 4096, {}), (0, 127, 128, 1023, 1024, 1100, 2046)),                                     # from 1024 on two heads a unit
+    "wide_groups": ((2, 768, 12, 3, 1280, {}), (0, 31, 127, 128, 260)),                                                # 256-column groups, the last shares of five
     "eight_to_one": ((2, 1024, 16, 2, 2048, {}), (3, 200, 2040)),
     "variant": ((2, 768, 12, 3, 2048, dict(rope_conjugate=True, attn_bias=True)), (0, 60, 127, 128, 200)),
 }
@@ -32,7 +33,8 @@ def _models(tmp_path, monkeypatch, name, wtype, vocab=512, seq_len=2048):
     return shape, dev, plain
 
 
-@pytest.mark.parametrize("name,wtype", [(n, w) for n in SHAPES for w in ("q8_0", "q4_0")] + [("middle", "q5_0")])
+@pytest.mark.parametrize("name,wtype", [(n, w) for n in SHAPES for w in ("q8_0", "q4_0")] + [("middle", "q5_0")] +
+                         [(n, w) for n in ("middle", "wide_groups", "eight_to_one") for w in ("q4_k", "q6_k")])
 def test_against_the_five_launch_plan(tmp_path, monkeypatch, name, wtype):
     shape, dev, plain = _models(tmp_path, monkeypatch, name, wtype)
     assert dev.debug_read("layers_max_pos", 1)[0] == 2048 and plain.debug_read("layers_max_pos", 1)[0] == 0
@@ -91,7 +93,7 @@ def test_a_wait_that_gives_up_is_redone_on_the_five_launch_plan(tmp_path, monkey
     dev.close(); plain.close()
 
 
-@pytest.mark.parametrize("layers,wtype,runs", [(2, "q8_0", False), (4, "q8_0", True), (4, "q4_k", False)])
+@pytest.mark.parametrize("layers,wtype,runs", [(2, "q8_0", False), (4, "q8_0", True), (4, "q4_k", True), (4, "f16", False)])
 def test_models_that_take_the_launch(tmp_path, monkeypatch, layers, wtype, runs):
     from nanollama_amd import model as hip
     monkeypatch.delenv("NL_LAYERS", raising=False)
