@@ -420,6 +420,7 @@ struct BMergeParams {
     int heads, nsplit_max, head_dim;
     uint4 *xf;   // attention output [N][heads*hd] as MFMA fragments for the WO GEMM
     int nt16, form;
+    int pos_base;   // >= 0: a prompt from this position on, one partial per 128 positions (nothing to read)
     int fast_exp;   // split weights on v_exp_f32 (prompts: their partials come from attn_tile16_kernel's v_exp_f32 already)
 };
 
@@ -435,7 +436,7 @@ __global__ void battn_merge_kernel(BMergeParams P, int n_items) {
     const long long total = (long long)n_items * upi;
     for (long long idx = (long long)xcd_run(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; idx < total; idx += (long long)gridDim.x * blockDim.x) {
         const int item = (int)(idx / upi), u = (int)(idx - (long long)item * upi);
-        const int ns = min(P.nparts ? P.nparts[item] : P.pos[item] / ATT_CH + 1, MAXS);
+        const int ns = min(P.pos_base >= 0 ? (P.pos_base + item) / ATT_CH + 1 : P.nparts ? P.nparts[item] : P.pos[item] / ATT_CH + 1, MAXS);
         const long long pbase = (long long)item * P.heads * P.nsplit_max;
         const int blk = u >> 2, w = u & 3;
         const int h = blk * 32 / hd;                 // a 32-column block never straddles heads (hd = 32 or 64)
@@ -905,8 +906,9 @@ __device__ __forceinline__ float rows4_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int HD, int G, int QT, bool SHADOW>
-__global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16_kernel(AttnParams P, int n_items) {
+// ALONE: a grid of at most a workgroup a compute unit, whose wavefronts may take all the registers there are
+template <int HD, int G, int QT, bool SHADOW, bool ALONE = false>
+__global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 && !ALONE ? 4 : 2) attn_tile16_kernel(AttnParams P, int n_items) {
     constexpr int VH = QT * G;               // rows (token, query head) per workgroup
     static_assert(VH % 16 == 0 && VH <= 256, "16 rows per wavefront");
     constexpr int NTH = VH * 4, NW = NTH / 64;
@@ -920,9 +922,10 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
     __shared__ int npos[VH];                 // keys visible to each row: its position + 1 (0: no such item)
 
     // a workgroup = one query tile x a RUN of consecutive 128-key chunks, folded with the online softmax in registers;
-    // its (max, sum, sum p*v) leaves as partial `slot` of the tile's items.  Prompts come with the host's list of runs
+    // its (max, sum, sum p*v) leaves as partial `slot` of the tile's items.  Prompts whose runs are longer than a chunk come with the host's list of runs
     // (AttnParams::live_map, one entry per blockIdx.x: kv head << 24 | tile << 16 | slot << 12 | first chunk << 6 | chunks);
-    // without it the grid is (kv head, chunk, tile) with one chunk per workgroup.
+    // without it the grid is (kv head, chunk, tile) with one chunk per workgroup, and those above the diagonal leave at once: short prompts' launches are
+    // memory round trips in a row (70 % of a wavefront's life), and reading the list is one more.
     const int tid = threadIdx.x;
     const int code = P.live_map ? sload_i32(P.live_map + blockIdx.x) : 0;
     const int kvh = P.live_map ? (int)((unsigned)code >> 24) : (int)blockIdx.x;
@@ -971,14 +974,25 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
     [[maybe_unused]] auto dma_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
     if constexpr (SHADOW) dma_chunk(c_first, 0);
 
-    // B operand of S^T: row w*16+j, head_dim elements 32*ks + 8*kq .. +7, as hi / lo halves
+    // B operand of S^T: row w*16+j, head_dim elements 32*ks + 8*kq .. +7, as hi / lo halves.  ALONE: they are split once the first chunk
+    // is in LDS, in flight together with its rows: one memory round trip for all three (with two workgroups a compute unit 30 registers would spill).
     half8_t qh[NKS], ql[NKS];
-    {
+    float4 qraw[2 * NKS];
+    int row_pos = 0;
+    auto q_load = [&]() __attribute__((always_inline)) {
         const int vh = w * 16 + j, item = min(i0 + vh / G, n_items - 1), g = vh % G;
         const float *qp = P.qbuf + (long long)item * P.q_item_stride + (kvh * G + g) * HD + 8 * kq;
 #pragma unroll
+        for (int k = 0; k < 2 * NKS; k++) qraw[k] = *reinterpret_cast<const float4 *>(qp + 32 * (k >> 1) + 4 * (k & 1));
+        if (tid < VH) {
+            const int it = i0 + tid / G;
+            row_pos = it < n_items ? (P.pos_base_valid ? P.pos_base + it : P.bpos[it]) + 1 : 0;
+        }
+    };
+    auto q_split = [&]() __attribute__((always_inline)) {
+#pragma unroll
         for (int ks = 0; ks < NKS; ks++) {
-            const float4 a = *reinterpret_cast<const float4 *>(qp + 32 * ks), b = *reinterpret_cast<const float4 *>(qp + 32 * ks + 4);
+            const float4 a = qraw[2 * ks], b = qraw[2 * ks + 1];
             const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -987,10 +1001,11 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
                 qh[ks][e] = h; ql[ks][e] = l;
             }
         }
-    }
-    if (tid < VH) {
-        const int item = i0 + tid / G;
-        npos[tid] = item < n_items ? P.bpos[item] + 1 : 0;
+    };
+    q_load();
+    if constexpr (!ALONE) {
+        q_split();
+        if (tid < VH) npos[tid] = row_pos;
     }
     const long long soff = P.single_stream ? 0 : (long long)sload_i32(P.bstream + i0) * P.kv_stream_stride;
     constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
@@ -1014,6 +1029,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
             const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
             const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
             kv16_stage<HD, NTH, true>(K4, V4, nrows, tid, Kh, Kl, VTh, VTl, c > 0);
+            if (ALONE && c == 0 && tid < VH) npos[tid] = row_pos;
         }
         ATT_STAMP(10 * c + 3);
         __syncthreads();                               // the chunk is in LDS; every wavefront is past the previous chunk
@@ -1023,6 +1039,11 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 ? 4 : 2) attn_tile16
         ATT_STAMP(10 * c + 4);
         if (!SHADOW && i0 + w * 16 / G >= n_items) continue;      // no query in this wavefront: the pipes are the others'
 
+        if constexpr (ALONE) {
+#pragma unroll
+            for (int k = 0; k < 2 * NKS; k++) asm volatile("" : "+v"(qraw[k].x), "+v"(qraw[k].y), "+v"(qraw[k].z), "+v"(qraw[k].w));   // (hipcc would split them in front of the loop)
+            q_split();
+        }
         // ---- S^T = K q^T: 8 key tiles x 16 rows; lane (j, kq) ends up with row j's scores for keys 16*mt + 4*kq + r
         v4f acc[8];
 #pragma unroll

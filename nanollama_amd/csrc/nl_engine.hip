@@ -575,26 +575,27 @@ static const AttnKnobs &attn_knobs() {
 }
 
 template <int HD, int G>
-void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st, bool f32_tile) {
+void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, int num_cus, hipStream_t st, bool f32_tile) {
     constexpr int QT = AttnTileQT<G>::value;
     if (f32_tile) hipLaunchKernelGGL((attn_tile_kernel<HD, G, QT>), dim3(kvs, nsplit, (n + QT - 1) / QT), dim3(QT * G * 4), 0, st, P, n);
     else {
         constexpr int QT16 = AttnTile16QT<G>::value;
         if (P.live_map && P.kv16) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, AttnTile16ShadowQT<G>::value, true>), dim3(nsplit /* = listed workgroups */), dim3(AttnTile16ShadowQT<G>::value * G * 4), 0, st, P, n);
         else if (P.live_map) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false>), dim3(nsplit /* = listed workgroups */), dim3(QT16 * G * 4), 0, st, P, n);
+        else if (kvs * nsplit * ((n + QT16 - 1) / QT16) <= num_cus) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false, true>), dim3(kvs, nsplit, (n + QT16 - 1) / QT16), dim3(QT16 * G * 4), 0, st, P, n);
         else hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false>), dim3(kvs, nsplit, (n + QT16 - 1) / QT16), dim3(QT16 * G * 4), 0, st, P, n);
     }
 }
 inline int attn_tile16_qt(int gqa) { return NL_ATT16_MUL * (gqa == 1 ? 64 : gqa == 2 ? 32 : gqa == 8 ? 8 : 16); }   // = AttnTile16QT<G>::value
 inline bool attn_tile_supported(int gqa) { return gqa == 1 || gqa == 2 || gqa == 3 || gqa == 4 || gqa == 8; }
 template <int HD>
-hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, hipStream_t st, bool f32_tile) {
+hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, int num_cus, hipStream_t st, bool f32_tile) {
     switch (gqa) {
-    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, st, f32_tile); break;
-    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, st, f32_tile); break;
-    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, st, f32_tile); break;
-    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, st, f32_tile); break;
-    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, st, f32_tile); break;
+    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
+    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
+    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
+    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
+    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1275,7 +1276,6 @@ nl_engine::PlanSet &pick_plan(nl_engine *e, int pos_last) { return e->ps[plan_in
 std::mutex g_turn_mu;
 struct ChipTurns { std::vector<nl_engine *> handles; nl_engine *last = nullptr; };
 ChipTurns g_turns[64];
-// (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
 // (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
 template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
     if (!e->turn_on || !waits) return launch();
@@ -2144,7 +2144,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     // Run length: the shortest that lets every workgroup be resident at once (2 per CU); tiles are cut into equal runs.
     // Prompts of several query tiles (n >= NL_KV16_MIN_TOKENS): the chunks are split into fp16 halves once per layer
     // (kv16_build_kernel, or the Q|K|V launch) and a workgroup takes twice the rows, one workgroup per CU (AttnTile16ShadowQT).
-    int n_live = 0, max_nparts = 0;
+    int n_live = 0, max_nparts = 0, run = 0;
     bool kv16_on = false;
     const int exact = kquant_file(e) ? 1 : 0;
     const bool f32_tile = attn_knobs().f32_tile || exact;
@@ -2159,7 +2159,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         if (cons && ntile <= 256 && e->KVs <= 255) {
             auto chunks_of = [&](int z) { return std::min((p0 + std::min((z + 1) * qt, n) - 1) / ATT_CH + 1, e->nsplit_max); };
             const int run_knob = getenv("NL_ATT_RUN") ? atoi(getenv("NL_ATT_RUN")) : 0;   // developer knob: fixed run length (read per step: a test sets it)
-            int run = run_knob > 0 ? run_knob : 1;
+            run = run_knob > 0 ? run_knob : 1;
             for (; run_knob <= 0 && run < e->nsplit_max; run++) {
                 long long wgs = 0;
                 for (int z = 0; z < ntile; z++) wgs += (chunks_of(z) + run - 1) / run;
@@ -2203,6 +2203,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     for (int i = 1; i < n && consecutive; i++) consecutive = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
     nsplit = std::min(nsplit, e->nsplit_max);
     const bool tile_attn = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;   // prompts: attn_tile16_kernel
+    // ... a partial per 128 positions: nothing about them to read in the launches
+    const bool by_chunk = tile_attn && consecutive && (f32_tile || (n_live > 0 && run == 1 && !kv16_on));
     const bool fin_attn = !tile_attn && nsplit == 1 && !no_fin;                                 // one split: attn_kernel<..., FIN>
     const char *rk = getenv("NL_ROPE_IN_ATTN");    // knob (tests, tools; read per step): 0 keeps the brope_kv launch
     const bool rope_attn_knob = !(rk && atoi(rk) == 0);
@@ -2322,10 +2324,13 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 // prefill: the step's tokens share a stream -> K/V split staged once per tile of tokens, fp16 MFMA with hi/lo-split operands (attn_tile16_kernel)
                 AttnParams T = P;
                 T.x1 = x1_attn;
-                T.single_stream = c.max_streams == 1 ? 1 : 0;
+                // (the prompt's stream is known here)
+                const long long so = c.max_streams == 1 ? 0 : (long long)b.h_meta[2 * b.cap] * e->kv_stream_stride;
+                T.kcache = kc + so; T.vcache = vc + so;
+                T.single_stream = 1;
                 T.pos_base_valid = consecutive ? 1 : 0;   // (a prompt: the kernel derives its key range without reading bpos)
                 T.pos_base = b.h_meta[b.cap];
-                T.live_map = n_live > 0 ? b.tok + 3 * b.cap : nullptr;
+                T.live_map = n_live > 0 && !by_chunk ? b.tok + 3 * b.cap : nullptr;
                 // every row's keys in one run: no partials, the launch writes WO's fragments (not the float32 tile)
                 if ((f32_tile ? nsplit == 1 : n_live > 0 && max_nparts == 1 && !kv16_on) && !no_fin) {
                     T.fin_xf = b.xfrag; T.fin_nt16 = nt16; T.fin_form = form(L.wo);
@@ -2334,7 +2339,6 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 }
                 if (n_live > 0 && kv16_on) {
                     // every chunk the prompt can see, split into fp16 halves once for all the tiles that read it
-                    const long long so = T.single_stream ? 0 : (long long)b.h_meta[2 * b.cap] * e->kv_stream_stride;
                     const int n_keys = b.h_meta[b.cap] + n;
                     Kv16BuildParams KB{kc + so, vc + so, b.kv16, c.seq_len, e->nsplit_max, n_keys};
                     const dim3 kg(e->KVs, (n_keys + ATT_CH - 1) / ATT_CH);
@@ -2342,8 +2346,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                     else if (hd != 64) hipLaunchKernelGGL(kv16_build_kernel<32>, kg, dim3(512), 0, st, KB);
                     T.kv16 = b.kv16;
                 }
-                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st, f32_tile)
-                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, n_live > 0 ? n_live : nsplit, st, f32_tile));
+                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, st, f32_tile)
+                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, st, f32_tile));
             } else if (fin_attn) {
                 // every position < 128: one split per row, the attention kernel normalises and writes the fragments
                 P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_form = form(L.wo);
@@ -2362,10 +2366,10 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             }
             if (!merged) {
             const bool tile16 = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;
-            BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, form(L.wo), tile16 && !exact ? 1 : 0};
+            BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, form(L.wo), by_chunk ? b.h_meta[b.cap] : -1, tile16 && !exact ? 1 : 0};
             {
                 const long long units = (long long)n * e->Hs * hd / 8;
-                if (M.nparts && max_nparts <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
+                if (by_chunk ? nsplit <= 4 : M.nparts && max_nparts <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
                 else hipLaunchKernelGGL(battn_merge_kernel<16>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
             }
             }
