@@ -187,6 +187,7 @@ struct nl_engine {
     int *h_box = nullptr, *d_box = nullptr;              // [0, CTL_WORDS): control words, [8]: sequence number of the call
     unsigned long long *h_done = nullptr, *d_done = nullptr;
     unsigned box_seq = 0;
+    int *ctl_prompt = nullptr;   // the control words of a prompt's LM head: no chain, logits to the pinned buffer
     float *d_h_logits = nullptr; // device address of h_logits (the LM head of a per-call Forward stores the logits there itself)
     float *h_logits = nullptr;   // pinned [vocab] + one int behind it: the per-call read-backs of nl_forward / nl_forward_argmax /
                                  // nl_prefill land here by DMA and are copied to the caller's (pageable) buffer by the CPU -- a
@@ -669,27 +670,41 @@ BlockParams attn_block_params(nl_engine *e, int l, const float *x_in) {
     return B;
 }
 
-// final RMSNorm, LM head and argmax of a plan that leaves the finished residual stream in x
+// final RMSNorm + LM head of one row x (go/model.go:616-619), the argmax behind it
+GemvParams head_params(nl_engine *e, const float *x) {
+    GemvParams P = base_params(e, e->lm_head);
+    P.x = x; P.normw = e->output_norm;
+    P.out = e->logits; P.amax_val = e->amax_val; P.amax_idx = e->amax_idx;
+    P.host_out = e->d_h_logits;
+    return P;
+}
+ArgmaxParams head_argmax_params(nl_engine *e, const GemvParams &P, int *ctl) {
+    const int lm_blocks = (P.ntiles + P.tw - 1) / P.tw, lm_spb = (P.tw * TR + 63) / 64;
+    return ArgmaxParams{e->logits, e->cfg.vocab, e->amax_val, e->amax_idx, lm_blocks * lm_spb, ctl, e->ids, e->result};
+}
+// ... of a plan that leaves the finished residual stream in x
 void push_head(nl_engine *e, std::vector<Op> &plan, const float *x) {
-    const nl_config &c = e->cfg;
-    int lm_blocks, lm_spb;
-    {   // final RMSNorm + LM head (go/model.go:616-619)
-        GemvParams P = base_params(e, e->lm_head);
-        P.x = x; P.normw = e->output_norm;
-        P.out = e->logits; P.amax_val = e->amax_val; P.amax_idx = e->amax_idx;
-        P.host_out = e->d_h_logits;
-        lm_blocks = (P.ntiles + P.tw - 1) / P.tw;
-        lm_spb = (P.tw * TR + 63) / 64;
-        push_gemv(plan, K_LMHEAD, 0, e->logits, (size_t)e->Vs, e->lm_head.wtype, PRO_NORM, EPI_STORE, P);
-    }
-    {
-        ArgmaxParams P{e->logits, c.vocab, e->amax_val, e->amax_idx, lm_blocks * lm_spb, e->ctl, e->ids, e->result};
-        e->plan_argmax = P;
-        plan.push_back({K_ARGMAX, 0, nullptr, 0, [P](hipStream_t st) {
-                               hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, P);
-                               return hipGetLastError();
-                           }});
-    }
+    const GemvParams G = head_params(e, x);
+    push_gemv(plan, K_LMHEAD, 0, e->logits, (size_t)e->Vs, e->lm_head.wtype, PRO_NORM, EPI_STORE, G);
+    const ArgmaxParams P = head_argmax_params(e, G, e->ctl);
+    e->plan_argmax = P;
+    plan.push_back({K_ARGMAX, 0, nullptr, 0, [P](hipStream_t st) {
+                           hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, P);
+                           return hipGetLastError();
+                       }});
+}
+// ... of a prompt's last token, whose logits go to the pinned buffer too where the caller wants them.  One row is the single-token plan's work: norm, a product
+// of fragments (in split-K slabs: and their sum) and an argmax over the whole row, then a copy by DMA, were four to five of a prompt's launches.  us from the
+// norm to the argmax: 32000 x 576 Q8_0 18.8 and a copy, now 15.5, 48000 x 1536 Q8_0 43.1 and a copy, now
+// 24.5, Q6_K 75.4 and a copy, now 25.9
+hipError_t launch_prompt_head(nl_engine *e, const float *x, bool to_host, hipStream_t st) {
+    GemvParams G = head_params(e, x);
+    G.ctl = e->ctl_prompt;
+    if (!to_host) G.host_out = nullptr;
+    const hipError_t s = launch_gemv_dyn(e->lm_head.wtype, PRO_NORM, EPI_STORE, G, st);
+    if (s != hipSuccess) return s;
+    hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, head_argmax_params(e, G, e->ctl_prompt));
+    return hipGetLastError();
 }
 
 // Small models at short contexts, both halves of a layer fused (nl_block.h): embed -> { attn_block -> ffn_block } x L ->
@@ -2133,9 +2148,9 @@ hipError_t launch_qgemm_plain(nl_engine *e, nl_engine::Batch &bt, const PackedMa
 }
 
 // One multi-token step: n <= 64 (token, pos, stream) triples through every layer on the MFMA path.
-// lm_mode: 0 = no LM head, 1 = logits + argmax for every token, 2 = logits + argmax for the LAST token only, in e->logits / e->result.
+// lm_mode: 0 = no LM head, 1 = logits + argmax for every token, 2 = logits + argmax for the LAST token only, in e->logits / e->result (to_host: and the pinned buffer).
 // The caller has filled bt.h_meta; stream-ordered, no synchronisation inside.
-int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int lm_mode, bool one_stream = false) {
+int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int lm_mode, bool one_stream = false, bool to_host = false) {
     const nl_config &c = e->cfg;
     const int D = c.dim, hd = e->hd, HQ = e->Hs * hd, R = (e->Hs + 2 * e->KVs) * hd;
 #define LCK(expr) do { hipError_t s_ = (expr); if (s_ != hipSuccess) return e->fail(NL_ERR_HIP, "batched step: %s: %s", #expr, hipGetErrorString(s_)); } while (0)
@@ -2450,9 +2465,13 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         }
     }
     if (lm_mode) {
-        // logits rows [0, cnt) of bt.logits / ids [0, cnt): all tokens (mode 1, n <= lm_cap); or just the last one's (mode 2)
-        const int first = lm_mode == 2 ? n - 1 : 0, cnt = lm_mode == 2 ? 1 : n;
-        if (cnt > b.lm_cap) return e->fail(NL_ERR_INVALID, "LM head batch %d exceeds %d", cnt, b.lm_cap);
+        if (lm_mode == 2) {
+            if (pend.ks > 1) LCK(norm(e->output_norm, e->lm_head, n - 1, 1));        // (adds the last product's slabs to the row)
+            LCK(launch_prompt_head(e, b.x + (size_t)(n - 1) * D, to_host, st));
+            return NL_OK;
+        }
+        // logits rows [0, n) of bt.logits / ids [0, n), n <= lm_cap
+        if (n > b.lm_cap) return e->fail(NL_ERR_INVALID, "LM head batch %d exceeds %d", n, b.lm_cap);
         if (dg_head) {
             // final RMSNorm folded (the last down launch wrote the fragments and sums of squares), logits + one argmax candidate
             // per (token, 16 rows) from the GEMM's epilogue, the candidates merged by a launch that reads 1 / 8 of the logits' bytes
@@ -2463,11 +2482,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(launch_dgemm_head(P, st, e->num_cus));
             hipLaunchKernelGGL(dg_argmax_kernel, dim3(n), dim3(1024), 0, st, reinterpret_cast<const uint2 *>(b.kpart), m.ntiles, b.ids);
         } else {
-            // (the last token's go where single-token steps leave theirs)
-            float *const rows = lm_mode == 2 ? e->logits : b.logits;
-            LCK(norm(e->output_norm, e->lm_head, first, cnt));
-            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, rows, c.vocab, st, exact));
-            hipLaunchKernelGGL(bargmax_kernel, dim3(cnt), dim3(1024), 0, st, rows, c.vocab, lm_mode == 2 ? e->result : b.ids);
+            LCK(norm(e->output_norm, e->lm_head, 0, n));
+            LCK(launch_qgemm_plain(e, b, e->lm_head, n, b.logits, c.vocab, st, exact));
+            hipLaunchKernelGGL(bargmax_kernel, dim3(n), dim3(1024), 0, st, b.logits, c.vocab, b.ids);
         }
         LCK(hipGetLastError());
     }
@@ -3002,7 +3019,8 @@ int nl_finalize(nl_handle e) {
     HIPCK(e, hipMemsetAsync(e->vcache, 0, kvn * 4, e->stream));
     e->hw.assign(c.max_streams, 0);
     e->ids_cap = c.seq_len + 1;
-    HIPCK(e, dalloc(&e->ctl, (size_t)CTL_WORDS, &e->bytes_state));
+    HIPCK(e, dalloc(&e->ctl, (size_t)2 * CTL_WORDS, &e->bytes_state));
+    e->ctl_prompt = e->ctl + CTL_WORDS;
     HIPCK(e, dalloc(&e->ids, (size_t)e->ids_cap, &e->bytes_state));
     HIPCK(e, dalloc(&e->result, (size_t)1, &e->bytes_state));
     e->amax_slots = ((e->Vs + TR - 1) / TR) + 64;  // >= one slot per wave of LM-head rows for any tw
@@ -3025,6 +3043,11 @@ int nl_finalize(nl_handle e) {
     HIPCK(e, hipHostMalloc((void **)&e->h_ctl_ring, (size_t)e->ctl_ring_cap * CTL_WORDS * sizeof(int), hipHostMallocDefault));
     memset(e->h_ctl_ring, 0, (size_t)e->ctl_ring_cap * CTL_WORDS * sizeof(int));       // (the callers fill five of the eight words)
     HIPCK(e, hipMemcpy(e->ctl, e->h_ctl, CTL_WORDS * sizeof(int), hipMemcpyHostToDevice));
+    {
+        int words[CTL_WORDS] = {};
+        words[CTL_HOSTOUT] = 1;
+        HIPCK(e, hipMemcpy(e->ctl_prompt, words, sizeof words, hipMemcpyHostToDevice));
+    }
     if (e->G > 1 && !e->comm && !e->p2p.on && !(c.flags & NL_FLAG_LOCAL_GROUP))
         return e->fail(NL_ERR_STATE, "tp_size %d needs nl_comm_init or nl_p2p_import before nl_finalize", e->G);
     if (e->stage) { hipFree(e->stage); e->stage = nullptr; e->stage_cap = 0; }
@@ -3775,6 +3798,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     if ((rc = note_positions(e, stream, pos0, n))) return rc;
+    bool direct = false;                                     // the LM head has stored the logits into the pinned buffer
     if (n >= batch_min(e) && batch_supported(e)) {
         // multi-token path: 64-token tiles on the matrix cores; causality comes from each token's own pos
         { std::lock_guard<std::mutex> setup(g_setup_mu); if ((rc = batch_alloc(e, e->bt)) || (rc = dgemm_prepare(e))) return rc; }
@@ -3788,8 +3812,9 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
                 b.h_meta[2 * b.cap + i] = stream;
             }
             const bool last = t0 + m == n;
-            if ((rc = batched_step(e, b, e->stream, m, last ? 2 : 0, true))) return rc;      // (2: logits / argmax of the last token, in e->logits / e->result)
+            if ((rc = batched_step(e, b, e->stream, m, last ? 2 : 0, true, last_logits_out != nullptr))) return rc;      // (2: logits / argmax of the last token, in e->logits / e->result)
         }
+        direct = e->d_h_logits != nullptr;
     } else {
         for (int attempt = 0;; attempt++) {
             for (int i = 0; i < n; i++) {
@@ -3803,7 +3828,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
             break;
         }
     }
-    if (last_logits_out)
+    if (last_logits_out && !direct)
         HIPCK(e, hipMemcpyAsync(e->h_logits, e->logits, (size_t)e->cfg.vocab * 4, hipMemcpyDeviceToHost, e->stream));
     HIPCK(e, hipStreamSynchronize(e->stream));
     if (int prc = p2p_check(e)) return prc;
