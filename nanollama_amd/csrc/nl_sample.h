@@ -472,42 +472,76 @@ __device__ __forceinline__ samp_u64 samp_wave_scan_u64(samp_u64 v) {
 // wavefronts (one per SIMD) do the work, eight buckets per lane -- the selection runs on ONE compute unit and is bound by
 // its vector issue slots, so work that a quarter of the wavefronts can do is not spread over all sixteen.  scr: 2 x 8 words
 // of LDS used alternately (par), so that no barrier is needed behind the result read.
+// (in parts: level 1's buckets are requested with the kernel's first loads and scanned once for both selections)
 struct SampSel { int bucket; samp_u64 rem, x, total; };
-template <typename XF>
-__device__ __forceinline__ SampSel samp_select_bucket(const samp_u64 *h, XF x_of, samp_u64 *scr, int &par) {
-    const int tid = threadIdx.x, ln = tid & 63, wv = tid >> 6;
-    samp_u64 *wtot = scr + par * 8, *res = scr + par * 8 + 4;
-    par ^= 1;
-    samp_u64 v[8], inc = 0;
-    if (tid < 256) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(h + 2040 - 8 * tid);      // buckets 2040 - 8 tid .. 2047 - 8 tid
+struct SampScan { samp_u64 v[8], before; };                  // of threads 0 .. 255: eight buckets; the sum of those ahead of them in the wavefront
+__device__ __forceinline__ void samp_scan_load(SampScan &s, const samp_u64 *h) {
+    if (threadIdx.x >= 256) return;
+    const uint4 *src = reinterpret_cast<const uint4 *>(h + 2040 - 8 * threadIdx.x);      // buckets 2040 - 8 tid .. 2047 - 8 tid
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint4 t = src[3 - q];
-            v[2 * q] = ((samp_u64)t.w << 32) | t.z;         // descending: the higher bucket of the pair first
-            v[2 * q + 1] = ((samp_u64)t.y << 32) | t.x;
-        }
-        samp_u64 local = 0;
-#pragma unroll
-        for (int q = 0; q < 8; q++) local += v[q];
-        inc = samp_wave_scan_u64(local);
-        if (ln == 63) wtot[wv] = inc;
-        inc -= local;                                        // exclusive, within the wavefront
+    for (int q = 0; q < 4; q++) {
+        const uint4 t = src[3 - q];
+        s.v[2 * q] = ((samp_u64)t.w << 32) | t.z;            // descending: the higher bucket of the pair first
+        s.v[2 * q + 1] = ((samp_u64)t.y << 32) | t.x;
     }
-    __syncthreads();
+}
+__device__ __forceinline__ void samp_scan_sum(SampScan &s, samp_u64 *wtot) {             // (a barrier, then samp_scan_cross)
+    if (threadIdx.x >= 256) return;
+    samp_u64 local = 0;
+#pragma unroll
+    for (int q = 0; q < 8; q++) local += s.v[q];
+    const samp_u64 inc = samp_wave_scan_u64(local);
+    if ((threadIdx.x & 63) == 63) wtot[threadIdx.x >> 6] = inc;
+    s.before = inc - local;
+}
+template <typename XF>
+__device__ __forceinline__ SampSel samp_scan_cross(const SampScan &s, const samp_u64 *wtot, XF x_of, samp_u64 *res) {
+    const int tid = threadIdx.x, wv = tid >> 6;
     if (tid < 256) {
         const samp_u64 t0 = wtot[0], t1 = wtot[1], t2 = wtot[2], t3 = wtot[3];
         const samp_u64 total = (t0 + t1) + (t2 + t3);
         const samp_u64 x = x_of(total);
-        samp_u64 run = inc + (wv > 0 ? t0 : 0) + (wv > 1 ? t1 : 0) + (wv > 2 ? t2 : 0);
+        samp_u64 run = s.before + (wv > 0 ? t0 : 0) + (wv > 1 ? t1 : 0) + (wv > 2 ? t2 : 0);
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            if (run < x && x <= run + v[q]) { res[0] = (samp_u64)(2047 - 8 * tid - q); res[1] = x - run; res[2] = x; res[3] = total; }
-            run += v[q];
+            if (run < x && x <= run + s.v[q]) { res[0] = (samp_u64)(2047 - 8 * tid - q); res[1] = x - run; res[2] = x; res[3] = total; }
+            run += s.v[q];
         }
     }
     __syncthreads();
     return SampSel{(int)res[0], res[1], res[2], res[3]};
+}
+template <typename XF>
+__device__ __forceinline__ SampSel samp_select_bucket(const samp_u64 *h, XF x_of, samp_u64 *scr, int &par) {
+    samp_u64 *wtot = scr + par * 8, *res = scr + par * 8 + 4;
+    par ^= 1;
+    SampScan s;
+    samp_scan_load(s, h);
+    samp_scan_sum(s, wtot);
+    __syncthreads();
+    return samp_scan_cross(s, wtot, x_of, res);
+}
+
+// the rank-th id, ascending, whose key is kpick, into s_pick: contiguous ids per thread (uncoalesced reads: the rare path)
+__device__ __forceinline__ void samp_tie_pick(const unsigned *kin, int V, unsigned kpick, unsigned rank, unsigned *wcnt, int *s_pick) {
+    const int tid = threadIdx.x, C = (V + SAMP_THREADS - 1) / SAMP_THREADS, lo = tid * C;
+    unsigned cnt = 0;
+    for (int k = 0; k < C; k++) cnt += (lo + k < V && kin[lo + k] == kpick) ? 1u : 0u;
+    unsigned inc = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned o = __shfl_up(inc, d);
+        if ((tid & 63) >= d) inc += o;
+    }
+    if ((tid & 63) == 63) wcnt[tid >> 6] = inc;
+    __syncthreads();
+    unsigned pre = inc - cnt;
+    for (int w = 0; w < (tid >> 6); w++) pre += wcnt[w];
+    if (pre < rank && rank <= pre + cnt) {
+        unsigned seen = pre;
+        for (int k = 0; k < C; k++)
+            if (lo + k < V && kin[lo + k] == kpick) { seen++; if (seen == rank) *s_pick = lo + k; }
+    }
 }
 
 // 1 workgroup: C candidates per thread in registers (1024 * C >= vocab), the cut, the pick, the decode state.
@@ -518,6 +552,9 @@ __device__ __forceinline__ SampSel samp_select_bucket(const samp_u64 *h, XF x_of
 // (Until the histogram moved out, this workgroup also took the range of the keys and built level 1 relative to the smallest
 // candidate -- a flat distribution's keys share three exponents and LDS atomics on one address are served one at a time:
 // 0.6 + 3.8 us of the launch's 20.)
+// Loads: level 1, the decode state and the keys leave together, the keys in whole KiB past the L1 (a thread's C keys in a row cost a request 64 lines); both
+// selections scan the same registers (17.1 -> 14.9 us a launch at 32000 candidates).  Up to 65536 candidates stay in registers: 48000 of them 24.0 us streamed out of
+// L2 in three passes, 19.2 here.
 #ifdef NL_SAMP_STAMPS   // developer build (tools/samp_probe.hip): shader-clock stamps of thread 0
 __device__ unsigned long long g_samp_stamps[32];
 #define SAMP_STAMP(i) do { if (threadIdx.x == 0) g_samp_stamps[i] = wall_clock64(); } while (0)
@@ -529,37 +566,44 @@ template <int C>
 __global__ void __launch_bounds__(SAMP_THREADS) samp_select_radix_kernel(SampleParams P) {
     __shared__ samp_u64 hw[2048];
     __shared__ unsigned list[SAMP_LIST_CAP];
-    __shared__ samp_u64 scr[16];
+    __shared__ samp_u64 scr[16], w1[4];
     __shared__ unsigned wcnt[SAMP_THREADS / 64];
     __shared__ unsigned list_n;
     __shared__ int s_pick;
-    const int tid = threadIdx.x, V = P.vocab, lo = tid * C;
-    const int step = P.ctl[CTL_STEP];
-    const float u = P.uniforms[step];
-    unsigned key[C];                                        // bits of p >= 0: unsigned order = float order
+    const int tid = threadIdx.x, V = P.vocab;
+    unsigned key[C];                                        // bits of p >= 0: unsigned order = float order; key[k]: id 4 (1024 (k / 4) + tid) + k % 4
     const unsigned *kin = reinterpret_cast<const unsigned *>(P.keys_in);
-    SAMP_STAMP(0);
-#pragma unroll
-    for (int k = 0; k < C; k += 4) {                        // (keys_in holds 1024 * C entries; the tail past vocab is masked)
-        const uint4 t4 = *reinterpret_cast<const uint4 *>(kin + lo + k);
-        key[k] = lo + k < V ? t4.x : 0u; key[k + 1] = lo + k + 1 < V ? t4.y : 0u;
-        key[k + 2] = lo + k + 2 < V ? t4.z : 0u; key[k + 3] = lo + k + 3 < V ? t4.w : 0u;
-    }
-    if (tid == 0) s_pick = 0x7fffffff;
-    int par = 0;
-    SAMP_STAMP(1);
     // level 1 comes from samp_prob_hist_kernel (global memory, built by every compute unit); keys relative to SAMP_KEY_MIN
     constexpr unsigned kmin = SAMP_KEY_MIN;
     constexpr int s1 = SAMP_S1, s2 = SAMP_S2;
-    const samp_u64 *const h1 = P.h1g;
+    SampScan l1;
+    SAMP_STAMP(0);
+    const int step = P.ctl[CTL_STEP], pos = P.ctl[CTL_POS], n_recent = *P.recent_n;
+    samp_scan_load(l1, P.h1g);
+    auto id_of = [&](int k) { return 4 * (SAMP_THREADS * (k >> 2) + tid) + (k & 3); };
+#pragma unroll
+    for (int k = 0; k < C; k += 4) {
+        const uint4 t4 = samp_ld_l2(kin, (unsigned)min(id_of(k), (V - 1) & ~3));
+        key[k] = t4.x; key[k + 1] = t4.y; key[k + 2] = t4.z; key[k + 3] = t4.w;
+    }
+    const float u = P.uniforms[step];
+    const int shifted = P.rep_window > 0 && n_recent >= P.rep_window && tid + 1 < n_recent ? P.recent[tid + 1] : 0;      // (rep_window <= 1024)
+#pragma unroll
+    for (int k = 0; k < C; k++) key[k] = id_of(k) < V ? key[k] : 0u;
+    samp_scan_sum(l1, w1);
+    if (tid == 0) s_pick = 0x7fffffff;
+    int par = 0;
+    SAMP_STAMP(1);
     auto weight_of = [](unsigned k) { return samp_weight_of(k); };
+    __syncthreads();
     SAMP_STAMP(2);
     SAMP_STAMP(3);
     [[maybe_unused]] int stamp_base = 4;
     // one weighted selection: up to three levels; returns the relative key of the crossing candidates and what is left of x
     // among them
     auto select = [&](auto x_of, unsigned &dout, samp_u64 &rem, samp_u64 &x) {
-        const SampSel a = samp_select_bucket(h1, x_of, scr, par);
+        const SampSel a = samp_scan_cross(l1, w1, x_of, scr + par * 8 + 4);
+        par ^= 1;
         unsigned prefix = (unsigned)a.bucket;               // = d >> s1 of the crossing candidates
         rem = a.rem;
         x = a.x;
@@ -571,7 +615,9 @@ __global__ void __launch_bounds__(SAMP_THREADS) samp_select_radix_kernel(SampleP
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < C; k++) {
-            const unsigned d = key[k] - kmin;               // (a non-candidate wraps to >= 2^32 - 2^30: its d >> s1 is no bucket)
+            unsigned kk = key[k];
+            asm volatile("" : "+v"(kk));                    // (hipcc would keep all the differences for the second selection: spilled)
+            const unsigned d = kk - kmin;                   // (a non-candidate wraps to >= 2^32 - 2^30: its d >> s1 is no bucket)
             if ((d >> s1) == prefix) {
                 const unsigned at = atomicAdd(&list_n, 1u);
                 if (at < (unsigned)SAMP_LIST_CAP) list[at] = d;
@@ -636,64 +682,41 @@ __global__ void __launch_bounds__(SAMP_THREADS) samp_select_radix_kernel(SampleP
     select([u, cum](samp_u64) { const samp_u64 x = samp_ceil_mul(u, cum); return x < 1 ? (samp_u64)1 : x; }, dp, rem, xr);
     SAMP_STAMP(12);
     const unsigned rank = (unsigned)tie_rank(rem, weight_of(dp + kmin));   // 1-based among the candidates with this p, by id
-    // the rank-th candidate with relative key dp in ascending id (thread chunks are contiguous in id)
+    // the rank-th candidate with relative key dp in ascending id
     const unsigned kpick = dp + kmin;
     if (rank == 1) {
         // (the usual case: the first candidate with this p = the smallest id)
         int first = 0x7fffffff;
 #pragma unroll
-        for (int k = C - 1; k >= 0; k--) first = key[k] == kpick ? lo + k : first;
+        for (int k = C - 1; k >= 0; k--) first = key[k] == kpick ? id_of(k) : first;
         if (first != 0x7fffffff) atomicMin(&s_pick, first);
     } else {
-        unsigned cnt = 0;
-#pragma unroll
-        for (int k = 0; k < C; k++) cnt += key[k] == kpick ? 1u : 0u;
-        unsigned inc = cnt;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned o = __shfl_up(inc, d);
-            if ((tid & 63) >= d) inc += o;
-        }
-        if ((tid & 63) == 63) wcnt[tid >> 6] = inc;
-        __syncthreads();
-        unsigned pre = inc - cnt;
-        for (int w = 0; w < (tid >> 6); w++) pre += wcnt[w];
-        if (pre < rank && rank <= pre + cnt) {
-            unsigned seen = pre;
-#pragma unroll
-            for (int k = 0; k < C; k++) {
-                if (key[k] == kpick) { seen++; if (seen == rank) s_pick = lo + k; }
-            }
-        }
+        samp_tie_pick(kin, V, kpick, rank, wcnt, &s_pick);
     }
     __syncthreads();
     SAMP_STAMP(13);
     const int pick = s_pick == 0x7fffffff ? 0 : s_pick;
     samp_embed_tail(P, pick);
     // recent window: append, drop the oldest when full (go/main.go:197-200)
-    const int n = *P.recent_n;
-    int shifted = 0;
-    if (P.rep_window > 0 && n >= P.rep_window && tid + 1 < n) shifted = P.recent[tid + 1];   // rep_window <= 1024
-    __syncthreads();
     if (P.rep_window > 0) {
-        if (n >= P.rep_window) {
-            if (tid + 1 < n) P.recent[tid] = shifted;
-            if (tid == 0) P.recent[n - 1] = pick;
+        if (n_recent >= P.rep_window) {
+            if (tid + 1 < n_recent) P.recent[tid] = shifted;
+            if (tid == 0) P.recent[n_recent - 1] = pick;
         } else if (tid == 0) {
-            P.recent[n] = pick;
-            *P.recent_n = n + 1;
+            P.recent[n_recent] = pick;
+            *P.recent_n = n_recent + 1;
         }
     }
     if (tid == 0) {
         P.ids[step] = pick;
         P.ctl[CTL_STEP] = step + 1;
         P.ctl[CTL_TOKEN] = pick;
-        P.ctl[CTL_POS] = P.ctl[CTL_POS] + 1;
+        P.ctl[CTL_POS] = pos + 1;
     }
     SAMP_STAMP(14);
 }
 
-// ---- the same selection for vocabularies of 32769 .. 131072 candidates (the 7.9B tier): they do not fit the registers of one
+// ---- the same selection for vocabularies of 65537 .. 131072 candidates (the 7.9B tier): they do not fit the registers of one
 // workgroup, so every pass STREAMS the keys out of L2 -- coalesced 16-byte loads through the L2 only (agent scope: plain loads
 // of an L2-resident array reach 37 GB/s per compute unit, these 60-110, tools/ingest_probe.hip), eight in flight per lane.
 // Passes over the keys: range, level-1 histogram, one list pass per selection, the pick's id -- five instead of a 2 x 12-launch
@@ -784,25 +807,7 @@ __global__ void __launch_bounds__(SAMP_THREADS) samp_select_radix_stream_kernel(
         samp_each_key(kin, V, [&](unsigned key, int i) { if (key == kpick) first = min(first, i); });
         if (first != 0x7fffffff) atomicMin(&s_pick, first);
     } else {
-        // ties: the rank-th candidate with this p in ascending id -- contiguous ids per thread (uncoalesced reads: the rare path)
-        const int C = (V + SAMP_THREADS - 1) / SAMP_THREADS, lo = tid * C;
-        unsigned cnt = 0;
-        for (int k = 0; k < C; k++) cnt += (lo + k < V && kin[lo + k] == kpick) ? 1u : 0u;
-        unsigned inc = cnt;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned o = __shfl_up(inc, d);
-            if ((tid & 63) >= d) inc += o;
-        }
-        if ((tid & 63) == 63) wcnt[tid >> 6] = inc;
-        __syncthreads();
-        unsigned pre = inc - cnt;
-        for (int w = 0; w < (tid >> 6); w++) pre += wcnt[w];
-        if (pre < rank && rank <= pre + cnt) {
-            unsigned seen = pre;
-            for (int k = 0; k < C; k++)
-                if (lo + k < V && kin[lo + k] == kpick) { seen++; if (seen == rank) s_pick = lo + k; }
-        }
+        samp_tie_pick(kin, V, kpick, rank, wcnt, &s_pick);
     }
     __syncthreads();
     const int pick = s_pick == 0x7fffffff ? 0 : s_pick;
@@ -864,13 +869,15 @@ inline hipError_t launch_sample(const SampScratch &s, float *logits, int vocab, 
     P.scal = s.scal; P.pmax = s.pmax; P.nblocks = (vocab + 255) / 256;
     P.h1g = s.h1g; P.nblocks_pen = P.nblocks;
     // Three selections, none with a sort (nl_sample.h): temp <= 0 -> argmax of the penalised logits; top_p < 1 -> sampleTopP by
-    // weighted radix selection (<= 32768 candidates in the registers of the one workgroup, up to 131072 streamed out of L2);
+    // weighted radix selection (<= 65536 candidates in the registers of the one workgroup, up to 131072 streamed out of L2);
     // otherwise sampleTopK by a 2-bit-per-pass selection of the k-th largest logit + a bitonic network over the <= 1024 candidates
     P.radix = p.temperature > 0.f && p.top_p < 1.0f ? 1 : 0;
     hipLaunchKernelGGL(samp_penalty_kernel, dim3(P.nblocks), dim3(256), 0, st, P);
     if (P.radix) {
         hipLaunchKernelGGL(samp_prob_hist_kernel, dim3((vocab + SAMP_THREADS - 1) / SAMP_THREADS), dim3(SAMP_THREADS), 0, st, P);
-        if (samp_chunk(vocab) == 32) hipLaunchKernelGGL(samp_select_radix_kernel<32>, dim3(1), dim3(SAMP_THREADS), 0, st, P);
+        if (vocab <= 32 * SAMP_THREADS) hipLaunchKernelGGL(samp_select_radix_kernel<32>, dim3(1), dim3(SAMP_THREADS), 0, st, P);
+        else if (vocab <= 48 * SAMP_THREADS) hipLaunchKernelGGL(samp_select_radix_kernel<48>, dim3(1), dim3(SAMP_THREADS), 0, st, P);
+        else if (vocab <= 64 * SAMP_THREADS) hipLaunchKernelGGL(samp_select_radix_kernel<64>, dim3(1), dim3(SAMP_THREADS), 0, st, P);
         else hipLaunchKernelGGL(samp_select_radix_stream_kernel, dim3(1), dim3(SAMP_THREADS), 0, st, P);
     } else if (p.temperature > 0.f) {
         if (samp_chunk(vocab) == 32) hipLaunchKernelGGL(samp_topk_kernel<false>, dim3(1), dim3(SAMP_THREADS), 0, st, P);
