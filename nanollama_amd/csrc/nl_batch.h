@@ -764,6 +764,151 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     }
 }
 
+// The same for grids that leave compute units idle: a workgroup takes ONE tile of 16 rows, and its four wavefronts share it -- two key tiles of the scores
+// each, then, by way of LDS, 16 columns of the output.  A wavefront above is a chain of up to 256 products of 32 cycles; here 64, and a quarter of the
+// exponentials.  Every sum is taken in the same order: the same bits.  A prompt's consecutive positions only, its stream's cache as the base.
+// us a launch, tiles and rows: three kv heads of four, 100 tokens 10.6 and 6.7; six, 120 tokens 10.9 and 6.7
+template <int HD, int G>
+__global__ void __launch_bounds__(256, 2) attn_rows_kernel(AttnParams P, int n_items) {
+    constexpr int KS = HD + 4, VS = HD + 4, PS = ATT_CH + 4, DK = HD / 4, NTO = HD / 16, R4 = HD / 4, NTH = 256;
+    __shared__ __attribute__((aligned(16))) float Ks[ATT_CH * KS];
+    __shared__ __attribute__((aligned(16))) float Vs[ATT_CH * VS];
+    __shared__ __attribute__((aligned(16))) float Ps[16 * PS];
+    __shared__ float mred[4][16];
+    const int kvh = blockIdx.x, split = blockIdx.y, r0 = blockIdx.z * 16, tid = threadIdx.x, t0 = split * ATT_CH;
+    const int maxpos = P.pos_base + min((r0 + 15) / G, n_items - 1);
+    if (t0 > maxpos) return;
+    const int nrows = min(ATT_CH, maxpos + 1 - t0), nfill = (nrows + 31) & ~31;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, kq = lane >> 4;
+    const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + ((long long)kvh * P.seq_len + t0) * HD);
+    const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + ((long long)kvh * P.seq_len + t0) * HD);
+    // keys of the split that row r of the tile sees
+    auto sees = [&](int r) __attribute__((always_inline)) { const int item = (r0 + r) / G; return item < n_items ? min(ATT_CH, max(0, P.pos_base + item + 1 - t0)) : 0; };
+    float qa[DK];
+    {
+        const int item = min((r0 + j) / G, n_items - 1), g = (r0 + j) % G;
+        const float4 *q4 = reinterpret_cast<const float4 *>(P.qbuf + (long long)item * P.q_item_stride + (kvh * G + g) * HD + DK * kq);
+#pragma unroll
+        for (int s = 0; s < DK / 4; s++) {
+            const float4 t = q4[s];
+            qa[4 * s] = t.x; qa[4 * s + 1] = t.y; qa[4 * s + 2] = t.z; qa[4 * s + 3] = t.w;
+        }
+    }
+    constexpr int NIT = ATT_CH * R4 / NTH;
+    float4 kreg[NIT], vreg[NIT];
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+        const int i = tid + it * NTH;
+        kreg[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+        vreg[it] = kreg[it];
+        if (i / R4 < nrows) { kreg[it] = K4[i]; vreg[it] = V4[i]; }
+    }
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+        const int i = tid + it * NTH, row = i / R4, c4 = i % R4;
+        if (row < nfill) {
+            *reinterpret_cast<float4 *>(Ks + row * KS + c4 * 4) = kreg[it];
+            *reinterpret_cast<float4 *>(Vs + row * VS + c4 * 4) = vreg[it];
+        }
+    }
+    __syncthreads();
+    // ---- scores of key tiles 2w and 2w + 1, as above ----
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    const int nvj = sees(j);
+    const bool mine = w * 32 < nfill;
+    v4f acc[2] = {zero, zero};
+    float m = -INFINITY;
+    if (mine) {
+#pragma unroll
+        for (int s4 = 0; s4 < DK / 4; s4++) {
+            float4 kb[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) kb[mt] = *reinterpret_cast<const float4 *>(Ks + ((2 * w + mt) * 16 + j) * KS + DK * kq + 4 * s4);
+            v4f part[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].x, qa[4 * s4], zero, 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].y, qa[4 * s4 + 1], part[mt], 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) part[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].z, qa[4 * s4 + 2], part[mt], 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) acc[mt] += __builtin_amdgcn_mfma_f32_16x16x4f32(kb[mt].w, qa[4 * s4 + 3], part[mt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float sv = (2 * w + mt) * 16 + 4 * kq + r < nvj ? acc[mt][r] * P.scale : -INFINITY;
+                acc[mt][r] = sv;
+                m = fmaxf(m, sv);
+            }
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+    }
+    if (kq == 0) mred[w][j] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(mred[0][j], mred[1][j]), fmaxf(mred[2][j], mred[3][j]));
+    if (mine) {
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+            float pv[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) pv[r] = (2 * w + mt) * 16 + 4 * kq + r < nvj ? expf(acc[mt][r] - m) : 0.f;
+            *reinterpret_cast<float4 *>(Ps + j * PS + (2 * w + mt) * 16 + 4 * kq) = make_float4(pv[0], pv[1], pv[2], pv[3]);
+        }
+    }
+    __syncthreads();
+    // ---- the rows' sums, and columns 16 w .. 16 w + 15 of P V ----
+    float l = 0.f;
+    v4f o = zero;
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        if (s * 16 >= nfill) continue;
+        const float4 p4 = *reinterpret_cast<const float4 *>(Ps + j * PS + 16 * s + 4 * kq);
+        const float p[4] = {p4.x, p4.y, p4.z, p4.w};
+        v4f part = zero;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            l += p[i];
+            part = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], Vs[(16 * s + 4 * kq + i) * VS + 16 * (w % NTO) + j], part, 0, 0, 0);
+        }
+        o += part;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (P.fin_xf) {
+        constexpr int OS = HD + 4;                                       // (where K was: every wavefront is past the scores)
+        const float il = 1.0f / l;
+        if (w < NTO)
+#pragma unroll
+            for (int r = 0; r < 4; r++) Ks[(4 * kq + r) * OS + 16 * w + j] = o[r] * __shfl(il, 4 * kq + r);
+        __syncthreads();
+        if (tid < 16 * HD / 8) {
+            const int row = tid & 15, e = tid >> 4, item = (r0 + row) / G, g = (r0 + row) % G;
+            if (item < n_items) {
+                const float *src = Ks + row * OS + (e >> 2) * 32;
+                int offa, offb;
+                slot_offsets(P.fin_form, e & 3, offa, offb);
+                float v[8];
+                slots_from(P.fin_form, *reinterpret_cast<const float4 *>(src + offa), *reinterpret_cast<const float4 *>(src + offb), v);
+                store_frag(P.fin_xf, P.fin_nt16, item, ((kvh * G + g) * HD) / 32 + (e >> 2), e & 3, v, P.fin_form);
+            }
+        }
+        return;
+    }
+    auto slot = [&](int r) __attribute__((always_inline)) {
+        return (long long)((r0 + r) / G) * P.part_item_stride + (long long)(kvh * G + (r0 + r) % G) * P.nsplit_max + split;
+    };
+    if (w < NTO)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (sees(4 * kq + r) > 0) P.part_o[slot(4 * kq + r) * HD + 16 * w + j] = o[r];
+    if (w == 0 && kq == 0 && nvj > 0) {
+        P.part_ml[slot(j) * 2] = m;
+        P.part_ml[slot(j) * 2 + 1] = l;
+    }
+}
+
 // ---- the same tile on the fp16 matrix cores -------------------------------------------------------------
 // v_mfma_f32_16x16x4_f32 runs at the f32 VECTOR rate (1/16 of the fp16 MFMA rate); the f32 kernel above spends
 // 256 of them (8192 SIMD cycles) per wavefront.  Here every f32 operand is split x = hi + lo into two fp16 values

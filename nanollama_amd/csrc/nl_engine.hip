@@ -138,7 +138,7 @@ struct Op {
 // nl_engine::step_path: which kernels a layer of a multi-token step ran on (none of the first two: qgemm_kernel / pgemm_kernel, by matrix)
 enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */,
        PATH_IMAGES = 16 /* the projections of a prompt wrote the attention's K and V^T images */, PATH_FOLD = 32 /* norms folded around the GEMMs */,
-       PATH_ATTN_WIDE = 64 /* decode attention with eight wavefronts a workgroup */ };
+       PATH_ATTN_WIDE = 64 /* decode attention with eight wavefronts a workgroup */, PATH_ATTN_ROWS = 128 /* attn_rows_kernel */ };
 
 struct nl_engine {
     nl_config cfg{};
@@ -576,13 +576,16 @@ static const AttnKnobs &attn_knobs() {
 }
 
 template <int HD, int G>
-void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, int num_cus, hipStream_t st, bool f32_tile) {
+void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, int num_cus, bool rows, hipStream_t st, bool f32_tile) {
     constexpr int QT = AttnTileQT<G>::value;
-    if (f32_tile) hipLaunchKernelGGL((attn_tile_kernel<HD, G, QT>), dim3(kvs, nsplit, (n + QT - 1) / QT), dim3(QT * G * 4), 0, st, P, n);
+    if (f32_tile && rows) hipLaunchKernelGGL((attn_rows_kernel<HD, G>), dim3(kvs, nsplit, (n * G + 15) / 16), dim3(256), 0, st, P, n);
+    else if (f32_tile) hipLaunchKernelGGL((attn_tile_kernel<HD, G, QT>), dim3(kvs, nsplit, (n + QT - 1) / QT), dim3(QT * G * 4), 0, st, P, n);
     else {
         constexpr int QT16 = AttnTile16QT<G>::value;
         if (P.live_map && P.kv16) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, AttnTile16ShadowQT<G>::value, true>), dim3(nsplit /* = listed workgroups */), dim3(AttnTile16ShadowQT<G>::value * G * 4), 0, st, P, n);
         else if (P.live_map) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false>), dim3(nsplit /* = listed workgroups */), dim3(QT16 * G * 4), 0, st, P, n);
+        // (a workgroup a compute unit: registers for everything in flight.  us a launch: 40 tokens behind 300, three kv heads of four 10.2 and 7.9; nine heads, 24 tokens
+        //  6.5 and 5.5, 200 tokens 10.4 and 8.3)
         else if (kvs * nsplit * ((n + QT16 - 1) / QT16) <= num_cus) hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false, true>), dim3(kvs, nsplit, (n + QT16 - 1) / QT16), dim3(QT16 * G * 4), 0, st, P, n);
         else hipLaunchKernelGGL((attn_tile16_kernel<HD, G, QT16, false>), dim3(kvs, nsplit, (n + QT16 - 1) / QT16), dim3(QT16 * G * 4), 0, st, P, n);
     }
@@ -590,13 +593,13 @@ void launch_attn_tile_g(const AttnParams &P, int n, int kvs, int nsplit, int num
 inline int attn_tile16_qt(int gqa) { return NL_ATT16_MUL * (gqa == 1 ? 64 : gqa == 2 ? 32 : gqa == 8 ? 8 : 16); }   // = AttnTile16QT<G>::value
 inline bool attn_tile_supported(int gqa) { return gqa == 1 || gqa == 2 || gqa == 3 || gqa == 4 || gqa == 8; }
 template <int HD>
-hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, int num_cus, hipStream_t st, bool f32_tile) {
+hipError_t launch_attn_tile_hd(int gqa, const AttnParams &P, int n, int kvs, int nsplit, int num_cus, bool rows, hipStream_t st, bool f32_tile) {
     switch (gqa) {
-    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
-    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
-    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
-    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
-    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, num_cus, st, f32_tile); break;
+    case 1: launch_attn_tile_g<HD, 1>(P, n, kvs, nsplit, num_cus, rows, st, f32_tile); break;
+    case 2: launch_attn_tile_g<HD, 2>(P, n, kvs, nsplit, num_cus, rows, st, f32_tile); break;
+    case 3: launch_attn_tile_g<HD, 3>(P, n, kvs, nsplit, num_cus, rows, st, f32_tile); break;
+    case 4: launch_attn_tile_g<HD, 4>(P, n, kvs, nsplit, num_cus, rows, st, f32_tile); break;
+    case 8: launch_attn_tile_g<HD, 8>(P, n, kvs, nsplit, num_cus, rows, st, f32_tile); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -2220,6 +2223,15 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const bool tile_attn = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;   // prompts: attn_tile16_kernel
     // ... a partial per 128 positions: nothing about them to read in the launches
     const bool by_chunk = tile_attn && consecutive && (f32_tile || (n_live > 0 && run == 1 && !kv16_on));
+    // attn_rows_kernel: while its workgroups, one per 16 rows and chunk that they see, find two to a compute unit at once.  us a prompt of K-quants, tiles and rows:
+    // 173M, 100 tokens 1091 and 1003 (42 workgroups a kv head), 330 1454 and 1386 (459 in all), 128 behind 300 1169 and 1124 (320), 200 behind 300 1278 and 1295
+    // (525); 841M, 100 tokens 2258 and 2122, 200 2997 and 2931 (408); 4096 columns, 128 tokens 1205 and 1216 (512).  NL_ATTN_ROWS=0 (knob of tests, read per step): never
+    bool rows = by_chunk && f32_tile && !(getenv("NL_ATTN_ROWS") && atoi(getenv("NL_ATTN_ROWS")) == 0);
+    if (rows) {
+        long long wgs = 0;
+        for (int r = 0; r < n * e->gqa; r += 16) wgs += (b.h_meta[b.cap] + std::min((r + 15) / e->gqa, n - 1)) / ATT_CH + 1;
+        rows = wgs * e->KVs < 2 * e->num_cus;
+    }
     const bool fin_attn = !tile_attn && nsplit == 1 && !no_fin;                                 // one split: attn_kernel<..., FIN>
     const char *rk = getenv("NL_ROPE_IN_ATTN");    // knob (tests, tools; read per step): 0 keeps the brope_kv launch
     const bool rope_attn_knob = !(rk && atoi(rk) == 0);
@@ -2346,6 +2358,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 T.pos_base_valid = consecutive ? 1 : 0;   // (a prompt: the kernel derives its key range without reading bpos)
                 T.pos_base = b.h_meta[b.cap];
                 T.live_map = n_live > 0 && !by_chunk ? b.tok + 3 * b.cap : nullptr;
+                if (rows) e->step_path |= PATH_ATTN_ROWS;
                 // every row's keys in one run: no partials, the launch writes WO's fragments (not the float32 tile)
                 if ((f32_tile ? nsplit == 1 : n_live > 0 && max_nparts == 1 && !kv16_on) && !no_fin) {
                     T.fin_xf = b.xfrag; T.fin_nt16 = nt16; T.fin_form = form(L.wo);
@@ -2361,8 +2374,8 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                     else if (hd != 64) hipLaunchKernelGGL(kv16_build_kernel<32>, kg, dim3(512), 0, st, KB);
                     T.kv16 = b.kv16;
                 }
-                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, st, f32_tile)
-                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, st, f32_tile));
+                LCK(hd == 64 ? launch_attn_tile_hd<64>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, rows, st, f32_tile)
+                             : launch_attn_tile_hd<32>(e->gqa, T, n, e->KVs, T.live_map ? n_live : nsplit, e->num_cus, rows, st, f32_tile));
             } else if (fin_attn) {
                 // every position < 128: one split per row, the attention kernel normalises and writes the fragments
                 P.fin_xf = b.xfrag; P.fin_nt16 = nt16; P.fin_form = form(L.wo);
@@ -3268,7 +3281,7 @@ int nl_finalize(nl_handle e) {
             const nl_engine::Layer &L0 = e->layers[0];
             std::vector<LayersEntry> tab;
             for (const auto &L : e->layers)
-                tab.push_back(LayersEntry{{L.qkv.q, L.wo.q, L.gate.q, L.up.q, L.down.q}, {L.qkv.s, L.wo.s, L.gate.s, L.up.s, L.down.s}, L.attn_norm, L.ffn_norm, L.bq, L.bk, L.bv, L.bo});
+                tab.push_back(LayersEntry{{L.qkv.q, L.wo.q, L.gate.q, L.up.q, L.down.q}, {L.qkv.s, L.wo.s, L.gate.s, L.up.s, L.down.s}, {L.attn_norm, L.ffn_norm}, L.bq, L.bk, L.bv, L.bo});
             HIPCK(e, dalloc(&e->ly.tab, tab.size(), &e->bytes_state));
             HIPCK(e, hipMemcpy(e->ly.tab, tab.data(), tab.size() * sizeof(LayersEntry), hipMemcpyHostToDevice));
             const size_t n = (size_t)L0.qkv.ntiles * GPT + (size_t)e->Hs * (layers_records(c.seq_len) + 1) * LY_REC +
