@@ -2397,7 +2397,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             BMergeParams M{b.part_o, b.part_ml, b.pos, tile16 && n_live > 0 ? b.tok + 4 * b.cap : nullptr, e->Hs, e->nsplit_max, hd, b.xfrag, nt16, form(L.wo), by_chunk ? b.h_meta[b.cap] : -1, tile16 && !exact ? 1 : 0};
             {
                 const long long units = (long long)n * e->Hs * hd / 8;
-                if (by_chunk ? nsplit <= 4 : M.nparts && max_nparts <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
+                const int most = by_chunk ? nsplit : M.nparts ? max_nparts : 16;      // (five to eight partials, 33 tokens of 1536 columns: 6.3 us of loads for sixteen, 5.0)
+                if (most <= 4) hipLaunchKernelGGL(battn_merge_kernel<4>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
+                else if (most <= 8) hipLaunchKernelGGL(battn_merge_kernel<8>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
                 else hipLaunchKernelGGL(battn_merge_kernel<16>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, M, n);
             }
             }
