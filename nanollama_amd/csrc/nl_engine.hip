@@ -698,8 +698,8 @@ void push_head(nl_engine *e, std::vector<Op> &plan, const float *x) {
 }
 // ... of a prompt's last token, whose logits go to the pinned buffer too where the caller wants them.  One row is the single-token plan's work: norm, a product
 // of fragments (in split-K slabs: and their sum) and an argmax over the whole row, then a copy by DMA, were four to five of a prompt's launches.  us from the
-// norm to the argmax: 32000 x 576 Q8_0 18.8 and a copy, now 15.5, 48000 x 1536 Q8_0 43.1 and a copy, now
-// 24.5, Q6_K 75.4 and a copy, now 25.9
+// norm to the argmax: 32000 x 576 Q8_0 18.8 and a copy, now 15.5, 48000 x 1536 43.1 and a copy, now 24.5.  (K-quant files keep
+// theirs: batched_step)
 hipError_t launch_prompt_head(nl_engine *e, const float *x, bool to_host, hipStream_t st) {
     GemvParams G = head_params(e, x);
     G.ctl = e->ctl_prompt;
@@ -2480,13 +2480,15 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         }
     }
     if (lm_mode) {
-        if (lm_mode == 2) {
+        if (lm_mode == 2 && !exact) {
             if (pend.ks > 1) LCK(norm(e->output_norm, e->lm_head, n - 1, 1));        // (adds the last product's slabs to the row)
             LCK(launch_prompt_head(e, b.x + (size_t)(n - 1) * D, to_host, st));
             return NL_OK;
         }
-        // logits rows [0, n) of bt.logits / ids [0, n), n <= lm_cap
-        if (n > b.lm_cap) return e->fail(NL_ERR_INVALID, "LM head batch %d exceeds %d", n, b.lm_cap);
+        // logits rows [0, cnt) of bt.logits / ids [0, cnt): all tokens (mode 1, n <= lm_cap); or the last one's, where single-token steps leave theirs (mode 2 of K-quant
+        // files, whose products here carry their rounding on: 1.2e-7 of a page's logits from 64 bits, 1.3e-7 by the single-token head)
+        const int first = lm_mode == 2 ? n - 1 : 0, cnt = lm_mode == 2 ? 1 : n;
+        if (cnt > b.lm_cap) return e->fail(NL_ERR_INVALID, "LM head batch %d exceeds %d", cnt, b.lm_cap);
         if (dg_head) {
             // final RMSNorm folded (the last down launch wrote the fragments and sums of squares), logits + one argmax candidate
             // per (token, 16 rows) from the GEMM's epilogue, the candidates merged by a launch that reads 1 / 8 of the logits' bytes
@@ -2497,9 +2499,10 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(launch_dgemm_head(P, st, e->num_cus));
             hipLaunchKernelGGL(dg_argmax_kernel, dim3(n), dim3(1024), 0, st, reinterpret_cast<const uint2 *>(b.kpart), m.ntiles, b.ids);
         } else {
-            LCK(norm(e->output_norm, e->lm_head, 0, n));
-            LCK(launch_qgemm_plain(e, b, e->lm_head, n, b.logits, c.vocab, st, exact));
-            hipLaunchKernelGGL(bargmax_kernel, dim3(n), dim3(1024), 0, st, b.logits, c.vocab, b.ids);
+            float *const rows_out = lm_mode == 2 ? e->logits : b.logits;
+            LCK(norm(e->output_norm, e->lm_head, first, cnt));
+            LCK(launch_qgemm_plain(e, b, e->lm_head, cnt, rows_out, c.vocab, st, exact));
+            hipLaunchKernelGGL(bargmax_kernel, dim3(cnt), dim3(1024), 0, st, rows_out, c.vocab, lm_mode == 2 ? e->result : b.ids);
         }
         LCK(hipGetLastError());
     }
@@ -3829,7 +3832,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
             const bool last = t0 + m == n;
             if ((rc = batched_step(e, b, e->stream, m, last ? 2 : 0, true, last_logits_out != nullptr))) return rc;      // (2: logits / argmax of the last token, in e->logits / e->result)
         }
-        direct = e->d_h_logits != nullptr;
+        direct = e->d_h_logits != nullptr && !kquant_file(e);
     } else {
         for (int attempt = 0;; attempt++) {
             for (int i = 0; i < n; i++) {

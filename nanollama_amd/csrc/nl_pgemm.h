@@ -737,8 +737,13 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     if (rb * ((P.n_tokens + 31) / 32) <= 256) return go(four, one, two, two);
     if (tiles <= 256) return go(four, one, two, one);
     // (three parts, the sums of a chunk pair and what their additions drop leave no registers for a second token tile: 46 to 150 spilled)
-    if constexpr (PREC == PG_EXACT) return go(four, one, one, one);
-    else {
+    if constexpr (PREC == PG_EXACT) {
+        // (one token, the LM head of a prompt: 16 of them are multiplied, not 64.  Q6_K, us, 48000 x 1536 57.8 and 34.9, 32000 x 768 22.4 and
+        //  12.8)
+        if constexpr (EPI == QG_EPI_PLAIN)
+            if (P.n_tokens <= 16) return go(four, one, one, four);
+        return go(four, one, one, one);
+    } else {
         if (tiles <= 512) return go(four, two, two, one);
         if (tiles < 1024 && !(WT == WT_F16 && EPI == QG_EPI_SWIGLU)) return go(four, one, one, one);
         if constexpr (WT == WT_Q4_0 || WT == WT_F16)
