@@ -138,7 +138,8 @@ struct Op {
 // nl_engine::step_path: which kernels a layer of a multi-token step ran on (none of the first two: qgemm_kernel / pgemm_kernel, by matrix)
 enum { PATH_DGEMM = 1, PATH_SGEMM = 2, PATH_TILE_FIN = 4 /* attention of a prompt wrote WO's fragments */, PATH_ATTN_FIN = 8 /* ... of a decode batch */,
        PATH_IMAGES = 16 /* the projections of a prompt wrote the attention's K and V^T images */, PATH_FOLD = 32 /* norms folded around the GEMMs */,
-       PATH_ATTN_WIDE = 64 /* decode attention with eight wavefronts a workgroup */, PATH_ATTN_ROWS = 128 /* attn_rows_kernel */ };
+       PATH_ATTN_WIDE = 64 /* decode attention with eight wavefronts a workgroup */, PATH_ATTN_ROWS = 128 /* attn_rows_kernel */,
+       PATH_SLIM = 256 /* pgemm_kernel's slim tiles */ };
 
 struct nl_engine {
     nl_config cfg{};
@@ -2010,7 +2011,7 @@ int batch_alloc(nl_engine *e, nl_engine::Batch &b, int cap_limit = 2048) {
         HIPCK(e, dalloc(&raw, nx2 * 4, &e->bytes_state));
         b.xfrag2 = reinterpret_cast<uint4 *>(raw);
     }
-    HIPCK(e, dalloc(&b.ssq, n * (size_t)((c.dim + 31) / 32), &e->bytes_state));   // (one partial per 64 rows on pgemm_kernel, per 32 on dgemm_kernel)
+    HIPCK(e, dalloc(&b.ssq, n * (size_t)((c.dim + 15) / 16), &e->bytes_state));   // (one partial per 64 rows on pgemm_kernel, 16 on its slim tiles, 32 on dgemm_kernel)
     HIPCK(e, dalloc(&b.nscale, 2 * n, &e->bytes_state));
     b.kpart_cap = (size_t)16 * QG_TOK * std::max<size_t>(std::max<size_t>(R, c.dim), e->Is);
     HIPCK(e, dalloc(&b.kpart, b.kpart_cap, &e->bytes_state));
@@ -2124,13 +2125,27 @@ bool sgemm_step_ok(const nl_engine *e, const nl_engine::Batch &b, int n, bool pr
     return true;
 }
 
+// pgemm_kernel's slim tiles (nl_pgemm.h): prompts of up to 64 tokens where every layer is Q6_K and the 64-row tiles of its matrices are at most one a
+// compute unit
+bool pg_slim_step(const nl_engine *e, int n) {
+    const char *k = getenv("NL_PG_SLIM");               // knob (tests; read per step): 0 keeps the 64-row tiles
+    if ((k && atoi(k) == 0) || n > 64) return false;
+    for (const auto &L : e->layers) {
+        for (const PackedMat *m : {&L.qkv, &L.wo, &L.gate, &L.up, &L.down})
+            if (m->wtype != WT_Q6_K || m->ntiles * TR != m->rows || (m->ntiles + 3) / 4 > 256) return false;
+        if ((2 * L.gate.ntiles + 3) / 4 > 256) return false;
+    }
+    return true;
+}
+
 // GEMM of the multi-token step: input = the fragment store the producing kernel just filled; output = `out`
 // (with resid / bias applied) when it ran unsplit, else split-K slabs in `part` for the consumer to add.
 hipError_t qg(nl_engine *e, nl_engine::Batch &bt, const PackedMat &m, int n, float *out, int ldo, const float *resid, hipStream_t st,
               GemmOut *res, float *part, const float *bias = nullptr, const uint4 *xf = nullptr,
-              const QGemmParams::NormOut *nout = nullptr, int x1 = 0, int out_q4 = 1, int exact = 0) {
+              const QGemmParams::NormOut *nout = nullptr, int x1 = 0, int out_q4 = 1, int exact = 0, bool slim = false) {
     QGemmParams P{};
     P.bias = bias;
+    P.slim = slim ? 1 : 0;
     P.x1 = x1;
     P.exact = exact;
     if (nout) { P.nrm_out = *nout; P.out_q4 = out_q4; }
@@ -2267,8 +2282,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         P.xf = in; P.out = b.x; P.bias = bias;
         return sg_launch<QG_EPI_PLAIN>(m.wtype, P, st);
     };
-    e->step_path = (dg ? PATH_DGEMM : sg ? PATH_SGEMM : 0) | (fold ? PATH_FOLD : 0);
-    const int nrb = dg ? D / 32 : D / 64;      // partial sums of squares per token
+    const bool slim = exact && fold && pg_slim_step(e, n);
+    e->step_path = (dg ? PATH_DGEMM : sg ? PATH_SGEMM : 0) | (fold ? PATH_FOLD : 0) | (slim ? PATH_SLIM : 0);
+    const int nrb = dg ? D / 32 : slim ? D / 16 : D / 64;      // partial sums of squares per token
     // NL_PREFILL_PRECISION=fp16x1 (read per step: tests and bench.py flip it): the long-prompt GEMMs of Q4_0 files (pgemm_kernel) and the
     // prompt attention multiply only the fp16 hi half of every activation / probability -- half / a third of the matrix work,
     // activations rounded to 11 bits.  The default x = hi + lo keeps float32-grade results (logit tolerance 1e-4).
@@ -2312,7 +2328,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             const PackedMat &m = L.qkv;
             P.q = dg ? m.q3 : m.q; P.s = dg ? m.s3 : m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
             P.xf = folded_in ? b.xfrag2 : b.xfrag; P.nrm_in = folded_in ? nin_attn : nin_off;
-            P.n_tokens = n; P.ldo = (int)R; P.x1 = x1_gemm; P.exact = exact;
+            P.n_tokens = n; P.ldo = (int)R; P.x1 = x1_gemm; P.exact = exact; P.slim = slim ? 1 : 0;
             P.rope = QGemmParams::Rope{b.pos, b.stream, e->rope_cos, e->rope_sin, b.q, kc, vc, e->kv_stream_stride,
                                        L.bq, L.bk, L.bv, hd, e->Hs, e->KVs, c.seq_len, c.rope_conjugate, b.tcos, b.tsin, b.tkv};
             // (a prompt from position 0, whose token tiles are the images' chunks or halves of them)
@@ -2421,7 +2437,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             LCK(dg_plain(L.wo, b.xfrag, L.bo, &nout));
         } else if (fold) {
             const QGemmParams::NormOut nout{L.ffn_norm, b.xfrag2, b.ssq, sB};
-            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm, L.gate.wtype == WT_Q4_0 ? 1 : 0, exact));
+            LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, &nout, x1_gemm, L.gate.wtype == WT_Q4_0 ? 1 : 0, exact, slim));
         } else {
             LCK(qg(e, b, L.wo, n, b.x, D, b.x, st, &pend, b.kpart, L.bo, nullptr, nullptr, x1_gemm, 1, exact));
             LCK(norm(L.ffn_norm, L.gate, 0, n));
@@ -2443,7 +2459,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
             const PackedMat &m = L.gate;
             P.q = dg ? m.q3 : m.q; P.s = dg ? m.s3 : m.s; P.rows = m.rows; P.cols = m.cols; P.npairs = m.npairs; P.ntiles = m.ntiles;
             P.xf = fold ? b.xfrag2 : b.xfrag; P.nrm_in = fold ? nin_ffn : nin_off;
-            P.n_tokens = n; P.ldo = e->Is; P.x1 = x1_gemm; P.exact = exact;
+            P.n_tokens = n; P.ldo = e->Is; P.x1 = x1_gemm; P.exact = exact; P.slim = slim ? 1 : 0;
             P.q1 = dg ? L.up.q3 : L.up.q; P.s1 = dg ? L.up.s3 : L.up.s;
             P.xf_out = fold ? b.xfrag : b.xfrag2; P.out_q4 = L.down.wtype == WT_Q4_0 ? 1 : 0;
             LCK(dg ? launch_dgemm_swiglu(P, st) : launch_qgemm_swiglu(m.wtype, P, st));
@@ -2474,9 +2490,9 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
         } else if (fold && l + 1 < c.n_layers) {
             const nl_engine::Layer &Ln = e->layers[l + 1];
             const QGemmParams::NormOut nout{Ln.attn_norm, b.xfrag2, b.ssq, sA};
-            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm, Ln.qkv.wtype == WT_Q4_0 ? 1 : 0, exact));
+            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, &nout, x1_gemm, Ln.qkv.wtype == WT_Q4_0 ? 1 : 0, exact, slim));
         } else {
-            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, nullptr, x1_gemm, 1, exact));
+            LCK(qg(e, b, L.down, n, b.x, D, b.x, st, &pend, b.kpart, nullptr, down_in, nullptr, x1_gemm, 1, exact, slim));
         }
     }
     if (lm_mode) {

@@ -189,10 +189,13 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
     using F = typename std::conditional_t<EXACT, PgExact<WT>, PgFmt<WT>>;
     static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");
+    static_assert(RT >= 4 || (EXACT && NTW == 1 && WR <= RT && KW == 2 && RT == (EPI == QG_EPI_SWIGLU ? 2 : 1)), "slim tiles");
     constexpr int NP = X1 ? 1 : EXACT ? 3 : 2, PS = EXACT ? 3 : 2;      // parts of an activation that are read, and that are stored
     constexpr int KB = 4;                                   // blocks per chunk
     constexpr int RTW = RT / WR, TTW = 4 * NTW / WR;        // row tiles of a wavefront, token tiles of a workgroup
-    constexpr int ROWS = RT * TR, TOK = TTW * 16, IPT = ROWS * KB / 256, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
+    // tiles of one or two row tiles (pg_slim): four or two wavefronts share a block's expansion, one or two of its four parts each
+    constexpr int SPL = RT >= 4 ? 1 : 4 / RT, NPT = 4 / SPL;
+    constexpr int ROWS = RT * TR, TOK = TTW * 16, IPT = RT >= 4 ? ROWS * KB / 256 : 1, LD = ROWS + 4, SWN = F::SW ? F::SW : 1;
     constexpr int SC = X1 ? PG_NONE : F::SC;
     constexpr bool MINS = WT == WT_Q4_K, PAIRS = EXACT || WT == WT_Q4_0;
     // The bounded tile whose epilogue spills makes the scales' offset of the weights' (52 bytes of scratch otherwise: 2112 columns, 1000 tokens, all of its
@@ -226,7 +229,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     // nothing to gain (Q|K|V 17.3 and 17.6, 11.8 and 11.9).
     // A last group of one or two pairs is one chunk of both their blocks.
     // staging items: block kk of the chunk, row r, row tile
-    const int i_kk = PAIRS ? 2 * (tid & 1) + ((tid >> 5) & 1) : tid & 3, i_r = (PAIRS ? tid >> 1 : tid >> 2) & 15, i_t = wave;
+    const int i_kk = PAIRS ? 2 * (tid & 1) + ((tid >> 5) & 1) : tid & 3, i_r = (PAIRS ? tid >> 1 : tid >> 2) & 15, i_t = SPL == 1 ? wave : wave % RT, i_w = SPL == 1 ? 0 : wave / RT * NPT;
     struct Raw { uint4 c[F::NC]; uint32_t s[SWN]; };
     // Weights as raw buffer loads from the workgroup's first tile: the wavefront's row tile and the chunk are scalar arithmetic, the lane's part is a
     // register that changes in the last group only.  (With a 64-bit address per load a chunk's staging was 100 of a wavefront's 224 vector
@@ -255,7 +258,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         const unsigned first = k0 * 16u + (paired(g) ? 0u : (unsigned)F::chunk(c & 1, 0) * step);
 #pragma unroll
         for (int i = 0; i < IPT; i++) {
-            const int rt = wave + 4 * i, dt = min(FUSED ? rt % TPW : rt, P.ntiles - 1 - tile0);
+            const int rt = i_t + 4 * i, dt = min(FUSED ? rt % TPW : rt, P.ntiles - 1 - tile0);
             const bool second = FUSED && rt >= TPW;
             const unsigned gp = (unsigned)(dt * P.npairs + g * KL);
 #pragma unroll
@@ -277,7 +280,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         const int g = group_of(chunk);
         return g * 2 * KL + (paired(g) ? b : 2 * b + (chunk & 1));
     };
-    auto stage_part = [&](int chunk, int buf, int w, const Raw (&r)[IPT]) {
+    auto stage_expand = [&](int chunk, int buf, int w, const Raw (&r)[IPT]) __attribute__((always_inline)) {
         const int g = group_of(chunk), i_h = paired(g) ? i_kk & 1 : chunk & 1, b = i_kk;
         const bool live = (PAIRS || chunk < nchunks) && block_of(chunk, i_kk) < nblocks;     // a block past the end of K contributes nothing
 #pragma unroll
@@ -298,6 +301,15 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
                 if (w == 0) *reinterpret_cast<float *>(s_sc + buf * SCB + (b * SCP + rt * 16 + i_r) * 4) = live ? F::scale(r[i].s, i_h) : 0.f;
             if constexpr (MINS)
                 if (w == 0) *reinterpret_cast<float *>(s_mn + buf * SCB + (b * SCP + rt * 16 + i_r) * 4) = live ? F::least(r[i].s, i_h) : 0.f;
+        }
+    };
+    auto stage_part = [&](int chunk, int buf, int w, const Raw (&r)[IPT]) __attribute__((always_inline)) {
+        if constexpr (SPL == 1) stage_expand(chunk, buf, w, r);
+        else switch (i_w + w) {                             // (the wavefront's: constants inside)
+            case 0: stage_expand(chunk, buf, 0, r); break;
+            case 1: stage_expand(chunk, buf, 1, r); break;
+            case 2: stage_expand(chunk, buf, 2, r); break;
+            default: stage_expand(chunk, buf, 3, r); break;
         }
     };
     // activation fragments [block][token tile][part][lane] x 16 bytes: kernel argument + 32-bit offset, the block part wave-uniform
@@ -372,7 +384,7 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
         }
     }
 #pragma unroll
-    for (int w = 0; w < 4; w++) stage_part(chunk, 0, w, rb[1]);
+    for (int w = 0; w < NPT; w++) stage_part(chunk, 0, w, rb[1]);
     stage_load(chunk + 2 * KW, rb[1]);
     // The K loop is a pipeline of groups (RG row tiles x NTW token tiles: four independent MFMA chains): while group i is on the matrix
     // cores, group i + 1's weight fragments leave LDS and group i - 1's sums are scaled.  One barrier per chunk, in front of its last
@@ -469,9 +481,9 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
             if (idx) scale_sums(idx - 1);
             if (g == NG - 1) {
                 xload(nxt, b);
-                if (b < KB - 1) stage_part(nxt, PAR ^ 1, b, rb[PAR]);
+                if (b < KB - 1 && b < NPT) stage_part(nxt, PAR ^ 1, b, rb[PAR]);
                 if (b == KB - 2) {
-                    stage_part(nxt, PAR ^ 1, KB - 1, rb[PAR]);
+                    if constexpr (NPT == 4) stage_part(nxt, PAR ^ 1, KB - 1, rb[PAR]);
                     stage_load(nxt + 2 * KW, rb[PAR]);
                 }
             }
@@ -520,14 +532,14 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
     const bool folded_in = EPI != QG_EPI_PLAIN && P.nrm_in.ssq != nullptr;
 
     if constexpr (EPI == QG_EPI_SWIGLU) {
-        // h = SiLU(gate) * up (go/quant.go:629-631, go/model.go:604-606), stored as the down projection's fragments
+        // h = SiLU(gate) * up (go/quant.go:629-631, go/model.go:604-606), stored as the down projection's fragments (RT = 2: half of a block's k-slots)
 #pragma unroll
-        for (int it0 = 0; it0 < TOK * 4 * (RT / 4); it0 += NTHR) {
-            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % TTW, hb = (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t;
+        for (int it0 = 0; it0 < TOK * RT; it0 += NTHR) {
+            const int it = it0 + et, w = RT == 2 ? (tile0 & 1) * 2 + (lq & 1) : lane >> 4, tt = RT == 2 ? it >> 5 : (it >> 6) % TTW, hb = RT == 2 ? 0 : (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t;
             const int hblk = tile0 / 2 + hb;
-            if (NTHR > TOK * RT && hb >= RT / 4) break;     // (more threads than items of 32 rows)
+            if (NTHR > TOK * RT && (RT == 2 ? tt >= TTW : hb >= RT / 4)) break;     // (more threads than items of 32 rows)
             int oa, ob;
-            slot_offsets(P.out_q4, w, oa, ob);
+            slot_offsets(RT == 2 ? 0 : P.out_q4, RT == 2 ? lq & 1 : w, oa, ob);
             const int sg = t * LD + hb * 32, su = sg + ROWS / 2;
             f32x4_t ga = sum4(sg + oa), gb = sum4(sg + ob);
             f32x4_t ua = sum4(su + oa), ub = sum4(su + ob);
@@ -675,27 +687,28 @@ __global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT ==
                     }
                 }
                 if (fold) {
-                    // folded RMSNorm, producer side (QGemmParams::NormOut): sum of squares of 64 rows of the new residual stream, in
+                    // folded RMSNorm, producer side (QGemmParams::NormOut): sum of squares of 64 rows (RT = 1: 16) of the new residual stream, in
                     // float64 and a fixed order; the values stay in LDS for the fragments below
+                    constexpr int SL = RT == 1 ? 4 : 16;
                     *reinterpret_cast<f32x4_t *>(SW + t * LD + 4 * a) = v[i];
                     double ss = 0.0;
 #pragma unroll
                     for (int j = 0; j < 4; j++) ss = fma((double)v[i][j], (double)v[i][j], ss);
 #pragma unroll
-                    for (int m = 1; m < 16; m *= 2) ss += __shfl_xor(ss, m);
-                    if ((a & 15) == 0 && n < P.n_tokens && row < P.rows) P.nrm_out.ssq[(size_t)n * (P.rows / 64) + row / 64] = ss;
+                    for (int m = 1; m < SL; m *= 2) ss += __shfl_xor(ss, m);
+                    if ((a & (SL - 1)) == 0 && n < P.n_tokens && row < P.rows) P.nrm_out.ssq[(size_t)n * (P.rows / (4 * SL)) + row / (4 * SL)] = ss;
                 }
             }
         }
         if (!fold) return;
         __syncthreads();
 #pragma unroll 2
-        for (int it0 = 0; it0 < TOK * 4 * (ROWS / 32); it0 += NTHR) {
-            const int it = it0 + et, w = lane >> 4, tt = (it >> 6) % TTW, kb = (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t, c0 = row0 + kb * 32;
-            if (NTHR > TOK * ROWS / 8 && kb >= ROWS / 32) break;
+        for (int it0 = 0; it0 < TOK * ROWS / 8; it0 += NTHR) {
+            const int it = it0 + et, w = RT == 1 ? (rbk & 1) * 2 + (lq & 1) : lane >> 4, tt = RT == 1 ? it >> 5 : (it >> 6) % TTW, kb = RT == 1 ? 0 : (it >> 6) / TTW, t = tt * 16 + li, n = tok0 + t, c0 = row0 + kb * 32;
+            if (NTHR > TOK * ROWS / 8 && (RT == 1 ? tt >= TTW : kb >= ROWS / 32)) break;
             if (n >= P.n_tokens || c0 >= P.rows) continue;
             int oa, ob;
-            slot_offsets(P.out_q4, w, oa, ob);
+            slot_offsets(RT == 1 ? 0 : P.out_q4, RT == 1 ? lq & 1 : w, oa, ob);
             const float psc = s_tok[t], *sp = S0 + t * LD + kb * 32, *gp = s_gain + kb * 32;
             const f32x4_t ya = (*reinterpret_cast<const f32x4_t *>(sp + oa) * *reinterpret_cast<const f32x4_t *>(gp + oa)) * psc;
             const f32x4_t yb = (*reinterpret_cast<const f32x4_t *>(sp + ob) * *reinterpret_cast<const f32x4_t *>(gp + ob)) * psc;
@@ -717,6 +730,15 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     };
     const integral_constant<int, 1> one{};
     const integral_constant<int, 2> two{};
+    if constexpr (PREC == PG_EXACT && WT == WT_Q6_K)
+        if (P.slim) {
+            // (a row tile and all tokens a workgroup: a block's expansion is a quarter a wavefront, and four times as many units work.  us a launch, Q6_K, 17 tokens:
+            //  the mean of 768 x 768 and x 2048 12.5 and 10.2, gate and up 11.6 and 9.7, in halves of the tokens while those find a unit each -- 1536 columns, 33 tokens,
+            //  512 halves 25.7; prompts of 173M, 17 tokens 1035 and 897, of 841M, 17 and 33 tokens 2140 and 1919, 2197 and 2025.  Q4_K, whose expansion is two thirds of
+            //  that: 173M 940 and 920, 841M 1880 and 1950: not there)
+            if constexpr (EPI == QG_EPI_SWIGLU) return P.ntiles * ((P.n_tokens + 31) / 32) <= 256 ? go(two, one, two, two) : go(two, one, two, one);
+            else return go(one, one, two, one);
+        }
     const integral_constant<int, 4> four{};
     const integral_constant<int, 8> eight{};
     // Tiles by how many 64 x 64 ones there are.  Up to one per compute unit: eight wavefronts on each (K dealt to two sets), since the four

@@ -47,6 +47,7 @@ struct QGemmParams {
     int nt16, n_tokens;
     int x1;              // prompt precision mode fp16x1 (pgemm_kernel, Q4_0): only the hi half of every activation is multiplied
     int exact;           // files with K-quant matrices (pgemm_kernel): fragments of three bf16 parts (FRAG_EXACT)
+    int slim;            // ... on tiles of 16 rows (pg_slim_step)
     float *out;          // [N][ldo]
     int ldo;
     const float *resid;  // optional [N][ldo]: out = resid + y
