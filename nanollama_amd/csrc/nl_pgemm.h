@@ -26,11 +26,11 @@
 //
 // Measured (us a launch inside a model, profiled; Q|K|V, gate and up, mean of WO and down; in brackets the kernels that these launches ran on
 // before): Q4_0, 2047 tokens, 768 columns: 18.9 (21.8), 37.2 (40.5), 18.5 (23.5); F16, 993 tokens, 1536 columns: 27.6 (35.6), 53.5 (85.0), 28.3
-// (43.2), Q|K|V of both with the attention's images; Q4_K, 333 tokens, 768 columns, PG_EXACT: 12.6, 22.0, 18.6.  A 64 x 64 tile's block costs a
+// (43.2), Q|K|V of both with the attention's images; Q4_K, 333 tokens, 768 columns, PG_EXACT: 9.9, 20.7, 12.0.  A 64 x 64 tile's block costs a
 // wavefront about 310 cycles: 128 on the matrix pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses).  Those
 // overlap with the MFMAs of the SIMD's other wavefronts (1.47 PFLOP/s beside four vector instructions an MFMA) and not with its own, and a SIMD
 // holds two or three; larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
-// be 333 single-token steps: 151 ms, now 1.92 ms (1.49 with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
+// be 333 single-token steps: 151 ms, now 1.44 ms (1.92 at first, 1.49 then with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
 // steps and 1.19e-7 now, and whose range ends at 65504).
 #pragma once
 #include "nl_qgemm.h"
