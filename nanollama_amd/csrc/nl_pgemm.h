@@ -184,8 +184,10 @@ enum { PG_HILO = 0, PG_HI = 1, PG_EXACT = 2 };
 // Wavefronts per SIMD: a plain 64 x 64 Q4_0 tile is held to 168 registers, three workgroups a compute unit (172 without the bound, since the
 // loads are buffer loads: two.  WO and down of 2112 x 2112 and 2112 x 5632, 1000 tokens, 528 workgroups, mean of both: 63.4 us two at a time,
 // 53.9 three).  What it spills is a value of the epilogue's, around the K loop.
-template <int WT, int RT, int NTW, int KW, int EPI, int PREC = PG_HILO, int WR = 1>
-__global__ void __launch_bounds__(256 * KW, (KW > 1 ? 1 : WT == WT_Q4_0 && RT == 4 && NTW == 1 && PREC == PG_HILO ? 3 : 2)) pgemm_kernel(QGemmParams P) {
+// KWR: sets + 16 (WR - 1)
+template <int WT, int RT, int NTW, int KWR, int EPI, int PREC = PG_HILO>
+__global__ void __launch_bounds__(256 * (KWR & 15), ((KWR & 15) > 1 ? 1 : WT == WT_Q4_0 && RT == 4 && NTW == 1 && PREC == PG_HILO ? 3 : 2)) pgemm_kernel(QGemmParams P) {
+    constexpr int KW = KWR & 15, WR = (KWR >> 4) + 1;
     constexpr bool X1 = PREC == PG_HI, EXACT = PREC == PG_EXACT;
     using F = typename std::conditional_t<EXACT, PgExact<WT>, PgFmt<WT>>;
     static_assert(!X1 || WT == WT_Q4_0, "the single-product mode is Q4_0's");
@@ -725,7 +727,7 @@ hipError_t pg_launch_as(const QGemmParams &P, hipStream_t st) {
     auto go = [&](auto rt, auto ntw, auto kw, auto wr) {
         constexpr int RT = decltype(rt)::value, NTW = decltype(ntw)::value, KW = decltype(kw)::value, WR = decltype(wr)::value, TPW = EPI == QG_EPI_SWIGLU ? RT / 2 : RT, TOK = 64 * NTW / WR;
         const int total = ((P.ntiles + TPW - 1) / TPW) * ((P.n_tokens + TOK - 1) / TOK);
-        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW, EPI, PREC, WR>), dim3((total + 7) / 8 * 8), dim3(256 * KW), 0, st, P);
+        hipLaunchKernelGGL((pgemm_kernel<WT, RT, NTW, KW + 16 * (WR - 1), EPI, PREC>), dim3((total + 7) / 8 * 8), dim3(256 * KW), 0, st, P);
         return hipGetLastError();
     };
     const integral_constant<int, 1> one{};
