@@ -3294,7 +3294,9 @@ int nl_finalize(nl_handle e) {
         }
         if (e->fused || e->ly.on) {
             HIPCK(e, dalloc(&e->tick, (size_t)2, &e->bytes_state));
-            HIPCK(e, hipMemset(e->tick, 0, 8));
+            const char *fc = getenv("NL_FORWARD_COUNTER");     // knob (tests): forwards that the handle counts from
+            const unsigned words[2] = {fc ? (unsigned)strtoul(fc, nullptr, 0) : 0u, 0u};
+            HIPCK(e, hipMemcpy(e->tick, words, sizeof words, hipMemcpyHostToDevice));
             HIPCK(e, hipHostMalloc((void **)&e->h_status, sizeof(unsigned), hipHostMallocMapped | hipHostMallocCoherent));
             *e->h_status = 0;
         }

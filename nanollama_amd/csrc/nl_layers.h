@@ -250,7 +250,9 @@ __device__ __forceinline__ void ly_merge_head(const u32x4 *rec, u32x4 *out, int 
 // competes with the weights: 2.4 - 2.8 us an exchange.  So one workgroup of an XCD reads a 32nd of the vector from the fabric and stores it
 // into the XCD's own L2, where all 32 of them find it (24.4 -> 22.6 us a layer; not for the heads' outputs, where the wait is for the
 // slowest unit and the second hop costs what it saves: 21.8 with, 21.5 without).
-// (a later layer's granules: nobody on this XCD has read the vector, or it could not have been written again)
+// (a later layer's granules of the same step: nobody on this XCD has read the vector, or it could not have been written again.  Of the same step
+// only: the counter is shared with the other plans, so what this launch left may be any number of steps old, and "ahead of the tag" by a signed
+// difference is also what a granule of 2^23 to 2^24 steps ago looks like)
 __device__ __forceinline__ void ly_relay(const u32x4 *src, u32x4 *dst, int ng, int slot, unsigned tag, LyPoll &Q, int lane) {
     const int per = (ng + LY_PER_XCD - 1) / LY_PER_XCD, i = slot * per + lane, n = min(per, ng - slot * per);
     if (n <= 0) return;
@@ -258,7 +260,7 @@ __device__ __forceinline__ void ly_relay(const u32x4 *src, u32x4 *dst, int ng, i
     u32x4 g;
     for (int spins = 0;;) {
         g = ly_granule(r, (unsigned)min(i, slot * per + n - 1));
-        if (__all((int)(g.x - tag) >= 0) || !ly_again(Q, spins, 1024u, lane)) break;
+        if (__all(g.x >> 8 == tag >> 8 && g.x >= tag) || !ly_again(Q, spins, 1024u, lane)) break;
     }
     if (lane < n) __builtin_amdgcn_raw_buffer_store_b128(g, w, i * 16, 0, 0);
 }

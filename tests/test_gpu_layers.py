@@ -102,3 +102,17 @@ def test_models_that_take_the_launch(tmp_path, monkeypatch, layers, wtype, runs)
     m = hip.load_llama_model(gguf.load_gguf(str(p)))
     assert m.debug_read("layers_max_pos", 1)[0] == (160 if runs else 0)
     m.close()
+
+
+# forwards since the launch last wrote its buffers (here: since they were cleared): half the counter's range back is not ahead
+@pytest.mark.parametrize("counter", [0x7ffff0, 0x7fffff, 0x800000, 0xfffff0, 0xffffff, 0x1000000])
+def test_the_age_of_a_buffer_does_not_matter(tmp_path, monkeypatch, counter):
+    monkeypatch.setenv("NL_FORWARD_COUNTER", str(counter))
+    monkeypatch.setenv("NL_QUIET", "1")
+    shape, dev, plain = _models(tmp_path, monkeypatch, "wide_groups", "q8_0", seq_len=300)
+    toks = synth.prompt_ids(20, shape.vocab, seed=3)
+    for m in (dev, plain):
+        m.prefill(toks, want_logits=False)
+    assert dev.decode_greedy(5, 20, 40) == plain.decode_greedy(5, 20, 40)
+    assert dev.last_error() == "" and dev.debug_read("layers_max_pos", 1)[0] > 0
+    dev.close(); plain.close()
