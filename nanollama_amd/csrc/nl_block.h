@@ -315,8 +315,8 @@ __global__ void __launch_bounds__(BLK_THREADS) attn_block_kernel(BlockParams P) 
 #pragma unroll
             for (int kk = 0; kk < NV; kk++) {
                 const float pw = __shfl(p, (vg + 4 * kk) * 4);
-                const bool vcurrow = t0 + wave * 16 + vg + 4 * kk == pos;
-                const float4 v4 = vcurrow ? vc4 : vreg[kk];       // (a masked row's V may be stale but is finite, and its p is 0)
+                const bool vcurrow = t0 + wave * 16 + vg + 4 * kk >= pos;
+                const float4 v4 = vcurrow ? vc4 : vreg[kk];       // (a masked row's p is 0, and what lies at `pos` may not be finite)
                 o.x = fmaf(pw, v4.x, o.x); o.y = fmaf(pw, v4.y, o.y); o.z = fmaf(pw, v4.z, o.z); o.w = fmaf(pw, v4.w, o.w);
             }
             o.x += __shfl_xor(o.x, 16); o.y += __shfl_xor(o.y, 16); o.z += __shfl_xor(o.z, 16); o.w += __shfl_xor(o.w, 16);

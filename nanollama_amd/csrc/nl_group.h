@@ -235,7 +235,8 @@ __global__ void __launch_bounds__(GRP_THREADS) qkv_attn_kernel(GroupParams P) {
 #pragma unroll
             for (int kk = 0; kk < NV; kk++) {
                 const int row = tg + kk * NGR;
-                const bool cur = t0 + row == pos;   // the row this launch produced: taken from LDS, not from memory
+                const bool cur = t0 + row >= pos;   // the row this launch produced: taken from LDS, not from memory; rows past it, whose p is 0, likewise:
+                                                    // what lies at `pos` may not be finite
                 kreg[kk].x = cur ? kc4.x : kreg[kk].x; kreg[kk].y = cur ? kc4.y : kreg[kk].y;
                 kreg[kk].z = cur ? kc4.z : kreg[kk].z; kreg[kk].w = cur ? kc4.w : kreg[kk].w;
                 vreg[kk].x = cur ? vc4.x : vreg[kk].x; vreg[kk].y = cur ? vc4.y : vreg[kk].y;
@@ -266,7 +267,7 @@ __global__ void __launch_bounds__(GRP_THREADS) qkv_attn_kernel(GroupParams P) {
 #pragma unroll
             for (int kk = 0; kk < NV; kk++) {
                 const int row = tg + kk * NGR;
-                const float pw = row < n ? sc[row] : 0.f;   // (a masked row's V may be stale but is finite)
+                const float pw = row < n ? sc[row] : 0.f;   // (a masked row's V is this position's)
                 o.x = fmaf(pw, vreg[kk].x, o.x); o.y = fmaf(pw, vreg[kk].y, o.y);
                 o.z = fmaf(pw, vreg[kk].z, o.z); o.w = fmaf(pw, vreg[kk].w, o.w);
             }

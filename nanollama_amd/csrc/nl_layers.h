@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(LY_THREADS) layers_kernel(LayersParams P0) {
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         const float pw = __shfl(p, (vg + 4 * k) * 4);
-                        const bool vcurrow = t0 + wave * 16 + vg + 4 * k == pos;
+                        const bool vcurrow = t0 + wave * 16 + vg + 4 * k >= pos;        // (its own row and those past it, whose p is 0: what lies there may not be finite)
                         const float4 v4 = vcurrow ? vc4 : vreg[k];
                         o.x = fmaf(pw, v4.x, o.x); o.y = fmaf(pw, v4.y, o.y); o.z = fmaf(pw, v4.z, o.z); o.w = fmaf(pw, v4.w, o.w);
                     }

@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(PD_THREADS, 2) pd_decode_kernel(PdParams P0) {
                         const float pw[4] = {pw4.x, pw4.y, pw4.z, pw4.w};
 #pragma unroll
                         for (int kk = 0; kk < 4; kk++) {
-                            const bool vcurrow = t0 + wave * 16 + 4 * vg + kk == pos;
+                            const bool vcurrow = t0 + wave * 16 + 4 * vg + kk >= pos;      // (rows past it have p 0, and what lies at `pos` may not be finite)
                             const float4 v4 = vcurrow ? vc4 : vreg[kk];
                             o.x = fmaf(pw[kk], v4.x, o.x); o.y = fmaf(pw[kk], v4.y, o.y); o.z = fmaf(pw[kk], v4.z, o.z); o.w = fmaf(pw[kk], v4.w, o.w);
                         }
