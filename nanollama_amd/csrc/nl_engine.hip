@@ -293,7 +293,7 @@ struct nl_engine {
         bool on = false;
         int min_pos = 0, max_pos = 0;
         LayersEntry *tab = nullptr;
-        u32x4 *gran = nullptr;    // gq | gr | go | gp | gh | gx | the XCDs' copies | tickets
+        u32x4 *gran = nullptr;    // nl_layers_map.h
     } ly;
     hipEvent_t turn_done = nullptr;   // chip_turn: behind this handle's last launch whose workgroups wait for each other
     bool turn_on = false;             // ... the handle is on its device's list
@@ -800,12 +800,11 @@ void build_plan_layers(nl_engine *e, std::vector<Op> &plan) {
     P.kcache = e->kcache; P.vcache = e->vcache; P.kv_layer_stride = e->kv_layer_stride; P.kv_stream_stride = e->kv_stream_stride;
     P.ctl = e->ctl; P.tick = e->tick; P.status = e->tick + 1; P.host_status = e->h_status; P.spin_limit = e->spin_limit;
     P.rec_max = layers_records(c.seq_len);
-    P.loc_n = layers_loc(P.t_d, P.t_i);
-    u32x4 *g = e->ly.gran;
-    auto take = [&](int n) { u32x4 *at = g; g += n; return at; };
-    P.gq = take(P.t_qkv * GPT); P.gr = take(P.H * P.rec_max * LY_REC); P.go = take(P.H * LY_REC);
-    P.gp = take(P.t_d * 2 * LY_HG); P.gh = take(P.t_i * GPT); P.gx = take(P.t_d * 2 * LY_HG); P.loc = take(LY_XCDS * P.loc_n);
-    P.tickets = reinterpret_cast<unsigned *>(g);                         // (LY_XCDS * 4 granules)
+    const LayersMap m = layers_map(P.t_qkv, P.H, P.rec_max, P.t_d, P.t_i);
+    u32x4 *const g = e->ly.gran;
+    P.gq = g + m.gq; P.gr = g + m.gr; P.go = g + m.go; P.gp = g + m.gp; P.gh = g + m.gh; P.gx = g + m.gx;
+    P.loc = g + m.loc; P.loc_n = m.loc_n;
+    P.tickets = reinterpret_cast<unsigned *>(g + m.tickets);
     const int wt = L0.qkv.wtype, grid = e->num_cus;
     plan.push_back({K_FFNBLOCK, 0, nullptr, 0, [P, wt, grid](hipStream_t st) { return launch_layers(wt, P, grid, st); }});
     push_head(e, plan, e->x[0]);
@@ -3307,8 +3306,7 @@ int nl_finalize(nl_handle e) {
                 tab.push_back(LayersEntry{{L.qkv.q, L.wo.q, L.gate.q, L.up.q, L.down.q}, {L.qkv.s, L.wo.s, L.gate.s, L.up.s, L.down.s}, {L.attn_norm, L.ffn_norm}, L.bq, L.bk, L.bv, L.bo});
             HIPCK(e, dalloc(&e->ly.tab, tab.size(), &e->bytes_state));
             HIPCK(e, hipMemcpy(e->ly.tab, tab.data(), tab.size() * sizeof(LayersEntry), hipMemcpyHostToDevice));
-            const size_t n = (size_t)L0.qkv.ntiles * GPT + (size_t)e->Hs * (layers_records(c.seq_len) + 1) * LY_REC +
-                             (size_t)(LY_XCDS + 1) * layers_loc(L0.wo.ntiles, L0.gate.ntiles) + LY_XCDS * 4;
+            const size_t n = (size_t)layers_map(L0.qkv.ntiles, e->Hs, layers_records(c.seq_len), L0.wo.ntiles, L0.gate.ntiles).total;
             HIPCK(e, dalloc(&e->ly.gran, n, &e->bytes_state));
             HIPCK(e, hipMemset(e->ly.gran, 0, n * sizeof(u32x4)));
         }

@@ -30,17 +30,17 @@
 // count of loads in flight holds across the phases.  They go out a quarter of a microsecond apart: all at once they stand before
 // the exchange that follows in every queue of the chip (22.5 us a layer; sleeps of 2, 4, 8: 22.1, 21.7, 21.85).
 #pragma once
+#include "nl_layers_map.h"
 #include "nl_tp.h"
 
 namespace nl {
 
 constexpr int LY_CW = 8, LY_GW = 4, LY_WAVES = LY_CW + LY_GW, LY_THREADS = LY_WAVES * 64, LY_GT = LY_GW * 64;
 constexpr int LY_PASS = 128;               // positions of a unit
-constexpr int LY_REC = 22;                 // granules of an attention record: max, sum, 64 values
 constexpr int LY_MAX_REC = 16;             // records of a head
 constexpr int LY_MAX_HPU = 8;              // heads of a unit
-constexpr int LY_HG = 3;                   // granules of half a tile
-constexpr int LY_XCDS = 8, LY_PER_XCD = 32; // a launch is one workgroup a compute unit of a whole chip
+constexpr int LY_PER_XCD = 32;             // a launch is one workgroup a compute unit of a whole chip
+static_assert(LY_TG == GPT, "granules of a tile");
 constexpr int LY_RELAY = 1;                // the exchanging wavefront that relays
 constexpr int LY_MAX_COLS = 2048, LY_MAX_FF = 4096;
 
@@ -67,7 +67,7 @@ struct LayersParams {
     u32x4 *go, *gp, *gh, *gx;              // the heads' outputs [H][LY_REC] (values from 2 on); x' half tiles; h tiles; x half tiles
     u32x4 *loc;                            // [LY_XCDS] copies of gp | gh | gx, `loc_n` granules each
     int loc_n;
-    unsigned *tickets;                     // [LY_XCDS], 64 bytes apart: workgroups that started on the XCD, ever
+    unsigned *tickets;                     // [LY_XCDS], a line apart: workgroups that started on the XCD, ever
     int rec_max;
     unsigned *status, *host_status;
     int spin_limit;
@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(LY_THREADS) layers_kernel(LayersParams P0) {
     xcd &= LY_XCDS - 1;
     if (tid == 0) {
         lds_dead = 0;
-        lds_slot = (int)(atomicAdd(P.tickets + xcd * 16, 1u) % LY_PER_XCD);      // (every launch adds 32: a launch that does not gives up, and is the handle's last)
+        lds_slot = (int)(atomicAdd(P.tickets + xcd * (LY_LINE * 4), 1u) % LY_PER_XCD);      // (every launch adds 32: a launch that does not gives up, and is the handle's last)
     }
     for (int i = tid; i < P.L * LY_ENTRY; i += LY_THREADS) tab[i] = reinterpret_cast<const uint2 *>(P.layers)[i];
     const int pos = sload_i32(P.ctl + CTL_POS), strm = sload_i32(P.ctl + CTL_STREAM);
@@ -641,7 +641,6 @@ __global__ void __launch_bounds__(LY_THREADS) layers_kernel(LayersParams P0) {
 
 // records of a head
 inline int layers_records(int seq_len) { return std::min((seq_len + LY_PASS - 1) / LY_PASS, LY_MAX_REC); }
-inline int layers_loc(int t_d, int t_i) { return t_d * 4 * LY_HG + t_i * GPT; }
 
 inline hipError_t launch_layers(int wtype, const LayersParams &P, int grid, hipStream_t st) {
     switch (wtype) {
