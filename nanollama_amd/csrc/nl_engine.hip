@@ -12,6 +12,7 @@
 #include "nl_kernels.h"
 #include "nl_qgemm.h"
 #include "nl_layers.h"
+#include "nl_turns.h"
 #include "nl_pgemm.h"
 #include "nl_dgemm.h"
 #include "nl_sgemm.h"
@@ -295,7 +296,7 @@ struct nl_engine {
         LayersEntry *tab = nullptr;
         u32x4 *gran = nullptr;    // nl_layers_map.h
     } ly;
-    hipEvent_t turn_done = nullptr;   // chip_turn: behind this handle's last launch whose workgroups wait for each other
+    hipEvent_t turn_done = nullptr;   // nl_turns.h: behind this handle's last launch in a turn
     bool turn_on = false;             // ... the handle is on its device's list
     float *parts = nullptr;       // [Hs][D] per-head WO partials of the fused block
     unsigned long long *xchg = nullptr;   // [Hs][192] granules exchanged inside a head's cluster
@@ -1214,7 +1215,34 @@ void destroy_graphs(nl_engine::PlanSet &S) {
     if (S.graph) { (void)hipGraphDestroy(S.graph); S.graph = nullptr; }
 }
 
+// nl_turns.h.  One per device
+Turns<nl_engine> g_turns[64];
+template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
+    if (!e->turn_on || !waits) return launch();
+    return g_turns[e->dev].run(e, launch,
+        [&](nl_engine *o) -> int { HIPCK(e, hipStreamWaitEvent(e->stream, o->turn_done, 0)); return NL_OK; },
+        [&]() -> int { HIPCK(e, hipEventRecord(e->turn_done, e->stream)); return NL_OK; });
+}
+// (nl_finalize, nl_destroy)
+int chip_turn_join(nl_engine *e) {
+    if (e->dev < 0 || e->dev >= 64 || e->G != 1 || e->force_tp_plan || e->p2p.on || !(e->fused || e->ly.on || e->pd.candidate)) return NL_OK;
+    HIPCK(e, hipEventCreateWithFlags(&e->turn_done, hipEventDisableTiming));
+    std::lock_guard<std::mutex> setup(g_setup_mu);           // (the other handles' streams must not be in a capture)
+    if (int rc = g_turns[e->dev].join(e, e->ly.on, [&](nl_engine *o) -> int { HIPCK(e, hipEventRecord(o->turn_done, o->stream)); return NL_OK; })) return rc;
+    e->turn_on = true;
+    return NL_OK;
+}
+// for the length of a capture on e->stream (the caller holds g_setup_mu)
+std::unique_lock<std::shared_mutex> chip_turn_capture(nl_engine *e) { return e->turn_on ? g_turns[e->dev].capture() : std::unique_lock<std::shared_mutex>(); }
+void chip_turn_leave(nl_engine *e) {
+    if (e->turn_on) g_turns[e->dev].leave(e);
+    if (e->turn_done) (void)hipEventDestroy(e->turn_done);
+    e->turn_done = nullptr;
+    e->turn_on = false;
+}
+
 int capture_graph(nl_engine *e, nl_engine::PlanSet &S) {
+    const auto turn = chip_turn_capture(e);
     HIPCK(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
     int rc = run_plan_eager(e, S);
     hipGraph_t g = nullptr;
@@ -1283,57 +1311,6 @@ int plan_index(const nl_engine *e, int pos_last) {
     if (e->ly.on && pos_last >= e->ly.min_pos && pos_last < e->ly.max_pos) return 3;
     if (!(e->fused && pos_last < e->fused_max_pos)) return 0;
     return (e->attn_helpers && pos_last >= TP_PASS) ? 2 : 1;
-}
-nl_engine::PlanSet &pick_plan(nl_engine *e, int pos_last) { return e->ps[plan_index(e, pos_last)]; }
-
-// A launch of nl_layers.h needs every compute unit of its device.  Two of them, of two handles whose threads decode at the same time, or one beside another
-// launch whose workgroups wait for each other (nl_block.h, nl_group.h, nl_tp.h, nl_persist.h), could each hold units that the other waits for until a bounded
-// poll gives up: half a second, and the handle is back on five launches a layer.  So where a device has several handles with such plans, and one of them
-// nl_layers.h's, these launches take turns, on the device: each waits for the event behind the last one of another handle.  A handle that is alone
-// records and waits for nothing.
-std::mutex g_turn_mu;
-struct ChipTurns { std::vector<nl_engine *> handles; nl_engine *last = nullptr; };
-ChipTurns g_turns[64];
-// (an event is not waited for while the stream behind it is in a capture: hence g_setup_mu)
-template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
-    if (!e->turn_on || !waits) return launch();
-    ChipTurns &T = g_turns[e->dev];
-    auto shared = [&] { return T.handles.size() > 1 && std::any_of(T.handles.begin(), T.handles.end(), [](const nl_engine *h) { return h->ly.tab != nullptr; }); };
-    {
-        std::lock_guard<std::mutex> lk(g_turn_mu);
-        if (!shared()) return launch();
-    }
-    std::scoped_lock lk(g_setup_mu, g_turn_mu);
-    if (T.last && T.last != e) HIPCK(e, hipStreamWaitEvent(e->stream, T.last->turn_done, 0));
-    const int rc = launch();
-    HIPCK(e, hipEventRecord(e->turn_done, e->stream));
-    T.last = e;
-    return rc;
-}
-// (nl_finalize, nl_destroy)
-int chip_turn_join(nl_engine *e) {
-    if (e->dev < 0 || e->dev >= 64 || e->G != 1 || e->force_tp_plan || e->p2p.on || !(e->fused || e->ly.on || e->pd.candidate)) return NL_OK;
-    HIPCK(e, hipEventCreateWithFlags(&e->turn_done, hipEventDisableTiming));
-    std::scoped_lock lk(g_setup_mu, g_turn_mu);              // (the other handle's stream must not be in a capture)
-    ChipTurns &T = g_turns[e->dev];
-    if (T.handles.size() == 1) {                             // what the other one launched while it was alone
-        T.last = T.handles[0];
-        HIPCK(e, hipEventRecord(T.last->turn_done, T.last->stream));
-    }
-    T.handles.push_back(e);
-    e->turn_on = true;
-    return NL_OK;
-}
-void chip_turn_leave(nl_engine *e) {
-    if (e->turn_on) {
-        std::lock_guard<std::mutex> lk(g_turn_mu);
-        ChipTurns &T = g_turns[e->dev];
-        T.handles.erase(std::remove(T.handles.begin(), T.handles.end(), e), T.handles.end());
-        if (T.last == e) T.last = nullptr;
-    }
-    if (e->turn_done) (void)hipEventDestroy(e->turn_done);
-    e->turn_done = nullptr;
-    e->turn_on = false;
 }
 
 int launch_step(nl_engine *e, int pos) {
@@ -3733,6 +3710,7 @@ int nl_sample_decode(nl_handle e, int stream, int pos, int n_steps, const nl_sam
             const int k = plan_index(e, pos + i + e->graph_steps - 1);
             if (!e->samp_graph_exec[k] || memcmp(&e->samp_graph_params[k], p, sizeof(*p)) != 0) {
                 std::lock_guard<std::mutex> setup(g_setup_mu);
+                const auto turn = chip_turn_capture(e);
                 if (e->samp_graph_exec[k]) { hipGraphExecDestroy(e->samp_graph_exec[k]); e->samp_graph_exec[k] = nullptr; }
                 if (e->samp_graph[k]) { hipGraphDestroy(e->samp_graph[k]); e->samp_graph[k] = nullptr; }
                 hipError_t cs = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal);
@@ -3998,6 +3976,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
                     if (G.n == m && G.nsplit == key_split) { exec = G.exec; e->step_path = G.path; }
                 if (!exec) {
                     std::lock_guard<std::mutex> setup(g_setup_mu);      // (a capture must not overlap another thread's allocations)
+                    const auto turn = chip_turn_capture(e);
                     hipGraph_t gr = nullptr;
                     if (hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
                         const int rc2 = batched_step(e, b, e->stream, m, 1);
@@ -4084,11 +4063,11 @@ int nl_profile_forward(nl_handle e, int stream, int token, int pos, int iters, f
     for (int k = 0; k < NL_NUM_KINDS; k++) { ms_out[k] = 0.f; calls_out[k] = 0; }
     if ((rc = note_positions(e, stream, pos, 1))) return rc;
     if ((rc = set_ctl(e, token, pos, 0, stream))) return rc;
-    const nl_engine::PlanSet *Sp = &pick_plan(e, pos);   // the plan a step at this position runs
+    const nl_engine::PlanSet *Sp = &e->ps[plan_index(e, pos)];   // the plan a step at this position runs
     if ((rc = run_plan_eager(e, *Sp))) return rc;
     HIPCK(e, hipStreamSynchronize(e->stream));
     if (take_fused_timeout(e)) {
-        Sp = &pick_plan(e, pos);
+        Sp = &e->ps[plan_index(e, pos)];
         if ((rc = run_plan_eager(e, *Sp))) return rc;
         HIPCK(e, hipStreamSynchronize(e->stream));
     }
