@@ -1228,7 +1228,9 @@ int chip_turn_join(nl_engine *e) {
     if (e->dev < 0 || e->dev >= 64 || e->G != 1 || e->force_tp_plan || e->p2p.on || !(e->fused || e->ly.on || e->pd.candidate)) return NL_OK;
     HIPCK(e, hipEventCreateWithFlags(&e->turn_done, hipEventDisableTiming));
     std::lock_guard<std::mutex> setup(g_setup_mu);           // (the other handles' streams must not be in a capture)
-    if (int rc = g_turns[e->dev].join(e, e->ly.on, [&](nl_engine *o) -> int { HIPCK(e, hipEventRecord(o->turn_done, o->stream)); return NL_OK; })) return rc;
+    if (int rc = g_turns[e->dev].join(e, e->ly.on,
+            [&](nl_engine *o) -> int { HIPCK(e, hipStreamWaitEvent(e->stream, o->turn_done, 0)); return NL_OK; },
+            [&](nl_engine *o) -> int { HIPCK(e, hipEventRecord(o->turn_done, o->stream)); return NL_OK; })) return rc;
     e->turn_on = true;
     return NL_OK;
 }
@@ -1439,6 +1441,7 @@ bool take_fused_timeout(nl_engine *e) {
     (void)hipStreamSynchronize(e->stream);
     e->fused = e->ly.on = false;
     e->fused_retired = true;
+    if (e->turn_on) g_turns[e->dev].retire(e);
     destroy_samp_graphs(e);
     e->fail(NL_OK, "warning: a fused-launch cluster exchange timed out (status %u); the step was redone on the general plan, "
                    "which this handle keeps from now on", st);
@@ -4063,23 +4066,26 @@ int nl_profile_forward(nl_handle e, int stream, int token, int pos, int iters, f
     for (int k = 0; k < NL_NUM_KINDS; k++) { ms_out[k] = 0.f; calls_out[k] = 0; }
     if ((rc = note_positions(e, stream, pos, 1))) return rc;
     if ((rc = set_ctl(e, token, pos, 0, stream))) return rc;
-    const nl_engine::PlanSet *Sp = &e->ps[plan_index(e, pos)];   // the plan a step at this position runs
-    if ((rc = run_plan_eager(e, *Sp))) return rc;
+    int k = plan_index(e, pos);                          // the plan a step at this position runs
+    if ((rc = chip_turn(e, k > 0, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
     HIPCK(e, hipStreamSynchronize(e->stream));
     if (take_fused_timeout(e)) {
-        Sp = &e->ps[plan_index(e, pos)];
-        if ((rc = run_plan_eager(e, *Sp))) return rc;
+        k = plan_index(e, pos);
+        if ((rc = chip_turn(e, k > 0, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
         HIPCK(e, hipStreamSynchronize(e->stream));
     }
-    const nl_engine::PlanSet &S = *Sp;
-    for (const Op &op : S.ops) {
-        HIPCK(e, hipEventRecord(e->ev0, e->stream));
-        for (int it = 0; it < iters; it++) {
-            hipError_t s = op.fn(e->stream);
-            if (s != hipSuccess) return e->fail(NL_ERR_HIP, "launch %s: %s", kKindNames[op.kind], hipGetErrorString(s));
-            if ((rc = run_collective(e, op))) return rc;
-        }
-        HIPCK(e, hipEventRecord(e->ev1, e->stream));
+    for (const Op &op : e->ps[k].ops) {
+        rc = chip_turn(e, k > 0, [&]() -> int {
+            HIPCK(e, hipEventRecord(e->ev0, e->stream));
+            for (int it = 0; it < iters; it++) {
+                hipError_t s = op.fn(e->stream);
+                if (s != hipSuccess) return e->fail(NL_ERR_HIP, "launch %s: %s", kKindNames[op.kind], hipGetErrorString(s));
+                if (int cc = run_collective(e, op)) return cc;
+            }
+            HIPCK(e, hipEventRecord(e->ev1, e->stream));
+            return NL_OK;
+        });
+        if (rc) return rc;
         HIPCK(e, hipEventSynchronize(e->ev1));
         float ms = 0.f;
         HIPCK(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));

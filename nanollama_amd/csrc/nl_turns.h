@@ -42,15 +42,23 @@ public:
         last = h;
         return rc;
     }
-    // record(other): other's event behind what it launched while it was alone
-    template <class R> int join(H *h, bool whole, R record) {
+    // a newcomer; where it makes the launches take turns, it waits for whatever the others launched at will
+    template <class W, class R> int join(H *h, bool whole, W wait, R record) {
         std::unique_lock<std::shared_mutex> lk(mu);
-        if (members.size() == 1) {
-            last = members[0].h;
-            if (const int rc = record(last)) return rc;
-        }
         members.push_back({h, whole});
+        if (shared())
+            for (size_t i = 0; i + 1 < members.size(); i++) {
+                int rc = record(members[i].h);
+                if (!rc) rc = wait(members[i].h);
+                if (rc) { members.pop_back(); return rc; }
+            }
         return 0;
+    }
+    // h no longer takes the whole device
+    void retire(H *h) {
+        std::unique_lock<std::shared_mutex> lk(mu);
+        for (Member &m : members)
+            if (m.h == h) m.whole = false;
     }
     void leave(H *h) {
         std::unique_lock<std::shared_mutex> lk(mu);

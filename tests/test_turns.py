@@ -18,13 +18,13 @@ DRIVER = r"""
 struct H { const char *name; };
 static std::string out;
 static nl::Turns<H> T, other_device;
-static H a{"a"}, b{"b"};
+static H a{"a"}, b{"b"}, c{"c"};
 static int go(nl::Turns<H> &t, H *h) {
     return t.run(h, [&] { out += std::string(" launch:") + h->name; return 0; },
                  [&](H *o) { out += std::string(" ") + h->name + "<" + o->name; return 0; }, [&] { out += std::string(" rec:") + h->name; return 0; });
 }
 static int join(H *h, bool whole) {
-    return T.join(h, whole, [&](H *o) { out += std::string(" rec:") + o->name; return 0; });
+    return T.join(h, whole, [&](H *o) { out += std::string(" ") + h->name + "<" + o->name; return 0; }, [&](H *o) { out += std::string(" rec:") + o->name; return 0; });
 }
 static bool soon(std::atomic<int> &n, int want) {       // (a second at most)
     for (int i = 0; i < 1000 && n < want; i++) std::this_thread::sleep_for(std::chrono::milliseconds(1));
@@ -45,6 +45,15 @@ int main(int, char **argv) {
     if (what == "alone") { join(&a, true); go(T, &a); go(T, &a); }
     if (what == "at_will") { join(&a, false); join(&b, false); go(T, &a); go(T, &b); go(T, &a); }
     if (what == "pair") { join(&a, true); go(T, &a); join(&b, false); go(T, &b); go(T, &b); go(T, &a); T.leave(&b); go(T, &a); }
+    if (what == "third") { join(&a, false); join(&b, false); go(T, &a); go(T, &b); join(&c, true); go(T, &c); go(T, &b); go(T, &a); }
+    if (what == "retired") { join(&a, true); join(&b, false); go(T, &b); T.retire(&a); go(T, &a); go(T, &b); join(&c, true); go(T, &c); }
+    if (what == "gone") { join(&a, true); join(&b, true); go(T, &a); T.leave(&a); go(T, &b); join(&c, false); go(T, &c); }
+    if (what == "failed_join") {
+        join(&a, true);
+        int rc = T.join(&b, false, [](H *) { return -7; }, [](H *) { return 0; });
+        out += " " + std::to_string(rc);
+        go(T, &a);
+    }
     if (what == "failed_wait") {
         join(&a, true); join(&b, true); go(T, &a);
         int rc = T.run(&b, [] { out += " launched"; return 0; }, [](H *) { return -7; }, [] { return 0; });
@@ -52,16 +61,16 @@ int main(int, char **argv) {
     }
     if (what == "locks") {
         join(&a, true);
-        other_device.join(&b, true, [](H *) { return 0; });
+        other_device.join(&b, true, [](H *) { return 0; }, [](H *) { return 0; });
         out = overlap(T, other_device) ? " devices_apart" : " devices_together";
         nl::Turns<H> u;
-        u.join(&a, false, [](H *) { return 0; });
-        u.join(&b, false, [](H *) { return 0; });
+        u.join(&a, false, [](H *) { return 0; }, [](H *) { return 0; });
+        u.join(&b, false, [](H *) { return 0; }, [](H *) { return 0; });
         out += overlap(u, u) ? " at_will_apart" : " at_will_together";
         { auto hold = u.capture(); out += hold ? " held" : " free"; }
         nl::Turns<H> v;
-        v.join(&a, true, [](H *) { return 0; });
-        v.join(&b, false, [](H *) { return 0; });
+        v.join(&a, true, [](H *) { return 0; }, [](H *) { return 0; });
+        v.join(&b, false, [](H *) { return 0; }, [](H *) { return 0; });
         { auto hold = v.capture(); out += hold ? " held" : " free"; }
         out += overlap(v, v) ? " turns_together" : " turns_apart";
     }
@@ -70,9 +79,14 @@ int main(int, char **argv) {
 """
 EXPECT = {
     "alone": "launch:a launch:a",
-    "at_will": "rec:a launch:a launch:b launch:a",
+    "at_will": "launch:a launch:b launch:a",
     "pair": "launch:a rec:a b<a launch:b rec:b launch:b rec:b a<b launch:a rec:a launch:a",
-    "failed_wait": "rec:a launch:a rec:a -7",
+    # two that launched at will: the newcomer waits for both, and then everybody for the last
+    "third": "launch:a launch:b rec:a c<a rec:b c<b launch:c rec:c b<c launch:b rec:b a<b launch:a rec:a",
+    "retired": "rec:a b<a launch:b rec:b launch:a launch:b rec:a c<a rec:b c<b c<b launch:c rec:c",
+    "gone": "rec:a b<a launch:a rec:a launch:b rec:b c<b launch:c rec:c",
+    "failed_join": "-7 launch:a",
+    "failed_wait": "rec:a b<a launch:a rec:a -7",
     "locks": "devices_apart at_will_apart free held turns_apart",
 }
 
