@@ -293,6 +293,7 @@ struct nl_engine {
     struct Layers {               // nl_layers.h: steps below max_pos and from min_pos on run all layers in one launch (ps[3])
         bool on = false;
         int min_pos = 0, max_pos = 0;
+        int give_ups = 0;         // launches whose exchanges timed out (take_fused_timeout)
         LayersEntry *tab = nullptr;
         u32x4 *gran = nullptr;    // nl_layers_map.h
     } ly;
@@ -305,7 +306,8 @@ struct nl_engine {
     unsigned *h_status = nullptr; // pinned, device-visible: non-zero after an in-kernel exchange gave up
     int spin_limit = 400000;      // polls before a cluster exchange gives up (NL_FUSED_SPIN_LIMIT)
     int num_cus = 256;            // compute units of the device: a fused launch must fit on them all at once
-    bool fused_retired = false;   // an exchange timed out once: the handle stays on the general plan
+    bool fused_retired = false;   // an exchange of a fused launch timed out once: the handle does without them
+    bool redo = false;            // a call is redone on the general plan (take_fused_timeout)
     int graph_steps = 1;
     EmbedParams plan_embed{};    // kept for the fused argmax + embed launch of the multi-step graph
     ArgmaxParams plan_argmax{};
@@ -1310,6 +1312,7 @@ void destroy_samp_graphs(nl_engine *e) {
 // (ps[2]: the fused plan of the wide tier on one GPU from the second attention pass on -- its attention launch is the variant
 //  whose passes are shared by helper blocks, nl_tp.h; the first pass keeps the launch compiled without them: 0.7 us per layer)
 int plan_index(const nl_engine *e, int pos_last) {
+    if (e->redo) return 0;
     if (e->ly.on && pos_last >= e->ly.min_pos && pos_last < e->ly.max_pos) return 3;
     if (!(e->fused && pos_last < e->fused_max_pos)) return 0;
     return (e->attn_helpers && pos_last >= TP_PASS) ? 2 : 1;
@@ -1427,24 +1430,39 @@ int p2p_check(nl_engine *e) {
     return NL_OK;
 }
 
-// After a synchronize: did a cluster exchange of a fused launch (nl_block.h, nl_group.h) give up?  HIP promises nothing
-// about which workgroups of a launch are resident together, so on a GPU shared with another tenant a member can wait
+// After a synchronize: did an exchange of a fused launch (nl_block.h, nl_group.h, nl_tp.h) or of the layer launch (nl_layers.h) give up?  HIP promises
+// nothing about which workgroups of a launch are resident together, so on a GPU shared with another tenant a member can wait
 // for a peer that has not been dispatched.  Forward cannot fail in the reference (go/model.go:490): the flag is
-// cleared, the fused plan is retired for this handle, and the caller redoes its whole call on the general plan (every
-// buffer a step writes -- residual stream, K/V rows of its positions, logits, ids -- is rewritten by the redo).
-// nl_last_error carries a one-time note while the call returns NL_OK.
+// cleared and the caller redoes its whole call on the general plan (every buffer a step writes -- residual stream, K/V rows of
+// its positions, logits, ids -- is rewritten by the redo).  The fused plan is then retired for this handle.  The layer launch needs every compute unit, where
+// the others leave a margin, and meets any launch of another process that waits too: it is tried again, up to three give-ups, and the fused plan that
+// served its positions before is what the handle keeps then.  nl_last_error carries a note while the call returns NL_OK.
+constexpr int LY_TRIES = 3;
+struct RedoScope {                           // the length of a call: its redo stays on the general plan, the next call does not
+    nl_engine *e;
+    explicit RedoScope(nl_engine *h) : e(h) {}
+    ~RedoScope() { e->redo = false; }
+};
 bool take_fused_timeout(nl_engine *e) {
     if (!e->h_status || !*e->h_status) return false;
-    const unsigned st = *e->h_status;
+    unsigned st = *e->h_status, all = 0;
+    if (hipMemcpy(&all, e->tick + 1, sizeof all, hipMemcpyDeviceToHost) == hipSuccess) st |= all;      // (the host's word is the last code, the device's all of them)
     *e->h_status = 0;
     (void)hipMemsetAsync(e->tick + 1, 0, sizeof(unsigned), e->stream);
     (void)hipStreamSynchronize(e->stream);
-    e->fused = e->ly.on = false;
-    e->fused_retired = true;
-    if (e->turn_on) g_turns[e->dev].retire(e);
-    destroy_samp_graphs(e);
-    e->fail(NL_OK, "warning: a fused-launch cluster exchange timed out (status %u); the step was redone on the general plan, "
-                   "which this handle keeps from now on", st);
+    e->redo = true;
+    const bool layers = st >> LY_CODES, fused = (st & ((1u << LY_CODES) - 1)) || !layers;
+    if (fused) {
+        e->fused = false;
+        e->fused_retired = true;
+    }
+    if (layers && ++e->ly.give_ups >= LY_TRIES) {
+        e->ly.on = false;
+        if (e->turn_on) g_turns[e->dev].retire(e);
+    }
+    if (fused || !e->ly.on) destroy_samp_graphs(e);
+    e->fail(NL_OK, "warning: a %s's exchange timed out (status %u); the step was redone on the general plan%s", layers ? "layer launch" : "fused launch", st,
+            fused && !e->ly.on ? ", which this handle keeps from now on" : layers && e->ly.on ? " (the next call tries that launch again)" : ", and this handle does without that launch from now on");
     if (!getenv("NL_QUIET")) fprintf(stderr, "[nanollama_hip] %s\n", e->err.c_str());
     return true;
 }
@@ -3501,6 +3519,7 @@ int nl_forward(nl_handle e, int stream, int token, int pos, float *logits_out) {
     if (!e) return NL_ERR_INVALID;
     int rc = check_step_args(e, stream, token, pos);
     if (rc) return rc;
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     {
         // the smallest tier: the resident session takes the token (nl_persist.h: no launch, no weight fetch, the LM-head units
@@ -3556,6 +3575,7 @@ int nl_forward_argmax(nl_handle e, int stream, int token, int pos, int *next_id)
     if (!e || !next_id) return NL_ERR_INVALID;
     int rc = check_step_args(e, stream, token, pos);
     if (rc) return rc;
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     {
         bool served = false;
@@ -3601,6 +3621,7 @@ int nl_decode_greedy(nl_handle e, int stream, int token, int pos, int n_steps, i
     if (!e || !ids_out || n_steps < 0) return NL_ERR_INVALID;
     int rc = check_step_args(e, stream, token, pos);
     if (rc) return rc;
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     int n = std::min(n_steps, e->cfg.seq_len - pos);
@@ -3675,6 +3696,7 @@ int nl_sample_decode(nl_handle e, int stream, int pos, int n_steps, const nl_sam
     if (stream < 0 || stream >= e->cfg.max_streams) return e->fail(NL_ERR_INVALID, "stream %d out of range", stream);
     if (pos < 1 || pos > e->cfg.seq_len) return e->fail(NL_ERR_INVALID, "pos %d out of range [1,%d]", pos, e->cfg.seq_len);
     if (*n_recent < 0 || *n_recent > p->rep_window) return e->fail(NL_ERR_INVALID, "n_recent %d exceeds rep_window %d", *n_recent, p->rep_window);
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     int n = std::min(n_steps, e->cfg.seq_len - pos);
@@ -3810,6 +3832,7 @@ int nl_prefill(nl_handle e, int stream, const int *tokens, int n, int pos0, floa
     if (pos0 + n > e->cfg.seq_len) return e->fail(NL_ERR_INVALID, "prefill of %d tokens at pos %d exceeds seq_len %d", n, pos0, e->cfg.seq_len);
     for (int i = 0; i < n; i++)
         if (tokens[i] < 0 || tokens[i] >= e->cfg.vocab) return e->fail(NL_ERR_INVALID, "token %d out of range [0,%d)", tokens[i], e->cfg.vocab);
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     if ((rc = note_positions(e, stream, pos0, n))) return rc;
@@ -3869,6 +3892,7 @@ int nl_forward_batch(nl_handle e, const int *streams, const int *tokens, const i
             if (streams[j] == streams[i]) return e->fail(NL_ERR_INVALID, "stream %d appears twice in one batch", streams[i]);
     }
     if (n == 0) return NL_OK;
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     for (int i = 0; i < n; i++)
@@ -4061,6 +4085,7 @@ int nl_profile_forward(nl_handle e, int stream, int token, int pos, int iters, f
     if (!e || !ms_out || !calls_out || iters <= 0) return NL_ERR_INVALID;
     int rc = check_step_args(e, stream, token, pos);
     if (rc) return rc;
+    const RedoScope scope(e);
     HIPCK(e, hipSetDevice(e->dev));
     if (int qrc = pd_session_close(e)) return qrc;
     for (int k = 0; k < NL_NUM_KINDS; k++) { ms_out[k] = 0.f; calls_out[k] = 0; }

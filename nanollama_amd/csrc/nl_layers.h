@@ -24,7 +24,8 @@
 // own tag: whoever writes the next layer's granules has, through the phases between, waited for everyone who reads this layer's.
 // The K / V row of the step's position reaches the attention as granules; the unit that holds the position stores it.  Other units read rows
 // that earlier launches wrote.
-// Every poll is bounded; a give-up (some workgroup was not resident) sets the status words and the host redoes the step on the launch plans.
+// Every poll is bounded; a give-up (some workgroup was not resident) sets the status words and the host redoes the step on the launch plans (and, up to
+// three times, tries this launch again with the next call).
 //
 // Weights are requested by buffer loads whose range is empty where a wavefront has nothing to do: no branch around a load, so the compiler's
 // count of loads in flight holds across the phases.  They go out a quarter of a microsecond apart: all at once they stand before
@@ -43,6 +44,7 @@ constexpr int LY_PER_XCD = 32;             // a launch is one workgroup a comput
 static_assert(LY_TG == GPT, "granules of a tile");
 constexpr int LY_RELAY = 1;                // the exchanging wavefront that relays
 constexpr int LY_MAX_COLS = 2048, LY_MAX_FF = 4096;
+constexpr int LY_CODES = 16;               // this launch's status codes are above those of the other launches on the same word
 
 struct LayersEntry {                       // one layer: Q|K|V, WO, gate, up, down
     const uint8_t *q[5];
@@ -136,7 +138,7 @@ __device__ __forceinline__ bool ly_again(LyPoll &Q, int &spins, unsigned code, i
     if ((spins & 63) == 63) stop = stop || __builtin_amdgcn_readfirstlane((int)__hip_atomic_load(Q.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
     if (stop) {
         Q.dead = true;
-        if (lane == 0) { atomicOr(Q.status, code); *Q.host_status = code; *Q.lds_dead = 1; }
+        if (lane == 0) { atomicOr(Q.status, code << LY_CODES); *Q.host_status = code << LY_CODES; *Q.lds_dead = 1; }
         return false;
     }
     asm volatile("" ::: "memory");
@@ -344,7 +346,7 @@ __global__ void __launch_bounds__(LY_THREADS) layers_kernel(LayersParams P0) {
     xcd &= LY_XCDS - 1;
     if (tid == 0) {
         lds_dead = 0;
-        lds_slot = (int)(atomicAdd(P.tickets + xcd * (LY_LINE * 4), 1u) % LY_PER_XCD);      // (every launch adds 32: a launch that does not gives up, and is the handle's last)
+        lds_slot = (int)(atomicAdd(P.tickets + xcd * (LY_LINE * 4), 1u) % LY_PER_XCD);      // (32 of a launch have the 32 places, wherever the count stands)
     }
     for (int i = tid; i < P.L * LY_ENTRY; i += LY_THREADS) tab[i] = reinterpret_cast<const uint2 *>(P.layers)[i];
     const int pos = sload_i32(P.ctl + CTL_POS), strm = sload_i32(P.ctl + CTL_STREAM);

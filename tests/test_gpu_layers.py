@@ -116,3 +116,31 @@ def test_the_age_of_a_buffer_does_not_matter(tmp_path, monkeypatch, counter):
     assert dev.decode_greedy(5, 20, 40) == plain.decode_greedy(5, 20, 40)
     assert dev.last_error() == "" and dev.debug_read("layers_max_pos", 1)[0] > 0
     dev.close(); plain.close()
+
+
+# a launch that gives up (it met another process's on the card, say) is tried again; the plans that served its positions before outlive it
+@pytest.mark.parametrize("name,wtype,mode", [("middle", "q4_k", 0), ("variant", "q8_0", 1), ("middle", "q8_0", 4)])
+def test_three_give_ups(tmp_path, monkeypatch, name, wtype, mode):
+    monkeypatch.setenv("NL_FUSED_SPIN_LIMIT", "0")
+    monkeypatch.setenv("NL_QUIET", "1")
+    shape, dev, plain = _models(tmp_path, monkeypatch, name, wtype, seq_len=300)
+    toks = synth.prompt_ids(30, shape.vocab, seed=3)
+    for m in (dev, plain):
+        m.prefill(toks, want_logits=False)
+        m.reset()
+    state = lambda: (dev.debug_read("layers_max_pos", 1)[0], dev.plan_info()["fused_mode"])
+    assert state() == (300, mode) and dev.last_error() == ""
+    for m in (dev, plain):
+        m.forward(toks[0], 0)
+    assert np.array_equal(dev.state.logits, plain.state.logits)
+    assert state() == (300, mode) and "timed out" in dev.last_error() and "tries" in dev.last_error()
+    assert dev.decode_greedy(toks[1], 1, 37) == plain.decode_greedy(toks[1], 1, 37)
+    assert state() == (300, mode)
+    us = np.random.default_rng(9).random(20, dtype=np.float32)
+    assert dev.sample_decode(38, 20, 0.9, 0.9, 50, 1.15, 8, us, [3, 4]) == plain.sample_decode(38, 20, 0.9, 0.9, 50, 1.15, 8, us, [3, 4])
+    assert state() == (0, mode)                                 # ... the third
+    for m in (dev, plain):
+        m.forward(toks[5], 58)
+    assert np.array_equal(dev.state.logits, plain.state.logits)
+    assert state() == (0, 0)                                    # (a fused plan gave up as well, once)
+    dev.close(); plain.close()
