@@ -345,6 +345,9 @@ def run_workload(tier, wtype, rdv, steps, warmup, profile_pos, model, tp=True, c
         prof = dev.profile_forward(first, ppos, iters=20)
         wo_in_block = bool(prof.get("attn_block", (0, 0))[1]) and not prof.get("wo_resid", (0, 0))[1]
         kb = kernel_bytes(shape, wtype, ppos, tp=shard_of or world, wo_in_block=wo_in_block)
+        layers = dev.layers_info()
+        if layers["min_pos"] <= ppos < layers["max_pos"]:      # (that launch is filed under ffn_block: all layers of the step)
+            kb["ffn_block"] = shape.n_layer * sum(kb[k] for k in ("qkv_rope", "attention", "wo_resid", "gate_up_swiglu", "down_resid"))
         kernels = {}
         for kind, (ms, calls) in prof.items():
             if calls:
@@ -417,7 +420,7 @@ def run_workload(tier, wtype, rdv, steps, warmup, profile_pos, model, tp=True, c
             "tier": tier, "wtype": wtype, "path": path, "prompt": prompt,
             "tok_s": replicas * steps / (wall_ms / 1e3), "ms_per_step": ms_per_step, "device_ms_per_step": evs[med] / steps,
             "ms_per_step_min": min(walls) / steps, "ms_per_step_max": max(walls) / steps,
-            "replicas": replicas, "tp": world, "p2p": p2p, "plan": dev.plan_info(),
+            "replicas": replicas, "tp": world, "p2p": p2p, "plan": dict(dev.plan_info(), layers=dev.layers_info()),
             "step_bytes": int(step_bytes), "hbm_frac_whole_step": step_gbs / (HBM_PEAK_GBS * max(world, 1)),
             "kernels": kernels, "last_ids": ids[-4:], "head_ids": head_ids, "first_id": first, "prefill_logits": prefill_logits,
             "dropin": (dropin_rates(dev, first, pos0, 64 if tier != "big" else 32, head_ids) if dropin and world == 1 and not shard_of else None),

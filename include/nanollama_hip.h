@@ -174,7 +174,8 @@ NL_API int nl_timer_stop(nl_handle h, float *ms);
 /* Per-kernel-kind device time of one eager Forward (events around every
  * launch, each replayed `iters` times).  kinds: see nl_kernel_kind_name.  ms_out/calls_out have NL_NUM_KINDS
  * entries.  Measurement only: the replays leave x, the logits and the K/V rows at `pos` in a state no Forward
- * produces, so the stream's positions >= pos count as unwritten afterwards (re-run them before decoding on). */
+ * produces, so the stream's positions >= pos count as unwritten afterwards (re-run them before decoding on).
+ * A step whose layers are one launch (nl_layers_info) has that launch under "ffn_block", one call, and no other layer kind. */
 #define NL_NUM_KINDS 11
 NL_API const char *nl_kernel_kind_name(int kind);
 NL_API int nl_profile_forward(nl_handle h, int stream, int token, int pos, int iters, float *ms_out, int *calls_out);
@@ -182,8 +183,11 @@ NL_API int nl_profile_forward(nl_handle h, int stream, int token, int pos, int i
  * general five-launches-per-layer plan; 1 = small tiers, attention block + feed-forward block (2 per layer); 2 = wide
  * tiers, projection + attention fused (4 per layer); 3 = a tensor-parallel rank's layer as two launches with the push
  * all-reduce finished in their tails; 4 = wide tiers on one GPU, projection + attention + WO fused (3 per layer).  fused_max_pos: steps below this position take the fused plan.  launches_*: kernel
- * launches per token of the fused / general plan (0 when the plan does not exist). */
+ * launches per token of the fused / general plan (0 when the plan does not exist).  Positions of nl_layers_info take neither. */
 NL_API int nl_plan_info(nl_handle h, int *fused_mode, int *fused_max_pos, int *launches_fused, int *launches_general);
+/* Steps at positions [min_pos, max_pos) run all layers in one launch; launches: kernel launches per token there (all 0: the
+ * handle has no such plan, or its exchanges timed out three times). */
+NL_API int nl_layers_info(nl_handle h, int *min_pos, int *max_pos, int *launches);
 /* The weight-stationary persistent decode of the smallest tier (nl_persist.h; no reference counterpart, the Go loop is
  * go/main.go:173-219): ready = nl_decode_greedy takes ONE launch per chunk while the chunk ends below max_pos (Q8_0 files of
  * nano's shape class on a 256-CU device), and consecutive nl_forward / nl_forward_argmax calls below max_pos are steps of
@@ -196,8 +200,9 @@ NL_API int nl_memory_usage(nl_handle h, uint64_t *weights, uint64_t *kv_cache, u
  * "k_cache","v_cache"), or, as one float, which kernels the last multi-token step
  * ran on ("step_path": 1 | 2 decode-batch / short-step GEMM, 4 | 8 attention of a
  * prompt / of a decode batch in one launch, 16 its images from the projections, 32
- * folded norms, 64 decode attention with eight wavefronts; "num_cus": the
- * device's compute units; layer-stack models "one_query": layers
+ * folded norms, 64 decode attention with eight wavefronts, 128 | 256 a prompt's attention
+ * / products on 16 rows a workgroup; "num_cus": the
+ * device's compute units; "forwards": the fused launches' counter; layer-stack models "one_query": layers
  * whose queries took one launch, "prompt_tiles": the tiles of a prompt's products,
  * "splits": key-range splits of the last decode step);
  * returns floats copied (<= max_floats). */

@@ -217,6 +217,12 @@ class LlamaModel(HipModel):
         self._check(self._L.nl_plan_info(self._h, *[C.byref(x) for x in v]))
         return {"fused_mode": v[0].value, "fused_max_pos": v[1].value, "launches_fused": v[2].value, "launches_general": v[3].value}
 
+    def layers_info(self):
+        """nl_layers_info: positions whose steps run all layers in one launch, and launches per token there."""
+        v = [C.c_int(0) for _ in range(3)]
+        self._check(self._L.nl_layers_info(self._h, *[C.byref(x) for x in v]))
+        return {"min_pos": v[0].value, "max_pos": v[1].value, "launches": v[2].value}
+
     def persist_info(self):
         """nl_persist_info: is the one-launch-per-chunk persistent decode (nl_persist.h) serving greedy chains of this handle."""
         ready, max_pos = C.c_int(0), C.c_int(0)

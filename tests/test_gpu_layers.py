@@ -144,3 +144,21 @@ def test_three_give_ups(tmp_path, monkeypatch, name, wtype, mode):
     assert np.array_equal(dev.state.logits, plain.state.logits)
     assert state() == (0, 0)                                    # (a fused plan gave up as well, once)
     dev.close(); plain.close()
+
+
+# a replay without a forward of its own finds every granule already there, and what it times leaves the exchanges out
+def test_profiled_replays_are_forwards(tmp_path, monkeypatch):
+    shape, dev, plain = _models(tmp_path, monkeypatch, "middle", "q8_0", seq_len=300)
+    assert dev.layers_info() == {"min_pos": 0, "max_pos": 300, "launches": 4} and plain.layers_info() == {"min_pos": 0, "max_pos": 0, "launches": 0}
+    toks = synth.prompt_ids(20, shape.vocab, seed=3)
+    for m in (dev, plain):
+        m.prefill(toks, want_logits=False)
+    before = dev.debug_read("forwards", 1)[0]
+    kinds = {k: c for k, (ms, c) in dev.profile_forward(5, 20, iters=7).items() if c}
+    assert kinds == {"embed": 1, "ffn_block": 1, "lm_head": 1, "argmax": 1}
+    assert dev.debug_read("forwards", 1)[0] - before == 1 + 7 + 7           # one ahead, the embed launch's replays, the layer launch's
+    assert dev.last_error() == ""
+    for m in (dev, plain):
+        m.forward(5, 20)
+    assert np.abs(dev.state.logits - plain.state.logits).max() <= 1e-4 * max(1.0, float(plain.state.logits.std()))
+    dev.close(); plain.close()
