@@ -777,9 +777,12 @@ void build_plan_blocks(nl_engine *e, std::vector<Op> &plan) {
 // Models and positions whose steps gain by nl_layers.h.  Its start (pointers into LDS, the first weights cold) costs as much as two layers gain: 2 layers of
 // 1024 columns 56.5 -> 54.5 us a token in Q8_0 and 49.0 -> 51.8 in Q4_0, four 97.2 -> 86.4 and 87.7 -> 83.7, sixteen 338 -> 284 and 307 -> 273,
 // 28 of 1536 747 -> 576 and 633 -> 546 (position 130; 400: 775 -> 590 and 696 -> 559).  Against two launches a layer (mode 1) it loses while their
-// attention is at its first or second pass: 20 layers of 768 columns 313 -> 328 us at position 140, 323 -> 331 at 230, 349 -> 334 at 256, 384 -> 334 at 400.
+// attention is at its first or second pass, models of fewer than eight layers also at the third: at positions 140 / 260 / 380, four layers of 256 columns 67 and 73 /
+// 70 and 73 / 75 and 73 us, of 384 65 and 73 / 72 and 74 / 77 and 74, of 768 73 and 80 / 80 and 80, six of 256 at 260 / 380 101 and 102 / 109 and 101; eight of 512 126
+// and 132 / 139 and 133, twelve of 384 179 and 191 / 200 and 193, twenty of 768 313 and 328 / 349 and 334, thirty of 576 443 and 468 / 496 and 474.  The other modes
+// gain from position 0 on, 4 - 12 layers of 1024 - 2048 columns 3 - 30 % (four of 2048 in Q4_0 94 and 91, at 140 94 and 95), K-quants of 256 - 1536 8 - 24 %.
 bool layers_pay(const nl_engine *e) { return e->cfg.n_layers >= 4; }
-int layers_min_pos(const nl_engine *e) { return e->fused_mode == 1 ? 2 * LY_PASS : 0; }
+int layers_min_pos(const nl_engine *e) { return e->fused_mode == 1 ? (e->cfg.n_layers < 8 ? 3 : 2) * LY_PASS : 0; }
 
 // nl_layers.h: embed -> all layers -> lm_head -> argmax
 void build_plan_layers(nl_engine *e, std::vector<Op> &plan) {

@@ -162,3 +162,14 @@ def test_profiled_replays_are_forwards(tmp_path, monkeypatch):
         m.forward(5, 20)
     assert np.abs(dev.state.logits - plain.state.logits).max() <= 1e-4 * max(1.0, float(plain.state.logits.std()))
     dev.close(); plain.close()
+
+
+@pytest.mark.parametrize("layers,dim,heads,min_pos", [(4, 256, 4, 384), (7, 256, 4, 384), (8, 256, 4, 256), (4, 1024, 16, 0)])
+def test_where_the_launch_takes_over(tmp_path, monkeypatch, layers, dim, heads, min_pos):
+    from nanollama_amd import model as hip
+    monkeypatch.delenv("NL_LAYERS", raising=False)
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("rule", layers, dim, heads, 2, 512, seq_len=512, interm=1024), "q8_0", 5, mode="qrand")
+    m = hip.load_llama_model(gguf.load_gguf(str(p)))
+    assert m.layers_info()["min_pos"] == min_pos and m.layers_info()["max_pos"] == 512
+    m.close()
