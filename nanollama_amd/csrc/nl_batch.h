@@ -581,11 +581,7 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
 
     const int kvh = blockIdx.x, split = blockIdx.y, i0 = blockIdx.z * QT, tid = threadIdx.x;
     const int t0 = split * ATT_CH;
-    int maxpos = -1;
-    if (P.pos_base_valid) maxpos = P.pos_base + min(i0 + QT, n_items) - 1;      // a prompt: consecutive positions, nothing to read
-    else
-        for (int i = 0; i < QT; i++)
-            if (i0 + i < n_items) maxpos = max(maxpos, P.bpos[i0 + i]);
+    const int maxpos = P.pos_base + min(i0 + QT, n_items) - 1;      // a prompt: consecutive positions, nothing to read
     if (t0 > maxpos) return;
     const int nrows = min(ATT_CH, maxpos + 1 - t0);
     const int lane = tid & 63, w = tid >> 6, j = lane & 15, kq = lane >> 4;
@@ -607,9 +603,8 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
             for (int s = 0; s < DK; s++) qa[s] = 0.f;
         }
     }
-    const long long soff = P.single_stream ? 0 : (long long)P.bstream[i0] * P.kv_stream_stride;
-    const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
-    const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
+    const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + ((long long)kvh * P.seq_len + t0) * HD);
+    const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + ((long long)kvh * P.seq_len + t0) * HD);
     // every global load of the staging pass is issued before the first LDS store (one memory latency, not NIT).
     // Key tiles are computed two at a time and only where a row of the workgroup can see one (uniform tests: masked probabilities are zeros, so
     // the sums are the same bits); rows beyond nrows of the last two are zero-filled (masked to p = 0 by the softmax, and 0 * garbage could be
@@ -636,7 +631,7 @@ __global__ void __launch_bounds__(QT * G * 4, 2) attn_tile_kernel(AttnParams P, 
     }
     if (tid < VH) {
         const int item = i0 + tid / G;
-        nv[tid] = item < n_items ? min(ATT_CH, max(0, (P.pos_base_valid ? P.pos_base + item : P.bpos[item]) + 1 - t0)) : 0;
+        nv[tid] = item < n_items ? min(ATT_CH, max(0, P.pos_base + item + 1 - t0)) : 0;
     }
     __syncthreads();
 
@@ -1078,17 +1073,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 && !ALONE ? 4 : 2) a
     const int split = P.live_map ? ((code >> 12) & 15) : (int)blockIdx.y;           // partial slot
     const int c_first = P.live_map ? ((code >> 6) & 63) : (int)blockIdx.y;
     int c_count = P.live_map ? (code & 63) : 1;
-    int maxpos = -1, minpos = 0x7fffffff;
-    if (P.pos_base_valid) {   // a prompt: consecutive positions, nothing to read
-        minpos = P.pos_base + i0;
-        maxpos = P.pos_base + min(i0 + QT, n_items) - 1;
-    } else {
-        for (int i = 0; i < QT; i++) {
-            const int pp = i0 + i < n_items ? P.bpos[i0 + i] : -1;
-            maxpos = max(maxpos, pp);
-            minpos = min(minpos, pp);
-        }
-    }
+    const int minpos = P.pos_base + i0, maxpos = P.pos_base + min(i0 + QT, n_items) - 1;      // a prompt: consecutive positions, nothing to read
     if (c_first * ATT_CH > maxpos) return;
     c_count = min(c_count, maxpos / ATT_CH + 1 - c_first);
     const int lane = tid & 63, w = tid >> 6, j = lane & 15, kq = lane >> 4;
@@ -1131,7 +1116,7 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 && !ALONE ? 4 : 2) a
         for (int k = 0; k < 2 * NKS; k++) qraw[k] = *reinterpret_cast<const float4 *>(qp + 32 * (k >> 1) + 4 * (k & 1));
         if (tid < VH) {
             const int it = i0 + tid / G;
-            row_pos = it < n_items ? (P.pos_base_valid ? P.pos_base + it : P.bpos[it]) + 1 : 0;
+            row_pos = it < n_items ? P.pos_base + it + 1 : 0;
         }
     };
     auto q_split = [&]() __attribute__((always_inline)) {
@@ -1152,7 +1137,6 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 && !ALONE ? 4 : 2) a
         q_split();
         if (tid < VH) npos[tid] = row_pos;
     }
-    const long long soff = P.single_stream ? 0 : (long long)sload_i32(P.bstream + i0) * P.kv_stream_stride;
     constexpr float LOG2E = 1.44269504088896340736f, LN2 = 0.69314718055994530942f;
     typedef float v2f __attribute__((ext_vector_type(2)));
     const float c2 = P.scale * LOG2E;
@@ -1171,8 +1155,8 @@ __global__ void __launch_bounds__(QT * G * 4, QT * G >= 128 && !ALONE ? 4 : 2) a
             dma_landed();                              // this wavefront's pieces of the chunk (issued a chunk ago)
             ATT_STAMP(10 * c + 1);
         } else {
-            const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
-            const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + soff + ((long long)kvh * P.seq_len + t0) * HD);
+            const float4 *K4 = reinterpret_cast<const float4 *>(P.kcache + ((long long)kvh * P.seq_len + t0) * HD);
+            const float4 *V4 = reinterpret_cast<const float4 *>(P.vcache + ((long long)kvh * P.seq_len + t0) * HD);
             kv16_stage<HD, NTH, true>(K4, V4, nrows, tid, Kh, Kl, VTh, VTl, c > 0);
             if (ALONE && c == 0 && tid < VH) npos[tid] = row_pos;
         }

@@ -213,7 +213,7 @@ struct nl_engine {
         int cap = 0, lm_cap = 0;
         uint4 *xfrag = nullptr;  // fp16 hi/lo activation fragments of the GEMM being run
         uint4 *xfrag2 = nullptr; // second store: output of the fused gate/up/SwiGLU GEMM, input of down
-        double *ssq = nullptr;   // [cap][dim / 64] sums of squares of the residual rows (RMSNorm folded around the prompt GEMMs)
+        double *ssq = nullptr;   // [cap][dim / 64; slim tiles: / 16, dgemm_kernel: / 32] sums of squares of the residual rows (RMSNorm folded around the prompt GEMMs)
         float *nscale = nullptr; // [2][cap] per-token power-of-two pre-scales of the folded norm's fragments (norm_prescale, nl_qgemm.h)
         float *kpart = nullptr, *kpart2 = nullptr;  // split-K partial sums (second buffer: up, alive beside gate)
         size_t kpart_cap = 0;    // floats, each
@@ -2168,6 +2168,7 @@ hipError_t launch_qgemm_plain(nl_engine *e, nl_engine::Batch &bt, const PackedMa
 
 // One multi-token step: n <= 64 (token, pos, stream) triples through every layer on the MFMA path.
 // lm_mode: 0 = no LM head, 1 = logits + argmax for every token, 2 = logits + argmax for the LAST token only, in e->logits / e->result (to_host: and the pinned buffer).
+// one_stream: a prompt, consecutive positions of one stream (nl_prefill).
 // The caller has filled bt.h_meta; stream-ordered, no synchronisation inside.
 int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int lm_mode, bool one_stream = false, bool to_host = false) {
     const nl_config &c = e->cfg;
@@ -2184,8 +2185,7 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const bool f32_tile = attn_knobs().f32_tile || exact;
     auto form = [&](const PackedMat &next) { return (next.wtype == WT_Q4_0 ? FRAG_Q4_0 : 0) | (exact ? FRAG_EXACT : 0); };
     {
-        bool cons = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !f32_tile && !attn_knobs().no_tile;
-        for (int i = 1; i < n && cons; i++) cons = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
+        const bool cons = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !f32_tile && !attn_knobs().no_tile;
         const int kv16_min = getenv("NL_KV16_MIN_TOKENS") ? atoi(getenv("NL_KV16_MIN_TOKENS")) : 256;   // (read per step: a test lowers it)
         kv16_on = cons && n >= kv16_min && b.kv16 != nullptr;
         const int qt = attn_tile16_qt(e->gqa) * (kv16_on ? 2 : 1), ntile = (n + qt - 1) / qt, p0 = b.h_meta[b.cap];
@@ -2233,12 +2233,10 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
     const bool no_tile = attn_knobs().no_tile, no_fin = getenv("NL_NO_ATTN_FIN") != nullptr;   // (no_fin: knob of tests, read per step: the merge launch always)
     int nsplit = 1;
     for (int i = 0; i < n; i++) nsplit = std::max(nsplit, b.h_meta[b.cap + i] / ATT_CH + 1);
-    bool consecutive = true;   // positions pos0, pos0 + 1, ...: a prompt
-    for (int i = 1; i < n && consecutive; i++) consecutive = b.h_meta[b.cap + i] == b.h_meta[b.cap] + i;
     nsplit = std::min(nsplit, e->nsplit_max);
     const bool tile_attn = one_stream && n >= 8 && attn_tile_supported(e->gqa) && !no_tile;   // prompts: attn_tile16_kernel
     // ... a partial per 128 positions: nothing about them to read in the launches
-    const bool by_chunk = tile_attn && consecutive && (f32_tile || (n_live > 0 && run == 1 && !kv16_on));
+    const bool by_chunk = tile_attn && (f32_tile || (n_live > 0 && run == 1 && !kv16_on));
     // attn_rows_kernel: while its workgroups, one per 16 rows and chunk that they see, find two to a compute unit at once.  us a prompt of K-quants, tiles and rows:
     // 173M, 100 tokens 1091 and 1003 (42 workgroups a kv head), 330 1454 and 1386 (459 in all), 128 behind 300 1169 and 1124 (320), 200 behind 300 1278 and 1295
     // (525); 841M, 100 tokens 2258 and 2122, 200 2997 and 2931 (408); 4096 columns, 128 tokens 1205 and 1216 (512).  NL_ATTN_ROWS=0 (knob of tests, read per step): never
@@ -2371,8 +2369,6 @@ int batched_step(nl_engine *e, nl_engine::Batch &b, hipStream_t st, int n, int l
                 // (the prompt's stream is known here)
                 const long long so = c.max_streams == 1 ? 0 : (long long)b.h_meta[2 * b.cap] * e->kv_stream_stride;
                 T.kcache = kc + so; T.vcache = vc + so;
-                T.single_stream = 1;
-                T.pos_base_valid = consecutive ? 1 : 0;   // (a prompt: the kernel derives its key range without reading bpos)
                 T.pos_base = b.h_meta[b.cap];
                 T.live_map = n_live > 0 && !by_chunk ? b.tok + 3 * b.cap : nullptr;
                 if (rows) e->step_path |= PATH_ATTN_ROWS;

@@ -1112,10 +1112,10 @@ struct AttnParams {
     uint4 *fin_xf;
     int fin_nt16, fin_form;
     int x1;   // attn_tile16_kernel: prompt precision mode fp16x1 -- one fp16 product per q.k and p.v term instead of hi*hi + lo*hi + hi*lo
-    // attn_tile16_kernel: the step's positions are pos_base + item (a prompt) when pos_base_valid -- the workgroup then
-    // knows its key range without reading bpos, and its K / V requests leave at entry
-    int pos_base_valid, pos_base;
-    // ... and the launch is COMPACT then: blockIdx.x indexes the host-built list of workgroups, each a kv head, a query tile
+    // prompts (attn_tile_kernel, attn_rows_kernel, attn_tile16_kernel): the step's positions are pos_base + item and kcache / vcache are its stream's -- a
+    // workgroup knows its key range without reading bpos, and its K / V requests leave at entry
+    int pos_base;
+    // ... and the launch is COMPACT where runs are longer than a chunk: blockIdx.x indexes the host-built list of workgroups, each a kv head, a query tile
     // and a run of consecutive 128-key chunks under the causal diagonal (kv head << 24 | tile << 16 | partial slot << 12 |
     // first chunk << 6 | chunks) instead of a tiles x chunks grid half of whose workgroups -- the ones above the diagonal --
     // are dispatched, given LDS and exit.  The list is ordered so that the two workgroups of a CU (i and i + #CUs, measured)

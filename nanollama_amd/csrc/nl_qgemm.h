@@ -92,12 +92,12 @@ struct QGemmParams {
     struct NormOut {
         const float *w;      // [rows] norm weights of the consuming GEMM; nullptr = not folded
         uint4 *xf;           // fragment store the consumer reads
-        double *ssq;         // [n_tokens][rows / 64]
+        double *ssq;         // [n_tokens][rows / 64; slim tiles: / 16, dgemm_kernel: / 32]
         const float *scale;  // [n_tokens] exact power of two the fragments are multiplied by (norm_prescale below); nullptr = 1
     } nrm_out;               // (k-slot order of the consumer's weight type: out_q4)
     struct NormIn {
         const double *ssq;   // nullptr = the input fragments are already normalised
-        int nrb;             // partial sums per token (dim / 64)
+        int nrb;             // partial sums per token
         int dim;
         float eps;
         const float *scale;  // the power of two the producer multiplied this token's fragments by (undone through inv); nullptr = 1
