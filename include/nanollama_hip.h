@@ -202,7 +202,9 @@ NL_API int nl_memory_usage(nl_handle h, uint64_t *weights, uint64_t *kv_cache, u
  * prompt / of a decode batch in one launch, 16 its images from the projections, 32
  * folded norms, 64 decode attention with eight wavefronts, 128 | 256 a prompt's attention
  * / products on 16 rows a workgroup; "num_cus": the
- * device's compute units; "forwards": the fused launches' counter; layer-stack models "one_query": layers
+ * device's compute units; "forwards": the fused launches' counter; "plan": what the
+ * last single-token step ran on, 0 the general plan, 1 | 2 a fused one, 3 all layers in
+ * one launch, 4 the persistent launch; layer-stack models "one_query": layers
  * whose queries took one launch, "prompt_tiles": the tiles of a prompt's products,
  * "splits": key-range splits of the last decode step);
  * returns floats copied (<= max_floats). */

@@ -241,6 +241,7 @@ struct nl_engine {
     bool dg_head = false;         // ... and the LM head has one too (decode batches: dgemm_kernel with the argmax candidates in its epilogue)
     std::vector<SubBatch::G> bt_graphs;   // step graphs of the whole-batch decode step (bt), same key
     hipEvent_t sub_fork = nullptr;
+    int last_plan = -1;           // the plan of the last single-token step or chain (nl_debug_read "plan")
     int step_path = 0;            // launches of the last multi-token step (PATH_* bits; nl_debug_read "step_path")
     int sub_batches = 1;          // NL_SUB_BATCHES: groups a decode batch is cut into (1 = the whole batch as one step: measured fastest, profiles/r04_subbatch_groups.log)
 
@@ -1220,10 +1221,13 @@ void destroy_graphs(nl_engine::PlanSet &S) {
     if (S.graph) { (void)hipGraphDestroy(S.graph); S.graph = nullptr; }
 }
 
+constexpr int PLAN_LAYERS = 3, PLAN_PERSIST = 4;      // ps[3]; nl_persist.h
 // nl_turns.h.  One per device
 Turns<nl_engine> g_turns[64];
-template <class F> int chip_turn(nl_engine *e, bool waits, F launch) {
-    if (!e->turn_on || !waits) return launch();
+// a launch of plan `plan` (ps[0]: workgroups that wait for nobody)
+template <class F> int chip_turn(nl_engine *e, int plan, F launch) {
+    e->last_plan = plan;
+    if (!e->turn_on || plan == 0) return launch();
     return g_turns[e->dev].run(e, launch,
         [&](nl_engine *o) -> int { HIPCK(e, hipStreamWaitEvent(e->stream, o->turn_done, 0)); return NL_OK; },
         [&]() -> int { HIPCK(e, hipEventRecord(e->turn_done, e->stream)); return NL_OK; });
@@ -1311,7 +1315,6 @@ void destroy_samp_graphs(nl_engine *e) {
     }
 }
 
-constexpr int PLAN_LAYERS = 3;
 // the plan that serves a step (or a run of steps) whose highest position is pos_last
 // (ps[2]: the fused plan of the wide tier on one GPU from the second attention pass on -- its attention launch is the variant
 //  whose passes are shared by helper blocks, nl_tp.h; the first pass keeps the launch compiled without them: 0.7 us per layer)
@@ -1325,7 +1328,7 @@ int plan_index(const nl_engine *e, int pos_last) {
 int launch_step(nl_engine *e, int pos) {
     const int k = plan_index(e, pos);
     nl_engine::PlanSet &S = e->ps[k];
-    return chip_turn(e, k > 0, [&]() -> int {
+    return chip_turn(e, k, [&]() -> int {
         if (S.exec) {
             HIPCK(e, hipGraphLaunch(S.exec, e->stream));
             return NL_OK;
@@ -1345,7 +1348,7 @@ bool call_step(nl_engine *e, int token, int pos, int stream, int hostout, int *i
     e->h_box[CTL_TOKEN] = token; e->h_box[CTL_POS] = pos; e->h_box[CTL_CHAIN] = 0; e->h_box[CTL_STEP] = 0;
     e->h_box[CTL_STREAM] = stream; e->h_box[CTL_HOSTOUT] = hostout;
     __atomic_store_n(e->h_box + 8, (int)seq, __ATOMIC_RELEASE);
-    *rc = chip_turn(e, k > 0, [&]() -> int {
+    *rc = chip_turn(e, k, [&]() -> int {
         if (hipGraphLaunch(S.call_exec, e->stream) != hipSuccess) return e->fail(NL_ERR_HIP, "hipGraphLaunch (call graph): %s", hipGetErrorString(hipGetLastError()));
         return NL_OK;
     });
@@ -1608,7 +1611,7 @@ int pd_launch(nl_engine *e, int stream, int token, int pos, int n, float *host_l
     P.gx = d.gx; P.gqkv = d.gqkv; P.go = d.go; P.gxp = d.gxp; P.gh = d.gh; P.gam = d.gam; P.gpart = d.gpart;
     P.ids_out = e->ids; P.logits = e->logits; P.host_logits = host_logits;
     P.status = d.status; P.host_status = d.h_status; P.dbg = d.dbg;
-    const int rc = chip_turn(e, true, [&]() -> int {
+    const int rc = chip_turn(e, PLAN_PERSIST, [&]() -> int {
         if (c.dim == 576 && c.n_kv_heads == 9) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 9>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
         else if (c.dim == 576) hipLaunchKernelGGL((pd_decode_kernel<18, 48, 3>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
         else if (c.n_kv_heads == 4) hipLaunchKernelGGL((pd_decode_kernel<8, 16, 4>), dim3(PD_GRID), dim3(PD_THREADS), pd_lds_bytes(), e->stream, P);
@@ -3646,7 +3649,7 @@ int nl_decode_greedy(nl_handle e, int stream, int token, int pos, int n_steps, i
                 const int k = plan_index(e, p0 + i + e->graph_steps - 1);   // highest position of these steps
                 nl_engine::PlanSet &S = e->ps[k];
                 if (!S.multi_exec) break;
-                if ((rc = chip_turn(e, k > 0, [&]() -> int { HIPCK(e, hipGraphLaunch(S.multi_exec, e->stream)); return NL_OK; }))) return rc;
+                if ((rc = chip_turn(e, k, [&]() -> int { HIPCK(e, hipGraphLaunch(S.multi_exec, e->stream)); return NL_OK; }))) return rc;
             }
             for (; i < m; i++)
                 if ((rc = launch_step(e, p0 + i))) return rc;
@@ -3767,7 +3770,7 @@ int nl_sample_decode(nl_handle e, int stream, int pos, int n_steps, const nl_sam
                     break;
                 }
             }
-            if ((rc = chip_turn(e, k > 0, [&]() -> int { HIPCK(e, hipGraphLaunch(e->samp_graph_exec[k], e->stream)); return NL_OK; }))) return rc;
+            if ((rc = chip_turn(e, k, [&]() -> int { HIPCK(e, hipGraphLaunch(e->samp_graph_exec[k], e->stream)); return NL_OK; }))) return rc;
             i += e->graph_steps;
         }
         for (; i < n; i++) {
@@ -4092,18 +4095,18 @@ int nl_profile_forward(nl_handle e, int stream, int token, int pos, int iters, f
     if ((rc = note_positions(e, stream, pos, 1))) return rc;
     if ((rc = set_ctl(e, token, pos, 0, stream))) return rc;
     int k = plan_index(e, pos);                          // the plan a step at this position runs
-    if ((rc = chip_turn(e, k > 0, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
+    if ((rc = chip_turn(e, k, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
     HIPCK(e, hipStreamSynchronize(e->stream));
     if (take_fused_timeout(e)) {
         k = plan_index(e, pos);
-        if ((rc = chip_turn(e, k > 0, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
+        if ((rc = chip_turn(e, k, [&]() -> int { return run_plan_eager(e, e->ps[k]); }))) return rc;
         HIPCK(e, hipStreamSynchronize(e->stream));
     }
     for (const Op &op : e->ps[k].ops) {
         // The layer launch's waits are for granules of its own forward: without a new one, all of them are there before it starts and no wait is in the time.
         // Its replays come with the embed launch, which counts forwards (and sets the residual stream), and that launch's time is taken off
         const bool counted = k == PLAN_LAYERS && op.kind == K_FFNBLOCK;
-        rc = chip_turn(e, k > 0, [&]() -> int {
+        rc = chip_turn(e, k, [&]() -> int {
             HIPCK(e, hipEventRecord(e->ev0, e->stream));
             for (int it = 0; it < iters; it++) {
                 hipError_t s = counted ? e->ps[k].ops[0].fn(e->stream) : hipSuccess;
@@ -4181,6 +4184,7 @@ int64_t nl_debug_read(nl_handle e, const char *which, int stream, float *out, in
     if (w == "num_cus") { if (max_floats < 1) return 0; out[0] = (float)e->num_cus; return 1; }
     if (w == "layers_max_pos") { if (max_floats < 1) return 0; out[0] = e->ly.on ? (float)e->ly.max_pos : 0.f; return 1; }      // (host state)
     if (w == "step_path") { if (max_floats < 1) return 0; out[0] = (float)e->step_path; return 1; }      // (host state)
+    if (w == "plan") { if (max_floats < 1) return 0; out[0] = (float)e->last_plan; return 1; }      // (host state)
     if (w == "forwards") {                   // the fused launches' counter
         unsigned c = 0;
         if (max_floats < 1 || !e->tick) return 0;

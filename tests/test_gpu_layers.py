@@ -173,3 +173,76 @@ def test_where_the_launch_takes_over(tmp_path, monkeypatch, layers, dim, heads, 
     m = hip.load_llama_model(gguf.load_gguf(str(p)))
     assert m.layers_info()["min_pos"] == min_pos and m.layers_info()["max_pos"] == 512
     m.close()
+
+
+def _plan(m):
+    return int(m.debug_read("plan", 1)[0])
+
+
+# two launches a layer below position 256, one launch for all from there on: what ran on both sides, and a greedy chain across against the handle that keeps the former
+def test_the_launch_takes_over_within_a_chain(tmp_path, monkeypatch):
+    from nanollama_amd import model as hip
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("over", 8, 768, 12, 3, 512, seq_len=400, interm=2048), "q8_0", 97, mode="qrand")
+    g = gguf.load_gguf(str(p))
+    monkeypatch.delenv("NL_LAYERS", raising=False)
+    dev = hip.load_llama_model(g)
+    monkeypatch.setenv("NL_LAYERS", "0")
+    blocks = hip.load_llama_model(g)
+    assert dev.layers_info()["min_pos"] == 256 and blocks.plan_info()["fused_mode"] == 1
+    toks = synth.prompt_ids(400, 512, seed=4)
+    for m in (dev, blocks):
+        m.prefill(toks[:254], want_logits=False)
+    for pos, plan in ((254, 1), (255, 1), (256, 3), (257, 3)):
+        for m in (dev, blocks):
+            m.forward(toks[pos], pos)
+        assert (_plan(dev), _plan(blocks)) == (plan, 1), pos
+        assert np.abs(dev.state.logits - blocks.state.logits).max() <= 1e-4 * max(1.0, float(blocks.state.logits.std())), pos
+    ids = [m.decode_greedy(7, 200, 150) for m in (dev, blocks)]
+    assert ids[0] == ids[1] and (_plan(dev), _plan(blocks)) == (3, 1)
+    dev.close(); blocks.close()
+
+
+# more positions than units for them: 20 kv heads have 12 of 128 positions each, and the launch ends there
+def test_the_launch_ends_below_the_context(tmp_path, monkeypatch):
+    from nanollama_amd import model as hip
+    p = tmp_path / "m.gguf"
+    synth.generate_gguf(str(p), synth.ModelShape("ends", 2, 1280, 20, 20, 512, seq_len=2048, interm=1024), "q8_0", 98, mode="qrand")
+    g = gguf.load_gguf(str(p))
+    monkeypatch.setenv("NL_LAYERS", "2")
+    monkeypatch.setenv("NL_FUSED_MAX_POS", "0")
+    dev = hip.load_llama_model(g)
+    monkeypatch.setenv("NL_LAYERS", "0")
+    monkeypatch.setenv("NL_FUSED_ATTN", "0")
+    plain = hip.load_llama_model(g)
+    assert dev.layers_info()["max_pos"] == 1536
+    toks = synth.prompt_ids(2048, 512, seed=4)
+    for m in (dev, plain):
+        m.prefill(toks[:1534], want_logits=False)
+    for pos, plan in ((1534, 3), (1535, 3), (1536, 0), (1537, 0)):
+        for m in (dev, plain):
+            m.forward(toks[pos], pos)
+        assert _plan(dev) == plan, pos
+        assert np.abs(dev.state.logits - plain.state.logits).max() <= 1e-4 * max(1.0, float(plain.state.logits.std())), pos
+    assert dev.decode_greedy(7, 1500, 60) == plain.decode_greedy(7, 1500, 60)
+    assert dev.last_error() == ""
+    dev.close(); plain.close()
+
+
+@pytest.mark.parametrize("name,wtype", [("middle", "q8_0"), ("wide_groups", "q4_0"), ("eight_to_one", "q4_k"), ("middle", "q6_k")])
+def test_every_call_runs_on_the_launch(tmp_path, monkeypatch, name, wtype):
+    shape, dev, plain = _models(tmp_path, monkeypatch, name, wtype, seq_len=300)
+    for m, plan in ((dev, 3), (plain, 0)):
+        m.prefill([5, 6])
+        assert _plan(m) == plan
+        m.forward(7, 2)
+        assert _plan(m) == plan
+        m.forward_argmax(8, 3)
+        assert _plan(m) == plan
+        m.decode_greedy(9, 4, 20)
+        assert _plan(m) == plan
+        m.sample_decode(24, 20, 0.9, 0.9, 50, 1.15, 8, np.linspace(0, 0.99, 20, dtype=np.float32), [3, 4])
+        assert _plan(m) == plan
+        m.forward_batch([0], [7], [44])
+        assert _plan(m) == plan
+    dev.close(); plain.close()
