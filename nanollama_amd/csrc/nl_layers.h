@@ -323,7 +323,7 @@ __device__ __forceinline__ void ly_publish(u32x4 *rec, unsigned tag, float v, in
 template <int WT>
 __global__ void __launch_bounds__(LY_THREADS) layers_kernel(LayersParams P0) {
     // (arguments are read again every layer through an opaque pointer: kept in scalar registers across the loop, with all that follows from
-    //  them, they and their derivatives were 270 values spilled into vector lanes)
+    //  them, they and their derivatives were 270 values spilled into vector lanes; 66 still are with Q8_0 and Q6_K weights, 78 with Q4_0 and Q4_K)
     typedef const __attribute__((address_space(4))) LayersParams *Args;
     Args pk = (Args)__builtin_amdgcn_kernarg_segment_ptr();
 #define P (*pk)

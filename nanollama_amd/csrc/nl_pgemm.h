@@ -30,7 +30,7 @@
 // wavefront about 310 cycles: 128 on the matrix pipe, the rest vector instructions (16 scalings, its share of the expansion, addresses).  Those
 // overlap with the MFMAs of the SIMD's other wavefronts (1.47 PFLOP/s beside four vector instructions an MFMA) and not with its own, and a SIMD
 // holds two or three; larger tiles share the expansion and the LDS reads.  A Q4_K prompt of 333 tokens (173M parameters) used to
-// be 333 single-token steps: 151 ms, now 1.44 ms (1.92 at first, 1.49 then with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
+// be 333 single-token steps: 151 ms, now 1.47 ms (1.92 at first, 1.49 then with two fp16 parts an activation, whose error was 1.59e-7 against 1.32e-7 of those
 // steps and 1.19e-7 now, and whose range ends at 65504).
 #pragma once
 #include "nl_qgemm.h"
